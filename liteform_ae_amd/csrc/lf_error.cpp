@@ -1,4 +1,10 @@
-// Error state and status strings of the C ABI.
+// Error state and status strings of the C ABI, and the pool of page-locked read-back buffers.
+#include <hip/hip_runtime.h>
+
+#include <cstdlib>
+#include <mutex>
+#include <vector>
+
 #include "lf_internal.h"
 
 namespace lf {
@@ -16,6 +22,53 @@ int fail(int status, const char* fmt, ...) {
     va_end(ap);
     last_error() = buf;
     return status;
+}
+
+namespace {
+std::mutex g_pinned_lock;
+// (never destroyed: a plan may still be released while the process ends)
+std::vector<void*>& pinned_pool() {
+    static std::vector<void*>* pool = new std::vector<void*>();
+    return *pool;
+}
+}  // namespace
+
+PinnedLoan::PinnedLoan(size_t bytes) {
+    if (bytes <= kPooledBytes) {
+        {
+            std::lock_guard<std::mutex> hold(g_pinned_lock);
+            auto& pool = pinned_pool();
+            if (!pool.empty()) {
+                p_ = pool.back();
+                pool.pop_back();
+                pinned_ = true;
+                return;
+            }
+        }
+        if (hipHostMalloc(&p_, kPooledBytes, hipHostMallocPortable) == hipSuccess) {
+            pinned_ = true;
+            return;
+        }
+        (void)hipGetLastError();
+        p_ = nullptr;
+    }
+    p_ = std::malloc(bytes ? bytes : 1);
+}
+
+PinnedLoan::~PinnedLoan() {
+    if (!pinned_) {
+        std::free(p_);
+        return;
+    }
+    {
+        std::lock_guard<std::mutex> hold(g_pinned_lock);
+        auto& pool = pinned_pool();
+        if (pool.size() < kPooledBuffers) {
+            pool.push_back(p_);
+            return;
+        }
+    }
+    (void)hipHostFree(p_);
 }
 
 }  // namespace lf

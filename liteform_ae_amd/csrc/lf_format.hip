@@ -192,9 +192,75 @@ __device__ __forceinline__ void width_class(int deg, int kmax, int& k, int& cost
     }
 }
 
-// One thread per (row, partition) segment for the counters; blockIdx.y is the partition.
-//   stats[p][k] += {cost rows, nnz, 1}
-//   plane[k][c]  = 1             for every column c of a segment of class k  (skipped when planes is null)
+// Where the counters of partition p and class k lie: field f (0 cost rows, 1 nnz, 2 segments) has a
+// 128-byte line of its own, because atomics of all workgroups on one line are taken one after the
+// other (all counters of a partition side by side: 25 us of class_count_kernel's time).
+constexpr int kStatLine = 16;              // 64-bit words
+__host__ __device__ constexpr size_t stat_at(int p, int k, int f) { return (((size_t)p * LF_MAX_CLASSES + k) * 3 + f) * kStatLine; }
+
+// stats(p, k) += {cost rows, nnz, 1} for every segment of partition p = blockIdx.y.
+// A thread keeps the counters of its rows in registers; a workgroup adds its sums with one atomic
+// per counter.  (LDS atomics per row, from 2048 workgroups, took 48 us for 2.45M rows, this takes
+// 21.)
+constexpr int kCountGrid = 512;
+constexpr int kRowUnroll = 4;              // rows whose bounds a thread requests together
+
+// Degrees of the segments of rows r0, r0 + stride, ... (0 past `end`).
+__device__ __forceinline__ void seg_degrees(const SegView& v, const int32_t* __restrict__ seg_deg, int p, int64_t r0,
+                                            int64_t stride, int64_t end, int (&deg)[kRowUnroll]) {
+#pragma unroll
+    for (int u = 0; u < kRowUnroll; ++u) {
+        const int64_t r = r0 + u * stride;
+        deg[u] = 0;
+        if (r >= end) continue;
+        int start;
+        seg_range(v, r, p, start, deg[u]);
+        if (seg_deg) deg[u] = seg_deg[(int64_t)p * v.rows + r];
+    }
+}
+
+__global__ void __launch_bounds__(kBlock)
+class_count_kernel(SegView v, const int32_t* __restrict__ seg_deg, int kmax, unsigned long long* __restrict__ stats) {
+    constexpr int kStride = kBlock + 4;
+    __shared__ uint32_t s_sum[LF_MAX_CLASSES * 3 * kStride];
+    const int p = blockIdx.y;
+    uint32_t cost[LF_MAX_CLASSES] = {}, nnz[LF_MAX_CLASSES] = {}, cnt[LF_MAX_CLASSES] = {};
+    const int64_t stride = (int64_t)gridDim.x * kBlock;
+    for (int64_t r0 = (int64_t)blockIdx.x * kBlock + threadIdx.x; r0 < v.rows; r0 += kRowUnroll * stride) {
+        int deg[kRowUnroll];
+        seg_degrees(v, seg_deg, p, r0, stride, v.rows, deg);
+#pragma unroll
+        for (int u = 0; u < kRowUnroll; ++u) {
+            int k = -1, cost_rows = 0;
+            if (deg[u] > 0) width_class(deg[u], kmax, k, cost_rows);
+#pragma unroll
+            for (int i = 0; i < LF_MAX_CLASSES; ++i) {
+                cost[i] += k == i ? (uint32_t)cost_rows : 0u;
+                nnz[i] += k == i ? (uint32_t)deg[u] : 0u;
+                cnt[i] += k == i ? 1u : 0u;
+            }
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < LF_MAX_CLASSES; ++i) {
+        s_sum[(3 * i) * kStride + threadIdx.x] = cost[i];
+        s_sum[(3 * i + 1) * kStride + threadIdx.x] = nnz[i];
+        s_sum[(3 * i + 2) * kStride + threadIdx.x] = cnt[i];
+    }
+    __syncthreads();
+    // four threads to a counter
+    const int c = threadIdx.x >> 2, part = threadIdx.x & 3;
+    if (c < 3 * LF_MAX_CLASSES) {
+        uint32_t sum = 0;
+        for (int i = part; i < kBlock; i += 4) sum += s_sum[c * kStride + i];
+        sum += __shfl_xor(sum, 1);
+        sum += __shfl_xor(sum, 2);
+        if (part == 0 && sum) atomicAdd(&stats[stat_at(p, c / 3, c % 3)], (unsigned long long)sum);
+    }
+}
+
+// Column sets as byte planes, for matrices that the bitmaps below do not take: plane[k][c] = 1 for
+// every column c of a segment of class k; blockIdx.y is the partition.
 // Column sets are one byte per (class, column), written with plain stores after an "already
 // set?" probe: no atomics, and a stale probe (another XCD's L2 still holds the old line) only
 // repeats a store of the same value.  blockIdx.z is the class a workgroup marks: workgroups
@@ -213,22 +279,15 @@ __device__ __forceinline__ void width_class(int deg, int kmax, int& k, int& cost
 constexpr int kMarkUnroll = 4;
 
 __global__ void __launch_bounds__(kBlock)
-bucket_stats_kernel(SegView v, const int32_t* __restrict__ indices, const int32_t* __restrict__ seg_deg,
-                    int kmax, uint8_t* __restrict__ planes, int64_t cols,
-                    unsigned long long* __restrict__ stats) {
-    __shared__ unsigned long long s_stats[LF_MAX_CLASSES * LF_STATS_FIELDS];
+mark_planes_kernel(SegView v, const int32_t* __restrict__ indices, const int32_t* __restrict__ seg_deg,
+                   int kmax, uint8_t* __restrict__ planes, int64_t cols) {
     __shared__ int s_off[kBlock + 1];      // exclusive prefix of the lengths of this class's segments
     __shared__ int s_start[kBlock];
     __shared__ int s_wave[kBlock / 64];
-    for (int i = threadIdx.x; i < LF_MAX_CLASSES * LF_STATS_FIELDS; i += kBlock) s_stats[i] = 0ull;
-    __syncthreads();
-
     const int p = blockIdx.y;
     const int kz = blockIdx.z;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    uint8_t* plane = planes ? planes + (size_t)kz * (size_t)cols : nullptr;
-    // a workgroup walks several blocks of rows, so that the global counters below see a few
-    // thousand updates per launch and not one per 256 rows
+    uint8_t* plane = planes + (size_t)kz * (size_t)cols;
     for (int64_t base = (int64_t)blockIdx.x * kBlock; base < v.rows; base += (int64_t)gridDim.x * kBlock) {
         const int64_t r = base + threadIdx.x;
         int start = 0, fill = 0, deg = 0;
@@ -240,14 +299,7 @@ bucket_stats_kernel(SegView v, const int32_t* __restrict__ indices, const int32_
         if (deg > 0) {
             int cost_rows;
             width_class(deg, kmax, k, cost_rows);
-            if (kz == 0) {
-                atomicAdd(&s_stats[k * LF_STATS_FIELDS + 0], (unsigned long long)cost_rows);
-                atomicAdd(&s_stats[k * LF_STATS_FIELDS + 1], (unsigned long long)deg);
-                atomicAdd(&s_stats[k * LF_STATS_FIELDS + 2], 1ull);
-            }
         }
-        if (plane == nullptr) continue;                // uniform over the launch
-
         const int x = k == kz ? fill : 0;
         if (!__syncthreads_or(x)) continue;            // no segment of this class among these rows
         int incl = x;
@@ -289,10 +341,6 @@ bucket_stats_kernel(SegView v, const int32_t* __restrict__ indices, const int32_
         }
         __syncthreads();                               // the tables are rewritten by the next block of rows
     }
-    if (kz != 0) return;
-    __syncthreads();
-    for (int i = threadIdx.x; i < LF_MAX_CLASSES * LF_STATS_FIELDS; i += kBlock)
-        if (s_stats[i]) atomicAdd(&stats[(size_t)p * LF_MAX_CLASSES * LF_STATS_FIELDS + i], s_stats[i]);
 }
 
 // hist[p][mask] = number of columns of partition p whose set of classes is mask
@@ -314,6 +362,335 @@ colmask_hist_kernel(const uint8_t* __restrict__ planes, int num_classes, int64_t
     }
     __syncthreads();
     for (int i = threadIdx.x; i < kBins; i += kBlock)
+        if (s_hist[i]) atomicAdd(&hist[(size_t)p * kBins + i], (unsigned long long)s_hist[i]);
+}
+
+// ---- column sets through bitmaps in LDS
+// The byte planes above cost one line over the fabric per probe and per first-touch store.  Where
+// a partition's columns fit a few bitmaps of one LDS each, a workgroup instead owns one (partition,
+// slice of columns, class) at a time: it walks its share of the class's segments, ORs their
+// columns into a bitmap in LDS and writes the bitmap out once; colbits_hist_kernel ORs the bitmaps
+// of the workgroups that shared an item and counts the class masks.  The indices are streamed once
+// per slice, everything else stays in the CU.  2.45M columns (two slices), 81M entries: the
+// column pass takes 0.25 ms where the planes took 1.38 (marking 0.20, listing 0.03, histogram 0.02).
+//
+// Segments are first listed by class (class_list_kernel), because a class is a scattered subset of
+// the rows: finding it again in every workgroup would cost 11 sweeps over the row pointer.
+constexpr int kMarkThreads = 1024;
+constexpr int kMarkMaxWords = 38912;       // 152 KB of the 160 KB of LDS: 1,245,184 columns
+constexpr int kMarkTwoPerCu = 18432;       // bitmaps of up to 72 KB: two workgroups share a CU
+constexpr int kMarkItems = 512;            // (partition, slice, class) triples at most
+constexpr int kMarkMaxSlices = 8;          // every slice of a partition streams the indices again
+// Below this many rows the two launches more cost what the planes' lines do (search statistics, 30
+// entries a row: 54 us either way at 30K rows, 89 against 97 at 100K rows and two partitions).
+constexpr int64_t kMarkMinRows = 131072;
+constexpr int64_t kMarkMaxSegments = 1ll << 26;     // 8 bytes each in the workspace
+constexpr int kMarkUnrollB = 8;
+constexpr int kMarkBigSegment = 8192;      // longer segments are shared by all workgroups of their item
+constexpr int kMarkEntries = 16384;        // entries that are worth one more workgroup
+constexpr int kListGrid = 512;
+
+struct MarkShape {
+    int slices;              // slices of a partition; 0: the bitmap path does not apply
+    int words;               // bitmap words of a slice
+    int64_t slice_cols;      // columns of a slice (a multiple of 32)
+    int groups;              // workgroups
+};
+
+MarkShape mark_shape(int64_t rows, int64_t cols, int parts) {
+    MarkShape m{};
+    const int64_t psize = (cols + parts - 1) / parts;
+    const int64_t slices = (psize + (int64_t)kMarkMaxWords * 32 - 1) / ((int64_t)kMarkMaxWords * 32);
+    if (rows < kMarkMinRows || slices > kMarkMaxSlices || slices * parts * LF_MAX_CLASSES > kMarkItems || rows * parts > kMarkMaxSegments) return m;
+    m.slices = (int)slices;
+    m.slice_cols = ((psize + slices - 1) / slices + 31) / 32 * 32;
+    m.words = (int)(m.slice_cols / 32);
+    m.groups = m.words <= kMarkTwoPerCu ? 512 : 256;
+    if (m.groups < m.slices * parts * LF_MAX_CLASSES) m.groups = kMarkItems;
+    return m;
+}
+
+// lists[p * rows + first segment of class k ..) = (start, fill) of the segments of class k of partition
+// p; the classes follow one another, a class's segments are in no particular order except that those
+// of more than kMarkBigSegment entries are the last of the last class.
+__global__ void __launch_bounds__(kBlock)
+class_list_kernel(SegView v, const int32_t* __restrict__ seg_deg, int kmax,
+                  unsigned long long* __restrict__ stats,
+                  int2* __restrict__ lists) {
+    __shared__ uint32_t s_cnt[LF_MAX_CLASSES + 1], s_at[LF_MAX_CLASSES + 1];
+    const int p = blockIdx.y;
+    if (threadIdx.x <= LF_MAX_CLASSES) s_cnt[threadIdx.x] = 0;
+    __syncthreads();
+    const int64_t per = (v.rows + gridDim.x - 1) / gridDim.x;
+    const int64_t lo = (int64_t)blockIdx.x * per, hi = lo + per < v.rows ? lo + per : v.rows;
+    for (int64_t r0 = lo + threadIdx.x; r0 < hi; r0 += kRowUnroll * kBlock) {
+        int deg[kRowUnroll];
+        seg_degrees(v, seg_deg, p, r0, kBlock, hi, deg);
+#pragma unroll
+        for (int u = 0; u < kRowUnroll; ++u) {
+            int k, cost_rows;
+            if (deg[u] <= 0) continue;
+            width_class(deg[u], kmax, k, cost_rows);
+            atomicAdd(&s_cnt[deg[u] > kMarkBigSegment && k == kmax ? kmax + 1 : k], 1u);
+        }
+    }
+    __syncthreads();
+    if (threadIdx.x <= (unsigned)kmax + 1) {
+        // (the cursors are spare words of the counters' lines; kmax + 1 are the last class's longest
+        // segments, listed from its end)
+        const int k = min((int)threadIdx.x, kmax), big = (int)threadIdx.x > kmax;
+        uint32_t first = 0;
+        for (int i = 0; i < k + big; ++i) first += (uint32_t)stats[stat_at(p, i, 2)];
+        const uint32_t n = s_cnt[threadIdx.x];
+        const uint32_t taken = n ? (uint32_t)atomicAdd(&stats[stat_at(p, k, 2) + 1 + big], (unsigned long long)n) : 0u;
+        s_at[threadIdx.x] = big ? first - taken - n : first + taken;
+    }
+    __syncthreads();
+    int2* out = lists + (size_t)p * (size_t)v.rows;
+    for (int64_t r0 = lo + threadIdx.x; r0 < hi; r0 += kRowUnroll * kBlock) {
+        int deg[kRowUnroll], start[kRowUnroll], fill[kRowUnroll];
+        seg_degrees(v, seg_deg, p, r0, kBlock, hi, deg);
+#pragma unroll
+        for (int u = 0; u < kRowUnroll; ++u) {
+            start[u] = fill[u] = 0;
+            if (r0 + u * kBlock < hi) seg_range(v, r0 + u * kBlock, p, start[u], fill[u]);
+        }
+#pragma unroll
+        for (int u = 0; u < kRowUnroll; ++u) {
+            int k, cost_rows;
+            if (deg[u] <= 0) continue;
+            width_class(deg[u], kmax, k, cost_rows);
+            out[atomicAdd(&s_at[deg[u] > kMarkBigSegment && k == kmax ? kmax + 1 : k], 1u)] = make_int2(start[u], fill[u]);
+        }
+    }
+}
+
+// Marks up to 64 * kMarkUnrollB entries of a segment from its entry j on.
+template <typename Mark>
+__device__ __forceinline__ void mark_piece(const int32_t* __restrict__ indices, int start, int j, int fill, Mark mark) {
+    const int lane = threadIdx.x & 63;
+    uint32_t c[kMarkUnrollB];
+#pragma unroll
+    for (int u = 0; u < kMarkUnrollB; ++u) {
+        const int i = j + u * 64 + lane;
+        c[u] = i < fill ? (uint32_t)indices[start + i] : 0xFFFFFFFFu;
+    }
+#pragma unroll
+    for (int u = 0; u < kMarkUnrollB; ++u)
+        if (c[u] != 0xFFFFFFFFu) mark(c[u]);
+}
+
+// The segments of the last class, of any length, one at a time per wavefront.
+template <typename Mark>
+__device__ __forceinline__ void mark_long(const int32_t* __restrict__ indices, const int2* __restrict__ list, int n_seg,
+                                          int first_wave, int waves, Mark mark) {
+    int2 seg = first_wave < n_seg ? list[first_wave] : make_int2(0, 0);
+    for (int i = first_wave; i < n_seg; i += waves) {
+        const int2 cur = seg;
+        if (i + waves < n_seg) seg = list[i + waves];                // a round ahead
+        for (int j = 0; j < cur.y; j += 64 * kMarkUnrollB) mark_piece(indices, cur.x, j, cur.y, mark);
+    }
+}
+
+// Marks the segments of class k (at most 2^k entries) that fall to one wavefront; K = min(k, 6).
+// The wavefront takes a group of segments at a time, one lane holding each, and walks it in steps of
+// 64 entries - 64 / 2^K segments side by side, or a 64-entry piece of a longer one - eight steps'
+// loads in flight.
+template <int K, typename Mark>
+__device__ __forceinline__ void mark_class(const int32_t* __restrict__ indices, const int2* __restrict__ list, int n_seg,
+                                           int k, int first_wave, int waves, Mark mark) {
+    constexpr int kSide = 64 >> K;                     // segments side by side
+    const int lane = threadIdx.x & 63;
+    const int q = lane & ((1 << K) - 1), sub = lane >> K;
+    const int log_pieces = k - K;
+    const int group = K < 6 ? 64 : (64 >> (log_pieces < 4 ? log_pieces : 4));     // segments of a group
+    const int steps = (group / kSide) << log_pieces;
+    int64_t i0 = (int64_t)first_wave * group;
+    const int64_t stride = (int64_t)waves * group;
+    int2 seg = make_int2(0, 0);
+    if (lane < group && i0 + lane < n_seg) seg = list[i0 + lane];
+    for (; i0 < n_seg; i0 += stride) {
+        const int2 cur = seg;
+        seg = make_int2(0, 0);
+        if (lane < group && i0 + stride + lane < n_seg) seg = list[i0 + stride + lane];      // a round ahead
+        for (int t0 = 0; t0 < steps; t0 += kMarkUnrollB) {
+            uint32_t c[kMarkUnrollB];
+            bool on[kMarkUnrollB];
+#pragma unroll
+            for (int u = 0; u < kMarkUnrollB; ++u) {
+                const int t = t0 + u;
+                int start, fill, at = q;
+                if constexpr (K == 6) {
+                    const int src = (t >> log_pieces) & 63;
+                    start = __builtin_amdgcn_readlane(cur.x, src);
+                    fill = __builtin_amdgcn_readlane(cur.y, src);
+                    at = ((t & ((1 << log_pieces) - 1)) << 6) + lane;
+                } else {
+                    start = __shfl(cur.x, (t * kSide + sub) & 63);
+                    fill = __shfl(cur.y, (t * kSide + sub) & 63);
+                }
+                on[u] = t < steps && at < fill;
+                c[u] = on[u] ? (uint32_t)indices[start + at] : 0u;
+            }
+#pragma unroll
+            for (int u = 0; u < kMarkUnrollB; ++u)
+                if (on[u]) mark(c[u]);
+        }
+    }
+}
+
+// One workgroup per share of an item (partition p, slice s, class k), i = (p * slices + s) * classes
+// + k: workgroups are dealt out in proportion to the entries of the item's class, at least one to an
+// item that has any.  table[i] = first workgroup of item i, table[n_items] = workgroups in use.
+__global__ void __launch_bounds__(kMarkThreads)
+mark_columns_kernel(const int32_t* __restrict__ indices, const int2* __restrict__ lists, int64_t rows, int parts,
+                    int num_classes, MarkShape shape, int64_t psize, int64_t cols,
+                    const unsigned long long* __restrict__ stats, int32_t* __restrict__ table,
+                    uint32_t* __restrict__ bitmaps) {
+    extern __shared__ uint32_t s_bits[];
+    __shared__ int s_first[kMarkItems + 1];
+    __shared__ unsigned long long s_sum[kMarkThreads / 64];
+    __shared__ int s_cnt[kMarkThreads / 64];
+    __shared__ int s_item;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int n_items = parts * shape.slices * num_classes;
+
+    // ---- which item, and which share of it
+    unsigned long long w = 0;                          // entries and unused lanes (a step costs what it costs)
+    if (tid < n_items) {
+        const int kk = tid % num_classes, pp = tid / num_classes / shape.slices;
+        const unsigned long long entries = stats[stat_at(pp, kk, 1)], segs = stats[stat_at(pp, kk, 2)];
+        w = kk <= 6 ? segs << kk : entries + 32 * segs;
+        if (kk == num_classes - 1) w += entries;
+        if (kk < 3) w *= 4 - kk;                       // (short segments: every lane or pair of lanes on a line of its own)
+    }
+    unsigned long long sum = w;
+    for (int d = 32; d > 0; d >>= 1) sum += __shfl_xor(sum, d);
+    if (lane == 0) { s_sum[wave] = sum; }
+    const int nz_wave = __popcll(__ballot(w > 0));
+    if (lane == 0) s_cnt[wave] = nz_wave;
+    __syncthreads();
+    unsigned long long total = 0;
+    int nz = 0;
+    for (int i = 0; i < kMarkThreads / 64; ++i) { total += s_sum[i]; nz += s_cnt[i]; }
+    const unsigned long long worth = total / kMarkEntries;      // a small matrix is not spread over more bitmaps than it pays for
+    const unsigned long long more = worth < gridDim.x - nz ? worth : gridDim.x - nz;
+    const int m = w > 0 ? 1 + (int)(more * w / total) : 0;
+    int incl = m;
+    for (int d = 1; d < 64; d <<= 1) {
+        const int y = __shfl_up(incl, d);
+        if (lane >= d) incl += y;
+    }
+    __syncthreads();
+    if (lane == 63) s_cnt[wave] = incl;
+    if (tid == 0) s_item = -1;
+    __syncthreads();
+    int before = incl - m;
+    for (int i = 0; i < wave; ++i) before += s_cnt[i];
+    if (tid < n_items) {
+        s_first[tid] = before;
+        if (tid == n_items - 1) s_first[n_items] = before + m;
+        if ((int)blockIdx.x >= before && (int)blockIdx.x < before + m) s_item = tid;
+    }
+    for (int i = tid; i < shape.words; i += kMarkThreads) s_bits[i] = 0;
+    __syncthreads();
+    if (blockIdx.x == 0)
+        for (int i = tid; i <= n_items; i += kMarkThreads) table[i] = s_first[i];
+    const int item = s_item;
+    if (item < 0) return;                              // more workgroups than shares
+
+    const int k = item % num_classes, s = item / num_classes % shape.slices, p = item / num_classes / shape.slices;
+    const int share = (int)blockIdx.x - s_first[item], shares = s_first[item + 1] - s_first[item];
+    const int64_t c0 = (int64_t)p * psize + (int64_t)s * shape.slice_cols;
+    int64_t c1 = c0 + shape.slice_cols;
+    if (c1 > (int64_t)(p + 1) * psize) c1 = (int64_t)(p + 1) * psize;
+    if (c1 > cols) c1 = cols;
+    const uint32_t span = c1 > c0 ? (uint32_t)(c1 - c0) : 0u;
+    const uint32_t base_col = (uint32_t)c0;
+    uint32_t first = 0;
+    for (int i = 0; i < k; ++i) first += (uint32_t)stats[stat_at(p, i, 2)];
+    const int n_big = k == num_classes - 1 ? (int)stats[stat_at(p, k, 2) + 2] : 0;
+    const int n_seg = (int)stats[stat_at(p, k, 2)] - n_big;
+    const int2* list = lists + (size_t)p * (size_t)rows + first;
+    auto mark = [&](uint32_t c) {
+        const uint32_t x = c - base_col;               // (wraps to a large value below the slice)
+        if (x < span) atomicOr(&s_bits[x >> 5], 1u << (x & 31u));
+    };
+
+    const int waves = shares * (kMarkThreads / 64);
+    const int first_wave = share * (kMarkThreads / 64) + wave;
+    switch (k < num_classes - 1 ? k : LF_MAX_CLASSES) {
+        case 0: mark_class<0>(indices, list, n_seg, k, first_wave, waves, mark); break;
+        case 1: mark_class<1>(indices, list, n_seg, k, first_wave, waves, mark); break;
+        case 2: mark_class<2>(indices, list, n_seg, k, first_wave, waves, mark); break;
+        case 3: mark_class<3>(indices, list, n_seg, k, first_wave, waves, mark); break;
+        case 4: mark_class<4>(indices, list, n_seg, k, first_wave, waves, mark); break;
+        case 5: mark_class<5>(indices, list, n_seg, k, first_wave, waves, mark); break;
+        default:
+            if (k < num_classes - 1) mark_class<6>(indices, list, n_seg, k, first_wave, waves, mark);
+            break;
+    }
+    if (k == num_classes - 1) mark_long(indices, list, n_seg, first_wave, waves, mark);
+    for (int i = 0; i < n_big; ++i) {
+        const int2 seg = list[n_seg + i];
+        const int64_t stride = (int64_t)waves * 64 * kMarkUnrollB;
+        for (int64_t j = (int64_t)first_wave * 64 * kMarkUnrollB; j < seg.y; j += stride)
+            mark_piece(indices, seg.x, (int)j, seg.y, mark);
+    }
+    __syncthreads();
+    uint32_t* out = bitmaps + (size_t)blockIdx.x * shape.words;
+    for (int i = tid; i < shape.words; i += kMarkThreads) out[i] = s_bits[i];
+}
+
+// hist[p][mask] from the bitmaps; blockIdx.y = p * slices + s.  A workgroup takes tiles of 64 words:
+// thread (class, word) ORs the bitmaps of the workgroups that shared the item, all classes' loads in
+// flight together, then every thread builds the masks of two of the tile's 2048 columns.
+constexpr int kHistThreads = 1024;
+constexpr int kHistGrid = 256;
+__global__ void __launch_bounds__(kHistThreads)
+colbits_hist_kernel(const uint32_t* __restrict__ bitmaps, const int32_t* __restrict__ table, int num_classes,
+                    MarkShape shape, int64_t psize, int64_t cols, unsigned long long* __restrict__ hist) {
+    constexpr int kBins = 1 << LF_MAX_CLASSES;
+    __shared__ uint32_t s_hist[kBins];
+    __shared__ uint32_t s_bits[16][64];
+    for (int i = threadIdx.x; i < kBins; i += kHistThreads) s_hist[i] = 0;
+    const int p = blockIdx.y / shape.slices, s = blockIdx.y % shape.slices;
+    const int64_t c0 = (int64_t)p * psize + (int64_t)s * shape.slice_cols;
+    int64_t c1 = c0 + shape.slice_cols;
+    if (c1 > (int64_t)(p + 1) * psize) c1 = (int64_t)(p + 1) * psize;
+    if (c1 > cols) c1 = cols;
+    const int k = threadIdx.x >> 6, word = threadIdx.x & 63;
+    int g0 = 0, g1 = 0;
+    if (k < num_classes) {
+        g0 = table[(int)blockIdx.y * num_classes + k];
+        g1 = table[(int)blockIdx.y * num_classes + k + 1];
+    }
+    for (int w0 = blockIdx.x * 64; w0 < shape.words && c0 + (int64_t)w0 * 32 < c1; w0 += gridDim.x * 64) {      // uniform
+        uint32_t bits = 0;
+        if (w0 + word < shape.words) {
+            for (int g = g0; g < g1; g += 8) {
+                uint32_t x[8];
+#pragma unroll
+                for (int u = 0; u < 8; ++u) x[u] = bitmaps[(size_t)min(g + u, g1 - 1) * shape.words + w0 + word];
+#pragma unroll
+                for (int u = 0; u < 8; ++u) bits |= x[u];
+            }
+        }
+        s_bits[k][word] = bits;
+        __syncthreads();
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            const int c = h * kHistThreads + threadIdx.x;        // column of the tile
+            if (c0 + (int64_t)w0 * 32 + c < c1) {
+                uint32_t mask = 0;
+#pragma unroll
+                for (int i = 0; i < LF_MAX_CLASSES; ++i) mask |= ((s_bits[i][c >> 5] >> (c & 31)) & 1u) << i;
+                atomicAdd(&s_hist[mask], 1u);
+            }
+        }
+        __syncthreads();
+    }
+    for (int i = threadIdx.x; i < kBins; i += kHistThreads)
         if (s_hist[i]) atomicAdd(&hist[(size_t)p * kBins + i], (unsigned long long)s_hist[i]);
 }
 
@@ -617,7 +994,7 @@ hyb_fill_kernel(SegView v, const int32_t* __restrict__ seg_deg, const int32_t* _
 
 // ---------------------------------------------------------------------------- host helpers
 struct StatsLayout {
-    size_t bnd, planes, stats, hist, total;
+    size_t bnd, planes, lists, bitmaps, table, stats, hist, total;
 };
 
 StatsLayout stats_layout(int64_t rows, int64_t cols, int parts) {
@@ -625,10 +1002,19 @@ StatsLayout stats_layout(int64_t rows, int64_t cols, int parts) {
     size_t off = 0;
     L.bnd = off;
     if (parts > 1) off += align_up((size_t)(parts + 1) * rows * 4, 256);
-    L.planes = off;
-    off += align_up((size_t)LF_MAX_CLASSES * (size_t)cols, 256);
+    const MarkShape m = mark_shape(rows, cols, parts);
+    L.planes = L.lists = L.bitmaps = L.table = off;      // byte planes, or segment lists and bitmaps
+    if (m.slices > 0) {
+        off += align_up((size_t)parts * (size_t)rows * 8, 256);
+        L.bitmaps = off;
+        off += align_up((size_t)m.groups * (size_t)m.words * 4, 256);
+        L.table = off;
+        off += align_up((size_t)(kMarkItems + 1) * 4, 256);
+    } else {
+        off += align_up((size_t)LF_MAX_CLASSES * (size_t)cols, 256);
+    }
     L.stats = off;
-    off += align_up((size_t)parts * LF_MAX_CLASSES * LF_STATS_FIELDS * 8, 256);
+    off += align_up(stat_at(parts, 0, 0) * 8, 256);
     L.hist = off;
     off += align_up((size_t)parts * (1 << LF_MAX_CLASSES) * 8, 256);
     L.total = off;
@@ -758,10 +1144,11 @@ int lf_bucket_stats(const int32_t* d_indptr, const int32_t* d_indices, const int
     unsigned long long* stats = (unsigned long long*)(ws + L.stats);
     unsigned long long* hist = (unsigned long long*)(ws + L.hist);
     const int64_t psize = lf::ceil_div(num_cols, num_parts);
-    const size_t stats_bytes = (size_t)num_parts * LF_MAX_CLASSES * LF_STATS_FIELDS * 8;
     const size_t hist_bytes = (size_t)num_parts * (1 << LF_MAX_CLASSES) * 8;
 
-    if (h_colhist)
+    const MarkShape mark = mark_shape(num_rows, num_cols, num_parts);
+    const bool use_planes = h_colhist && mark.slices == 0;
+    if (use_planes)
         LF_HIP(fill_u32(planes, (L.total - L.planes) / 4, 0u, s));   // planes, stats and hist
     else
         LF_HIP(fill_u32(stats, (L.total - L.stats) / 4, 0u, s));
@@ -773,18 +1160,45 @@ int lf_bucket_stats(const int32_t* d_indptr, const int32_t* d_indices, const int
         }
         SegView v{d_indptr, bnd, num_rows, num_parts};
         const int num_classes = lf::ilog2(width_limit) + 1;
-        bucket_stats_kernel<<<dim3(std::min(nblk, kStatsGrid), num_parts, h_colhist ? num_classes : 1), kBlock, 0, s>>>(
-            v, d_indices, d_seg_deg, num_classes - 1, h_colhist ? planes : nullptr, num_cols, stats);
+        class_count_kernel<<<dim3(std::min(nblk, kCountGrid), num_parts), kBlock, 0, s>>>(v, d_seg_deg, num_classes - 1, stats);
         LF_HIP(hipGetLastError());
-        if (h_colhist) {
+        if (h_colhist && !use_planes) {
+            int2* lists = (int2*)(ws + L.lists);
+            uint32_t* bitmaps = (uint32_t*)(ws + L.bitmaps);
+            int32_t* table = (int32_t*)(ws + L.table);
+            class_list_kernel<<<dim3(std::min(nblk, kListGrid), num_parts), kBlock, 0, s>>>(
+                v, d_seg_deg, num_classes - 1, stats, lists);
+            LF_HIP(hipGetLastError());
+            LF_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(mark_columns_kernel),
+                                       hipFuncAttributeMaxDynamicSharedMemorySize, kMarkMaxWords * 4));
+            mark_columns_kernel<<<mark.groups, kMarkThreads, (size_t)mark.words * 4, s>>>(
+                d_indices, lists, num_rows, num_parts, num_classes, mark, psize, num_cols, stats, table, bitmaps);
+            LF_HIP(hipGetLastError());
+            colbits_hist_kernel<<<dim3(std::min((mark.words + 63) / 64, kHistGrid), num_parts * mark.slices), kHistThreads, 0, s>>>(
+                bitmaps, table, num_classes, mark, psize, num_cols, hist);
+            LF_HIP(hipGetLastError());
+        }
+        if (use_planes) {
+            mark_planes_kernel<<<dim3(std::min(nblk, kStatsGrid), num_parts, num_classes), kBlock, 0, s>>>(
+                v, d_indices, d_seg_deg, num_classes - 1, planes, num_cols);
+            LF_HIP(hipGetLastError());
             const int hgrid = (int)std::min<int64_t>((psize + kBlock - 1) / kBlock, 1024);
             colmask_hist_kernel<<<dim3(hgrid, num_parts), kBlock, 0, s>>>(planes, num_classes, num_cols, psize, hist);
             LF_HIP(hipGetLastError());
         }
     }
-    LF_HIP(hipMemcpyAsync(h_stats, stats, stats_bytes, hipMemcpyDeviceToHost, s));
-    if (h_colhist) LF_HIP(hipMemcpyAsync(h_colhist, hist, hist_bytes, hipMemcpyDeviceToHost, s));
+    const size_t lines_bytes = stat_at(num_parts, 0, 0) * 8;
+    lf::PinnedLoan back(lines_bytes + (h_colhist ? hist_bytes : 0));
+    LF_REQUIRE(back.ok(), LF_ERR_HIP, "out of host memory");
+    const unsigned long long* h_lines = back.as<unsigned long long>();
+    LF_HIP(hipMemcpyAsync(back.as<char>(), stats, lines_bytes, hipMemcpyDeviceToHost, s));
+    if (h_colhist) LF_HIP(hipMemcpyAsync(back.as<char>(lines_bytes), hist, hist_bytes, hipMemcpyDeviceToHost, s));
     LF_HIP(hipStreamSynchronize(s));
+    for (int p = 0; p < num_parts; ++p)
+        for (int k = 0; k < LF_MAX_CLASSES; ++k)
+            for (int f = 0; f < LF_STATS_FIELDS; ++f)
+                h_stats[((size_t)p * LF_MAX_CLASSES + k) * LF_STATS_FIELDS + f] = f < 3 ? (int64_t)h_lines[stat_at(p, k, f)] : 0;
+    if (h_colhist) std::memcpy(h_colhist, back.as<char>(lines_bytes), hist_bytes);
     return LF_OK;
 }
 

@@ -5,6 +5,7 @@ Format structures must match bit for bit."""
 import numpy as np
 import pytest
 
+from liteform_ae_amd.format_matrix_market import MTX
 from oracle import liteform_oracle as O
 
 from helpers import assert_hyb_equal, mtx_from_rows, skewed_matrix, stats_from_oracle
@@ -45,6 +46,47 @@ def test_bucket_stats_match_oracle(fa, seed):
     wstats, whist = stats_from_oracle(g, parts)
     np.testing.assert_array_equal(stats, wstats)
     np.testing.assert_array_equal(hist, whist)
+
+
+@pytest.mark.parametrize("nr,nc,parts,limit", [
+    (131072, 70_001, 1, 1024),          # the smallest matrix whose column sets are LDS bitmaps
+    (131071, 70_001, 1, 1024),          # ... and the largest below it
+    (131073, 1_245_184, 1, 1024),       # the largest single slice
+    (131073, 1_245_185, 1, 1024),       # two slices
+    (140_000, 2_600_011, 2, 1024),      # two partitions of two slices
+    (140_000, 31, 2, 1024),             # a bitmap of one word
+    (131072, 9000, 46, 1024),           # the most (partition, class) pairs
+    (131072, 9000, 47, 1024),           # one more: byte planes
+    (131072, 40_000, 3, 16),            # most entries in segments beyond the last class's width
+])
+def test_column_sets_of_large_matrices(fa, nr, nc, parts, limit):
+    rng = np.random.default_rng(nr + nc + parts)
+    deg = np.minimum(rng.geometric(0.2, size=nr) - 1, nc)
+    deg[rng.integers(0, nr, size=40)] = np.minimum(rng.integers(60, 1100, size=40), nc)
+    deg[[0, nr // 2, nr - 1]] = min(nc, 8193), min(nc, 8192), min(nc, 30_000)
+    row = np.repeat(np.arange(nr), deg)
+    key = np.unique(row * nc + rng.integers(0, nc, size=len(row)))
+    row, col = key // nc, key % nc
+    g = MTX.from_coo(row, col, (nr, nc))
+    stats, hist = fa.bucket_statistics(g, parts, width_limit=limit)
+
+    psize = -(-nc // parts)
+    seg = (col // psize) * nr + row
+    fill = np.bincount(seg, minlength=parts * nr)
+    pow2 = np.where(fill > 0, 2 ** np.ceil(np.log2(np.maximum(fill, 1))).astype(np.int64), 0)
+    k = np.log2(np.maximum(np.minimum(pow2, limit), 1)).astype(np.int64)
+    touched = np.unique(k[seg] * nc + col)                        # every (class, column) once
+    masks = np.zeros(nc, np.int64)
+    np.add.at(masks, touched % nc, 1 << (touched // nc))
+    for p in range(parts):
+        lo, hi = p * psize, min(nc, (p + 1) * psize)
+        want = np.bincount(masks[lo:hi], minlength=2048) if hi > lo else np.zeros(2048, np.int64)
+        np.testing.assert_array_equal(hist[p], want)
+        mine, f = k[p * nr:(p + 1) * nr], fill[p * nr:(p + 1) * nr]
+        for c in range(11):
+            on = (f > 0) & (mine == c)
+            rows = np.maximum(1, pow2[p * nr:(p + 1) * nr][on] // limit).sum()
+            assert stats[p, c].tolist() == [rows, f[on].sum(), on.sum(), 0]
 
 
 @pytest.mark.parametrize("seed", range(8))
