@@ -149,35 +149,47 @@ row_features_kernel(const int32_t* __restrict__ indptr, int64_t rows, unsigned l
 }
 
 // out[0] += entries of row r that also occur in row r - 1, out[1] += entries of row r, for every
-// stride-th row r >= 1 (two-pointer walk over the two ascending column lists).  Only the first
-// kOverlapEntries entries of either row are looked at: one thread walks a pair of rows, and a
-// sample that lands on a row of 100,000 entries would otherwise take longer than composing the
-// whole format (11 ms against 0.3 ms for a 500k x 2M matrix with 50 such rows).
+// stride-th row r >= 1.  A wavefront takes a pair of rows: lane i holds the i-th entry of either row
+// and looks its entry of row r up among those of row r - 1.  Only the first kOverlapEntries = 64
+// entries of either row are looked at: a sample that lands on a row of 100,000 entries would
+// otherwise take longer than composing the whole format (11 ms against 0.3 ms for a 500k x 2M matrix
+// with 50 such rows).  Bound by latency: a thread per pair with a two-pointer walk was a chain of up
+// to 128 loads, 15.6 us for 8192 pairs.
 constexpr int kOverlapEntries = 64;
 __global__ void __launch_bounds__(kBlock)
 row_overlap_kernel(const int32_t* __restrict__ indptr, const int32_t* __restrict__ indices, int64_t rows,
                    int64_t stride, unsigned long long* __restrict__ out) {
-    unsigned long long both = 0, seen = 0;
-    for (int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x;; i += (int64_t)gridDim.x * kBlock) {
+    const int lane = threadIdx.x & 63;
+    uint32_t both = 0, seen = 0;
+    const int64_t waves = (int64_t)gridDim.x * (kBlock / 64);
+    for (int64_t i = (int64_t)blockIdx.x * (kBlock / 64) + (threadIdx.x >> 6);; i += waves) {
         const int64_t r = 1 + i * stride;
         if (r >= rows) break;
-        int a = indptr[r - 1], b = indptr[r];
-        const int a_end = min(b, a + kOverlapEntries), b_end = min(indptr[r + 1], b + kOverlapEntries);
-        seen += (unsigned long long)(b_end - b);
-        while (a < a_end && b < b_end) {
-            const int ca = indices[a], cb = indices[b];
-            both += ca == cb;
-            a += ca <= cb;
-            b += cb <= ca;
+        const int a = indptr[r - 1], b = indptr[r];
+        const int na = min(b - a, kOverlapEntries), nb = min(indptr[r + 1] - b, kOverlapEntries);
+        const int ca = lane < na ? indices[a + lane] : 0x7FFFFFFF;      // columns are below 2^31 - 1
+        const int cb = lane < nb ? indices[b + lane] : -1;
+        int lo = 0;                                     // entries of row r - 1 below cb
+#pragma unroll
+        for (int step = 32; step > 0; step >>= 1) {
+            const int x = __shfl(ca, lo + step - 1);
+            if (x < cb) lo += step;
         }
+        const int hit = __shfl(ca, lo & 63);            // (all lanes take part)
+        both += lane < nb && hit == cb;
+        seen += lane < nb;
     }
     for (int d = 32; d > 0; d >>= 1) {
         both += __shfl_xor(both, d);
         seen += __shfl_xor(seen, d);
     }
-    if ((threadIdx.x & 63) == 0 && seen) {
-        atomicAdd(&out[0], both);
-        atomicAdd(&out[1], seen);
+    __shared__ uint32_t s_sum[2][kBlock / 64];
+    if (lane == 0) { s_sum[0][threadIdx.x >> 6] = both; s_sum[1][threadIdx.x >> 6] = seen; }
+    __syncthreads();
+    if (threadIdx.x < 2) {
+        unsigned long long sum = 0;
+        for (int w = 0; w < kBlock / 64; ++w) sum += s_sum[threadIdx.x][w];
+        if (sum) atomicAdd(&out[threadIdx.x], sum);
     }
 }
 
@@ -1160,7 +1172,7 @@ int lf_bucket_stats(const int32_t* d_indptr, const int32_t* d_indices, const int
         }
         SegView v{d_indptr, bnd, num_rows, num_parts};
         const int num_classes = lf::ilog2(width_limit) + 1;
-        class_count_kernel<<<dim3(std::min(nblk, kCountGrid), num_parts), kBlock, 0, s>>>(v, d_seg_deg, num_classes - 1, stats);
+        class_count_kernel<<<dim3(std::min((nblk + kRowUnroll - 1) / kRowUnroll, kCountGrid), num_parts), kBlock, 0, s>>>(v, d_seg_deg, num_classes - 1, stats);
         LF_HIP(hipGetLastError());
         if (h_colhist && !use_planes) {
             int2* lists = (int2*)(ws + L.lists);
@@ -1234,7 +1246,7 @@ int lf_row_overlap(const int32_t* d_indptr, const int32_t* d_indices, int64_t nu
     unsigned long long* acc = (unsigned long long*)d_scratch;
     LF_HIP(fill_u32(acc, 4, 0u, s));
     const int64_t samples = (num_rows - 1 + sample_stride - 1) / sample_stride;
-    const int grid = (int)std::min<int64_t>((samples + kBlock - 1) / kBlock, 1024);
+    const int grid = (int)std::min<int64_t>((samples + kBlock / 64 - 1) / (kBlock / 64), 1024);
     row_overlap_kernel<<<grid, kBlock, 0, s>>>(d_indptr, d_indices, num_rows, sample_stride, acc);
     LF_HIP(hipGetLastError());
     LF_HIP(hipMemcpyAsync(h_out, acc, 16, hipMemcpyDeviceToHost, s));

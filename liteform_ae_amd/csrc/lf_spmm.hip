@@ -660,40 +660,19 @@ __device__ __forceinline__ int merge_group(const int32_t* __restrict__ cols, con
     return m;
 }
 
-// One candidate bucket of the row-group analysis.
+// One bucket of the row-group analysis.
 struct RowGroupCand {
     const int32_t* cols;
     const int32_t* meta;
     long long n_rows;
     long long n_groups;
-    int32_t* m_out;            // merged length of every group, or null
+    int32_t* m_out;            // merged length of every group
     int log_w;
-    int stride;                // > 1: only every stride-th group is looked at (sampling)
+    int pad_;
 };
 
-// counters[3 * cand + ...]: [0] merged entries, [1] gathers of the plain path (row lengths
-// rounded up to the unroll; when sampling, the slots that the merged entries consumed),
-// [2] longest group.  blockIdx.y is the candidate.
-__global__ void __launch_bounds__(256)
-rowgroup_count_kernel(const RowGroupCand* __restrict__ cands, unsigned long long* __restrict__ counters) {
-    const RowGroupCand cd = cands[blockIdx.y];
-    const long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    const long long g = t * cd.stride;
-    int m = 0, plain = 0;
-    if (g < cd.n_groups) {
-        if (cd.stride > 1) {
-            // sampling: the first merged entries of the group against the slots they consume
-            m = merge_group<false>(cd.cols, nullptr, cd.meta, g, cd.n_rows, cd.log_w,
-                                   [](int, int, const float*, uint32_t) {}, kRowGroupSampleEntries, &plain);
-        } else {
-            m = merge_group<false>(cd.cols, nullptr, cd.meta, g, cd.n_rows, cd.log_w, [](int, int, const float*, uint32_t) {});
-            for (int r = 0; r < kGroupRows; ++r) {
-                const long long e = g * kGroupRows + r;
-                if (e < cd.n_rows) plain += ((cd.meta[e] & (int)kMetaLenMask) + kUnroll - 1) / kUnroll * kUnroll;
-            }
-        }
-        if (cd.m_out) cd.m_out[g] = m;
-    }
+// One atomic per wavefront and counter: [0] sum of m, [1] sum of plain, [2] largest m.
+__device__ __forceinline__ void add_rowgroup_counters(int m, int plain, unsigned long long* __restrict__ c) {
     int sm = m, sp = plain, mx = m;
     for (int d = 32; d > 0; d >>= 1) {
         sm += __shfl_xor(sm, d);
@@ -701,11 +680,28 @@ rowgroup_count_kernel(const RowGroupCand* __restrict__ cands, unsigned long long
         mx = max(mx, __shfl_xor(mx, d));
     }
     if ((threadIdx.x & 63) == 0 && sp > 0) {
-        unsigned long long* c = counters + 3 * blockIdx.y;
         atomicAdd(&c[0], (unsigned long long)sm);
         atomicAdd(&c[1], (unsigned long long)sp);
         atomicMax(&c[2], (unsigned long long)mx);
     }
+}
+
+// counters[3 * i + ...] of bucket i = blockIdx.y: merged entries, gathers of the plain path (row
+// lengths rounded up to the unroll), longest group.
+__global__ void __launch_bounds__(256)
+rowgroup_count_kernel(const RowGroupCand* __restrict__ cands, unsigned long long* __restrict__ counters) {
+    const RowGroupCand cd = cands[blockIdx.y];
+    const long long g = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+    int m = 0, plain = 0;
+    if (g < cd.n_groups) {
+        m = merge_group<false>(cd.cols, nullptr, cd.meta, g, cd.n_rows, cd.log_w, [](int, int, const float*, uint32_t) {});
+        for (int r = 0; r < kGroupRows; ++r) {
+            const long long e = g * kGroupRows + r;
+            if (e < cd.n_rows) plain += ((cd.meta[e] & (int)kMetaLenMask) + kUnroll - 1) / kUnroll * kUnroll;
+        }
+        cd.m_out[g] = m;
+    }
+    add_rowgroup_counters(m, plain, counters + 3 * blockIdx.y);
 }
 
 __global__ void __launch_bounds__(256)
@@ -932,63 +928,6 @@ derive_meta_kernel(const int32_t* __restrict__ rows, const float* __restrict__ v
     meta[e] = (int32_t)((uint32_t)len | (field << kMetaLenBits) | cont);
 }
 
-// Checks what the SpMM kernels take on trust from a bucket: source rows inside the matrix,
-// column indices inside B, 1..W valid slots per ELL row, and segments (a head that announces
-// n ELL rows followed by continuation rows 1..n-1 with the same row id) that are complete
-// and stay inside the bucket.  flags[0] bad column, [1] bad row, [2] bad meta.
-__global__ void __launch_bounds__(256)
-validate_bucket_kernel(const int32_t* __restrict__ rows, const int32_t* __restrict__ meta,
-                       const int32_t* __restrict__ cols, long long n_rows, int log_w,
-                       long long num_rows, long long num_cols, int* __restrict__ flags) {
-    const long long stride = (long long)gridDim.x * blockDim.x;
-    const long long t0 = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    bool bad_col = false, bad_row = false, bad_meta = false;
-    const long long n_slots = n_rows << log_w;
-    for (long long i = t0 * 4; i < n_slots; i += stride * 4) {
-        if (i + 4 <= n_slots) {
-            const int4 c = *reinterpret_cast<const int4*>(cols + i);
-            bad_col |= (unsigned)c.x >= (unsigned long long)num_cols || (unsigned)c.y >= (unsigned long long)num_cols ||
-                       (unsigned)c.z >= (unsigned long long)num_cols || (unsigned)c.w >= (unsigned long long)num_cols;
-        } else {
-            for (long long k = i; k < n_slots; ++k) bad_col |= (unsigned)cols[k] >= (unsigned long long)num_cols;
-        }
-    }
-    for (long long e = t0; e < n_rows; e += stride) {
-        bad_row |= (unsigned)rows[e] >= (unsigned long long)num_rows;
-        const int m = meta[e];
-        const int len = m & (int)kMetaLenMask;
-        bad_meta |= len < 1 || len > (1 << log_w);
-        const long long field = (long long)(((uint32_t)m & 0x7FFFFFFFu) >> kMetaLenBits);
-        // what the next ELL row must be: a continuation row with index `want`, or a head (0)
-        long long want = 0;
-        if (m >= 0) {
-            bad_meta |= field < 1 || e + field > n_rows;
-            want = field > 1 ? 1 : 0;
-        } else {
-            const long long h = e - field;
-            if (field < 1 || h < 0) {
-                bad_meta = true;
-            } else {
-                const int hm = meta[h];
-                const long long n = (long long)((uint32_t)hm >> kMetaLenBits);
-                bad_meta |= hm < 0 || field >= n || rows[h] != rows[e];
-                want = field + 1 < n ? field + 1 : 0;
-            }
-        }
-        if (e == 0) bad_meta |= m < 0;
-        if (e + 1 < n_rows) {
-            const int nm = meta[e + 1];
-            const long long nf = (long long)(((uint32_t)nm & 0x7FFFFFFFu) >> kMetaLenBits);
-            bad_meta |= want == 0 ? nm < 0 : (nm >= 0 || nf != want);
-        } else {
-            bad_meta |= want != 0;
-        }
-    }
-    if (__ballot(bad_col) != 0 && (threadIdx.x & 63) == 0) flags[0] = 1;
-    if (__ballot(bad_row) != 0 && (threadIdx.x & 63) == 0) flags[1] = 1;
-    if (__ballot(bad_meta) != 0 && (threadIdx.x & 63) == 0) flags[2] = 1;
-}
-
 // One ELL row as the chunk planner sees it.
 struct ChunkedRow {
     long long total;     // slots of its segment
@@ -1022,17 +961,158 @@ __device__ __forceinline__ ChunkedRow chunked_row(const int32_t* __restrict__ me
     return x;
 }
 
-// Finds the source rows of a bucket that take the cooperative path (more than kCoopSlots
-// slots) and cuts them into chunks.  Runs twice: with chunks == nullptr it only counts
-// (counters[0] chunks, [1] rows with several chunks, [2] their partial rows, [3] "the bucket
-// has rows spanning several ELL rows"); the second run fills the tables, taking ranges with
-// the same counters.  Table order depends on scheduling, results do not: every row's
-// partials are private and are summed in chunk order.
-// A workgroup owns a contiguous range of ELL rows and takes its ranges of the tables with one
-// atomic per counter: a sweep over its rows counts, a second one fills.  With one atomic per
-// wavefront and counter - and one on counters[3] for every wavefront that holds part of a split
-// row - the widest bucket of a folded 2.45M-row graph (850K ELL rows) took 1.35 ms for the two
-// passes, all of it updates of one cache line; this form takes 0.07.
+// One bucket as the plan-time kernels see it.
+struct PlanBucket {
+    const int32_t* rows;
+    const int32_t* meta;
+    const int32_t* cols;
+    long long n_rows;
+    int log_w;
+    int part;
+    int n_blocks;              // workgroups of plan_scan_kernel
+    int sample_stride;         // row-group sampling: every sample_stride-th group is looked at (0: no candidate)
+};
+
+// One pass over all buckets of a plan:
+//   * checks what the SpMM kernels take on trust: source rows inside the matrix, column indices
+//     inside B, 1..W valid slots per ELL row, and segments (a head that announces n ELL rows followed
+//     by continuation rows 1..n-1 with the same row id) that are complete and stay inside the
+//     bucket.  flags[0] bad column, [1] bad row, [2] bad meta;
+//   * counts the chunks of rows that take the cooperative path: counters[(4 k + i) * kCounterLine]
+//     of bucket k = chunks, rows with several chunks, their partial rows, ChunkedRow::found of all rows;
+//   * marks the rows that partition 0 writes.
+// Bound by the stream of the column slabs.  Workgroup -> bucket by the first workgroups of the
+// buckets, so that all of them share one launch however many there are: three launches per bucket
+// (checks, counts, marks) were 60 us of GPU time for the 11 buckets of a 170K-row graph, whose slabs
+// take 3 us to read, and each read the row ids or the meta words again.
+constexpr int kScanSlotsPerBlock = 16384;
+constexpr int kScanMaxBlocks = 1024;       // per bucket: more only queue up at its counters
+constexpr int kScanUnroll = 4;             // 16-byte loads of columns in flight per thread
+constexpr int kCounterLine = 32;           // words between the counters of a bucket: each has a 128-byte line of its
+                                           // own, as atomics on one line are taken one after the other (17 ns each)
+__global__ void __launch_bounds__(256)
+plan_scan_kernel(const PlanBucket* __restrict__ buckets, const int32_t* __restrict__ first_block, int n_buckets,
+                 long long num_rows, long long num_cols, int chunk_slots, long long dense_min_slots,
+                 int* __restrict__ counters, int* __restrict__ flags, uint8_t* __restrict__ covered) {
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    int k = -1;                                       // last bucket whose first workgroup is not behind this one
+    for (int i = 0; i < n_buckets; i += 64)
+        k += __popcll(__ballot(i + lane < n_buckets && first_block[i + lane] <= (int)blockIdx.x));
+    k = __builtin_amdgcn_readfirstlane(k);
+    const PlanBucket bk = buckets[k];
+    const long long stride = (long long)bk.n_blocks * 256;
+    const long long t0 = ((long long)blockIdx.x - first_block[k]) * 256 + threadIdx.x;
+    const int32_t *rows = bk.rows, *meta = bk.meta;
+    const int log_w = bk.log_w;
+    const long long n_rows = bk.n_rows;
+    bool bad_col = false, bad_row = false, bad_meta = false;
+    const long long n_slots = n_rows << log_w;
+    const unsigned limit = (unsigned)num_cols;               // < 2^31
+    for (long long i = t0 * 4; i < n_slots; i += stride * 4 * kScanUnroll) {
+        int4 c[kScanUnroll];
+#pragma unroll
+        for (int u = 0; u < kScanUnroll; ++u) {
+            const long long j = i + u * stride * 4;
+            c[u] = make_int4(0, 0, 0, 0);
+            if (j + 4 <= n_slots) c[u] = *reinterpret_cast<const int4*>(bk.cols + j);
+            else if (j < n_slots)
+                for (long long q = j; q < n_slots; ++q) bad_col |= (unsigned)bk.cols[q] >= limit;
+        }
+#pragma unroll
+        for (int u = 0; u < kScanUnroll; ++u)
+            bad_col |= (unsigned)c[u].x >= limit || (unsigned)c[u].y >= limit || (unsigned)c[u].z >= limit || (unsigned)c[u].w >= limit;
+    }
+    int sum[3] = {0, 0, 0}, found = 0;
+    for (long long e = t0; e < n_rows; e += stride) {
+        const int row = rows[e];
+        const bool row_ok = (unsigned)row < (unsigned long long)num_rows;
+        bad_row |= !row_ok;
+        if (bk.part == 0 && row_ok) covered[row] = 1;
+        const int m = meta[e];
+        const int len = m & (int)kMetaLenMask;
+        bad_meta |= len < 1 || len > (1 << log_w);
+        const long long field = (long long)(((uint32_t)m & 0x7FFFFFFFu) >> kMetaLenBits);
+        // what the next ELL row must be: a continuation row with index `want`, or a head (0)
+        long long want = 0;
+        if (m >= 0) {
+            bad_meta |= field < 1 || e + field > n_rows;
+            want = field > 1 ? 1 : 0;
+        } else {
+            const long long h = e - field;
+            if (field < 1 || h < 0) {
+                bad_meta = true;
+            } else {
+                const int hm = meta[h];
+                const long long n = (long long)((uint32_t)hm >> kMetaLenBits);
+                bad_meta |= hm < 0 || field >= n || rows[h] != row;
+                want = field + 1 < n ? field + 1 : 0;
+            }
+        }
+        if (e == 0) bad_meta |= m < 0;
+        if (e + 1 < n_rows) {
+            const int nm = meta[e + 1];
+            const long long nf = (long long)(((uint32_t)nm & 0x7FFFFFFFu) >> kMetaLenBits);
+            bad_meta |= want == 0 ? nm < 0 : (nm >= 0 || nf != want);
+        } else {
+            bad_meta |= want != 0;
+        }
+        const ChunkedRow x = chunked_row(meta, e, n_rows, log_w, chunk_slots, dense_min_slots);
+        found |= x.found;
+        sum[0] += x.n_chunks;
+        sum[1] += x.n_chunks > 1;
+        sum[2] += x.n_chunks > 1 ? x.n_chunks : 0;
+    }
+    if (__ballot(bad_col) != 0 && lane == 0) flags[0] = 1;
+    if (__ballot(bad_row) != 0 && lane == 0) flags[1] = 1;
+    if (__ballot(bad_meta) != 0 && lane == 0) flags[2] = 1;
+    // one atomic per workgroup and counter
+    __shared__ int s_sum[4][4];
+    for (int d = 32; d > 0; d >>= 1) {
+        found |= __shfl_xor(found, d);
+        for (int i = 0; i < 3; ++i) sum[i] += __shfl_xor(sum[i], d);
+    }
+    if (lane == 0) {
+        for (int i = 0; i < 3; ++i) s_sum[wave][i] = sum[i];
+        s_sum[wave][3] = found;
+    }
+    __syncthreads();
+    int* mine = counters + (size_t)(4 * k + (int)(threadIdx.x & 3)) * kCounterLine;
+    if (threadIdx.x < 3) {
+        const int all = s_sum[0][threadIdx.x] + s_sum[1][threadIdx.x] + s_sum[2][threadIdx.x] + s_sum[3][threadIdx.x];
+        if (all) atomicAdd(mine, all);
+    } else if (threadIdx.x == 3) {
+        const int all = s_sum[0][3] | s_sum[1][3] | s_sum[2][3] | s_sum[3][3];
+        // what the shared word holds already need not be added again
+        if ((all & ~__hip_atomic_load(mine, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) != 0) atomicOr(mine, all);
+    }
+}
+
+// Every sample_stride-th group of four rows of the candidate buckets (blockIdx.y: all buckets of the
+// plan): counters[3 k ..] = merged entries among the first kRowGroupSampleEntries of a group, the
+// slots they consumed, the largest count.  Enqueued behind plan_scan_kernel, before its verdict has
+// been read: where a check failed nothing is followed through the slabs.
+__global__ void __launch_bounds__(256)
+rowgroup_sample_kernel(const PlanBucket* __restrict__ buckets, const int* __restrict__ flags,
+                       unsigned long long* __restrict__ counters) {
+    if (flags[0] | flags[1] | flags[2] | flags[3]) return;
+    const PlanBucket& bk = buckets[blockIdx.y];
+    if (bk.sample_stride == 0) return;
+    const long long g = ((long long)blockIdx.x * blockDim.x + threadIdx.x) * bk.sample_stride;
+    int m = 0, plain = 0;
+    if (g * kGroupRows < bk.n_rows)
+        m = merge_group<false>(bk.cols, nullptr, bk.meta, g, bk.n_rows, bk.log_w,
+                               [](int, int, const float*, uint32_t) {}, kRowGroupSampleEntries, &plain);
+    add_rowgroup_counters(m, plain, counters + 3 * blockIdx.y);
+}
+
+// Fills the chunk table of a bucket (rows of more than kCoopSlots slots, cut into chunks) and its
+// part of the heavy-row table.  counters (kCounterLine words apart): chunks, rows with several chunks
+// and their partial rows handed out so far.  Table order depends on scheduling, results do not: every row's partials are
+// private and are summed in chunk order.
+// A workgroup owns a contiguous range of ELL rows and takes its ranges of the tables with one atomic
+// per counter: a sweep over its rows counts, a second one fills.  With one atomic per wavefront and
+// counter, counting and filling the widest bucket of a folded 2.45M-row graph (850K ELL rows)
+// took 1.35 ms, all of it updates of one cache line; now the filling pass takes 0.04.
 constexpr int kPlanChunksGrid = 512;
 __global__ void __launch_bounds__(256)
 plan_chunks_kernel(const int32_t* __restrict__ rows, const int32_t* __restrict__ meta,
@@ -1045,30 +1125,23 @@ plan_chunks_kernel(const int32_t* __restrict__ rows, const int32_t* __restrict__
     const long long per_wave = ((n_rows + (long long)gridDim.x * 4 - 1) / ((long long)gridDim.x * 4) + 63) / 64 * 64;
     const long long lo = ((long long)blockIdx.x * 4 + wave) * per_wave;
     const long long hi = min(lo + per_wave, n_rows);
-    int sum[3] = {0, 0, 0}, found = 0;
+    int sum[3] = {0, 0, 0};
     for (long long e = lo + lane; e < hi; e += 64) {
         const ChunkedRow x = chunked_row(meta, e, n_rows, log_w, chunk_slots, dense_min_slots);
-        found |= x.found;
         sum[0] += x.n_chunks;
         sum[1] += x.n_chunks > 1;
         sum[2] += x.n_chunks > 1 ? x.n_chunks : 0;
     }
     for (int d = 32; d > 0; d >>= 1) {
-        found |= __shfl_xor(found, d);
         for (int i = 0; i < 3; ++i) sum[i] += __shfl_xor(sum[i], d);
     }
-    if (lane == 0) {
-        // what the shared word holds already need not be added again
-        if ((found & ~__hip_atomic_load(&counters[3], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) != 0)
-            atomicOr(&counters[3], found);
+    if (lane == 0)
         for (int i = 0; i < 3; ++i) s_sum[wave][i] = sum[i];
-    }
     __syncthreads();
     if (threadIdx.x < 3) {
         const int all = s_sum[0][threadIdx.x] + s_sum[1][threadIdx.x] + s_sum[2][threadIdx.x] + s_sum[3][threadIdx.x];
-        s_base[threadIdx.x] = all ? atomicAdd(&counters[threadIdx.x], all) : 0;
+        s_base[threadIdx.x] = all ? atomicAdd(&counters[threadIdx.x * kCounterLine], all) : 0;
     }
-    if (chunks == nullptr) return;
     __syncthreads();
     int at[3];
     for (int i = 0; i < 3; ++i) {
@@ -1108,11 +1181,6 @@ plan_chunks_kernel(const int32_t* __restrict__ rows, const int32_t* __restrict__
         }
         if (several) heavy[heavy_base + h] = HeavyRow{row, partial_base + p0, x.n_chunks, 0};
     }
-}
-
-__global__ void mark_rows_kernel(const int32_t* __restrict__ rows, long long n, uint8_t* __restrict__ covered) {
-    const long long e = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (e < n) covered[rows[e]] = 1;
 }
 
 // Rows that no bucket of partition 0 writes: counted (list == nullptr) or listed.  Each
@@ -1325,6 +1393,7 @@ int lf_spmm_create(lf_spmm_plan** out_plan, const lf_bucket_desc* h_buckets, int
     plan->ch = ch;
     auto bail = [&](int rc) {
         std::string keep = lf::last_error();
+        (void)hipStreamSynchronize(s);       // nothing enqueued may outlive the scratch and the read-back buffers
         lf_spmm_destroy(plan);
         lf::last_error() = keep;
         return rc;
@@ -1346,29 +1415,13 @@ int lf_spmm_create(lf_spmm_plan** out_plan, const lf_bucket_desc* h_buckets, int
     LF_TRY_HIP(hipGetDeviceProperties(&prop, plan->device));
     plan->num_cus = prop.multiProcessorCount;
 
-    // ---- meta: derive where missing; count the chunks of rows that take the cooperative path.
-    // Every bucket has its own four counters (plus one set for the rows to clear), so that
-    // the counting pass, the filling pass and the coverage pass each cost one copy back and
-    // one synchronisation for the whole plan, not one per bucket.
+    // ---- meta: derive where missing; check the slabs; count the chunks of rows that take the
+    // cooperative path; find the rows that nothing writes; sample the row-group candidates.  All of it
+    // is enqueued together and read back with one copy and one synchronisation.
     std::vector<const int32_t*> meta((size_t)num_buckets, nullptr);
-    const int n_counters = 4 * (num_buckets + 2);
-    int* d_counters = nullptr;              // [4k .. 4k+3]: plan_chunks_kernel's counters of bucket k
-    LF_TRY(dev_alloc(plan, &d_counters, (size_t)n_counters, true));
-    int* d_zero_count = d_counters + 4 * num_buckets;
-    int* d_flags = d_counters + 4 * (num_buckets + 1);   // validate_bucket_kernel, derive_meta_kernel
-    std::vector<int> h_counters((size_t)n_counters, 0);
-    std::vector<int> is_multi((size_t)num_buckets, 0), has_dense((size_t)num_buckets, 0), has_wide((size_t)num_buckets, 0);
     struct ChunkCount { int chunks = 0, heavy = 0, partials = 0; };
     std::vector<ChunkCount> counts((size_t)num_buckets);
-    auto clear_counters = [&]() {
-        fill_bytes_kernel<<<1, 64, 0, s>>>((uint32_t*)d_counters, n_counters, 0u);
-        return hipGetLastError();
-    };
-    auto read_counters = [&]() {
-        hipError_t e = hipMemcpyAsync(h_counters.data(), d_counters, (size_t)n_counters * 4, hipMemcpyDeviceToHost, s);
-        if (e == hipSuccess) e = hipStreamSynchronize(s);
-        return e;
-    };
+    std::vector<int> is_multi((size_t)num_buckets, 0), has_dense((size_t)num_buckets, 0), has_wide((size_t)num_buckets, 0);
     // Chunk size of the rows that a whole workgroup reduces.  Small matrices want many short
     // chunks (a 170k-row graph: 0.076 ms with 2048-slot chunks, 0.112 ms with 8192), large ones
     // fewer partial rows and a shorter second kernel (500k x 2M with 50 rows of 100k entries:
@@ -1388,22 +1441,49 @@ int lf_spmm_create(lf_spmm_plan** out_plan, const lf_bucket_desc* h_buckets, int
     const long long dense_min_slots = (env_dense && env_dense[0] == '0') || b_is_cached
                                           ? (1ll << 62)
                                           : std::max<long long>(kDenseRowMinSlots, cols_p / kDenseRowShare);
-    auto launch_plan_chunks = [&](int k, Chunk* out, HeavyRow* hout, int partial_base, int heavy_base) {
-        const lf_bucket_desc& b = h_buckets[k];
-        const int grid = (int)std::min<long long>((b.num_ell_rows + 255) / 256, kPlanChunksGrid);
-        plan_chunks_kernel<<<grid, 256, 0, s>>>(b.d_rows, meta[k], b.d_cols, b.num_ell_rows, lf::ilog2(b.width),
-                                                d_counters + 4 * k, out, hout, partial_base, heavy_base, chunk_slots,
-                                                dense_min_slots);
-        return hipGetLastError();
+
+    // Scratch: the words that are read back (chunk counters and fill cursors of every bucket, sampling
+    // counters, flags), then the coverage bytes - cleared by one launch - then the bucket table.
+    const size_t nb_s = (size_t)num_buckets;
+    const size_t o_counters = 0, o_cursors = o_counters + nb_s * 4 * kCounterLine * 4, o_flags = o_cursors + nb_s * 4 * kCounterLine * 4;
+    const size_t o_zero = o_flags + 16, o_sample = o_zero + 16, back_bytes = o_sample + nb_s * 24;
+    const size_t o_covered = (back_bytes + 255) / 256 * 256;
+    const size_t o_table = (o_covered + (size_t)num_rows + 255) / 256 * 256;
+    const size_t table_bytes = nb_s * (sizeof(PlanBucket) + 4);
+    char* d_scratch = nullptr;
+    LF_TRY(dev_alloc(plan, &d_scratch, o_table + std::max<size_t>(table_bytes, 16), true));
+    int* d_counters = (int*)(d_scratch + o_counters);
+    int* d_cursors = (int*)(d_scratch + o_cursors);
+    int* d_flags = (int*)(d_scratch + o_flags);          // bad column, bad row, bad meta; derive_meta_kernel
+    int* d_zero_count = (int*)(d_scratch + o_zero);      // rows to clear; listed so far
+    unsigned long long* d_sample = (unsigned long long*)(d_scratch + o_sample);
+    uint8_t* d_cov = (uint8_t*)(d_scratch + o_covered);
+    lf::PinnedLoan back(back_bytes);
+    lf::PinnedLoan table(table_bytes);
+    if (!back.ok() || !table.ok()) return bail(lf::fail(LF_ERR_HIP, "out of host memory"));
+    const int* h_counters = back.as<int>(o_counters);
+    auto read_back = [&]() {
+        hipError_t e = hipMemcpyAsync(back.as<char>(), d_scratch, back_bytes, hipMemcpyDeviceToHost, s);
+        if (e == hipSuccess) e = hipStreamSynchronize(s);
+        return e;
     };
-    LF_TRY_HIP(clear_counters());
+    {
+        const long long words = (long long)(o_table / 4);
+        fill_bytes_kernel<<<(int)std::min<long long>((words + 255) / 256, 4096), 256, 0, s>>>((uint32_t*)d_scratch, words, 0u);
+        LF_TRY_HIP(hipGetLastError());
+    }
+    const char* env_groups = getenv("LF_ROW_GROUPS");
+    std::vector<int> cand;                                 // buckets that may be rewritten as row groups or cells
+    PlanBucket* h_table = table.as<PlanBucket>();
+    int32_t* h_first = table.as<int32_t>(nb_s * sizeof(PlanBucket));
+    const PlanBucket* d_table = (const PlanBucket*)(d_scratch + o_table);
+    const int32_t* d_first = (const int32_t*)(d_scratch + o_table + nb_s * sizeof(PlanBucket));
+    int scan_blocks = 0;
+    long long most_samples = 0;
     for (int k = 0; k < num_buckets; ++k) {
         const lf_bucket_desc& b = h_buckets[k];
-        if (b.num_ell_rows == 0) continue;
         const int log_w = lf::ilog2(b.width);
-        if (b.d_meta) {
-            meta[k] = b.d_meta;
-        } else {
+        if (b.num_ell_rows > 0 && !b.d_meta) {
             int32_t *m = nullptr, *blk_first = nullptr, *blk_last = nullptr;
             const int n_blocks = (int)((b.num_ell_rows + 255) / 256);
             LF_TRY(dev_alloc(plan, &m, (size_t)b.num_ell_rows));
@@ -1415,21 +1495,49 @@ int lf_spmm_create(lf_spmm_plan** out_plan, const lf_bucket_desc* h_buckets, int
                                                         blk_last, n_blocks, m, d_flags);
             LF_TRY_HIP(hipGetLastError());
             meta[k] = m;
+        } else if (b.num_ell_rows > 0) {
+            meta[k] = b.d_meta;
         }
-        {
-            const long long units = std::max<long long>(b.num_ell_rows, ((long long)b.num_ell_rows << log_w) / 4);
-            const int vgrid = (int)std::min<long long>(lf::ceil_div(units, 256), 4096);
-            validate_bucket_kernel<<<vgrid, 256, 0, s>>>(b.d_rows, meta[k], b.d_cols, b.num_ell_rows, log_w,
-                                                         num_rows, num_cols, d_flags);
-            LF_TRY_HIP(hipGetLastError());
+        PlanBucket& t = h_table[k];
+        t.rows = b.d_rows;
+        t.meta = meta[k];
+        t.cols = b.d_cols;
+        t.n_rows = b.num_ell_rows;
+        t.log_w = log_w;
+        t.part = b.part;
+        const long long units = std::max<long long>(lf::ceil_div(b.num_ell_rows, 1024),
+                                                    lf::ceil_div((long long)b.num_ell_rows << log_w, kScanSlotsPerBlock));
+        t.n_blocks = (int)std::min<long long>(units, kScanMaxBlocks);
+        h_first[k] = scan_blocks;
+        scan_blocks += t.n_blocks;
+        t.sample_stride = 0;
+        if (ch == 1 && !(env_groups && env_groups[0] == '0') && b.num_ell_rows >= kRowGroupMinRows && b.width >= kUnroll && b.width <= 64) {
+            const long long n_groups = lf::ceil_div(b.num_ell_rows, kGroupRows);
+            t.sample_stride = (int)std::max<long long>(1, n_groups / kRowGroupSample);
+            most_samples = std::max<long long>(most_samples, lf::ceil_div(n_groups, t.sample_stride));
+            cand.push_back(k);
         }
-        LF_TRY_HIP(launch_plan_chunks(k, nullptr, nullptr, 0, 0));
     }
-    LF_TRY_HIP(read_counters());
+    if (num_buckets > 0) LF_TRY_HIP(hipMemcpyAsync(d_scratch + o_table, h_table, table_bytes, hipMemcpyHostToDevice, s));
+    if (scan_blocks > 0) {
+        plan_scan_kernel<<<scan_blocks, 256, 0, s>>>(d_table, d_first, num_buckets, num_rows, num_cols, chunk_slots,
+                                                     dense_min_slots, d_counters, d_flags, d_cov);
+        LF_TRY_HIP(hipGetLastError());
+    }
+    const int rgrid = (int)std::min<int64_t>((num_rows + 255) / 256, 1024);
+    if (num_rows > 0) {
+        collect_uncovered_kernel<<<rgrid, 256, 0, s>>>(d_cov, num_rows, d_zero_count, nullptr);
+        LF_TRY_HIP(hipGetLastError());
+    }
+    if (!cand.empty()) {
+        rowgroup_sample_kernel<<<dim3((unsigned)lf::ceil_div(most_samples, 256), (unsigned)num_buckets), 256, 0, s>>>(d_table, d_flags, d_sample);
+        LF_TRY_HIP(hipGetLastError());
+    }
+    LF_TRY_HIP(read_back());
     {
         // nothing below (and no SpMM launch) may run on slabs that fail these checks: a column
         // or row index out of range would be an out-of-range gather or store
-        const int* f = &h_counters[4 * (num_buckets + 1)];
+        const int* f = back.as<int>(o_flags);
         if (f[0]) return bail(lf::fail(LF_ERR_INVALID, "a bucket holds a column index outside [0, %lld)", (long long)num_cols));
         if (f[1]) return bail(lf::fail(LF_ERR_INVALID, "a bucket holds a row index outside [0, %lld)", (long long)num_rows));
         if (f[2]) return bail(lf::fail(LF_ERR_INVALID, "a bucket's meta array is inconsistent (valid slots outside 1..W, "
@@ -1437,12 +1545,20 @@ int lf_spmm_create(lf_spmm_plan** out_plan, const lf_bucket_desc* h_buckets, int
         if (f[3]) return bail(lf::fail(LF_ERR_UNSUPPORTED, "a row is split over more than %d ELL rows", (1 << (31 - kMetaLenBits)) - 1));
     }
     for (int k = 0; k < num_buckets; ++k) {
-        counts[k].chunks = h_counters[4 * k + 0];
-        counts[k].heavy = h_counters[4 * k + 1];
-        counts[k].partials = h_counters[4 * k + 2];
-        is_multi[k] = h_counters[4 * k + 3] & 1;
-        has_dense[k] = (h_counters[4 * k + 3] >> 1) & 1;
-        has_wide[k] = (h_counters[4 * k + 3] >> 2) & 1;
+        const int* c = h_counters + (size_t)4 * k * kCounterLine;
+        counts[k].chunks = c[0];
+        counts[k].heavy = c[kCounterLine];
+        counts[k].partials = c[2 * kCounterLine];
+        const int found = c[3 * kCounterLine];
+        is_multi[k] = found & 1;
+        has_dense[k] = (found >> 1) & 1;
+        has_wide[k] = (found >> 2) & 1;
+    }
+    const int n_zero = *back.as<int>(o_zero);
+    std::vector<int> chosen;                               // candidates whose sample shows shared columns
+    for (int k : cand) {
+        const unsigned long long* c = back.as<unsigned long long>(o_sample) + 3 * k;
+        if (!is_multi[k] && c[1] > 0 && c[0] * 100 <= c[1] * kRowGroupMaxPercent) chosen.push_back(k);
     }
 
     // ---- chunk tables, heavy-row table (grouped by bucket, hence by partition) and partial rows
@@ -1462,63 +1578,40 @@ int lf_spmm_create(lf_spmm_plan** out_plan, const lf_bucket_desc* h_buckets, int
     }
     Chunk* d_chunks_all = nullptr;
     LF_TRY(dev_alloc(plan, &d_chunks_all, (size_t)chunk_base[num_buckets]));
-    LF_TRY_HIP(clear_counters());
     for (int k = 0; k < num_buckets; ++k) {
         if (counts[k].chunks == 0) continue;
+        const lf_bucket_desc& b = h_buckets[k];
         d_chunks[k] = d_chunks_all + chunk_base[k];
-        LF_TRY_HIP(launch_plan_chunks(k, d_chunks[k], plan->d_heavy, partial_base[k], heavy_base[k]));
+        const int grid = (int)std::min<long long>((b.num_ell_rows + 255) / 256, kPlanChunksGrid);
+        plan_chunks_kernel<<<grid, 256, 0, s>>>(b.d_rows, meta[k], b.d_cols, b.num_ell_rows, lf::ilog2(b.width), d_cursors + (size_t)4 * k * kCounterLine,
+                                                d_chunks[k], plan->d_heavy, partial_base[k], heavy_base[k], chunk_slots,
+                                                dense_min_slots);
+        LF_TRY_HIP(hipGetLastError());
+    }
+    for (int k = 0; k < num_buckets; ++k) {
+        if (!has_dense[k] || counts[k].chunks == 0) continue;
+        // The chunks of dense rows go behind the others, in column order (ties: by row, so
+        // the order is the same in every plan): some thousands of records, sorted on the host.
+        std::vector<Chunk> h_chunks((size_t)counts[k].chunks);
+        LF_TRY_HIP(hipMemcpyAsync(h_chunks.data(), d_chunks[k], h_chunks.size() * sizeof(Chunk), hipMemcpyDeviceToHost, s));
+        LF_TRY_HIP(hipStreamSynchronize(s));
+        const auto mid = std::stable_partition(h_chunks.begin(), h_chunks.end(),
+                                               [](const Chunk& x) { return (x.n_slots & kChunkDenseBit) == 0; });
+        std::sort(mid, h_chunks.end(), [](const Chunk& x, const Chunk& y) {
+            if (x.first_col != y.first_col) return x.first_col < y.first_col;
+            if (x.row != y.row) return x.row < y.row;
+            return x.slot_begin < y.slot_begin;
+        });
+        for (auto it = mid; it != h_chunks.end(); ++it) it->n_slots &= ~kChunkDenseBit;
+        LF_TRY_HIP(hipMemcpyAsync(d_chunks[k], h_chunks.data(), h_chunks.size() * sizeof(Chunk), hipMemcpyHostToDevice, s));
+        LF_TRY_HIP(hipStreamSynchronize(s));
     }
 
     // ---- rows that partition 0 does not write are cleared by its launch
     int32_t* d_zero_rows = nullptr;
-    int n_zero = 0;
-    uint8_t* d_cov = nullptr;
-    const int rgrid = (int)std::min<int64_t>((num_rows + 255) / 256, 1024);
-    if (num_rows > 0) {
-        const size_t cov_words = ((size_t)num_rows + 3) / 4;
-        uint32_t* cov = nullptr;
-        LF_TRY(dev_alloc(plan, &cov, cov_words, true));
-        d_cov = (uint8_t*)cov;
-        fill_bytes_kernel<<<(int)std::min<size_t>((cov_words + 255) / 256, 4096), 256, 0, s>>>(cov, (long long)cov_words, 0u);
-        LF_TRY_HIP(hipGetLastError());
-        for (int k = 0; k < num_buckets; ++k) {
-            const lf_bucket_desc& b = h_buckets[k];
-            if (b.part != 0 || b.num_ell_rows == 0) continue;
-            mark_rows_kernel<<<(int)((b.num_ell_rows + 255) / 256), 256, 0, s>>>(b.d_rows, b.num_ell_rows, d_cov);
-            LF_TRY_HIP(hipGetLastError());
-        }
-        collect_uncovered_kernel<<<rgrid, 256, 0, s>>>(d_cov, num_rows, d_zero_count, nullptr);
-        LF_TRY_HIP(hipGetLastError());
-    }
-    LF_TRY_HIP(read_counters());             // the filling pass must have taken the same ranges
-    for (int k = 0; k < num_buckets; ++k) {
-        if (counts[k].chunks == 0) continue;
-        if (h_counters[4 * k] != counts[k].chunks || h_counters[4 * k + 1] != counts[k].heavy ||
-            h_counters[4 * k + 2] != counts[k].partials)
-            return bail(lf::fail(LF_ERR_INVALID, "bucket %d changed while the plan was being built", k));
-        if (has_dense[k]) {
-            // The chunks of dense rows go behind the others, in column order (ties: by row, so
-            // the order is the same in every plan): some thousands of records, sorted on the host.
-            std::vector<Chunk> h_chunks((size_t)counts[k].chunks);
-            LF_TRY_HIP(hipMemcpyAsync(h_chunks.data(), d_chunks[k], h_chunks.size() * sizeof(Chunk), hipMemcpyDeviceToHost, s));
-            LF_TRY_HIP(hipStreamSynchronize(s));
-            const auto mid = std::stable_partition(h_chunks.begin(), h_chunks.end(),
-                                                   [](const Chunk& x) { return (x.n_slots & kChunkDenseBit) == 0; });
-            std::sort(mid, h_chunks.end(), [](const Chunk& x, const Chunk& y) {
-                if (x.first_col != y.first_col) return x.first_col < y.first_col;
-                if (x.row != y.row) return x.row < y.row;
-                return x.slot_begin < y.slot_begin;
-            });
-            for (auto it = mid; it != h_chunks.end(); ++it) it->n_slots &= ~kChunkDenseBit;
-            LF_TRY_HIP(hipMemcpyAsync(d_chunks[k], h_chunks.data(), h_chunks.size() * sizeof(Chunk), hipMemcpyHostToDevice, s));
-            LF_TRY_HIP(hipStreamSynchronize(s));
-        }
-    }
-    n_zero = h_counters[4 * num_buckets];
     if (n_zero > 0) {
         LF_TRY(dev_alloc(plan, &d_zero_rows, (size_t)n_zero));
-        fill_bytes_kernel<<<1, 64, 0, s>>>((uint32_t*)d_zero_count, 4, 0u);
-        collect_uncovered_kernel<<<rgrid, 256, 0, s>>>(d_cov, num_rows, d_zero_count, d_zero_rows);
+        collect_uncovered_kernel<<<rgrid, 256, 0, s>>>(d_cov, num_rows, d_zero_count + 1, d_zero_rows);
         LF_TRY_HIP(hipGetLastError());
     }
 
@@ -1528,16 +1621,13 @@ int lf_spmm_create(lf_spmm_plan** out_plan, const lf_bucket_desc* h_buckets, int
     std::vector<LfCellBucket> cells;                       // in bucket (hence partition) order
     std::vector<int> cell_of((size_t)num_buckets, -1);
     {
-        const char* env = getenv("LF_ROW_GROUPS");
-        std::vector<int> cand;
-        for (int k = 0; k < num_buckets && ch == 1 && !(env && env[0] == '0'); ++k) {
-            const lf_bucket_desc& b = h_buckets[k];
-            if (b.num_ell_rows >= kRowGroupMinRows && b.width >= kUnroll && b.width <= 64 && !is_multi[k]) cand.push_back(k);
-        }
-        unsigned long long* d_rg = nullptr;                // three counters per candidate
-        std::vector<unsigned long long> h_rg(cand.size() * 3, 0);
-        RowGroupCand* d_cands = nullptr;
-        auto count_pass = [&](const std::vector<int>& which, bool sample, std::vector<int32_t*>* m_arrays) -> int {
+        std::vector<unsigned long long> h_rg(chosen.size() * 3, 0);   // three counters per bucket
+        // merged lengths of all groups of the buckets `which`, and their totals
+        auto count_pass = [&](const std::vector<int>& which, const std::vector<int32_t*>& m_arrays) -> int {
+            unsigned long long* d_rg = nullptr;
+            RowGroupCand* d_cands = nullptr;
+            if (int rc = dev_alloc(plan, &d_rg, which.size() * 3, true)) return rc;
+            if (int rc = dev_alloc(plan, &d_cands, which.size(), true)) return rc;
             std::vector<RowGroupCand> h_cands(which.size());
             long long most = 1;
             for (size_t i = 0; i < which.size(); ++i) {
@@ -1547,12 +1637,11 @@ int lf_spmm_create(lf_spmm_plan** out_plan, const lf_bucket_desc* h_buckets, int
                 c.meta = meta[which[i]];
                 c.n_rows = b.num_ell_rows;
                 c.n_groups = lf::ceil_div(b.num_ell_rows, kGroupRows);
-                c.m_out = m_arrays ? (*m_arrays)[i] : nullptr;
+                c.m_out = m_arrays[i];
                 c.log_w = lf::ilog2(b.width);
-                c.stride = sample ? (int)std::max<long long>(1, c.n_groups / kRowGroupSample) : 1;
-                most = std::max<long long>(most, lf::ceil_div(c.n_groups, c.stride));
+                most = std::max<long long>(most, c.n_groups);
             }
-            fill_bytes_kernel<<<1, 64, 0, s>>>((uint32_t*)d_rg, (long long)cand.size() * 6, 0u);
+            fill_bytes_kernel<<<1, 64, 0, s>>>((uint32_t*)d_rg, (long long)which.size() * 6, 0u);
             LF_HIP(hipGetLastError());
             LF_HIP(hipMemcpyAsync(d_cands, h_cands.data(), h_cands.size() * sizeof(RowGroupCand), hipMemcpyHostToDevice, s));
             rowgroup_count_kernel<<<dim3((unsigned)lf::ceil_div(most, 256), (unsigned)which.size()), 256, 0, s>>>(d_cands, d_rg);
@@ -1561,20 +1650,14 @@ int lf_spmm_create(lf_spmm_plan** out_plan, const lf_bucket_desc* h_buckets, int
             LF_HIP(hipStreamSynchronize(s));               // also keeps h_cands alive until the copy is done
             return LF_OK;
         };
-        if (!cand.empty()) {
-            LF_TRY(dev_alloc(plan, &d_rg, cand.size() * 3, true));
-            LF_TRY(dev_alloc(plan, &d_cands, cand.size(), true));
-            LF_TRY(count_pass(cand, true, nullptr));       // a sample of the groups decides
-            std::vector<int> chosen;
-            for (size_t i = 0; i < cand.size(); ++i)
-                if (h_rg[3 * i + 1] > 0 && h_rg[3 * i] * 100 <= h_rg[3 * i + 1] * kRowGroupMaxPercent) chosen.push_back(cand[i]);
+        if (!chosen.empty()) {
             // fp32 B, one 16-byte load per lane and 32 or 64 lanes per row of B (128 or 256
             // features per pass): the chosen buckets are rewritten as cells of rows that are
             // neighbours in up to three directions where that structure is found, else four
             // consecutive rows at a time (as are all other operand shapes: the cells measured
             // slower there).
             const bool cells_fit = (feat_size == 256 || feat_size == 128) && b_dtype == LF_DTYPE_F32;
-            if (!chosen.empty() && cells_fit && !(env && env[0] == '4')) {
+            if (cells_fit && !(env_groups && env_groups[0] == '4')) {
                 std::vector<int> rest;
                 for (int k : chosen) {
                     LfCellBucket cb{};
@@ -1594,7 +1677,7 @@ int lf_spmm_create(lf_spmm_plan** out_plan, const lf_bucket_desc* h_buckets, int
                 std::vector<int32_t*> m_arrays(chosen.size(), nullptr);
                 for (size_t i = 0; i < chosen.size(); ++i)
                     LF_TRY(dev_alloc(plan, &m_arrays[i], (size_t)lf::ceil_div(h_buckets[chosen[i]].num_ell_rows, kGroupRows), true));
-                LF_TRY(count_pass(chosen, false, &m_arrays));
+                LF_TRY(count_pass(chosen, m_arrays));
                 for (size_t i = 0; i < chosen.size(); ++i) {
                     const int k = chosen[i];
                     const lf_bucket_desc& b = h_buckets[k];
@@ -1764,17 +1847,25 @@ int lf_spmm_create(lf_spmm_plan** out_plan, const lf_bucket_desc* h_buckets, int
         L.grid = (int)(longest * kXcds);
         total_tiles += L.tiles;
     }
-    if (!merged.empty()) {
-        LF_TRY(dev_alloc(plan, &plan->d_merged, merged.size()));
-        LF_TRY_HIP(hipMemcpy(plan->d_merged, merged.data(), merged.size() * sizeof(MergedBucket), hipMemcpyHostToDevice));
-    }
-    if (!cells.empty()) {
-        LF_TRY(dev_alloc(plan, &plan->d_cells, cells.size()));
-        LF_TRY_HIP(hipMemcpy(plan->d_cells, cells.data(), cells.size() * sizeof(LfCellBucket), hipMemcpyHostToDevice));
-    }
-    if (!groups.empty()) {
-        LF_TRY(dev_alloc(plan, &plan->d_groups, groups.size()));
-        LF_TRY_HIP(hipMemcpy(plan->d_groups, groups.data(), groups.size() * sizeof(Group), hipMemcpyHostToDevice));
+    // the tables go up together, in one allocation
+    const size_t o_merged = (groups.size() * sizeof(Group) + 255) / 256 * 256;
+    const size_t o_cells = (o_merged + merged.size() * sizeof(MergedBucket) + 255) / 256 * 256;
+    const size_t tables_bytes = o_cells + cells.size() * sizeof(LfCellBucket);
+    lf::PinnedLoan h_tables(tables_bytes);
+    if (!h_tables.ok()) return bail(lf::fail(LF_ERR_HIP, "out of host memory"));
+    if (tables_bytes > 0) {
+        char* d_tables = nullptr;
+        LF_TRY(dev_alloc(plan, &d_tables, tables_bytes));
+        auto put = [&](size_t at, const void* src, size_t bytes) {
+            if (bytes) std::memcpy(h_tables.as<char>(at), src, bytes);
+        };
+        put(0, groups.data(), groups.size() * sizeof(Group));
+        put(o_merged, merged.data(), merged.size() * sizeof(MergedBucket));
+        put(o_cells, cells.data(), cells.size() * sizeof(LfCellBucket));
+        LF_TRY_HIP(hipMemcpyAsync(d_tables, h_tables.as<char>(), tables_bytes, hipMemcpyHostToDevice, s));
+        plan->d_groups = (Group*)d_tables;
+        plan->d_merged = (MergedBucket*)(d_tables + o_merged);
+        plan->d_cells = (LfCellBucket*)(d_tables + o_cells);
     }
 
     KernelSet ks;
@@ -1802,7 +1893,12 @@ int lf_spmm_create(lf_spmm_plan** out_plan, const lf_bucket_desc* h_buckets, int
     (void)occ;
     plan->info[7] = (int64_t)(merged.size() + cells.size());
     plan->info[8] = (int64_t)cells.size();
-    LF_TRY_HIP(hipStreamSynchronize(s));     // the tables are complete: the plan may run on any stream
+    LF_TRY_HIP(read_back());                 // the tables are complete: the plan may run on any stream
+    for (int k = 0; k < num_buckets; ++k) {  // the filling pass must have taken the counted ranges
+        const int* c = back.as<int>(o_cursors) + (size_t)4 * k * kCounterLine;
+        if (counts[k].chunks > 0 && (c[0] != counts[k].chunks || c[kCounterLine] != counts[k].heavy || c[2 * kCounterLine] != counts[k].partials))
+            return bail(lf::fail(LF_ERR_INVALID, "bucket %d changed while the plan was being built", k));
+    }
     if (free_temporaries(plan) != LF_OK) return bail(lf::fail(LF_ERR_HIP, "hipFree failed on plan-time scratch"));
     *out_plan = plan;
     return LF_OK;

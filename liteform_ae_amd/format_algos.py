@@ -438,10 +438,10 @@ class HybSpMM:
             fmt = fmt_or_slabs
             self._keep.append(fmt)
             descs = (_lib.BucketDesc * max(fmt.num_buckets, 1))()
-            for k in range(fmt.num_buckets):
-                rows, cols, vals, meta = fmt.slab(k)[:4]
-                descs[k] = _lib.BucketDesc(fmt.flat_widths[k], fmt.part_of[k], int(fmt.ell_rows[k]),
-                                           rows.data_ptr(), cols.data_ptr(), vals.data_ptr(), meta.data_ptr())
+            rows, cols, vals, meta = (t.data_ptr() for t in (fmt.rows, fmt.cols, fmt.vals, fmt.meta))
+            for k, (w, p, n, r0, s0) in enumerate(zip(fmt.flat_widths, fmt.part_of, fmt.ell_rows.tolist(),
+                                                      fmt.row_off.tolist(), fmt.slot_off.tolist())):
+                descs[k] = _lib.BucketDesc(w, p, n, rows + 4 * r0, cols + 4 * s0, vals + 4 * s0, meta + 4 * r0)
             nb, P = fmt.num_buckets, fmt.num_parts
             num_rows, num_cols = fmt.num_rows, fmt.num_cols
         else:
