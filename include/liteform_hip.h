@@ -164,6 +164,17 @@ int lf_model_spmm_ms(const int64_t* h_stats, int32_t num_parts, int32_t n_window
 int lf_row_overlap(const int32_t* d_indptr, const int32_t* d_indices, int64_t num_rows, int64_t sample_stride,
                    void* d_scratch, int64_t* h_out /* [2] */, lf_stream_t stream);
 
+/* The inputs of the launch-shape choice from one pass: the statistics of lf_bucket_stats (CSR
+ * segment lengths, no column sets) for every candidate partition count h_parts[0..n_candidates),
+ * [sum of h_parts][LF_MAX_CLASSES][LF_STATS_FIELDS] in candidate order, and lf_row_overlap's two
+ * sums.  At most 16 candidates and 128 partitions together (LF_ERR_UNSUPPORTED beyond).  Takes the
+ * workspace that lf_shape_stats_workspace_bytes(sum of h_parts) names.  Synchronises the stream. */
+size_t lf_shape_stats_workspace_bytes(int32_t total_parts);
+int lf_shape_stats(const int32_t* d_indptr, const int32_t* d_indices, int64_t num_rows, int64_t num_cols,
+                   const int32_t* h_parts, int32_t n_candidates, int32_t width_limit, int64_t sample_stride,
+                   void* d_workspace, size_t workspace_bytes, int64_t* h_stats, int64_t* h_overlap /* [2] */,
+                   lf_stream_t stream);
+
 /* ------------------------------------------------------------------------------------
  * hyb composition.  Replaces build_hyb_format (format_algos.py:226-385).
  * Bucket k = (partition p, width index b) in row-major (p, b) order; widths of partition

@@ -33,11 +33,9 @@ LF_CSR_UNIT_VALUES = 2
 LIB_PATH = os.environ.get("LITEFORM_HIP_LIB") or os.path.join(os.path.dirname(os.path.abspath(__file__)),
                                                               "liblfhip.so")
 
-i32p = C.POINTER(C.c_int32)
-i64p = C.POINTER(C.c_int64)
-f32p = C.POINTER(C.c_float)
-f64p = C.POINTER(C.c_double)
 vp = C.c_void_p
+# host arrays go in as addresses (np_ptr): converting to a typed pointer costs 2 us an argument
+i32p = i64p = f32p = f64p = vp
 
 
 class BucketDesc(C.Structure):
@@ -61,6 +59,9 @@ SIGNATURES = {
                                           i32p, i32p, f64p, i32p]),
     "lf_model_spmm_ms": (C.c_int, [i64p, C.c_int32, C.c_int32, C.c_int64, C.c_int64, C.c_int32, C.c_int32, f64p]),
     "lf_row_overlap": (C.c_int, [vp, vp, C.c_int64, C.c_int64, vp, vp, vp]),
+    "lf_shape_stats_workspace_bytes": (C.c_size_t, [C.c_int32]),
+    "lf_shape_stats": (C.c_int, [vp, vp, C.c_int64, C.c_int64, i32p, C.c_int32, C.c_int32, C.c_int64, vp, C.c_size_t,
+                                 i64p, i64p, vp]),
     "lf_hyb_workspace_bytes": (C.c_size_t, [C.c_int64, C.c_int32, C.c_int32]),
     "lf_hyb_layout": (C.c_int, [i64p, i32p, C.c_int32, i64p, i64p, i64p, i64p]),
     "lf_stats_seg_bounds": (vp, [vp, C.c_int64, C.c_int32]),
@@ -142,4 +143,5 @@ def ptr(t):
 
 
 def np_ptr(a, ctype):
-    return a.ctypes.data_as(C.POINTER(ctype))
+    """Address of a numpy array of C type `ctype` for a call into the library."""
+    return a.__array_interface__["data"][0]

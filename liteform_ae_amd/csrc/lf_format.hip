@@ -156,13 +156,15 @@ row_features_kernel(const int32_t* __restrict__ indptr, int64_t rows, unsigned l
 // with 50 such rows).  Bound by latency: a thread per pair with a two-pointer walk was a chain of up
 // to 128 loads, 15.6 us for 8192 pairs.
 constexpr int kOverlapEntries = 64;
-__global__ void __launch_bounds__(kBlock)
+constexpr int kOverlapThreads = 1024;      // few, large workgroups: each ends with two atomics on one line
+constexpr int kOverlapGrid = 128;
+__global__ void __launch_bounds__(kOverlapThreads)
 row_overlap_kernel(const int32_t* __restrict__ indptr, const int32_t* __restrict__ indices, int64_t rows,
                    int64_t stride, unsigned long long* __restrict__ out) {
     const int lane = threadIdx.x & 63;
     uint32_t both = 0, seen = 0;
-    const int64_t waves = (int64_t)gridDim.x * (kBlock / 64);
-    for (int64_t i = (int64_t)blockIdx.x * (kBlock / 64) + (threadIdx.x >> 6);; i += waves) {
+    const int64_t waves = (int64_t)gridDim.x * (kOverlapThreads / 64);
+    for (int64_t i = (int64_t)blockIdx.x * (kOverlapThreads / 64) + (threadIdx.x >> 6);; i += waves) {
         const int64_t r = 1 + i * stride;
         if (r >= rows) break;
         const int a = indptr[r - 1], b = indptr[r];
@@ -183,14 +185,21 @@ row_overlap_kernel(const int32_t* __restrict__ indptr, const int32_t* __restrict
         both += __shfl_xor(both, d);
         seen += __shfl_xor(seen, d);
     }
-    __shared__ uint32_t s_sum[2][kBlock / 64];
+    __shared__ uint32_t s_sum[2][kOverlapThreads / 64];
     if (lane == 0) { s_sum[0][threadIdx.x >> 6] = both; s_sum[1][threadIdx.x >> 6] = seen; }
     __syncthreads();
     if (threadIdx.x < 2) {
         unsigned long long sum = 0;
-        for (int w = 0; w < kBlock / 64; ++w) sum += s_sum[threadIdx.x][w];
+        for (int w = 0; w < kOverlapThreads / 64; ++w) sum += s_sum[threadIdx.x][w];
         if (sum) atomicAdd(&out[threadIdx.x], sum);
     }
+}
+
+inline hipError_t launch_row_overlap(const int32_t* indptr, const int32_t* indices, int64_t rows, int64_t stride,
+                                     unsigned long long* out, hipStream_t s) {
+    const int64_t samples = (rows - 1 + stride - 1) / stride, per = kOverlapThreads / 64;
+    row_overlap_kernel<<<(int)std::min<int64_t>((samples + per - 1) / per, kOverlapGrid), kOverlapThreads, 0, s>>>(indptr, indices, rows, stride, out);
+    return hipGetLastError();
 }
 
 // Initial width class of a segment of `deg` entries: width = min(next_pow2(deg), limit),
@@ -268,6 +277,93 @@ class_count_kernel(SegView v, const int32_t* __restrict__ seg_deg, int kmax, uns
         sum += __shfl_xor(sum, 1);
         sum += __shfl_xor(sum, 2);
         if (part == 0 && sum) atomicAdd(&stats[stat_at(p, c / 3, c % 3)], (unsigned long long)sum);
+    }
+}
+
+// ---- statistics of several partition counts at once
+// What the launch-shape choice prices: the counters of class_count_kernel for every partition of
+// every candidate count, from one pass over the rows.  A thread finds the partition bounds of its
+// row for each candidate in turn (binary search in the row's ascending columns) and adds the
+// segments to counters in LDS; a workgroup leaves its counters in the workspace and
+// shape_reduce_kernel adds the workgroups up.  Bound by the latency of the searches.  One statistics
+// call per candidate - bounds written to memory and read back, a launch of its own for each kernel
+// and a synchronisation - took 41 us each for a 170K-row graph (four candidates and the row overlap
+// 235 us, now 86 with the Python around it).
+constexpr int kShapeCands = 16;
+constexpr int kShapeParts = 128;           // partitions of all candidates together
+constexpr int kShapeGrid = 512;
+struct ShapeCands {
+    int n, total;
+    int parts[kShapeCands];
+};
+
+// A workgroup's counters: total * LF_MAX_CLASSES words {nnz in the low half, segments in the high half}
+// (both sums stay below 2^31), then per partition the cost rows of the last class beyond one per segment.
+constexpr int shape_words(int total) { return total * (LF_MAX_CLASSES + 1); }
+
+__global__ void __launch_bounds__(kBlock)
+shape_stats_kernel(const int32_t* __restrict__ indptr, const int32_t* __restrict__ indices, int64_t rows, int64_t cols,
+                   ShapeCands cands, int kmax, unsigned long long* __restrict__ partial,
+                   unsigned long long* __restrict__ overlap) {
+    __shared__ unsigned long long s_cnt[shape_words(kShapeParts)];
+    const int n_words = shape_words(cands.total);
+    for (int i = threadIdx.x; i < n_words; i += kBlock) s_cnt[i] = 0;
+    if (blockIdx.x == 0 && threadIdx.x < 2) overlap[threadIdx.x] = 0;      // for row_overlap_kernel behind this one
+    __syncthreads();
+    for (int64_t r = (int64_t)blockIdx.x * kBlock + threadIdx.x; r < rows; r += (int64_t)gridDim.x * kBlock) {
+        const int lo = indptr[r], hi = indptr[r + 1];
+        if (lo >= hi) continue;
+        int q = 0;
+        for (int c = 0; c < cands.n; ++c) {
+            const int parts = cands.parts[c];
+            const int64_t psize = (cols + parts - 1) / parts;
+            int cur = lo;
+            for (int p = 0; p < parts; ++p, ++q) {
+                const int end = p + 1 < parts ? lower_bound_i32(indices, cur, hi, (int64_t)(p + 1) * psize) : hi;
+                const int fill = end - cur;
+                cur = end;
+                if (fill <= 0) continue;
+                int k, cost_rows;
+                width_class(fill, kmax, k, cost_rows);
+                atomicAdd(&s_cnt[q * LF_MAX_CLASSES + k], (1ull << 32) | (unsigned long long)fill);
+                if (cost_rows > 1) atomicAdd(&s_cnt[cands.total * LF_MAX_CLASSES + q], (unsigned long long)(cost_rows - 1));
+            }
+        }
+    }
+    __syncthreads();
+    for (int i = threadIdx.x; i < n_words; i += kBlock) partial[(size_t)blockIdx.x * n_words + i] = s_cnt[i];
+}
+
+// out[q][k] = {cost rows, nnz, segments, 0}: 64 words to a workgroup, 16 threads add up each.
+__global__ void __launch_bounds__(1024)
+shape_reduce_kernel(const unsigned long long* __restrict__ partial, int n_groups, int total, int kmax,
+                    unsigned long long* __restrict__ out) {
+    __shared__ unsigned long long s_sum[16][64];
+    const int n_words = shape_words(total);
+    const int w = blockIdx.x * 64 + (threadIdx.x & 63), slice = threadIdx.x >> 6;
+    unsigned long long sum = 0;
+    if (w < n_words) {
+        for (int g0 = slice; g0 < n_groups; g0 += 16 * 8) {
+            unsigned long long x[8];
+#pragma unroll
+            for (int u = 0; u < 8; ++u) x[u] = g0 + 16 * u < n_groups ? partial[(size_t)(g0 + 16 * u) * n_words + w] : 0ull;
+#pragma unroll
+            for (int u = 0; u < 8; ++u) sum += x[u];
+        }
+    }
+    s_sum[slice][threadIdx.x & 63] = sum;
+    __syncthreads();
+    if (slice != 0 || w >= n_words) return;
+    for (int i = 1; i < 16; ++i) sum += s_sum[i][threadIdx.x];
+    // the cost rows of the last class come from two words: each adds its part to a cleared field
+    if (w < total * LF_MAX_CLASSES) {
+        unsigned long long* o = out + (size_t)w * LF_STATS_FIELDS;
+        atomicAdd(&o[0], sum >> 32);
+        o[1] = sum & 0xFFFFFFFFull;
+        o[2] = sum >> 32;
+        o[3] = 0;
+    } else if (sum) {
+        atomicAdd(&out[((size_t)(w - total * LF_MAX_CLASSES) * LF_MAX_CLASSES + kmax) * LF_STATS_FIELDS], sum);
     }
 }
 
@@ -1245,12 +1341,58 @@ int lf_row_overlap(const int32_t* d_indptr, const int32_t* d_indices, int64_t nu
     LF_REQUIRE((uintptr_t)d_scratch % 8 == 0, LF_ERR_INVALID, "scratch must be 8-byte aligned");
     unsigned long long* acc = (unsigned long long*)d_scratch;
     LF_HIP(fill_u32(acc, 4, 0u, s));
-    const int64_t samples = (num_rows - 1 + sample_stride - 1) / sample_stride;
-    const int grid = (int)std::min<int64_t>((samples + kBlock / 64 - 1) / (kBlock / 64), 1024);
-    row_overlap_kernel<<<grid, kBlock, 0, s>>>(d_indptr, d_indices, num_rows, sample_stride, acc);
-    LF_HIP(hipGetLastError());
+    LF_HIP(launch_row_overlap(d_indptr, d_indices, num_rows, sample_stride, acc, s));
     LF_HIP(hipMemcpyAsync(h_out, acc, 16, hipMemcpyDeviceToHost, s));
     LF_HIP(hipStreamSynchronize(s));
+    return LF_OK;
+}
+
+size_t lf_shape_stats_workspace_bytes(int32_t total_parts) {
+    if (total_parts < 1 || total_parts > kShapeParts) return 0;
+    const size_t out = ((size_t)total_parts * LF_MAX_CLASSES * LF_STATS_FIELDS + 2) * 8;
+    return align_up(out, 256) + (size_t)kShapeGrid * shape_words(total_parts) * 8;
+}
+
+int lf_shape_stats(const int32_t* d_indptr, const int32_t* d_indices, int64_t num_rows, int64_t num_cols,
+                   const int32_t* h_parts, int32_t n_candidates, int32_t width_limit, int64_t sample_stride,
+                   void* d_workspace, size_t workspace_bytes, int64_t* h_stats, int64_t* h_overlap, lf_stream_t stream) {
+    hipStream_t s = (hipStream_t)stream;
+    LF_REQUIRE(h_parts && h_stats && h_overlap, LF_ERR_INVALID, "null argument");
+    LF_REQUIRE(n_candidates >= 1 && n_candidates <= kShapeCands, LF_ERR_UNSUPPORTED, "1..%d candidates (got %d)", kShapeCands, n_candidates);
+    LF_REQUIRE(sample_stride >= 1, LF_ERR_INVALID, "bad sample stride");
+    LF_REQUIRE(lf::is_pow2(width_limit) && width_limit <= (1 << (LF_MAX_CLASSES - 1)), LF_ERR_INVALID,
+               "width_limit must be a power of two <= %d", 1 << (LF_MAX_CLASSES - 1));
+    ShapeCands cands{};
+    cands.n = n_candidates;
+    for (int c = 0; c < n_candidates; ++c) {
+        if (int rc = check_common(d_indptr, d_indices, num_rows, num_cols, h_parts[c])) return rc;
+        LF_REQUIRE(cands.total + h_parts[c] <= kShapeParts, LF_ERR_UNSUPPORTED, "at most %d partitions of all candidates together", kShapeParts);
+        cands.parts[c] = h_parts[c];
+        cands.total += h_parts[c];
+    }
+    LF_REQUIRE(d_workspace && workspace_bytes >= lf_shape_stats_workspace_bytes(cands.total), LF_ERR_WORKSPACE,
+               "workspace has %zu bytes, %zu needed", workspace_bytes, lf_shape_stats_workspace_bytes(cands.total));
+    const size_t n_stats = (size_t)cands.total * LF_MAX_CLASSES * LF_STATS_FIELDS;
+    std::memset(h_stats, 0, n_stats * 8);
+    h_overlap[0] = h_overlap[1] = 0;
+    if (num_rows == 0) return LF_OK;
+    LF_REQUIRE(d_indices, LF_ERR_INVALID, "indices is null");
+    unsigned long long* out = (unsigned long long*)d_workspace;       // statistics, then the two overlap sums
+    unsigned long long* partial = (unsigned long long*)((char*)d_workspace + align_up((n_stats + 2) * 8, 256));
+    const int grid = (int)std::min<int64_t>((num_rows + kBlock - 1) / kBlock, kShapeGrid);
+    const int kmax = lf::ilog2(width_limit);
+    LF_HIP(fill_u32(out, (int64_t)n_stats * 2, 0u, s));
+    shape_stats_kernel<<<grid, kBlock, 0, s>>>(d_indptr, d_indices, num_rows, num_cols, cands, kmax, partial, out + n_stats);
+    LF_HIP(hipGetLastError());
+    shape_reduce_kernel<<<(shape_words(cands.total) + 63) / 64, 1024, 0, s>>>(partial, grid, cands.total, kmax, out);
+    LF_HIP(hipGetLastError());
+    if (num_rows > 1) LF_HIP(launch_row_overlap(d_indptr, d_indices, num_rows, sample_stride, out + n_stats, s));
+    lf::PinnedLoan back((n_stats + 2) * 8);
+    LF_REQUIRE(back.ok(), LF_ERR_HIP, "out of host memory");
+    LF_HIP(hipMemcpyAsync(back.as<char>(), out, (n_stats + 2) * 8, hipMemcpyDeviceToHost, s));
+    LF_HIP(hipStreamSynchronize(s));
+    std::memcpy(h_stats, back.as<char>(), n_stats * 8);
+    std::memcpy(h_overlap, back.as<char>(n_stats * 8), 16);
     return LF_OK;
 }
 

@@ -55,16 +55,25 @@ class CostModelSettings:
 
 
 # --------------------------------------------------------------------------- device plumbing
+_gpu_torch = None                # the torch module, once a GPU has been seen
+
+
 def _torch():
-    import torch
-    if not torch.cuda.is_available():
-        raise RuntimeError("liteform_ae_amd needs a ROCm GPU (torch.cuda.is_available() is False); "
-                           "there is no CPU fallback")
-    return torch
+    global _gpu_torch
+    if _gpu_torch is None:
+        import torch
+        if not torch.cuda.is_available():
+            raise RuntimeError("liteform_ae_amd needs a ROCm GPU (torch.cuda.is_available() is False); "
+                               "there is no CPU fallback")
+        torch.cuda.init()
+        _gpu_torch = torch
+    return _gpu_torch
 
 
 def _stream():
-    return _torch().cuda.current_stream().cuda_stream
+    """hipStream_t of the current stream of the current device, as an integer."""
+    cuda = _torch()._C
+    return cuda._cuda_getCurrentRawStream(cuda._cuda_getDevice())
 
 
 _STAGE_BYTES = 16 << 20          # per staging buffer
@@ -793,28 +802,56 @@ def predict_launch_shape(g, feat_size: int, b_dtype: str = "f32", candidates: Se
     if windows is None:
         windows = _window_candidates(feat_size, b_dtype)
     rows, cols = int(g.num_src_nodes()), int(g.num_dst_nodes())
+    dense = int(g.num_edges()) > DENSE_USES_PER_B_ROW * cols
+    few = [p for p in candidates if p <= 4] or [min(candidates)]
+    priced = [p for p in candidates if p in few or dense]
+    at_once = _shape_statistics(g, priced)
     predicted = {}
-    if row_overlap_device(g) >= ROW_OVERLAP_STRUCTURED:
+    overlap = at_once[1] if at_once is not None else row_overlap_device(g)
+    if overlap >= ROW_OVERLAP_STRUCTURED:
         best = (min(candidates), _structured_windows(feat_size, b_dtype, windows))
     else:
-        dense = int(g.num_edges()) > DENSE_USES_PER_B_ROW * cols
-        few = [p for p in candidates if p <= 4] or [min(candidates)]
-        for p in candidates:
-            if p not in few and not dense:
-                continue
-            try:
-                stats, _ = bucket_statistics(g, p, with_columns=False)
-            except ValueError:
-                continue
+        for i, p in enumerate(priced):
+            if at_once is not None:
+                stats = at_once[0][i]
+            else:
+                try:
+                    stats, _ = bucket_statistics(g, p, with_columns=False)
+                except ValueError:
+                    continue
             for w in windows:
                 predicted[(p, w)] = model_spmm_ms(stats, w, rows, cols, feat_size, b_dtype)
         best = pick_launch_shape(predicted)
-        # every statistics pass left its per-partition row bounds behind for the slab builder
+        # a statistics pass leaves its per-partition row bounds behind for the slab builder
         # ((P + 1) x rows words each); only those of the chosen partition count are of use
         kept = _device_csr(g)._stats_ws
         for p in [p for p in kept if p != best[0]]:
             del kept[p]
     return (best, predicted) if return_predictions else best
+
+
+def _shape_statistics(g, parts: Sequence[int], max_samples: int = 8192):
+    """(statistics of every partition count in ``parts``, row overlap) from one pass on the GPU
+    (lf_shape_stats), or None where its limits do not allow it: degrees that are not the CSR's
+    (duplicates in the COO), more than 16 counts or 128 partitions together."""
+    dev = _device_csr(g)
+    total = sum(parts)
+    if dev.coo_nnz != dev.nnz or dev.nnz == 0 or dev.num_rows < 2 or len(parts) > 16 or total > 128 or min(parts) < 1:
+        return None
+    torch = _torch()
+    lib = _lib.load()
+    stats = np.empty((total, _lib.LF_MAX_CLASSES, _lib.LF_STATS_FIELDS), dtype=np.int64)
+    shared = np.empty(2, dtype=np.int64)
+    counts = np.asarray(parts, dtype=np.int32)
+    nbytes = lib.lf_shape_stats_workspace_bytes(total)
+    ws = torch.empty(nbytes, dtype=torch.uint8, device="cuda")
+    _lib.check(lib.lf_shape_stats(dev.indptr.data_ptr(), dev.indices.data_ptr(), dev.num_rows, dev.num_cols,
+                                  _lib.np_ptr(counts, C.c_int32), len(parts), WIDTH_LIMIT, max(1, dev.num_rows // max_samples),
+                                  ws.data_ptr(), nbytes, _lib.np_ptr(stats, C.c_int64), _lib.np_ptr(shared, C.c_int64),
+                                  _stream()))
+    ends = np.cumsum(counts)
+    overlap = float(shared[0]) / float(shared[1]) if shared[1] else 0.0
+    return [stats[e - p:e] for p, e in zip(parts, ends.tolist())], overlap
 
 
 def _structured_windows(feat_size: int, b_dtype: str, windows: Sequence[int]) -> int:

@@ -64,3 +64,19 @@ def test_structured_and_small_matrices_get_one_launch(fa):
     sparse = skewed_matrix(rng, 30000, 30000, mean_deg=2, heavy_rows=0)
     assert set(fa.predict_launch_shape(sparse, 128, return_predictions=True)[1]) == {(p, w) for p in (1, 2, 3, 4) for w in (1, 2)}
     assert fa.guess_num_partitions(g, 128) == 1
+
+
+@pytest.mark.parametrize("nr,nc,parts", [
+    (2, 5, (1, 2, 3)),                               # more partitions than some rows have columns
+    (255, 40, (1, 32, 64)),
+    (256, 3000, (1,)),
+    (257, 3000, (128,)),                             # the most partitions
+    (140_000, 9000, (1, 2, 3, 4, 8, 16, 32)),        # more rows than the launch has threads
+])
+def test_shape_statistics_match_one_by_one(fa, nr, nc, parts):
+    rng = np.random.default_rng(nr)
+    g = skewed_matrix(rng, nr, nc, mean_deg=4, heavy_rows=min(3, nr - 1), heavy_len=min(nc, 2500))
+    stats, overlap = fa._shape_statistics(g, parts)
+    assert overlap == fa.row_overlap_device(g)
+    for s, p in zip(stats, parts):
+        np.testing.assert_array_equal(s, fa.bucket_statistics(g, p, with_columns=False)[0])
