@@ -847,11 +847,30 @@ hyb_count_kernel(SegView v, const int32_t* __restrict__ seg_deg, const int32_t* 
         blockcnt[(int64_t)(w[12] + threadIdx.x) * nblk + blockIdx.x] = s_cnt[threadIdx.x];
 }
 
-// Exclusive scan over blocks, one workgroup per bucket; totals[k] = ELL rows of bucket k.
+struct BucketOffsets {
+    long long slot_off;    // first slot of the bucket in the flat slab arrays
+    long long row_off;     // first ELL row of the bucket in the flat row arrays
+};
+
+// Flat slab layout shared by the builder and its callers: ELL rows of bucket k start at a
+// multiple of 64 entries, its slots at a multiple of 1024, so every slab is at least 256-byte
+// aligned inside 256-byte aligned allocations.
+constexpr int64_t kRowAlign = 64;
+constexpr int64_t kSlotAlign = 1024;
+__host__ __device__ inline void flat_layout_step(int64_t ell_rows, int64_t width, int64_t* rows, int64_t* slots) {
+    *rows += (ell_rows + kRowAlign - 1) / kRowAlign * kRowAlign;
+    *slots += (ell_rows * width + kSlotAlign - 1) / kSlotAlign * kSlotAlign;
+}
+
+// Exclusive scan over blocks, one workgroup per bucket; totals[k] = ELL rows of bucket k.  The
+// workgroup that ends last derives the flat layout from the totals, so that the fill needs
+// nothing more from the host.
 __global__ void __launch_bounds__(1024)
-hyb_scan_kernel(int32_t* __restrict__ blockcnt, int nblk, long long* __restrict__ totals) {
+hyb_scan_kernel(int32_t* __restrict__ blockcnt, int nblk, long long* __restrict__ totals,
+                const int32_t* __restrict__ widths, int* __restrict__ done, BucketOffsets* __restrict__ offs) {
     __shared__ long long s_wave[16];
     __shared__ long long s_carry;
+    __shared__ int s_last;
     int32_t* a = blockcnt + (int64_t)blockIdx.x * nblk;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     if (threadIdx.x == 0) s_carry = 0;
@@ -874,7 +893,32 @@ hyb_scan_kernel(int32_t* __restrict__ blockcnt, int nblk, long long* __restrict_
         if (threadIdx.x == 1023) s_carry = carry + wave_off + incl;
         __syncthreads();
     }
-    if (threadIdx.x == 0) totals[blockIdx.x] = s_carry;
+    if (threadIdx.x == 0) {
+        __hip_atomic_store(&totals[blockIdx.x], s_carry, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        // (release: the total above is visible before the count; acquire: so are the others')
+        s_last = __hip_atomic_fetch_add(done, 1, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT) == (int)gridDim.x - 1;
+    }
+    __syncthreads();
+    if (!s_last) return;
+    const int nb = gridDim.x;
+    int64_t row = 0, slot = 0;                        // carried by thread 0
+    for (int base = 0; base < nb; base += 1024) {     // staged through LDS: the layout is a serial sum
+        __shared__ long long s_rows[1024];
+        __shared__ int s_width[1024];
+        const int i = base + threadIdx.x;
+        if (i < nb) {
+            s_rows[threadIdx.x] = __hip_atomic_load(&totals[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            s_width[threadIdx.x] = widths[i];
+        }
+        __syncthreads();
+        if (threadIdx.x == 0) {
+            for (int k = 0; k < 1024 && base + k < nb; ++k) {
+                offs[base + k] = BucketOffsets{slot, row};
+                flat_layout_step(s_rows[k], s_width[k], &row, &slot);
+            }
+        }
+        __syncthreads();
+    }
 }
 
 // Fills the slabs.  One workgroup per 256 source rows, four column partitions at a time.
@@ -889,11 +933,6 @@ hyb_scan_kernel(int32_t* __restrict__ blockcnt, int nblk, long long* __restrict_
 // Reading in row order matters: a source row is ~130 bytes at an arbitrary offset, and when
 // the slabs were filled bucket by bucket every row cost two full cache lines (1.27 GB fetched
 // for 0.65 GB of entries on an 81.6M-nonzero matrix).
-struct BucketOffsets {
-    long long slot_off;    // first slot of the bucket in the flat slab arrays
-    long long row_off;     // first ELL row of the bucket in the flat row arrays
-};
-
 constexpr int kFillUnroll = 4;
 constexpr int kPartGroup = 4;        // column partitions whose segments are walked together
 // four consecutive 32-bit values at a 4-byte aligned address (one 16-byte load)
@@ -1130,7 +1169,7 @@ StatsLayout stats_layout(int64_t rows, int64_t cols, int parts) {
 }
 
 struct HybLayout {
-    size_t bnd, wtab, flags, totals, row_off, scatter, blockcnt, total;
+    size_t bnd, wtab, widths, flags, totals, scatter, blockcnt, total;
     int nblk;
 };
 
@@ -1143,11 +1182,11 @@ HybLayout hyb_layout(int64_t rows, int parts, int total_buckets) {
     if (parts > 1) off += align_up((size_t)(parts + 1) * rows * 4, 256);
     L.wtab = off;
     off += align_up((size_t)parts * kWtabStride * 4, 256);
-    L.flags = off;
+    L.widths = off;                     // (behind wtab: they go up together)
+    off += align_up((size_t)std::max(total_buckets, 1) * 4, 256);
+    L.flags = off;                      // error flags, finished workgroups of the scan
     off += 256;
-    L.totals = off;
-    off += align_up((size_t)std::max(total_buckets, 1) * 8, 256);
-    L.row_off = off;
+    L.totals = off;                     // (behind the flags: cleared and read back together)
     off += align_up((size_t)std::max(total_buckets, 1) * 8, 256);
     L.scatter = off;
     off += align_up((size_t)std::max(total_buckets, 1) * sizeof(BucketOffsets), 256);
@@ -1157,20 +1196,13 @@ HybLayout hyb_layout(int64_t rows, int parts, int total_buckets) {
     return L;
 }
 
-// Flat slab layout shared by the builder and its callers: ELL rows of bucket k start at a
-// multiple of 64 entries, its slots at a multiple of the scatter workgroup span (1024
-// slots), so every slab is at least 256-byte aligned inside 256-byte aligned allocations.
-constexpr int64_t kRowAlign = 64;
-constexpr int64_t kSlotAlign = 1024;   // a bucket's slots start at a multiple of this in the flat slab arrays
-
 void flat_layout(const int64_t* ell_rows, const int32_t* widths, int nb, int64_t* row_off,
                  int64_t* slot_off, int64_t* total_rows, int64_t* total_slots) {
     int64_t r = 0, s = 0;
     for (int k = 0; k < nb; ++k) {
         row_off[k] = r;
         slot_off[k] = s;
-        r += (ell_rows[k] + kRowAlign - 1) / kRowAlign * kRowAlign;
-        s += (ell_rows[k] * widths[k] + kSlotAlign - 1) / kSlotAlign * kSlotAlign;
+        flat_layout_step(ell_rows[k], widths[k], &r, &s);
     }
     *total_rows = r;
     *total_slots = s;
@@ -1325,8 +1357,7 @@ int lf_row_features(const int32_t* d_indptr, int64_t num_rows, void* d_scratch, 
     const int grid = (int)std::min<int64_t>((num_rows + kBlock - 1) / kBlock, 1024);
     row_features_kernel<<<grid, kBlock, 0, s>>>(d_indptr, num_rows, acc);
     LF_HIP(hipGetLastError());
-    LF_HIP(hipMemcpyAsync(h_out, acc, 32, hipMemcpyDeviceToHost, s));
-    LF_HIP(hipStreamSynchronize(s));
+    LF_HIP(lf::read_back(h_out, acc, 32, s));
     return LF_OK;
 }
 
@@ -1342,8 +1373,7 @@ int lf_row_overlap(const int32_t* d_indptr, const int32_t* d_indices, int64_t nu
     unsigned long long* acc = (unsigned long long*)d_scratch;
     LF_HIP(fill_u32(acc, 4, 0u, s));
     LF_HIP(launch_row_overlap(d_indptr, d_indices, num_rows, sample_stride, acc, s));
-    LF_HIP(hipMemcpyAsync(h_out, acc, 16, hipMemcpyDeviceToHost, s));
-    LF_HIP(hipStreamSynchronize(s));
+    LF_HIP(lf::read_back(h_out, acc, 16, s));
     return LF_OK;
 }
 
@@ -1484,17 +1514,22 @@ int lf_hyb_plan(const int32_t* d_indptr, const int32_t* d_indices, const int32_t
     int32_t* blockcnt = (int32_t*)(ws + L.blockcnt);
     const int64_t psize = lf::ceil_div(num_cols, num_parts);
 
-    std::vector<int32_t> h_wtab((size_t)num_parts * kWtabStride, 0);
+    const size_t up_bytes = L.flags - L.wtab, back_bytes = L.totals - L.flags + (size_t)nb * 8;
+    lf::PinnedLoan up(up_bytes), back(back_bytes);
+    LF_REQUIRE(up.ok() && back.ok(), LF_ERR_HIP, "out of host memory");
+    int32_t* h_wtab = up.as<int32_t>();
+    std::memset(h_wtab, 0, up_bytes);
     for (int p = 0; p < num_parts; ++p) {
         const int n = h_widths_off[p + 1] - h_widths_off[p];
         h_wtab[(size_t)p * kWtabStride] = n;
         for (int b = 0; b < n; ++b) h_wtab[(size_t)p * kWtabStride + 1 + b] = h_widths_flat[h_widths_off[p] + b];
         h_wtab[(size_t)p * kWtabStride + 12] = h_widths_off[p];
     }
-    LF_HIP(hipMemcpyAsync(wtab, h_wtab.data(), h_wtab.size() * 4, hipMemcpyHostToDevice, s));
-    LF_HIP(hipStreamSynchronize(s));     // h_wtab is pageable and about to go out of scope
-    LF_HIP(fill_u32(flags, 64, 0u, s));
-    LF_HIP(fill_u32(totals, (int64_t)std::max(nb, 1) * 2, 0u, s));
+    if (nb > 0) std::memcpy(up.as<char>(L.widths - L.wtab), h_widths_flat, (size_t)nb * 4);
+    // The loans go back when this returns: every way out from here on waits for the stream first.
+    struct Wait { hipStream_t s; ~Wait() { (void)hipStreamSynchronize(s); } } wait{s};
+    LF_HIP(hipMemcpyAsync(wtab, h_wtab, up_bytes, hipMemcpyHostToDevice, s));
+    LF_HIP(fill_u32(flags, (int64_t)(back_bytes / 4), 0u, s));
     if (num_rows > 0) {
         if (num_parts > 1 && d_seg_bounds) {       // bounds already known (the statistics pass made them)
             LF_HIP(hipMemcpyAsync(bnd, d_seg_bounds, (size_t)(num_parts + 1) * num_rows * 4,
@@ -1507,20 +1542,19 @@ int lf_hyb_plan(const int32_t* d_indptr, const int32_t* d_indices, const int32_t
         hyb_count_kernel<<<dim3(L.nblk, num_parts), kBlock, 0, s>>>(v, d_seg_deg, wtab, L.nblk, blockcnt, flags);
         LF_HIP(hipGetLastError());
         if (nb > 0) {
-            hyb_scan_kernel<<<nb, 1024, 0, s>>>(blockcnt, L.nblk, totals);
+            hyb_scan_kernel<<<nb, 1024, 0, s>>>(blockcnt, L.nblk, totals, (const int32_t*)(ws + L.widths), flags + 1,
+                                                (BucketOffsets*)(ws + L.scatter));
             LF_HIP(hipGetLastError());
         }
     }
-    int32_t h_flags = 0;
-    std::vector<long long> h_tot((size_t)std::max(nb, 1), 0);
-    LF_HIP(hipMemcpyAsync(&h_flags, flags, 4, hipMemcpyDeviceToHost, s));
-    if (nb > 0) LF_HIP(hipMemcpyAsync(h_tot.data(), totals, (size_t)nb * 8, hipMemcpyDeviceToHost, s));
+    LF_HIP(hipMemcpyAsync(back.as<char>(), flags, back_bytes, hipMemcpyDeviceToHost, s));
     LF_HIP(hipStreamSynchronize(s));
+    const int32_t h_flags = *back.as<int32_t>();
     if (h_flags & 1)
         return lf::fail(LF_ERR_CONFIG, "list index out of range: a partition with nonzeros has no bucket widths");
     if (h_flags & 2)
         return lf::fail(LF_ERR_UNSUPPORTED, "a row is split over more than %d ELL rows", kMetaSegMax);
-    for (int k = 0; k < nb; ++k) h_ell_rows[k] = h_tot[k];
+    for (int k = 0; k < nb; ++k) h_ell_rows[k] = num_rows > 0 ? back.as<long long>(L.totals - L.flags)[k] : 0;
     return LF_OK;
 }
 
@@ -1551,17 +1585,7 @@ int lf_hyb_build(const int32_t* d_indptr, const int32_t* d_indices, const float*
     BucketOffsets* offs = (BucketOffsets*)(ws + L.scatter);
     int32_t* blockoff = (int32_t*)(ws + L.blockcnt);
 
-    std::vector<BucketOffsets> h_offs((size_t)nb);
-    std::vector<int64_t> roff((size_t)nb), soff((size_t)nb);
-    int64_t flat_rows, flat_slots;
-    flat_layout(h_ell_rows, h_widths_flat, nb, roff.data(), soff.data(), &flat_rows, &flat_slots);
-    for (int k = 0; k < nb; ++k) {
-        h_offs[k].slot_off = soff[k];
-        h_offs[k].row_off = roff[k];
-    }
-    LF_HIP(hipMemcpyAsync(offs, h_offs.data(), (size_t)nb * sizeof(BucketOffsets), hipMemcpyHostToDevice, s));
-    LF_HIP(hipStreamSynchronize(s));     // the pageable source goes out of scope below
-
+    // (the bucket offsets are in the workspace: hyb_scan_kernel left them there)
     SegView v{d_indptr, bnd, num_rows, num_parts};
     hyb_fill_kernel<<<L.nblk, kBlock, 0, s>>>(v, d_seg_deg, wtab, L.nblk, blockoff, offs, d_indices, d_values,
                                               d_rows, d_meta, d_cols, d_vals, d_mask);

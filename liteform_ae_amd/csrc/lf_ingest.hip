@@ -183,8 +183,7 @@ int csr_check(const int32_t* d_indptr, const int32_t* d_indices, const float* d_
     csr_check_kernel<<<grid, 256, 0, s>>>(d_indptr, d_indices, d_values, num_rows, num_cols, nnz, out);
     LF_HIP(hipGetLastError());
     unsigned int h[4] = {0, 0, 0, 0};
-    LF_HIP(hipMemcpyAsync(h, out, 16, hipMemcpyDeviceToHost, s));
-    LF_HIP(hipStreamSynchronize(s));
+    LF_HIP(lf::read_back(h, out, 16, s));
     LF_REQUIRE(h[0] == 0, LF_ERR_INVALID,
                "%s: the row pointer is not a non-decreasing sequence from 0 to nnz = %lld, or an index lies outside [0, %lld)",
                what, (long long)nnz, (long long)num_cols);
@@ -253,8 +252,7 @@ int lf_coo_to_csr(const int32_t* d_coo_row, const int32_t* d_coo_col, const floa
     row_pointer_kernel<<<(int)((num_rows + 1 + 255) / 256), 256, 0, s>>>(keys_a, count, num_rows, num_cols, d_indptr);
     LF_HIP(hipGetLastError());
     int h_count = 0;
-    LF_HIP(hipMemcpyAsync(&h_count, count, 4, hipMemcpyDeviceToHost, s));
-    LF_HIP(hipStreamSynchronize(s));
+    LF_HIP(lf::read_back(&h_count, count, 4, s));
     *h_nnz_out = h_count;
     return LF_OK;
 }

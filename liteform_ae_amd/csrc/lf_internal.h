@@ -3,6 +3,7 @@
 #include <cstdarg>
 #include <cstdint>
 #include <cstdio>
+#include <cstring>
 #include <string>
 
 #include "liteform_hip.h"
@@ -43,6 +44,17 @@ private:
     void* p_ = nullptr;
     bool pinned_ = false;
 };
+
+// A few words from the GPU, and the wait for them.
+inline hipError_t read_back(void* h_dst, const void* d_src, size_t bytes, hipStream_t s) {
+    PinnedLoan loan(bytes);
+    if (!loan.ok()) return hipErrorOutOfMemory;
+    hipError_t e = hipMemcpyAsync(loan.as<char>(), d_src, bytes, hipMemcpyDeviceToHost, s);
+    const hipError_t w = hipStreamSynchronize(s);
+    if (e == hipSuccess) e = w;
+    if (e == hipSuccess) std::memcpy(h_dst, loan.as<char>(), bytes);
+    return e;
+}
 
 // Structural check of caller-supplied CSR (or BSR block) index arrays on the GPU, behind
 // lf_csr_check and in front of lf_csr_spmm / lf_bsr_spmm; `what` names the arrays in the
