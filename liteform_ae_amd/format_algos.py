@@ -24,6 +24,7 @@ from __future__ import annotations
 
 import ctypes as C
 import os
+import threading
 import time
 from typing import List, Sequence
 
@@ -76,37 +77,53 @@ def _stream():
     return cuda._cuda_getCurrentRawStream(cuda._cuda_getDevice())
 
 
-_STAGE_BYTES = 16 << 20          # per staging buffer
-_stage = None                    # two pinned buffers and their events, made on first use
+# Page-locked staging buffers: (bytes of one, how many), for arrays below and from _STAGE_LARGE on.
+# Large arrays want large pieces (a 326 MB index array 48 GB/s, 27 as a plain copy from pageable
+# memory); small ones want the first piece to leave early (three 3 MB arrays 360 us as plain
+# copies).  The buffers belong to the process, one set per device, are made on first use and are shared
+# under a lock.
+_STAGE_LARGE = 64 << 20
+_STAGE_SHAPES = {False: (2 << 20, 4), True: (16 << 20, 2)}
+_stages = {}
+_stage_lock = threading.Lock()
+_TORCH_TYPES = ("bool", "uint8", "int8", "int16", "int32", "int64", "float16", "float32", "float64")
 
 
 def _upload(array, dtype):
-    """A host array as a device tensor of `dtype` (int32 or float32).  Large arrays go through two
-    pinned 16 MB staging buffers: the copy into a pinned buffer runs on the host's threads while
-    the previous chunk crosses PCIe, which moves a 326 MB index array at 48 GB/s where a plain copy
-    from pageable memory reaches 27.  The two buffers belong to the process: one upload at a time
-    (the reference's driver is single-threaded too)."""
-    global _stage
+    """A host array as a device tensor of `dtype` (int32 or float32), enqueued on the current stream.
+    It goes through page-locked staging buffers: the copy into one runs on the host's threads, the
+    conversion to `dtype` with it, while the piece before crosses PCIe."""
     torch = _torch()
-    src = torch.from_numpy(np.ascontiguousarray(array, dtype=dtype))
+    array = np.ascontiguousarray(array)
+    if array.dtype.name not in _TORCH_TYPES or not array.dtype.isnative:
+        array = np.ascontiguousarray(array, dtype=dtype)
+    src = torch.from_numpy(array).reshape(-1)
     n = src.numel()
-    chunk = _STAGE_BYTES // src.element_size()
-    if n < 4 * chunk:
-        return src.cuda()
-    if _stage is None:
-        _stage = ([torch.empty(_STAGE_BYTES, dtype=torch.uint8, pin_memory=True) for _ in range(2)],
-                  [torch.cuda.Event() for _ in range(2)])
-    bufs, events = _stage
-    out = torch.empty(n, dtype=src.dtype, device="cuda")
-    for k, off in enumerate(range(0, n, chunk)):
-        m = min(chunk, n - off)
-        b = k & 1
-        stage = bufs[b].view(src.dtype)[:m]
-        events[b].synchronize()                      # the buffer's previous chunk has left
-        stage.copy_(src[off:off + m])
-        out[off:off + m].copy_(stage, non_blocking=True)
-        events[b].record()
+    out = torch.empty(n, dtype=torch.int32 if dtype is np.int32 else torch.float32, device="cuda")
+    large = 4 * n >= _STAGE_LARGE
+    stage_bytes, count = _STAGE_SHAPES[large]
+    with _stage_lock:
+        key = (large, torch.cuda.current_device())      # an event belongs to a device
+        stage = _stages.get(key)
+        if stage is None:
+            stage = _stages[key] = ([torch.empty(stage_bytes, dtype=torch.uint8, pin_memory=True) for _ in range(count)],
+                                    [torch.cuda.Event() for _ in range(count)], [0])
+        bufs, events, turn = stage
+        chunk = stage_bytes // 4
+        for off in range(0, n, chunk):
+            m = min(chunk, n - off)
+            b = turn[0] = (turn[0] + 1) % count
+            piece = bufs[b].view(out.dtype)[:m]
+            events[b].synchronize()                      # the buffer's previous piece has left
+            piece.copy_(src[off:off + m])
+            out[off:off + m].copy_(piece, non_blocking=True)
+            events[b].record()
     return out
+
+
+def _all_ones(data) -> bool:
+    """Whether a host array holds nothing but 1 (the first entries settle it for most that do not)."""
+    return bool(np.all(data[:1024] == 1)) and bool(np.all(data == 1))
 
 
 class _DeviceCSR:
@@ -136,7 +153,11 @@ class _DeviceCSR:
         if src is not None and self._from_csr(src, bool(getattr(g, "_unit_values", False))):
             self.path = "csr"
         else:
-            self._from_coo(g.coo_mtx)
+            triplets = getattr(g, "_triplets", None)
+            if triplets is None:
+                coo = g.coo_mtx
+                triplets = (coo.row, coo.col, coo.data)
+            self._from_coo(*triplets[:3])
             self.path = "coo"
         torch.cuda.current_stream().synchronize()
 
@@ -167,13 +188,13 @@ class _DeviceCSR:
             self._values = _torch().ones(self.nnz, dtype=_torch().float32, device="cuda")
         return self._values
 
-    def _from_coo(self, coo):
+    def _from_coo(self, row, col, data):
         torch = _torch()
         lib = _lib.load()
-        row = _upload(coo.row, np.int32)
-        col = _upload(coo.col, np.int32)
-        data = np.asarray(coo.data)
-        ones = bool(np.all(data == 1))
+        row = _upload(row, np.int32)
+        col = _upload(col, np.int32)
+        data = np.asarray(data)
+        ones = _all_ones(data)
         val = None if ones else _upload(data, np.float32)
         n = max(self.coo_nnz, 1)
         self.indptr = torch.empty(self.num_rows + 1, dtype=torch.int32, device="cuda")
@@ -209,10 +230,13 @@ class _DeviceCSR:
 
 
 def _matrix_identity(g):
-    """The object whose replacement means "another matrix": the CSR arrays a container was
-    made from, else its COO matrix."""
-    src = getattr(g, "_csr_source", None)
-    return src if src is not None else g.coo_mtx
+    """The object whose replacement means "another matrix": the CSR arrays or the triplets a
+    container was made from, else its COO matrix."""
+    for name in ("_csr_source", "_triplets"):
+        src = getattr(g, name, None)
+        if src is not None:
+            return src
+    return g.coo_mtx
 
 
 def _device_csr(g) -> _DeviceCSR:

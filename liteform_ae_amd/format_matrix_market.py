@@ -25,6 +25,19 @@ __all__ = ["MTX", "Bucket"]
 _GRAPH_DATASETS = ("cora", "citeseer", "pubmed", "ppi", "arxiv", "proteins", "reddit")
 
 
+def _are_plain_triplets(row, col, data, shape):
+    """Whether scipy would keep the arrays as they are: int32 indices inside the shape, one real value
+    each.  (Anything else is left to scipy, which converts it or raises.)  One pass over either
+    index array - a negative index is a large unsigned one - where scipy's constructor makes four."""
+    if not (row.dtype == col.dtype == np.int32 and data.dtype in (np.float32, np.float64)):
+        return False
+    if not (row.ndim == col.ndim == data.ndim == 1 and 0 < len(row) == len(col) == len(data)):
+        return False
+    if not (isinstance(shape, tuple) and len(shape) == 2 and all(isinstance(n, (int, np.integer)) and 0 < n < 2**31 for n in shape)):
+        return False
+    return all(int(i.view(np.uint32).max()) < n for i, n in zip((row, col), shape))
+
+
 class Bucket:
     """One (partition, width) bucket as the cost model sees it
     (format_matrix_market.py:12-37)."""
@@ -57,6 +70,7 @@ class MTX:
         self._coo = None
         self._csr = None
         self._csr_source = None       # the CSR matrix this container was made from (from_csr), as given
+        self._triplets = None         # (row, col, data, shape) this container was made from (from_coo)
         self._unit_values = False     # from_csr without data: every stored value is 1
         if filename is None:
             self.name = None
@@ -73,12 +87,16 @@ class MTX:
             self.coo_mtx = coo
 
     # ``coo_mtx`` is the reference's one data attribute (format_matrix_market.py:44-46).  A
-    # container made from CSR arrays keeps them and builds the COO view only when it is asked
-    # for, so that a CSR input can go to the GPU as it is.
+    # container made from CSR arrays or checked triplets keeps them and builds the COO view only
+    # when it is asked for, so that they can go to the GPU as they are.
     @property
     def coo_mtx(self):
-        if self._coo is None and self._csr_source is not None:
-            self._coo = self._csr_source.tocoo()
+        if self._coo is None:
+            if self._csr_source is not None:
+                self._coo = self._csr_source.tocoo()
+            elif self._triplets is not None:
+                row, col, data, shape = self._triplets
+                self._coo = sp.coo_matrix((data, (row, col)), shape=shape)
         return self._coo
 
     @coo_mtx.setter
@@ -86,6 +104,7 @@ class MTX:
         self._coo = value
         self._csr = None                               # cached views follow the COO
         self._csr_source = None
+        self._triplets = None
         self._unit_values = False
 
     # ---- constructors without a file -------------------------------------------------
@@ -97,7 +116,11 @@ class MTX:
         col = np.asarray(col)
         if data is None:
             data = np.ones(len(row))
-        m.coo_mtx = sp.coo_matrix((np.asarray(data), (row, col)), shape=shape)
+        data = np.asarray(data)
+        if _are_plain_triplets(row, col, data, shape):
+            m._triplets = (row, col, data, (int(shape[0]), int(shape[1])))
+        else:
+            m.coo_mtx = sp.coo_matrix((data, (row, col)), shape=shape)
         return m
 
     @classmethod
@@ -128,6 +151,8 @@ class MTX:
         return self._csr
 
     def _shape(self):
+        if self._coo is None and self._triplets is not None:
+            return self._triplets[3]
         return (self._csr_source if self._coo is None and self._csr_source is not None else self.coo_mtx).shape
 
     def adj_tensors(self, format: str):
@@ -151,6 +176,8 @@ class MTX:
         # stored entries: the COO view of a CSR matrix holds exactly its stored entries
         if self._coo is None and self._csr_source is not None:
             return self._csr_source.nnz
+        if self._coo is None and self._triplets is not None:
+            return len(self._triplets[2])
         return self.coo_mtx.nnz
 
     def dot(self, B):
