@@ -83,10 +83,21 @@ def _stream():
 # copies).  The buffers belong to the process, one set per device, are made on first use and are shared
 # under a lock.
 _STAGE_LARGE = 64 << 20
-_STAGE_SHAPES = {False: (2 << 20, 4), True: (16 << 20, 2)}
+_STAGE_SHAPES = {False: (2 << 20, 6), True: (16 << 20, 3)}
 _stages = {}
 _stage_lock = threading.Lock()
 _TORCH_TYPES = ("bool", "uint8", "int8", "int16", "int32", "int64", "float16", "float32", "float64")
+
+
+def _staging(nbytes):
+    """(buffers, their events, [the one used last]) for an array of that size on the current device."""
+    torch = _torch()
+    key = (nbytes >= _STAGE_LARGE, torch.cuda.current_device())      # an event belongs to a device
+    if key not in _stages:
+        stage_bytes, count = _STAGE_SHAPES[key[0]]
+        _stages[key] = ([torch.empty(stage_bytes, dtype=torch.uint8, pin_memory=True) for _ in range(count)],
+                        [torch.cuda.Event() for _ in range(count)], [0])
+    return _stages[key]
 
 
 def _upload(array, dtype):
@@ -100,25 +111,65 @@ def _upload(array, dtype):
     src = torch.from_numpy(array).reshape(-1)
     n = src.numel()
     out = torch.empty(n, dtype=torch.int32 if dtype is np.int32 else torch.float32, device="cuda")
-    large = 4 * n >= _STAGE_LARGE
-    stage_bytes, count = _STAGE_SHAPES[large]
     with _stage_lock:
-        key = (large, torch.cuda.current_device())      # an event belongs to a device
-        stage = _stages.get(key)
-        if stage is None:
-            stage = _stages[key] = ([torch.empty(stage_bytes, dtype=torch.uint8, pin_memory=True) for _ in range(count)],
-                                    [torch.cuda.Event() for _ in range(count)], [0])
-        bufs, events, turn = stage
-        chunk = stage_bytes // 4
+        bufs, events, turn = _staging(4 * n)
+        chunk = bufs[0].numel() // 4
         for off in range(0, n, chunk):
             m = min(chunk, n - off)
-            b = turn[0] = (turn[0] + 1) % count
+            b = turn[0] = (turn[0] + 1) % len(bufs)
             piece = bufs[b].view(out.dtype)[:m]
             events[b].synchronize()                      # the buffer's previous piece has left
             piece.copy_(src[off:off + m])
             out[off:off + m].copy_(piece, non_blocking=True)
             events[b].record()
     return out
+
+
+class _Downloads:
+    """32-bit device tensors as host tensors of given types, through the staging buffers: as many
+    pieces as there are buffers are under way from the start, and ``get(i)`` converts (on the host's
+    threads) what has arrived until tensor i is complete.  To be used as a context, tensors in order."""
+
+    def __init__(self, wanted):
+        torch = _torch()
+        self._out = [torch.empty(t.numel(), dtype=dtype) for t, dtype in wanted]
+        self._wanted = wanted
+
+    def __enter__(self):
+        _stage_lock.acquire()
+        try:
+            self._bufs, self._events, self._turn = _staging(max((4 * t.numel() for t, _ in self._wanted), default=0))
+            chunk = self._bufs[0].numel() // 4
+            self._todo = [(i, off, min(chunk, t.numel() - off)) for i, (t, _) in enumerate(self._wanted)
+                          for off in range(0, t.numel(), chunk)][::-1]
+            self._ahead = []
+            self._request()
+        except BaseException:
+            _stage_lock.release()
+            raise
+        return self
+
+    def _request(self):
+        while self._todo and len(self._ahead) < len(self._bufs):
+            i, off, m = self._todo.pop()
+            b = self._turn[0] = (self._turn[0] + 1) % len(self._bufs)
+            self._events[b].synchronize()                # (an upload's piece may be leaving it)
+            src = self._wanted[i][0]
+            piece = self._bufs[b].view(src.dtype)[:m]
+            piece.copy_(src[off:off + m], non_blocking=True)
+            self._events[b].record()
+            self._ahead.append((i, off, b, piece))
+
+    def get(self, i):
+        while self._ahead and self._ahead[0][0] <= i:
+            j, off, b, piece = self._ahead.pop(0)
+            self._events[b].synchronize()
+            self._out[j][off:off + len(piece)].copy_(piece)
+            self._request()
+        return self._out[i]
+
+    def __exit__(self, *exc):
+        _stage_lock.release()
 
 
 def _all_ones(data) -> bool:
@@ -357,27 +408,32 @@ class HybFormat:
     def to_numpy(self, with_values: bool = False):
         """The reference's return value of build_hyb_format (format_algos.py:361-385):
         per partition and bucket rows (R,), cols (R, W), mask (R, W) as int64 arrays."""
+        torch = _torch()
+        wanted = [(self.meta, torch.int64), (self.rows, torch.int64), (self.cols, torch.int64)]
+        if with_values:
+            wanted.append((self.vals, torch.float32))
         rows_nd, cols_nd, mask_nd, vals_nd = [], [], [], []
-        k = 0
+        mask = torch.empty(self.cols.numel(), dtype=torch.int64)
+        place = torch.arange(WIDTH_LIMIT)
+        buckets = [(k, w, int(self.ell_rows[k]), int(self.row_off[k]), int(self.slot_off[k]))
+                   for k, w in enumerate(self.flat_widths)]
+        with _Downloads(wanted) as down:
+            # the mask follows from the valid slots of every ELL row, in the low bits of its meta
+            # word; it is made while the columns arrive
+            lens = down.get(0).bitwise_and_(0x7FF)
+            for _, w, R, r0, s0 in buckets:
+                torch.lt(place[:w], lens[r0:r0 + R].view(R, 1), out=mask[s0:s0 + R * w].view(R, w))
+            rows, cols = down.get(1), down.get(2)
+            vals = down.get(3) if with_values else None
+        of_bucket = lambda flat, k, w, R, r0, s0: flat[s0:s0 + R * w].view(R, w).numpy()          # noqa: E731
+        at = iter(buckets)
         for ws in self.bucket_widths:
-            rp, cp, mp, vp = [], [], [], []
-            for w in ws:
-                R = int(self.ell_rows[k])
-                sl = self.slab(k)
-                rp.append(sl[0].cpu().numpy().astype(np.int64).reshape(R))
-                cp.append(sl[1].cpu().numpy().astype(np.int64).reshape(R, w))
-                vals = sl[2].cpu().numpy().reshape(R, w)
-                if self.mask is not None:
-                    mp.append(sl[4].cpu().numpy().astype(np.int64).reshape(R, w))
-                else:
-                    lens = (sl[3].cpu().numpy() & 0x7FF).reshape(R, 1)
-                    mp.append((np.arange(w).reshape(1, w) < lens).astype(np.int64))
-                vp.append(vals)
-                k += 1
-            rows_nd.append(rp)
-            cols_nd.append(cp)
-            mask_nd.append(mp)
-            vals_nd.append(vp)
+            mine = [next(at) for _ in ws]
+            rows_nd.append([rows[r0:r0 + R].numpy() for _, _, R, r0, _ in mine])
+            cols_nd.append([of_bucket(cols, *b) for b in mine])
+            mask_nd.append([of_bucket(mask, *b) for b in mine])
+            if with_values:
+                vals_nd.append([of_bucket(vals, *b) for b in mine])
         if with_values:
             return rows_nd, cols_nd, mask_nd, vals_nd
         return rows_nd, cols_nd, mask_nd
@@ -446,8 +502,7 @@ def build_hyb_format_device(g, bucket_widths, with_values: bool = True, with_mas
 def build_hyb_format(g, bucket_widths):
     """format_algos.py:226-385: (row_indices_nd, col_indices_nd, mask_nd), each a list over
     partitions of lists over buckets of numpy arrays with shapes (R,), (R, W), (R, W)."""
-    fmt = build_hyb_format_device(g, bucket_widths, with_values=False, with_mask=True)
-    return fmt.to_numpy()
+    return build_hyb_format_device(g, bucket_widths, with_values=False).to_numpy()
 
 
 # --------------------------------------------------------------------------- SpMM

@@ -150,3 +150,18 @@ def test_matrix_features_on_device(fa, torch):
         for key in want:
             if key.startswith(("avg", "std", "min_nnz_density", "max_nnz_density")):
                 assert got[key] == pytest.approx(want[key], rel=1e-9, abs=1e-15), key
+
+
+@pytest.mark.parametrize("n", [1, 524_287, 524_288, 524_289, 7 * 524_288 + 5, 16_777_216 + 3])
+def test_staged_transfers_round_trip(fa, n):
+    """One piece, whole pieces, a remainder, more pieces than buffers, the large buffers."""
+    import torch
+    ints = np.arange(n, dtype=np.int64) - n // 2
+    reals = np.linspace(-1.0, 1.0, n)
+    up = fa._upload(ints, np.int32), fa._upload(reals, np.float32), fa._upload(ints.astype(np.int16), np.int32)
+    assert [t.dtype for t in up] == [torch.int32, torch.float32, torch.int32]
+    with fa._Downloads([(up[0], torch.int64), (up[1], torch.float32), (up[2], torch.int64)]) as down:
+        back = [down.get(i).numpy() for i in range(3)]
+    np.testing.assert_array_equal(back[0], ints)
+    np.testing.assert_array_equal(back[1], reals.astype(np.float32))
+    np.testing.assert_array_equal(back[2], ints.astype(np.int16))
