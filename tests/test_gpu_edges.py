@@ -165,3 +165,29 @@ def test_staged_transfers_round_trip(fa, n):
     np.testing.assert_array_equal(back[0], ints)
     np.testing.assert_array_equal(back[1], reals.astype(np.float32))
     np.testing.assert_array_equal(back[2], ints.astype(np.int16))
+
+
+@pytest.mark.parametrize("nr,feat,b_dtype", [
+    *((nr, feat, b) for nr in (1, 31, 33, 65) for feat, b in ((32, "f32"), (64, "f32"), (96, "f32"), (128, "f32"), (256, "f32"),
+                                                              (512, "f32"), (1024, "f32"), (64, "bf16"), (320, "bf16"), (1024, "bf16"))),
+    (524_288, 64, "f32"), (524_289, 64, "f32"),          # the most rows in groups of 32, the fewest in groups of 64
+])
+def test_csr_product_at_group_edges(fa, torch, nr, feat, b_dtype):
+    """Rows that end a group of 32 or 64, empty rows at both ends and in a row, rows at and past the
+    length that a whole workgroup sums."""
+    import scipy.sparse as sp
+    rng = np.random.default_rng(nr + feat)
+    nc = 700
+    deg = rng.integers(0, 12, size=nr)
+    deg[rng.random(nr) < 0.3] = 0
+    deg[(7 * np.arange(5) + nr // 2) % nr] = (128, 129, 700, 127, 300)
+    deg[-1] = 0 if nr > 1 else 129
+    indptr = np.concatenate([[0], np.cumsum(deg)]).astype(np.int32)
+    row = np.repeat(np.arange(nr), deg)
+    key = np.sort(row * nc + (row * 13 + 31 * (np.arange(len(row)) - indptr[row])) % nc)      # 31 and 700 share no factor
+    vals = rng.uniform(-1, 1, size=len(key)).astype(np.float32)
+    A = sp.csr_matrix((vals.astype(np.float64), key % nc, indptr), shape=(nr, nc))
+    B = torch.from_numpy(rng.uniform(-1, 1, size=(nc, feat)).astype(np.float32)).cuda().to(torch.bfloat16 if b_dtype == "bf16" else torch.float32)
+    got = fa.spmm_csr(MTX.from_csr(indptr, (key % nc).astype(np.int32), (nr, nc), data=vals), B, b_dtype).cpu().numpy()
+    Bh = B.float().cpu().numpy().astype(np.float64)
+    assert (np.abs(got - A @ Bh) <= 1e-5 * (abs(A) @ np.abs(Bh)) + 1e-30).all()
