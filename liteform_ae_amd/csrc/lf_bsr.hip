@@ -5,24 +5,28 @@
 // 16x16x16 fragments (playground_pipline/format_algos.py:1182-1643; any block size that is a
 // multiple of 16 there, format_algos.py:1581-1582; 32 is what the driver passes,
 // proc05.spmm.end-to-end.py:205).  This is the one place of the library where dense-block
-// matrix-core work is the right shape; it is still HBM-bound (2 KiB of A and 32 rows of X per
-// 32x32xF block product: ~26 flop/byte at F = 128), so the kernels are organised around
-// coalesced loads, not around MFMA occupancy.
+// matrix-core work is the right shape; it is still bound by memory (2 KiB of A and 32 rows of X
+// per 32x32xF block product: ~26 flop/byte at F = 128), so the kernel is organised around
+// keeping wide, coalesced loads in flight.
 //
-// One workgroup (4 wavefronts) per (block row, 128-feature tile); wavefront w owns features
-// [32w, 32w+32) of the tile.
-//   * blocks of 32 and 64: one 32x32 fp32 accumulator tile per 32 rows of the block row
-//     (v_mfma_f32_32x32x8_f16, BS / 8 K-steps per nonzero block);
-//   * blocks of 16: two 16x16 accumulator tiles (v_mfma_f32_16x16x16_f16, one K-step per
-//     nonzero block and tile).
-// The X tile needs four consecutive k (= four different rows of X) per lane, so it is loaded
-// row-wise with 16-byte accesses and transposed through LDS: stored as XT[feature][k], read
-// back as one 8-byte access; the next block's tile is in flight during the matrix
-// instructions (two LDS buffers).  A blocks of 16 rows are read straight from global memory in
-// the MFMA A layout (lane: one row, four consecutive k - 512 contiguous bytes per block);
-// larger blocks are staged through LDS with 16-byte loads.  The accumulators hold one feature and many rows
-// per lane; the result goes back through LDS so that a lane stores 16 contiguous bytes of one
-// row of Y instead of one 2-byte element per row.
+// A wavefront owns one block row and 128 features and needs neither LDS nor barriers.  It uses
+// v_mfma_f32_16x16x32_f16, whose B operand is eight k (rows of X) of one column per lane:
+//   * lane (kq = lane / 16, li = lane % 16) loads the rows k = 8 kq .. 8 kq + 7 of X at the
+//     features 8 li .. 8 li + 7, 16 bytes each: every load instruction reads four whole
+//     256-byte pieces of rows of X;
+//   * which column of the instruction a feature takes is free, so instruction f = 0..7 is
+//     given the features 8 li + f: the eight k of one of a lane's eight features are the same
+//     half of the same word of its eight loads, put together by four v_perm_b32;
+//   * the results of the eight instructions are then eight consecutive features of a row in
+//     one lane, which stores them as 16 bytes.
+// A operands are 16 bytes of a row of the block (8 kq ..), read in memory order.  Blocks of 16 are
+// taken in pairs - the upper half of the wavefront (kq >= 2) works on the second one -, blocks of 64 in two
+// steps of 32 columns.  The loads of the next step are under way during the products of this one.
+// The kernel before this transposed X through LDS in 2-byte stores, with a barrier and one block's
+// loads in flight per workgroup: 1M x 1M, 8 blocks per block row, N = 128, blocks of 16 / 32 / 64:
+// 0.517 / 0.424 / 0.533 -> 0.382 / 0.411 / 0.509 ms, N = 256, blocks of 32: 0.896 -> 0.758 (all at
+// 7 TB/s of A blocks and rows of X, what a gather that misses the L2s reaches); 40K x 40K, blocks of
+// 16, N = 200: 45 -> 20 us.
 #include <hip/hip_runtime.h>
 #include <hip/hip_fp16.h>
 
@@ -32,213 +36,116 @@
 
 namespace {
 
-constexpr int kFeatTile = 128;     // features per workgroup
-constexpr int kWgBsr = 256;
-constexpr int kYPad = 8;           // halves of padding per staged row of Y (keeps 16-byte reads aligned)
+constexpr int kFeatTile = 128;     // features per wavefront
+constexpr int kWgBsr = 256;        // four wavefronts, independent of each other
 
-typedef _Float16 half4_t __attribute__((ext_vector_type(4)));
-typedef float float16_t __attribute__((ext_vector_type(16)));
+typedef _Float16 half8_t __attribute__((ext_vector_type(8)));
 typedef float float4_t __attribute__((ext_vector_type(4)));
 
-// halves per XT row: BS + 4 keeps 8-byte reads aligned and spreads banks
-template <int BS> constexpr int xt_stride() { return BS + 4; }
-template <int BS> constexpr int lds_halves() {
-    const int xt = 2 * kFeatTile * xt_stride<BS>();
-    const int y = BS * (kFeatTile + kYPad);
-    return xt > y ? xt : y;
-}
+// What a wavefront loads for one step of 32 columns of A: eight rows of X and a row of each of A's
+// row tiles per lane.
+template <int BS> struct BsrStep {
+    static constexpr int kTiles = BS / 16;
+    uint4 x[8];
+    uint4 a[kTiles];
+};
 
-// The staged tile of Y, rows x 128 features, to global memory: 16 bytes per lane, 16 rows per pass.
-template <int BS>
-__device__ __forceinline__ void store_y_tile(const _Float16* s_y, _Float16* __restrict__ Y, size_t row0, int f0, int feat) {
-    const int tid = threadIdx.x;
-    const int vec = tid & 15;                // features 8 * vec .. + 7 of the tile
-    const int f = f0 + 8 * vec;
-    if (f >= feat) return;                   // feat is a multiple of 8: a vector is inside or outside
-#pragma unroll
-    for (int r = tid >> 4; r < BS; r += kWgBsr / 16) {
-        const uint4 v = *reinterpret_cast<const uint4*>(s_y + r * (kFeatTile + kYPad) + 8 * vec);
-        *reinterpret_cast<uint4*>(Y + (row0 + r) * feat + f) = v;
-    }
-}
-
-// Blocks of 32 (RH = 1) or 64 (RH = 2) rows and columns.  The A block goes through LDS as well:
-// read straight from global memory in the MFMA layout, a lane's 8 bytes lie a whole block row
-// (64 or 128 bytes) from its neighbour's, one cache line per lane or pair of lanes, and all four
-// wavefronts fetch the same block (64 x 64 blocks, N = 128: 1.13 ms that way).
 template <int BS>
 __global__ void __launch_bounds__(kWgBsr)
 bsr_spmm_kernel(const int32_t* __restrict__ indptr, const int32_t* __restrict__ indices,
                 const _Float16* __restrict__ data, const _Float16* __restrict__ X,
-                _Float16* __restrict__ Y, int feat) {
-    constexpr int RH = BS / 32;              // 32-row halves of a block row
-    constexpr int KP = xt_stride<BS>();
-    constexpr int AP = BS + 4;               // halves per staged row of A
-    constexpr int AV = BS * BS / 8 / kWgBsr > 0 ? BS * BS / 8 / kWgBsr : 1;   // 16-byte vectors of A per thread
-    __shared__ __align__(16) _Float16 s_raw[lds_halves<BS>()];
-    __shared__ __align__(16) _Float16 s_a[2][BS * AP];
-    auto xt_buf = [&](int buf) { return s_raw + buf * kFeatTile * KP; };
-
-    const int brow = blockIdx.x;
-    const int f0 = blockIdx.y * kFeatTile;
-    const int tid = threadIdx.x;
-    const int wave = tid >> 6, lane = tid & 63;
-    const int li = lane & 31, kq = lane >> 5;
-
-    // cooperative X-tile load: thread t reads rows t/8 (+32) of the block, two 16-byte vectors each
-    const int xr = tid >> 3;                 // 0..31: row inside the block (= k)
-    const int xv = tid & 7;                  // vector 0..7 -> features 8*xv and 64 + 8*xv
-    const bool in0 = f0 + 8 * xv < feat, in1 = f0 + 64 + 8 * xv < feat;
-    // cooperative A-block load: 16-byte vectors in memory order (BS / 8 per row)
-    const bool a_on = tid < BS * BS / 8;     // 32 x 32: the first 128 threads
-
-    float16_t acc[RH];
-#pragma unroll
-    for (int h = 0; h < RH; ++h)
-#pragma unroll
-        for (int v = 0; v < 16; ++v) acc[h][v] = 0.f;
-
+                _Float16* __restrict__ Y, int feat, int n_tiles, long long n_units) {
+    constexpr int RT = BS / 16;                          // row tiles of a block row
+    constexpr int SPB = BS == 64 ? 2 : 1;                // steps per block
+    constexpr int BPS = BS == 16 ? 2 : 1;                // blocks per step
+    const int lane = threadIdx.x & 63, li = lane & 15, kq = lane >> 4;
+    // the feature tiles of a block row go to neighbouring wavefronts, which read the same blocks of A
+    const long long unit = (long long)blockIdx.x * (kWgBsr / 64) + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    if (unit >= n_units) return;
+    const int brow = (int)(unit / n_tiles);
+    const int f = (int)(unit % n_tiles) * kFeatTile + 8 * li;
+    const bool on = f < feat;                            // feat is a multiple of 8: a vector is inside or outside
     const int jb = indptr[brow], je = indptr[brow + 1];
-    uint4 x0[RH], x1[RH], av[AV];
-    auto load_x = [&](int j) {
-        const _Float16* src = X + ((size_t)indices[j] * BS + xr) * feat + f0 + 8 * xv;
+
+    float4_t acc[RT][8];
 #pragma unroll
-        for (int h = 0; h < RH; ++h) {
-            x0[h] = in0 ? *reinterpret_cast<const uint4*>(src + (size_t)32 * h * feat) : make_uint4(0, 0, 0, 0);
-            x1[h] = in1 ? *reinterpret_cast<const uint4*>(src + (size_t)32 * h * feat + 64) : make_uint4(0, 0, 0, 0);
-        }
-        const uint4* asrc = reinterpret_cast<const uint4*>(data + (size_t)j * BS * BS);
+    for (int t = 0; t < RT; ++t)
 #pragma unroll
-        for (int i = 0; i < AV; ++i)
-            if (a_on) av[i] = asrc[tid + i * kWgBsr];
+        for (int i = 0; i < 8; ++i) acc[t][i] = float4_t{0.f, 0.f, 0.f, 0.f};
+
+    const int n_steps = BPS == 2 ? (je - jb + 1) / 2 : (je - jb) * SPB;
+    // Every load below is unconditional - lanes past the last feature read what the tile's first lane
+    // reads, steps past the end the last block - so that the wait for one step's loads need not
+    // allow for a path on which the next step's were not issued.
+    const int f_in = on ? f : f - 8 * li;
+    // step s: block jb + s / SPB, columns 32 * (s % SPB) ..; or blocks jb + 2 s and jb + 2 s + 1
+    auto block_of = [&](int s, int half) { return min(BPS == 2 ? jb + 2 * s + half : jb + s / SPB, je - 1); };
+    struct Cols { int c0, c1; };
+    auto cols_of = [&](int s) { return Cols{indices[block_of(s, 0)], BPS == 2 ? indices[block_of(s, 1)] : 0}; };
+    auto load = [&](int s, Cols c, BsrStep<BS>& st) {
+        const bool second = BPS == 2 && kq >= 2;
+        const int k0 = BPS == 2 ? 8 * (kq & 1) : 32 * (s % SPB) + 8 * kq;
+        const _Float16* src = X + ((size_t)(second ? c.c1 : c.c0) * BS + k0) * feat + f_in;
+#pragma unroll
+        for (int r = 0; r < 8; ++r) st.x[r] = *reinterpret_cast<const uint4*>(src + (size_t)r * feat);
+        const int j = second ? block_of(s, 1) : block_of(s, 0);
+        const _Float16* blk = data + (size_t)j * BS * BS + li * BS + k0;
+#pragma unroll
+        for (int t = 0; t < RT; ++t) st.a[t] = *reinterpret_cast<const uint4*>(blk + 16 * t * BS);
+        // an odd last block of 16 has no partner
+        if (BPS == 2 && second && jb + 2 * s + 1 >= je) st.a[0] = make_uint4(0, 0, 0, 0);
     };
-    auto store_lds = [&](int buf) {
-        _Float16* dst = xt_buf(buf);
+    auto multiply = [&](const BsrStep<BS>& st) {
 #pragma unroll
-        for (int h = 0; h < RH; ++h) {
-            const _Float16* h0 = reinterpret_cast<const _Float16*>(&x0[h]);
-            const _Float16* h1 = reinterpret_cast<const _Float16*>(&x1[h]);
+        for (int i = 0; i < 8; ++i) {                    // feature f + i
+            union { uint32_t w[4]; half8_t h; } b;
+            const uint32_t sel = i & 1 ? 0x07060302u : 0x05040100u;
 #pragma unroll
-            for (int i = 0; i < 8; ++i) {
-                dst[(8 * xv + i) * KP + 32 * h + xr] = h0[i];
-                dst[(64 + 8 * xv + i) * KP + 32 * h + xr] = h1[i];
+            for (int q = 0; q < 4; ++q) {
+                const uint32_t lo = (&st.x[2 * q].x)[i >> 1], hi = (&st.x[2 * q + 1].x)[i >> 1];
+                b.w[q] = __builtin_amdgcn_perm(hi, lo, sel);
+            }
+#pragma unroll
+            for (int t = 0; t < RT; ++t) {
+                union { uint4 w; half8_t h; } a;
+                a.w = st.a[t];
+                acc[t][i] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a.h, b.h, acc[t][i], 0, 0, 0);
             }
         }
-#pragma unroll
-        for (int i = 0; i < AV; ++i) {
-            if (!a_on) continue;
-            const int v = tid + i * kWgBsr;                  // vector v: row v / (BS / 8), halves 8 * (v % (BS / 8)) ..
-            _Float16* d = s_a[buf] + (v / (BS / 8)) * AP + 8 * (v % (BS / 8));
-            *reinterpret_cast<uint2*>(d) = make_uint2(av[i].x, av[i].y);           // (rows are 8-byte aligned: AP = BS + 4)
-            *reinterpret_cast<uint2*>(d + 4) = make_uint2(av[i].z, av[i].w);
-        }
     };
-
-    if (jb < je) {
-        load_x(jb);
-        store_lds(0);
-    }
-    __syncthreads();
-    for (int j = jb; j < je; ++j) {
-        const int buf = (j - jb) & 1;
-        if (j + 1 < je) load_x(j + 1);                       // next tiles in flight during the MFMAs
-        const _Float16* ablk = s_a[buf] + li * AP + 4 * kq;
-        const _Float16* xt = xt_buf(buf) + (32 * wave + li) * KP + 4 * kq;
-#pragma unroll
-        for (int s = 0; s < BS / 8; ++s) {
-            const half4_t b = *reinterpret_cast<const half4_t*>(xt + 8 * s);
-#pragma unroll
-            for (int h = 0; h < RH; ++h) {
-                const half4_t a = *reinterpret_cast<const half4_t*>(ablk + 32 * h * AP + 8 * s);
-                acc[h] = __builtin_amdgcn_mfma_f32_32x32x8f16(a, b, acc[h], 0, 0, 0);
-            }
+    if (n_steps > 0) {
+        BsrStep<BS> s0, s1;
+        Cols even = cols_of(0), odd = cols_of(1);
+        load(0, even, s0);
+        int s = 0;
+        for (; s + 2 < n_steps; s += 2) {
+            load(s + 1, odd, s1);
+            even = cols_of(s + 2);
+            multiply(s0);
+            load(s + 2, even, s0);
+            odd = cols_of(s + 3);
+            multiply(s1);
         }
-        if (j + 1 < je) store_lds(buf ^ 1);
-        __syncthreads();
-    }
-
-    // D layout of the 32x32 MFMA: lane holds column li, rows 8*(v/4) + 4*kq + v%4.  (The last
-    // barrier of the loop - or the one before it for an empty block row - has retired every read
-    // of the X tiles, so the staging buffer can take their place.)
-    _Float16* s_y = s_raw;
-#pragma unroll
-    for (int h = 0; h < RH; ++h)
-#pragma unroll
-        for (int v = 0; v < 16; ++v) {
-            const int row = 32 * h + 8 * (v >> 2) + 4 * kq + (v & 3);
-            s_y[row * (kFeatTile + kYPad) + 32 * wave + li] = (_Float16)acc[h][v];
+        if (s + 1 < n_steps) {
+            load(s + 1, odd, s1);
+            multiply(s0);
+            multiply(s1);
+        } else {
+            multiply(s0);
         }
-    __syncthreads();
-    store_y_tile<BS>(s_y, Y, (size_t)brow * BS, f0, feat);
-}
-
-// Blocks of 16 rows and columns: two 16x16 accumulator tiles per wavefront.
-__global__ void __launch_bounds__(kWgBsr)
-bsr16_spmm_kernel(const int32_t* __restrict__ indptr, const int32_t* __restrict__ indices,
-                  const _Float16* __restrict__ data, const _Float16* __restrict__ X,
-                  _Float16* __restrict__ Y, int feat) {
-    constexpr int BS = 16;
-    constexpr int KP = xt_stride<BS>();
-    __shared__ __align__(16) _Float16 s_raw[lds_halves<BS>()];
-    auto xt_buf = [&](int buf) { return s_raw + buf * kFeatTile * KP; };
-
-    const int brow = blockIdx.x;
-    const int f0 = blockIdx.y * kFeatTile;
-    const int tid = threadIdx.x;
-    const int wave = tid >> 6, lane = tid & 63;
-    const int li = lane & 15, kq = lane >> 4;            // row (A) / column (B, D) and group of four k
-
-    // cooperative X-tile load: thread t reads row t/16 of the block, one 16-byte vector
-    const int xr = tid >> 4;                 // 0..15
-    const int xv = tid & 15;                 // features 8*xv .. + 7
-    const bool in0 = f0 + 8 * xv < feat;
-
-    float4_t acc[2];
-#pragma unroll
-    for (int t = 0; t < 2; ++t)
-#pragma unroll
-        for (int v = 0; v < 4; ++v) acc[t][v] = 0.f;
-
-    const int jb = indptr[brow], je = indptr[brow + 1];
-    uint4 x0 = make_uint4(0, 0, 0, 0);
-    auto load_x = [&](int j) {
-        const _Float16* src = X + ((size_t)indices[j] * BS + xr) * feat + f0 + 8 * xv;
-        x0 = in0 ? *reinterpret_cast<const uint4*>(src) : make_uint4(0, 0, 0, 0);
-    };
-    auto store_xt = [&](int buf) {
-        _Float16* dst = xt_buf(buf);
-        const _Float16* h0 = reinterpret_cast<const _Float16*>(&x0);
-#pragma unroll
-        for (int i = 0; i < 8; ++i) dst[(8 * xv + i) * KP + xr] = h0[i];
-    };
-
-    if (jb < je) {
-        load_x(jb);
-        store_xt(0);
     }
-    __syncthreads();
-    for (int j = jb; j < je; ++j) {
-        const int buf = (j - jb) & 1;
-        if (j + 1 < je) load_x(j + 1);
-        const half4_t a = *reinterpret_cast<const half4_t*>(data + (size_t)j * BS * BS + li * BS + 4 * kq);
+
+    // D layout of the instruction: lane holds column li, rows 4 kq + v
+    if (!on) return;
 #pragma unroll
-        for (int t = 0; t < 2; ++t) {
-            const half4_t b = *reinterpret_cast<const half4_t*>(xt_buf(buf) + (32 * wave + 16 * t + li) * KP + 4 * kq);
-            acc[t] = __builtin_amdgcn_mfma_f32_16x16x16f16(a, b, acc[t], 0, 0, 0);
+    for (int t = 0; t < RT; ++t)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+            half8_t o;
+#pragma unroll
+            for (int i = 0; i < 8; ++i) o[i] = (_Float16)acc[t][i][v];
+            *reinterpret_cast<half8_t*>(Y + ((size_t)brow * BS + 16 * t + 4 * kq + v) * feat + f) = o;
         }
-        if (j + 1 < je) store_xt(buf ^ 1);
-        __syncthreads();
-    }
-
-    // D layout of the 16x16 MFMA: lane holds column li, rows 4*kq + v
-    _Float16* s_y = s_raw;
-#pragma unroll
-    for (int t = 0; t < 2; ++t)
-#pragma unroll
-        for (int v = 0; v < 4; ++v)
-            s_y[(4 * kq + v) * (kFeatTile + kYPad) + 32 * wave + 16 * t + li] = (_Float16)acc[t][v];
-    __syncthreads();
-    store_y_tile<BS>(s_y, Y, (size_t)brow * BS, f0, feat);
 }
 
 }  // namespace
@@ -259,13 +166,14 @@ int lf_bsr_spmm_trusted(const int32_t* d_indptr, const int32_t* d_indices, const
     LF_REQUIRE(d_indptr && d_X && d_Y, LF_ERR_INVALID, "null argument");
     LF_REQUIRE((uintptr_t)d_X % 16 == 0 && (uintptr_t)d_Y % 16 == 0 && (uintptr_t)d_data % 16 == 0, LF_ERR_INVALID,
                "X, Y and the block data must be 16-byte aligned");
-    const dim3 grid((unsigned)num_block_rows, (unsigned)((feat_size + kFeatTile - 1) / kFeatTile));
+    const int n_tiles = (feat_size + kFeatTile - 1) / kFeatTile;
+    const long long units = (long long)num_block_rows * n_tiles, groups = lf::ceil_div(units, kWgBsr / 64);
+    LF_REQUIRE(groups < (1ll << 31), LF_ERR_UNSUPPORTED, "too many block rows and features");
     const _Float16* data = (const _Float16*)d_data;
     const _Float16* X = (const _Float16*)d_X;
     _Float16* Y = (_Float16*)d_Y;
-    if (block_size == 16) bsr16_spmm_kernel<<<grid, kWgBsr, 0, s>>>(d_indptr, d_indices, data, X, Y, feat_size);
-    else if (block_size == 32) bsr_spmm_kernel<32><<<grid, kWgBsr, 0, s>>>(d_indptr, d_indices, data, X, Y, feat_size);
-    else bsr_spmm_kernel<64><<<grid, kWgBsr, 0, s>>>(d_indptr, d_indices, data, X, Y, feat_size);
+    const auto kernel = block_size == 16 ? bsr_spmm_kernel<16> : block_size == 32 ? bsr_spmm_kernel<32> : bsr_spmm_kernel<64>;
+    kernel<<<(unsigned)groups, kWgBsr, 0, s>>>(d_indptr, d_indices, data, X, Y, feat_size, n_tiles, units);
     LF_HIP(hipGetLastError());
     return LF_OK;
 }

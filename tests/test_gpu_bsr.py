@@ -129,3 +129,16 @@ def test_driver_block_and_csr_branches(fa, torch, monkeypatch):
     assert (df["format"] == "BSR").all() and (df["time_exe_our(ms)"] > 0).all() and (df["num_parts"] == 0).all()
     df = driver.run_end_to_end([g], feat_sizes=(64,), select_format=lambda m: "CSR")
     assert (df["format"] == "CSR").all() and (df["time_exe_our(ms)"] > 0).all()
+
+
+@pytest.mark.parametrize("bs", [16, 32, 64])
+@pytest.mark.parametrize("feat", [120, 136, 392])
+def test_every_short_block_row(fa, torch, feat, bs):
+    """Block rows of 0 to 9 blocks - every way the two steps in flight can start and end, odd
+    partners of 16-row blocks - and feature tiles that are nearly full, nearly empty and several."""
+    rng = np.random.default_rng(bs + feat)
+    counts = rng.permutation(10)
+    indptr = np.concatenate([[0], np.cumsum(counts)]).astype(np.int32)
+    indices = np.concatenate([np.sort(rng.choice(12, size=n, replace=False)) for n in counts]).astype(np.int32)
+    data = rng.uniform(-1, 1, size=(len(indices), bs, bs)).astype(np.float16).astype(np.float32)
+    check(fa, torch, sp.bsr_matrix((data, indices, indptr), shape=(10 * bs, 12 * bs)), feat)
