@@ -39,6 +39,10 @@ namespace {
 constexpr int kFeatTile = 128;     // features per wavefront
 constexpr int kWgBsr = 256;        // four wavefronts, independent of each other
 
+// A Y of this size or more is stored past the caches, which leaves them to X (128K x 128K, blocks of 32,
+// N = 512: 104 -> 96 us; 1M x 1M, N = 256: 759 -> 734); a smaller one the next operation may find there.
+constexpr int64_t kStreamYBytes = 64ll << 20;
+
 typedef _Float16 half8_t __attribute__((ext_vector_type(8)));
 typedef float float4_t __attribute__((ext_vector_type(4)));
 
@@ -54,7 +58,7 @@ template <int BS>
 __global__ void __launch_bounds__(kWgBsr)
 bsr_spmm_kernel(const int32_t* __restrict__ indptr, const int32_t* __restrict__ indices,
                 const _Float16* __restrict__ data, const _Float16* __restrict__ X,
-                _Float16* __restrict__ Y, int feat, int n_tiles, long long n_units) {
+                _Float16* __restrict__ Y, int feat, int n_tiles, long long n_units, int stream_y) {
     constexpr int RT = BS / 16;                          // row tiles of a block row
     constexpr int SPB = BS == 64 ? 2 : 1;                // steps per block
     constexpr int BPS = BS == 16 ? 2 : 1;                // blocks per step
@@ -144,7 +148,12 @@ bsr_spmm_kernel(const int32_t* __restrict__ indptr, const int32_t* __restrict__ 
             half8_t o;
 #pragma unroll
             for (int i = 0; i < 8; ++i) o[i] = (_Float16)acc[t][i][v];
-            *reinterpret_cast<half8_t*>(Y + ((size_t)brow * BS + 16 * t + 4 * kq + v) * feat + f) = o;
+            half8_t* dst = reinterpret_cast<half8_t*>(Y + ((size_t)brow * BS + 16 * t + 4 * kq + v) * feat + f);
+            // (through an integer, or the compiler folds the two stores into one ordinary store)
+            if (stream_y)
+                __builtin_nontemporal_store(o, reinterpret_cast<half8_t __attribute__((address_space(1)))*>(reinterpret_cast<uintptr_t>(dst)));
+            else
+                *dst = o;
         }
 }
 
@@ -173,7 +182,8 @@ int lf_bsr_spmm_trusted(const int32_t* d_indptr, const int32_t* d_indices, const
     const _Float16* X = (const _Float16*)d_X;
     _Float16* Y = (_Float16*)d_Y;
     const auto kernel = block_size == 16 ? bsr_spmm_kernel<16> : block_size == 32 ? bsr_spmm_kernel<32> : bsr_spmm_kernel<64>;
-    kernel<<<(unsigned)groups, kWgBsr, 0, s>>>(d_indptr, d_indices, data, X, Y, feat_size, n_tiles, units);
+    kernel<<<(unsigned)groups, kWgBsr, 0, s>>>(d_indptr, d_indices, data, X, Y, feat_size, n_tiles, units,
+                                              (int64_t)num_block_rows * block_size * feat_size * 2 >= kStreamYBytes);
     LF_HIP(hipGetLastError());
     return LF_OK;
 }
