@@ -221,10 +221,11 @@ int lf_hyb_build(const int32_t* d_indptr, const int32_t* d_indices, const float*
  * bench_hyb_with_config builds and launches (format_algos.py:388-605): one launch per
  * column partition (and per feature window, lf_spmm_set_windows) walks every bucket of that
  * partition - "fused" here means the buckets of a partition, not the partitions; rows served
- * with shared gathers and the second stage of very long rows have small launches of their
- * own behind it.  Partitions run in ascending order on the stream, partition 0 stores and
- * later partitions add, so the result does not depend on scheduling and no atomics are used.
- * C needs no clearing.
+ * with shared gathers, and rows of very many chunks, have small launches of their own behind
+ * it.  Partitions run in ascending order on the stream, partition 0 stores and later partitions
+ * add, the chunks of a long row are added up in a fixed order by whichever comes last: the
+ * result does not depend on scheduling.  C needs no clearing.  A plan holds partial rows and their
+ * counters: its runs must not overlap.
  *
  * A bucket is described the way the reference passes it to the kernel
  * (format_algos.py:552-578: values float32, rows int32, cols int32 row-major), plus the

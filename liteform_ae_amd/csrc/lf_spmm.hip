@@ -16,8 +16,8 @@
 //     shuffles instead;
 //   * a source row split over several ELL rows is summed by one owner; rows longer than
 //     kCoopSlots are reduced by a whole workgroup, kChunkSlots at a time: a row that fits one
-//     chunk is written directly, a longer one leaves one partial row per chunk and a small
-//     second kernel adds the partials in chunk order;
+//     chunk is written directly, a longer one leaves one partial row per chunk, which the
+//     workgroup that comes last adds up (rows of very many chunks: a small second kernel);
 //   * partitions run as consecutive launches: partition 0 stores every output row (rows it
 //     does not touch are cleared by the same launch), later partitions add.  Nothing
 //     depends on scheduling, so results are bit-reproducible, and there are no atomics.
@@ -390,6 +390,17 @@ __device__ __forceinline__ void run_zero_tile(const Group& g, long long tile, co
     for (int r = sw; r < n; r += SW) store_row<LPR, CH, VEC>(a.C, g.rows[e0 + r], ln, zero, a.accumulate & kStreamC);
 }
 
+// Two floats at agent scope: stored to, and read from, where all XCDs see them.
+__device__ __forceinline__ void store_pair_agent(float* dst, float x, float y) {
+    const unsigned long long v = (unsigned long long)__float_as_uint(x) | (unsigned long long)__float_as_uint(y) << 32;
+    __hip_atomic_store(reinterpret_cast<unsigned long long*>(dst), v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ void load_pair_agent(const float* src, float& x, float& y) {
+    const unsigned long long v = __hip_atomic_load(reinterpret_cast<const unsigned long long*>(src), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    x = __uint_as_float((unsigned int)v);
+    y = __uint_as_float((unsigned int)(v >> 32));
+}
+
 // One chunk of a heavy source row: the workgroup's sub-waves take consecutive slices of
 // the chunk, their sums are combined through LDS in sub-wave order.
 template <int LPR, int CH, typename BT>
@@ -414,28 +425,76 @@ __device__ __forceinline__ void run_chunk_tile(const Group& g, long long tile, f
 #pragma unroll
         for (int i = 0; i < VEC; ++i) s_red[((sw * CH + c) * LPR + sl) * VEC + i] = acc.v[c][i];
     __syncthreads();
+    if (tid >= 64) return;
+    acc.clear();
     if (sw == 0) {
-        Acc<CH, VEC> sum;
-        sum.clear();
 #pragma unroll
         for (int c = 0; c < CH; ++c)
             for (int s = 0; s < SW; ++s)
 #pragma unroll
-                for (int i = 0; i < VEC; ++i) sum.v[c][i] += s_red[((s * CH + c) * LPR + sl) * VEC + i];
-        if (ck.partial < 0) {
-            store_row<LPR, CH, VEC>(a.C, ck.row, ln, sum, a.accumulate);
-        } else {
+                for (int i = 0; i < VEC; ++i) acc.v[c][i] += s_red[((s * CH + c) * LPR + sl) * VEC + i];
+    }
+    if (ck.partial < 0) {                            // the row's only chunk
+        if (sw == 0) store_row<LPR, CH, VEC>(a.C, ck.row, ln, acc, a.accumulate);
+        return;
+    }
+    // The first wavefront leaves the chunk's partial row, counts it, and adds the row's partial rows
+    // up if it was the last: sub-wave s takes partial rows s, s + n_sub, ..., the sub-waves' sums are
+    // added in sub-wave order - the same order whoever comes last.  Partial rows are written and read at
+    // agent scope, past the L2s that the XCDs do not share, and are complete (the wait) before they
+    // are counted.  A release and acquire at the counter would do the same by writing back and invalidating the
+    // whole L2 of the XCD, once per chunk: 500k x 2M matrix with 4911 partial rows 1.34 -> 1.72 ms.
+    // (170K-row graph with 27 such rows: one launch less, 85.7 -> 81.9 us a product.)  Where a row has
+    // many chunks they are short and the wait and the count would hold up their workgroups more than
+    // a launch costs (that matrix: 1.37 ms): those rows are left to spmm_finalize_wide_kernel.
+    if (sw == 0) {
 #pragma unroll
-            for (int c = 0; c < CH; ++c) {
-                if (!ln.on[c]) continue;
-                float* dst = a.partials + (size_t)ck.partial * a.feat + ln.f[c];
+        for (int c = 0; c < CH; ++c) {
+            if (!ln.on[c]) continue;
+            float* dst = a.partials + (size_t)ck.partial * a.feat + ln.f[c];
 #pragma unroll
-                for (int i = 0; i < VEC; i += 4)
-                    *reinterpret_cast<float4*>(dst + i) =
-                        make_float4(sum.v[c][i], sum.v[c][i + 1], sum.v[c][i + 2], sum.v[c][i + 3]);
-            }
+            for (int i = 0; i < VEC; i += 2) store_pair_agent(dst + i, acc.v[c][i], acc.v[c][i + 1]);
         }
     }
+    HeavyRow* hr = a.heavy + ck.heavy;
+    const int n = hr->n_partials;
+    if (n > kWideFinalPartials) return;
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    int before = 0;
+    if (tid == 0) before = __hip_atomic_fetch_add(&hr->done, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (__builtin_amdgcn_readfirstlane(before) != n - 1) return;
+    if (tid == 0) hr->done = 0;                      // for the next launch
+    constexpr int kSub = 64 / LPR;
+    constexpr int U = VEC * CH <= 8 ? 8 : 2;         // partial rows in flight per sub-wave
+    acc.clear();
+    for (int k0 = sw; k0 < n; k0 += kSub * U) {
+        float x[U][CH][VEC];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int k = min(k0 + u * kSub, n - 1); // (clamped loads, masked below)
+#pragma unroll
+            for (int c = 0; c < CH; ++c) {
+                const float* src = a.partials + (size_t)(hr->partial_begin + k) * a.feat + (ln.on[c] ? ln.f[c] : 0);
+#pragma unroll
+                for (int i = 0; i < VEC; i += 2) load_pair_agent(src + i, x[u][c][i], x[u][c][i + 1]);
+            }
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const bool in = k0 + u * kSub < n;
+#pragma unroll
+            for (int c = 0; c < CH; ++c)
+#pragma unroll
+                for (int i = 0; i < VEC; ++i) acc.v[c][i] += in ? x[u][c][i] : 0.f;
+        }
+    }
+    Acc<CH, VEC> sum = acc;
+    for (int s = 1; s < kSub; ++s)
+#pragma unroll
+        for (int c = 0; c < CH; ++c)
+#pragma unroll
+            for (int i = 0; i < VEC; ++i) sum.v[c][i] += __shfl(acc.v[c][i], s * LPR + sl);
+    if (sw == 0) store_row<LPR, CH, VEC>(a.C, ck.row, ln, sum, a.accumulate);
 }
 
 // ------------------------------------------------------------------------------------
@@ -480,34 +539,7 @@ spmm_partition_kernel(LaunchArgs a) {
     }
 }
 
-// Adds the partial rows of every heavy source row in chunk order and writes the row (rows with
-// more than kWideFinalPartials partial rows are left to spmm_finalize_wide_kernel).
-template <int LPR, int CH, typename BT>
-__global__ void __launch_bounds__(kWG)
-spmm_finalize_kernel(const HeavyRow* __restrict__ heavy, int n_heavy, LaunchArgs a) {
-    constexpr int VEC = Dense<BT>::kVec;
-    constexpr int SW = kWG / LPR;
-    const int sw = threadIdx.x / LPR, sl = threadIdx.x % LPR;
-    const Lane<LPR, CH, VEC> ln(sl, a.feat, a.ldb, a.ldc);
-    for (int h = blockIdx.x * SW + sw; h < n_heavy; h += gridDim.x * SW) {
-        const HeavyRow hr = heavy[h];
-        if (hr.n_partials > kWideFinalPartials) continue;
-        Acc<CH, VEC> acc;
-        acc.clear();
-        for (int k = 0; k < hr.n_partials; ++k) {
-#pragma unroll
-            for (int c = 0; c < CH; ++c) {
-                if (!ln.on[c]) continue;
-                const float* src = a.partials + (size_t)(hr.partial_begin + k) * a.feat + ln.f[c];
-#pragma unroll
-                for (int i = 0; i < VEC; ++i) acc.v[c][i] += src[i];
-            }
-        }
-        store_row<LPR, CH, VEC>(a.C, hr.row, ln, acc, a.accumulate);
-    }
-}
-
-// The same for rows with many partial rows (dense rows cut into short chunks): one workgroup per
+// Rows of many partial rows (dense rows cut into short chunks; more than kWideFinalPartials): one workgroup per
 // row, sub-wave s adds partial rows s, s + SW, s + 2 SW, ... four at a time, and the sub-waves'
 // sums are added in sub-wave order - a fixed order, so the result does not depend on scheduling.
 template <int LPR, int CH, typename BT>
@@ -1315,6 +1347,8 @@ plan_chunks_kernel(const int32_t* __restrict__ rows, const int32_t* __restrict__
             ck.partial = several ? partial_base + p0 + i : -1;
             ck.row = row;
             ck.first_col = cols[ck.slot_begin];
+            ck.heavy = heavy_base + h;
+            ck.pad_ = 0;
             chunks[c0 + i] = ck;
         }
         if (several) heavy[heavy_base + h] = HeavyRow{row, partial_base + p0, x.n_chunks, 0};
@@ -1380,8 +1414,8 @@ struct lf_spmm_plan {
         int cell_begin = 0, n_cell_buckets = 0, cell_grid = 0; // buckets rewritten as cells
         long long tiles = 0;
         int heavy_begin = 0, n_heavy = 0;
-        bool stream_c = false;       // store C past the caches (when this is the run's last partition)
         bool wide_rows = false;      // some rows have more than kWideFinalPartials partial rows
+        bool stream_c = false;       // store C past the caches (when this is the run's last partition)
     };
     std::vector<Launch> launches;
     bool stream_slabs = false;          // read the slabs non-temporally
@@ -1423,7 +1457,6 @@ using RowGroupFn = void (*)(const MergedBucket*, int, LaunchArgs);
 
 struct KernelSet {
     KernelFn tiles = nullptr;
-    FinalFn finalize = nullptr;
     FinalFn finalize_wide = nullptr;
     CsrFn csr = nullptr;
     RowGroupFn rowgroup = nullptr;   // one 16-byte chunk per lane only
@@ -1436,12 +1469,10 @@ template <int LPR, int CH> void pick_kernels(int dtype, KernelSet* k) {
     }
     if (dtype == LF_DTYPE_BF16) {
         k->tiles = spmm_partition_kernel<LPR, CH, bf16_t>;
-        k->finalize = spmm_finalize_kernel<LPR, CH, bf16_t>;
         k->finalize_wide = spmm_finalize_wide_kernel<LPR, CH, bf16_t>;
         k->csr = csr_spmm_kernel<LPR, CH, bf16_t>;
     } else {
         k->tiles = spmm_partition_kernel<LPR, CH, float>;
-        k->finalize = spmm_finalize_kernel<LPR, CH, float>;
         k->finalize_wide = spmm_finalize_wide_kernel<LPR, CH, float>;
         k->csr = csr_spmm_kernel<LPR, CH, float>;
     }
@@ -2075,6 +2106,7 @@ int lf_spmm_run(lf_spmm_plan* plan, const void* d_B, float* d_C, lf_stream_t str
             a.B = (const char*)d_B + (size_t)w * plan->feat * b_elem;
             a.C = d_C + (size_t)w * plan->feat;
             a.partials = plan->d_partials;
+            a.heavy = plan->d_heavy;
             if (L.grid > 0) {
                 ks.tiles<<<L.grid, kWG, L.dyn_lds, s>>>(a);
                 LF_HIP(hipGetLastError());
@@ -2088,15 +2120,9 @@ int lf_spmm_run(lf_spmm_plan* plan, const void* d_B, float* d_C, lf_stream_t str
                                               a.B, a.C, a.feat, a.ldb, a.ldc, a.accumulate, s))
                     return rc;
             }
-            if (L.n_heavy > 0) {
-                const int sw = kWG / plan->lpr;
-                const int fgrid = std::min((L.n_heavy + sw - 1) / sw, 1024);
-                ks.finalize<<<fgrid, kWG, 0, s>>>(plan->d_heavy + L.heavy_begin, L.n_heavy, a);
+            if (L.wide_rows) {
+                ks.finalize_wide<<<L.n_heavy, kWG, 0, s>>>(plan->d_heavy + L.heavy_begin, L.n_heavy, a);
                 LF_HIP(hipGetLastError());
-                if (L.wide_rows) {
-                    ks.finalize_wide<<<L.n_heavy, kWG, 0, s>>>(plan->d_heavy + L.heavy_begin, L.n_heavy, a);
-                    LF_HIP(hipGetLastError());
-                }
             }
         }
     }

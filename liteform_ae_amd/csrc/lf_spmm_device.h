@@ -49,7 +49,7 @@ constexpr int kDenseRowShare = 32;
 constexpr int kDenseRowMinSlots = 4096;
 constexpr long long kDenseMinBBytes = 128ll << 20;   // ... in a partition whose part of B is larger than this
 constexpr int kDenseChunkSlots = 1024;
-constexpr int kWideFinalPartials = 64;       // rows with more partial rows are added up by a whole workgroup
+constexpr int kWideFinalPartials = 64;       // rows with more partial rows are added up by a kernel of their own
 constexpr int kXcds = 8;
 constexpr int kPartBytesMax = 16384;   // LDS for per-ELL-row sums of a balanced segment tile at most
 constexpr int kUnroll = LF_UNROLL;  // B-row gathers in flight per sub-wave
@@ -67,13 +67,15 @@ struct Chunk {
                             // whole source row and goes straight to C
     int row;                // source row
     int first_col;          // column of the chunk's first slot (chunks of dense rows are ordered by it)
+    int heavy;              // entry of the row in the heavy-row table (rows of several chunks)
+    int pad_;
 };
 
 struct HeavyRow {
     int row;
     int partial_begin;
     int n_partials;
-    int pad_;
+    int done;               // chunks of the row that have left their partial row in the present launch
 };
 
 struct Group {
@@ -102,6 +104,7 @@ struct LaunchArgs {
     const void* B;
     float* C;
     float* partials;
+    HeavyRow* heavy;
 };
 
 // ------------------------------------------------------------------------------------

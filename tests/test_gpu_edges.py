@@ -191,3 +191,27 @@ def test_csr_product_at_group_edges(fa, torch, nr, feat, b_dtype):
     got = fa.spmm_csr(MTX.from_csr(indptr, (key % nc).astype(np.int32), (nr, nc), data=vals), B, b_dtype).cpu().numpy()
     Bh = B.float().cpu().numpy().astype(np.float64)
     assert (np.abs(got - A @ Bh) <= 1e-5 * (abs(A) @ np.abs(Bh)) + 1e-30).all()
+
+
+@pytest.mark.parametrize("feat,b_dtype", [(32, "f32"), (128, "f32"), (320, "f32"), (1024, "f32"), (64, "bf16"), (512, "bf16")])
+def test_rows_of_several_chunks(fa, torch, monkeypatch, feat, b_dtype):
+    """Long rows of one chunk, a few, the most that the last chunk's workgroup adds up and one more;
+    several runs of one plan, which has to reset its counters, give the same bits."""
+    monkeypatch.setenv("LF_DENSE_ROWS", "0")          # chunks of 2048 slots whatever the size of B
+    rng = np.random.default_rng(feat)
+    nc = 140_000
+    lens = [257, 2048, 2049, 4096, 4097, 3 * 2048, 64 * 2048, 64 * 2048 + 1]
+    row = np.repeat(np.arange(len(lens)), lens)
+    col = np.concatenate([np.sort(rng.choice(nc, size=n, replace=False)) for n in lens])
+    g = MTX.from_coo(row, col, (len(lens), nc), data=rng.uniform(-1, 1, size=len(row)).astype(np.float32))
+    B = torch.from_numpy(rng.uniform(-1, 1, size=(nc, feat)).astype(np.float32)).cuda()
+    if b_dtype == "bf16":
+        B = B.to(torch.bfloat16)
+    plan = fa.HybSpMM(fa.build_hyb_format_device(g, [[64, 1024]]), feat, b_dtype)
+    assert plan.info["heavy_rows"] == 6 and plan.info["partial_rows"] == 2 + 2 + 3 + 3 + 64 + 65
+    runs = [plan.run(B).clone() for _ in range(4)]
+    assert all(torch.equal(r, runs[0]) for r in runs)
+    indptr, indices, data = g.adj_tensors("csr")
+    Bh = B.float().cpu().numpy()
+    ref = O.spmm_csr_f64(indptr, indices, data, (len(lens), nc), Bh)
+    assert (np.abs(runs[0].cpu().numpy() - ref) <= 1e-5 * O.spmm_abs_bound(indptr, indices, data, (len(lens), nc), Bh)).all()
