@@ -1899,15 +1899,20 @@ int lf_spmm_create(lf_spmm_plan** out_plan, const lf_bucket_desc* h_buckets, int
         std::vector<int> mine;
         for (int k = 0; k < num_buckets; ++k)
             if (h_buckets[k].part == p && h_buckets[k].num_ell_rows > 0) mine.push_back(k);
-        // Streaming stores leave the caches to B, but a launch whose rows are mostly short is
-        // made of stores as much as of gathers and loses by them: 2.45M-row graph (33 entries per
-        // row) 6.23 -> 6.13 ms, 500k x 2M matrix (most rows 2-4 entries) 1.46 -> 1.53 ms.
+        // Streaming stores leave the caches to B (2.45M-row graph, 33 entries per row: 6.23 -> 6.13
+        // ms; short rows too: 392K x 680K, 4 entries per row, N = 64 88 -> 77 us, 1.47M x 2.73M, 8
+        // per row, N = 96 910 -> 874), except where a lane's eight features of a bf16 product go out
+        // as 16 of 32 bytes per instruction: the pieces then need the L2 to be put together, and a
+        // launch of mostly short rows is made of stores as much as of gathers (500k x 2M matrix, most
+        // rows 2-4 entries, 1.46 -> 1.53 ms; 1.19M x 1.83M, 3.6 per row, N = 128 296 -> 376 us).  A
+        // C that the L2s hold is left there.
         long long rows_wide = 0, rows_all = 0;
         for (int k : mine) {
             rows_all += h_buckets[k].num_ell_rows;
             if (h_buckets[k].width >= kStreamMinWidth) rows_wide += h_buckets[k].num_ell_rows;
         }
-        L.stream_c = rows_wide * 2 >= rows_all;
+        const bool c_fits_l2 = (long long)num_rows * feat_size * 4 <= kL2Bytes;
+        L.stream_c = rows_wide * 2 >= rows_all || (b_dtype == LF_DTYPE_F32 && !c_fits_l2);
         for (int k : mine) L.wide_rows = L.wide_rows || has_wide[k];
         L.heavy_begin = mine.empty() ? 0 : heavy_base[mine.front()];
         L.n_heavy = mine.empty() ? 0 : heavy_base[mine.back() + 1] - L.heavy_begin;

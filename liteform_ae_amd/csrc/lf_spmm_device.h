@@ -195,11 +195,11 @@ __device__ __forceinline__ void gather_fma(const void* B, const Lane<LPR, CH, De
 }
 
 // flags: LaunchArgs::accumulate.  Rows that nothing reads again in this run are stored
-// non-temporally where the launch's rows are mostly wide, which leaves the caches to B (2.45M-row
-// graph, N = 128: 6.23 -> 6.13 ms); rows that a later column partition adds to stay cached
+// non-temporally where that leaves the caches to B (lf_spmm_create decides); rows that a later column partition adds to stay cached
 // (170k-row graph, two partitions: streaming them costs 7 %).
 constexpr int kAccumulateC = 1, kStreamC = 2, kStreamSlabs = 4;
-constexpr int kStreamMinWidth = 16;      // a launch streams C when at least half of its ELL rows are this wide
+constexpr int kStreamMinWidth = 16;      // a launch of mostly wide rows: at least half of its ELL rows are this wide
+constexpr long long kL2Bytes = 32ll << 20;   // of the eight XCDs together
 typedef float lf_f32x4 __attribute__((ext_vector_type(4)));
 
 // 16 bytes to global memory, streamed or not by a run-time flag.  The streaming store goes
