@@ -15,7 +15,7 @@
 //     (whose source rows may span several ELL rows) stream slots through wavefront
 //     shuffles instead;
 //   * a source row split over several ELL rows is summed by one owner; rows longer than
-//     kCoopSlots are reduced by a whole workgroup, kChunkSlots at a time: a row that fits one
+//     coop_slots (64 to 256) are reduced by a whole workgroup, kChunkSlots at a time: a row that fits one
 //     chunk is written directly, a longer one leaves one partial row per chunk, which the
 //     workgroup that comes last adds up (rows of very many chunks: a small second kernel);
 //   * partitions run as consecutive launches: partition 0 stores every output row (rows it
@@ -195,7 +195,7 @@ __device__ __forceinline__ void ell_tile_segments(const Group& g, long long e0, 
         const int2 rm = s_rm[r];
         if (rm.y < 0) continue;                                  // continuation row
         const int seg = (int)((uint32_t)rm.y >> kMetaLenBits);
-        if (((long long)seg << log_w) > kCoopSlots) continue;   // reduced by a whole workgroup
+        if (((long long)seg << log_w) > a.coop_slots) continue; // reduced by a whole workgroup
         int total = rm.y & kMetaLenMask;
         if (seg > 1) {
             const int last = r + seg - 1;
@@ -245,7 +245,7 @@ __device__ __forceinline__ void ell_tile_segments_balanced(const Group& g, long 
         const int head = cont ? r - (int)(((uint32_t)rm.y & 0x7FFFFFFFu) >> kMetaLenBits) : r;
         if (head < 0) continue;                                  // belongs to the previous tile's last segment
         const int seg = (int)((uint32_t)s_rm[head].y >> kMetaLenBits);
-        if (((long long)seg << log_w) > kCoopSlots) continue;   // reduced by a whole workgroup
+        if (((long long)seg << log_w) > a.coop_slots) continue; // reduced by a whole workgroup
         const int len = rm.y & kMetaLenMask;
         const int2* rp = s_pairs + (r << log_w);
         const int c0 = rp[0].x;
@@ -282,7 +282,7 @@ __device__ __forceinline__ void ell_tile_segments_balanced(const Group& g, long 
         const int2 rm = s_rm[r];
         if (rm.y < 0) continue;
         const int seg = (int)((uint32_t)rm.y >> kMetaLenBits);
-        if (seg == 1 || ((long long)seg << log_w) > kCoopSlots) continue;
+        if (seg == 1 || ((long long)seg << log_w) > a.coop_slots) continue;
         Acc<CH, VEC> acc;
         acc.clear();
         const int inside = min(seg, n - r);
@@ -351,7 +351,7 @@ __device__ __forceinline__ void run_ell_tile(const Group& g, long long tile, int
 
 // Bucket whose source rows may span several ELL rows, or whose rows are too wide to stage:
 // the first ELL row of a segment owns it and streams all of its slots; continuation rows
-// and segments above kCoopSlots (handled as chunks) are skipped.
+// and segments above coop_slots (handled as chunks) are skipped.
 template <int LPR, int CH, typename BT>
 __device__ __forceinline__ void run_seg_tile(const Group& g, long long tile, const LaunchArgs& a) {
     constexpr int VEC = Dense<BT>::kVec;
@@ -366,7 +366,7 @@ __device__ __forceinline__ void run_seg_tile(const Group& g, long long tile, con
         const int m = g.meta[e];
         if (m < 0) continue;                                   // continuation row
         const int seg = (int)((uint32_t)m >> kMetaLenBits);
-        if (((long long)seg << g.log_w) > kCoopSlots) continue;
+        if (((long long)seg << g.log_w) > a.coop_slots) continue;
         int total = m & kMetaLenMask;
         if (seg > 1) total = ((seg - 1) << g.log_w) + (g.meta[e + seg - 1] & kMetaLenMask);
         Acc<CH, VEC> acc;
@@ -401,6 +401,9 @@ __device__ __forceinline__ void load_pair_agent(const float* src, float& x, floa
     y = __uint_as_float((unsigned int)(v >> 32));
 }
 
+constexpr int kSlice = 8;
+constexpr int kSlicedSlots = 128;
+
 // One chunk of a heavy source row: the workgroup's sub-waves take consecutive slices of
 // the chunk, their sums are combined through LDS in sub-wave order.
 template <int LPR, int CH, typename BT>
@@ -412,12 +415,37 @@ __device__ __forceinline__ void run_chunk_tile(const Group& g, long long tile, f
     const int sw = tid / LPR, sl = tid % LPR;
     const Lane<LPR, CH, VEC> ln(sl, a.feat, a.ldb, a.ldc);
     const Chunk ck = g.chunks[tile];
-    int per = (ck.n_slots + SW - 1) / SW;
-    per = (per + LPR - 1) / LPR * LPR;
+    constexpr int kPart = kUnroll < LPR ? kUnroll : LPR;
+    const int per = ((ck.n_slots + SW - 1) / SW + kPart - 1) / kPart * kPart;
     const int lo = min(sw * per, ck.n_slots);
     const int hi = min(lo + per, ck.n_slots);
     Acc<CH, VEC> acc;
     acc.clear();
+    if (ck.partial < 0 && ck.n_slots <= kSlicedSlots) {
+        // A short row in slices of kSlice slots, added in their order: the same sums whatever the lane
+        // count, so that such rows do not depend on the feature windows of the plan.
+        Acc<CH, VEC> sum;
+        sum.clear();
+        for (int s0 = 0; s0 * kSlice < ck.n_slots; s0 += SW) {
+            const int at = (s0 + sw) * kSlice;
+            acc.clear();
+            stream_slots<LPR, CH, BT>(g.cols, g.vals, ck.slot_begin + at, min(kSlice, ck.n_slots - at), a.B, ln, acc);
+            if (s0 > 0) __syncthreads();             // the slices before have been read
+#pragma unroll
+            for (int c = 0; c < CH; ++c)
+#pragma unroll
+                for (int i = 0; i < VEC; ++i) s_red[((sw * CH + c) * LPR + sl) * VEC + i] = acc.v[c][i];
+            __syncthreads();
+            const int n = min(SW, (ck.n_slots + kSlice - 1) / kSlice - s0);
+#pragma unroll
+            for (int c = 0; c < CH; ++c)
+                for (int s = 0; s < n && sw == 0; ++s)
+#pragma unroll
+                    for (int i = 0; i < VEC; ++i) sum.v[c][i] += s_red[((s * CH + c) * LPR + sl) * VEC + i];
+        }
+        if (sw == 0) store_row<LPR, CH, VEC>(a.C, ck.row, ln, sum, a.accumulate);
+        return;
+    }
     stream_slots<LPR, CH, BT>(g.cols, g.vals, ck.slot_begin + lo, hi - lo, a.B, ln, acc);
     // s_red[sw][c][sl][i]
 #pragma unroll
@@ -1107,7 +1135,7 @@ struct ChunkedRow {
 };
 
 __device__ __forceinline__ ChunkedRow chunked_row(const int32_t* __restrict__ meta, long long e, long long n_rows,
-                                                  int log_w, int chunk_slots, long long dense_min_slots) {
+                                                  int log_w, int coop_slots, int chunk_slots, long long dense_min_slots) {
     ChunkedRow x{0, 0, chunk_slots, 0};
     const int m = meta[e];
     if (m < 0) {
@@ -1119,7 +1147,7 @@ __device__ __forceinline__ ChunkedRow chunked_row(const int32_t* __restrict__ me
     // The counting pass is enqueued together with the slab checks, before their verdict has been
     // read: a head that announces more ELL rows than the bucket holds (which the checks flag and
     // the plan is then refused) must not be followed past the array.
-    if (((long long)seg << log_w) > kCoopSlots && e + seg <= n_rows) {
+    if (((long long)seg << log_w) > coop_slots && e + seg <= n_rows) {
         x.total = ((long long)(seg - 1) << log_w) + (meta[e + seg - 1] & (int)kMetaLenMask);
         if (x.total >= dense_min_slots) {
             x.chunk_slots = kDenseChunkSlots;
@@ -1162,7 +1190,7 @@ constexpr int kCounterLine = 32;           // words between the counters of a bu
                                            // own, as atomics on one line are taken one after the other (17 ns each)
 __global__ void __launch_bounds__(256)
 plan_scan_kernel(const PlanBucket* __restrict__ buckets, const int32_t* __restrict__ first_block, int n_buckets,
-                 long long num_rows, long long num_cols, int chunk_slots, long long dense_min_slots,
+                 long long num_rows, long long num_cols, int coop_slots, int chunk_slots, long long dense_min_slots,
                  int* __restrict__ counters, int* __restrict__ flags, uint8_t* __restrict__ covered) {
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     int k = -1;                                       // last bucket whose first workgroup is not behind this one
@@ -1226,7 +1254,7 @@ plan_scan_kernel(const PlanBucket* __restrict__ buckets, const int32_t* __restri
         } else {
             bad_meta |= want != 0;
         }
-        const ChunkedRow x = chunked_row(meta, e, n_rows, log_w, chunk_slots, dense_min_slots);
+        const ChunkedRow x = chunked_row(meta, e, n_rows, log_w, coop_slots, chunk_slots, dense_min_slots);
         found |= x.found;
         sum[0] += x.n_chunks;
         sum[1] += x.n_chunks > 1;
@@ -1275,7 +1303,7 @@ rowgroup_sample_kernel(const PlanBucket* __restrict__ buckets, const int* __rest
     add_rowgroup_counters(m, plain, counters + 3 * blockIdx.y);
 }
 
-// Fills the chunk table of a bucket (rows of more than kCoopSlots slots, cut into chunks) and its
+// Fills the chunk table of a bucket (rows of more than coop_slots slots, cut into chunks) and its
 // part of the heavy-row table.  counters (kCounterLine words apart): chunks, rows with several chunks
 // and their partial rows handed out so far.  Table order depends on scheduling, results do not: every row's partials are
 // private and are summed in chunk order.
@@ -1288,7 +1316,7 @@ __global__ void __launch_bounds__(256)
 plan_chunks_kernel(const int32_t* __restrict__ rows, const int32_t* __restrict__ meta,
                    const int32_t* __restrict__ cols, long long n_rows, int log_w, int* __restrict__ counters,
                    Chunk* __restrict__ chunks, HeavyRow* __restrict__ heavy,
-                   int partial_base, int heavy_base, int chunk_slots, long long dense_min_slots) {
+                   int partial_base, int heavy_base, int coop_slots, int chunk_slots, long long dense_min_slots) {
     __shared__ int s_sum[4][3];
     __shared__ int s_base[3];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -1297,7 +1325,7 @@ plan_chunks_kernel(const int32_t* __restrict__ rows, const int32_t* __restrict__
     const long long hi = min(lo + per_wave, n_rows);
     int sum[3] = {0, 0, 0};
     for (long long e = lo + lane; e < hi; e += 64) {
-        const ChunkedRow x = chunked_row(meta, e, n_rows, log_w, chunk_slots, dense_min_slots);
+        const ChunkedRow x = chunked_row(meta, e, n_rows, log_w, coop_slots, chunk_slots, dense_min_slots);
         sum[0] += x.n_chunks;
         sum[1] += x.n_chunks > 1;
         sum[2] += x.n_chunks > 1 ? x.n_chunks : 0;
@@ -1321,7 +1349,7 @@ plan_chunks_kernel(const int32_t* __restrict__ rows, const int32_t* __restrict__
     for (long long e0 = lo; e0 < hi && sum[0] > 0; e0 += 64) {
         const long long e = e0 + lane;
         ChunkedRow x{0, 0, chunk_slots, 0};
-        if (e < hi) x = chunked_row(meta, e, n_rows, log_w, chunk_slots, dense_min_slots);
+        if (e < hi) x = chunked_row(meta, e, n_rows, log_w, coop_slots, chunk_slots, dense_min_slots);
         const bool several = x.n_chunks > 1;
         const unsigned long long votes = __ballot(several);
         if (__ballot(x.n_chunks > 0) == 0) continue;
@@ -1418,6 +1446,7 @@ struct lf_spmm_plan {
         bool stream_c = false;       // store C past the caches (when this is the run's last partition)
     };
     std::vector<Launch> launches;
+    int coop_slots = kCoopSlots;        // source rows of more slab slots are reduced by whole workgroups
     bool stream_slabs = false;          // read the slabs non-temporally
     MergedBucket* d_merged = nullptr;   // row-group buckets, grouped by partition
     LfCellBucket* d_cells = nullptr;    // buckets rewritten as cells, grouped by partition
@@ -1592,17 +1621,38 @@ int lf_spmm_create(lf_spmm_plan** out_plan, const lf_bucket_desc* h_buckets, int
     std::vector<ChunkCount> counts((size_t)num_buckets);
     std::vector<int> is_multi((size_t)num_buckets, 0), has_dense((size_t)num_buckets, 0), has_wide((size_t)num_buckets, 0);
     // Chunk size of the rows that a whole workgroup reduces.  Small matrices want many short
-    // chunks (a 170k-row graph: 0.076 ms with 2048-slot chunks, 0.112 ms with 8192), large ones
+    // chunks (a 170k-row graph: 0.076 ms with 2048-slot chunks, 0.112 ms with 8192; the smaller the
+    // matrix, the more a chunk's chain of gathers is of the whole: 13K rows, 58K entries, N = 320
+    // bf16, chunks of 2048 / 1024 / 512: 47 / 29 / 19 us, 30K rows, 130K entries, N = 192 41 / 26 / 25,
+    // 149K rows, 640K entries, N = 128 58 / 59 / 60), large ones
     // fewer partial rows and a shorter second kernel (500k x 2M with 50 rows of 100k entries:
     // 1.56 -> 1.51 ms with 8192); the chunk tiles lead the launch, so their length hides behind
     // the rest of the work.
     long long total_slots = 0;
     for (int k = 0; k < num_buckets; ++k) total_slots += h_buckets[k].num_ell_rows * h_buckets[k].width;
-    const int chunk_slots = total_slots >= kLargeMatrixSlots ? kChunkSlotsLarge : kChunkSlots;
+    const int chunk_slots = total_slots >= kLargeMatrixSlots ? kChunkSlotsLarge
+                            : total_slots >= (512 << 10)     ? kChunkSlots
+                            : total_slots >= (192 << 10)     ? kChunkSlots / 4 * 3
+                            : total_slots >= (128 << 10)     ? kChunkSlots / 2
+                                                             : kChunkSlots / 4;
     // Slabs of a large matrix are read past the caches' retention (2.45M-row graph 6.15 -> 6.09 ms,
     // 500k x 2M matrix 1.457 -> 1.443); those of a small one are worth keeping between products
     // (170k-row graph, 6 MB of slabs: 0.073 ms cached, 0.076 ms streamed).
     plan->stream_slabs = total_slots >= kLargeMatrixSlots;
+    // A sub-wave sums kUnroll slots of its row per round trip to B, so a row of kCoopSlots is a
+    // chain of 32; where a launch holds few rows of more than 64 slots - a few workgroups per CU - they
+    // set its length, and whole workgroups take them too.  (56K-row power-law graph, bf16, N = 128: 33
+    // -> 21 us; 36K rows, N = 64: 33 -> 16; with some thousand such rows the workgroups' set-up costs more
+    // than the chains: 26K rows of 46 entries, N = 64 34 -> 40.)  In between, for small N with its many
+    // sub-waves to a workgroup, rows of more than 128 (25K rows of 62 entries, N = 32: 26 -> 22 us).
+    long long over64 = 0, over128 = 0;
+    for (int k = 0; k < num_buckets; ++k) {
+        const lf_bucket_desc& b = h_buckets[k];
+        if (b.width > 64 && b.width <= kCoopSlots) over64 += b.num_ell_rows;
+        if (b.width > 128 && b.width <= kCoopSlots) over128 += b.num_ell_rows;
+    }
+    if (over64 <= 4 * plan->num_cus) plan->coop_slots = 64;
+    else if (lpr <= 16 && over128 <= 8 * plan->num_cus) plan->coop_slots = 128;
     const char* env_dense = getenv("LF_DENSE_ROWS");       // "0": dense rows are chunked like the other long rows
     // (where the memory-side cache holds the partition's part of B anyway there is nothing to order)
     const long long cols_p = lf::ceil_div(num_cols, num_parts);
@@ -1689,8 +1739,8 @@ int lf_spmm_create(lf_spmm_plan** out_plan, const lf_bucket_desc* h_buckets, int
     }
     if (num_buckets > 0) LF_TRY_HIP(hipMemcpyAsync(d_scratch + o_table, h_table, table_bytes, hipMemcpyHostToDevice, s));
     if (scan_blocks > 0) {
-        plan_scan_kernel<<<scan_blocks, 256, 0, s>>>(d_table, d_first, num_buckets, num_rows, num_cols, chunk_slots,
-                                                     dense_min_slots, d_counters, d_flags, d_cov);
+        plan_scan_kernel<<<scan_blocks, 256, 0, s>>>(d_table, d_first, num_buckets, num_rows, num_cols, plan->coop_slots,
+                                                     chunk_slots, dense_min_slots, d_counters, d_flags, d_cov);
         LF_TRY_HIP(hipGetLastError());
     }
     const int rgrid = (int)std::min<int64_t>((num_rows + 255) / 256, 1024);
@@ -1753,8 +1803,8 @@ int lf_spmm_create(lf_spmm_plan** out_plan, const lf_bucket_desc* h_buckets, int
         d_chunks[k] = d_chunks_all + chunk_base[k];
         const int grid = (int)std::min<long long>((b.num_ell_rows + 255) / 256, kPlanChunksGrid);
         plan_chunks_kernel<<<grid, 256, 0, s>>>(b.d_rows, meta[k], b.d_cols, b.num_ell_rows, lf::ilog2(b.width), d_cursors + (size_t)4 * k * kCounterLine,
-                                                d_chunks[k], plan->d_heavy, partial_base[k], heavy_base[k], chunk_slots,
-                                                dense_min_slots);
+                                                d_chunks[k], plan->d_heavy, partial_base[k], heavy_base[k], plan->coop_slots,
+                                                chunk_slots, dense_min_slots);
         LF_TRY_HIP(hipGetLastError());
     }
     for (int k = 0; k < num_buckets; ++k) {
@@ -1931,7 +1981,7 @@ int lf_spmm_create(lf_spmm_plan** out_plan, const lf_bucket_desc* h_buckets, int
         std::sort(mine.begin(), mine.end(), [&](int x, int y) { return h_buckets[x].width > h_buckets[y].width; });
         for (int k : mine) {
             const lf_bucket_desc& b = h_buckets[k];
-            if (b.width > kCoopSlots) continue;            // every row of this bucket is a chunk
+            if (b.width > plan->coop_slots) continue;           // every row of this bucket is a chunk
             if (merged_of[k] >= 0 || cell_of[k] >= 0) continue;   // served by the row-group or the cell kernel
             Group g{};
             g.log_w = lf::ilog2(b.width);
@@ -2112,6 +2162,7 @@ int lf_spmm_run(lf_spmm_plan* plan, const void* d_B, float* d_C, lf_stream_t str
             a.C = d_C + (size_t)w * plan->feat;
             a.partials = plan->d_partials;
             a.heavy = plan->d_heavy;
+            a.coop_slots = plan->coop_slots;
             if (L.grid > 0) {
                 ks.tiles<<<L.grid, kWG, L.dyn_lds, s>>>(a);
                 LF_HIP(hipGetLastError());

@@ -100,7 +100,7 @@ struct LaunchArgs {
                                   // the slabs are too large to be worth caching
     int feat;                     // N: features computed by the launch
     int ldb, ldc;                 // row strides of B and C in elements (N, or more for a feature window)
-    int pad_;
+    int coop_slots;               // source rows of more slab slots are reduced by whole workgroups
     const void* B;
     float* C;
     float* partials;

@@ -197,10 +197,10 @@ def test_csr_product_at_group_edges(fa, torch, nr, feat, b_dtype):
 def test_rows_of_several_chunks(fa, torch, monkeypatch, feat, b_dtype):
     """Long rows of one chunk, a few, the most that the last chunk's workgroup adds up and one more;
     several runs of one plan, which has to reset its counters, give the same bits."""
-    monkeypatch.setenv("LF_DENSE_ROWS", "0")          # chunks of 2048 slots whatever the size of B
+    monkeypatch.setenv("LF_DENSE_ROWS", "0")          # (dense rows would be cut differently where B is large)
     rng = np.random.default_rng(feat)
     nc = 140_000
-    lens = [257, 2048, 2049, 4096, 4097, 3 * 2048, 64 * 2048, 64 * 2048 + 1]
+    lens = [257, 1024, 1025, 2048, 2049, 3 * 1024, 64 * 1024, 64 * 1024 + 1]          # chunks of 1024 at this size
     row = np.repeat(np.arange(len(lens)), lens)
     col = np.concatenate([np.sort(rng.choice(nc, size=n, replace=False)) for n in lens])
     g = MTX.from_coo(row, col, (len(lens), nc), data=rng.uniform(-1, 1, size=len(row)).astype(np.float32))
@@ -215,3 +215,25 @@ def test_rows_of_several_chunks(fa, torch, monkeypatch, feat, b_dtype):
     Bh = B.float().cpu().numpy()
     ref = O.spmm_csr_f64(indptr, indices, data, (len(lens), nc), Bh)
     assert (np.abs(runs[0].cpu().numpy() - ref) <= 1e-5 * O.spmm_abs_bound(indptr, indices, data, (len(lens), nc), Bh)).all()
+
+
+@pytest.mark.parametrize("feat,b_dtype", [(32, "f32"), (256, "f32"), (512, "f32"), (128, "bf16")])
+@pytest.mark.parametrize("n_long", [0, 1024, 1025, 3000])
+def test_rows_around_the_cooperative_length(fa, torch, feat, b_dtype, n_long):
+    """Whole workgroups take rows of more than 64, 128 or 256 slots, by how many rows there are of
+    more than 64 and of more than 128: rows on either side of every length, at every choice."""
+    rng = np.random.default_rng(n_long + feat)
+    nc = 900
+    lens = np.concatenate([[1, 63, 64, 65, 127, 128, 129, 255, 256, 257, 511, 512, 513],
+                           rng.integers(65, 129, size=n_long), rng.integers(129, 257, size=n_long // 2)]).astype(np.int64)
+    if n_long == 0:
+        lens = lens[:4]
+    row = np.repeat(np.arange(len(lens)), lens)
+    pos = np.arange(len(row)) - np.repeat(np.cumsum(lens) - lens, lens)
+    g = MTX.from_coo(row, (row * 17 + pos * 7) % nc, (len(lens), nc), data=rng.uniform(-1, 1, size=len(row)).astype(np.float32))
+    B = torch.from_numpy(rng.uniform(-1, 1, size=(nc, feat)).astype(np.float32)).cuda().to(torch.bfloat16 if b_dtype == "bf16" else torch.float32)
+    got = fa.HybSpMM(fa.build_hyb_format_device(g, [[1, 64, 128, 256, 512]]), feat, b_dtype).run(B).cpu().numpy()
+    indptr, indices, data = g.adj_tensors("csr")
+    Bh = B.float().cpu().numpy()
+    assert (np.abs(got - O.spmm_csr_f64(indptr, indices, data, (len(lens), nc), Bh))
+            <= 1e-5 * O.spmm_abs_bound(indptr, indices, data, (len(lens), nc), Bh)).all()
