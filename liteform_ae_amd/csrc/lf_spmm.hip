@@ -546,24 +546,37 @@ spmm_partition_kernel(LaunchArgs a) {
     __shared__ int s_next;                     // next ELL row of a tile whose rows are taken dynamically
     extern __shared__ __align__(16) float s_dyn[];   // per-ELL-row sums of a balanced segment tile
 
+    // position in this XCD's tile list -> group and tile.  The groups' tile counts come with the
+    // arguments: reading the groups one after the other took a round trip to memory each.
     const int xcd = blockIdx.x % kXcds;
-    long long v = blockIdx.x / kXcds;          // position in this XCD's tile list
-    for (int gi = 0; gi < a.n_groups; ++gi) {
-        const Group& g = a.groups[gi];         // uniform address: scalar loads
-        const long long lo = g.n_tiles * xcd / kXcds;
-        const long long hi = g.n_tiles * (xcd + 1) / kXcds;
-        if (v < hi - lo) {
-            const long long tile = lo + v;
-            switch (g.type) {
-                case kEll:
-                case kEllSeg: run_ell_tile<LPR, CH, BT>(g, tile, s_pairs, s_rm, &s_next, s_dyn, a); break;
-                case kSeg: run_seg_tile<LPR, CH, BT>(g, tile, a); break;
-                case kZero: run_zero_tile<LPR, CH, BT>(g, tile, a); break;
-                default: run_chunk_tile<LPR, CH, BT>(g, tile, reinterpret_cast<float*>(s_raw), a); break;
-            }
-            return;
+    long long v = blockIdx.x / kXcds;
+    auto in_group = [&](long long n_tiles) {
+        const long long lo = n_tiles * xcd / kXcds, n = n_tiles * (xcd + 1) / kXcds - lo;
+        if (v < n) {
+            v += lo;
+            return true;
         }
-        v -= hi - lo;
+        v -= n;
+        return false;
+    };
+    int gi = 0;
+    bool found = false;
+#pragma unroll
+    for (int i = 0; i < kInlineGroups; ++i) {
+        if (found || i >= a.n_groups) break;
+        found = in_group(a.n_tiles[i]);
+        if (!found) ++gi;
+    }
+    for (; !found && gi < a.n_groups; ++gi)
+        if ((found = in_group(a.groups[gi].n_tiles))) break;
+    if (!found) return;
+    const Group& g = a.groups[gi];             // uniform address: scalar loads
+    switch (g.type) {
+        case kEll:
+        case kEllSeg: run_ell_tile<LPR, CH, BT>(g, v, s_pairs, s_rm, &s_next, s_dyn, a); break;
+        case kSeg: run_seg_tile<LPR, CH, BT>(g, v, a); break;
+        case kZero: run_zero_tile<LPR, CH, BT>(g, v, a); break;
+        default: run_chunk_tile<LPR, CH, BT>(g, v, reinterpret_cast<float*>(s_raw), a); break;
     }
 }
 
@@ -1443,6 +1456,7 @@ struct lf_spmm_plan {
         long long tiles = 0;
         int heavy_begin = 0, n_heavy = 0;
         bool wide_rows = false;      // some rows have more than kWideFinalPartials partial rows
+        int n_tiles[kInlineGroups] = {0};    // of the first groups
         bool stream_c = false;       // store C past the caches (when this is the run's last partition)
     };
     std::vector<Launch> launches;
@@ -2065,7 +2079,10 @@ int lf_spmm_create(lf_spmm_plan** out_plan, const lf_bucket_desc* h_buckets, int
                 len += groups[gi].n_tiles * (x + 1) / kXcds - groups[gi].n_tiles * x / kXcds;
             longest = std::max(longest, len);
         }
-        for (int gi = L.group_begin; gi < (int)groups.size(); ++gi) L.tiles += groups[gi].n_tiles;
+        for (int gi = L.group_begin; gi < (int)groups.size(); ++gi) {
+            L.tiles += groups[gi].n_tiles;
+            if (gi - L.group_begin < kInlineGroups) L.n_tiles[gi - L.group_begin] = (int)groups[gi].n_tiles;   // (checked below)
+        }
         if (longest * kXcds >= (1ll << 31))
             return bail(lf::fail(LF_ERR_UNSUPPORTED, "partition %d needs too many tiles", p));
         L.grid = (int)(longest * kXcds);
@@ -2163,6 +2180,7 @@ int lf_spmm_run(lf_spmm_plan* plan, const void* d_B, float* d_C, lf_stream_t str
             a.partials = plan->d_partials;
             a.heavy = plan->d_heavy;
             a.coop_slots = plan->coop_slots;
+            std::memcpy(a.n_tiles, L.n_tiles, sizeof(a.n_tiles));
             if (L.grid > 0) {
                 ks.tiles<<<L.grid, kWG, L.dyn_lds, s>>>(a);
                 LF_HIP(hipGetLastError());

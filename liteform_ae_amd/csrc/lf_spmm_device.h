@@ -92,6 +92,8 @@ struct Group {
     const Chunk* chunks;          // kChunk
 };
 
+constexpr int kInlineGroups = 16;
+
 struct LaunchArgs {
     const Group* groups;
     int n_groups;
@@ -105,6 +107,7 @@ struct LaunchArgs {
     float* C;
     float* partials;
     HeavyRow* heavy;
+    int n_tiles[kInlineGroups];   // of the first groups: a workgroup finds its group without reading the others
 };
 
 // ------------------------------------------------------------------------------------

@@ -553,6 +553,8 @@ class HybSpMM:
         self.num_rows, self.num_cols = int(num_rows), int(num_cols)
         dt = {"f32": _lib.LF_DTYPE_F32, "bf16": _lib.LF_DTYPE_BF16}[b_dtype]
         self.windows = int(windows)
+        self._b_type = torch.float32 if b_dtype == "f32" else torch.bfloat16
+        self._b_shape, self._c_shape = (self.num_cols, self.feat_size), (self.num_rows, self.feat_size)
         _lib.check(lib.lf_spmm_create(C.byref(self.handle), descs, nb, P, self.num_rows, self.num_cols,
                                       self.feat_size // self.windows, dt, _stream()))
         if self.windows > 1:
@@ -565,20 +567,19 @@ class HybSpMM:
         self.info["windows"] = self.windows
 
     def _check_operands(self, B, Cout):
-        torch = _torch()
-        want = torch.float32 if self.b_dtype == "f32" else torch.bfloat16
-        if B.dtype != want or not B.is_cuda or not B.is_contiguous() or tuple(B.shape) != (self.num_cols, self.feat_size):
-            raise ValueError(f"B must be a contiguous CUDA tensor of shape {(self.num_cols, self.feat_size)} and dtype {want}")
-        if (Cout.dtype != torch.float32 or not Cout.is_cuda or not Cout.is_contiguous()
-                or tuple(Cout.shape) != (self.num_rows, self.feat_size)):
-            raise ValueError(f"C must be a contiguous float32 CUDA tensor of shape {(self.num_rows, self.feat_size)}")
+        if B.dtype is not self._b_type or not B.is_cuda or not B.is_contiguous() or B.shape != self._b_shape:
+            raise ValueError(f"B must be a contiguous CUDA tensor of shape {self._b_shape} and dtype {self._b_type}")
+        if Cout is not None and (Cout.dtype is not _gpu_torch.float32 or not Cout.is_cuda or not Cout.is_contiguous()
+                                 or Cout.shape != self._c_shape):
+            raise ValueError(f"C must be a contiguous float32 CUDA tensor of shape {self._c_shape}")
 
     def run(self, B, Cout=None):
-        torch = _torch()
-        if Cout is None:
-            Cout = torch.empty((self.num_rows, self.feat_size), dtype=torch.float32, device="cuda")
         self._check_operands(B, Cout)
-        _lib.check(self._lib.lf_spmm_run(self.handle, B.data_ptr(), Cout.data_ptr(), _stream()))
+        if Cout is None:
+            Cout = B.new_empty(self._c_shape, dtype=_gpu_torch.float32)
+        rc = self._lib.lf_spmm_run(self.handle, B.data_ptr(), Cout.data_ptr(), _stream())
+        if rc:
+            _lib.check(rc)
         return Cout
 
     def time_ms(self, B, Cout, warmup: int = 10, repeat: int = 100, flush=None):
