@@ -89,12 +89,10 @@ __device__ __forceinline__ void ell_tile_narrow(const int2* s_pairs, const int2*
     constexpr int RPI = kUnroll / W;
     const Lane<LPR, CH, VEC> ln(sl, a.feat, a.ldb, a.ldc);
     for (int r0 = sw * RPI; r0 < n; r0 += SW * RPI) {
-        Acc<CH, VEC> acc[RPI];
         int c[kUnroll];
         float v[kUnroll];
 #pragma unroll
         for (int q = 0; q < RPI; ++q) {
-            acc[q].clear();
             const int r = min(r0 + q, n - 1);
             const int len = s_rm[r].y & kMetaLenMask;
             const int c0 = s_pairs[r * W].x;
@@ -105,24 +103,21 @@ __device__ __forceinline__ void ell_tile_narrow(const int2* s_pairs, const int2*
                 v[q * W + j] = __int_as_float(cv.y);
             }
         }
-        {
-            float x[kUnroll][CH][VEC];
+        typename Dense<BT>::Raw x[kUnroll][CH];
 #pragma unroll
-            for (int u = 0; u < kUnroll; ++u)
+        for (int u = 0; u < kUnroll; ++u)
 #pragma unroll
-                for (int cc = 0; cc < CH; ++cc)
-                    Dense<BT>::load(dense_row<BT>(a.B, ln, cc, c[u]), x[u][cc]);
+            for (int cc = 0; cc < CH; ++cc) x[u][cc] = load_dense<BT>(a.B, ln, cc, c[u]);
 #pragma unroll
-            for (int u = 0; u < kUnroll; ++u)
+        for (int q = 0; q < RPI; ++q) {
+            Acc<CH, VEC> acc;
+            acc.clear();
 #pragma unroll
-                for (int cc = 0; cc < CH; ++cc)
+            for (int j = 0; j < W; ++j)
 #pragma unroll
-                    for (int i = 0; i < VEC; ++i)
-                        acc[u / W].v[cc][i] = fmaf(v[u], x[u][cc][i], acc[u / W].v[cc][i]);
+                for (int cc = 0; cc < CH; ++cc) fma_dense<BT>(v[q * W + j], x[q * W + j][cc], acc.v[cc]);
+            if (r0 + q < n) store_row<LPR, CH, VEC>(a.C, s_rm[r0 + q].x, ln, acc, a.accumulate);
         }
-#pragma unroll
-        for (int q = 0; q < RPI; ++q)
-            if (r0 + q < n) store_row<LPR, CH, VEC>(a.C, s_rm[r0 + q].x, ln, acc[q], a.accumulate);
     }
 }
 
@@ -493,7 +488,7 @@ __device__ __forceinline__ void run_chunk_tile(const Group& g, long long tile, f
     if (__builtin_amdgcn_readfirstlane(before) != n - 1) return;
     if (tid == 0) hr->done = 0;                      // for the next launch
     constexpr int kSub = 64 / LPR;
-    constexpr int U = VEC * CH <= 8 ? 8 : 2;         // partial rows in flight per sub-wave
+    constexpr int U = VEC * CH <= 4 ? 8 : VEC * CH <= 8 ? 4 : 2;   // partial rows in flight per sub-wave
     acc.clear();
     for (int k0 = sw; k0 < n; k0 += kSub * U) {
         float x[U][CH][VEC];
@@ -532,12 +527,28 @@ __device__ __forceinline__ void run_chunk_tile(const Group& g, long long tile, f
 // concatenated.  The hardware hands out workgroups in index order as slots free up, which
 // keeps the tiles in flight on an XCD next to each other and balances the load; a resident
 // grid that strides over the tiles measured 2-7 % slower on every workload.
-template <int LPR, int CH, typename BT>
-__global__ void __launch_bounds__(kWG)
+//
+// RESIDENT: the partition's part of B stays in the XCD's L2.  Gathers that hit are short, so what counts is how many
+// wavefronts are there to issue them: registers are held to 7 wavefronts per SIMD (bf16 6, two chunks
+// per lane 4), and a tile of a float product holds twice the slots, since the wait for a tile's
+// slots is a larger part of it.  132K-row graph, 300 entries a row, 16 partitions, N = 96: 1186 -> 1046
+// us (occupancy alone 1100, tiles alone 1096); 90K rows, 8 partitions, N = 192 862 -> 767; 22K rows of
+// 91, 8 partitions, N = 288 363 -> 327.  Where gathers miss, more of them in flight gain nothing and
+// bf16 pays for the spills (500k x 2M matrix 1.32 -> 1.39 ms).  Eight lanes per row spend more on
+// their addresses than on waiting and take the occupancy everywhere (25K rows of 320, N = 32: 90 -> 75).
+constexpr int partition_min_waves(int lpr, int ch, bool bf16, bool resident) {
+    if (ch != 1) return resident ? 4 : 1;
+    if (!bf16) return lpr == 8 ? 6 : resident ? 7 : 1;
+    return resident ? 6 : 1;
+}
+constexpr bool has_resident_kernel(int lpr, int ch, bool bf16) { return bf16 ? ch == 1 : ch <= 2 && lpr > 8; }
+
+template <int LPR, int CH, typename BT, bool RESIDENT>
+__global__ void __launch_bounds__(kWG, partition_min_waves(LPR, CH, Dense<BT>::kVec == 8, RESIDENT))
 spmm_partition_kernel(LaunchArgs a) {
     // one LDS buffer, used either as the staged tile ((col, val) pairs then (row, meta)
     // entries) or as the reduction scratch of a chunk tile (one accumulator per thread)
-    constexpr int kTileSlots = tile_slots(LPR);
+    constexpr int kTileSlots = tile_slots(LPR, RESIDENT && Dense<BT>::kVec == 4);
     constexpr int kStageBytes = (kTileSlots + kTileRows) * (int)sizeof(int2);
     constexpr int kReduceBytes = kWG * CH * Dense<BT>::kVec * (int)sizeof(float);
     __shared__ __align__(16) char s_raw[kStageBytes > kReduceBytes ? kStageBytes : kReduceBytes];
@@ -849,12 +860,13 @@ spmm_rowgroup_kernel(const MergedBucket* __restrict__ buckets, int n_buckets, La
                         w[u] = in ? s_val[idx] : make_float4(0.f, 0.f, 0.f, 0.f);
                         k[u] = in ? s_msk[idx] : 0u;
                     }
-                    float x[U][VEC];
+                    typename Dense<BT>::Raw raw[U];
 #pragma unroll
-                    for (int u = 0; u < U; ++u)
-                        Dense<BT>::load(dense_row<BT>(a.B, ln, 0, c[u]), x[u]);
+                    for (int u = 0; u < U; ++u) raw[u] = load_dense<BT>(a.B, ln, 0, c[u]);
 #pragma unroll
                     for (int u = 0; u < U; ++u) {
+                        float x[VEC];
+                        Dense<BT>::unpack(raw[u], x);
                         const float wr[kGroupRows] = {w[u].x, w[u].y, w[u].z, w[u].w};
 #pragma unroll
                         for (int r = 0; r < kGroupRows; ++r) {
@@ -862,13 +874,13 @@ spmm_rowgroup_kernel(const MergedBucket* __restrict__ buckets, int n_buckets, La
                                 // one group per wavefront: rows without the column are skipped outright
                                 if (__builtin_amdgcn_readfirstlane(k[u]) & (1u << r)) {
 #pragma unroll
-                                    for (int i = 0; i < VEC; ++i) acc[r].v[0][i] = fmaf(wr[r], x[u][i], acc[r].v[0][i]);
+                                    for (int i = 0; i < VEC; ++i) acc[r].v[0][i] = fmaf(wr[r], x[i], acc[r].v[0][i]);
                                 }
                             } else {
                                 // several groups per wavefront: the value is 0 where the row lacks the
                                 // column (like a padded slot, this adds 0 * B: only non-finite B differs)
 #pragma unroll
-                                for (int i = 0; i < VEC; ++i) acc[r].v[0][i] = fmaf(wr[r], x[u][i], acc[r].v[0][i]);
+                                for (int i = 0; i < VEC; ++i) acc[r].v[0][i] = fmaf(wr[r], x[i], acc[r].v[0][i]);
                             }
                         }
                     }
@@ -934,20 +946,19 @@ __device__ __forceinline__ void csr_stream_rows(const int32_t* __restrict__ indi
         next_v = idx < end ? (values ? values[idx] : 1.f) : 0.f;
         const int cnt = min(LPR, end - base);
         for (int j = 0; j < cnt; j += U) {
-            float v[U], x[U][CH][VEC];
+            float v[U];
+            typename Dense<BT>::Raw x[U][CH];
 #pragma unroll
             for (int u = 0; u < U; ++u) {
                 const int c = __shfl(my_c, j + u, LPR);      // past the end: the first column again, value 0
                 v[u] = __shfl(my_v, j + u, LPR);
 #pragma unroll
-                for (int cc = 0; cc < CH; ++cc) Dense<BT>::load(dense_row<BT>(a.B, ln, cc, c), x[u][cc]);
+                for (int cc = 0; cc < CH; ++cc) x[u][cc] = load_dense<BT>(a.B, ln, cc, c);
             }
 #pragma unroll
             for (int u = 0; u < U; ++u) {
 #pragma unroll
-                for (int cc = 0; cc < CH; ++cc)
-#pragma unroll
-                    for (int i = 0; i < VEC; ++i) acc.v[cc][i] = fmaf(v[u], x[u][cc][i], acc.v[cc][i]);
+                for (int cc = 0; cc < CH; ++cc) fma_dense<BT>(v[u], x[u][cc], acc.v[cc]);
                 if (base + j + u + 1 == row_end) {           // the row's last entry
                     store_row<LPR, CH, VEC>(a.C, (int)(first_row + r), ln, acc, kStreamC);
                     acc.clear();
@@ -1461,6 +1472,7 @@ struct lf_spmm_plan {
     };
     std::vector<Launch> launches;
     int coop_slots = kCoopSlots;        // source rows of more slab slots are reduced by whole workgroups
+    bool resident = false;              // parts of B that the L2s hold: the kernels of that case
     bool stream_slabs = false;          // read the slabs non-temporally
     MergedBucket* d_merged = nullptr;   // row-group buckets, grouped by partition
     LfCellBucket* d_cells = nullptr;    // buckets rewritten as cells, grouped by partition
@@ -1500,6 +1512,7 @@ using RowGroupFn = void (*)(const MergedBucket*, int, LaunchArgs);
 
 struct KernelSet {
     KernelFn tiles = nullptr;
+    KernelFn tiles_resident = nullptr;   // the same where there is no such kernel
     FinalFn finalize_wide = nullptr;
     CsrFn csr = nullptr;
     RowGroupFn rowgroup = nullptr;   // one 16-byte chunk per lane only
@@ -1511,11 +1524,13 @@ template <int LPR, int CH> void pick_kernels(int dtype, KernelSet* k) {
         else k->rowgroup = spmm_rowgroup_kernel<LPR, float>;
     }
     if (dtype == LF_DTYPE_BF16) {
-        k->tiles = spmm_partition_kernel<LPR, CH, bf16_t>;
+        k->tiles = spmm_partition_kernel<LPR, CH, bf16_t, false>;
+        k->tiles_resident = spmm_partition_kernel<LPR, CH, bf16_t, has_resident_kernel(LPR, CH, true)>;
         k->finalize_wide = spmm_finalize_wide_kernel<LPR, CH, bf16_t>;
         k->csr = csr_spmm_kernel<LPR, CH, bf16_t>;
     } else {
-        k->tiles = spmm_partition_kernel<LPR, CH, float>;
+        k->tiles = spmm_partition_kernel<LPR, CH, float, false>;
+        k->tiles_resident = spmm_partition_kernel<LPR, CH, float, has_resident_kernel(LPR, CH, false)>;
         k->finalize_wide = spmm_finalize_wide_kernel<LPR, CH, float>;
         k->csr = csr_spmm_kernel<LPR, CH, float>;
     }
@@ -1653,6 +1668,17 @@ int lf_spmm_create(lf_spmm_plan** out_plan, const lf_bucket_desc* h_buckets, int
     // 500k x 2M matrix 1.457 -> 1.443); those of a small one are worth keeping between products
     // (170k-row graph, 6 MB of slabs: 0.073 ms cached, 0.076 ms streamed).
     plan->stream_slabs = total_slots >= kLargeMatrixSlots;
+    // Parts of B that an L2 (4 MB) about holds, and for float products rows that are mostly staged (those of
+    // hundreds of slots per partition stream them by shuffle, which gains nothing: 5774 rows of 368 in two
+    // partitions, N = 288 162 -> 173 us).  A single float partition is not latency-bound enough (10K rows of 182, N =
+    // 64: 36 -> 38); a bf16 one is up to 32 lanes per row (5805 rows of 364, N = 128 46 -> 39).
+    {
+        const bool bf16 = b_dtype == LF_DTYPE_BF16;
+        const long long part_bytes = lf::ceil_div(num_cols, (int64_t)num_parts) * feat_size * (bf16 ? 2 : 4);
+        plan->resident = has_resident_kernel(lpr, ch, bf16) &&
+                         part_bytes <= (num_parts > 1 ? 2 * kL2XcdBytes : bf16 && lpr <= 32 ? kL2XcdBytes : 0) &&
+                         (bf16 || total_slots <= 96 * num_rows * num_parts);
+    }
     // A sub-wave sums kUnroll slots of its row per round trip to B, so a row of kCoopSlots is a
     // chain of 32; where a launch holds few rows of more than 64 slots - a few workgroups per CU - they
     // set its length, and whole workgroups take them too.  (56K-row power-law graph, bf16, N = 128: 33
@@ -1999,7 +2025,7 @@ int lf_spmm_create(lf_spmm_plan** out_plan, const lf_bucket_desc* h_buckets, int
             if (merged_of[k] >= 0 || cell_of[k] >= 0) continue;   // served by the row-group or the cell kernel
             Group g{};
             g.log_w = lf::ilog2(b.width);
-            const int fit = tile_slots(lpr) >> g.log_w;     // ELL rows whose slots fit the LDS tile
+            const int fit = tile_slots(lpr, plan->resident && b_dtype == LF_DTYPE_F32) >> g.log_w;   // ELL rows whose slots fit the LDS tile
             const bool staged = fit >= sw;
             g.type = staged ? (is_multi[k] ? kEllSeg : kEll) : kSeg;
             g.rows_per_tile = staged ? std::min(kTileRows, fit) : std::max(sw, fit);
@@ -2111,27 +2137,24 @@ int lf_spmm_create(lf_spmm_plan** out_plan, const lf_bucket_desc* h_buckets, int
 
     KernelSet ks;
     LF_TRY(select_kernels(lpr, ch, b_dtype, &ks));
-    int occ = 0;
     int dyn_lds = 0;
     plan->grid = 0;
     for (const auto& L : plan->launches) {
         plan->grid = std::max(plan->grid, L.grid);
         dyn_lds = std::max(dyn_lds, L.dyn_lds);
     }
-    LF_TRY_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, ks.tiles, kWG, dyn_lds));
 
     plan->info[0] = total_tiles;
     plan->info[1] = plan->grid;
     plan->info[2] = num_parts;
     {
         hipFuncAttributes fa;
-        LF_TRY_HIP(hipFuncGetAttributes(&fa, reinterpret_cast<const void*>(ks.tiles)));
+        LF_TRY_HIP(hipFuncGetAttributes(&fa, reinterpret_cast<const void*>(plan->resident ? ks.tiles_resident : ks.tiles)));
         plan->info[3] = (int64_t)fa.sharedSizeBytes + dyn_lds;
     }
     plan->info[4] = n_heavy_total;
     plan->info[5] = n_partials;
     plan->info[6] = n_zero;
-    (void)occ;
     plan->info[7] = (int64_t)(merged.size() + cells.size());
     plan->info[8] = (int64_t)cells.size();
     LF_TRY_HIP(read_back());                 // the tables are complete: the plan may run on any stream
@@ -2182,7 +2205,7 @@ int lf_spmm_run(lf_spmm_plan* plan, const void* d_B, float* d_C, lf_stream_t str
             a.coop_slots = plan->coop_slots;
             std::memcpy(a.n_tiles, L.n_tiles, sizeof(a.n_tiles));
             if (L.grid > 0) {
-                ks.tiles<<<L.grid, kWG, L.dyn_lds, s>>>(a);
+                (plan->resident ? ks.tiles_resident : ks.tiles)<<<L.grid, kWG, L.dyn_lds, s>>>(a);
                 LF_HIP(hipGetLastError());
             }
             if (L.n_merged > 0) {

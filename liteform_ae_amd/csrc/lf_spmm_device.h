@@ -22,9 +22,11 @@ constexpr int kWG = 256;            // threads per workgroup (4 wavefronts)
 #endif
 // (col, val) pairs staged in LDS per tile: a fixed amount of work per sub-wave, so narrow
 // feature sizes (many sub-waves per workgroup) get larger tiles.  N = 128 -> 512 slots.
-constexpr int tile_slots(int lpr) {
+// `resident`: see spmm_partition_kernel.
+constexpr int tile_slots(int lpr, bool resident) {
     const int n = LF_TILE_SLOTS_PER_SUBWAVE * (kWG / lpr);
-    return n < LF_TILE_MIN ? LF_TILE_MIN : n;
+    const int least = resident && lpr >= 32 ? 2 * LF_TILE_MIN : LF_TILE_MIN;
+    return n < least ? least : n;
 }
 constexpr int kTileRows = 512;      // ELL rows per tile at most (<= tile_slots)
 #ifndef LF_COOP_SLOTS
@@ -117,8 +119,8 @@ template <typename BT> struct Dense;
 template <> struct Dense<float> {
     static constexpr int kVec = 4;
     static constexpr int kElemBytes = 4;
-    __device__ static __forceinline__ void load(const char* at, float (&x)[4]) {
-        const float4 v = *reinterpret_cast<const float4*>(at);
+    using Raw = float4;
+    __device__ static __forceinline__ void unpack(const Raw& v, float (&x)[4]) {
         x[0] = v.x; x[1] = v.y; x[2] = v.z; x[3] = v.w;
     }
 };
@@ -128,8 +130,8 @@ struct bf16_t { uint16_t bits; };
 template <> struct Dense<bf16_t> {
     static constexpr int kVec = 8;
     static constexpr int kElemBytes = 2;
-    __device__ static __forceinline__ void load(const char* at, float (&x)[8]) {
-        const uint4 v = *reinterpret_cast<const uint4*>(at);
+    using Raw = uint4;
+    __device__ static __forceinline__ void unpack(const Raw& v, float (&x)[8]) {
         x[0] = __uint_as_float(v.x << 16); x[1] = __uint_as_float(v.x & 0xFFFF0000u);
         x[2] = __uint_as_float(v.y << 16); x[3] = __uint_as_float(v.y & 0xFFFF0000u);
         x[4] = __uint_as_float(v.z << 16); x[5] = __uint_as_float(v.z & 0xFFFF0000u);
@@ -178,23 +180,35 @@ __device__ __forceinline__ const char* dense_row(const void* B, const Lane<LPR, 
     return lane0 + (uint64_t)(uint32_t)col * pitch;
 }
 
+template <typename BT, int LPR, int CH>
+__device__ __forceinline__ typename Dense<BT>::Raw load_dense(const void* B, const Lane<LPR, CH, Dense<BT>::kVec>& ln,
+                                                              int c, int col) {
+    return *reinterpret_cast<const typename Dense<BT>::Raw*>(dense_row<BT>(B, ln, c, col));
+}
+
+// acc += v * x.  The 16 bytes stay as they were loaded until here: unpacked while further loads are in
+// flight, bf16 would hold twice the registers.
+template <typename BT>
+__device__ __forceinline__ void fma_dense(float v, const typename Dense<BT>::Raw& raw, float (&acc)[Dense<BT>::kVec]) {
+    float x[Dense<BT>::kVec];
+    Dense<BT>::unpack(raw, x);
+#pragma unroll
+    for (int i = 0; i < Dense<BT>::kVec; ++i) acc[i] = fmaf(v, x[i], acc[i]);
+}
+
 template <int U, int LPR, int CH, typename BT>
 __device__ __forceinline__ void gather_fma(const void* B, const Lane<LPR, CH, Dense<BT>::kVec>& ln,
                                            const int (&col)[U], const float (&val)[U],
                                            Acc<CH, Dense<BT>::kVec>& acc) {
-    constexpr int VEC = Dense<BT>::kVec;
-    float x[U][CH][VEC];
+    typename Dense<BT>::Raw x[U][CH];
 #pragma unroll
     for (int u = 0; u < U; ++u)
 #pragma unroll
-        for (int c = 0; c < CH; ++c)
-            Dense<BT>::load(dense_row<BT>(B, ln, c, col[u]), x[u][c]);
+        for (int c = 0; c < CH; ++c) x[u][c] = load_dense<BT>(B, ln, c, col[u]);
 #pragma unroll
     for (int u = 0; u < U; ++u)
 #pragma unroll
-        for (int c = 0; c < CH; ++c)
-#pragma unroll
-            for (int i = 0; i < VEC; ++i) acc.v[c][i] = fmaf(val[u], x[u][c][i], acc.v[c][i]);
+        for (int c = 0; c < CH; ++c) fma_dense<BT>(val[u], x[u][c], acc.v[c]);
 }
 
 // flags: LaunchArgs::accumulate.  Rows that nothing reads again in this run are stored
@@ -202,7 +216,8 @@ __device__ __forceinline__ void gather_fma(const void* B, const Lane<LPR, CH, De
 // (170k-row graph, two partitions: streaming them costs 7 %).
 constexpr int kAccumulateC = 1, kStreamC = 2, kStreamSlabs = 4;
 constexpr int kStreamMinWidth = 16;      // a launch of mostly wide rows: at least half of its ELL rows are this wide
-constexpr long long kL2Bytes = 32ll << 20;   // of the eight XCDs together
+constexpr long long kL2XcdBytes = 4ll << 20;
+constexpr long long kL2Bytes = 8 * kL2XcdBytes;   // of the eight XCDs together
 typedef float lf_f32x4 __attribute__((ext_vector_type(4)));
 
 // 16 bytes to global memory, streamed or not by a run-time flag.  The streaming store goes

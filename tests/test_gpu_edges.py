@@ -237,3 +237,23 @@ def test_rows_around_the_cooperative_length(fa, torch, feat, b_dtype, n_long):
     Bh = B.float().cpu().numpy()
     assert (np.abs(got - O.spmm_csr_f64(indptr, indices, data, (len(lens), nc), Bh))
             <= 1e-5 * O.spmm_abs_bound(indptr, indices, data, (len(lens), nc), Bh)).all()
+
+
+@pytest.mark.parametrize("feat,b_dtype", [(32, "f32"), (64, "f32"), (96, "f32"), (288, "f32"), (64, "bf16"), (256, "bf16"), (512, "bf16")])
+@pytest.mark.parametrize("parts,n_rows", [(1, 700), (2, 17), (3, 8192 + 5)])
+def test_parts_of_b_that_the_l2_holds(fa, torch, feat, b_dtype, parts, n_rows):
+    """The kernels of launches whose part of B stays in the L2: every staged width, tiles that are
+    full and not, rows of several ELL rows, and rows that only some partitions add to."""
+    rng = np.random.default_rng(feat + parts)
+    nc = 600
+    lens = rng.integers(0, 130, size=n_rows) >> rng.integers(0, 7, size=n_rows)
+    row = np.repeat(np.arange(n_rows), lens)
+    pos = np.arange(len(row)) - np.repeat(np.cumsum(lens) - lens, lens)
+    g = MTX.from_coo(row, (row * 17 + pos * 7) % nc, (n_rows, nc), data=rng.uniform(-1, 1, size=len(row)).astype(np.float32))
+    B = torch.from_numpy(rng.uniform(-1, 1, size=(nc, feat)).astype(np.float32)).cuda().to(torch.bfloat16 if b_dtype == "bf16" else torch.float32)
+    fmt = fa.build_hyb_format_device(g, [[1, 2, 4, 8, 16, 32, 64]] * parts)
+    got = fa.HybSpMM(fmt, feat, b_dtype).run(B).cpu().numpy()
+    indptr, indices, data = g.adj_tensors("csr")
+    Bh = B.float().cpu().numpy()
+    assert (np.abs(got - O.spmm_csr_f64(indptr, indices, data, (n_rows, nc), Bh))
+            <= 1e-5 * O.spmm_abs_bound(indptr, indices, data, (n_rows, nc), Bh)).all()
