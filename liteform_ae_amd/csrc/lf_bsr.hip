@@ -37,7 +37,11 @@
 namespace {
 
 constexpr int kFeatTile = 128;     // features per wavefront
-constexpr int kWgBsr = 256;        // four wavefronts, independent of each other
+constexpr int kWgBsr = 256;        // four wavefronts, independent of each other; one where there are few
+// A product of up to this many wavefronts goes out one by one, which spreads them over the CUs (40K x 40K,
+// blocks of 32, N = 128: 15.9 -> 14.5 us, N = 24 10.5 -> 9.5); a larger one is bound by memory and gains 1 to
+// 3 % from four block rows side by side, and feature tiles of one block row share its blocks in the L1.
+constexpr long long kFewUnits = 4096;
 
 // A Y of this size or more is stored past the caches, which leaves them to X (128K x 128K, blocks of 32,
 // N = 512: 104 -> 96 us; 1M x 1M, N = 256: 759 -> 734); a smaller one the next operation may find there.
@@ -64,7 +68,7 @@ bsr_spmm_kernel(const int32_t* __restrict__ indptr, const int32_t* __restrict__ 
     constexpr int BPS = BS == 16 ? 2 : 1;                // blocks per step
     const int lane = threadIdx.x & 63, li = lane & 15, kq = lane >> 4;
     // the feature tiles of a block row go to neighbouring wavefronts, which read the same blocks of A
-    const long long unit = (long long)blockIdx.x * (kWgBsr / 64) + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const long long unit = (long long)blockIdx.x * (blockDim.x / 64) + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     if (unit >= n_units) return;
     const int brow = (int)(unit / n_tiles);
     const int f = (int)(unit % n_tiles) * kFeatTile + 8 * li;
@@ -176,13 +180,15 @@ int lf_bsr_spmm_trusted(const int32_t* d_indptr, const int32_t* d_indices, const
     LF_REQUIRE((uintptr_t)d_X % 16 == 0 && (uintptr_t)d_Y % 16 == 0 && (uintptr_t)d_data % 16 == 0, LF_ERR_INVALID,
                "X, Y and the block data must be 16-byte aligned");
     const int n_tiles = (feat_size + kFeatTile - 1) / kFeatTile;
-    const long long units = (long long)num_block_rows * n_tiles, groups = lf::ceil_div(units, kWgBsr / 64);
+    const long long units = (long long)num_block_rows * n_tiles;
+    const int threads = n_tiles == 1 && units <= kFewUnits ? 64 : kWgBsr;
+    const long long groups = lf::ceil_div(units, threads / 64);
     LF_REQUIRE(groups < (1ll << 31), LF_ERR_UNSUPPORTED, "too many block rows and features");
     const _Float16* data = (const _Float16*)d_data;
     const _Float16* X = (const _Float16*)d_X;
     _Float16* Y = (_Float16*)d_Y;
     const auto kernel = block_size == 16 ? bsr_spmm_kernel<16> : block_size == 32 ? bsr_spmm_kernel<32> : bsr_spmm_kernel<64>;
-    kernel<<<(unsigned)groups, kWgBsr, 0, s>>>(d_indptr, d_indices, data, X, Y, feat_size, n_tiles, units,
+    kernel<<<(unsigned)groups, threads, 0, s>>>(d_indptr, d_indices, data, X, Y, feat_size, n_tiles, units,
                                               (int64_t)num_block_rows * block_size * feat_size * 2 >= kStreamYBytes);
     LF_HIP(hipGetLastError());
     return LF_OK;

@@ -615,6 +615,9 @@ def spmm_hyb(fmt: HybFormat, B, b_dtype: str = "f32"):
     return out
 
 
+_B_DTYPES = {"f32": _lib.LF_DTYPE_F32, "bf16": _lib.LF_DTYPE_BF16}
+
+
 def spmm_csr(g, B, b_dtype: str = "f32", use_values: bool = True):
     """Row-parallel CSR product on the GPU (kernel of bench_naive, format_algos.py:1689-1755)."""
     torch = _torch()
@@ -622,11 +625,13 @@ def spmm_csr(g, B, b_dtype: str = "f32", use_values: bool = True):
     dev = _device_csr(g)
     feat = int(B.shape[1])
     out = torch.empty((dev.num_rows, feat), dtype=torch.float32, device="cuda")
-    dt = {"f32": _lib.LF_DTYPE_F32, "bf16": _lib.LF_DTYPE_BF16}[b_dtype]
     vals = dev.values if use_values else None
     # the device arrays were made by lf_coo_to_csr or have passed lf_csr_check: no second check
-    _lib.check(lib.lf_csr_spmm_trusted(_lib.ptr(dev.indptr), _lib.ptr(dev.indices), _lib.ptr(vals), dev.num_rows,
-                                       dev.num_cols, feat, dt, B.data_ptr(), out.data_ptr(), _stream()))
+    rc = lib.lf_csr_spmm_trusted(dev.indptr.data_ptr(), dev.indices.data_ptr(), None if vals is None else vals.data_ptr(),
+                                 dev.num_rows, dev.num_cols, feat, _B_DTYPES[b_dtype], B.data_ptr(), out.data_ptr(),
+                                 _stream())
+    if rc:
+        _lib.check(rc)
     return out
 
 
@@ -685,6 +690,8 @@ def bench_hyb_with_config(g, x, y_ndarray, feat_size=128, bucket_widths=[], buck
 class _DeviceBSR:
     """scipy BSR arrays on the GPU: int32 index arrays, fp16 blocks."""
 
+    checked = False                   # the first product checks the block index arrays on the GPU
+
     def __init__(self, bsr_mat, block_size: int):
         torch = _torch()
         if tuple(bsr_mat.blocksize) != (block_size, block_size):
@@ -699,7 +706,6 @@ class _DeviceBSR:
         self.indptr = torch.from_numpy(np.ascontiguousarray(bsr_mat.indptr, dtype=np.int32)).cuda()
         self.indices = torch.from_numpy(np.ascontiguousarray(bsr_mat.indices, dtype=np.int32)).cuda()
         self.data = torch.from_numpy(np.ascontiguousarray(bsr_mat.data, dtype=np.float16).reshape(-1)).cuda()
-        self.checked = False          # the first product checks the block index arrays on the GPU
 
 
 def spmm_bsr(bsr, x, block_size: int = 32):
@@ -708,19 +714,21 @@ def spmm_bsr(bsr, x, block_size: int = 32):
     torch = _torch()
     lib = _lib.load()
     dev = bsr if isinstance(bsr, _DeviceBSR) else _DeviceBSR(bsr, block_size)
-    feat = int(x.shape[1])
+    feat = x.shape[1]
     if x.dtype != torch.float16 or not x.is_cuda or not x.is_contiguous() or x.shape[0] != dev.nb * dev.block_size:
         raise ValueError(f"x must be a contiguous CUDA fp16 tensor with {dev.nb * dev.block_size} rows")
-    y = torch.empty((dev.mb * dev.block_size, feat), dtype=torch.float16, device="cuda")
-    if not getattr(dev, "checked", False):
+    y = x.new_empty((dev.mb * dev.block_size, feat))
+    if not dev.checked:
         scratch = torch.empty(4, dtype=torch.int32, device="cuda")
         _lib.check(lib.lf_bsr_spmm(_lib.ptr(dev.indptr), _lib.ptr(dev.indices), _lib.ptr(dev.data), dev.mb, dev.nb,
                                    dev.nnzb, dev.block_size, feat, x.data_ptr(), y.data_ptr(), _lib.ptr(scratch),
                                    _stream()))
         dev.checked = True
     else:
-        _lib.check(lib.lf_bsr_spmm_trusted(_lib.ptr(dev.indptr), _lib.ptr(dev.indices), _lib.ptr(dev.data), dev.mb,
-                                           dev.nb, dev.block_size, feat, x.data_ptr(), y.data_ptr(), _stream()))
+        rc = lib.lf_bsr_spmm_trusted(dev.indptr.data_ptr(), dev.indices.data_ptr(), dev.data.data_ptr(), dev.mb,
+                                     dev.nb, dev.block_size, feat, x.data_ptr(), y.data_ptr(), _stream())
+        if rc:
+            _lib.check(rc)
     return y
 
 

@@ -142,3 +142,9 @@ def test_every_short_block_row(fa, torch, feat, bs):
     indices = np.concatenate([np.sort(rng.choice(12, size=n, replace=False)) for n in counts]).astype(np.int32)
     data = rng.uniform(-1, 1, size=(len(indices), bs, bs)).astype(np.float16).astype(np.float32)
     check(fa, torch, sp.bsr_matrix((data, indices, indptr), shape=(10 * bs, 12 * bs)), feat)
+
+
+@pytest.mark.parametrize("mb,feat", [(4095, 40), (4096, 128), (4097, 40), (4099, 136)])
+def test_wavefronts_alone_and_in_fours(fa, torch, mb, feat):
+    """Up to 4096 block rows of one feature tile go out as single wavefronts, more in workgroups of four."""
+    check(fa, torch, random_bsr(np.random.default_rng(mb), mb, 50, 2, bs=16), feat)
