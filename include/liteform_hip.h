@@ -353,13 +353,17 @@ int lf_coo_to_csr(const int32_t* d_coo_row, const int32_t* d_coo_col, const floa
  * lf_bsr_spmm checks the block index arrays like lf_csr_check (d_scratch: 16 bytes of device
  * memory; synchronises for the verdict) and returns LF_ERR_INVALID without launching the
  * product when they fail; lf_bsr_spmm_trusted only enqueues the kernel, for arrays that have
- * passed the check before. */
+ * passed the check before; lf_bsr_spmm_trusted_nnz does the same and is told the number of blocks
+ * (0: not known), by which it chooses the launch. */
 int lf_bsr_spmm(const int32_t* d_indptr, const int32_t* d_indices, const void* d_data,
                 int64_t num_block_rows, int64_t num_block_cols, int64_t nnz_blocks, int32_t block_size,
                 int32_t feat_size, const void* d_X, void* d_Y, void* d_scratch, lf_stream_t stream);
 int lf_bsr_spmm_trusted(const int32_t* d_indptr, const int32_t* d_indices, const void* d_data,
                         int64_t num_block_rows, int64_t num_block_cols, int32_t block_size,
                         int32_t feat_size, const void* d_X, void* d_Y, lf_stream_t stream);
+int lf_bsr_spmm_trusted_nnz(const int32_t* d_indptr, const int32_t* d_indices, const void* d_data,
+                            int64_t num_block_rows, int64_t num_block_cols, int64_t nnz_blocks, int32_t block_size,
+                            int32_t feat_size, const void* d_X, void* d_Y, lf_stream_t stream);
 
 #ifdef __cplusplus
 }

@@ -24,7 +24,7 @@
 // steps of 32 columns.  The loads of the next step are under way during the products of this one.
 // The kernel before this transposed X through LDS in 2-byte stores, with a barrier and one block's
 // loads in flight per workgroup: 1M x 1M, 8 blocks per block row, N = 128, blocks of 16 / 32 / 64:
-// 0.517 / 0.424 / 0.533 -> 0.382 / 0.411 / 0.509 ms, N = 256, blocks of 32: 0.896 -> 0.758 (all at
+// 0.517 / 0.424 / 0.533 -> 0.369 / 0.394 / 0.493 ms, N = 256, blocks of 32: 0.896 -> 0.728 (all at
 // 7 TB/s of A blocks and rows of X, what a gather that misses the L2s reaches); 40K x 40K, blocks of
 // 16, N = 200: 45 -> 20 us.
 #include <hip/hip_runtime.h>
@@ -37,11 +37,18 @@
 namespace {
 
 constexpr int kFeatTile = 128;     // features per wavefront
-constexpr int kWgBsr = 256;        // four wavefronts, independent of each other; one where there are few
-// A product of up to this many wavefronts goes out one by one, which spreads them over the CUs (40K x 40K,
-// blocks of 32, N = 128: 15.9 -> 14.5 us, N = 24 10.5 -> 9.5); a larger one is bound by memory and gains 1 to
-// 3 % from four block rows side by side, and feature tiles of one block row share its blocks in the L1.
+
+// Wavefronts per workgroup; they are independent of each other.  Up to kFewUnits of them go out one by one, which
+// spreads them over the CUs (40K x 40K, blocks of 32, N = 128: 15.9 -> 14.5 us, N = 24 10.5 -> 9.5);
+// otherwise four, so that the feature tiles of a block row share its blocks in the L1.  Where a
+// product is bound by memory throughout - large, whole tiles of features, long block rows - eight that
+// start together move 2 to 6 % more (1M x 1M, 8 blocks a row, N = 128, blocks of 32 / 16: 405 / 383 ->
+// 394 / 369 us; 800K x 800K, 7 blocks of 16, N = 384: 720 -> 673); with short block rows the CU waits
+// for the last of eight (800K x 800K, 2 blocks a row, N = 128: 105 -> 110).  Two such workgroups of blocks of
+// 64 would not have the registers.
 constexpr long long kFewUnits = 4096;
+constexpr int kLongBlockRow = 6;       // blocks
+constexpr int most_threads(int block) { return block == 64 ? 256 : 512; }
 
 // A Y of this size or more is stored past the caches, which leaves them to X (128K x 128K, blocks of 32,
 // N = 512: 104 -> 96 us; 1M x 1M, N = 256: 759 -> 734); a smaller one the next operation may find there.
@@ -59,7 +66,7 @@ template <int BS> struct BsrStep {
 };
 
 template <int BS>
-__global__ void __launch_bounds__(kWgBsr)
+__global__ void __launch_bounds__(most_threads(BS))
 bsr_spmm_kernel(const int32_t* __restrict__ indptr, const int32_t* __restrict__ indices,
                 const _Float16* __restrict__ data, const _Float16* __restrict__ X,
                 _Float16* __restrict__ Y, int feat, int n_tiles, long long n_units, int stream_y) {
@@ -165,9 +172,9 @@ bsr_spmm_kernel(const int32_t* __restrict__ indptr, const int32_t* __restrict__ 
 
 extern "C" {
 
-int lf_bsr_spmm_trusted(const int32_t* d_indptr, const int32_t* d_indices, const void* d_data,
-                        int64_t num_block_rows, int64_t num_block_cols, int32_t block_size,
-                        int32_t feat_size, const void* d_X, void* d_Y, lf_stream_t stream) {
+int lf_bsr_spmm_trusted_nnz(const int32_t* d_indptr, const int32_t* d_indices, const void* d_data,
+                            int64_t num_block_rows, int64_t num_block_cols, int64_t nnz_blocks, int32_t block_size,
+                            int32_t feat_size, const void* d_X, void* d_Y, lf_stream_t stream) {
     hipStream_t s = (hipStream_t)stream;
     LF_REQUIRE(block_size == 16 || block_size == 32 || block_size == 64, LF_ERR_UNSUPPORTED,
                "blocks of 16, 32 or 64 rows and columns are supported (got %d)", block_size);
@@ -181,7 +188,9 @@ int lf_bsr_spmm_trusted(const int32_t* d_indptr, const int32_t* d_indices, const
                "X, Y and the block data must be 16-byte aligned");
     const int n_tiles = (feat_size + kFeatTile - 1) / kFeatTile;
     const long long units = (long long)num_block_rows * n_tiles;
-    const int threads = n_tiles == 1 && units <= kFewUnits ? 64 : kWgBsr;
+    const bool stream_y = (int64_t)num_block_rows * block_size * feat_size * 2 >= kStreamYBytes;
+    const bool eight = block_size != 64 && stream_y && feat_size % kFeatTile == 0 && nnz_blocks >= kLongBlockRow * num_block_rows;
+    const int threads = n_tiles == 1 && units <= kFewUnits ? 64 : eight ? 512 : 256;
     const long long groups = lf::ceil_div(units, threads / 64);
     LF_REQUIRE(groups < (1ll << 31), LF_ERR_UNSUPPORTED, "too many block rows and features");
     const _Float16* data = (const _Float16*)d_data;
@@ -189,9 +198,16 @@ int lf_bsr_spmm_trusted(const int32_t* d_indptr, const int32_t* d_indices, const
     _Float16* Y = (_Float16*)d_Y;
     const auto kernel = block_size == 16 ? bsr_spmm_kernel<16> : block_size == 32 ? bsr_spmm_kernel<32> : bsr_spmm_kernel<64>;
     kernel<<<(unsigned)groups, threads, 0, s>>>(d_indptr, d_indices, data, X, Y, feat_size, n_tiles, units,
-                                              (int64_t)num_block_rows * block_size * feat_size * 2 >= kStreamYBytes);
+                                              stream_y);
     LF_HIP(hipGetLastError());
     return LF_OK;
+}
+
+int lf_bsr_spmm_trusted(const int32_t* d_indptr, const int32_t* d_indices, const void* d_data,
+                        int64_t num_block_rows, int64_t num_block_cols, int32_t block_size,
+                        int32_t feat_size, const void* d_X, void* d_Y, lf_stream_t stream) {
+    return lf_bsr_spmm_trusted_nnz(d_indptr, d_indices, d_data, num_block_rows, num_block_cols, 0, block_size, feat_size,
+                                   d_X, d_Y, stream);
 }
 
 int lf_bsr_spmm(const int32_t* d_indptr, const int32_t* d_indices, const void* d_data,
@@ -205,8 +221,8 @@ int lf_bsr_spmm(const int32_t* d_indptr, const int32_t* d_indices, const void* d
     if (int rc = lf::csr_check(d_indptr, d_indices, nullptr, num_block_rows, num_block_cols, nnz_blocks, d_scratch, nullptr,
                                "lf_bsr_spmm", (hipStream_t)stream))
         return rc;
-    return lf_bsr_spmm_trusted(d_indptr, d_indices, d_data, num_block_rows, num_block_cols, block_size, feat_size,
-                               d_X, d_Y, stream);
+    return lf_bsr_spmm_trusted_nnz(d_indptr, d_indices, d_data, num_block_rows, num_block_cols, nnz_blocks, block_size,
+                                   feat_size, d_X, d_Y, stream);
 }
 
 }  // extern "C"

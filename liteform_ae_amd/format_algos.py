@@ -725,8 +725,8 @@ def spmm_bsr(bsr, x, block_size: int = 32):
                                    _stream()))
         dev.checked = True
     else:
-        rc = lib.lf_bsr_spmm_trusted(dev.indptr.data_ptr(), dev.indices.data_ptr(), dev.data.data_ptr(), dev.mb,
-                                     dev.nb, dev.block_size, feat, x.data_ptr(), y.data_ptr(), _stream())
+        rc = lib.lf_bsr_spmm_trusted_nnz(dev.indptr.data_ptr(), dev.indices.data_ptr(), dev.data.data_ptr(), dev.mb,
+                                         dev.nb, dev.nnzb, dev.block_size, feat, x.data_ptr(), y.data_ptr(), _stream())
         if rc:
             _lib.check(rc)
     return y

@@ -148,3 +148,19 @@ def test_every_short_block_row(fa, torch, feat, bs):
 def test_wavefronts_alone_and_in_fours(fa, torch, mb, feat):
     """Up to 4096 block rows of one feature tile go out as single wavefronts, more in workgroups of four."""
     check(fa, torch, random_bsr(np.random.default_rng(mb), mb, 50, 2, bs=16), feat)
+
+
+@pytest.mark.parametrize("bs,mb,feat", [(16, 16384, 128), (16, 8195, 256), (32, 8193, 128), (32, 4100, 256)])
+def test_long_block_rows_of_a_large_product(fa, torch, bs, mb, feat):
+    """Workgroups of eight wavefronts: six blocks a row, whole feature tiles, Y of 64 MB or more."""
+    rng = np.random.default_rng(mb)
+    cols = np.sort((rng.integers(0, 40, size=(mb, 1)) + np.arange(6) * 7) % 40, axis=1)
+    data = rng.uniform(-1, 1, size=(mb * 6, bs, bs)).astype(np.float16)
+    a = sp.bsr_matrix((data.astype(np.float32), cols.ravel(), np.arange(0, 6 * mb + 1, 6)), shape=(mb * bs, 40 * bs))
+    x = torch.rand((40 * bs, feat), device="cuda").sub_(0.5).to(torch.float16)
+    y = fa.spmm_bsr(a, x, block_size=bs)
+    xb = x.float().view(40, bs, feat)[torch.from_numpy(cols).cuda()]                # [mb, 6, bs, feat]
+    ab = torch.from_numpy(data).cuda().float().view(mb, 6, bs, bs)
+    for r in range(0, mb, 512):
+        ref = torch.matmul(ab[r:r + 512], xb[r:r + 512]).sum(1).view(-1, feat)
+        assert (y[r * bs:(r + 512) * bs].float() - ref).abs().max() < 2e-2
