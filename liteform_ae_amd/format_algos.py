@@ -281,13 +281,10 @@ class _DeviceCSR:
 
 
 def _matrix_identity(g):
-    """The object whose replacement means "another matrix": the CSR arrays or the triplets a
-    container was made from, else its COO matrix."""
-    for name in ("_csr_source", "_triplets"):
-        src = getattr(g, name, None)
-        if src is not None:
-            return src
-    return g.coo_mtx
+    """The object whose replacement means "another matrix": the container's own token, or the COO
+    matrix of a container that has none."""
+    token = getattr(g, "_identity", None)
+    return g.coo_mtx if token is None else token
 
 
 def _device_csr(g) -> _DeviceCSR:

@@ -72,6 +72,7 @@ class MTX:
         self._csr_source = None       # the CSR matrix this container was made from (from_csr), as given
         self._triplets = None         # (row, col, data, shape) this container was made from (from_coo)
         self._unit_values = False     # from_csr without data: every stored value is 1
+        self._identity = object()     # replaced with the matrix: what a copy on the GPU is kept under
         if filename is None:
             self.name = None
         elif filename in _GRAPH_DATASETS:
@@ -88,9 +89,17 @@ class MTX:
 
     # ``coo_mtx`` is the reference's one data attribute (format_matrix_market.py:44-46).  A
     # container made from CSR arrays or checked triplets keeps them and builds the COO view only
-    # when it is asked for, so that they can go to the GPU as they are.
+    # when it is asked for, so that they can go to the GPU as they are.  Whoever holds the view may
+    # change it in place (sum_duplicates, eliminate_zeros, ``.data = ...``): once it has been handed
+    # out it is the matrix, and the triplets it was built from are let go.
     @property
     def coo_mtx(self):
+        coo = self._coo_view()
+        self._triplets = None
+        return coo
+
+    def _coo_view(self):
+        """The COO view for use inside this class, where nothing is changed through it."""
         if self._coo is None:
             if self._csr_source is not None:
                 self._coo = self._csr_source.tocoo()
@@ -106,6 +115,7 @@ class MTX:
         self._csr_source = None
         self._triplets = None
         self._unit_values = False
+        self._identity = object()
 
     # ---- constructors without a file -------------------------------------------------
     @classmethod
@@ -147,19 +157,19 @@ class MTX:
             if src is not None and src.has_canonical_format:
                 self._csr = src
             else:
-                self._csr = self.coo_mtx.tocsr()
+                self._csr = self._coo_view().tocsr()
         return self._csr
 
     def _shape(self):
         if self._coo is None and self._triplets is not None:
             return self._triplets[3]
-        return (self._csr_source if self._coo is None and self._csr_source is not None else self.coo_mtx).shape
+        return (self._csr_source if self._coo is None and self._csr_source is not None else self._coo_view()).shape
 
     def adj_tensors(self, format: str):
         if format == "coo":
             return self.coo_mtx.row, self.coo_mtx.col
         elif format == "csc":
-            csc = self.coo_mtx.tocsc()
+            csc = self._coo_view().tocsc()
             return csc.indptr, csc.indices, csc.data
         elif format == "csr":
             csr = self._csr_view()
@@ -178,27 +188,27 @@ class MTX:
             return self._csr_source.nnz
         if self._coo is None and self._triplets is not None:
             return len(self._triplets[2])
-        return self.coo_mtx.nnz
+        return self._coo_view().nnz
 
     def dot(self, B):
         """A @ B through scipy (format_matrix_market.py:89-99)."""
-        return self.coo_mtx.tocsc().dot(B)
+        return self._coo_view().tocsc().dot(B)
 
     def tobsr(self, blocksize=None, copy=False):
         """scipy BSR view (format_matrix_market.py:101-112)."""
-        return self.coo_mtx.tobsr(blocksize=blocksize, copy=copy)
+        return self._coo_view().tobsr(blocksize=blocksize, copy=copy)
 
     def tobsr_with_padding(self, shape, blocksize=None):
         """BSR matrix of the given (padded) shape with fp16-valued entries, shape % blocksize == 0
         (format_matrix_market.py:115-136).  The reference stores the values as float16; scipy
         1.15 no longer accepts that dtype in sparse containers, so the values are rounded to
         fp16 and held as float32 (every value is exactly representable in fp16)."""
-        data = np.array(self.coo_mtx.data, dtype=np.float16).astype(np.float32)
-        ij = [self.coo_mtx.row, self.coo_mtx.col]
+        data = np.array(self._coo_view().data, dtype=np.float16).astype(np.float32)
+        ij = [self._coo_view().row, self._coo_view().col]
         return sp.bsr_matrix((data, ij), blocksize=blocksize, shape=shape)
 
     def tocsr(self, copy=False):
-        return self.coo_mtx.tocsr(copy=copy)
+        return self._coo_view().tocsr(copy=copy)
 
     def matrix_features(self):
         """Row-length statistics used by the format selector
@@ -225,4 +235,4 @@ class MTX:
         }
 
     def __str__(self):
-        return str(self.coo_mtx)
+        return str(self._coo_view())

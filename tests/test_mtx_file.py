@@ -80,6 +80,58 @@ def test_mtx_path_reads_pattern_and_forces_ones(mtx_file):
     np.testing.assert_array_equal(g.dot(B), want @ B)
 
 
+def _sent_to_the_gpu(monkeypatch, g):
+    """What _DeviceCSR would upload for g: ("csr" or "coo", its arrays, its entry count)."""
+    import types
+    from liteform_ae_amd import format_algos as fa
+
+    class Recorder(fa._DeviceCSR):
+        def _from_csr(self, csr, unit_values):
+            self.sent = tuple(np.array(x) for x in (csr.indptr, csr.indices, csr.data))
+            return True
+
+        def _from_coo(self, row, col, data):
+            self.sent = tuple(np.array(x) for x in (row, col, data))
+
+    stream = types.SimpleNamespace(synchronize=lambda: None)
+    monkeypatch.setattr(fa, "_torch", lambda: types.SimpleNamespace(cuda=types.SimpleNamespace(current_stream=lambda: stream)))
+    dev = Recorder(g)
+    return dev.path, dev.sent, dev.coo_nnz
+
+
+def _edits():
+    """In-place changes of a COO matrix, each through what scipy offers for it."""
+    def new_data(coo):
+        coo.data = np.full(len(coo.data), 3.0, dtype=np.float32)
+    return [lambda coo: coo.sum_duplicates(), lambda coo: coo.eliminate_zeros(), new_data]
+
+
+@pytest.mark.parametrize("edit", _edits(), ids=["sum_duplicates", "eliminate_zeros", "data"])
+def test_changes_of_the_coo_view_reach_the_gpu(monkeypatch, edit):
+    """A container made from triplets: what is done to its COO view before the first use counts."""
+    row, col = np.array([0, 0, 2], dtype=np.int32), np.array([1, 1, 0], dtype=np.int32)
+    data = np.array([1.0, 2.0, 0.0], dtype=np.float32)
+    g = MTX.from_coo(row, col, (3, 2), data=data)
+    assert _sent_to_the_gpu(monkeypatch, g)[1][2] is not None
+    edit(g.coo_mtx)
+    want = sp.coo_matrix((data, (row, col)), shape=(3, 2))
+    edit(want)
+    path, sent, nnz = _sent_to_the_gpu(monkeypatch, g)
+    assert path == "coo" and nnz == g.num_edges() == want.nnz
+    for got, ref in zip(sent, (want.row, want.col, want.data)):
+        np.testing.assert_array_equal(got, ref)
+
+
+def test_a_copy_on_the_gpu_is_kept_until_the_matrix_is_replaced():
+    """Looking at the COO view is no new matrix; assigning one is."""
+    from liteform_ae_amd import format_algos as fa
+    g = MTX.from_coo(np.array([0, 1], dtype=np.int32), np.array([1, 0], dtype=np.int32), (2, 2))
+    before = fa._matrix_identity(g)
+    assert g.coo_mtx.nnz == 2 and g.dot(np.eye(2)).shape == (2, 2) and fa._matrix_identity(g) is before
+    g.coo_mtx = sp.identity(2, format="coo")
+    assert fa._matrix_identity(g) is not before
+
+
 @pytest.mark.gpu
 def test_mtx_path_through_the_gpu_pipeline(mtx_file):
     import torch
