@@ -91,12 +91,19 @@ class MTX:
     # container made from CSR arrays or checked triplets keeps them and builds the COO view only
     # when it is asked for, so that they can go to the GPU as they are.  Whoever holds the view may
     # change it in place (sum_duplicates, eliminate_zeros, ``.data = ...``): once it has been handed
-    # out it is the matrix, and the triplets it was built from are let go.
+    # out it is the matrix, and the arrays it was built from are let go.
     @property
     def coo_mtx(self):
         coo = self._coo_view()
-        self._triplets = None
+        self._forget_sources()
         return coo
+
+    def _forget_sources(self):
+        if self._csr is not None and self._csr is self._csr_source:
+            self._csr = None
+        self._csr_source = None
+        self._triplets = None
+        self._unit_values = False
 
     def _coo_view(self):
         """The COO view for use inside this class, where nothing is changed through it."""
@@ -112,9 +119,7 @@ class MTX:
     def coo_mtx(self, value):
         self._coo = value
         self._csr = None                               # cached views follow the COO
-        self._csr_source = None
-        self._triplets = None
-        self._unit_values = False
+        self._forget_sources()
         self._identity = object()
 
     # ---- constructors without a file -------------------------------------------------

@@ -122,6 +122,30 @@ def test_changes_of_the_coo_view_reach_the_gpu(monkeypatch, edit):
         np.testing.assert_array_equal(got, ref)
 
 
+@pytest.mark.parametrize("edit", _edits(), ids=["sum_duplicates", "eliminate_zeros", "data"])
+def test_changes_of_the_coo_view_of_csr_arrays_reach_the_gpu(monkeypatch, edit):
+    """The same for a container made from CSR arrays, which go up as they are only while its COO view
+    has not been handed out; the host's CSR view follows the change as well."""
+    indptr, indices = np.array([0, 2, 2, 3], dtype=np.int32), np.array([1, 1, 0], dtype=np.int32)
+    data = np.array([1.0, 2.0, 0.0], dtype=np.float32)
+    g = MTX.from_csr(indptr, indices, (3, 2), data=data)
+    g.adj_tensors("csr")
+    path, sent, _ = _sent_to_the_gpu(monkeypatch, g)
+    assert path == "csr"
+    np.testing.assert_array_equal(sent[2], data)
+    edit(g.coo_mtx)
+    want = sp.csr_matrix((data, indices, indptr), shape=(3, 2)).tocoo()
+    edit(want)
+    path, sent, nnz = _sent_to_the_gpu(monkeypatch, g)
+    assert path == "coo" and nnz == g.num_edges() == want.nnz
+    for got, ref in zip(sent, (want.row, want.col, want.data)):
+        np.testing.assert_array_equal(got, ref)
+    unedited = MTX.from_csr(np.array([0, 1]), indices[:1], (1, 2), data=data[:1])     # (canonical: the CSR view is the source)
+    unedited.adj_tensors("csr")
+    edit(unedited.coo_mtx)
+    np.testing.assert_array_equal(unedited.adj_tensors("csr")[2], unedited.coo_mtx.tocsr().data)
+
+
 def test_a_copy_on_the_gpu_is_kept_until_the_matrix_is_replaced():
     """Looking at the COO view is no new matrix; assigning one is."""
     from liteform_ae_amd import format_algos as fa
