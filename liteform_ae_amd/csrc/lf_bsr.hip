@@ -107,8 +107,15 @@ bsr_spmm_kernel(const int32_t* __restrict__ indptr, const int32_t* __restrict__ 
         const _Float16* blk = data + (size_t)j * BS * BS + li * BS + k0;
 #pragma unroll
         for (int t = 0; t < RT; ++t) st.a[t] = *reinterpret_cast<const uint4*>(blk + 16 * t * BS);
-        // an odd last block of 16 has no partner
-        if (BPS == 2 && second && jb + 2 * s + 1 >= je) st.a[0] = make_uint4(0, 0, 0, 0);
+    };
+    // An odd last block of 16 has no partner: the half of the wavefront that read the block once more adds
+    // nothing.  Both operands are cleared: 0 * Inf is NaN whichever of them is infinite.
+    auto drop_missing = [&](BsrStep<BS>& st) {
+        if (BPS == 2 && kq >= 2 && ((je - jb) & 1)) {
+            st.a[0] = make_uint4(0, 0, 0, 0);
+#pragma unroll
+            for (int r = 0; r < 8; ++r) st.x[r] = make_uint4(0, 0, 0, 0);
+        }
     };
     auto multiply = [&](const BsrStep<BS>& st) {
 #pragma unroll
@@ -144,8 +151,10 @@ bsr_spmm_kernel(const int32_t* __restrict__ indptr, const int32_t* __restrict__ 
         if (s + 1 < n_steps) {
             load(s + 1, odd, s1);
             multiply(s0);
+            drop_missing(s1);
             multiply(s1);
         } else {
+            drop_missing(s0);
             multiply(s0);
         }
     }

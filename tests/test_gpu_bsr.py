@@ -164,3 +164,33 @@ def test_long_block_rows_of_a_large_product(fa, torch, bs, mb, feat):
     for r in range(0, mb, 512):
         ref = torch.matmul(ab[r:r + 512], xb[r:r + 512]).sum(1).view(-1, feat)
         assert (y[r * bs:(r + 512) * bs].float() - ref).abs().max() < 2e-2
+
+
+@pytest.mark.parametrize("bs", [16, 32, 64])
+@pytest.mark.parametrize("feat", [40, 128])
+def test_infinite_rows_of_x(fa, torch, feat, bs):
+    """A row of X of +Inf or -Inf, met by block rows of 1 to 6 blocks as their first, a middle or their
+    last block: Inf where the entries of A it meets are positive or negative, nothing elsewhere."""
+    rng = np.random.default_rng(bs)
+    counts = np.repeat(np.arange(1, 7), 3)
+    mb, nb = len(counts), 8
+    indptr = np.concatenate([[0], np.cumsum(counts)]).astype(np.int32)
+    indices = np.concatenate([np.sort(rng.choice(nb, size=n, replace=False)) for n in counts]).astype(np.int32)
+    data = rng.uniform(0.25, 1, size=(len(indices), bs, bs)).astype(np.float16)
+    data[rng.random(data.shape[0]) < 0.5] *= -1                      # a block is positive or negative as a whole
+    a = sp.bsr_matrix((data.astype(np.float32), indices, indptr), shape=(mb * bs, nb * bs))
+    dense = a.toarray().astype(np.float64)
+    for block in range(nb):
+        for value in (np.inf, -np.inf):
+            x = rng.uniform(-1, 1, size=(nb * bs, feat)).astype(np.float16)
+            k = block * bs + (7 * block + 3) % bs
+            x[k] = value
+            y = fa.spmm_bsr(a, torch.from_numpy(x).cuda(), block_size=bs).cpu().numpy().astype(np.float64)
+            hit = np.sign(dense[:, k])                               # 0: the row has no such block
+            finite = x.astype(np.float64)
+            finite[k] = 0
+            want = dense @ finite
+            want[hit != 0] = hit[hit != 0, None] * value
+            assert not np.isnan(y).any(), (block, value)
+            np.testing.assert_array_equal(y[hit != 0], want[hit != 0])
+            np.testing.assert_allclose(y[hit == 0], want[hit == 0], rtol=2.0 ** -10, atol=1e-5 * 6 * bs)   # (sums of 6 bs products below 1)
