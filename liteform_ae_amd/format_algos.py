@@ -22,6 +22,7 @@ Additions that the reference does not have:
 """
 from __future__ import annotations
 
+import contextlib
 import ctypes as C
 import os
 import threading
@@ -126,9 +127,12 @@ def _upload(array, dtype):
 
 
 class _Downloads:
-    """32-bit device tensors as host tensors of given types, through the staging buffers: as many
-    pieces as there are buffers are under way from the start, and ``get(i)`` converts (on the host's
-    threads) what has arrived until tensor i is complete.  To be used as a context, tensors in order."""
+    """32-bit tensors of one device as host tensors of given types, through that device's staging
+    buffers and behind the work on its current stream: as many pieces as there are buffers are under
+    way from the start, and ``get(i)`` converts (on the host's threads) what has arrived until tensor
+    i is complete.  To be used as a context, tensors in order.  The tensors' device is the current one
+    in it: a copy runs on a stream of the tensor's device, an event is recorded on one of the current
+    device's."""
 
     def __init__(self, wanted):
         torch = _torch()
@@ -136,17 +140,16 @@ class _Downloads:
         self._wanted = wanted
 
     def __enter__(self):
-        _stage_lock.acquire()
-        try:
-            self._bufs, self._events, self._turn = _staging(max((4 * t.numel() for t, _ in self._wanted), default=0))
+        with contextlib.ExitStack() as held:
+            held.enter_context(_stage_lock)
+            held.enter_context(_torch().cuda.device(self._wanted[0][0].device))
+            self._bufs, self._events, self._turn = _staging(max(4 * t.numel() for t, _ in self._wanted))
             chunk = self._bufs[0].numel() // 4
             self._todo = [(i, off, min(chunk, t.numel() - off)) for i, (t, _) in enumerate(self._wanted)
                           for off in range(0, t.numel(), chunk)][::-1]
             self._ahead = []
             self._request()
-        except BaseException:
-            _stage_lock.release()
-            raise
+            self._held = held.pop_all()
         return self
 
     def _request(self):
@@ -169,7 +172,7 @@ class _Downloads:
         return self._out[i]
 
     def __exit__(self, *exc):
-        _stage_lock.release()
+        self._held.close()
 
 
 def _all_ones(data) -> bool:
