@@ -224,8 +224,13 @@ int lf_hyb_build(const int32_t* d_indptr, const int32_t* d_indices, const float*
  * with shared gathers, and rows of very many chunks, have small launches of their own behind
  * it.  Partitions run in ascending order on the stream, partition 0 stores and later partitions
  * add, the chunks of a long row are added up in a fixed order by whichever comes last: the
- * result does not depend on scheduling.  C needs no clearing.  A plan holds partial rows and their
- * counters: its runs must not overlap.
+ * result does not depend on scheduling.  C needs no clearing.  A plan holds the partial rows of its
+ * long rows and their counters (h_info: heavy rows), which two runs must not use at once: a run on
+ * another stream than the one before waits on the GPU for the run before (if that stream has been
+ * destroyed, or is another thread's hipStreamPerThread, the call waits for the device).  Runs that are
+ * recorded into a HIP graph are ordered by whoever launches the graph: no such launch may overlap
+ * another run of the same plan, nor a run on another stream be made while the last one's is being
+ * recorded.
  *
  * A bucket is described the way the reference passes it to the kernel
  * (format_algos.py:552-578: values float32, rows int32, cols int32 row-major), plus the

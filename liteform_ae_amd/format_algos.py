@@ -511,7 +511,12 @@ class HybSpMM:
 
     ``windows`` > 1 computes the product in that many passes over ``feat_size // windows``
     features each (lf_spmm_set_windows): same result up to the summation order of the
-    cooperatively reduced rows, and faster when B is much larger than the memory-side cache."""
+    cooperatively reduced rows, and faster when B is much larger than the memory-side cache.
+
+    Runs may be made on any stream.  The runs of a plan with long rows (``info["heavy_rows"]``) share
+    scratch memory: one on another stream than the run before waits for it on the GPU.  A run that is
+    recorded into a HIP graph has no such guard: the graph must not be launched while another run of
+    the plan is under way."""
 
     def __init__(self, fmt_or_slabs, feat_size: int, b_dtype: str = "f32", num_rows=None, num_cols=None,
                  bucket_widths=None, windows: int = 1):

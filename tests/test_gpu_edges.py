@@ -133,6 +133,38 @@ def test_graph_replay_matches_eager(fa, torch):
         plan.close()
 
 
+def test_runs_of_one_plan_on_several_streams(fa, torch):
+    """The runs of a plan share its partial rows and counters: on several streams, with operands of
+    their own, each gives what it gives alone - also behind a run that was recorded into a graph."""
+    rng = np.random.default_rng(31)
+    g = skewed_matrix(rng, 3000, 30000, mean_deg=6, heavy_rows=40, heavy_len=9000)
+    plan = fa.HybSpMM(fa.build_hyb_format_device(g, [[1, 4, 16, 64]]), 64)
+    assert plan.info["heavy_rows"] >= 30
+    streams = [torch.cuda.current_stream()] + [torch.cuda.Stream() for _ in range(3)]
+    Bs = [torch.rand((30000, 64), device="cuda") - 0.5 for _ in streams]
+    alone = [plan.run(B).clone() for B in Bs]
+    outs = [[torch.full_like(alone[0], float("nan")) for _ in range(12)] for _ in streams]
+    graph, in_graph = torch.cuda.CUDAGraph(), torch.full_like(alone[0], float("nan"))
+    torch.cuda.synchronize()
+    for i in range(12):
+        for stream, B, out in zip(streams, Bs, outs):
+            with torch.cuda.stream(stream):
+                plan.run(B, out[i])
+        if i == 5:
+            torch.cuda.synchronize()
+            with torch.cuda.graph(graph):
+                plan.run(Bs[1], in_graph)
+    torch.cuda.synchronize()
+    for ref, out in zip(alone, outs):
+        assert all(torch.equal(ref, x) for x in out)
+    for _ in range(3):
+        in_graph.fill_(float("nan"))
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(in_graph, alone[1])
+
+
 def test_matrix_features_on_device(fa, torch):
     """Integer fields exact, float fields to 1e-9 relative against the host routine
     (numpy's two-pass standard deviation against sqrt(E[d^2] - E[d]^2) on exact sums)."""
