@@ -1201,8 +1201,10 @@ struct PlanBucket {
 //     inside B, 1..W valid slots per ELL row, and segments (a head that announces n ELL rows followed
 //     by continuation rows 1..n-1 with the same row id) that are complete and stay inside the
 //     bucket.  flags[0] bad column, [1] bad row, [2] bad meta;
-//   * counts the chunks of rows that take the cooperative path: counters[(4 k + i) * kCounterLine]
-//     of bucket k = chunks, rows with several chunks, their partial rows, ChunkedRow::found of all rows;
+//   * counts what lf_spmm_create sizes its tables by: counters[(kScanCounters k + i) * kCounterLine] of bucket
+//     k = chunks of the rows of more than kCoopSlots slots, rows with several chunks, their partial
+//     rows, rows of 65 .. 128 and of 129 .. kCoopSlots slots (a chunk each if they take the cooperative
+//     path), ChunkedRow::found of all rows;
 //   * marks the rows that partition 0 writes.
 // Bound by the stream of the column slabs.  Workgroup -> bucket by the first workgroups of the
 // buckets, so that all of them share one launch however many there are: three launches per bucket
@@ -1211,11 +1213,12 @@ struct PlanBucket {
 constexpr int kScanSlotsPerBlock = 16384;
 constexpr int kScanMaxBlocks = 1024;       // per bucket: more only queue up at its counters
 constexpr int kScanUnroll = 4;             // 16-byte loads of columns in flight per thread
+constexpr int kScanCounters = 6;
 constexpr int kCounterLine = 32;           // words between the counters of a bucket: each has a 128-byte line of its
                                            // own, as atomics on one line are taken one after the other (17 ns each)
 __global__ void __launch_bounds__(256)
 plan_scan_kernel(const PlanBucket* __restrict__ buckets, const int32_t* __restrict__ first_block, int n_buckets,
-                 long long num_rows, long long num_cols, int coop_slots, int chunk_slots, long long dense_min_slots,
+                 long long num_rows, long long num_cols, int chunk_slots, long long dense_min_slots,
                  int* __restrict__ counters, int* __restrict__ flags, uint8_t* __restrict__ covered) {
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     int k = -1;                                       // last bucket whose first workgroup is not behind this one
@@ -1245,7 +1248,8 @@ plan_scan_kernel(const PlanBucket* __restrict__ buckets, const int32_t* __restri
         for (int u = 0; u < kScanUnroll; ++u)
             bad_col |= (unsigned)c[u].x >= limit || (unsigned)c[u].y >= limit || (unsigned)c[u].z >= limit || (unsigned)c[u].w >= limit;
     }
-    int sum[3] = {0, 0, 0}, found = 0;
+    constexpr int kSums = kScanCounters - 1;
+    int sum[kSums] = {}, found = 0;
     for (long long e = t0; e < n_rows; e += stride) {
         const int row = rows[e];
         const bool row_ok = (unsigned)row < (unsigned long long)num_rows;
@@ -1279,32 +1283,36 @@ plan_scan_kernel(const PlanBucket* __restrict__ buckets, const int32_t* __restri
         } else {
             bad_meta |= want != 0;
         }
-        const ChunkedRow x = chunked_row(meta, e, n_rows, log_w, coop_slots, chunk_slots, dense_min_slots);
+        const ChunkedRow x = chunked_row(meta, e, n_rows, log_w, kCoopSlots, chunk_slots, dense_min_slots);
         found |= x.found;
         sum[0] += x.n_chunks;
         sum[1] += x.n_chunks > 1;
         sum[2] += x.n_chunks > 1 ? x.n_chunks : 0;
+        const long long slots = m >= 0 ? field << log_w : 0;     // of the row that starts here
+        sum[3] += slots > 64 && slots <= 128;
+        sum[4] += slots > 128 && slots <= kCoopSlots;
     }
     if (__ballot(bad_col) != 0 && lane == 0) flags[0] = 1;
     if (__ballot(bad_row) != 0 && lane == 0) flags[1] = 1;
     if (__ballot(bad_meta) != 0 && lane == 0) flags[2] = 1;
     // one atomic per workgroup and counter
-    __shared__ int s_sum[4][4];
+    __shared__ int s_sum[4][kScanCounters];
     for (int d = 32; d > 0; d >>= 1) {
         found |= __shfl_xor(found, d);
-        for (int i = 0; i < 3; ++i) sum[i] += __shfl_xor(sum[i], d);
+        for (int i = 0; i < kSums; ++i) sum[i] += __shfl_xor(sum[i], d);
     }
     if (lane == 0) {
-        for (int i = 0; i < 3; ++i) s_sum[wave][i] = sum[i];
-        s_sum[wave][3] = found;
+        for (int i = 0; i < kSums; ++i) s_sum[wave][i] = sum[i];
+        s_sum[wave][kSums] = found;
     }
     __syncthreads();
-    int* mine = counters + (size_t)(4 * k + (int)(threadIdx.x & 3)) * kCounterLine;
-    if (threadIdx.x < 3) {
-        const int all = s_sum[0][threadIdx.x] + s_sum[1][threadIdx.x] + s_sum[2][threadIdx.x] + s_sum[3][threadIdx.x];
+    const int i = threadIdx.x;
+    int* mine = counters + ((size_t)kScanCounters * k + min(i, kSums)) * kCounterLine;
+    if (i < kSums) {
+        const int all = s_sum[0][i] + s_sum[1][i] + s_sum[2][i] + s_sum[3][i];
         if (all) atomicAdd(mine, all);
-    } else if (threadIdx.x == 3) {
-        const int all = s_sum[0][3] | s_sum[1][3] | s_sum[2][3] | s_sum[3][3];
+    } else if (i == kSums) {
+        const int all = s_sum[0][i] | s_sum[1][i] | s_sum[2][i] | s_sum[3][i];
         // what the shared word holds already need not be added again
         if ((all & ~__hip_atomic_load(mine, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) != 0) atomicOr(mine, all);
     }
@@ -1686,20 +1694,6 @@ int lf_spmm_create(lf_spmm_plan** out_plan, const lf_bucket_desc* h_buckets, int
                          part_bytes <= (num_parts > 1 ? 2 * kL2XcdBytes : bf16 && lpr <= 32 ? kL2XcdBytes : 0) &&
                          (bf16 || total_slots <= 96 * num_rows * num_parts);
     }
-    // A sub-wave sums kUnroll slots of its row per round trip to B, so a row of kCoopSlots is a
-    // chain of 32; where a launch holds few rows of more than 64 slots - a few workgroups per CU - they
-    // set its length, and whole workgroups take them too.  (56K-row power-law graph, bf16, N = 128: 33
-    // -> 21 us; 36K rows, N = 64: 33 -> 16; with some thousand such rows the workgroups' set-up costs more
-    // than the chains: 26K rows of 46 entries, N = 64 34 -> 40.)  In between, for small N with its many
-    // sub-waves to a workgroup, rows of more than 128 (25K rows of 62 entries, N = 32: 26 -> 22 us).
-    long long over64 = 0, over128 = 0;
-    for (int k = 0; k < num_buckets; ++k) {
-        const lf_bucket_desc& b = h_buckets[k];
-        if (b.width > 64 && b.width <= kCoopSlots) over64 += b.num_ell_rows;
-        if (b.width > 128 && b.width <= kCoopSlots) over128 += b.num_ell_rows;
-    }
-    if (over64 <= 4 * plan->num_cus) plan->coop_slots = 64;
-    else if (lpr <= 16 && over128 <= 8 * plan->num_cus) plan->coop_slots = 128;
     const char* env_dense = getenv("LF_DENSE_ROWS");       // "0": dense rows are chunked like the other long rows
     // (where the memory-side cache holds the partition's part of B anyway there is nothing to order)
     const long long cols_p = lf::ceil_div(num_cols, num_parts);
@@ -1711,7 +1705,7 @@ int lf_spmm_create(lf_spmm_plan** out_plan, const lf_bucket_desc* h_buckets, int
     // Scratch: the words that are read back (chunk counters and fill cursors of every bucket, sampling
     // counters, flags), then the coverage bytes - cleared by one launch - then the bucket table.
     const size_t nb_s = (size_t)num_buckets;
-    const size_t o_counters = 0, o_cursors = o_counters + nb_s * 4 * kCounterLine * 4, o_flags = o_cursors + nb_s * 4 * kCounterLine * 4;
+    const size_t o_counters = 0, o_cursors = o_counters + nb_s * kScanCounters * kCounterLine * 4, o_flags = o_cursors + nb_s * 3 * kCounterLine * 4;
     const size_t o_zero = o_flags + 16, o_sample = o_zero + 16, back_bytes = o_sample + nb_s * 24;
     const size_t o_covered = (back_bytes + 255) / 256 * 256;
     const size_t o_table = (o_covered + (size_t)num_rows + 255) / 256 * 256;
@@ -1786,8 +1780,8 @@ int lf_spmm_create(lf_spmm_plan** out_plan, const lf_bucket_desc* h_buckets, int
     }
     if (num_buckets > 0) LF_TRY_HIP(hipMemcpyAsync(d_scratch + o_table, h_table, table_bytes, hipMemcpyHostToDevice, s));
     if (scan_blocks > 0) {
-        plan_scan_kernel<<<scan_blocks, 256, 0, s>>>(d_table, d_first, num_buckets, num_rows, num_cols, plan->coop_slots,
-                                                     chunk_slots, dense_min_slots, d_counters, d_flags, d_cov);
+        plan_scan_kernel<<<scan_blocks, 256, 0, s>>>(d_table, d_first, num_buckets, num_rows, num_cols, chunk_slots,
+                                                     dense_min_slots, d_counters, d_flags, d_cov);
         LF_TRY_HIP(hipGetLastError());
     }
     const int rgrid = (int)std::min<int64_t>((num_rows + 255) / 256, 1024);
@@ -1810,12 +1804,31 @@ int lf_spmm_create(lf_spmm_plan** out_plan, const lf_bucket_desc* h_buckets, int
                                                         "or a segment that is incomplete or leaves the bucket)"));
         if (f[3]) return bail(lf::fail(LF_ERR_UNSUPPORTED, "a row is split over more than %d ELL rows", (1 << (31 - kMetaLenBits)) - 1));
     }
+    // A sub-wave sums kUnroll slots of its row per round trip to B, so a row of kCoopSlots is a
+    // chain of 32; where a product holds few rows of more than 64 slots - a few workgroups per CU - they
+    // set its length, and whole workgroups take them too.  (56K-row power-law graph, bf16, N = 128: 33
+    // -> 21 us; 36K rows, N = 64: 33 -> 16; with some thousand such rows the workgroups' set-up costs more
+    // than the chains: 26K rows of 46 entries, N = 64 34 -> 40.)  In between, for small N with its many
+    // sub-waves to a workgroup, rows of more than 128 (25K rows of 62 entries, N = 32: 26 -> 22 us).
+    // It is rows that count, whatever the bucket: in a folded format they are segments of narrow ELL rows.
+    // (Counted by the widths of the buckets, a folded format had none, and every such row became a chunk:
+    // 2.45M-row graph, widths 1 .. 32, 302K chunks instead of 20K, N = 32 1.86 -> 1.60 ms now, N = 128 7.03 -> 6.84;
+    // 132K rows of 300 entries, widths 1 .. 32 in four partitions, N = 32 0.998 -> 0.450.)
+    auto scanned = [&](int k, int i) { return h_counters[((size_t)kScanCounters * k + i) * kCounterLine]; };
+    long long over64 = 0, over128 = 0;
     for (int k = 0; k < num_buckets; ++k) {
-        const int* c = h_counters + (size_t)4 * k * kCounterLine;
-        counts[k].chunks = c[0];
-        counts[k].heavy = c[kCounterLine];
-        counts[k].partials = c[2 * kCounterLine];
-        const int found = c[3 * kCounterLine];
+        over64 += (long long)scanned(k, 3) + scanned(k, 4);
+        over128 += scanned(k, 4);
+    }
+    if (over64 <= 4 * plan->num_cus) plan->coop_slots = 64;
+    else if (lpr <= 16 && over128 <= 8 * plan->num_cus) plan->coop_slots = 128;
+    // the rows that this adds are one chunk each
+    static_assert(kCoopSlots >= 128 && kCoopSlots <= kChunkSlots / 4 && kCoopSlots <= kDenseChunkSlots && kCoopSlots < kDenseRowMinSlots);
+    for (int k = 0; k < num_buckets; ++k) {
+        counts[k].chunks = scanned(k, 0) + (plan->coop_slots <= 64 ? scanned(k, 3) : 0) + (plan->coop_slots <= 128 ? scanned(k, 4) : 0);
+        counts[k].heavy = scanned(k, 1);
+        counts[k].partials = scanned(k, 2);
+        const int found = scanned(k, 5);
         is_multi[k] = found & 1;
         has_dense[k] = (found >> 1) & 1;
         has_wide[k] = (found >> 2) & 1;
@@ -1849,7 +1862,7 @@ int lf_spmm_create(lf_spmm_plan** out_plan, const lf_bucket_desc* h_buckets, int
         const lf_bucket_desc& b = h_buckets[k];
         d_chunks[k] = d_chunks_all + chunk_base[k];
         const int grid = (int)std::min<long long>((b.num_ell_rows + 255) / 256, kPlanChunksGrid);
-        plan_chunks_kernel<<<grid, 256, 0, s>>>(b.d_rows, meta[k], b.d_cols, b.num_ell_rows, lf::ilog2(b.width), d_cursors + (size_t)4 * k * kCounterLine,
+        plan_chunks_kernel<<<grid, 256, 0, s>>>(b.d_rows, meta[k], b.d_cols, b.num_ell_rows, lf::ilog2(b.width), d_cursors + (size_t)3 * k * kCounterLine,
                                                 d_chunks[k], plan->d_heavy, partial_base[k], heavy_base[k], plan->coop_slots,
                                                 chunk_slots, dense_min_slots);
         LF_TRY_HIP(hipGetLastError());
@@ -2166,7 +2179,7 @@ int lf_spmm_create(lf_spmm_plan** out_plan, const lf_bucket_desc* h_buckets, int
     plan->info[8] = (int64_t)cells.size();
     LF_TRY_HIP(read_back());                 // the tables are complete: the plan may run on any stream
     for (int k = 0; k < num_buckets; ++k) {  // the filling pass must have taken the counted ranges
-        const int* c = back.as<int>(o_cursors) + (size_t)4 * k * kCounterLine;
+        const int* c = back.as<int>(o_cursors) + (size_t)3 * k * kCounterLine;
         if (counts[k].chunks > 0 && (c[0] != counts[k].chunks || c[kCounterLine] != counts[k].heavy || c[2 * kCounterLine] != counts[k].partials))
             return bail(lf::fail(LF_ERR_INVALID, "bucket %d changed while the plan was being built", k));
     }

@@ -271,6 +271,35 @@ def test_rows_around_the_cooperative_length(fa, torch, feat, b_dtype, n_long):
             <= 1e-5 * O.spmm_abs_bound(indptr, indices, data, (len(lens), nc), Bh)).all()
 
 
+@pytest.mark.parametrize("feat,b_dtype,lanes", [(32, "f32", 8), (128, "f32", 32), (512, "f32", 64), (128, "bf16", 16)])
+@pytest.mark.parametrize("n_mid,n_long", [(0, 0), (700, 300), (3000, 0), (3000, 1500), (3000, 2500)])
+def test_cooperative_length_of_a_folded_format(fa, torch, feat, b_dtype, lanes, n_mid, n_long):
+    """Widest bucket of 32: a row of 65 to 256 entries is several narrow ELL rows, and it is the rows that
+    count.  Where a matrix has many of them they are not given a workgroup each."""
+    rng = np.random.default_rng(n_mid + n_long + feat)
+    nc = 900
+    lens = np.concatenate([[1, 2, 3, 31, 32, 33, 63, 64, 65, 96, 97, 128, 129, 255, 256],
+                           rng.integers(65, 129, size=n_mid), rng.integers(129, 257, size=n_long)]).astype(np.int64)
+    row = np.repeat(np.arange(len(lens)), lens)
+    pos = np.arange(len(row)) - np.repeat(np.cumsum(lens) - lens, lens)
+    g = MTX.from_coo(row, (row * 17 + pos * 7) % nc, (len(lens), nc), data=rng.uniform(-1, 1, size=len(row)).astype(np.float32))
+    B = torch.from_numpy(rng.uniform(-1, 1, size=(nc, feat)).astype(np.float32)).cuda().to(torch.bfloat16 if b_dtype == "bf16" else torch.float32)
+    fmt = fa.build_hyb_format_device(g, [[1, 4, 32]])
+    plan = fa.HybSpMM(fmt, feat, b_dtype)
+    got = plan.run(B).cpu().numpy()
+    indptr, indices, data = g.adj_tensors("csr")
+    Bh = B.float().cpu().numpy()
+    assert (np.abs(got - O.spmm_csr_f64(indptr, indices, data, (len(lens), nc), Bh))
+            <= 1e-5 * O.spmm_abs_bound(indptr, indices, data, (len(lens), nc), Bh)).all()
+    slots = -(-lens // 32) * 32
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    over64, over128 = int((slots > 64).sum()), int((slots > 128).sum())
+    length = 64 if over64 <= 4 * cus else 128 if lanes <= 16 and over128 <= 8 * cus else 256
+    chunks = int((slots > length).sum())                    # one each: none is longer than a chunk
+    tiles = int(fmt.ell_rows.sum()) // 16 + 4 * cus + 40    # of ELL rows: 16 or more to a tile, or four tiles per CU
+    assert chunks <= plan.info["tiles"] <= chunks + tiles, (length, chunks, plan.info)
+
+
 @pytest.mark.parametrize("feat,b_dtype", [(32, "f32"), (64, "f32"), (96, "f32"), (288, "f32"), (64, "bf16"), (256, "bf16"), (512, "bf16")])
 @pytest.mark.parametrize("parts,n_rows", [(1, 700), (2, 17), (3, 8192 + 5)])
 def test_parts_of_b_that_the_l2_holds(fa, torch, feat, b_dtype, parts, n_rows):
