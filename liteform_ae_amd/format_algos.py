@@ -22,7 +22,6 @@ Additions that the reference does not have:
 """
 from __future__ import annotations
 
-import contextlib
 import ctypes as C
 import os
 import threading
@@ -140,17 +139,26 @@ class _Downloads:
         self._wanted = wanted
 
     def __enter__(self):
-        with contextlib.ExitStack() as held:
-            held.enter_context(_stage_lock)
-            held.enter_context(_torch().cuda.device(self._wanted[0][0].device))
+        self._outer = _torch().cuda.current_device()
+        self._device = self._wanted[0][0].device.index
+        _stage_lock.acquire()
+        try:
+            self._switch(self._outer, self._device)
             self._bufs, self._events, self._turn = _staging(max(4 * t.numel() for t, _ in self._wanted))
             chunk = self._bufs[0].numel() // 4
             self._todo = [(i, off, min(chunk, t.numel() - off)) for i, (t, _) in enumerate(self._wanted)
                           for off in range(0, t.numel(), chunk)][::-1]
             self._ahead = []
             self._request()
-            self._held = held.pop_all()
+        except BaseException:
+            self.__exit__()
+            raise
         return self
+
+    @staticmethod
+    def _switch(current, wanted):
+        if current != wanted:
+            _torch().cuda.set_device(wanted)
 
     def _request(self):
         while self._todo and len(self._ahead) < len(self._bufs):
@@ -172,7 +180,10 @@ class _Downloads:
         return self._out[i]
 
     def __exit__(self, *exc):
-        self._held.close()
+        try:
+            self._switch(self._device, self._outer)
+        finally:
+            _stage_lock.release()
 
 
 def _all_ones(data) -> bool:

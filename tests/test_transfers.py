@@ -1,6 +1,5 @@
 """Host side of the staged transfers, with stand-ins for the GPU: on which device's streams the
 copies, events and buffers of a read-back lie."""
-import contextlib
 import types
 
 import torch
@@ -29,13 +28,8 @@ class _Cuda:
     def current_device(self):
         return self.current
 
-    @contextlib.contextmanager
-    def device(self, device):
-        before, self.current = self.current, torch.device(device).index
-        try:
-            yield
-        finally:
-            self.current = before
+    def set_device(self, device):
+        self.current = device
 
 
 class _OnDevice1:
