@@ -2312,8 +2312,7 @@ int lf_csr_spmm_trusted(const int32_t* d_indptr, const int32_t* d_indices, const
     a.B = d_B;
     a.C = d_C;
     const int threads = csr_threads(lpr, ch * (b_dtype == LF_DTYPE_BF16 ? 8 : 4));
-    const size_t lds = (size_t)(threads / lpr) * feat_size * 4;           // at most 64 KB
-    if (lds > (32 << 10)) LF_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(ks.csr), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+    const size_t lds = (size_t)(threads / lpr) * feat_size * 4;     // at most 16 KB: csr_threads times values per lane is at most 4096
     // Short runs of rows spread a matrix over the CUs (57K rows, 28 entries each, N = 64: 69 us with 32,
     // 80 with 64, 66 with 16); a workgroup's set-up wants long ones where there are rows enough (1M
     // rows of 5 entries: 227 / 219 / 281) and where a wavefront holds eight rows (N = 32: 53 / 45 / 57).
