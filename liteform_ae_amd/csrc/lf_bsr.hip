@@ -23,10 +23,11 @@
 // taken in pairs - the upper half of the wavefront (kq >= 2) works on the second one -, blocks of 64 in two
 // steps of 32 columns.  The loads of the next step are under way during the products of this one.
 // The kernel before this transposed X through LDS in 2-byte stores, with a barrier and one block's
-// loads in flight per workgroup: 1M x 1M, 8 blocks per block row, N = 128, blocks of 16 / 32 / 64:
-// 0.517 / 0.424 / 0.533 -> 0.369 / 0.394 / 0.493 ms, N = 256, blocks of 32: 0.896 -> 0.728 (all at
-// 7 TB/s of A blocks and rows of X, what a gather that misses the L2s reaches); 40K x 40K, blocks of
-// 16, N = 200: 45 -> 20 us.
+// loads in flight per workgroup.  Both in turn on one GPU: 1M x 1M, 8 blocks per block row, N = 128, blocks
+// of 16 / 32 / 64: 0.514 / 0.397 / 0.519 -> 0.360 / 0.393 / 0.497 ms, N = 256, blocks of 32: 0.842 -> 0.712
+// (all at 7 TB/s of A blocks and rows of X, what a gather that misses the L2s reaches); 40K x 40K, blocks of 16,
+// N = 200: 44 -> 19.5 us, blocks of 32, N = 128: 18.8 -> 14.0.  It loses where block rows are very short:
+// 800K x 800K, 2 blocks of 32 a row, N = 128: 102 -> 106.
 #include <hip/hip_runtime.h>
 #include <hip/hip_fp16.h>
 
@@ -42,10 +43,11 @@ constexpr int kFeatTile = 128;     // features per wavefront
 // spreads them over the CUs (40K x 40K, blocks of 32, N = 128: 15.9 -> 14.5 us, N = 24 10.5 -> 9.5);
 // otherwise four, so that the feature tiles of a block row share its blocks in the L1.  Where a
 // product is bound by memory throughout - large, whole tiles of features, long block rows - eight that
-// start together move 2 to 6 % more (1M x 1M, 8 blocks a row, N = 128, blocks of 32 / 16: 405 / 383 ->
-// 394 / 369 us; 800K x 800K, 7 blocks of 16, N = 384: 720 -> 673); with short block rows the CU waits
-// for the last of eight (800K x 800K, 2 blocks a row, N = 128: 105 -> 110).  Two such workgroups of blocks of
-// 64 would not have the registers.
+// start together move more.  Four against eight in turn on one GPU, 15 shapes of 262K to 1M rows, 6 to 24
+// blocks a row, N = 128 .. 512: 0.9 to 7.4 % faster each (1M x 1M, 8 blocks a row, N = 128, blocks of 32 / 16: 405.8 /
+// 372.5 -> 395.4 / 364.9 us; 800K x 800K, 7 blocks of 16, N = 384: 709.5 -> 660.7); with short block rows
+// the CU waits for the last of eight (800K x 800K, 2 blocks a row, N = 128: 105 -> 110).  Two such workgroups
+// of blocks of 64 would not have the registers.
 constexpr long long kFewUnits = 4096;
 constexpr int kLongBlockRow = 6;       // blocks
 constexpr int most_threads(int block) { return block == 64 ? 256 : 512; }

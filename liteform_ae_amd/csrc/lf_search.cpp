@@ -275,6 +275,13 @@ extern "C" int lf_search_bucket_config(const int64_t* h_stats, const int64_t* h_
 // shapes) the pick is 8 % slower than the fastest measured shape on average, 17 % at worst:
 // the model finds the regime (how many partitions make the slice fit an L2) but not always the
 // best neighbour.  tests/golden/launch_shape_measurements.json holds the three sets.
+//
+// All three were measured before launches whose part of B stays in the L2 had a kernel of their own and
+// before long rows were finished in the same launch.  Today's kernels are faster where the model
+// sees launches and L2 hits: a small product takes 5.4 us where kLaunchMs alone says 29, and many partitions
+// cost less than it thinks (132K rows of 300 entries, N = 128, 8 partitions x 2 windows: 1.43 then, 1.21 ms
+// now; 233K of 490, 16 x 2: 4.49 then, 3.76 now; one partition unchanged).  It errs towards
+// fewer partitions therefore.
 constexpr double kHbmBytesPerPs = 5.528;
 constexpr double kMallShare = 0.5534;
 constexpr double kMallBytes = 256.0 * 1048576.0;

@@ -15,12 +15,13 @@
 //     (whose source rows may span several ELL rows) stream slots through wavefront
 //     shuffles instead;
 //   * a source row split over several ELL rows is summed by one owner; rows longer than
-//     coop_slots (64 to 256) are reduced by a whole workgroup, kChunkSlots at a time: a row that fits one
-//     chunk is written directly, a longer one leaves one partial row per chunk, which the
+//     coop_slots (64, 128 or 256) are reduced by a whole workgroup in chunks of 512 to 8192 slots: a row
+//     that fits one chunk is written directly, a longer one leaves one partial row per chunk, which the
 //     workgroup that comes last adds up (rows of very many chunks: a small second kernel);
 //   * partitions run as consecutive launches: partition 0 stores every output row (rows it
-//     does not touch are cleared by the same launch), later partitions add.  Nothing
-//     depends on scheduling, so results are bit-reproducible, and there are no atomics.
+//     does not touch are cleared by the same launch), later partitions add.  No sum is made with
+//     atomics and the order of every sum is fixed, so results are bit-reproducible; the one atomic of a
+//     product counts the chunks of a long row that have left their partial row.
 //
 // The workgroup -> tile mapping is XCD-aware: workgroup i runs on XCD i % 8, and each
 // group of tiles is cut into 8 contiguous ranges, one per XCD, so that neighbouring ELL
@@ -1664,14 +1665,20 @@ int lf_spmm_create(lf_spmm_plan** out_plan, const lf_bucket_desc* h_buckets, int
     struct ChunkCount { int chunks = 0, heavy = 0, partials = 0; };
     std::vector<ChunkCount> counts((size_t)num_buckets);
     std::vector<int> is_multi((size_t)num_buckets, 0), has_dense((size_t)num_buckets, 0), has_wide((size_t)num_buckets, 0);
-    // Chunk size of the rows that a whole workgroup reduces.  Small matrices want many short
-    // chunks (a 170k-row graph: 0.076 ms with 2048-slot chunks, 0.112 ms with 8192; the smaller the
-    // matrix, the more a chunk's chain of gathers is of the whole: 13K rows, 58K entries, N = 320
-    // bf16, chunks of 2048 / 1024 / 512: 47 / 29 / 19 us, 30K rows, 130K entries, N = 192 41 / 26 / 25,
-    // 149K rows, 640K entries, N = 128 58 / 59 / 60), large ones
-    // fewer partial rows and a shorter second kernel (500k x 2M with 50 rows of 100k entries:
-    // 1.56 -> 1.51 ms with 8192); the chunk tiles lead the launch, so their length hides behind
-    // the rest of the work.
+    // Chunk size of the rows that a whole workgroup reduces.  The smaller the matrix, the more a chunk's
+    // chain of gathers is of the whole: short chunks; where there is work enough to hide it, longer ones
+    // leave fewer partial rows.  By total slots because nothing else is known before the scan; the
+    // steps lie where the sizes crossed on the first matrices measured (13K rows, 58K entries, N = 320 bf16,
+    // chunks of 2048 / 1024 / 512: 47 / 29 / 19 us, 30K rows, 130K entries, N = 192 41 / 26 / 25, 149K
+    // rows, 640K entries, N = 128 58 / 59 / 60) and are not all at the best place.  Power-law graphs of
+    // 8K to 1.5M rows, rows cut at 13,000 or 1500, N = 64, 128 and bf16 320, every size tried:
+    //   below 128K slots    512: the fastest, 2048 takes up to 2.6 times as long
+    //   128K - 192K        1024: loses 24 - 32 % to 512 at 135K slots
+    //   192K - 512K        1536: loses 22 - 51 % to 512 at 205K, 4 - 8 % to 1024 at 366K - 435K
+    //   512K - 4M          2048: within 4 % of the fastest (9 % at 670K), 8192 takes up to 2.5 times as long
+    //   from 4M on         8192: within 5 %; where long rows hold most entries it loses more (1M rows, 400
+    //                            of 20,000 entries, N = 128: 1.18 ms, 1024 1.04; 500k x 2M, 150 of 30,000, N =
+    //                            64: 0.311, 4096 0.286) or gains a little (the same, bf16 N = 256: 666 against 699)
     long long total_slots = 0;
     for (int k = 0; k < num_buckets; ++k) total_slots += h_buckets[k].num_ell_rows * h_buckets[k].width;
     const int chunk_slots = total_slots >= kLargeMatrixSlots ? kChunkSlotsLarge
@@ -1684,9 +1691,11 @@ int lf_spmm_create(lf_spmm_plan** out_plan, const lf_bucket_desc* h_buckets, int
     // (170k-row graph, 6 MB of slabs: 0.073 ms cached, 0.076 ms streamed).
     plan->stream_slabs = total_slots >= kLargeMatrixSlots;
     // Parts of B that an L2 (4 MB) about holds, and for float products rows that are mostly staged (those of
-    // hundreds of slots per partition stream them by shuffle, which gains nothing: 5774 rows of 368 in two
-    // partitions, N = 288 162 -> 173 us).  A single float partition is not latency-bound enough (10K rows of 182, N =
-    // 64: 36 -> 38); a bf16 one is up to 32 lanes per row (5805 rows of 364, N = 128 46 -> 39).
+    // hundreds of slots per partition stream them by shuffle: 5774 rows of 368 in two partitions, N = 288
+    // 145 -> 149 us).  A single float partition is not latency-bound enough (10K and 20K rows, 2.4 to 22 MB: -2 to
+    // + 4 %); a bf16 one is up to 32 lanes per row (10K rows of 182, N = 128: 38.4 -> 36.5 us).  Where the line
+    // loses: the same 5774 rows at N = 64 .. 128 would gain 18 - 23 % (53.6 -> 43.6 us), a bf16 B of 4.9 MB in
+    // one partition 3 %; two partitions of 12K rows of 60 entries lose 1 - 7 % with it (N = 192: 42.7 -> 45.8).
     {
         const bool bf16 = b_dtype == LF_DTYPE_BF16;
         const long long part_bytes = lf::ceil_div(num_cols, (int64_t)num_parts) * feat_size * (bf16 ? 2 : 4);
@@ -1805,11 +1814,16 @@ int lf_spmm_create(lf_spmm_plan** out_plan, const lf_bucket_desc* h_buckets, int
         if (f[3]) return bail(lf::fail(LF_ERR_UNSUPPORTED, "a row is split over more than %d ELL rows", (1 << (31 - kMetaLenBits)) - 1));
     }
     // A sub-wave sums kUnroll slots of its row per round trip to B, so a row of kCoopSlots is a
-    // chain of 32; where a product holds few rows of more than 64 slots - a few workgroups per CU - they
-    // set its length, and whole workgroups take them too.  (56K-row power-law graph, bf16, N = 128: 33
-    // -> 21 us; 36K rows, N = 64: 33 -> 16; with some thousand such rows the workgroups' set-up costs more
-    // than the chains: 26K rows of 46 entries, N = 64 34 -> 40.)  In between, for small N with its many
-    // sub-waves to a workgroup, rows of more than 128 (25K rows of 62 entries, N = 32: 26 -> 22 us).
+    // chain of 32; where a product (all partitions together) holds few rows of more than 64 slots - a few
+    // workgroups per CU - they set its length, and whole workgroups take them too: 56K-row power-law graph, bf16,
+    // N = 128 33 -> 21 us with 64 instead of 256; 4K rows of 40 entries, N = 32 16 -> 6.5.  With some thousand
+    // such rows the workgroups' set-up costs more than the chains (60K rows of 40, N = 64: 64 us with 256, 71
+    // with 64).  In between, for small N with its many sub-waves to a workgroup, rows of more than 128 (30K
+    // rows of 40, N = 32: 17 us, 64 20, 256 24).  Graphs of 4K to 500K rows, N = 32 .. 256, folded and not: the
+    // length taken is within 6 % of the best, but where the first limit has just been passed (8K rows of 40,
+    // 1255 of them above 64 slots: 4 - 48 %, 64 would be best up to N = 64, 128 above), up to 25 % for 15K
+    // rows and N >= 128, which have no middle step, 11 % for such rows folded, and one folded 170K-row
+    // power-law graph at N = 256 (64 taken: 174 us, 256 142).
     // It is rows that count, whatever the bucket: in a folded format they are segments of narrow ELL rows.
     // (Counted by the widths of the buckets, a folded format had none, and every such row became a chunk:
     // 2.45M-row graph, widths 1 .. 32, 302K chunks instead of 20K, N = 32 1.86 -> 1.60 ms now, N = 128 7.03 -> 6.84;

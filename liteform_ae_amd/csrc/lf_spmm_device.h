@@ -36,7 +36,8 @@ constexpr int kTileRows = 512;      // ELL rows per tile at most (<= tile_slots)
 #define LF_CHUNK_SLOTS 2048
 #endif
 constexpr int kCoopSlots = LF_COOP_SLOTS;    // a source row with more slab slots is reduced by a whole workgroup
-constexpr int kChunkSlots = LF_CHUNK_SLOTS;  // ... in chunks of this many slots (a whole number of ELL rows)
+constexpr int kChunkSlots = LF_CHUNK_SLOTS;  // ... in chunks of this many slots, or of a quarter to three quarters of it in
+                                             // small matrices (lf_spmm_create); a chunk may end inside an ELL row
 constexpr int kChunkSlotsLarge = 8192;       // ... or this many, in a matrix of at least kLargeMatrixSlots slots
 constexpr long long kLargeMatrixSlots = 4ll << 20;
 // Dense rows: a row holding at least 1/kDenseRowShare of its partition's columns.  Several of
