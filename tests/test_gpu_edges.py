@@ -202,7 +202,7 @@ def test_staged_transfers_round_trip(fa, n):
 @pytest.mark.parametrize("nr,feat,b_dtype", [
     *((nr, feat, b) for nr in (1, 31, 33, 65) for feat, b in ((32, "f32"), (64, "f32"), (96, "f32"), (128, "f32"), (256, "f32"),
                                                               (512, "f32"), (1024, "f32"), (64, "bf16"), (320, "bf16"), (1024, "bf16"))),
-    (524_288, 64, "f32"), (524_289, 64, "f32"),          # the most rows in groups of 32, the fewest in groups of 64
+    (524_288, 64, "f32"), (524_289, 64, "f32"),          # many groups
 ])
 def test_csr_product_at_group_edges(fa, torch, nr, feat, b_dtype):
     """Rows that end a group of 32 or 64, empty rows at both ends and in a row, rows at and past the
@@ -223,6 +223,42 @@ def test_csr_product_at_group_edges(fa, torch, nr, feat, b_dtype):
     got = fa.spmm_csr(MTX.from_csr(indptr, (key % nc).astype(np.int32), (nr, nc), data=vals), B, b_dtype).cpu().numpy()
     Bh = B.float().cpu().numpy().astype(np.float64)
     assert (np.abs(got - A @ Bh) <= 1e-5 * (abs(A) @ np.abs(Bh)) + 1e-30).all()
+
+
+@pytest.mark.parametrize("nr,feat,b_dtype,usual,longest", [
+    *((nr, feat, b, *rows) for nr in (3, 4, 5, 9, 16, 17, 32, 63)
+      for feat, b in ((32, "f32"), (64, "f32"), (224, "f32"), (448, "f32"), (1024, "f32"), (128, "bf16"), (512, "bf16"), (1024, "bf16"))
+      for rows in ((0, 128), (0, 129), (80, 270), (80, 299))),
+    *((nr, feat, "f32", 0, longest) for longest in (32, 33, 128, 129) for nr, feat in (
+        (4096, 224), (4097, 224),                            # the most rows in groups of 16, the fewest in groups of 32
+        (1 << 20, 32), ((1 << 20) + 1, 32))),                # ... in groups of as many as sub-waves, in groups of 64
+])
+def test_csr_product_of_short_rows(fa, torch, nr, feat, b_dtype, usual, longest):
+    """Groups whose longest row has 128 entries (32 where a sub-wave has two rows) or three average rows,
+    summed a row to a sub-wave, and groups with more than that, cut into runs; rows of every remainder of a
+    batch of eight gathers; infinite rows of B give Inf, not NaN."""
+    import scipy.sparse as sp
+    rng = np.random.default_rng(nr + feat)
+    nc = 300
+    deg = usual + np.arange(nr) * 5 % 34
+    deg[nr // 2] = longest
+    indptr = np.concatenate([[0], np.cumsum(deg)]).astype(np.int32)
+    row = np.repeat(np.arange(nr), deg)
+    key = np.sort(row * nc + (row * 13 + 31 * (np.arange(len(row)) - indptr[row])) % nc)      # 31 and 300 share no factor
+    vals = rng.uniform(0.25, 1, size=len(key)).astype(np.float32)
+    A = sp.csr_matrix((vals.astype(np.float64), key % nc, indptr), shape=(nr, nc))
+    B = torch.from_numpy(rng.uniform(-1, 1, size=(nc, feat)).astype(np.float32)).cuda().to(torch.bfloat16 if b_dtype == "bf16" else torch.float32)
+    g = MTX.from_csr(indptr, (key % nc).astype(np.int32), (nr, nc), data=vals)
+    finite = B.float().cpu().numpy().astype(np.float64)
+    want, bound = A @ finite, 1e-5 * (abs(A) @ np.abs(finite)) + 1e-30
+    assert (np.abs(fa.spmm_csr(g, B, b_dtype).cpu().numpy() - want) <= bound).all()
+    for col in (0, 31, 93):
+        Binf = B.clone()
+        Binf[col] = float("inf")
+        got = fa.spmm_csr(g, Binf, b_dtype).cpu().numpy()
+        hit = np.diff(A[:, [col]].indptr) > 0
+        assert np.isposinf(got[hit]).all()
+        assert (np.abs(got[~hit] - want[~hit]) <= bound[~hit]).all()
 
 
 @pytest.mark.parametrize("feat,b_dtype", [(32, "f32"), (128, "f32"), (320, "f32"), (1024, "f32"), (64, "bf16"), (512, "bf16")])
