@@ -279,7 +279,7 @@ int lf_spmm_destroy(lf_spmm_plan* plan);
  * the same bits).  Narrow
  * windows pay off when B is much larger than the memory-side cache: the part of B that one
  * pass touches is a fraction of the whole, and C is still written once (cfg3, 2.45M rows,
- * N = 128: 6.27 ms in two windows of 64 against 6.94 ms in one pass).  Applies to lf_spmm_run and lf_spmm_time_ms; the default is one window.  No
+ * N = 128: 6.04 ms in two windows of 64 against 6.76 ms in one pass).  Applies to lf_spmm_run and lf_spmm_time_ms; the default is one window.  No
  * counterpart in the reference (its feature tiling lives inside one launch,
  * format_algos.py:491-520). */
 int lf_spmm_set_windows(lf_spmm_plan* plan, int32_t n_windows);
