@@ -21,7 +21,8 @@
  *     (documented per function).
  *   - Index arrays are int32, row-major; values are float32.  A matrix must have
  *     fewer than 2^31 stored entries.
- *   - Handles and workspaces must not be used from two threads at once.
+ *   - Handles and workspaces must not be used from two threads at once, but for lf_spmm_run on
+ *     one plan.
  */
 #ifndef LITEFORM_HIP_H
 #define LITEFORM_HIP_H

@@ -31,6 +31,7 @@
 #include <algorithm>
 #include <cstdlib>
 #include <cstring>
+#include <mutex>
 #include <thread>
 #include <vector>
 
@@ -1582,6 +1583,7 @@ struct lf_spmm_plan {
     hipStream_t last_stream = nullptr;
     std::thread::id last_thread;
     bool has_run = false;
+    std::mutex order_mutex;              // from the wait for the run before to this run's last launch
     int64_t info[LF_SPMM_INFO_FIELDS] = {0};
 };
 
@@ -2304,6 +2306,8 @@ int lf_spmm_info(const lf_spmm_plan* plan, int64_t* h_info) {
 // nothing to runs on one stream.  Where the runtime refuses the stream of the run before (it has been
 // destroyed), or that was another thread's hipStreamPerThread, the device is waited for.  While either
 // stream is being recorded into a graph no event may cross over: those runs are ordered by the caller.
+// To be called with order_mutex held: a run that another thread has ordered but not launched yet is not
+// behind the event.
 static int order_behind_last_run(lf_spmm_plan* plan, hipStream_t s) {
     if (!plan->d_heavy) return LF_OK;
     const bool same = plan->has_run && plan->last_stream == s;
@@ -2342,6 +2346,8 @@ int lf_spmm_run(lf_spmm_plan* plan, const void* d_B, float* d_C, lf_stream_t str
     LF_REQUIRE((uintptr_t)d_B % 16 == 0 && (uintptr_t)d_C % 16 == 0, LF_ERR_INVALID, "B and C must be 16-byte aligned");
     KernelSet ks;
     if (int rc = select_kernels(plan->lpr, plan->ch, plan->b_dtype, &ks)) return rc;
+    std::unique_lock<std::mutex> order(plan->order_mutex, std::defer_lock);
+    if (plan->d_heavy) order.lock();
     if (int rc = order_behind_last_run(plan, s)) return rc;
     // One pass per feature window (all partitions inside), each on its own columns of B and C.
     const size_t b_elem = plan->b_dtype == LF_DTYPE_BF16 ? 2 : 4;

@@ -524,7 +524,7 @@ class HybSpMM:
     features each (lf_spmm_set_windows): same result up to the summation order of the
     cooperatively reduced rows, and faster when B is much larger than the memory-side cache.
 
-    Runs may be made on any stream.  The runs of a plan with long rows (``info["heavy_rows"]``) share
+    Runs may be made on any stream and thread.  The runs of a plan with long rows (``info["heavy_rows"]``) share
     scratch memory: one on another stream than the run before waits for it on the GPU.  A run that is
     recorded into a HIP graph has no such guard: the graph must not be launched while another run of
     the plan is under way."""

@@ -1,5 +1,7 @@
 """Edge cases through the reference-shaped API on the GPU: empty and degenerate shapes,
 many partitions, HIP-graph replay of the fused kernel."""
+from concurrent.futures import ThreadPoolExecutor
+
 import numpy as np
 import pytest
 
@@ -163,6 +165,30 @@ def test_runs_of_one_plan_on_several_streams(fa, torch):
         graph.replay()
         torch.cuda.synchronize()
         assert torch.equal(in_graph, alone[1])
+
+
+def test_runs_of_one_plan_from_several_threads(fa, torch):
+    """The same with a thread to each stream: what a run waits for has been launched, not just begun."""
+    rng = np.random.default_rng(32)
+    g = skewed_matrix(rng, 3000, 30000, mean_deg=6, heavy_rows=40, heavy_len=9000)
+    plan = fa.HybSpMM(fa.build_hyb_format_device(g, [[1, 4, 16, 64]]), 64)
+    assert plan.info["heavy_rows"] >= 30
+    streams = [torch.cuda.Stream() for _ in range(4)]
+    Bs = [torch.rand((30000, 64), device="cuda") - 0.5 for _ in streams]
+    alone = [plan.run(B).clone() for B in Bs]
+    outs = [[torch.full_like(alone[0], float("nan")) for _ in range(12)] for _ in streams]
+    torch.cuda.synchronize()
+
+    def runs(stream, B, out):
+        with torch.cuda.stream(stream):
+            for C in out:
+                plan.run(B, C)
+
+    with ThreadPoolExecutor(len(streams)) as pool:
+        list(pool.map(runs, streams, Bs, outs))
+    torch.cuda.synchronize()
+    for ref, out in zip(alone, outs):
+        assert all(torch.equal(ref, x) for x in out)
 
 
 def test_matrix_features_on_device(fa, torch):
