@@ -326,13 +326,18 @@ int lf_csr_check(const int32_t* d_indptr, const int32_t* d_indices, const float*
  * lf_csr_spmm runs lf_csr_check on the arrays first (d_scratch: its 16 bytes; the stream is
  * synchronised for the verdict) and returns LF_ERR_INVALID without launching the product when
  * they fail.  lf_csr_spmm_trusted is the same product without the check, for arrays that
- * lf_csr_check has accepted or that lf_coo_to_csr produced: it only enqueues the kernel. */
+ * lf_csr_check has accepted or that lf_coo_to_csr produced: it only enqueues the kernel.
+ * lf_csr_spmm_trusted_nnz is told the number of entries, which helps it choose how the features
+ * are split over the XCDs (0: unknown). */
 int lf_csr_spmm(const int32_t* d_indptr, const int32_t* d_indices, const float* d_values,
                 int64_t num_rows, int64_t num_cols, int64_t nnz, int32_t feat_size, int32_t b_dtype,
                 const void* d_B, float* d_C, void* d_scratch, lf_stream_t stream);
 int lf_csr_spmm_trusted(const int32_t* d_indptr, const int32_t* d_indices, const float* d_values,
                         int64_t num_rows, int64_t num_cols, int32_t feat_size, int32_t b_dtype,
                         const void* d_B, float* d_C, lf_stream_t stream);
+int lf_csr_spmm_trusted_nnz(const int32_t* d_indptr, const int32_t* d_indices, const float* d_values,
+                            int64_t num_rows, int64_t num_cols, int64_t nnz, int32_t feat_size,
+                            int32_t b_dtype, const void* d_B, float* d_C, lf_stream_t stream);
 
 /* COO -> canonical CSR on the GPU: entries sorted by (row, column), duplicates added up,
  * row pointer built - what the reference's container does with scipy's coo.tocsr() on every

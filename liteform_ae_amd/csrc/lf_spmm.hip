@@ -902,247 +902,6 @@ spmm_rowgroup_kernel(const MergedBucket* __restrict__ buckets, int n_buckets, La
 }
 
 // ------------------------------------------------------------------------------------
-// CSR product without a plan.  A workgroup of SW sub-waves takes SW (or 32, or 64) consecutive rows, whose
-// entries are contiguous.  Where none of them is longer than kCsrLongRow or three average rows (kCsrLongRow / 4
-// where a sub-wave has several), a sub-wave sums a row at a time.  Otherwise the rows are cut into SW runs of
-// whole rows with about equal cost; a sub-wave streams its run as one sequence of entries - kUnroll gathers in
-// flight whatever the row lengths, the next entries requested ahead - and stores a row whenever its last entry
-// has been added.  A row that would be longer than the average run (and kCsrLongRow) is left out and then summed
-// by all sub-waves together, their sums combined in sub-wave order.
-// One sub-wave per row for every row, the first form, waited for the longest row of every wavefront and of the
-// matrix: N = 64, 170K-row power-law graph (rows up to 13,000) 911 us, with runs 97.  Runs for every row, of 32
-// rows and more to a workgroup, the second form, left small matrices to a few workgroups with a check for a
-// row's end behind every gather.  Log-normal rows, us by form (first / second / this):
-//   rows x      N = 32                 N = 64                 N = 256                bf16 N = 128
-//   2000 x 5    4.1 / 7.9 / 4.8        4.1 / 7.1 / 4.9        3.9 / 6.8 / 4.7        5.9 / 8.6 / 6.3
-//   7162 x 42   22.3 / 29.5 / 22.7     24.1 / 24.7 / 18.1     39.0 / 35.9 / 36.4     38.5 / 32.0 / 23.0
-//   7162 x 200  96.6 / 124 / 79.3      106 / 98.3 / 59.8      166 / 115 / 116        185 / 131 / 79.9
-//   12000 x 40  20.2 / 32.8 / 24.3     23.7 / 26.5 / 20.0     62.3 / 64.9 / 65.1     36.4 / 33.1 / 25.9
-//   57000 x 28  37.3 / 42.4 / 41.3     59.0 / 63.3 / 59.9     227 / 222 / 221        68.2 / 70.3 / 65.9
-//   120000 x 10 30.1 / 34.5 / 30.0     53.0 / 52.3 / 48.8     182 / 185 / 180        63.5 / 59.1 / 55.0
-//   600000 x 12 152 / 160 / 153        268 / 295 / 268        1058 / 1075 / 1072     295 / 317 / 290
-// Rows of more even length still suit the first form at N = 32 (sigma 0.47, 12000 x 40: 10.7 / 25.0 / 18.6).  A
-// limit of 192 for the longest row helps some (2000 x 40, N = 64: 15.1 -> 11.4) and costs where one such row comes
-// last in the grid (120000 x 10, N = 64: 48.8 -> 54.9); four average rows cost 11 % at sigma 1 (12000 x 90).
-constexpr int kCsrRows = 64;               // at most: one wavefront scans their costs
-constexpr int kCsrLongRow = 128;
-constexpr long long kCsrManyRows = 1ll << 20;
-constexpr int kCsrStoreCost = 4;           // a row's store against one of its entries
-// 16 sub-waves where the gathers in flight (kUnroll * values per lane registers) leave the room
-constexpr int csr_threads(int lpr, int per_lane) {
-    const int most = per_lane <= 4 ? 1024 : per_lane <= 8 ? 512 : 256;
-    return lpr <= 16 ? 256 : 16 * lpr < most ? 16 * lpr : most;
-}
-
-// Sum of `len` entries from `lo` on.  Gathers past the end fetch the first column's row again and are cleared
-// before they are added (with a value of 0 alone an infinite element would make NaN), by selects: under a branch
-// each the compiler moves the load there as well, and the gathers go out one after the other (2K rows of 40
-// entries, N = 64: 31 us, 18 so).
-template <int LPR, int CH, typename BT>
-__device__ __forceinline__ void csr_sum(const int32_t* __restrict__ indices, const float* __restrict__ values, int lo, int len,
-                                        const Lane<LPR, CH, Dense<BT>::kVec>& ln, const void* B,
-                                        Acc<CH, Dense<BT>::kVec>& acc) {
-    constexpr int U = kUnroll < LPR ? kUnroll : LPR;
-    if (len <= 0) return;
-    const int c_first = indices[lo];
-    int next_c = ln.sl < len ? indices[lo + ln.sl] : c_first;
-    float next_v = ln.sl < len ? (values ? values[lo + ln.sl] : 1.f) : 0.f;
-    for (int base = 0; base < len; base += LPR) {
-        const int my_c = next_c;
-        const float my_v = next_v;
-        const int idx = base + LPR + ln.sl;
-        next_c = idx < len ? indices[lo + idx] : c_first;
-        next_v = idx < len ? (values ? values[lo + idx] : 1.f) : 0.f;
-        const int cnt = min(LPR, len - base);
-        for (int j = 0; j < cnt; j += U) {
-            float v[U];
-            typename Dense<BT>::Raw x[U][CH];
-#pragma unroll
-            for (int u = 0; u < U; ++u) {
-                const int c = __shfl(my_c, j + u, LPR);
-                v[u] = __shfl(my_v, j + u, LPR);
-#pragma unroll
-                for (int cc = 0; cc < CH; ++cc) x[u][cc] = load_dense<BT>(B, ln, cc, c);
-            }
-            if (j + U <= cnt) {
-#pragma unroll
-                for (int u = 0; u < U; ++u)
-#pragma unroll
-                    for (int cc = 0; cc < CH; ++cc) fma_dense<BT>(v[u], x[u][cc], acc.v[cc]);
-                continue;
-            }
-#pragma unroll
-            for (int u = 0; u < U; ++u) {
-                const bool in = j + u < cnt;
-#pragma unroll
-                for (int cc = 0; cc < CH; ++cc) {
-                    auto y = x[u][cc];
-                    y.x = in ? y.x : 0;
-                    y.y = in ? y.y : 0;
-                    y.z = in ? y.z : 0;
-                    y.w = in ? y.w : 0;
-                    fma_dense<BT>(v[u], y, acc.v[cc]);
-                }
-            }
-        }
-    }
-}
-
-// Entries [at, end) of the arrays: rows r .. of the workgroup until their entries are used up; every
-// row that ends at or before `end` is stored, empty ones with zeros.
-template <int LPR, int CH, typename BT>
-__device__ __forceinline__ void csr_stream_rows(const int32_t* __restrict__ indices, const float* __restrict__ values,
-                                                const int* s_ptr, int r, int r_end, long long first_row,
-                                                const Lane<LPR, CH, Dense<BT>::kVec>& ln, const LaunchArgs& a) {
-    constexpr int VEC = Dense<BT>::kVec;
-    constexpr int U = kUnroll < LPR ? kUnroll : LPR;
-    const int at = s_ptr[r], end = s_ptr[r_end];
-    Acc<CH, VEC> acc;
-    acc.clear();
-    int row_end = s_ptr[r + 1];
-    while (r < r_end && row_end == at) {                     // leading empty rows
-        store_row<LPR, CH, VEC>(a.C, (int)(first_row + r), ln, acc, kStreamC);
-        ++r;
-        if (r < r_end) row_end = s_ptr[r + 1];
-    }
-    if (r >= r_end) return;
-    const int c_first = indices[at];
-    int next_c = at + ln.sl < end ? indices[at + ln.sl] : c_first;
-    float next_v = at + ln.sl < end ? (values ? values[at + ln.sl] : 1.f) : 0.f;
-    for (int base = at; base < end; base += LPR) {
-        const int my_c = next_c;
-        const float my_v = next_v;
-        const int idx = base + LPR + ln.sl;
-        next_c = idx < end ? indices[idx] : c_first;
-        next_v = idx < end ? (values ? values[idx] : 1.f) : 0.f;
-        const int cnt = min(LPR, end - base);
-        for (int j = 0; j < cnt; j += U) {
-            float v[U];
-            typename Dense<BT>::Raw x[U][CH];
-#pragma unroll
-            for (int u = 0; u < U; ++u) {
-                const int c = __shfl(my_c, j + u, LPR);      // past the end: the first column again, value 0
-                v[u] = __shfl(my_v, j + u, LPR);
-#pragma unroll
-                for (int cc = 0; cc < CH; ++cc) x[u][cc] = load_dense<BT>(a.B, ln, cc, c);
-            }
-#pragma unroll
-            for (int u = 0; u < U; ++u) {
-#pragma unroll
-                for (int cc = 0; cc < CH; ++cc) fma_dense<BT>(v[u], x[u][cc], acc.v[cc]);
-                if (base + j + u + 1 == row_end) {           // the row's last entry
-                    store_row<LPR, CH, VEC>(a.C, (int)(first_row + r), ln, acc, kStreamC);
-                    acc.clear();
-                    row_end = 0;
-                    while (++r < r_end) {
-                        row_end = s_ptr[r + 1];
-                        if (row_end > base + j + u + 1) break;
-                        store_row<LPR, CH, VEC>(a.C, (int)(first_row + r), ln, acc, kStreamC);      // an empty row
-                    }
-                }
-            }
-        }
-    }
-}
-
-template <int LPR, int CH, typename BT>
-__global__ void __launch_bounds__(csr_threads(LPR, CH * Dense<BT>::kVec))
-csr_spmm_kernel(const int32_t* __restrict__ indptr, const int32_t* __restrict__ indices,
-                const float* __restrict__ values, long long n_rows, int rows_per_group, LaunchArgs a) {
-    constexpr int VEC = Dense<BT>::kVec;
-    constexpr int kThreads = csr_threads(LPR, CH * VEC);
-    constexpr int SW = kThreads / LPR;
-    __shared__ int s_ptr[kCsrRows + 1];
-    __shared__ int s_cost[kCsrRows + 1];       // exclusive prefix of the rows' costs (a long row's is 0)
-    __shared__ unsigned long long s_long;
-    extern __shared__ __align__(16) float s_red[];         // [SW][feat]: sums of a long row's parts
-    const int tid = threadIdx.x, sw = tid / LPR, sl = tid % LPR;
-    const Lane<LPR, CH, VEC> ln(sl, a.feat, a.ldb, a.ldc);
-    const long long first_row = (long long)blockIdx.x * rows_per_group;
-    const int n = (int)min((long long)rows_per_group, n_rows - first_row);
-    const int lane = tid & 63;
-    const int start = indptr[first_row + min(lane, n)], end = indptr[first_row + min(lane + 1, n)];
-    const int average = (__builtin_amdgcn_readlane(end, 63) - __builtin_amdgcn_readfirstlane(start)) / SW;
-    const int limit = rows_per_group > SW ? kCsrLongRow / 4 : max(kCsrLongRow, 3 * average);
-    if (rows_per_group < kCsrRows && __ballot(end - start > limit) == 0) {       // the same in every wavefront
-        for (int r0 = 0; r0 < n; r0 += SW) {
-            const int r = r0 + sw, from = min(r, n - 1);
-            const int lo = __shfl(start, from), len = __shfl(end, from) - lo;
-            if (r < n) {
-                Acc<CH, VEC> acc;
-                acc.clear();
-                csr_sum<LPR, CH, BT>(indices, values, lo, len, ln, a.B, acc);
-                store_row<LPR, CH, VEC>(a.C, (int)(first_row + r), ln, acc, kStreamC);
-            }
-        }
-        return;
-    }
-    if (tid < 64) {
-        const int total = __shfl(end, 63) - __shfl(start, 0);
-        const bool is_long = end - start > max(kCsrLongRow, total / SW);
-        const unsigned long long longs = __ballot(is_long);
-        int incl = tid < n && !is_long ? end - start + kCsrStoreCost : 0;
-        for (int d = 1; d < 64; d <<= 1) {
-            const int y = __shfl_up(incl, d);
-            if (tid >= d) incl += y;
-        }
-        s_ptr[tid] = start;
-        s_cost[tid + 1] = incl;
-        if (tid == 63) s_ptr[kCsrRows] = end;
-        if (tid == 0) { s_cost[0] = 0; s_long = longs; }
-    }
-    __syncthreads();
-    const unsigned long long longs = s_long;
-    {
-        // the rows whose cost prefix falls into this sub-wave's share
-        const long long all = s_cost[kCsrRows];
-        auto first_at = [&](long long want) {                // first row whose prefix is >= want
-            int lo = 0, hi = n;
-            while (lo < hi) {
-                const int mid = (lo + hi) >> 1;
-                if ((long long)s_cost[mid] < want) lo = mid + 1; else hi = mid;
-            }
-            return lo;
-        };
-        int r = sw == 0 ? 0 : first_at((all * sw + SW - 1) / SW);
-        const int r_end = sw == SW - 1 ? n : first_at((all * (sw + 1) + SW - 1) / SW);
-        while (r < r_end) {                                  // runs between long rows
-            if ((longs >> r) & 1ull) { ++r; continue; }
-            const unsigned long long ahead = longs >> r;
-            const int stop = min(r_end, ahead ? r + __ffsll((long long)ahead) - 1 : r_end);
-            csr_stream_rows<LPR, CH, BT>(indices, values, s_ptr, r, stop, first_row, ln, a);
-            r = stop;
-        }
-    }
-    unsigned long long todo = longs;
-    while (todo) {                                           // uniform
-        const int r = __ffsll((long long)todo) - 1;
-        todo &= todo - 1;
-        const int lo = s_ptr[r], len = s_ptr[r + 1] - lo;
-        const int per = ((len + SW - 1) / SW + LPR - 1) / LPR * LPR;
-        const int from = min(sw * per, len), to = min(from + per, len);
-        Acc<CH, VEC> acc;
-        acc.clear();
-        const int whole = (to - from) / kUnroll * kUnroll;   // (stream_slots adds its padding)
-        stream_slots<LPR, CH, BT>(indices, values, (long long)lo + from, whole, a.B, ln, acc);
-        csr_sum<LPR, CH, BT>(indices, values, lo + from + whole, to - from - whole, ln, a.B, acc);
-        __syncthreads();                                     // the row before has been read out
-#pragma unroll
-        for (int c = 0; c < CH; ++c) {
-            if (!ln.on[c]) continue;
-#pragma unroll
-            for (int i = 0; i < VEC; ++i) s_red[sw * a.feat + ln.f[c] + i] = acc.v[c][i];
-        }
-        __syncthreads();
-        for (int f = tid; f < a.feat; f += kThreads) {
-            float sum = 0.f;
-            for (int k = 0; k < SW; ++k) sum += s_red[k * a.feat + f];
-            a.C[(size_t)(first_row + r) * a.ldc + f] = sum;
-        }
-    }
-}
-
-// ------------------------------------------------------------------------------------
 // Plan-time kernels.
 
 // Inclusive scans over a 256-thread workgroup: the largest value at or before a thread, the
@@ -1609,7 +1368,6 @@ int free_temporaries(lf_spmm_plan* p) {
 
 using KernelFn = void (*)(LaunchArgs);
 using FinalFn = void (*)(const HeavyRow*, int, LaunchArgs);
-using CsrFn = void (*)(const int32_t*, const int32_t*, const float*, long long, int, LaunchArgs);
 
 using RowGroupFn = void (*)(const MergedBucket*, int, LaunchArgs);
 
@@ -1617,7 +1375,6 @@ struct KernelSet {
     KernelFn tiles = nullptr;
     KernelFn tiles_resident = nullptr;   // the same where there is no such kernel
     FinalFn finalize_wide = nullptr;
-    CsrFn csr = nullptr;
     RowGroupFn rowgroup = nullptr;   // one 16-byte chunk per lane only
 };
 
@@ -1630,12 +1387,10 @@ template <int LPR, int CH> void pick_kernels(int dtype, KernelSet* k) {
         k->tiles = spmm_partition_kernel<LPR, CH, bf16_t, false>;
         k->tiles_resident = spmm_partition_kernel<LPR, CH, bf16_t, has_resident_kernel(LPR, CH, true)>;
         k->finalize_wide = spmm_finalize_wide_kernel<LPR, CH, bf16_t>;
-        k->csr = csr_spmm_kernel<LPR, CH, bf16_t>;
     } else {
         k->tiles = spmm_partition_kernel<LPR, CH, float, false>;
         k->tiles_resident = spmm_partition_kernel<LPR, CH, float, has_resident_kernel(LPR, CH, false)>;
         k->finalize_wide = spmm_finalize_wide_kernel<LPR, CH, float>;
-        k->csr = csr_spmm_kernel<LPR, CH, float>;
     }
 }
 
@@ -1653,22 +1408,6 @@ int select_kernels(int lpr, int ch, int dtype, KernelSet* k) {
         pick_kernels<64, 4>(dtype, k);
     }
     LF_REQUIRE(k->tiles != nullptr, LF_ERR_UNSUPPORTED, "no kernel for %d lanes x %d chunks", lpr, ch);
-    return LF_OK;
-}
-
-int feature_shape(int feat, int dtype, int* lpr, int* ch) {
-    const int vec = dtype == LF_DTYPE_BF16 ? 8 : 4;
-    LF_REQUIRE(feat >= 32 && feat % 32 == 0, LF_ERR_UNSUPPORTED,
-               "feat_size must be a positive multiple of 32 (got %d)", feat);
-    LF_REQUIRE(feat <= 1024, LF_ERR_UNSUPPORTED, "feat_size above 1024 is not supported (got %d)", feat);
-    const int lanes = feat / vec;
-    int l = 8;
-    while (l < lanes && l < 64) l <<= 1;
-    int c = (lanes + l - 1) / l;
-    if (c == 3) c = 4;
-    LF_REQUIRE(c == 1 || c == 2 || c == 4, LF_ERR_UNSUPPORTED, "feat_size %d is not supported", feat);
-    *lpr = l;
-    *ch = c;
     return LF_OK;
 }
 
@@ -2397,58 +2136,6 @@ int lf_spmm_set_windows(lf_spmm_plan* plan, int32_t n_windows) {
                "bad number of feature windows (%d)", n_windows);
     plan->windows = n_windows;
     return LF_OK;
-}
-
-int lf_csr_spmm_trusted(const int32_t* d_indptr, const int32_t* d_indices, const float* d_values,
-                        int64_t num_rows, int64_t num_cols, int32_t feat_size, int32_t b_dtype,
-                        const void* d_B, float* d_C, lf_stream_t stream) {
-    hipStream_t s = (hipStream_t)stream;
-    LF_REQUIRE(num_rows >= 0 && num_rows < (1ll << 31) && num_cols >= 1, LF_ERR_INVALID, "bad shape");
-    if (num_rows == 0) return LF_OK;
-    LF_REQUIRE(d_indptr && d_B && d_C, LF_ERR_INVALID, "null argument");
-    LF_REQUIRE(b_dtype == LF_DTYPE_F32 || b_dtype == LF_DTYPE_BF16, LF_ERR_INVALID, "unknown B dtype %d", b_dtype);
-    LF_REQUIRE((uintptr_t)d_B % 16 == 0 && (uintptr_t)d_C % 16 == 0, LF_ERR_INVALID, "B and C must be 16-byte aligned");
-    int lpr, ch;
-    if (int rc = feature_shape(feat_size, b_dtype, &lpr, &ch)) return rc;
-    KernelSet ks;
-    if (int rc = select_kernels(lpr, ch, b_dtype, &ks)) return rc;
-    LaunchArgs a{};
-    a.feat = feat_size;
-    a.ldb = a.ldc = feat_size;
-    a.B = d_B;
-    a.C = d_C;
-    const int threads = csr_threads(lpr, ch * (b_dtype == LF_DTYPE_BF16 ? 8 : 4));
-    const size_t lds = (size_t)(threads / lpr) * feat_size * 4;     // at most 16 KB: csr_threads times values per lane is at most 4096
-    // As many rows as sub-waves spread a matrix over the CUs and give each one to sum.  Workgroups of 16 whole
-    // wavefronts, of which a CU holds one, take twice as many where 16 rows each would be more than one round of
-    // the 256 CUs (N = 256, 5K rows of 100 entries: 63 us with 32, 72 with 16; 2K rows of 40: 23 with 32, 16 with 16).
-    // Above kCsrManyRows a workgroup's start is paid too often for rows that are short themselves, and runs over
-    // 64 rows are streamed instead (1.5M rows of 8, N = 128: 0.96 ms, with a row per sub-wave 1.11; 600K rows
-    // of 12: 567 us, with a row per sub-wave 530; N = 224 0.94 ms, 0.96).
-    const bool whole = threads == 1024;                      // a sub-wave is a wavefront, and they fill a CU
-    const int rows_per_group = num_rows > (whole ? kCsrManyRows / 2 : kCsrManyRows) ? kCsrRows : whole && num_rows > 4096 ? 32 : threads / lpr;
-    ks.csr<<<(unsigned)lf::ceil_div(num_rows, rows_per_group), threads, lds, s>>>(d_indptr, d_indices, d_values, num_rows,
-                                                                                  rows_per_group, a);
-    LF_HIP(hipGetLastError());
-    return LF_OK;
-}
-
-int lf_csr_spmm(const int32_t* d_indptr, const int32_t* d_indices, const float* d_values,
-                int64_t num_rows, int64_t num_cols, int64_t nnz, int32_t feat_size, int32_t b_dtype,
-                const void* d_B, float* d_C, void* d_scratch, lf_stream_t stream) {
-    // arguments first, so that a bad feature size or operand is reported without touching the GPU
-    LF_REQUIRE(num_rows >= 0 && num_rows < (1ll << 31) && num_cols >= 1, LF_ERR_INVALID, "bad shape");
-    if (num_rows > 0) {
-        LF_REQUIRE(d_indptr && d_B && d_C, LF_ERR_INVALID, "null argument");
-        LF_REQUIRE(b_dtype == LF_DTYPE_F32 || b_dtype == LF_DTYPE_BF16, LF_ERR_INVALID, "unknown B dtype %d", b_dtype);
-        int lpr, ch;
-        if (int rc = feature_shape(feat_size, b_dtype, &lpr, &ch)) return rc;
-    }
-    // no gather before the index arrays have passed
-    if (int rc = lf::csr_check(d_indptr, d_indices, nullptr, num_rows, num_cols, nnz, d_scratch, nullptr, "lf_csr_spmm",
-                               (hipStream_t)stream))
-        return rc;
-    return lf_csr_spmm_trusted(d_indptr, d_indices, d_values, num_rows, num_cols, feat_size, b_dtype, d_B, d_C, stream);
 }
 
 int lf_spmm_time_ms(lf_spmm_plan* plan, const void* d_B, float* d_C, int32_t warmup, int32_t repeat,

@@ -322,4 +322,21 @@ inline hipError_t exclusive_scan_i32(const int32_t* m, long long n, int32_t* par
     return hipGetLastError();
 }
 
+// Lanes per row of B and 16-byte chunks per lane of a product of `feat` features.
+inline int feature_shape(int feat, int dtype, int* lpr, int* ch) {
+    const int vec = dtype == LF_DTYPE_BF16 ? 8 : 4;
+    LF_REQUIRE(feat >= 32 && feat % 32 == 0, LF_ERR_UNSUPPORTED,
+               "feat_size must be a positive multiple of 32 (got %d)", feat);
+    LF_REQUIRE(feat <= 1024, LF_ERR_UNSUPPORTED, "feat_size above 1024 is not supported (got %d)", feat);
+    const int lanes = feat / vec;
+    int l = 8;
+    while (l < lanes && l < 64) l <<= 1;
+    int c = (lanes + l - 1) / l;
+    if (c == 3) c = 4;
+    LF_REQUIRE(c == 1 || c == 2 || c == 4, LF_ERR_UNSUPPORTED, "feat_size %d is not supported", feat);
+    *lpr = l;
+    *ch = c;
+    return LF_OK;
+}
+
 }  // namespace

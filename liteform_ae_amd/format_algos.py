@@ -643,9 +643,9 @@ def spmm_csr(g, B, b_dtype: str = "f32", use_values: bool = True):
     out = torch.empty((dev.num_rows, feat), dtype=torch.float32, device="cuda")
     vals = dev.values if use_values else None
     # the device arrays were made by lf_coo_to_csr or have passed lf_csr_check: no second check
-    rc = lib.lf_csr_spmm_trusted(dev.indptr.data_ptr(), dev.indices.data_ptr(), None if vals is None else vals.data_ptr(),
-                                 dev.num_rows, dev.num_cols, feat, _B_DTYPES[b_dtype], B.data_ptr(), out.data_ptr(),
-                                 _stream())
+    rc = lib.lf_csr_spmm_trusted_nnz(dev.indptr.data_ptr(), dev.indices.data_ptr(), None if vals is None else vals.data_ptr(),
+                                     dev.num_rows, dev.num_cols, dev.nnz, feat, _B_DTYPES[b_dtype], B.data_ptr(),
+                                     out.data_ptr(), _stream())
     if rc:
         _lib.check(rc)
     return out

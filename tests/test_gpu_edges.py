@@ -287,6 +287,42 @@ def test_csr_product_of_short_rows(fa, torch, nr, feat, b_dtype, usual, longest)
         assert (np.abs(got[~hit] - want[~hit]) <= bound[~hit]).all()
 
 
+@pytest.mark.parametrize("nr,nc,feat,b_dtype", [
+    *((nr, 3000, feat, b) for nr in (1, 7, 9, 300) for feat, b in ((32, "f32"), (64, "f32"), (96, "f32"), (128, "f32"), (256, "f32"),
+                                                                   (512, "f32"), (1024, "f32"), (128, "bf16"), (256, "bf16"), (512, "bf16"))),
+    (24_575, 3000, 32, "f32"), (24_576, 3000, 64, "f32"), (24_577, 3000, 256, "f32"),          # the two group sizes
+    (300, 1_060_000, 1024, "f32"),                           # 4.3 GB of B: past what 32-bit offsets reach
+    (40, 2_200_000, 992, "bf16"),
+])
+def test_csr_product_of_uneven_rows(fa, torch, nr, nc, feat, b_dtype):
+    """Long rows between short ones (a wavefront's teams hold rows of both kinds), rows of every remainder of a
+    batch, first and last column, features split over the XCDs (small matrices and whole multiples of 128 bytes
+    are), with and without values; twice the same bits."""
+    import scipy.sparse as sp
+    rng = np.random.default_rng(nr + feat)
+    deg = np.arange(nr) * 7 % 19
+    deg[nr // 3::11] = 33
+    deg[(np.arange(6) * 3 + nr // 2) % nr] = (257, 300, 1025, 0, 2999, 256)
+    indptr = np.concatenate([[0], np.cumsum(deg)]).astype(np.int32)
+    col = np.concatenate([np.sort(rng.choice(nc, size=n, replace=False)) if n > 40 else np.sort((rng.integers(nc) + 61 * np.arange(n)) % nc)
+                          for n in deg]).astype(np.int32)
+    if deg[-1]:
+        col[-1] = nc - 1
+    if deg[0]:
+        col[0] = 0
+    vals = rng.uniform(-1, 1, size=len(col)).astype(np.float32)
+    gen = torch.Generator(device="cuda").manual_seed(nr)
+    B = torch.rand((nc, feat), device="cuda", generator=gen, dtype=torch.float32 if b_dtype == "f32" else torch.bfloat16)
+    used, at = np.unique(col, return_inverse=True)
+    Bh = B[torch.from_numpy(used.astype(np.int64)).cuda()].float().cpu().numpy().astype(np.float64)
+    g = MTX.from_csr(indptr, col, (nr, nc), data=vals)
+    for use_values in (True, False):
+        A = sp.csr_matrix((vals.astype(np.float64) if use_values else np.ones(len(col)), at, indptr), shape=(nr, len(used)))
+        got = fa.spmm_csr(g, B, b_dtype, use_values=use_values)
+        assert torch.equal(got, fa.spmm_csr(g, B, b_dtype, use_values=use_values))
+        assert (np.abs(got.cpu().numpy() - A @ Bh) <= 1e-5 * (abs(A) @ np.abs(Bh)) + 1e-30).all()
+
+
 @pytest.mark.parametrize("feat,b_dtype", [(32, "f32"), (128, "f32"), (320, "f32"), (1024, "f32"), (64, "bf16"), (512, "bf16")])
 def test_rows_of_several_chunks(fa, torch, monkeypatch, feat, b_dtype):
     """Long rows of one chunk, a few, the most that the last chunk's workgroup adds up and one more;
