@@ -6,9 +6,6 @@
 // or a row each, as the lengths of the workgroup's rows ask for.
 #include <hip/hip_runtime.h>
 
-#include <algorithm>
-#include <cmath>
-#include <utility>
 
 #include "lf_internal.h"
 #include "lf_spmm_device.h"
@@ -21,7 +18,6 @@ constexpr int kCsrThreads = 256;
 constexpr int kCsrRowsFew = 8, kCsrRowsMany = 16;
 constexpr long long kCsrManyRows = 24576;
 constexpr int kCsrLongRow = 256;           // a row of more entries, and more than a wavefront's share, takes the whole workgroup
-constexpr int kCsrUnroll = 8;              // gathers in flight per sub-wave
 
 struct CsrArgs {
     const int32_t* indptr;
@@ -29,109 +25,11 @@ struct CsrArgs {
     const float* values;                   // null: ones
     long long n_rows, n_groups;
     int rows_per_group;
-    int slices;                            // feature slices, a power of two up to kXcds
+    int lg_slices;                         // log2 of the feature slices, up to kLgXcds
     int feat, ld;                          // features of a slice; elements between rows of B and of C
     const void* B;
     float* C;
     unsigned long long b_bytes;
-};
-
-// Gathers go through a buffer resource over B: the lane that fetched an entry multiplies its column by the bytes of a
-// row once, a gather then costs one addition (with the broadcast in it) for its address, and entries past the end of
-// a row get an offset past the end of B, for which the hardware returns zeros without touching memory - no padding
-// traffic, and nothing for an infinite element of B to turn into NaN.  Offsets have 32 bits: a larger B takes
-// 64-bit addresses and predicated loads instead (WIDE; 57K rows of 28 entries, N = 64 .. 256: 1 - 7 % slower).
-constexpr uint32_t kPastB = 0xFFFE0000u;   // (a lane's own offset is below 2^17)
-
-// Entry I of the sub-wave's batch, from the lane that holds it, by a DPP broadcast: one operand modifier of the
-// addition or move that uses it, where a shuffle is an LDS instruction and its latency.
-template <int LPR, int I> __device__ __forceinline__ int batch_entry(int x) {
-    constexpr int kRowBroadcast = 0x150;   // row_newbcast: a lane of each row of 16 to that row
-    if constexpr (LPR >= 16) {
-        return __builtin_amdgcn_update_dpp(0, x, kRowBroadcast + I, 0xF, 0xF, true);
-    } else {                               // two sub-waves to a row of 16 lanes
-        const int first = __builtin_amdgcn_update_dpp(0, x, kRowBroadcast + I, 0xF, 0x3, false);
-        return __builtin_amdgcn_update_dpp(first, x, kRowBroadcast + 8 + I, 0xF, 0xC, false);
-    }
-}
-
-typedef unsigned int lf_u32x4 __attribute__((ext_vector_type(4)));
-
-// A wavefront's teams of 2^lg sub-waves.  Entry e of a row goes to sub-wave e mod 2^lg of its team.
-template <int LPR, int CH, typename BT, bool WIDE> struct Teams {
-    static constexpr int VEC = Dense<BT>::kVec;
-    static constexpr int kBatch = LPR < 16 ? LPR : 16;      // entries of a sub-wave fetched at a time
-    using Raw = typename Dense<BT>::Raw;
-    const int32_t* indices;
-    const float* values;
-    const char* B;
-    __amdgpu_buffer_rsrc_t rsrc;
-    uint32_t pitch;                        // bytes between rows of B
-    uint32_t lane_at[CH];                  // the lane's own bytes in a row of B
-    int lg;
-    int sub;                               // sub-wave in its team
-    int slot;                              // entry of a batch that the lane fetches (in every 16 lanes again)
-
-    // The lane's entry of the batch at `base` of the row of `len` entries from `lo` on.
-    __device__ __forceinline__ void fetch(int lo, int len, int base, int& col, float& val) const {
-        const int e = base + (slot << lg) + sub;
-        col = -1;
-        val = 0.f;
-        if (e < len) {
-            col = indices[lo + e];
-            val = values ? values[lo + e] : 1.f;
-        }
-    }
-
-    template <int FIRST, size_t... I>
-    __device__ __forceinline__ void gather(int at, float val, Acc<CH, VEC>& acc, std::index_sequence<I...>) const {
-        Raw x[kCsrUnroll][CH];
-        auto load = [&](int u, int from) {
-#pragma unroll
-            for (int c = 0; c < CH; ++c) {
-                if constexpr (WIDE) {
-                    x[u][c] = Raw{};
-                    if (from >= 0) x[u][c] = *reinterpret_cast<const Raw*>(B + lane_at[c] + (uint64_t)(uint32_t)from * pitch);
-                } else {
-                    const lf_u32x4 raw = __builtin_amdgcn_raw_buffer_load_b128(rsrc, (uint32_t)from + lane_at[c], 0, 0);
-                    __builtin_memcpy(&x[u][c], &raw, sizeof(Raw));
-                }
-            }
-        };
-        (load(I, batch_entry<LPR, FIRST + I>(at)), ...);
-        auto add = [&](int u, float v) {
-#pragma unroll
-            for (int c = 0; c < CH; ++c) fma_dense<BT>(v, x[u][c], acc.v[c]);
-        };
-        (add(I, __int_as_float(batch_entry<LPR, FIRST + I>(__float_as_int(val)))), ...);
-    }
-
-    // Adds the entries of the team's row; `most` is the length of the wavefront's longest row (uniform).
-    __device__ __forceinline__ void sum(int lo, int len, int most, Acc<CH, VEC>& acc) const {
-        constexpr auto kEight = std::make_index_sequence<kCsrUnroll>();
-        int col;
-        float val;
-        fetch(lo, len, 0, col, val);
-        for (int base = 0; base < most;) {
-            const int at = WIDE ? col : col >= 0 ? (int)((uint32_t)col * pitch) : (int)kPastB;
-            const float v = val;
-            const int left = most - base;
-            base += kBatch << lg;
-            if (base < most) fetch(lo, len, base, col, val);
-            gather<0>(at, v, acc, kEight);
-            if constexpr (kBatch > kCsrUnroll)
-                if (left > (kCsrUnroll << lg)) gather<kCsrUnroll>(at, v, acc, kEight);
-        }
-    }
-
-    // The team's sums, added pairwise: every lane of the team holds them afterwards.
-    __device__ __forceinline__ void combine(Acc<CH, VEC>& acc) const {
-        for (int d = LPR; d < (LPR << lg); d <<= 1)
-#pragma unroll
-            for (int c = 0; c < CH; ++c)
-#pragma unroll
-                for (int i = 0; i < VEC; ++i) acc.v[c][i] += __shfl_xor(acc.v[c][i], d);
-    }
 };
 
 // Bound by the gathers where rows are long; by the chain row pointer - entries - gathers and the number of
@@ -153,28 +51,19 @@ __global__ void __launch_bounds__(kCsrThreads)
 csr_spmm_kernel(CsrArgs a) {
     constexpr int VEC = Dense<BT>::kVec;
     constexpr int kWaves = kCsrThreads / 64;
-    constexpr int kLgSubs = LPR == 64 ? 0 : LPR == 32 ? 1 : LPR == 16 ? 2 : 3;      // log2 of the wavefront's sub-waves
-    using T = Teams<LPR, CH, BT, WIDE>;
+    constexpr int kLgSubs = Teams<LPR, CH, BT, WIDE>::kLgSubs;
     __shared__ int s_next;
     extern __shared__ __align__(16) float s_red[];         // [kWaves][feat]: sums of a long row's parts
-    // workgroup i runs on XCD i % 8; XCD x computes slice x mod slices of its rows
-    const int xcd = blockIdx.x % kXcds, slice = xcd & (a.slices - 1);
-    const long long group = (long long)(blockIdx.x / kXcds) * (kXcds / a.slices) + xcd / a.slices;
+    // workgroup i runs on XCD i % 8; XCD x computes slice x mod 2^lg_slices of its rows
+    const int xcd = blockIdx.x % kXcds, slice = xcd & ((1 << a.lg_slices) - 1);
+    const long long group = ((long long)(blockIdx.x / kXcds) << (kLgXcds - a.lg_slices)) + (xcd >> a.lg_slices);
     if (group >= a.n_groups) return;
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int sl = lane % LPR, sub = lane / LPR;
-    const Lane<LPR, CH, VEC> ln(sl, a.feat, a.ld, a.ld);
+    const int sub = lane / LPR;
+    const Lane<LPR, CH, VEC> ln(lane % LPR, a.feat, a.ld, a.ld);
     const size_t skip = (size_t)slice * a.feat;
+    const RowsOfB<LPR, CH, BT, WIDE> b((const char*)a.B + skip * Dense<BT>::kElemBytes, a.b_bytes - skip * Dense<BT>::kElemBytes, ln);
     float* C = a.C + skip;
-    T t;
-    t.indices = a.indices;
-    t.values = a.values;
-    t.B = (const char*)a.B + skip * Dense<BT>::kElemBytes;
-    t.pitch = (uint32_t)a.ld * Dense<BT>::kElemBytes;
-    t.rsrc = __builtin_amdgcn_make_buffer_rsrc((void*)t.B, 0, WIDE ? 0 : (int)(uint32_t)(a.b_bytes - skip * Dense<BT>::kElemBytes), 0x00027000);
-#pragma unroll
-    for (int c = 0; c < CH; ++c) t.lane_at[c] = ln.f[c] * Dense<BT>::kElemBytes;
-    t.slot = sl % T::kBatch;
 
     const long long first_row = group * a.rows_per_group;
     const int n = (int)min((long long)a.rows_per_group, a.n_rows - first_row);       // at most 64
@@ -185,10 +74,9 @@ csr_spmm_kernel(CsrArgs a) {
     const unsigned long long longs = __ballot(end - start > max(kCsrLongRow, total / kWaves));      // the same in every wavefront
     // as many sub-waves as give each one batch of gathers of an average row (half or twice as many: 1 - 7 % slower)
     int lg = 0;
-    while (lg < kLgSubs && ((long long)(n * kCsrUnroll) << lg) < total) ++lg;
-    t.lg = lg = __builtin_amdgcn_readfirstlane(lg);
-    t.sub = sub & ((1 << lg) - 1);
-    const int lg_rows = kLgSubs - lg, team = sub >> lg;
+    while (lg < kLgSubs && ((long long)(n * kUnroll) << lg) < total) ++lg;
+    const Teams<LPR, CH, BT, WIDE> teams(b, __builtin_amdgcn_readfirstlane(lg));
+    const int lg_rows = kLgSubs - teams.lg, team = sub >> teams.lg;
     const int sets = (n + (1 << lg_rows) - 1) >> lg_rows;
     for (int set = wave; set < sets;) {                      // 2^lg_rows rows at a time
         const int r = (set << lg_rows) + team, from = min(r, n - 1);
@@ -196,20 +84,19 @@ csr_spmm_kernel(CsrArgs a) {
         const bool mine = r < n && ((longs >> from) & 1) == 0;
         const int len = mine ? hi - lo : 0;
         int most = len;
-        for (int d = LPR << lg; d < 64; d <<= 1) most = max(most, __shfl_xor(most, d));
+        for (int d = LPR << teams.lg; d < 64; d <<= 1) most = max(most, __shfl_xor(most, d));
         Acc<CH, VEC> acc;
         acc.clear();
-        t.sum(lo, len, __builtin_amdgcn_readfirstlane(most), acc);
-        t.combine(acc);
-        if (t.sub == 0 && mine) store_row<LPR, CH, VEC>(C, (int)(first_row + r), ln, acc, kStreamC);
+        teams.sum(a.indices, a.values, lo, len, __builtin_amdgcn_readfirstlane(most), acc);
+        teams.combine(acc);
+        if (teams.sub == 0 && mine) store_row<LPR, CH, VEC>(C, (int)(first_row + r), ln, acc, kStreamC);
         int next = 0;
         if (lane == 0) next = atomicAdd(&s_next, 1);
         set = __builtin_amdgcn_readfirstlane(next);
     }
     // Long rows: a part to each wavefront, the parts' sums added in their order.
-    t.lg = kLgSubs;
-    t.sub = sub;
-    constexpr int kStep = T::kBatch << kLgSubs;
+    const Teams<LPR, CH, BT, WIDE> all(b, kLgSubs);
+    constexpr int kStep = Teams<LPR, CH, BT, WIDE>::kBatch << kLgSubs;
     for (unsigned long long todo = longs; todo; todo &= todo - 1) {                  // uniform
         const int r = __ffsll((long long)todo) - 1;
         const int lo = __builtin_amdgcn_readlane(start, r), len = __builtin_amdgcn_readlane(end, r) - lo;
@@ -217,8 +104,8 @@ csr_spmm_kernel(CsrArgs a) {
         const int from = (int)min((long long)wave * per, (long long)len), part = min(per, len - from);
         Acc<CH, VEC> acc;
         acc.clear();
-        t.sum(lo + from, part, part, acc);
-        t.combine(acc);
+        all.sum(a.indices, a.values, lo + from, part, part, acc);
+        all.combine(acc);
         if (sub == 0) {
 #pragma unroll
             for (int c = 0; c < CH; ++c) {
@@ -251,34 +138,14 @@ CsrFn csr_kernel(int lpr, int ch, int dtype, bool wide) {
          : lpr == 32 ? csr_kernel<32, 1>(dtype, wide) : csr_kernel<64, 1>(dtype, wide);
 }
 
-// Feature slices: XCD x computes slice x mod S of the features for every (8 / S)-th group of rows, so that its L2
-// has 1 / S of B to hold instead of all of it, at the price of reading the entries S times.  A slice is
-// 128 bytes or a multiple: a gather of 64 moves the line all the same (a table in the L2s is gathered from at 28 TB/s
-// by rows of 128 bytes and more, 15.5 by rows of 64).  The S that a simple price puts first: gathers that miss at 7.3
-// TB/s and those that hit at 28, the share that hits from the slice's size and from how often an XCD uses a row of B
-// (from the second time on), and 10 % for every halving of the workgroups below 2048, which is what small matrices
-// gain from the split.  130 matrices of 2K to 1.2M rows, log-normal and power-law, N = 64 .. 512, f32 and bf16, every
-// S timed: the pick loses 2.1 % on average to the best, S = 1 24 %, S = 4 4.6 %.  Worst picks: 34 % (9K x 13K, 31K
-// entries, bf16 N = 256: 8.5 us with 2, 11.4 with 4), and against S = 1 14 % (335K power-law rows, N = 128: 119 -> 135).
-int csr_slices(int64_t num_rows, int64_t num_cols, int64_t nnz, int feat, int dtype) {
-    constexpr double kL2 = 5.5e6, kMissRate = 7.3, kHitRate = 28.0, kGroups = 2048.0;
-    const int elem = dtype == LF_DTYPE_BF16 ? 2 : 4, step = 128 / elem;
-    const double b_bytes = (double)num_cols * feat * elem, gathered = (double)nnz * feat * elem;
-    const double groups = (double)num_rows / (num_rows >= kCsrManyRows ? kCsrRowsMany : kCsrRowsFew) + 1.0;
-    int best = 1;
-    double least = 0.0;
-    for (int s = 1; s <= kXcds && nnz > 0; s *= 2) {
-        if (feat % (s * step) != 0) break;
-        const double uses = (double)nnz / (double)num_cols * s / kXcds;
-        const double hit = std::min(1.0, kL2 * s / b_bytes) * std::max(0.0, 1.0 - 1.0 / uses);
-        double price = gathered * ((1.0 - hit) / kMissRate + hit / kHitRate) + 8.0 * (double)nnz * s / kMissRate;
-        price *= 1.0 + 0.1 * std::max(0.0, std::log2(kGroups / (groups * s)));
-        if (s == 1 || price < 0.98 * least) {
-            least = price;
-            best = s;
-        }
-    }
-    return best;
+// 10 % for every halving of the workgroups below 2048: what small matrices gain from the split besides.  130 matrices of
+// 2K to 1.2M rows, log-normal and power-law, N = 64 .. 512, f32 and bf16, every S timed: the pick loses 2 % on average
+// to the best, S = 1 24 %, S = 4 4.6 %.  Worst picks: 34 % (9K x 13K, 31K entries, bf16 N = 256: 8.5 us with 2, 11.4
+// with 4), and against S = 1 14 % (335K power-law rows, N = 128: 119 -> 135).
+int csr_slices(int64_t groups, int64_t num_cols, int64_t nnz, int feat, int dtype) {
+    return feature_slices(num_cols, nnz, feat, dtype, [&](int s, double us) {
+        return us * (1.0 + 0.1 * std::max(0.0, std::log2(2048.0 / ((double)groups * s)))) * (s > 1 ? 1.02 : 1.0);
+    });
 }
 
 }  // namespace
@@ -296,20 +163,21 @@ int lf_csr_spmm_trusted_nnz(const int32_t* d_indptr, const int32_t* d_indices, c
     int lpr, ch;
     if (int rc = feature_shape(feat_size, b_dtype, &lpr, &ch)) return rc;
     CsrArgs a{};
-    a.slices = csr_slices(num_rows, num_cols, nnz, feat_size, b_dtype);
-    a.feat = feat_size / a.slices;
+    a.rows_per_group = num_rows >= kCsrManyRows ? kCsrRowsMany : kCsrRowsFew;
+    a.n_groups = lf::ceil_div(num_rows, (int64_t)a.rows_per_group);
+    const int slices = csr_slices(a.n_groups, num_cols, nnz, feat_size, b_dtype);
+    a.lg_slices = lf::ilog2(slices);
+    a.feat = feat_size / slices;
     if (int rc = feature_shape(a.feat, b_dtype, &lpr, &ch)) return rc;
     a.indptr = d_indptr;
     a.indices = d_indices;
     a.values = d_values;
     a.n_rows = num_rows;
-    a.rows_per_group = num_rows >= kCsrManyRows ? kCsrRowsMany : kCsrRowsFew;
-    a.n_groups = lf::ceil_div(num_rows, (int64_t)a.rows_per_group);
     a.ld = feat_size;
     a.B = d_B;
     a.C = d_C;
     a.b_bytes = (unsigned long long)num_cols * feat_size * (b_dtype == LF_DTYPE_BF16 ? 2 : 4);
-    const unsigned grid = (unsigned)(lf::ceil_div(a.n_groups, (int64_t)(kXcds / a.slices)) * kXcds);
+    const unsigned grid = (unsigned)(lf::ceil_div(a.n_groups, (int64_t)(kXcds / slices)) * kXcds);
     csr_kernel(lpr, ch, b_dtype, a.b_bytes > kPastB)<<<grid, kCsrThreads, (kCsrThreads / 64) * a.feat * sizeof(float), (hipStream_t)stream>>>(a);
     LF_HIP(hipGetLastError());
     return LF_OK;

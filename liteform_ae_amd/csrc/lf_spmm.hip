@@ -10,10 +10,9 @@
 //     features (float4, or 8 x bf16 = 16 bytes), so one B row is read with one 16-byte load
 //     per lane, coalesced along the feature dimension (N = 128 fp32 -> 32 lanes, two rows
 //     per 64-lane wavefront);
-//   * narrow buckets stage their (column, value) tile in LDS with coalesced 16-byte loads
-//     and read it back as broadcasts; wide buckets and the widest bucket of a partition
-//     (whose source rows may span several ELL rows) stream slots through wavefront
-//     shuffles instead;
+//   * narrow buckets stage their (row of B, value) tile in LDS with coalesced 16-byte loads
+//     and read it back as broadcasts; rows too wide to stage are streamed by a wavefront each, their slots spread
+//     over its sub-waves and broadcast by DPP;
 //   * a source row split over several ELL rows is summed by one owner; rows longer than
 //     coop_slots (64, 128 or 256) are reduced by a whole workgroup in chunks of 512 to 8192 slots: a row
 //     that fits one chunk is written directly, a longer one leaves one partial row per chunk, which the
@@ -23,8 +22,8 @@
 //     atomics and the order of every sum is fixed, so results are bit-reproducible; the one atomic of a
 //     product counts the chunks of a long row that have left their partial row.
 //
-// The workgroup -> tile mapping is XCD-aware: workgroup i runs on XCD i % 8, and each
-// group of tiles is cut into 8 contiguous ranges, one per XCD, so that neighbouring ELL
+// The workgroup -> tile mapping is XCD-aware: workgroup i runs on XCD i % 8, XCD x computes feature slice x mod S,
+// and each group of tiles is cut into 8 / S contiguous ranges, one per XCD of a slice, so that neighbouring ELL
 // rows (which tend to share B rows in structured matrices) meet in the same L2.
 #include <hip/hip_runtime.h>
 
@@ -41,76 +40,39 @@
 
 namespace {
 
-// Sum of `total` consecutive slab slots starting at `base`, streamed by one sub-wave: each
-// lane loads one (col, val), the sub-wave then walks them by shuffle.  Slots past `total`
-// are replaced by (first column, 0) so that every gather is unconditional and in range.
-template <int LPR, int CH, typename BT>
-__device__ __forceinline__ void stream_slots(const int32_t* __restrict__ cols, const float* __restrict__ vals,
-                                             long long base, int total, const void* B,
-                                             const Lane<LPR, CH, Dense<BT>::kVec>& ln,
-                                             Acc<CH, Dense<BT>::kVec>& acc) {
-    constexpr int U = kUnroll < LPR ? kUnroll : LPR;
-    if (total <= 0) return;
-    const int c_first = cols[base];
-    // the next batch of slots is requested before the current one is walked: a slab is read
-    // once, so each of these loads waits out the full memory latency
-    int next_c = ln.sl < total ? cols[base + ln.sl] : c_first;
-    float next_v = ln.sl < total ? (vals ? vals[base + ln.sl] : 1.f) : 0.f;
-    for (int off = 0; off < total; off += LPR) {
-        const int my_c = next_c;
-        const float my_v = next_v;
-        const int idx = off + LPR + ln.sl;
-        const bool have = idx < total;
-        next_c = have ? cols[base + idx] : c_first;
-        next_v = have ? (vals ? vals[base + idx] : 1.f) : 0.f;
-        const int cnt = min(LPR, total - off);
-        for (int j = 0; j < cnt; j += U) {
-            int c[U];
-            float v[U];
-#pragma unroll
-            for (int u = 0; u < U; ++u) {
-                c[u] = __shfl(my_c, j + u, LPR);
-                v[u] = __shfl(my_v, j + u, LPR);
-            }
-            gather_fma<U, LPR, CH, BT>(B, ln, c, v, acc);
-        }
-    }
-}
-
 // ------------------------------------------------------------------------------------
-// Tile bodies.  s_pairs / s_rm point into the workgroup's LDS: tile_slots(LPR) (col, val)
+// Tile bodies.  s_pairs / s_rm point into the workgroup's LDS: tile_slots(LPR) (key of B's row, val)
 // pairs followed by kTileRows (row, meta) entries.
 
 // Narrow bucket: W slots per ELL row, rows independent (one ELL row per source row).
 // RPI rows are processed together by a sub-wave so that kUnroll gathers are in flight
 // even when W < kUnroll.
-template <int W, int LPR, int CH, typename BT>
-__device__ __forceinline__ void ell_tile_narrow(const int2* s_pairs, const int2* s_rm, int n,
+template <int W, int LPR, int CH, typename BT, bool WIDE>
+__device__ __forceinline__ void ell_tile_narrow(const RowsOfB<LPR, CH, BT, WIDE>& b, const int2* s_pairs, const int2* s_rm, int n,
                                                 const LaunchArgs& a, int sw, int sl) {
     constexpr int VEC = Dense<BT>::kVec;
     constexpr int SW = kWG / LPR;
     constexpr int RPI = kUnroll / W;
     const Lane<LPR, CH, VEC> ln(sl, a.feat, a.ldb, a.ldc);
     for (int r0 = sw * RPI; r0 < n; r0 += SW * RPI) {
-        int c[kUnroll];
+        uint32_t k[kUnroll];
         float v[kUnroll];
 #pragma unroll
         for (int q = 0; q < RPI; ++q) {
             const int r = min(r0 + q, n - 1);
-            const int len = s_rm[r].y & kMetaLenMask;
-            const int c0 = s_pairs[r * W].x;
+            const int len = r0 + q < n ? s_rm[r].y & kMetaLenMask : 0;
 #pragma unroll
             for (int j = 0; j < W; ++j) {
-                const int2 cv = s_pairs[r * W + j];
-                c[q * W + j] = j < len ? cv.x : c0;
-                v[q * W + j] = __int_as_float(cv.y);
+                const int2 kv = s_pairs[r * W + j];
+                k[q * W + j] = j < len ? (uint32_t)kv.x : b.kNone;
+                v[q * W + j] = __int_as_float(kv.y);
             }
         }
         typename Dense<BT>::Raw x[kUnroll][CH];
 #pragma unroll
         for (int u = 0; u < kUnroll; ++u)
 #pragma unroll
-            for (int cc = 0; cc < CH; ++cc) x[u][cc] = load_dense<BT>(a.B, ln, cc, c[u]);
+            for (int cc = 0; cc < CH; ++cc) x[u][cc] = b.load(cc, k[u]);
 #pragma unroll
         for (int q = 0; q < RPI; ++q) {
             Acc<CH, VEC> acc;
@@ -124,35 +86,33 @@ __device__ __forceinline__ void ell_tile_narrow(const int2* s_pairs, const int2*
     }
 }
 
-// U staged slots of an ELL row from position j; slots at or past `len` are padding and are
-// redirected to the row's first column (their value is 0).
-template <int U, int LPR, int CH, typename BT>
-__device__ __forceinline__ void staged_group(const int2* rp, int j, int len, int c0, const void* B,
-                                             const Lane<LPR, CH, Dense<BT>::kVec>& ln,
+// U staged slots of an ELL row from position j; slots at or past `len` are padding (their value is 0).
+template <int U, int LPR, int CH, typename BT, bool WIDE>
+__device__ __forceinline__ void staged_group(const RowsOfB<LPR, CH, BT, WIDE>& b, const int2* rp, int j, int len,
                                              Acc<CH, Dense<BT>::kVec>& acc) {
-    int c[U];
+    uint32_t k[U];
     float v[U];
 #pragma unroll
     for (int u = 0; u < U; ++u) {
-        const int2 cv = rp[j + u];
-        c[u] = j + u < len ? cv.x : c0;
-        v[u] = __int_as_float(cv.y);
+        const int2 kv = rp[j + u];
+        k[u] = j + u < len ? (uint32_t)kv.x : b.kNone;
+        v[u] = __int_as_float(kv.y);
     }
-    gather_fma<U, LPR, CH, BT>(B, ln, c, v, acc);
+    gather_fma<U>(b, k, v, acc);
 }
 
 // Bucket with W >= kUnroll (a multiple of it) staged in LDS: one ELL row per sub-wave at a time.
-template <int LPR, int CH, typename BT>
-__device__ __forceinline__ void ell_tile_wide(const int2* s_pairs, const int2* s_rm, int n, int log_w,
+template <int LPR, int CH, typename BT, bool WIDE>
+__device__ __forceinline__ void ell_tile_wide(const RowsOfB<LPR, CH, BT, WIDE>& b, const int2* s_pairs, const int2* s_rm, int n, int log_w,
                                               const LaunchArgs& a, int sw, int sl) {
     constexpr int VEC = Dense<BT>::kVec;
     constexpr int SW = kWG / LPR;
     const Lane<LPR, CH, VEC> ln(sl, a.feat, a.ldb, a.ldc);
+#pragma unroll 1
     for (int r = sw; r < n; r += SW) {
         const int2 rm = s_rm[r];
         const int len = rm.y & kMetaLenMask;
         const int2* rp = s_pairs + (r << log_w);
-        const int c0 = rp[0].x;
         Acc<CH, VEC> acc;
         acc.clear();
         // Whole groups of kUnroll slots, then a tail of kUnroll or kUnroll / 2 gathers.  The
@@ -161,11 +121,13 @@ __device__ __forceinline__ void ell_tile_wide(const int2* s_pairs, const int2* s
         constexpr bool kShortTail = LPR >= 32;
         if constexpr (kShortTail) {
             int j = 0;
-            for (; j + kUnroll <= len; j += kUnroll) staged_group<kUnroll, LPR, CH, BT>(rp, j, len, c0, a.B, ln, acc);
-            if (len > j && len - j <= kUnroll / 2) staged_group<kUnroll / 2, LPR, CH, BT>(rp, j, len, c0, a.B, ln, acc);
-            else if (len > j) staged_group<kUnroll, LPR, CH, BT>(rp, j, len, c0, a.B, ln, acc);
+#pragma unroll 1
+            for (; j + kUnroll <= len; j += kUnroll) staged_group<kUnroll>(b, rp, j, len, acc);
+            if (len > j && len - j <= kUnroll / 2) staged_group<kUnroll / 2>(b, rp, j, len, acc);
+            else if (len > j) staged_group<kUnroll>(b, rp, j, len, acc);
         } else {
-            for (int j = 0; j < len; j += kUnroll) staged_group<kUnroll, LPR, CH, BT>(rp, j, len, c0, a.B, ln, acc);
+#pragma unroll 1
+            for (int j = 0; j < len; j += kUnroll) staged_group<kUnroll>(b, rp, j, len, acc);
         }
         store_row<LPR, CH, VEC>(a.C, rm.x, ln, acc, a.accumulate);
     }
@@ -175,8 +137,8 @@ __device__ __forceinline__ void ell_tile_wide(const int2* s_pairs, const int2* s
 // bucket of a partition): the first ELL row of a segment owns it.  The part of the segment
 // inside the tile is read from LDS, a part that runs past the tile's end is streamed from
 // global memory.  Continuation rows and rows that take the cooperative path are skipped.
-template <int LPR, int CH, typename BT>
-__device__ __forceinline__ void ell_tile_segments(const Group& g, long long e0, const int2* s_pairs,
+template <int LPR, int CH, typename BT, bool WIDE>
+__device__ __forceinline__ void ell_tile_segments(const RowsOfB<LPR, CH, BT, WIDE>& b, const Group& g, long long e0, const int2* s_pairs,
                                                   const int2* s_rm, int n, const LaunchArgs& a, int* s_next,
                                                   int sl) {
     constexpr int VEC = Dense<BT>::kVec;
@@ -202,23 +164,23 @@ __device__ __forceinline__ void ell_tile_segments(const Group& g, long long e0, 
         }
         const int staged = min(total, (n - r) << log_w);
         const int2* rp = s_pairs + (r << log_w);
-        const int c0 = rp[0].x;
         Acc<CH, VEC> acc;
         acc.clear();
+#pragma unroll 1
         for (int j = 0; j < staged; j += kUnroll) {
-            int c[kUnroll];
+            uint32_t k[kUnroll];
             float v[kUnroll];
 #pragma unroll
             for (int u = 0; u < kUnroll; ++u) {
                 const bool in = j + u < staged;
-                const int2 cv = rp[in ? j + u : 0];
-                c[u] = in ? cv.x : c0;
-                v[u] = in ? __int_as_float(cv.y) : 0.f;
+                const int2 kv = rp[in ? j + u : 0];
+                k[u] = in ? (uint32_t)kv.x : b.kNone;
+                v[u] = in ? __int_as_float(kv.y) : 0.f;
             }
-            gather_fma<kUnroll, LPR, CH, BT>(a.B, ln, c, v, acc);
+            gather_fma<kUnroll>(b, k, v, acc);
         }
         if (total > staged)
-            stream_slots<LPR, CH, BT>(g.cols, g.vals, ((e0 + r) << log_w) + staged, total - staged, a.B, ln, acc);
+            Teams<LPR, CH, BT, WIDE>(b, 0).sum(g.cols, g.vals, ((e0 + r) << log_w) + staged, total - staged, total - staged, acc);
         store_row<LPR, CH, VEC>(a.C, rm.x, ln, acc, a.accumulate);
     }
 }
@@ -229,8 +191,8 @@ __device__ __forceinline__ void ell_tile_segments(const Group& g, long long e0, 
 // variant above a tile of a folded configuration offers fewer segments than sub-waves at
 // small N (about 20 for 32 at N = 32), and the lanes in flight bound the gather rate.
 // Rows that continue a segment begun in an earlier tile are summed by that tile, as above.
-template <int LPR, int CH, typename BT>
-__device__ __forceinline__ void ell_tile_segments_balanced(const Group& g, long long e0, const int2* s_pairs,
+template <int LPR, int CH, typename BT, bool WIDE>
+__device__ __forceinline__ void ell_tile_segments_balanced(const RowsOfB<LPR, CH, BT, WIDE>& b, const Group& g, long long e0, const int2* s_pairs,
                                                            const int2* s_rm, int n, const LaunchArgs& a,
                                                            float* s_part, int sw, int sl) {
     constexpr int VEC = Dense<BT>::kVec;
@@ -246,20 +208,20 @@ __device__ __forceinline__ void ell_tile_segments_balanced(const Group& g, long 
         if (((long long)seg << log_w) > a.coop_slots) continue; // reduced by a whole workgroup
         const int len = rm.y & kMetaLenMask;
         const int2* rp = s_pairs + (r << log_w);
-        const int c0 = rp[0].x;
         Acc<CH, VEC> acc;
         acc.clear();
+#pragma unroll 1
         for (int j = 0; j < len; j += kUnroll) {
-            int c[kUnroll];
+            uint32_t k[kUnroll];
             float v[kUnroll];
 #pragma unroll
             for (int u = 0; u < kUnroll; ++u) {
                 const bool in = j + u < len;          // W may be below kUnroll: stay inside the row
-                const int2 cv = rp[in ? j + u : 0];
-                c[u] = in ? cv.x : c0;
-                v[u] = in ? __int_as_float(cv.y) : 0.f;
+                const int2 kv = rp[in ? j + u : 0];
+                k[u] = in ? (uint32_t)kv.x : b.kNone;
+                v[u] = in ? __int_as_float(kv.y) : 0.f;
             }
-            gather_fma<kUnroll, LPR, CH, BT>(a.B, ln, c, v, acc);
+            gather_fma<kUnroll>(b, k, v, acc);
         }
         if (seg == 1) {
             store_row<LPR, CH, VEC>(a.C, rm.x, ln, acc, a.accumulate);
@@ -299,14 +261,14 @@ __device__ __forceinline__ void ell_tile_segments_balanced(const Group& g, long 
         if (inside < seg) {                                      // the segment runs past the tile: stream the rest
             const int total = ((seg - 1) << log_w) + (g.meta[e0 + r + seg - 1] & kMetaLenMask);
             const int staged = inside << log_w;
-            stream_slots<LPR, CH, BT>(g.cols, g.vals, ((e0 + r) << log_w) + staged, total - staged, a.B, ln, acc);
+            Teams<LPR, CH, BT, WIDE>(b, 0).sum(g.cols, g.vals, ((e0 + r) << log_w) + staged, total - staged, total - staged, acc);
         }
         store_row<LPR, CH, VEC>(a.C, rm.x, ln, acc, a.accumulate);
     }
 }
 
-template <int LPR, int CH, typename BT>
-__device__ __forceinline__ void run_ell_tile(const Group& g, long long tile, int2* s_pairs, int2* s_rm,
+template <int LPR, int CH, typename BT, bool WIDE>
+__device__ __forceinline__ void run_ell_tile(const RowsOfB<LPR, CH, BT, WIDE>& b, const Group& g, long long tile, int2* s_pairs, int2* s_rm,
                                              int* s_next, float* s_part, const LaunchArgs& a) {
     const int tid = threadIdx.x;
     const long long e0 = tile * g.rows_per_tile;
@@ -317,13 +279,13 @@ __device__ __forceinline__ void run_ell_tile(const Group& g, long long tile, int
         if (i + 4 <= n_slots) {            // s0 and i are multiples of 4, slabs are 16-byte aligned
             const lf_i32x4 c = load_i32x4(g.cols + s0 + i, a.accumulate & kStreamSlabs);
             const lf_i32x4 v = load_i32x4(g.vals + s0 + i, a.accumulate & kStreamSlabs);
-            s_pairs[i + 0] = make_int2(c.x, v.x);
-            s_pairs[i + 1] = make_int2(c.y, v.y);
-            s_pairs[i + 2] = make_int2(c.z, v.z);
-            s_pairs[i + 3] = make_int2(c.w, v.w);
+            s_pairs[i + 0] = make_int2((int)b.key(c.x), v.x);
+            s_pairs[i + 1] = make_int2((int)b.key(c.y), v.y);
+            s_pairs[i + 2] = make_int2((int)b.key(c.z), v.z);
+            s_pairs[i + 3] = make_int2((int)b.key(c.w), v.w);
         } else {
             for (int k = i; k < n_slots; ++k)
-                s_pairs[k] = make_int2(g.cols[s0 + k], __float_as_int(g.vals[s0 + k]));
+                s_pairs[k] = make_int2((int)b.key(g.cols[s0 + k]), __float_as_int(g.vals[s0 + k]));
         }
     }
     for (int i = tid; i < n; i += kWG) s_rm[i] = make_int2(g.rows[e0 + i], g.meta[e0 + i]);
@@ -331,35 +293,30 @@ __device__ __forceinline__ void run_ell_tile(const Group& g, long long tile, int
     __syncthreads();
     const int sw = tid / LPR, sl = tid % LPR;
     if (g.type == kEllSeg) {
-        if (g.balanced) ell_tile_segments_balanced<LPR, CH, BT>(g, e0, s_pairs, s_rm, n, a, s_part, sw, sl);
-        else ell_tile_segments<LPR, CH, BT>(g, e0, s_pairs, s_rm, n, a, s_next, sl);
+        if (g.balanced) ell_tile_segments_balanced(b, g, e0, s_pairs, s_rm, n, a, s_part, sw, sl);
+        else ell_tile_segments(b, g, e0, s_pairs, s_rm, n, a, s_next, sl);
         return;
     }
     switch (g.log_w) {
-        case 0: ell_tile_narrow<1, LPR, CH, BT>(s_pairs, s_rm, n, a, sw, sl); break;
-        case 1: ell_tile_narrow<2, LPR, CH, BT>(s_pairs, s_rm, n, a, sw, sl); break;
-        case 2: ell_tile_narrow<4, LPR, CH, BT>(s_pairs, s_rm, n, a, sw, sl); break;
-        case 3:
-            if constexpr (kUnroll > 8) ell_tile_narrow<8, LPR, CH, BT>(s_pairs, s_rm, n, a, sw, sl);
-            else ell_tile_wide<LPR, CH, BT>(s_pairs, s_rm, n, g.log_w, a, sw, sl);
-            break;
-        default: ell_tile_wide<LPR, CH, BT>(s_pairs, s_rm, n, g.log_w, a, sw, sl); break;
+        case 0: ell_tile_narrow<1>(b, s_pairs, s_rm, n, a, sw, sl); break;
+        case 1: ell_tile_narrow<2>(b, s_pairs, s_rm, n, a, sw, sl); break;
+        case 2: ell_tile_narrow<4>(b, s_pairs, s_rm, n, a, sw, sl); break;
+        default: ell_tile_wide(b, s_pairs, s_rm, n, g.log_w, a, sw, sl); break;
     }
 }
 
-// Bucket whose source rows may span several ELL rows, or whose rows are too wide to stage:
-// the first ELL row of a segment owns it and streams all of its slots; continuation rows
-// and segments above coop_slots (handled as chunks) are skipped.
-template <int LPR, int CH, typename BT>
-__device__ __forceinline__ void run_seg_tile(const Group& g, long long tile, const LaunchArgs& a) {
+// Bucket whose source rows may span several ELL rows, or whose rows are too wide to stage: the first ELL row of a
+// segment owns it, a wavefront sums all of its slots, every sub-wave its share; continuation rows and segments
+// above coop_slots (handled as chunks) are skipped.
+template <int LPR, int CH, typename BT, bool WIDE>
+__device__ __forceinline__ void run_seg_tile(const RowsOfB<LPR, CH, BT, WIDE>& b, const Group& g, long long tile, const LaunchArgs& a) {
     constexpr int VEC = Dense<BT>::kVec;
-    constexpr int SW = kWG / LPR;
-    const int tid = threadIdx.x;
-    const int sw = tid / LPR, sl = tid % LPR;
-    const Lane<LPR, CH, VEC> ln(sl, a.feat, a.ldb, a.ldc);
+    const int lane = threadIdx.x & 63;
+    const Lane<LPR, CH, VEC> ln(lane % LPR, a.feat, a.ldb, a.ldc);
+    const Teams<LPR, CH, BT, WIDE> team(b, Teams<LPR, CH, BT, WIDE>::kLgSubs);
     const long long e0 = tile * g.rows_per_tile;
     const int n = (int)min((long long)g.rows_per_tile, g.n_items - e0);
-    for (int r = sw; r < n; r += SW) {
+    for (int r = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6); r < n; r += kWG / 64) {
         const long long e = e0 + r;
         const int m = g.meta[e];
         if (m < 0) continue;                                   // continuation row
@@ -369,8 +326,9 @@ __device__ __forceinline__ void run_seg_tile(const Group& g, long long tile, con
         if (seg > 1) total = ((seg - 1) << g.log_w) + (g.meta[e + seg - 1] & kMetaLenMask);
         Acc<CH, VEC> acc;
         acc.clear();
-        stream_slots<LPR, CH, BT>(g.cols, g.vals, e << g.log_w, total, a.B, ln, acc);
-        store_row<LPR, CH, VEC>(a.C, g.rows[e], ln, acc, a.accumulate);
+        team.sum(g.cols, g.vals, e << g.log_w, total, total, acc);
+        team.combine(acc);
+        if (lane < LPR) store_row<LPR, CH, VEC>(a.C, g.rows[e], ln, acc, a.accumulate);
     }
 }
 
@@ -399,13 +357,18 @@ __device__ __forceinline__ void load_pair_agent(const float* src, float& x, floa
     y = __uint_as_float((unsigned int)(v >> 32));
 }
 
+// Rows of a streamed tile: two to a wavefront.  A sub-wave per row, the form before, was a chain of up to 32 batches
+// for a row of 256 slots; a wavefront at N = 32 takes 4.  Log-normal rows, us, before -> now: 16000 x 128, N = 32
+// 25.5 -> 18.5, N = 64 35.3 -> 27.9; 32000 x 32, N = 32 16.7 -> 12.1.  (32 rows to a tile, as with sub-waves: 38.8, 38.6,
+// 27.6; 4 to a tile: within 3 % either way.)
+constexpr int kSegRows = 8;
 constexpr int kSlice = 8;
 constexpr int kSlicedSlots = 128;
 
-// One chunk of a heavy source row: the workgroup's sub-waves take consecutive slices of
-// the chunk, their sums are combined through LDS in sub-wave order.
-template <int LPR, int CH, typename BT>
-__device__ __forceinline__ void run_chunk_tile(const Group& g, long long tile, float* s_red,
+// One chunk of a heavy source row: the workgroup's wavefronts take consecutive parts of the chunk, a part's
+// slots are spread over the wavefront's sub-waves, the sums are combined through LDS in wavefront order.
+template <int LPR, int CH, typename BT, bool WIDE>
+__device__ __forceinline__ void run_chunk_tile(const RowsOfB<LPR, CH, BT, WIDE>& b, const Group& g, long long tile, float* s_red,
                                                const LaunchArgs& a) {
     constexpr int VEC = Dense<BT>::kVec;
     constexpr int SW = kWG / LPR;
@@ -413,10 +376,6 @@ __device__ __forceinline__ void run_chunk_tile(const Group& g, long long tile, f
     const int sw = tid / LPR, sl = tid % LPR;
     const Lane<LPR, CH, VEC> ln(sl, a.feat, a.ldb, a.ldc);
     const Chunk ck = g.chunks[tile];
-    constexpr int kPart = kUnroll < LPR ? kUnroll : LPR;
-    const int per = ((ck.n_slots + SW - 1) / SW + kPart - 1) / kPart * kPart;
-    const int lo = min(sw * per, ck.n_slots);
-    const int hi = min(lo + per, ck.n_slots);
     Acc<CH, VEC> acc;
     acc.clear();
     if (ck.partial < 0 && ck.n_slots <= kSlicedSlots) {
@@ -427,7 +386,7 @@ __device__ __forceinline__ void run_chunk_tile(const Group& g, long long tile, f
         for (int s0 = 0; s0 * kSlice < ck.n_slots; s0 += SW) {
             const int at = (s0 + sw) * kSlice;
             acc.clear();
-            stream_slots<LPR, CH, BT>(g.cols, g.vals, ck.slot_begin + at, min(kSlice, ck.n_slots - at), a.B, ln, acc);
+            Teams<LPR, CH, BT, WIDE>(b, 0).sum(g.cols, g.vals, ck.slot_begin + at, min(kSlice, ck.n_slots - at), kSlice, acc);
             if (s0 > 0) __syncthreads();             // the slices before have been read
 #pragma unroll
             for (int c = 0; c < CH; ++c)
@@ -444,21 +403,29 @@ __device__ __forceinline__ void run_chunk_tile(const Group& g, long long tile, f
         if (sw == 0) store_row<LPR, CH, VEC>(a.C, ck.row, ln, sum, a.accumulate);
         return;
     }
-    stream_slots<LPR, CH, BT>(g.cols, g.vals, ck.slot_begin + lo, hi - lo, a.B, ln, acc);
-    // s_red[sw][c][sl][i]
+    constexpr int kWaves = kWG / 64, kStep = Teams<LPR, CH, BT, WIDE>::kBatch << Teams<LPR, CH, BT, WIDE>::kLgSubs;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int per = ((ck.n_slots + kWaves - 1) / kWaves + kStep - 1) / kStep * kStep;
+    const int lo = min(wave * per, ck.n_slots), part = min(per, ck.n_slots - lo);
+    const Teams<LPR, CH, BT, WIDE> team(b, Teams<LPR, CH, BT, WIDE>::kLgSubs);
+    team.sum(g.cols, g.vals, ck.slot_begin + lo, part, part, acc);
+    team.combine(acc);
+    // s_red[wave][c][sl][i]
+    if ((tid & 63) < LPR) {
 #pragma unroll
-    for (int c = 0; c < CH; ++c)
+        for (int c = 0; c < CH; ++c)
 #pragma unroll
-        for (int i = 0; i < VEC; ++i) s_red[((sw * CH + c) * LPR + sl) * VEC + i] = acc.v[c][i];
+            for (int i = 0; i < VEC; ++i) s_red[((wave * CH + c) * LPR + sl) * VEC + i] = acc.v[c][i];
+    }
     __syncthreads();
     if (tid >= 64) return;
     acc.clear();
     if (sw == 0) {
 #pragma unroll
         for (int c = 0; c < CH; ++c)
-            for (int s = 0; s < SW; ++s)
+            for (int w = 0; w < kWaves; ++w)
 #pragma unroll
-                for (int i = 0; i < VEC; ++i) acc.v[c][i] += s_red[((s * CH + c) * LPR + sl) * VEC + i];
+                for (int i = 0; i < VEC; ++i) acc.v[c][i] += s_red[((w * CH + c) * LPR + sl) * VEC + i];
     }
     if (ck.partial < 0) {                            // the row's only chunk
         if (sw == 0) store_row<LPR, CH, VEC>(a.C, ck.row, ln, acc, a.accumulate);
@@ -532,21 +499,36 @@ __device__ __forceinline__ void run_chunk_tile(const Group& g, long long tile, f
 // grid that strides over the tiles measured 2-7 % slower on every workload.
 //
 // RESIDENT: the partition's part of B stays in the XCD's L2.  Gathers that hit are short, so what counts is how many
-// wavefronts are there to issue them: registers are held to 7 wavefronts per SIMD (bf16 6, two chunks
-// per lane 4), and a tile of a float product holds twice the slots, since the wait for a tile's
-// slots is a larger part of it.  132K-row graph, 300 entries a row, 16 partitions, N = 96: 1186 -> 1046
-// us (occupancy alone 1100, tiles alone 1096); 90K rows, 8 partitions, N = 192 862 -> 767; 22K rows of
-// 91, 8 partitions, N = 288 363 -> 327.  Where gathers miss, more of them in flight gain nothing and
-// bf16 pays for the spills (500k x 2M matrix 1.32 -> 1.39 ms).  Eight lanes per row spend more on
-// their addresses than on waiting and take the occupancy everywhere (25K rows of 320, N = 32: 90 -> 75).
+// wavefronts are there to issue them: registers are held to 6 wavefronts per SIMD (two chunks per lane 4), and a tile
+// of a float product holds twice the slots, since the wait for a tile's slots is a larger part of it.  132K-row graph,
+// 300 entries a row, 16 partitions, N = 96, with the kernels of its time: 1186 -> 1046 us (occupancy alone 1100, tiles
+// alone 1096); 1023 now.  (The loops over a row's slots are not unrolled beyond one batch of gathers: two batches in
+// flight spilled here, 1497 us, and elsewhere cost a wavefront per SIMD.)  Where gathers miss, more of them in flight
+// gain nothing and bf16 pays for the spills (500k x 2M matrix 1.32 -> 1.39 ms).
 constexpr int partition_min_waves(int lpr, int ch, bool bf16, bool resident) {
     if (ch != 1) return resident ? 4 : 1;
-    if (!bf16) return lpr == 8 ? 6 : resident ? 7 : 1;
+    if (!bf16) return lpr == 8 || resident ? 6 : 1;
     return resident ? 6 : 1;
 }
 constexpr bool has_resident_kernel(int lpr, int ch, bool bf16) { return bf16 ? ch == 1 : ch <= 2 && lpr > 8; }
 
-template <int LPR, int CH, typename BT, bool RESIDENT>
+__device__ __forceinline__ Group load_group(const __attribute__((address_space(4))) Group* from) {
+    Group g;
+    g.type = from->type;
+    g.log_w = from->log_w;
+    g.rows_per_tile = from->rows_per_tile;
+    g.balanced = from->balanced;
+    g.n_items = from->n_items;
+    g.n_tiles = from->n_tiles;
+    g.rows = from->rows;
+    g.meta = from->meta;
+    g.cols = from->cols;
+    g.vals = from->vals;
+    g.chunks = from->chunks;
+    return g;
+}
+
+template <int LPR, int CH, typename BT, bool RESIDENT, bool WIDE>
 __global__ void __launch_bounds__(kWG, partition_min_waves(LPR, CH, Dense<BT>::kVec == 8, RESIDENT))
 spmm_partition_kernel(LaunchArgs a) {
     // one LDS buffer, used either as the staged tile ((col, val) pairs then (row, meta)
@@ -560,37 +542,60 @@ spmm_partition_kernel(LaunchArgs a) {
     __shared__ int s_next;                     // next ELL row of a tile whose rows are taken dynamically
     extern __shared__ __align__(16) float s_dyn[];   // per-ELL-row sums of a balanced segment tile
 
-    // position in this XCD's tile list -> group and tile.  The groups' tile counts come with the
-    // arguments: reading the groups one after the other took a round trip to memory each.
+    // Position in this XCD's tile list -> group and tile.  The groups' tile counts come with the
+    // arguments: reading the groups one after the other took a round trip to memory each.  The group itself is read
+    // whole, by scalar loads (through the constant address space: nothing writes it while the launch runs): field by
+    // field, where it is used, each read was a round trip of its own.
     const int xcd = blockIdx.x % kXcds;
-    long long v = blockIdx.x / kXcds;
-    auto in_group = [&](long long n_tiles) {
-        const long long lo = n_tiles * xcd / kXcds, n = n_tiles * (xcd + 1) / kXcds - lo;
-        if (v < n) {
-            v += lo;
-            return true;
-        }
-        v -= n;
-        return false;
+    const int slice = xcd & ((1 << a.lg_slices) - 1), rank = xcd >> a.lg_slices, lg_ranks = kLgXcds - a.lg_slices;
+    const size_t skip = (size_t)slice * a.feat;
+    a.C += skip;
+    a.partials += (size_t)slice * a.slice_partials;
+    a.heavy += (size_t)slice * a.slice_heavy;
+    using ConstGroup = const __attribute__((address_space(4))) Group;
+    ConstGroup* groups = (ConstGroup*)(uintptr_t)a.groups;
+    int v = blockIdx.x / kXcds;
+    // the XCD's share of n_tiles tiles: [first, first + count)
+    auto share = [&](int n_tiles, int& first) {
+        const int whole = n_tiles >> lg_ranks, rest = n_tiles & ((1 << lg_ranks) - 1);
+        first = whole * rank + (rest * rank >> lg_ranks);
+        return whole * (rank + 1) + (rest * (rank + 1) >> lg_ranks) - first;
     };
-    int gi = 0;
-    bool found = false;
+    // a group to a lane, the shares' prefix sums by DPP, the group from one ballot: group by group the walk to the
+    // last of eleven was 300 scalar instructions
+    int n_tiles = 0, first;
 #pragma unroll
-    for (int i = 0; i < kInlineGroups; ++i) {
-        if (found || i >= a.n_groups) break;
-        found = in_group(a.n_tiles[i]);
-        if (!found) ++gi;
+    for (int i = 0; i < kInlineGroups; ++i) n_tiles = (int)(threadIdx.x & 63) == i ? a.n_tiles[i] : n_tiles;
+    const int count = share(n_tiles, first);
+    int until = count;
+    until += __builtin_amdgcn_update_dpp(0, until, 0x111, 0xF, 0xF, true);       // row_shr:1, 2, 4, 8
+    until += __builtin_amdgcn_update_dpp(0, until, 0x112, 0xF, 0xF, true);
+    until += __builtin_amdgcn_update_dpp(0, until, 0x114, 0xF, 0xF, true);
+    until += __builtin_amdgcn_update_dpp(0, until, 0x118, 0xF, 0xF, true);
+    const int behind = (int)(__ballot(v < until) & ((1ull << kInlineGroups) - 1));
+    int gi;
+    if (behind) {
+        gi = __builtin_ctz(behind);
+        v += __builtin_amdgcn_readlane(first - (until - count), gi);
+    } else {
+        v -= __builtin_amdgcn_readlane(until, kInlineGroups - 1);
+        for (gi = kInlineGroups; gi < a.n_groups; ++gi) {
+            const int n = share((int)groups[gi].n_tiles, first);
+            if (v < n) break;
+            v -= n;
+        }
+        if (gi >= a.n_groups) return;
+        v += first;
     }
-    for (; !found && gi < a.n_groups; ++gi)
-        if ((found = in_group(a.groups[gi].n_tiles))) break;
-    if (!found) return;
-    const Group& g = a.groups[gi];             // uniform address: scalar loads
+    const Group g = load_group(groups + gi);
+    const RowsOfB<LPR, CH, BT, WIDE> b((const char*)a.B + skip * Dense<BT>::kElemBytes, a.b_bytes - skip * Dense<BT>::kElemBytes,
+                                       Lane<LPR, CH, Dense<BT>::kVec>(threadIdx.x % LPR, a.feat, a.ldb, a.ldc));
     switch (g.type) {
         case kEll:
-        case kEllSeg: run_ell_tile<LPR, CH, BT>(g, v, s_pairs, s_rm, &s_next, s_dyn, a); break;
-        case kSeg: run_seg_tile<LPR, CH, BT>(g, v, a); break;
+        case kEllSeg: run_ell_tile(b, g, v, s_pairs, s_rm, &s_next, s_dyn, a); break;
+        case kSeg: run_seg_tile(b, g, v, a); break;
         case kZero: run_zero_tile<LPR, CH, BT>(g, v, a); break;
-        default: run_chunk_tile<LPR, CH, BT>(g, v, reinterpret_cast<float*>(s_raw), a); break;
+        default: run_chunk_tile(b, g, v, reinterpret_cast<float*>(s_raw), a); break;
     }
 }
 
@@ -608,6 +613,8 @@ spmm_finalize_wide_kernel(const HeavyRow* __restrict__ heavy, int n_heavy, Launc
     const Lane<LPR, CH, VEC> ln(sl, a.feat, a.ldb, a.ldc);
     const int h = blockIdx.x;
     if (h >= n_heavy) return;
+    a.C += (size_t)blockIdx.y * a.feat;                     // the feature slice
+    a.partials += (size_t)blockIdx.y * a.slice_partials;
     const HeavyRow hr = heavy[h];
     if (hr.n_partials <= kWideFinalPartials) return;
     Acc<CH, VEC> acc;
@@ -1196,7 +1203,7 @@ __global__ void __launch_bounds__(256)
 plan_chunks_kernel(const int32_t* __restrict__ rows, const int32_t* __restrict__ meta,
                    const int32_t* __restrict__ cols, long long n_rows, int log_w, int* __restrict__ counters,
                    Chunk* __restrict__ chunks, HeavyRow* __restrict__ heavy,
-                   int partial_base, int heavy_base, int coop_slots, int chunk_slots, long long dense_min_slots) {
+                   int partial_base, int heavy_base, int n_heavy, int slices, int coop_slots, int chunk_slots, long long dense_min_slots) {
     __shared__ int s_sum[4][3];
     __shared__ int s_base[3];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -1259,7 +1266,8 @@ plan_chunks_kernel(const int32_t* __restrict__ rows, const int32_t* __restrict__
             ck.pad_ = 0;
             chunks[c0 + i] = ck;
         }
-        if (several) heavy[heavy_base + h] = HeavyRow{row, partial_base + p0, x.n_chunks, 0};
+        for (int i = 0; i < slices && several; ++i)          // every feature slice counts its chunks
+            heavy[(size_t)i * n_heavy + heavy_base + h] = HeavyRow{row, partial_base + p0, x.n_chunks, 0};
     }
 }
 
@@ -1313,7 +1321,8 @@ struct lf_spmm_plan {
     int feat = 0, b_dtype = 0, num_parts = 0;
     int64_t num_rows = 0, num_cols = 0;
     int lpr = 0, ch = 0;
-    int windows = 1;                 // feature windows of `feat` features each that a run covers
+    int slices = 1;                  // feature slices of `feat` features that the XCDs share out within a launch
+    int windows = 1;                 // feature windows of slices * feat features each that a run covers
     int device = 0, num_cus = 0, grid = 0;
     struct Launch {
         int group_begin = 0, n_groups = 0, grid = 0;
@@ -1335,8 +1344,10 @@ struct lf_spmm_plan {
     std::vector<void*> owned;        // device allocations released by destroy
     std::vector<void*> temp;         // plan-time scratch, released when lf_spmm_create returns
     Group* d_groups = nullptr;
-    HeavyRow* d_heavy = nullptr;
-    float* d_partials = nullptr;
+    HeavyRow* d_heavy = nullptr;        // [slices][n_heavy]
+    float* d_partials = nullptr;        // [slices][partial rows][feat]
+    int n_heavy = 0;
+    long long slice_partials = 0;
     // d_partials and HeavyRow::done are written by every run; see order_behind_last_run
     hipEvent_t order_event = nullptr;    // made when a second stream appears
     hipStream_t last_stream = nullptr;
@@ -1374,6 +1385,7 @@ using RowGroupFn = void (*)(const MergedBucket*, int, LaunchArgs);
 struct KernelSet {
     KernelFn tiles = nullptr;
     KernelFn tiles_resident = nullptr;   // the same where there is no such kernel
+    KernelFn tiles_wide = nullptr;       // B past what 32-bit keys reach; its LDS holds the tiles of either
     FinalFn finalize_wide = nullptr;
     RowGroupFn rowgroup = nullptr;   // one 16-byte chunk per lane only
 };
@@ -1384,12 +1396,14 @@ template <int LPR, int CH> void pick_kernels(int dtype, KernelSet* k) {
         else k->rowgroup = spmm_rowgroup_kernel<LPR, float>;
     }
     if (dtype == LF_DTYPE_BF16) {
-        k->tiles = spmm_partition_kernel<LPR, CH, bf16_t, false>;
-        k->tiles_resident = spmm_partition_kernel<LPR, CH, bf16_t, has_resident_kernel(LPR, CH, true)>;
+        k->tiles = spmm_partition_kernel<LPR, CH, bf16_t, false, false>;
+        k->tiles_resident = spmm_partition_kernel<LPR, CH, bf16_t, has_resident_kernel(LPR, CH, true), false>;
+        k->tiles_wide = spmm_partition_kernel<LPR, CH, bf16_t, has_resident_kernel(LPR, CH, true), true>;
         k->finalize_wide = spmm_finalize_wide_kernel<LPR, CH, bf16_t>;
     } else {
-        k->tiles = spmm_partition_kernel<LPR, CH, float, false>;
-        k->tiles_resident = spmm_partition_kernel<LPR, CH, float, has_resident_kernel(LPR, CH, false)>;
+        k->tiles = spmm_partition_kernel<LPR, CH, float, false, false>;
+        k->tiles_resident = spmm_partition_kernel<LPR, CH, float, has_resident_kernel(LPR, CH, false), false>;
+        k->tiles_wide = spmm_partition_kernel<LPR, CH, float, has_resident_kernel(LPR, CH, false), true>;
         k->finalize_wide = spmm_finalize_wide_kernel<LPR, CH, float>;
     }
 }
@@ -1439,7 +1453,6 @@ int lf_spmm_create(lf_spmm_plan** out_plan, const lf_bucket_desc* h_buckets, int
     LF_REQUIRE(b_dtype == LF_DTYPE_F32 || b_dtype == LF_DTYPE_BF16, LF_ERR_INVALID, "unknown B dtype %d", b_dtype);
     int lpr, ch;
     if (int rc = feature_shape(feat_size, b_dtype, &lpr, &ch)) return rc;
-    const int sw = kWG / lpr;
     for (int k = 0; k < num_buckets; ++k) {
         const lf_bucket_desc& b = h_buckets[k];
         LF_REQUIRE(lf::is_pow2(b.width) && b.width <= 1024, LF_ERR_INVALID, "bucket %d: width %d", k, b.width);
@@ -1517,19 +1530,6 @@ int lf_spmm_create(lf_spmm_plan** out_plan, const lf_bucket_desc* h_buckets, int
     // 500k x 2M matrix 1.457 -> 1.443); those of a small one are worth keeping between products
     // (170k-row graph, 6 MB of slabs: 0.073 ms cached, 0.076 ms streamed).
     plan->stream_slabs = total_slots >= kLargeMatrixSlots;
-    // Parts of B that an L2 (4 MB) about holds, and for float products rows that are mostly staged (those of
-    // hundreds of slots per partition stream them by shuffle: 5774 rows of 368 in two partitions, N = 288
-    // 145 -> 149 us).  A single float partition is not latency-bound enough (10K and 20K rows, 2.4 to 22 MB: -2 to
-    // + 4 %); a bf16 one is up to 32 lanes per row (10K rows of 182, N = 128: 38.4 -> 36.5 us).  Where the line
-    // loses: the same 5774 rows at N = 64 .. 128 would gain 18 - 23 % (53.6 -> 43.6 us), a bf16 B of 4.9 MB in
-    // one partition 3 %; two partitions of 12K rows of 60 entries lose 1 - 7 % with it (N = 192: 42.7 -> 45.8).
-    {
-        const bool bf16 = b_dtype == LF_DTYPE_BF16;
-        const long long part_bytes = lf::ceil_div(num_cols, (int64_t)num_parts) * feat_size * (bf16 ? 2 : 4);
-        plan->resident = has_resident_kernel(lpr, ch, bf16) &&
-                         part_bytes <= (num_parts > 1 ? 2 * kL2XcdBytes : bf16 && lpr <= 32 ? kL2XcdBytes : 0) &&
-                         (bf16 || total_slots <= 96 * num_rows * num_parts);
-    }
     const char* env_dense = getenv("LF_DENSE_ROWS");       // "0": dense rows are chunked like the other long rows
     // (where the memory-side cache holds the partition's part of B anyway there is nothing to order)
     const long long cols_p = lf::ceil_div(num_cols, num_parts);
@@ -1640,6 +1640,50 @@ int lf_spmm_create(lf_spmm_plan** out_plan, const lf_bucket_desc* h_buckets, int
                                                         "or a segment that is incomplete or leaves the bucket)"));
         if (f[3]) return bail(lf::fail(LF_ERR_UNSUPPORTED, "a row is split over more than %d ELL rows", (1 << (31 - kMetaLenBits)) - 1));
     }
+    const int n_zero = *back.as<int>(o_zero);
+    std::vector<int> chosen;                               // candidates whose sample shows shared columns
+    for (int k : cand) {
+        const unsigned long long* c = back.as<unsigned long long>(o_sample) + 3 * k;
+        if (!is_multi[k] && c[1] > 0 && c[0] * 100 <= c[1] * kRowGroupMaxPercent) chosen.push_back(k);
+    }
+
+    auto scanned = [&](int k, int i) { return h_counters[((size_t)kScanCounters * k + i) * kCounterLine]; };
+
+    // ---- Feature slices; matrices whose kernels share gathers between rows read B through the L2s as it is.
+    // A doubling of S costs 0.8 us in rows' starts and ends, and sub-waves of fewer lanes are more of them to share a
+    // long row's chunk, whose chain of gathers (0.11 us a step; it overlaps with other work) sets the time of small
+    // power-law products.  1500 matrices of 2K to 1M rows, log-normal and power-law, N = 32 .. 512, f32 and bf16, every
+    // S timed at the shape that predict_launch_shape gives: 0.93 of the time with S = 1 on average (0.4 at best: 64000
+    // rows of 32 entries, N = 256 287 -> 213 us; 16000 56 -> 30), 3 % of them more than 3 % slower, 16 % at worst.
+    if (chosen.empty()) {
+        const int vec = b_dtype == LF_DTYPE_BF16 ? 8 : 4;
+        bool chains = false;                               // rows of several chunks
+        for (int k = 0; k < num_buckets; ++k) chains = chains || scanned(k, 1) > 0;
+        plan->slices = feature_slices(lf::ceil_div(num_cols, (int64_t)num_parts), total_slots / num_parts, feat_size, b_dtype,
+                                      [&](int n, double us) {
+            const int lanes = std::min(64, std::max(8, feat_size / n / vec));
+            const double steps = (double)chunk_slots * lanes / (kWG * kUnroll);
+            return us + 0.8 * lf::ilog2(n) + (chains ? 0.11 * steps : 0.0);
+        });
+        plan->feat = feat_size /= plan->slices;
+        LF_TRY(feature_shape(feat_size, b_dtype, &lpr, &ch));
+        plan->lpr = lpr;
+        plan->ch = ch;
+    }
+    const int sw = kWG / lpr;
+    // Parts of B that an L2 (4 MB) about holds, and for float products rows that are mostly staged (those of
+    // hundreds of slots per partition are streamed: 5774 rows of 368 in two partitions, N = 288
+    // 145 -> 149 us).  A single float partition is not latency-bound enough (10K and 20K rows, 2.4 to 22 MB: -2 to
+    // + 4 %); a bf16 one is up to 32 lanes per row (10K rows of 182, N = 128: 38.4 -> 36.5 us).  Where the line
+    // loses: the same 5774 rows at N = 64 .. 128 would gain 18 - 23 % (53.6 -> 43.6 us), a bf16 B of 4.9 MB in
+    // one partition 3 %; two partitions of 12K rows of 60 entries lose 1 - 7 % with it (N = 192: 42.7 -> 45.8).
+    {
+        const bool bf16 = b_dtype == LF_DTYPE_BF16;
+        const long long part_bytes = lf::ceil_div(num_cols, (int64_t)num_parts) * feat_size * (bf16 ? 2 : 4);
+        plan->resident = has_resident_kernel(lpr, ch, bf16) &&
+                         part_bytes <= (num_parts > 1 ? 2 * kL2XcdBytes : bf16 && lpr <= 32 ? kL2XcdBytes : 0) &&
+                         (bf16 || total_slots <= 96 * num_rows * num_parts);
+    }
     // A sub-wave sums kUnroll slots of its row per round trip to B, so a row of kCoopSlots is a
     // chain of 32; where a product (all partitions together) holds few rows of more than 64 slots - a few
     // workgroups per CU - they set its length, and whole workgroups take them too: 56K-row power-law graph, bf16,
@@ -1655,7 +1699,6 @@ int lf_spmm_create(lf_spmm_plan** out_plan, const lf_bucket_desc* h_buckets, int
     // (Counted by the widths of the buckets, a folded format had none, and every such row became a chunk:
     // 2.45M-row graph, widths 1 .. 32, 302K chunks instead of 20K, N = 32 1.86 -> 1.60 ms now, N = 128 7.03 -> 6.84;
     // 132K rows of 300 entries, widths 1 .. 32 in four partitions, N = 32 0.998 -> 0.450.)
-    auto scanned = [&](int k, int i) { return h_counters[((size_t)kScanCounters * k + i) * kCounterLine]; };
     long long over64 = 0, over128 = 0;
     for (int k = 0; k < num_buckets; ++k) {
         over64 += (long long)scanned(k, 3) + scanned(k, 4);
@@ -1674,13 +1717,6 @@ int lf_spmm_create(lf_spmm_plan** out_plan, const lf_bucket_desc* h_buckets, int
         has_dense[k] = (found >> 1) & 1;
         has_wide[k] = (found >> 2) & 1;
     }
-    const int n_zero = *back.as<int>(o_zero);
-    std::vector<int> chosen;                               // candidates whose sample shows shared columns
-    for (int k : cand) {
-        const unsigned long long* c = back.as<unsigned long long>(o_sample) + 3 * k;
-        if (!is_multi[k] && c[1] > 0 && c[0] * 100 <= c[1] * kRowGroupMaxPercent) chosen.push_back(k);
-    }
-
     // ---- chunk tables, heavy-row table (grouped by bucket, hence by partition) and partial rows
     std::vector<Chunk*> d_chunks((size_t)num_buckets, nullptr);
     std::vector<int> heavy_base((size_t)num_buckets + 1, 0), partial_base((size_t)num_buckets + 1, 0);
@@ -1693,8 +1729,10 @@ int lf_spmm_create(lf_spmm_plan** out_plan, const lf_bucket_desc* h_buckets, int
     const int n_heavy_total = heavy_base[num_buckets];
     const int n_partials = partial_base[num_buckets];
     if (n_heavy_total > 0) {
-        LF_TRY(dev_alloc(plan, &plan->d_heavy, (size_t)n_heavy_total));
-        LF_TRY(dev_alloc(plan, &plan->d_partials, (size_t)n_partials * feat_size));
+        plan->n_heavy = n_heavy_total;
+        plan->slice_partials = (long long)n_partials * feat_size;
+        LF_TRY(dev_alloc(plan, &plan->d_heavy, (size_t)n_heavy_total * plan->slices));
+        LF_TRY(dev_alloc(plan, &plan->d_partials, (size_t)plan->slice_partials * plan->slices));
     }
     Chunk* d_chunks_all = nullptr;
     LF_TRY(dev_alloc(plan, &d_chunks_all, (size_t)chunk_base[num_buckets]));
@@ -1704,7 +1742,7 @@ int lf_spmm_create(lf_spmm_plan** out_plan, const lf_bucket_desc* h_buckets, int
         d_chunks[k] = d_chunks_all + chunk_base[k];
         const int grid = (int)std::min<long long>((b.num_ell_rows + 255) / 256, kPlanChunksGrid);
         plan_chunks_kernel<<<grid, 256, 0, s>>>(b.d_rows, meta[k], b.d_cols, b.num_ell_rows, lf::ilog2(b.width), d_cursors + (size_t)3 * k * kCounterLine,
-                                                d_chunks[k], plan->d_heavy, partial_base[k], heavy_base[k], plan->coop_slots,
+                                                d_chunks[k], plan->d_heavy, partial_base[k], heavy_base[k], n_heavy_total, plan->slices, plan->coop_slots,
                                                 chunk_slots, dense_min_slots);
         LF_TRY_HIP(hipGetLastError());
     }
@@ -1862,7 +1900,7 @@ int lf_spmm_create(lf_spmm_plan** out_plan, const lf_bucket_desc* h_buckets, int
             rows_all += h_buckets[k].num_ell_rows;
             if (h_buckets[k].width >= kStreamMinWidth) rows_wide += h_buckets[k].num_ell_rows;
         }
-        const bool c_fits_l2 = (long long)num_rows * feat_size * 4 <= kL2Bytes;
+        const bool c_fits_l2 = (long long)num_rows * feat_size * plan->slices * 4 <= kL2Bytes;
         L.stream_c = rows_wide * 2 >= rows_all || (b_dtype == LF_DTYPE_F32 && !c_fits_l2);
         for (int k : mine) L.wide_rows = L.wide_rows || has_wide[k];
         L.heavy_begin = mine.empty() ? 0 : heavy_base[mine.front()];
@@ -1889,7 +1927,7 @@ int lf_spmm_create(lf_spmm_plan** out_plan, const lf_bucket_desc* h_buckets, int
             const int fit = tile_slots(lpr, plan->resident && b_dtype == LF_DTYPE_F32) >> g.log_w;   // ELL rows whose slots fit the LDS tile
             const bool staged = fit >= sw;
             g.type = staged ? (is_multi[k] ? kEllSeg : kEll) : kSeg;
-            g.rows_per_tile = staged ? std::min(kTileRows, fit) : std::max(sw, fit);
+            g.rows_per_tile = staged ? std::min(kTileRows, fit) : kSegRows;
             if (staged) {
                 // a small bucket is cut into more, shorter tiles so that it still spreads over
                 // the CUs: at least one pass of every sub-wave (8 rows at a time in the
@@ -1917,7 +1955,8 @@ int lf_spmm_create(lf_spmm_plan** out_plan, const lf_bucket_desc* h_buckets, int
         if (p == 0 && n_zero > 0) {
             Group g{};
             g.type = kZero;
-            g.rows_per_tile = 1024;
+            // (4096 rows, 1500 of them empty, N = 128: tiles of 1024 32 us, so 6)
+            g.rows_per_tile = (int)std::min<long long>(1024, std::max<long long>(4 * sw, lf::ceil_div(n_zero, (long long)4 * plan->num_cus)));
             g.n_items = n_zero;
             g.n_tiles = lf::ceil_div(g.n_items, g.rows_per_tile);
             g.rows = d_zero_rows;
@@ -1958,12 +1997,13 @@ int lf_spmm_create(lf_spmm_plan** out_plan, const lf_bucket_desc* h_buckets, int
             if (longest_m * kXcds >= (1ll << 31)) return bail(lf::fail(LF_ERR_UNSUPPORTED, "too many row-group tiles"));
             L.merged_grid = (int)(longest_m * kXcds);
         }
-        // grid: 8 x the longest per-XCD tile list
+        // grid: 8 x the longest per-XCD tile list; the XCDs of a feature slice share out all tiles
         long long longest = 0;
-        for (int x = 0; x < kXcds; ++x) {
+        const int ranks = kXcds / plan->slices;
+        for (int x = 0; x < ranks; ++x) {
             long long len = 0;
             for (int gi = L.group_begin; gi < (int)groups.size(); ++gi)
-                len += groups[gi].n_tiles * (x + 1) / kXcds - groups[gi].n_tiles * x / kXcds;
+                len += groups[gi].n_tiles * (x + 1) / ranks - groups[gi].n_tiles * x / ranks;
             longest = std::max(longest, len);
         }
         for (int gi = L.group_begin; gi < (int)groups.size(); ++gi) {
@@ -2090,7 +2130,9 @@ int lf_spmm_run(lf_spmm_plan* plan, const void* d_B, float* d_C, lf_stream_t str
     if (int rc = order_behind_last_run(plan, s)) return rc;
     // One pass per feature window (all partitions inside), each on its own columns of B and C.
     const size_t b_elem = plan->b_dtype == LF_DTYPE_BF16 ? 2 : 4;
-    const int ld = plan->feat * plan->windows;
+    const int window = plan->feat * plan->slices, ld = window * plan->windows;
+    const unsigned long long b_bytes = (unsigned long long)plan->num_cols * ld * b_elem;
+    const KernelFn tiles = b_bytes > kPastB ? ks.tiles_wide : plan->resident ? ks.tiles_resident : ks.tiles;
     for (int w = 0; w < plan->windows; ++w) {
         for (int p = 0; p < plan->num_parts; ++p) {
             const lf_spmm_plan::Launch& L = plan->launches[p];
@@ -2102,14 +2144,18 @@ int lf_spmm_run(lf_spmm_plan* plan, const void* d_B, float* d_C, lf_stream_t str
                            (plan->stream_slabs ? kStreamSlabs : 0);
             a.feat = plan->feat;
             a.ldb = a.ldc = ld;
-            a.B = (const char*)d_B + (size_t)w * plan->feat * b_elem;
-            a.C = d_C + (size_t)w * plan->feat;
+            a.B = (const char*)d_B + (size_t)w * window * b_elem;
+            a.C = d_C + (size_t)w * window;
+            a.b_bytes = b_bytes - (size_t)w * window * b_elem;
+            a.lg_slices = lf::ilog2(plan->slices);
+            a.slice_heavy = plan->n_heavy;
+            a.slice_partials = plan->slice_partials;
             a.partials = plan->d_partials;
             a.heavy = plan->d_heavy;
             a.coop_slots = plan->coop_slots;
             std::memcpy(a.n_tiles, L.n_tiles, sizeof(a.n_tiles));
             if (L.grid > 0) {
-                (plan->resident ? ks.tiles_resident : ks.tiles)<<<L.grid, kWG, L.dyn_lds, s>>>(a);
+                tiles<<<L.grid, kWG, L.dyn_lds, s>>>(a);
                 LF_HIP(hipGetLastError());
             }
             if (L.n_merged > 0) {
@@ -2122,7 +2168,7 @@ int lf_spmm_run(lf_spmm_plan* plan, const void* d_B, float* d_C, lf_stream_t str
                     return rc;
             }
             if (L.wide_rows) {
-                ks.finalize_wide<<<L.n_heavy, kWG, 0, s>>>(plan->d_heavy + L.heavy_begin, L.n_heavy, a);
+                ks.finalize_wide<<<dim3((unsigned)L.n_heavy, (unsigned)plan->slices), kWG, 0, s>>>(plan->d_heavy + L.heavy_begin, L.n_heavy, a);
                 LF_HIP(hipGetLastError());
             }
         }
@@ -2132,7 +2178,7 @@ int lf_spmm_run(lf_spmm_plan* plan, const void* d_B, float* d_C, lf_stream_t str
 
 int lf_spmm_set_windows(lf_spmm_plan* plan, int32_t n_windows) {
     LF_REQUIRE(plan, LF_ERR_INVALID, "plan is null");
-    LF_REQUIRE(n_windows >= 1 && (int64_t)n_windows * plan->feat <= (1 << 20), LF_ERR_INVALID,
+    LF_REQUIRE(n_windows >= 1 && (int64_t)n_windows * plan->slices * plan->feat <= (1 << 20), LF_ERR_INVALID,
                "bad number of feature windows (%d)", n_windows);
     plan->windows = n_windows;
     return LF_OK;

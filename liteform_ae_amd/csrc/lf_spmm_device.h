@@ -4,7 +4,10 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
+#include <cmath>
 #include <cstdint>
+#include <utility>
 
 #include "lf_internal.h"
 
@@ -53,9 +56,10 @@ constexpr int kDenseRowMinSlots = 4096;
 constexpr long long kDenseMinBBytes = 128ll << 20;   // ... in a partition whose part of B is larger than this
 constexpr int kDenseChunkSlots = 1024;
 constexpr int kWideFinalPartials = 64;       // rows with more partial rows are added up by a kernel of their own
-constexpr int kXcds = 8;
+constexpr int kLgXcds = 3, kXcds = 1 << kLgXcds;
 constexpr int kPartBytesMax = 16384;   // LDS for per-ELL-row sums of a balanced segment tile at most
 constexpr int kUnroll = LF_UNROLL;  // B-row gathers in flight per sub-wave
+static_assert(kUnroll == 8, "a batch of 8 or 16 entries is gathered eight at a time");
 constexpr uint32_t kMetaLenMask = 0x7FFu;
 constexpr int kMetaLenBits = 11;
 
@@ -95,7 +99,7 @@ struct Group {
     const Chunk* chunks;          // kChunk
 };
 
-constexpr int kInlineGroups = 16;
+constexpr int kInlineGroups = 16;      // a row of lanes
 
 struct LaunchArgs {
     const Group* groups;
@@ -108,9 +112,13 @@ struct LaunchArgs {
     int coop_slots;               // source rows of more slab slots are reduced by whole workgroups
     const void* B;
     float* C;
+    unsigned long long b_bytes;   // from B to the end of the matrix
+    int lg_slices;                // 2^lg_slices feature slices of `feat` features: XCD x computes slice x mod 2^lg_slices
+    int slice_heavy;              // heavy rows and partial values of a slice
+    long long slice_partials;
     float* partials;
     HeavyRow* heavy;
-    int n_tiles[kInlineGroups];   // of the first groups: a workgroup finds its group without reading the others
+    int n_tiles[kInlineGroups];   // of the first groups (0: none): a workgroup finds its group without reading the others
 };
 
 // ------------------------------------------------------------------------------------
@@ -197,20 +205,142 @@ __device__ __forceinline__ void fma_dense(float v, const typename Dense<BT>::Raw
     for (int i = 0; i < Dense<BT>::kVec; ++i) acc[i] = fmaf(v, x[i], acc[i]);
 }
 
-template <int U, int LPR, int CH, typename BT>
-__device__ __forceinline__ void gather_fma(const void* B, const Lane<LPR, CH, Dense<BT>::kVec>& ln,
-                                           const int (&col)[U], const float (&val)[U],
+// Rows of B by key: the bytes to the row, from one 32-bit multiplication where the column is read.  Gathers go
+// through a buffer resource over B, so a key and the lane's own offset are one addition away from the load, and
+// kNone, past the end of B, reads zeros without touching memory: no traffic for padding, and nothing for an
+// infinite element of B to turn into NaN.  Keys have 32 bits: where B is larger (WIDE) they are columns, and loads
+// are predicated and take a 64-bit multiply-add each.
+constexpr uint32_t kPastB = 0xFFFE0000u;       // (a lane's own offset is below 2^17)
+typedef unsigned int lf_u32x4 __attribute__((ext_vector_type(4)));
+
+template <int LPR, int CH, typename BT, bool WIDE> struct RowsOfB {
+    using Raw = typename Dense<BT>::Raw;
+    static constexpr int VEC = Dense<BT>::kVec;
+    static constexpr uint32_t kNone = WIDE ? 0xFFFFFFFFu : kPastB;
+    const char* base;
+    __amdgpu_buffer_rsrc_t rsrc;
+    uint32_t pitch;                            // bytes between rows
+    uint32_t lane_at[CH];                      // the lane's own bytes in a row
+    // `bytes`: from B to the end of the matrix
+    __device__ __forceinline__ RowsOfB(const void* B, unsigned long long bytes, const Lane<LPR, CH, VEC>& ln) {
+        base = reinterpret_cast<const char*>(B);
+        pitch = (uint32_t)ln.ldb * (uint32_t)Dense<BT>::kElemBytes;
+        rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(B), 0, WIDE ? 0 : (int)(uint32_t)bytes, 0x00027000);
+#pragma unroll
+        for (int c = 0; c < CH; ++c) lane_at[c] = (uint32_t)(ln.f[c] * Dense<BT>::kElemBytes);
+    }
+    __device__ __forceinline__ uint32_t key(int col) const { return WIDE ? (uint32_t)col : (uint32_t)col * pitch; }
+    __device__ __forceinline__ Raw load(int c, uint32_t k) const {
+        Raw x{};
+        if constexpr (WIDE) {
+            if (k != kNone) x = *reinterpret_cast<const Raw*>(base + lane_at[c] + (uint64_t)k * pitch);
+        } else {
+            const lf_u32x4 raw = __builtin_amdgcn_raw_buffer_load_b128(rsrc, k + lane_at[c], 0, 0);
+            __builtin_memcpy(&x, &raw, sizeof(Raw));
+        }
+        return x;
+    }
+};
+
+template <int U, int LPR, int CH, typename BT, bool WIDE>
+__device__ __forceinline__ void gather_fma(const RowsOfB<LPR, CH, BT, WIDE>& b, const uint32_t (&key)[U], const float (&val)[U],
                                            Acc<CH, Dense<BT>::kVec>& acc) {
     typename Dense<BT>::Raw x[U][CH];
 #pragma unroll
     for (int u = 0; u < U; ++u)
 #pragma unroll
-        for (int c = 0; c < CH; ++c) x[u][c] = load_dense<BT>(B, ln, c, col[u]);
+        for (int c = 0; c < CH; ++c) x[u][c] = b.load(c, key[u]);
 #pragma unroll
     for (int u = 0; u < U; ++u)
 #pragma unroll
         for (int c = 0; c < CH; ++c) fma_dense<BT>(val[u], x[u][c], acc.v[c]);
 }
+
+// Entry I of a sub-wave's batch, from the lane that holds it, by a DPP broadcast: an operand modifier of the
+// instruction that uses it, where a shuffle is an LDS instruction and its latency.  Lanes of other sub-waves need
+// not be active.
+template <int LPR, int I> __device__ __forceinline__ int batch_entry(int x) {
+    constexpr int kRowBroadcast = 0x150;       // row_newbcast: a lane of each row of 16 to that row
+    if constexpr (LPR >= 16) {
+        return __builtin_amdgcn_update_dpp(0, x, kRowBroadcast + I, 0xF, 0xF, true);
+    } else {                                   // two sub-waves to a row of 16 lanes
+        const int first = __builtin_amdgcn_update_dpp(0, x, kRowBroadcast + I, 0xF, 0x3, false);
+        return __builtin_amdgcn_update_dpp(first, x, kRowBroadcast + 8 + I, 0xF, 0xC, false);
+    }
+}
+
+// Teams of 2^lg sub-waves of a wavefront, each on a stretch of entries (column, value) in memory: entry e goes to
+// sub-wave e mod 2^lg.
+template <int LPR, int CH, typename BT, bool WIDE> struct Teams {
+    static constexpr int VEC = Dense<BT>::kVec;
+    static constexpr int kLgSubs = LPR == 64 ? 0 : LPR == 32 ? 1 : LPR == 16 ? 2 : 3;       // log2 of a wavefront's sub-waves
+    static constexpr int kBatch = LPR < 16 ? LPR : 16;      // entries of a sub-wave fetched at a time
+    const RowsOfB<LPR, CH, BT, WIDE>& b;
+    const int lg, sub;                         // size of the team; sub-wave in its team
+    const int slot;                            // entry of a batch that the lane fetches (in every 16 lanes again)
+
+    __device__ __forceinline__ Teams(const RowsOfB<LPR, CH, BT, WIDE>& b_, int lg_)
+        : b(b_), lg(lg_), sub((int)(threadIdx.x & 63) / LPR & ((1 << lg_) - 1)), slot((int)threadIdx.x % kBatch) {}
+
+    // The lane's entry of the batch at `base` of the `len` entries from `lo` on; no column (-1) past the end.  What is
+    // made of the column waits for it: not here, where the entry is requested ahead.
+    template <typename Pos>
+    __device__ __forceinline__ void fetch(const int32_t* __restrict__ cols, const float* __restrict__ vals, Pos lo, int len,
+                                          int base, int& col, float& val) const {
+        const int e = base + (slot << lg) + sub;
+        col = -1;
+        val = 0.f;
+        if (e < len) {
+            col = cols[lo + e];
+            val = vals ? vals[lo + e] : 1.f;
+        }
+    }
+
+    template <int FIRST, size_t... I>
+    __device__ __forceinline__ void gather(uint32_t key, float val, Acc<CH, VEC>& acc, std::index_sequence<I...>) const {
+        typename Dense<BT>::Raw x[kUnroll][CH];
+        auto load = [&](int u, uint32_t k) {
+#pragma unroll
+            for (int c = 0; c < CH; ++c) x[u][c] = b.load(c, k);
+        };
+        (load(I, (uint32_t)batch_entry<LPR, FIRST + I>((int)key)), ...);
+        auto add = [&](int u, float v) {
+#pragma unroll
+            for (int c = 0; c < CH; ++c) fma_dense<BT>(v, x[u][c], acc.v[c]);
+        };
+        (add(I, __int_as_float(batch_entry<LPR, FIRST + I>(__float_as_int(val)))), ...);
+    }
+
+    // Adds the team's `len` entries (column, value; no values: ones) from `lo` on.  `most`: at least len, the same in a
+    // team; teams with different ones diverge, and before combine() all of the wavefront have to be here again.
+    template <typename Pos>
+    __device__ __forceinline__ void sum(const int32_t* __restrict__ cols, const float* __restrict__ vals, Pos lo, int len,
+                                        int most, Acc<CH, VEC>& acc) const {
+        constexpr auto kEight = std::make_index_sequence<kUnroll>();
+        int col;
+        float val;
+        fetch(cols, vals, lo, len, 0, col, val);
+        for (int base = 0; base < most;) {
+            const uint32_t k = col >= 0 ? b.key(col) : b.kNone;
+            const float v = val;
+            const int left = most - base;
+            base += kBatch << lg;
+            if (base < most) fetch(cols, vals, lo, len, base, col, val);   // ahead: a latency of its own
+            gather<0>(k, v, acc, kEight);
+            if constexpr (kBatch > kUnroll)
+                if (left > (kUnroll << lg)) gather<kUnroll>(k, v, acc, kEight);
+        }
+    }
+
+    // The team's sums, added pairwise: every lane of the team holds them afterwards.
+    __device__ __forceinline__ void combine(Acc<CH, VEC>& acc) const {
+        for (int d = LPR; d < (LPR << lg); d <<= 1)
+#pragma unroll
+            for (int c = 0; c < CH; ++c)
+#pragma unroll
+                for (int i = 0; i < VEC; ++i) acc.v[c][i] += __shfl_xor(acc.v[c][i], d);
+    }
+};
 
 // flags: LaunchArgs::accumulate.  Rows that nothing reads again in this run are stored
 // non-temporally where that leaves the caches to B (lf_spmm_create decides); rows that a later column partition adds to stay cached
@@ -337,6 +467,33 @@ inline int feature_shape(int feat, int dtype, int* lpr, int* ch) {
     *lpr = l;
     *ch = c;
     return LF_OK;
+}
+
+// Feature slices: XCD x computes slice x mod S of the features for every (8 / S)-th part of the rows, so that its L2
+// has 1 / S of B to hold instead of all of it, at the price of reading the entries S times.  A slice is
+// 128 bytes or a multiple: a gather of 64 moves the line all the same (a table in the L2s is gathered from at 28 TB/s
+// by rows of 128 bytes and more, 15.5 by rows of 64).  The S of the least price in us: gathers that hit an L2 at 27
+// TB/s, those that miss and the entries at 7.15 (misses of 128 bytes 9 % slower), the share that hits from the slice's
+// size against 5 MB and from how often an XCD uses a row of B (the first use misses); `adjust` adds what else S changes.
+template <typename Adjust>
+inline int feature_slices(int64_t num_cols, int64_t entries, int feat, int dtype, Adjust adjust) {
+    constexpr double kL2 = 5.0e6, kHitRate = 27e6, kMissRate = 7.15e6, kMiss128 = 1.09;
+    const int elem = dtype == LF_DTYPE_BF16 ? 2 : 4, step = 128 / elem;
+    const double b_bytes = (double)num_cols * feat * elem, gathered = (double)entries * feat * elem;
+    int best = 1;
+    double least = 0.0;
+    for (int s = 1; s <= kXcds && entries > 0; s *= 2) {
+        if (feat % (s * step) != 0) break;
+        const double uses = (double)entries / (double)num_cols * s / kXcds;
+        const double hit = std::min(1.0, kL2 * s / b_bytes) * std::max(0.0, 1.0 - 1.0 / uses);
+        const double miss = (1.0 - hit) / kMissRate * (feat / s == step ? kMiss128 : 1.0);
+        const double price = adjust(s, gathered * (hit / kHitRate + miss) + 8.0 * (double)entries * s / kMissRate);
+        if (s == 1 || price < least) {
+            least = price;
+            best = s;
+        }
+    }
+    return best;
 }
 
 }  // namespace

@@ -464,3 +464,63 @@ def test_rows_sharing_columns_are_served_in_groups(fa, torch, feat, b_dtype, mon
     g = skewed_matrix(rng, 20000, 30000, mean_deg=20, heavy_rows=0)
     _, info = check(fa, torch, g, [[8, 16, 32, 64]], feat, b_dtype, seed=feat)
     assert info["row_group_buckets"] == 0
+
+
+def sliced_matrix(rng, nr, nc):
+    """Rows of every kind that a plan treats in its own way, in mixed order: empty, 1..64 entries, 65..256 in such
+    numbers that wavefronts take them (more than 1024 above 64 entries, more than 2048 above 128), and a few
+    of one chunk and of several."""
+    deg = np.concatenate([np.zeros(40, np.int64), rng.integers(1, 65, size=nr - 3300), rng.integers(65, 129, size=1050),
+                          rng.integers(129, 257, size=2200), [257, 512, 600, 1500, 2000, 2900, 2999, 3000, 300, 400]])
+    deg = rng.permutation(np.minimum(deg, nc))
+    row = np.repeat(np.arange(len(deg)), deg)
+    col = (rng.integers(nc, size=len(deg))[row] + 13 * (np.arange(len(row)) - (np.cumsum(deg) - deg)[row])) % nc
+    return MTX.from_coo(row, col, (len(deg), nc), data=rng.uniform(-1, 1, size=len(row)).astype(np.float32))
+
+
+@pytest.mark.parametrize("feat,b_dtype,nc,slices", [(32, "f32", 9001, 1), (64, "f32", 40_009, 2), (96, "f32", 40_009, 1), (128, "f32", 20_011, 4),
+                                                    (192, "f32", 40_009, 2), (256, "f32", 40_009, 8), (512, "f32", 20_011, 8),
+                                                    (1024, "f32", 9001, 8), (64, "bf16", 9001, 1), (128, "bf16", 40_009, 2),
+                                                    (512, "bf16", 40_009, 8)])
+def test_feature_slices(fa, torch, feat, b_dtype, nc, slices):
+    """XCD x computes slice x mod S of the features: every tile runs S times, each time for its part of a row of C."""
+    rng = np.random.default_rng(feat)
+    g = sliced_matrix(rng, 5000, nc)                     # 13 divides none of the column counts
+    for widths in ([[1, 2, 4, 8, 16, 32, 64, 128, 256, 512, 1024]], [[4, 16]], [[2, 8, 32, 128, 256], [16, 128]]):
+        _, info = check(fa, torch, g, widths, feat, b_dtype, seed=feat)
+        if len(widths) == 1:
+            assert info["heavy_rows"] >= 1 and info["cleared_rows"] == 40
+            most = max(1, info["grid"] // info["tiles"])                 # (the grid is rounded up to the longest XCD)
+            assert most == slices, (info, most)
+    if feat <= 512:
+        check(fa, torch, g, [[1, 2, 4, 8, 16, 32, 64, 128, 256, 512, 1024]], 2 * feat, b_dtype, seed=feat, windows=2)
+
+
+@pytest.mark.parametrize("cols,feat,windows,parts,b_dtype", [(4_200_000, 256, 1, 1, "f32"), (1_048_576, 1024, 16, 32, "f32"),
+                                                             (2_200_000, 1024, 2, 2, "bf16")])
+def test_operands_of_more_than_4_gb(fa, torch, cols, feat, windows, parts, b_dtype):
+    """Past what 32-bit offsets reach; the second shape in partitions that are small enough for the kernels of
+    parts of B that an L2 holds, whose tiles are larger."""
+    rng = np.random.default_rng(feat)
+    deg = np.concatenate([np.arange(70), [300, 5000, 0, 200], np.full(300, 9)])
+    row = np.repeat(np.arange(len(deg)), deg)
+    col = rng.integers(cols, size=len(row))
+    col[0], col[-1] = 0, cols - 1
+    key = np.unique(row * cols + col)
+    row, col = key // cols, key % cols
+    vals = rng.uniform(-1, 1, size=len(row)).astype(np.float32)
+    g = MTX.from_coo(row, col, (len(deg), cols), data=vals)
+    gen = torch.Generator(device="cuda").manual_seed(1)
+    B = torch.rand((cols, feat), device="cuda", generator=gen, dtype=torch.float32 if b_dtype == "f32" else torch.bfloat16)
+    assert B.numel() * B.element_size() > (1 << 32) - (1 << 17)
+    fmt = fa.build_hyb_format_device(g, [[1, 2, 4, 8, 16, 32, 64, 128, 256]] * parts)
+    plan = fa.HybSpMM(fmt, feat, b_dtype, windows=windows)
+    C = plan.run(B).clone()
+    assert torch.equal(C, plan.run(B))
+    plan.close()
+    used, at = np.unique(col, return_inverse=True)
+    Bh = B[torch.from_numpy(used).cuda()].float().cpu().numpy()
+    indptr = np.concatenate([[0], np.cumsum(np.bincount(row, minlength=len(deg)))])
+    shape = (len(deg), len(used))
+    ref = O.spmm_csr_f64(indptr, at, vals, shape, Bh)
+    assert (np.abs(C.cpu().numpy() - ref) <= TOL * O.spmm_abs_bound(indptr, at, vals, shape, Bh) + 1e-30).all()
