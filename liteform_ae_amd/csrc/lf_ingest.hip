@@ -2,9 +2,10 @@
 // the row pointer.  This is what the reference's matrix container does on the host every
 // time a CSR view is asked for (playground_pipline/format_matrix_market.py:74-76:
 // scipy's coo.tocsr(), which sorts columns and sums duplicates); it is the step that feeds
-// lf_bucket_stats / lf_hyb_build.  Sorting and the segmented sum are plain library
-// primitives (rocPRIM radix sort and reduce-by-key on a 64-bit key row * cols + col); the
-// kernels written here only pack / unpack keys and locate the row boundaries.
+// lf_bucket_stats / lf_hyb_build.  Up to some ten million entries without duplicates go through bins of rows
+// that are sorted in LDS, a kernel each for counting, offsets, distribution and sorting; anything else through plain
+// library primitives (rocPRIM radix sort and reduce-by-key on a 64-bit key row * cols + col), with kernels
+// that pack / unpack keys and locate the row boundaries.
 //
 // Also here: the structural check of CSR arrays that come from a caller (lf_csr_check), which
 // every entry point that gathers through caller-supplied CSR or BSR index arrays runs first,
@@ -20,6 +21,7 @@
 #include <rocprim/functional.hpp>
 
 #include "lf_internal.h"
+#include "lf_spmm_device.h"
 
 namespace {
 
@@ -55,6 +57,459 @@ __global__ void row_pointer_kernel(const unsigned long long* __restrict__ keys, 
         if (keys[mid] < bound) lo = mid + 1; else hi = mid;
     }
     indptr[r] = (int32_t)lo;
+}
+
+// ---- bins of rows sorted in LDS
+// A bin is 2^lg_rows consecutive rows, an entry in it one word - row in the bin, column - and its value.  Entries are
+// distributed to their bins (unordered within one), a workgroup then sorts a bin in LDS and writes its part of the
+// arrays and of the row pointer.  Bound by launches and by the latency of each kernel's two or three dependent passes.
+// With the wait for the flags, us, the library's sort with the kernels around it -> this: 6K entries 82 -> 43, 64K 80 -> 46,
+// 300K 166 -> 56, 760K of a power-law graph (a row of 13,000) 228 -> 105, 1.6M 200 -> 83, 4M 299 -> 193, 8M 590 -> 253;
+// with a duplicate 77 -> 71, 81 -> 76, 165 -> 90, 226 -> 148, 199 -> 135, 300 -> 275, 590 -> 477.  Beyond that many entries
+// bins outgrow the LDS, and the sort's few passes over memory are what counts.
+// flags: [kHard] an entry outside the matrix, a bin that does not fit or a duplicate in a very long row: the other way has
+// to be taken; [kLargeBins] bins left to bin_sort_large_kernel; [kTwice] duplicates, sorted and to be added up.
+constexpr int kBinThreads = 512;
+constexpr int kBinChunk = 4096;            // entries that a workgroup distributes at least
+constexpr int kBinMaxChunks = 1024;
+constexpr int kBinRowMost = 4096;          // entries in a row on average: a few long rows are a few bins' work (3 rows of
+                                           // 16,000: 109 us, the other way 75)
+constexpr int kBinMost = 4096;             // bins: counters and bases in LDS
+constexpr int kBinLgRows = 9;              // rows of a bin: the same
+constexpr int kBinFew = 128, kBinUsual = 1024;     // entries in a bin on average: the first up to kBinUsual bins, then the
+constexpr int kBinTargetMost = 2048;               // second, and this at most
+constexpr int kBinSmall = 4096;            // entries sorted in 48 KB of LDS
+constexpr int kBinLarge = 8192;            // ... in 96 KB, and again for every part of a row of up to kGiantMost
+constexpr int kBinLargeBytes = 3 * 4 * kBinLarge;
+constexpr int kBinLargeGrid = 64;
+
+struct BinShape {
+    int lg_rows, lg_cols, bins, chunks, per_chunk;     // bins == 0: too large, or more than 32 bits to an entry
+    size_t counts, totals, bases, list, flags, records, twice, before, partial, total;
+};
+
+BinShape bin_shape(long long nnz, long long rows, long long cols) {
+    BinShape b{};
+    if (nnz <= 0 || rows <= 0 || cols <= 0 || nnz > (long long)kBinMost * kBinTargetMost || nnz / rows > kBinRowMost) return b;
+    while ((1ll << b.lg_cols) < cols) ++b.lg_cols;
+    const long long by_entries = std::max<long long>(nnz / kBinUsual, std::min<long long>(nnz / kBinFew, kBinUsual));
+    const long long want = std::min<long long>(kBinMost, std::max<long long>(by_entries, (rows >> kBinLgRows) + 1));
+    while ((rows + (1ll << b.lg_rows) - 1) >> b.lg_rows > want) ++b.lg_rows;
+    if (b.lg_rows + b.lg_cols > 31 || b.lg_rows > kBinLgRows) return b;      // (the largest key fills up a sort)
+    b.bins = (int)((rows + (1ll << b.lg_rows) - 1) >> b.lg_rows);
+    b.per_chunk = (int)align_up((size_t)std::max<long long>(kBinChunk, (nnz + kBinMaxChunks - 1) / kBinMaxChunks), kBinThreads);
+    b.chunks = (int)((nnz + b.per_chunk - 1) / b.per_chunk);
+    size_t off = 0;
+    b.records = off; off += align_up((size_t)nnz * 8, 256);
+    b.counts = off; off += align_up((size_t)b.bins * b.chunks * 4, 256);
+    b.totals = off; off += align_up((size_t)b.bins * 4, 256);
+    b.bases = off; off += align_up((size_t)b.bins * 4, 256);
+    b.list = off; off += align_up((size_t)b.bins * 4, 256);
+    b.flags = off; off += 256;
+    b.twice = off; off += align_up((size_t)nnz * 4, 256);
+    b.before = off; off += align_up((size_t)(nnz + 1) * 4, 256);
+    b.partial = off; off += align_up((size_t)(nnz / 1024 + 2) * 4, 256);
+    b.total = off;
+    return b;
+}
+
+__device__ __forceinline__ bool in_matrix(int row, int col, long long rows, long long cols) {
+    return (unsigned long long)(unsigned)row < (unsigned long long)rows && (unsigned long long)(unsigned)col < (unsigned long long)cols;
+}
+
+// counter[i] += 1 for every active lane; what it held before, the lanes in their order.  To be called by whole wavefronts.
+// Lanes of one counter are taken one after the other by the LDS, and a power-law graph's longest row is most of its bin:
+// the first lanes' counters are served with one atomic for all that share them (760K entries with a row of 13,000,
+// sorting 79 -> 22 us together with the buckets).
+__device__ __forceinline__ int count_up(int* counter, int i, bool active) {
+    const int lane = threadIdx.x & 63;
+    int before = 0;
+#pragma unroll
+    for (int round = 0; round < 2; ++round) {
+        const unsigned long long left = __ballot(active);
+        if (left == 0) return before;
+        const int leader = __builtin_ctzll(left);
+        const bool same = active && i == __builtin_amdgcn_readlane(i, leader);
+        const unsigned long long shared = __ballot(same);
+        int first = 0;
+        if (lane == leader) first = atomicAdd(&counter[i], __popcll(shared));
+        first = __builtin_amdgcn_readlane(first, leader);
+        if (same) {
+            before = first + __popcll(shared & ((1ull << lane) - 1ull));
+            active = false;
+        }
+    }
+    if (active) before = atomicAdd(&counter[i], 1);
+    return before;
+}
+
+// counts[bin][chunk]: entries of a chunk (blockIdx.x) in a bin
+__global__ void __launch_bounds__(kBinThreads)
+bin_count_kernel(const int32_t* __restrict__ row, const int32_t* __restrict__ col, long long nnz, long long rows, long long cols,
+                 int lg_rows, int bins, int per_chunk, int* __restrict__ counts, int* __restrict__ flags) {
+    __shared__ int s_count[kBinMost];
+    for (int i = threadIdx.x; i < bins; i += kBinThreads) s_count[i] = 0;
+    __syncthreads();
+    const long long lo = (long long)blockIdx.x * per_chunk, hi = min(lo + per_chunk, nnz);
+    bool bad = false;
+    for (long long i0 = lo; i0 < hi; i0 += kBinThreads) {
+        const long long i = i0 + threadIdx.x;
+        const int r = i < hi ? row[i] : -1;
+        const bool ok = i < hi && in_matrix(r, col[i], rows, cols);
+        bad |= i < hi && !ok;
+        count_up(s_count, r >> lg_rows, ok);
+    }
+    if (__ballot(bad) != 0 && (threadIdx.x & 63) == 0) flags[0] = 1;
+    __syncthreads();
+    for (int i = threadIdx.x; i < bins; i += kBinThreads) counts[(size_t)i * gridDim.x + blockIdx.x] = s_count[i];
+}
+
+// A wavefront to a bin: its counts become the chunks' offsets in it, totals[bin] their sum.
+__global__ void __launch_bounds__(256)
+bin_offsets_kernel(int* __restrict__ counts, int bins, int chunks, int* __restrict__ totals) {
+    const int bin = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+    if (bin >= bins) return;
+    int* mine = counts + (size_t)bin * chunks;
+    int before = 0;
+    for (int c0 = 0; c0 < chunks; c0 += 64) {
+        const int x = c0 + lane < chunks ? mine[c0 + lane] : 0;
+        int incl = x;
+        for (int d = 1; d < 64; d <<= 1) {
+            const int y = __shfl_up(incl, d);
+            if (lane >= d) incl += y;
+        }
+        if (c0 + lane < chunks) mine[c0 + lane] = before + incl - x;
+        before += __shfl(incl, 63);
+    }
+    if (lane == 0) totals[bin] = before;
+}
+
+// Distributes a chunk's entries.  Every workgroup scans the bins' totals for itself; the first leaves the bases.
+__global__ void __launch_bounds__(kBinThreads)
+bin_distribute_kernel(const int32_t* __restrict__ row, const int32_t* __restrict__ col, const float* __restrict__ val, long long nnz,
+                      long long rows, long long cols, int lg_rows, int lg_cols, int bins, int per_chunk,
+                      const int* __restrict__ counts, const int* __restrict__ totals, int* __restrict__ bases,
+                      uint2* __restrict__ records) {
+    __shared__ int s_at[kBinMost];
+    __shared__ int s_wave[kBinThreads / 64];
+    constexpr int kPer = kBinMost / kBinThreads;           // consecutive bins of a thread
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, b0 = threadIdx.x * kPer;
+    int sum = 0;
+    for (int i = b0; i < min(b0 + kPer, bins); ++i) sum += totals[i];
+    int incl = sum;
+    for (int d = 1; d < 64; d <<= 1) {
+        const int y = __shfl_up(incl, d);
+        if (lane >= d) incl += y;
+    }
+    if (lane == 63) s_wave[wave] = incl;
+    __syncthreads();
+    int base = incl - sum;
+    for (int w = 0; w < wave; ++w) base += s_wave[w];
+    for (int i = b0; i < min(b0 + kPer, bins); ++i) {
+        s_at[i] = base + counts[(size_t)i * gridDim.x + blockIdx.x];
+        if (blockIdx.x == 0) bases[i] = base;
+        base += totals[i];
+    }
+    __syncthreads();
+    const long long lo = (long long)blockIdx.x * per_chunk, hi = min(lo + per_chunk, nnz);
+    const int row_mask = (1 << lg_rows) - 1;
+    for (long long i0 = lo; i0 < hi; i0 += kBinThreads) {
+        const long long i = i0 + threadIdx.x;
+        const int r = i < hi ? row[i] : -1, c = i < hi ? col[i] : -1;
+        const float v = i < hi && val ? val[i] : 1.0f;
+        const bool ok = in_matrix(r, c, rows, cols);       // (others are flagged: what is written here is not used)
+        const int at = count_up(s_at, r >> lg_rows, ok);
+        if (ok) records[at] = make_uint2(((unsigned)(r & row_mask) << lg_cols) | (unsigned)c, __float_as_uint(v));
+    }
+}
+
+// Inclusive scan of a workgroup's values; s_wave: a word per wavefront.
+template <int THREADS> __device__ __forceinline__ int scan_workgroup(int x, int* s_wave) {
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    for (int d = 1; d < 64; d <<= 1) {
+        const int y = __shfl_up(x, d);
+        if (lane >= d) x += y;
+    }
+    if (lane == 63) s_wave[wave] = x;
+    __syncthreads();
+    for (int w = 0; w < wave; ++w) x += s_wave[w];
+    __syncthreads();
+    return x;
+}
+
+struct BinSort {
+    const uint2* records;
+    const int *bases, *totals;
+    long long rows;
+    int lg_rows, lg_cols;
+    unsigned inverse;                          // 2^32 / columns: a column's place among them as a 32-bit fraction
+    int32_t *indptr, *indices;
+    float* values;
+    int *list, *flags;
+};
+
+// One bin.  The rows are counted, which gives the row pointer.  A row of len entries then has len buckets, the i-th for
+// the i-th part of the columns: counting puts its entries together bucket by bucket (s_key, s_val), and an entry's
+// place follows from the few of its bucket, equal keys by value.  Where the columns of rows crowd into few buckets
+// (more than kBucketReads reads an entry) the part is sorted bitonically.  Rows of more than kGiantRow entries are
+// sorted after the others, a range of columns at a time (LARGE only; s_giant: row and offset).
+// (Comparing an entry with its whole row: 57K rows of 28 entries 72 us for this kernel, 760K entries of a power-law
+// graph 79; so 25 and 22.)
+constexpr int kBinRows = 1 << kBinLgRows;
+constexpr int kBucketReads = 64;
+constexpr int kGiantRow = 1024, kGiantMost = 32768, kGiants = 256;
+constexpr int kHard = 0, kLargeBins = 1, kTwice = 2;       // flags
+template <int THREADS, int CAPACITY, bool LARGE>
+__device__ __forceinline__ void sort_bin(const BinSort& a, int bin, unsigned* s_key, unsigned* s_val, int* s_bucket, int* s_giant, int* s_wave) {
+    __shared__ int s_first[kBinRows + 1];      // of a row among the entries sorted together; a giant's: -1
+    __shared__ int s_count[kBinRows];
+    __shared__ int s_giants, s_sorted;
+    __shared__ float s_squares;
+    constexpr int kOwn = LARGE ? 16 : CAPACITY / THREADS;  // records in registers: usually all, loaded once
+    const int base = a.bases[bin], n = a.totals[bin];
+    const long long r0 = (long long)bin << a.lg_rows;
+    const int n_rows = (int)min(1ll << a.lg_rows, a.rows - r0);
+    const unsigned col_mask = (unsigned)((1ull << a.lg_cols) - 1);
+    const uint2* records = a.records + base;
+    uint2 own[kOwn];
+    auto load = [&](int from) {
+#pragma unroll
+        for (int k = 0; k < kOwn; ++k) {
+            const int i = from + k * THREADS + (int)threadIdx.x;
+            own[k] = i < n ? records[i] : make_uint2(0, 0);
+        }
+    };
+    const bool once = !LARGE || n <= kOwn * THREADS;
+    if (once) load(0);
+    auto each = [&](auto use) {                            // use(record, is there one), by whole wavefronts
+        for (int from = 0; from < (once ? 1 : n); from += kOwn * THREADS) {
+            if (!once) load(from);
+#pragma unroll
+            for (int k = 0; k < kOwn; ++k)
+                if (from + k * THREADS < n) use(own[k], from + k * THREADS + (int)threadIdx.x < n);
+        }
+    };
+    auto fraction = [&](unsigned key) { return (key & col_mask) * a.inverse; };      // (below 2^32: column < columns)
+    bool twice = false, hard = false;
+    // The records that `selected` takes: by bucket(key), which ascends with the key, and then in full; out(key, place)
+    // is where the place-th goes.  Their number; more than CAPACITY are too many.
+    auto sort_part = [&](auto selected, auto bucket, auto out) {
+        constexpr int kPer = CAPACITY / THREADS;
+        for (int i = threadIdx.x; i < CAPACITY; i += THREADS) s_bucket[i] = 0;
+        if (threadIdx.x == 0) s_squares = 0.f;
+        __syncthreads();
+        each([&](const uint2& x, bool in) {
+            if (in && selected(x.x)) atomicAdd(&s_bucket[bucket(x.x)], 1);
+        });
+        __syncthreads();
+        int sum = 0;
+        float squares = 0.f;
+        for (int k = 0; k < kPer; ++k) {
+            const int x = s_bucket[threadIdx.x * kPer + k];
+            sum += x;
+            squares += (float)x * (float)x;
+        }
+        const int upto = scan_workgroup<THREADS>(sum, s_wave);
+        int before = upto - sum;
+        for (int k = 0; k < kPer; ++k) {
+            const int x = s_bucket[threadIdx.x * kPer + k];
+            s_bucket[threadIdx.x * kPer + k] = before;
+            before += x;
+        }
+        if (squares > 0.f) atomicAdd(&s_squares, squares);
+        if (threadIdx.x == THREADS - 1) s_sorted = upto;
+        __syncthreads();
+        const int sorted = s_sorted;
+        if (sorted > CAPACITY) {
+            hard = true;
+            return sorted;
+        }
+        each([&](const uint2& x, bool in) {
+            if (!in || !selected(x.x)) return;
+            const int to = atomicAdd(&s_bucket[bucket(x.x)], 1);   // (and becomes the bucket's end)
+            s_key[to] = x.x;
+            s_val[to] = x.y;
+        });
+        __syncthreads();
+        if (s_squares <= (float)sorted * kBucketReads) {
+            for (int i = threadIdx.x; i < sorted; i += THREADS) {
+                const unsigned key = s_key[i], val = s_val[i];
+                const int q = bucket(key), first = q > 0 ? s_bucket[q - 1] : 0, end = s_bucket[q];
+                int place = first;
+                for (int j = first; j < end; ++j) {
+                    const unsigned other = s_key[j];
+                    place += other < key;
+                    if (other == key && j != i) {          // by value, then as they lie here
+                        twice = true;
+                        place += s_val[j] < val || (s_val[j] == val && j < i);
+                    }
+                }
+                const int to = out(key, place);
+                a.indices[to] = (int32_t)(key & col_mask);
+                a.values[to] = __uint_as_float(val);
+            }
+        } else {
+            int padded = 64;
+            while (padded < sorted) padded <<= 1;
+            for (int i = sorted + threadIdx.x; i < padded; i += THREADS) s_key[i] = s_val[i] = ~0u;
+            __syncthreads();
+            for (int size = 2; size <= padded; size <<= 1)
+                for (int stride = size >> 1; stride > 0; stride >>= 1) {
+                    for (int p = threadIdx.x; p < padded >> 1; p += THREADS) {
+                        const int i = ((p & ~(stride - 1)) << 1) | (p & (stride - 1)), j = i + stride;
+                        const unsigned ki = s_key[i], kj = s_key[j], vi = s_val[i], vj = s_val[j];
+                        if ((ki > kj || (ki == kj && vi > vj)) == ((i & size) == 0)) {
+                            s_key[i] = kj;
+                            s_key[j] = ki;
+                            s_val[i] = vj;
+                            s_val[j] = vi;
+                        }
+                    }
+                    __syncthreads();
+                }
+            for (int i = threadIdx.x; i < sorted; i += THREADS) {
+                const unsigned key = s_key[i];
+                const int to = out(key, i);
+                a.indices[to] = (int32_t)(key & col_mask);
+                a.values[to] = __uint_as_float(s_val[i]);
+                twice |= i > 0 && s_key[i - 1] == key;
+            }
+        }
+        return sorted;
+    };
+
+    for (int r = threadIdx.x; r < n_rows; r += THREADS) s_count[r] = 0;
+    if (threadIdx.x == 0) s_giants = 0;
+    __syncthreads();
+    each([&](const uint2& x, bool in) { count_up(s_count, (int)(x.x >> a.lg_cols), in); });
+    __syncthreads();
+    // a thread's consecutive rows: offsets among all entries (the row pointer) and among those sorted together
+    const int per = (n_rows + THREADS - 1) / THREADS, lo = min((int)threadIdx.x * per, n_rows), hi = min(lo + per, n_rows);
+    int all = 0, kept = 0;
+    for (int r = lo; r < hi; ++r) {
+        const int len = s_count[r];
+        all += len;
+        if (!LARGE || len <= kGiantRow) kept += len;
+    }
+    int at_all = scan_workgroup<THREADS>(all, s_wave) - all, at = (LARGE ? scan_workgroup<THREADS>(kept, s_wave) : at_all + kept) - kept;
+    for (int r = lo; r < hi; ++r) {
+        const int len = s_count[r];
+        a.indptr[r0 + r] = base + at_all;
+        s_first[r] = at;
+        if (LARGE && len > kGiantRow) {
+            hard |= len > kGiantMost;
+            const int g = atomicAdd(&s_giants, 1);
+            if (g < kGiants) {
+                s_giant[2 * g] = r;
+                s_giant[2 * g + 1] = at_all;
+            }
+            s_first[r] = -1;
+        } else {
+            at += len;
+        }
+        at_all += len;
+    }
+    if (r0 + n_rows == a.rows && threadIdx.x == THREADS - 1) a.indptr[a.rows] = base + n;
+    if (LARGE && threadIdx.x == THREADS - 1) s_sorted = at;                // (behind the last row)
+    hard = __syncthreads_or(hard) != 0 || (LARGE && (s_giants > kGiants || s_sorted > CAPACITY));
+    if (!hard) {
+        sort_part([&](unsigned key) { return !LARGE || s_first[key >> a.lg_cols] >= 0; },
+                  [&](unsigned key) {
+                      const int r = (int)(key >> a.lg_cols);
+                      return s_first[r] + (int)__umulhi(fraction(key), (unsigned)s_count[r]);
+                  },
+                  [&](unsigned key, int place) {
+                      int to = base + place;
+                      if (LARGE)                           // giants before the row
+                          for (int g = 0; g < s_giants; ++g)
+                              if (s_giant[2 * g] < (int)(key >> a.lg_cols)) to += s_count[s_giant[2 * g]];
+                      return to;
+                  });
+        for (int g = 0; LARGE && g < s_giants && !hard; ++g) {
+            const unsigned row = (unsigned)s_giant[2 * g];
+            const unsigned ranges = ((unsigned)s_count[row] + (unsigned)s_count[row] / 4) / CAPACITY + 1;
+            int done = base + s_giant[2 * g + 1];
+            for (unsigned k = 0; k < ranges && !hard; ++k) {
+                __syncthreads();                           // the part before has been read out
+                auto scaled = [&](unsigned key) { return (unsigned long long)fraction(key) * ranges; };
+                done += sort_part([&](unsigned key) { return key >> a.lg_cols == row && scaled(key) >> 32 == k; },
+                                  [&](unsigned key) { return (int)__umulhi((unsigned)scaled(key), CAPACITY); },
+                                  [&](unsigned, int place) { return done + place; });
+            }
+        }
+    }
+    if (__ballot(twice) != 0 && (threadIdx.x & 63) == 0) a.flags[kTwice] = 1;
+    if (__ballot(hard) != 0 && (threadIdx.x & 63) == 0) a.flags[kHard] = 1;
+}
+
+__global__ void __launch_bounds__(kBinThreads)
+bin_sort_kernel(BinSort a) {
+    __shared__ unsigned s_key[kBinSmall], s_val[kBinSmall];
+    __shared__ int s_bucket[kBinSmall];
+    __shared__ int s_wave[kBinThreads / 64];
+    if (a.totals[blockIdx.x] > kBinSmall) {
+        if (threadIdx.x == 0) a.list[atomicAdd(&a.flags[kLargeBins], 1)] = blockIdx.x;
+        return;
+    }
+    sort_bin<kBinThreads, kBinSmall, false>(a, blockIdx.x, s_key, s_val, s_bucket, nullptr, s_wave);
+}
+
+__global__ void __launch_bounds__(1024)
+bin_sort_large_kernel(BinSort a) {
+    extern __shared__ unsigned s_large[];                  // [3][kBinLarge]: keys, values, buckets
+    __shared__ int s_giant[2 * kGiants];
+    __shared__ int s_wave[16];
+    const int n = a.flags[kLargeBins];
+    for (int i = blockIdx.x; i < n; i += gridDim.x) {
+        __syncthreads();                                   // the bin before has been read out
+        sort_bin<1024, kBinLarge, true>(a, a.list[i], s_large, s_large + kBinLarge, (int*)(s_large + 2 * kBinLarge), s_giant, s_wave);
+    }
+}
+
+// ---- duplicates in the sorted arrays: marked, counted up to every entry, and added up into its first (in the order of
+// the sort: by value).
+__global__ void __launch_bounds__(256)
+mark_twice_kernel(const int32_t* __restrict__ indptr, const int32_t* __restrict__ indices, long long nnz, long long rows, int32_t* __restrict__ twice) {
+    const long long i = (long long)blockIdx.x * 256 + threadIdx.x;
+    if (i >= nnz) return;
+    bool same = i > 0 && indices[i - 1] == indices[i];
+    if (same) {                                            // or the first of its row?
+        long long lo = 0, hi = rows;
+        while (lo < hi) {
+            const long long mid = (lo + hi) >> 1;
+            if (indptr[mid] < i) lo = mid + 1; else hi = mid;
+        }
+        same = indptr[lo] != i;
+    }
+    twice[i] = same;
+}
+
+__global__ void __launch_bounds__(256)
+add_up_kernel(const int32_t* __restrict__ indices, const float* __restrict__ values, const int32_t* __restrict__ twice,
+              const int32_t* __restrict__ before, long long nnz, int32_t* __restrict__ out_indices, float* __restrict__ out_values) {
+    const long long i = (long long)blockIdx.x * 256 + threadIdx.x;
+    if (i >= nnz || twice[i]) return;
+    float sum = values[i];
+    for (long long j = i + 1; j < nnz && twice[j]; ++j) sum += values[j];
+    const long long to = i - before[i];
+    out_indices[to] = indices[i];
+    out_values[to] = sum;
+}
+
+// The rows' starts, and the entries back into the caller's arrays (one launch where two copies of the runtime's were 12 us).
+__global__ void __launch_bounds__(256)
+close_up_kernel(int32_t* __restrict__ indptr, const int32_t* __restrict__ before, long long rows, long long nnz, const int32_t* __restrict__ from_indices,
+                const float* __restrict__ from_values, int32_t* __restrict__ indices, float* __restrict__ values) {
+    const long long i = (long long)blockIdx.x * 256 + threadIdx.x;
+    if (i <= rows) indptr[i] -= before[indptr[i]];
+    if (i < nnz - before[nnz]) {
+        indices[i] = from_indices[i];
+        values[i] = from_values[i];
+    }
+}
+
+__global__ void clear_words_kernel(int* __restrict__ p, int n) {
+    if ((int)threadIdx.x < n) p[threadIdx.x] = 0;
 }
 
 // One pass over the row pointer and one over the column indices.  out[0] is raised for
@@ -205,7 +660,7 @@ size_t lf_coo_to_csr_workspace_bytes(int64_t nnz, int64_t num_rows, int64_t num_
     if (nnz <= 0 || num_rows <= 0 || num_cols <= 0) return 256;
     IngestLayout L{};
     if (ingest_layout(nnz, key_bits_for(num_rows, num_cols), &L) != hipSuccess) return 0;
-    return L.total;
+    return std::max(L.total, bin_shape(nnz, num_rows, num_cols).total);
 }
 
 int lf_coo_to_csr(const int32_t* d_coo_row, const int32_t* d_coo_col, const float* d_coo_val, int64_t nnz,
@@ -230,6 +685,45 @@ int lf_coo_to_csr(const int32_t* d_coo_row, const int32_t* d_coo_col, const floa
     LF_REQUIRE(d_workspace && workspace_bytes >= L.total, LF_ERR_WORKSPACE, "workspace has %zu bytes, %zu needed",
                workspace_bytes, L.total);
     char* ws = (char*)d_workspace;
+    const BinShape b = bin_shape(nnz, num_rows, num_cols);
+    if (b.bins > 0 && workspace_bytes >= b.total) {
+        int *counts = (int*)(ws + b.counts), *totals = (int*)(ws + b.totals), *bases = (int*)(ws + b.bases);
+        int *list = (int*)(ws + b.list), *flags = (int*)(ws + b.flags);
+        uint2* records = (uint2*)(ws + b.records);
+        const unsigned inverse = (unsigned)std::min<unsigned long long>((1ull << 32) / (unsigned long long)num_cols, 0xFFFFFFFFull);
+        const BinSort sort{records, bases, totals, num_rows, b.lg_rows, b.lg_cols, inverse, d_indptr, d_indices, d_values, list, flags};
+        LF_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(bin_sort_large_kernel), hipFuncAttributeMaxDynamicSharedMemorySize, kBinLargeBytes));
+        clear_words_kernel<<<1, 64, 0, s>>>(flags, 3);
+        bin_count_kernel<<<b.chunks, kBinThreads, 0, s>>>(d_coo_row, d_coo_col, nnz, num_rows, num_cols, b.lg_rows, b.bins, b.per_chunk, counts, flags);
+        bin_offsets_kernel<<<(b.bins + 3) / 4, 256, 0, s>>>(counts, b.bins, b.chunks, totals);
+        bin_distribute_kernel<<<b.chunks, kBinThreads, 0, s>>>(d_coo_row, d_coo_col, d_coo_val, nnz, num_rows, num_cols, b.lg_rows, b.lg_cols, b.bins,
+                                                               b.per_chunk, counts, totals, bases, records);
+        bin_sort_kernel<<<b.bins, kBinThreads, 0, s>>>(sort);
+        bin_sort_large_kernel<<<std::min(b.bins, kBinLargeGrid), 1024, kBinLargeBytes, s>>>(sort);
+        LF_HIP(hipGetLastError());
+        int h_flags[3] = {0, 0, 0};
+        LF_HIP(lf::read_back(h_flags, flags, sizeof(h_flags), s));
+        if (h_flags[kHard] == 0 && h_flags[kTwice] == 0) {
+            *h_nnz_out = nnz;
+            return LF_OK;
+        }
+        if (h_flags[kHard] == 0) {
+            int32_t *twice = (int32_t*)(ws + b.twice), *before = (int32_t*)(ws + b.before), *partial = (int32_t*)(ws + b.partial);
+            int32_t* out_indices = (int32_t*)records;
+            float* out_values = (float*)(out_indices + nnz);
+            const unsigned blocks = (unsigned)((nnz + 255) / 256);
+            mark_twice_kernel<<<blocks, 256, 0, s>>>(d_indptr, d_indices, nnz, num_rows, twice);
+            LF_HIP(exclusive_scan_i32(twice, nnz, partial, before, s));
+            add_up_kernel<<<blocks, 256, 0, s>>>(d_indices, d_values, twice, before, nnz, out_indices, out_values);
+            close_up_kernel<<<(unsigned)(std::max<long long>(num_rows + 1, nnz) + 255) / 256, 256, 0, s>>>(
+                d_indptr, before, num_rows, nnz, out_indices, out_values, d_indices, d_values);
+            LF_HIP(hipGetLastError());
+            int h_count = 0;
+            LF_HIP(lf::read_back(&h_count, before + nnz, 4, s));
+            *h_nnz_out = nnz - h_count;
+            return LF_OK;
+        }
+    }
     unsigned long long* keys_a = (unsigned long long*)(ws + L.keys_a);
     unsigned long long* keys_b = (unsigned long long*)(ws + L.keys_b);
     float* vals_a = (float*)(ws + L.vals_a);

@@ -200,6 +200,62 @@ def test_device_ingest_matches_scipy_tocsr(fa):
     assert dev.nnz == 0 and dev.indptr.cpu().numpy().tolist() == [0] * 8
 
 
+def coo_case(name):
+    """(rows, columns, shape) of triplets in no order, each place once."""
+    rng = np.random.default_rng(sum(map(ord, name)))
+    if name.startswith("n="):                              # entries around a chunk, a handful of rows to a bin
+        n, (nr, nc) = int(name[2:]), (700, 900)
+        key = rng.choice(nr * nc, size=n, replace=False)
+        return key // nc, key % nc, (nr, nc)
+    shapes = {"giant rows": (600, 40_000, [1024, 1025, 4096, 4097, 9000, 32_768]), "a row past the limit": (40, 90_000, [32_769, 5000]),
+              "crowded columns": (64, 1 << 21, [3000, 900, 2000, 1500]), "one column": (5000, 1, []), "one row": (1, 3000, [2500]),
+              "few entries": (2_100_000, 50, []), "wide keys": (300_000, 1 << 23, []), "long bins": (512 * 40, 30_000, [4000] * 60)}
+    nr, nc, lens = shapes[name]
+    deg = np.minimum(rng.integers(0, 9, size=nr), nc) if nr < 1_000_000 else (rng.random(nr) < 0.01).astype(np.int64)
+    deg[rng.choice(nr, size=len(lens), replace=False)] = lens
+    row = np.repeat(np.arange(nr), deg)
+    col = np.concatenate([rng.choice(min(nc, 4000) if name == "crowded columns" else nc, size=d, replace=False) for d in deg if d]
+                         or [np.zeros(0, np.int64)])
+    return row, col, (nr, nc)
+
+
+@pytest.mark.parametrize("twice", ["none", "some", "many"])
+@pytest.mark.parametrize("name", ["n=1", "n=63", "n=4095", "n=4096", "n=4097", "n=130000", "giant rows", "a row past the limit", "crowded columns",
+                                  "one column", "one row", "few entries", "wide keys", "long bins"])
+def test_triplets_through_bins_of_rows(fa, name, twice):
+    """Every way an entry can take: bins sorted by buckets or bitonically, large bins, rows that are sorted a range of
+    columns at a time, rows and bins past the limits, shapes that are left to the library's sort; without
+    duplicates (the values' bits are kept, not only numbers), with some and with 300 of one entry."""
+    import scipy.sparse as sp
+    from liteform_ae_amd.format_matrix_market import MTX
+    row, col, shape = coo_case(name)
+    rng = np.random.default_rng(len(row))
+    if twice != "none":
+        again = rng.integers(0, len(row), size=max(1, len(row) // 10))
+        if twice == "many":
+            again = np.concatenate([again, np.full(300, rng.integers(0, len(row)))])
+        row, col = np.concatenate([row, row[again]]), np.concatenate([col, col[again]])
+    order = rng.permutation(len(row))
+    row, col = row[order].astype(np.int32), col[order].astype(np.int32)
+    val = rng.uniform(-1, 1, size=len(row)).astype(np.float32)
+    if twice == "none":
+        val[:4] = np.array([np.inf, -0.0, np.nan, 1e-42], dtype=np.float32)[:len(val)]
+    dev = fa._DeviceCSR(MTX.from_coo(row, col, shape, data=val))
+    want = sp.coo_matrix((val.astype(np.float64), (row, col)), shape=shape).tocsr()
+    want.sort_indices()
+    assert dev.nnz == want.nnz
+    np.testing.assert_array_equal(dev.indptr.cpu().numpy(), want.indptr)
+    np.testing.assert_array_equal(dev.indices.cpu().numpy(), want.indices)
+    got = dev.values.cpu().numpy()
+    if twice == "none":
+        np.testing.assert_array_equal(got.view(np.int32), want.data.astype(np.float32).view(np.int32))
+    else:
+        # float32 sums of up to 310 values below 1 in some order: 310 roundings of partial sums below 310
+        np.testing.assert_allclose(got, want.data, rtol=0, atol=310 * 2.0 ** -24 * (310 if twice == "many" else 4))
+    again = fa._DeviceCSR(MTX.from_coo(row, col, shape, data=val))
+    assert np.array_equal(again.values.cpu().numpy().view(np.int32), got.view(np.int32))        # run to run the same bits
+
+
 def test_canonical_csr_input_goes_in_as_it_is(fa):
     """A container made from canonical CSR arrays is uploaded and checked (lf_csr_check), not
     converted to COO and sorted: same device arrays, statistics and slabs as the COO route."""
