@@ -138,13 +138,18 @@ CsrFn csr_kernel(int lpr, int ch, int dtype, bool wide) {
          : lpr == 32 ? csr_kernel<32, 1>(dtype, wide) : csr_kernel<64, 1>(dtype, wide);
 }
 
-// 10 % for every halving of the workgroups below 2048: what small matrices gain from the split besides.  130 matrices of
-// 2K to 1.2M rows, log-normal and power-law, N = 64 .. 512, f32 and bf16, every S timed: the pick loses 2 % on average
-// to the best, S = 1 24 %, S = 4 4.6 %.  Worst picks: 34 % (9K x 13K, 31K entries, bf16 N = 256: 8.5 us with 2, 11.4
-// with 4), and against S = 1 14 % (335K power-law rows, N = 128: 119 -> 135).
+// 10 % for every halving of the workgroups below 2048: what small matrices gain from the split besides; 2 % for every
+// doubling of S, for what its price does not hold; and 10 % where a row takes a whole wavefront (rows of B over 512
+// bytes): nothing then fills the gathers that its last batch leaves empty (433K rows of 9 entries, N = 256: 647 us with
+// S = 1, 604 with 2; 300K power-law rows of 5: 430, 346).  360 matrices of 2K to 2M rows, log-normal and power-law, N = 64
+// .. 512, f32 and bf16, every S timed: the pick loses 2.9 % on average to the best (3.1 without the last rule), S = 1 22 %,
+// S = 4 5.4 %.  Worst picks: S = 1 for 49K power-law rows of 5, N = 128 (63.9 us, 33.2 with 4); S = 8 for 10K rows of 8,
+// bf16 N = 512 (15.8, 11.5).
 int csr_slices(int64_t groups, int64_t num_cols, int64_t nnz, int feat, int dtype) {
+    const int row_bytes = feat * (dtype == LF_DTYPE_BF16 ? 2 : 4);
     return feature_slices(num_cols, nnz, feat, dtype, [&](int s, double us) {
-        return us * (1.0 + 0.1 * std::max(0.0, std::log2(2048.0 / ((double)groups * s)))) * (s > 1 ? 1.02 : 1.0);
+        return us * (1.0 + 0.1 * std::max(0.0, std::log2(2048.0 / ((double)groups * s))))
+                  * (row_bytes / s > 512 ? 1.1 : 1.0) * (1.0 + 0.02 * std::log2((double)s));
     });
 }
 
