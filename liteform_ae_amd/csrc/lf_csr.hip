@@ -25,8 +25,8 @@ struct CsrArgs {
     const float* values;                   // null: ones
     long long n_rows, n_groups;
     int rows_per_group;
-    int lg_slices;                         // log2 of the feature slices, up to kLgXcds
-    int feat, ld;                          // features of a slice; elements between rows of B and of C
+    int feat, ld;                          // features of a slice (the last may have fewer); elements between rows of B and of C
+    XcdParts parts;
     const void* B;
     float* C;
     unsigned long long b_bytes;
@@ -54,18 +54,24 @@ csr_spmm_kernel(CsrArgs a) {
     constexpr int kLgSubs = Teams<LPR, CH, BT, WIDE>::kLgSubs;
     __shared__ int s_next;
     extern __shared__ __align__(16) float s_red[];         // [kWaves][feat]: sums of a long row's parts
-    // workgroup i runs on XCD i % 8; XCD x computes slice x mod 2^lg_slices of its rows
-    const int xcd = blockIdx.x % kXcds, slice = xcd & ((1 << a.lg_slices) - 1);
-    const long long group = ((long long)(blockIdx.x / kXcds) << (kLgXcds - a.lg_slices)) + (xcd >> a.lg_slices);
-    if (group >= a.n_groups) return;
+    // workgroup i runs on XCD i % 8 and takes entry i / 8 of that XCD's part
+    const XcdPart part = xcd_part(a.parts, blockIdx.x % kXcds);
+    const int n_groups = (int)a.n_groups;
+    int slice = part.slice, group = tiles_before(n_groups, part.from) + blockIdx.x / kXcds;
+    if (group >= tiles_before(n_groups, part.upto)) {
+        group -= tiles_before(n_groups, part.upto);
+        if (group >= tiles_before(n_groups, part.next)) return;
+        ++slice;
+    }
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int sub = lane / LPR;
-    const Lane<LPR, CH, VEC> ln(lane % LPR, a.feat, a.ld, a.ld);
     const size_t skip = (size_t)slice * a.feat;
+    const int feat = min(a.feat, a.ld - (int)skip);
+    const Lane<LPR, CH, VEC> ln(lane % LPR, feat, a.ld, a.ld);
     const RowsOfB<LPR, CH, BT, WIDE> b((const char*)a.B + skip * Dense<BT>::kElemBytes, a.b_bytes - skip * Dense<BT>::kElemBytes, ln);
     float* C = a.C + skip;
 
-    const long long first_row = group * a.rows_per_group;
+    const long long first_row = (long long)group * a.rows_per_group;
     const int n = (int)min((long long)a.rows_per_group, a.n_rows - first_row);       // at most 64
     const int start = a.indptr[first_row + min(lane, n)], end = a.indptr[first_row + min(lane + 1, n)];
     if (tid == 0) s_next = kWaves;
@@ -111,13 +117,13 @@ csr_spmm_kernel(CsrArgs a) {
             for (int c = 0; c < CH; ++c) {
                 if (!ln.on[c]) continue;
 #pragma unroll
-                for (int i = 0; i < VEC; ++i) s_red[wave * a.feat + ln.f[c] + i] = acc.v[c][i];
+                for (int i = 0; i < VEC; ++i) s_red[wave * feat + ln.f[c] + i] = acc.v[c][i];
             }
         }
         __syncthreads();
-        for (int f = tid; f < a.feat; f += kCsrThreads) {
+        for (int f = tid; f < feat; f += kCsrThreads) {
             float sum = 0.f;
-            for (int w = 0; w < kWaves; ++w) sum += s_red[w * a.feat + f];
+            for (int w = 0; w < kWaves; ++w) sum += s_red[w * feat + f];
             C[(size_t)(first_row + r) * a.ld + f] = sum;
         }
         __syncthreads();                                     // before the next row's parts
@@ -138,18 +144,19 @@ CsrFn csr_kernel(int lpr, int ch, int dtype, bool wide) {
          : lpr == 32 ? csr_kernel<32, 1>(dtype, wide) : csr_kernel<64, 1>(dtype, wide);
 }
 
-// 10 % for every halving of the workgroups below 2048: what small matrices gain from the split besides; 2 % for every
-// doubling of S, for what its price does not hold; and 10 % where a row takes a whole wavefront (rows of B over 512
-// bytes): nothing then fills the gathers that its last batch leaves empty (433K rows of 9 entries, N = 256: 647 us with
-// S = 1, 604 with 2; 300K power-law rows of 5: 430, 346).  360 matrices of 2K to 2M rows, log-normal and power-law, N = 64
-// .. 512, f32 and bf16, every S timed: the pick loses 2.9 % on average to the best (3.1 without the last rule), S = 1 22 %,
-// S = 4 5.4 %.  Worst picks: S = 1 for 49K power-law rows of 5, N = 128 (63.9 us, 33.2 with 4); S = 8 for 10K rows of 8,
-// bf16 N = 512 (15.8, 11.5).
-int csr_slices(int64_t groups, int64_t num_cols, int64_t nnz, int feat, int dtype) {
-    const int row_bytes = feat * (dtype == LF_DTYPE_BF16 ? 2 : 4);
-    return feature_slices(num_cols, nnz, feat, dtype, [&](int s, double us) {
-        return us * (1.0 + 0.1 * std::max(0.0, std::log2(2048.0 / ((double)groups * s))))
-                  * (row_bytes / s > 512 ? 1.1 : 1.0) * (1.0 + 0.02 * std::log2((double)s));
+// 16 % for every halving of the workgroups below 2048: what small matrices gain from the split besides; 2 % for every
+// doubling of S and 7 us for a million rows' starts, for what its price does not hold; 0.3 us for every doubling of the
+// sub-waves to a wavefront; and 4 % where a row takes a whole wavefront (rows of B over 512 bytes): nothing then fills the
+// gathers that its last batch leaves empty (433K rows of 9 entries, N = 256: 647 us with S = 1, 604 with 2; 300K power-law
+// rows of 5: 430, 346).  1000 matrices of 2K to 2M rows, log-normal and power-law, N = 64 .. 512, f32 and bf16, every S
+// timed: the pick takes 0.89 of the time of S = 1 on average, 2.6 % more than the best; 3 % of them are more than 3 % slower
+// than with S = 1, 21 % at worst (25K rows of 4, N = 160: 12.9 us, 15.6 with 5).  128K rows of 100, N = 96: 635 us with 1,
+// 564 with 3.
+Slices csr_slices(int64_t rows, int64_t groups, int64_t num_cols, int64_t nnz, int feat, int dtype) {
+    return feature_slices(num_cols, nnz, feat, dtype, [&](int s, int width, int lg_subs, double us) {
+        return us * (1.0 + 0.16 * std::max(0.0, std::log2(2048.0 / ((double)groups * s))))
+                  * (width * (dtype == LF_DTYPE_BF16 ? 2 : 4) > 512 ? 1.04 : 1.0) * (1.0 + 0.02 * std::log2((double)s))
+               + 0.3 * lg_subs + 7e-6 * (double)rows * s;
     });
 }
 
@@ -170,9 +177,9 @@ int lf_csr_spmm_trusted_nnz(const int32_t* d_indptr, const int32_t* d_indices, c
     CsrArgs a{};
     a.rows_per_group = num_rows >= kCsrManyRows ? kCsrRowsMany : kCsrRowsFew;
     a.n_groups = lf::ceil_div(num_rows, (int64_t)a.rows_per_group);
-    const int slices = csr_slices(a.n_groups, num_cols, nnz, feat_size, b_dtype);
-    a.lg_slices = lf::ilog2(slices);
-    a.feat = feat_size / slices;
+    const Slices slices = csr_slices(num_rows, a.n_groups, num_cols, nnz, feat_size, b_dtype);
+    a.feat = slices.feat;
+    a.parts = slices.parts;
     if (int rc = feature_shape(a.feat, b_dtype, &lpr, &ch)) return rc;
     a.indptr = d_indptr;
     a.indices = d_indices;
@@ -182,7 +189,9 @@ int lf_csr_spmm_trusted_nnz(const int32_t* d_indptr, const int32_t* d_indices, c
     a.B = d_B;
     a.C = d_C;
     a.b_bytes = (unsigned long long)num_cols * feat_size * (b_dtype == LF_DTYPE_BF16 ? 2 : 4);
-    const unsigned grid = (unsigned)(lf::ceil_div(a.n_groups, (int64_t)(kXcds / slices)) * kXcds);
+    long long longest = 0;
+    for (int x = 0; x < kXcds; ++x) longest = std::max(longest, part_tiles(a.parts, x, a.n_groups));
+    const unsigned grid = (unsigned)(longest * kXcds);
     csr_kernel(lpr, ch, b_dtype, a.b_bytes > kPastB)<<<grid, kCsrThreads, (kCsrThreads / 64) * a.feat * sizeof(float), (hipStream_t)stream>>>(a);
     LF_HIP(hipGetLastError());
     return LF_OK;

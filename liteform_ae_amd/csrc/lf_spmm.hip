@@ -22,9 +22,9 @@
 //     atomics and the order of every sum is fixed, so results are bit-reproducible; the one atomic of a
 //     product counts the chunks of a long row that have left their partial row.
 //
-// The workgroup -> tile mapping is XCD-aware: workgroup i runs on XCD i % 8, XCD x computes feature slice x mod S,
-// and each group of tiles is cut into 8 / S contiguous ranges, one per XCD of a slice, so that neighbouring ELL
-// rows (which tend to share B rows in structured matrices) meet in the same L2.
+// The workgroup -> tile mapping is XCD-aware: workgroup i runs on XCD i % 8, an XCD computes an eighth of the features'
+// slices, and within a slice a contiguous range of each group of tiles, so that neighbouring ELL rows (which tend to
+// share B rows in structured matrices) meet in the same L2.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -493,8 +493,8 @@ __device__ __forceinline__ void run_chunk_tile(const RowsOfB<LPR, CH, BT, WIDE>&
 // ------------------------------------------------------------------------------------
 // The fused kernel: one workgroup per tile, all tile groups of one column partition in one
 // launch.  Workgroup i runs on XCD i % 8 and takes entry i / 8 of that XCD's tile list: for
-// every group the contiguous eighth of its tiles that belongs to the XCD, groups
-// concatenated.  The hardware hands out workgroups in index order as slots free up, which
+// every group the contiguous range of its tiles that belongs to the XCD, groups
+// concatenated, and where the XCD has a part of a second feature slice, the same for that.  The hardware hands out workgroups in index order as slots free up, which
 // keeps the tiles in flight on an XCD next to each other and balances the load; a resident
 // grid that strides over the tiles measured 2-7 % slower on every workload.
 //
@@ -530,7 +530,7 @@ __device__ __forceinline__ Group load_group(const __attribute__((address_space(4
 
 template <int LPR, int CH, typename BT, bool RESIDENT, bool WIDE>
 __global__ void __launch_bounds__(kWG, partition_min_waves(LPR, CH, Dense<BT>::kVec == 8, RESIDENT))
-spmm_partition_kernel(LaunchArgs a) {
+spmm_partition_kernel(LaunchArgs a, XcdParts parts) {
     // one LDS buffer, used either as the staged tile ((col, val) pairs then (row, meta)
     // entries) or as the reduction scratch of a chunk tile (one accumulator per thread)
     constexpr int kTileSlots = tile_slots(LPR, RESIDENT && Dense<BT>::kVec == 4);
@@ -546,47 +546,49 @@ spmm_partition_kernel(LaunchArgs a) {
     // arguments: reading the groups one after the other took a round trip to memory each.  The group itself is read
     // whole, by scalar loads (through the constant address space: nothing writes it while the launch runs): field by
     // field, where it is used, each read was a round trip of its own.
-    const int xcd = blockIdx.x % kXcds;
-    const int slice = xcd & ((1 << a.lg_slices) - 1), rank = xcd >> a.lg_slices, lg_ranks = kLgXcds - a.lg_slices;
-    const size_t skip = (size_t)slice * a.feat;
-    a.C += skip;
-    a.partials += (size_t)slice * a.slice_partials;
-    a.heavy += (size_t)slice * a.slice_heavy;
+    XcdPart part = xcd_part(parts, blockIdx.x % kXcds);
     using ConstGroup = const __attribute__((address_space(4))) Group;
     ConstGroup* groups = (ConstGroup*)(uintptr_t)a.groups;
     int v = blockIdx.x / kXcds;
-    // the XCD's share of n_tiles tiles: [first, first + count)
-    auto share = [&](int n_tiles, int& first) {
-        const int whole = n_tiles >> lg_ranks, rest = n_tiles & ((1 << lg_ranks) - 1);
-        first = whole * rank + (rest * rank >> lg_ranks);
-        return whole * (rank + 1) + (rest * (rank + 1) >> lg_ranks) - first;
-    };
     // a group to a lane, the shares' prefix sums by DPP, the group from one ballot: group by group the walk to the
     // last of eleven was 300 scalar instructions
-    int n_tiles = 0, first;
+    int n_tiles = 0, gi;
 #pragma unroll
     for (int i = 0; i < kInlineGroups; ++i) n_tiles = (int)(threadIdx.x & 63) == i ? a.n_tiles[i] : n_tiles;
-    const int count = share(n_tiles, first);
-    int until = count;
-    until += __builtin_amdgcn_update_dpp(0, until, 0x111, 0xF, 0xF, true);       // row_shr:1, 2, 4, 8
-    until += __builtin_amdgcn_update_dpp(0, until, 0x112, 0xF, 0xF, true);
-    until += __builtin_amdgcn_update_dpp(0, until, 0x114, 0xF, 0xF, true);
-    until += __builtin_amdgcn_update_dpp(0, until, 0x118, 0xF, 0xF, true);
-    const int behind = (int)(__ballot(v < until) & ((1ull << kInlineGroups) - 1));
-    int gi;
-    if (behind) {
-        gi = __builtin_ctz(behind);
-        v += __builtin_amdgcn_readlane(first - (until - count), gi);
-    } else {
-        v -= __builtin_amdgcn_readlane(until, kInlineGroups - 1);
-        for (gi = kInlineGroups; gi < a.n_groups; ++gi) {
-            const int n = share((int)groups[gi].n_tiles, first);
-            if (v < n) break;
-            v -= n;
+    for (;;) {
+        const int first = tiles_before(n_tiles, part.from), count = tiles_before(n_tiles, part.upto) - first;
+        int until = count;
+        until += __builtin_amdgcn_update_dpp(0, until, 0x111, 0xF, 0xF, true);       // row_shr:1, 2, 4, 8
+        until += __builtin_amdgcn_update_dpp(0, until, 0x112, 0xF, 0xF, true);
+        until += __builtin_amdgcn_update_dpp(0, until, 0x114, 0xF, 0xF, true);
+        until += __builtin_amdgcn_update_dpp(0, until, 0x118, 0xF, 0xF, true);
+        const int behind = (int)(__ballot(v < until) & ((1ull << kInlineGroups) - 1));
+        if (behind) {
+            gi = __builtin_ctz(behind);
+            v += __builtin_amdgcn_readlane(first - (until - count), gi);
+            break;
         }
-        if (gi >= a.n_groups) return;
-        v += first;
+        v -= __builtin_amdgcn_readlane(until, kInlineGroups - 1);
+        int skipped = 0;
+        for (gi = kInlineGroups; gi < a.n_groups; ++gi) {
+            const int n = (int)groups[gi].n_tiles;
+            skipped = tiles_before(n, part.from);
+            const int mine = tiles_before(n, part.upto) - skipped;
+            if (v < mine) break;
+            v -= mine;
+        }
+        if (gi < a.n_groups) {
+            v += skipped;
+            break;
+        }
+        if (part.next == 0) return;
+        part = XcdPart{part.slice + 1, 0, part.next, 0};
     }
+    const size_t skip = (size_t)part.slice * a.feat;
+    a.C += skip;
+    a.partials += (size_t)part.slice * a.slice_partials;
+    a.heavy += (size_t)part.slice * a.slice_heavy;
+    a.feat = min(a.feat, a.all_feat - (int)skip);
     const Group g = load_group(groups + gi);
     const RowsOfB<LPR, CH, BT, WIDE> b((const char*)a.B + skip * Dense<BT>::kElemBytes, a.b_bytes - skip * Dense<BT>::kElemBytes,
                                        Lane<LPR, CH, Dense<BT>::kVec>(threadIdx.x % LPR, a.feat, a.ldb, a.ldc));
@@ -610,11 +612,13 @@ spmm_finalize_wide_kernel(const HeavyRow* __restrict__ heavy, int n_heavy, Launc
     constexpr int U = 4;
     __shared__ float s_red[kWG * CH * VEC];
     const int sw = threadIdx.x / LPR, sl = threadIdx.x % LPR;
+    const int skip = blockIdx.y * a.feat;                   // the feature slice
+    a.C += skip;
+    a.partials += (size_t)blockIdx.y * a.slice_partials;
+    a.feat = min(a.feat, a.all_feat - skip);
     const Lane<LPR, CH, VEC> ln(sl, a.feat, a.ldb, a.ldc);
     const int h = blockIdx.x;
     if (h >= n_heavy) return;
-    a.C += (size_t)blockIdx.y * a.feat;                     // the feature slice
-    a.partials += (size_t)blockIdx.y * a.slice_partials;
     const HeavyRow hr = heavy[h];
     if (hr.n_partials <= kWideFinalPartials) return;
     Acc<CH, VEC> acc;
@@ -1321,8 +1325,10 @@ struct lf_spmm_plan {
     int feat = 0, b_dtype = 0, num_parts = 0;
     int64_t num_rows = 0, num_cols = 0;
     int lpr = 0, ch = 0;
-    int slices = 1;                  // feature slices of `feat` features that the XCDs share out within a launch
-    int windows = 1;                 // feature windows of slices * feat features each that a run covers
+    int window = 0;                  // features of a window
+    int slices = 1;                  // feature slices that the XCDs share out within a launch, of `feat` features (the last up to that)
+    XcdParts parts;
+    int windows = 1;                 // feature windows that a run covers
     int device = 0, num_cus = 0, grid = 0;
     struct Launch {
         int group_begin = 0, n_groups = 0, grid = 0;
@@ -1377,7 +1383,7 @@ int free_temporaries(lf_spmm_plan* p) {
     return rc;
 }
 
-using KernelFn = void (*)(LaunchArgs);
+using KernelFn = void (*)(LaunchArgs, XcdParts);
 using FinalFn = void (*)(const HeavyRow*, int, LaunchArgs);
 
 using RowGroupFn = void (*)(const MergedBucket*, int, LaunchArgs);
@@ -1467,7 +1473,8 @@ int lf_spmm_create(lf_spmm_plan** out_plan, const lf_bucket_desc* h_buckets, int
     }
 
     lf_spmm_plan* plan = new lf_spmm_plan();
-    plan->feat = feat_size;
+    plan->feat = plan->window = feat_size;
+    plan->parts = xcd_parts(1, 1);
     plan->b_dtype = b_dtype;
     plan->num_parts = num_parts;
     plan->num_rows = num_rows;
@@ -1650,22 +1657,27 @@ int lf_spmm_create(lf_spmm_plan** out_plan, const lf_bucket_desc* h_buckets, int
     auto scanned = [&](int k, int i) { return h_counters[((size_t)kScanCounters * k + i) * kCounterLine]; };
 
     // ---- Feature slices; matrices whose kernels share gathers between rows read B through the L2s as it is.
-    // A doubling of S costs 0.8 us in rows' starts and ends, and sub-waves of fewer lanes are more of them to share a
-    // long row's chunk, whose chain of gathers (0.11 us a step; it overlaps with other work) sets the time of small
-    // power-law products.  1500 matrices of 2K to 1M rows, log-normal and power-law, N = 32 .. 512, f32 and bf16, every
-    // S timed at the shape that predict_launch_shape gives: 0.93 of the time with S = 1 on average (0.4 at best: 64000
-    // rows of 32 entries, N = 256 287 -> 213 us; 16000 56 -> 30), 3 % of them more than 3 % slower, 16 % at worst.
+    // A doubling of S costs 0.5 us in rows' starts and ends, one of the sub-waves to a wavefront 0.35, and sub-waves of fewer
+    // lanes are more of them to share a long row's chunk, whose chain of gathers (0.11 us a step; it overlaps with other
+    // work) sets the time of small power-law products.  3900 matrices of 2K to 2M rows, log-normal and power-law, N = 32 ..
+    // 512, f32 and bf16, every S timed at the shape that predict_launch_shape gives: 0.925 of the time with S = 1 on
+    // average, 1.6 % above the best S; 3 % of them more than 3 % slower than S = 1, 30 % at worst (products of 8 to 17
+    // us with a B of 4 to 5 MB).  S that are no power of two, us, S = 1 or 2 before -> now: 32K rows of 32 entries, N = 96
+    // 40.6 -> 29.6, 160 81 -> 43, 192 78 -> 50, 224 118 -> 58; 64K rows of 32, N = 224 247 -> 168, 352 393 -> 331; 64K rows of
+    // 100, N = 288 in 16 partitions 825 -> 662; 132K rows of 300, N = 96 in 16 partitions 1025 -> 993, in 8 1003 -> 891.
     if (chosen.empty()) {
         const int vec = b_dtype == LF_DTYPE_BF16 ? 8 : 4;
         bool chains = false;                               // rows of several chunks
         for (int k = 0; k < num_buckets; ++k) chains = chains || scanned(k, 1) > 0;
-        plan->slices = feature_slices(lf::ceil_div(num_cols, (int64_t)num_parts), total_slots / num_parts, feat_size, b_dtype,
-                                      [&](int n, double us) {
-            const int lanes = std::min(64, std::max(8, feat_size / n / vec));
+        const Slices slices = feature_slices(lf::ceil_div(num_cols, (int64_t)num_parts), total_slots / num_parts, feat_size, b_dtype,
+                                             [&](int n, int width, int lg_subs, double us) {
+            const int lanes = std::min(64, std::max(8, width / vec));
             const double steps = (double)chunk_slots * lanes / (kWG * kUnroll);
-            return us + 0.8 * lf::ilog2(n) + (chains ? 0.11 * steps : 0.0);
+            return us + 0.5 * std::log2((double)n) + 0.35 * lg_subs + (chains ? 0.11 * steps : 0.0);
         });
-        plan->feat = feat_size /= plan->slices;
+        plan->slices = slices.n;
+        plan->parts = slices.parts;
+        plan->feat = feat_size = slices.feat;
         LF_TRY(feature_shape(feat_size, b_dtype, &lpr, &ch));
         plan->lpr = lpr;
         plan->ch = ch;
@@ -1900,7 +1912,7 @@ int lf_spmm_create(lf_spmm_plan** out_plan, const lf_bucket_desc* h_buckets, int
             rows_all += h_buckets[k].num_ell_rows;
             if (h_buckets[k].width >= kStreamMinWidth) rows_wide += h_buckets[k].num_ell_rows;
         }
-        const bool c_fits_l2 = (long long)num_rows * feat_size * plan->slices * 4 <= kL2Bytes;
+        const bool c_fits_l2 = (long long)num_rows * plan->window * 4 <= kL2Bytes;
         L.stream_c = rows_wide * 2 >= rows_all || (b_dtype == LF_DTYPE_F32 && !c_fits_l2);
         for (int k : mine) L.wide_rows = L.wide_rows || has_wide[k];
         L.heavy_begin = mine.empty() ? 0 : heavy_base[mine.front()];
@@ -1997,13 +2009,11 @@ int lf_spmm_create(lf_spmm_plan** out_plan, const lf_bucket_desc* h_buckets, int
             if (longest_m * kXcds >= (1ll << 31)) return bail(lf::fail(LF_ERR_UNSUPPORTED, "too many row-group tiles"));
             L.merged_grid = (int)(longest_m * kXcds);
         }
-        // grid: 8 x the longest per-XCD tile list; the XCDs of a feature slice share out all tiles
+        // grid: 8 x the longest per-XCD tile list
         long long longest = 0;
-        const int ranks = kXcds / plan->slices;
-        for (int x = 0; x < ranks; ++x) {
+        for (int x = 0; x < kXcds; ++x) {
             long long len = 0;
-            for (int gi = L.group_begin; gi < (int)groups.size(); ++gi)
-                len += groups[gi].n_tiles * (x + 1) / ranks - groups[gi].n_tiles * x / ranks;
+            for (int gi = L.group_begin; gi < (int)groups.size(); ++gi) len += part_tiles(plan->parts, x, groups[gi].n_tiles);
             longest = std::max(longest, len);
         }
         for (int gi = L.group_begin; gi < (int)groups.size(); ++gi) {
@@ -2130,7 +2140,7 @@ int lf_spmm_run(lf_spmm_plan* plan, const void* d_B, float* d_C, lf_stream_t str
     if (int rc = order_behind_last_run(plan, s)) return rc;
     // One pass per feature window (all partitions inside), each on its own columns of B and C.
     const size_t b_elem = plan->b_dtype == LF_DTYPE_BF16 ? 2 : 4;
-    const int window = plan->feat * plan->slices, ld = window * plan->windows;
+    const int window = plan->window, ld = window * plan->windows;
     const unsigned long long b_bytes = (unsigned long long)plan->num_cols * ld * b_elem;
     const KernelFn tiles = b_bytes > kPastB ? ks.tiles_wide : plan->resident ? ks.tiles_resident : ks.tiles;
     for (int w = 0; w < plan->windows; ++w) {
@@ -2143,11 +2153,11 @@ int lf_spmm_run(lf_spmm_plan* plan, const void* d_B, float* d_C, lf_stream_t str
             a.accumulate = (p > 0 ? kAccumulateC : 0) | (p + 1 == plan->num_parts && L.stream_c ? kStreamC : 0) |
                            (plan->stream_slabs ? kStreamSlabs : 0);
             a.feat = plan->feat;
+            a.all_feat = window;
             a.ldb = a.ldc = ld;
             a.B = (const char*)d_B + (size_t)w * window * b_elem;
             a.C = d_C + (size_t)w * window;
             a.b_bytes = b_bytes - (size_t)w * window * b_elem;
-            a.lg_slices = lf::ilog2(plan->slices);
             a.slice_heavy = plan->n_heavy;
             a.slice_partials = plan->slice_partials;
             a.partials = plan->d_partials;
@@ -2155,7 +2165,7 @@ int lf_spmm_run(lf_spmm_plan* plan, const void* d_B, float* d_C, lf_stream_t str
             a.coop_slots = plan->coop_slots;
             std::memcpy(a.n_tiles, L.n_tiles, sizeof(a.n_tiles));
             if (L.grid > 0) {
-                tiles<<<L.grid, kWG, L.dyn_lds, s>>>(a);
+                tiles<<<L.grid, kWG, L.dyn_lds, s>>>(a, plan->parts);
                 LF_HIP(hipGetLastError());
             }
             if (L.n_merged > 0) {
@@ -2178,7 +2188,7 @@ int lf_spmm_run(lf_spmm_plan* plan, const void* d_B, float* d_C, lf_stream_t str
 
 int lf_spmm_set_windows(lf_spmm_plan* plan, int32_t n_windows) {
     LF_REQUIRE(plan, LF_ERR_INVALID, "plan is null");
-    LF_REQUIRE(n_windows >= 1 && (int64_t)n_windows * plan->slices * plan->feat <= (1 << 20), LF_ERR_INVALID,
+    LF_REQUIRE(n_windows >= 1 && (int64_t)n_windows * plan->window <= (1 << 20), LF_ERR_INVALID,
                "bad number of feature windows (%d)", n_windows);
     plan->windows = n_windows;
     return LF_OK;

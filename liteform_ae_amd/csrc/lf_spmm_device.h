@@ -107,13 +107,13 @@ struct LaunchArgs {
     int accumulate;               // bit 0: C += result instead of C = result; bit 1 (kStreamC): no later
                                   // launch of the run reads these rows of C again; bit 2 (kStreamSlabs):
                                   // the slabs are too large to be worth caching
-    int feat;                     // N: features computed by the launch
+    int feat;                     // N: features computed by the launch, or of a slice of them (the last may have fewer)
+    int all_feat;                 // features computed by the launch
     int ldb, ldc;                 // row strides of B and C in elements (N, or more for a feature window)
     int coop_slots;               // source rows of more slab slots are reduced by whole workgroups
     const void* B;
     float* C;
     unsigned long long b_bytes;   // from B to the end of the matrix
-    int lg_slices;                // 2^lg_slices feature slices of `feat` features: XCD x computes slice x mod 2^lg_slices
     int slice_heavy;              // heavy rows and partial values of a slice
     long long slice_partials;
     float* partials;
@@ -469,31 +469,118 @@ inline int feature_shape(int feat, int dtype, int* lpr, int* ch) {
     return LF_OK;
 }
 
-// Feature slices: XCD x computes slice x mod S of the features for every (8 / S)-th part of the rows, so that its L2
-// has 1 / S of B to hold instead of all of it, at the price of reading the entries S times.  A slice is
-// 128 bytes or a multiple: a gather of 64 moves the line all the same (a table in the L2s is gathered from at 28 TB/s
-// by rows of 128 bytes and more, 15.5 by rows of 64).  The S of the least price in us: gathers that hit an L2 at 27
-// TB/s, those that miss and the entries at 7.15 (misses of 128 bytes 9 % slower), the share that hits from the slice's
-// size against 5 MB and from how often an XCD uses a row of B (the first use misses); `adjust` adds what else S changes.
+// Feature slices: the features are cut into S slices, and the work - all tiles for the first slice, then all tiles for the
+// second, .. - into a part for each XCD, so that an L2 has 1 / S of B to hold at a time instead of all of it, at the
+// price of reading the entries S times.  A slice is 128 bytes or a multiple: a gather of 64 moves the line all the same
+// (a table in the L2s is gathered from at 28 TB/s by rows of 128 bytes and more, 15.5 by rows of 64).  The last slice may
+// be narrower, the parts weigh the same.
+// A part is [from, upto) of the tiles of `slice` and [0, next) of those of the slice behind it, in 2^-32 of the tiles: an
+// XCD has T / 8 of T pieces of 128 bytes, and only the last slice can be shorter than that.
+struct XcdPart {
+    int slice;
+    unsigned from, upto, next;
+};
+constexpr unsigned kAllTiles = 0xFFFFFFFFu;
+
+template <typename Int> __host__ __device__ inline Int tiles_before(Int n_tiles, unsigned fraction) {
+    return fraction == kAllTiles ? n_tiles : (Int)((unsigned long long)n_tiles * fraction >> 32);
+}
+
+// What the parts are made from, in eighths of half a piece: a slice's length, the last slice's, and an XCD's.  (A table of
+// the parts among a launch's arguments was 0.4 us of each product.)
+struct XcdParts {
+    int slice_len, last_len, weight, n_slices;
+    int lg_near;                                           // log2 of the XCDs that take the same tiles at a time
+    unsigned slice_inverse, last_inverse;                  // 2^32 / length, rounded up
+};
+
+// The part of XCD x.  XCDs that take the same tiles at a time are neighbours (32K rows of 32 entries, N = 192, S = 2: 78 us;
+// with slice 0 on XCDs 0 .. 3 83).
+__host__ __device__ __forceinline__ XcdPart xcd_part(const XcdParts& p, int x) {
+    if (p.n_slices == 1) return XcdPart{0, (unsigned)x << 29, x + 1 == kXcds ? kAllTiles : (unsigned)(x + 1) << 29, 0u};
+    const int place = ((x & ((1 << p.lg_near) - 1)) << (kLgXcds - p.lg_near)) + (x >> p.lg_near);
+    const int begin = place * p.weight, end = begin + p.weight;
+    const int slice = (int)((unsigned long long)begin * p.slice_inverse >> 32);
+    auto fraction = [&](int at, int of_slice) {
+        const bool last = of_slice == p.n_slices - 1;
+        const int done = at - of_slice * p.slice_len;
+        return done >= (last ? p.last_len : p.slice_len) ? kAllTiles : done * (last ? p.last_inverse : p.slice_inverse);
+    };
+    return XcdPart{slice, fraction(begin, slice), fraction(end, slice), end > (slice + 1) * p.slice_len ? fraction(end, slice + 1) : 0u};
+}
+
+struct Slices {
+    int n = 1, feat = 0;                                   // slices, and features of each but the last
+    XcdParts parts;
+};
+
+// Workgroups that a list of `n_tiles` tiles takes on an XCD
+inline long long part_tiles(const XcdParts& parts, int x, long long n_tiles) {
+    const XcdPart p = xcd_part(parts, x);
+    return tiles_before(n_tiles, p.upto) - tiles_before(n_tiles, p.from) + tiles_before(n_tiles, p.next);
+}
+
+inline int slice_step(int dtype) { return dtype == LF_DTYPE_BF16 ? 64 : 32; }
+
+// `pieces` of 128 bytes in slices of `wide` of them.  A row of a narrower last slice takes as many lanes as of the others,
+// so it counts as half way between its width and theirs: by its width alone the XCD that has it was 2.3 times behind in
+// products whose gathers hit (N = 224 in slices of 96, 96 and 32).
+inline int slices_weight(int pieces, int wide) {
+    const int n = (int)lf::ceil_div(pieces, wide);
+    return 2 * wide * (n - 1) + wide + (pieces - (n - 1) * wide);        // in half pieces
+}
+
+inline XcdParts xcd_parts(int pieces, int wide) {
+    XcdParts p;
+    p.n_slices = (int)lf::ceil_div(pieces, wide);
+    p.lg_near = lf::ilog2(p.n_slices);
+    p.weight = slices_weight(pieces, wide);
+    p.slice_len = 2 * kXcds * wide;
+    p.last_len = kXcds * p.weight - (p.n_slices - 1) * p.slice_len;
+    p.slice_inverse = (unsigned)lf::ceil_div(1ll << 32, p.slice_len);
+    p.last_inverse = (unsigned)lf::ceil_div(1ll << 32, p.last_len);
+    return p;
+}
+
+// The S of the least price in us: gathers that hit an L2 at 27 TB/s of what their lanes could take (5 % less for every
+// doubling of the sub-waves to a wavefront, which wait for the longest of their rows), those that miss and the entries at
+// 7.15 (misses of 128 bytes 9 % slower), the share that hits from the slice's size against 4.3 MB and from how often an XCD
+// uses a row of B (the first use misses, unless it meets that of another XCD: 0.4 of one); `adjust` adds what else S and the
+// sub-waves, 2^lg_subs to a wavefront, change.
 template <typename Adjust>
-inline int feature_slices(int64_t num_cols, int64_t entries, int feat, int dtype, Adjust adjust) {
-    constexpr double kL2 = 5.0e6, kHitRate = 27e6, kMissRate = 7.15e6, kMiss128 = 1.09;
-    const int elem = dtype == LF_DTYPE_BF16 ? 2 : 4, step = 128 / elem;
-    const double b_bytes = (double)num_cols * feat * elem, gathered = (double)entries * feat * elem;
-    int best = 1;
+inline Slices feature_slices(int64_t num_cols, int64_t entries, int feat, int dtype, Adjust adjust) {
+    constexpr double kL2 = 4.3e6, kHitRate = 27e6, kMissRate = 7.15e6, kMiss128 = 1.09, kFirstUse = 0.4, kPerSub = 0.05;
+    const int elem = dtype == LF_DTYPE_BF16 ? 2 : 4, step = slice_step(dtype);
+    const double gathered = (double)entries * feat * elem;
+    const bool whole = feat % step == 0;
+    const int pieces = whole ? feat / step : 1;
+    int best = pieces;
     double least = 0.0;
-    for (int s = 1; s <= kXcds && entries > 0; s *= 2) {
-        if (feat % (s * step) != 0) break;
-        const double uses = (double)entries / (double)num_cols * s / kXcds;
-        const double hit = std::min(1.0, kL2 * s / b_bytes) * std::max(0.0, 1.0 - 1.0 / uses);
-        const double miss = (1.0 - hit) / kMissRate * (feat / s == step ? kMiss128 : 1.0);
-        const double price = adjust(s, gathered * (hit / kHitRate + miss) + 8.0 * (double)entries * s / kMissRate);
-        if (s == 1 || price < least) {
+    Slices slices;
+    for (int n = 1; n <= kXcds && entries > 0; ++n) {
+        const int wide = lf::ceil_div(pieces, n), width = whole ? wide * step : feat;
+        if (lf::ceil_div(pieces, wide) != n) continue;
+        int lpr, ch;
+        if (feature_shape(width, dtype, &lpr, &ch) != LF_OK) continue;
+        // an XCD's part of a slice's tiles, of its bytes and of the lanes' (the last slice's, the longest, against the average)
+        const double weight = slices_weight(pieces, wide);
+        const double share = weight / (2.0 * wide * kXcds);
+        const double bytes = gathered * weight / (2.0 * pieces);
+        const double lanes = 16.0 * (double)entries * lpr * ch * weight / (wide + pieces - (n - 1) * wide);
+        const double uses = (double)entries / (double)num_cols * share;
+        const double hit = std::min(1.0, kL2 / ((double)num_cols * width * elem)) * std::max(0.0, 1.0 - kFirstUse / uses);
+        const double miss = (1.0 - hit) / kMissRate * (width == step ? kMiss128 : 1.0);
+        const int lg_subs = lf::ilog2(64 / lpr);
+        const double price = adjust(n, width, lg_subs, lanes * hit / kHitRate * (1.0 + kPerSub * lg_subs) + bytes * miss + 8.0 * (double)entries * n / kMissRate);
+        if (n == 1 || price < least) {
             least = price;
-            best = s;
+            best = wide;
+            slices.n = n;
         }
     }
-    return best;
+    slices.feat = whole ? best * step : feat;
+    slices.parts = xcd_parts(pieces, best);
+    return slices;
 }
 
 }  // namespace

@@ -290,6 +290,7 @@ def test_csr_product_of_short_rows(fa, torch, nr, feat, b_dtype, usual, longest)
 @pytest.mark.parametrize("nr,nc,feat,b_dtype", [
     *((nr, 3000, feat, b) for nr in (1, 7, 9, 300) for feat, b in ((32, "f32"), (64, "f32"), (96, "f32"), (128, "f32"), (256, "f32"),
                                                                    (512, "f32"), (1024, "f32"), (128, "bf16"), (256, "bf16"), (512, "bf16"))),
+    *((nr, 9001, feat, b) for nr in (7, 300) for feat, b in ((160, "f32"), (224, "f32"), (288, "f32"), (352, "f32"), (448, "bf16"))),
     (24_575, 3000, 32, "f32"), (24_576, 3000, 64, "f32"), (24_577, 3000, 256, "f32"),          # the two group sizes
     (300, 1_060_000, 1024, "f32"),                           # 4.3 GB of B: past what 32-bit offsets reach
     (40, 2_200_000, 992, "bf16"),

@@ -478,20 +478,24 @@ def sliced_matrix(rng, nr, nc):
     return MTX.from_coo(row, col, (len(deg), nc), data=rng.uniform(-1, 1, size=len(row)).astype(np.float32))
 
 
-@pytest.mark.parametrize("feat,b_dtype,nc,slices", [(32, "f32", 9001, 1), (64, "f32", 40_009, 2), (96, "f32", 40_009, 1), (128, "f32", 20_011, 4),
-                                                    (192, "f32", 40_009, 2), (256, "f32", 40_009, 8), (512, "f32", 20_011, 8),
-                                                    (1024, "f32", 9001, 8), (64, "bf16", 9001, 1), (128, "bf16", 40_009, 2),
-                                                    (512, "bf16", 40_009, 8)])
+@pytest.mark.parametrize("feat,b_dtype,nc,slices", [(32, "f32", 9001, 1), (64, "f32", 40_009, 2), (96, "f32", 40_009, 3), (128, "f32", 20_011, 4),
+                                                    (160, "f32", 40_009, 5), (192, "f32", 40_009, 6), (224, "f32", 40_009, 7),
+                                                    (256, "f32", 40_009, 8), (288, "f32", 40_009, 5), (352, "f32", 40_009, 6), (352, "f32", 9001, 3),
+                                                    (512, "f32", 20_011, 8), (1024, "f32", 9001, 8), (64, "bf16", 9001, 1), (96, "bf16", 40_009, 1),
+                                                    (128, "bf16", 40_009, 2), (320, "bf16", 40_009, 5), (512, "bf16", 40_009, 8)])
 def test_feature_slices(fa, torch, feat, b_dtype, nc, slices):
-    """XCD x computes slice x mod S of the features: every tile runs S times, each time for its part of a row of C."""
+    """The XCDs share out S slices of the features, the last one narrower where they do not come out even: every tile
+    runs S times, each time for its part of a row of C."""
     rng = np.random.default_rng(feat)
     g = sliced_matrix(rng, 5000, nc)                     # 13 divides none of the column counts
     for widths in ([[1, 2, 4, 8, 16, 32, 64, 128, 256, 512, 1024]], [[4, 16]], [[2, 8, 32, 128, 256], [16, 128]]):
         _, info = check(fa, torch, g, widths, feat, b_dtype, seed=feat)
         if len(widths) == 1:
             assert info["heavy_rows"] >= 1 and info["cleared_rows"] == 40
-            most = max(1, info["grid"] // info["tiles"])                 # (the grid is rounded up to the longest XCD)
-            assert most == slices, (info, most)
+            # the grid is rounded up to the longest XCD: with a narrower last slice the one that has most of that
+            most = max(1, info["grid"] // info["tiles"])
+            uneven = feat // (32 if b_dtype == "f32" else 64) % slices != 0
+            assert slices <= most <= slices + uneven, (info, most)
     if feat <= 512:
         check(fa, torch, g, [[1, 2, 4, 8, 16, 32, 64, 128, 256, 512, 1024]], 2 * feat, b_dtype, seed=feat, windows=2)
 
