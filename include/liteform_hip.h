@@ -155,6 +155,12 @@ int lf_search_bucket_config(const int64_t* h_stats, const int64_t* h_colhist, in
 int lf_model_spmm_ms(const int64_t* h_stats, int32_t num_parts, int32_t n_windows, int64_t num_rows,
                      int64_t num_cols, int32_t feat_size, int32_t b_dtype, double* h_ms);
 
+/* The same prediction for the kernels as they are, with the feature slices that a plan would choose
+ * (lf_model_spmm_ms is fitted to kernels that had none and is kept for its measured shapes): what
+ * the launch shape is chosen by.  Host only. */
+int lf_model_shape_ms(const int64_t* h_stats, int32_t num_parts, int32_t n_windows, int64_t num_rows,
+                      int64_t num_cols, int32_t feat_size, int32_t b_dtype, double* h_ms);
+
 /* Share of the entries of every sample_stride-th row whose column also occurs in the row
  * before it (the first 64 entries of either row): h_out = {entries in both rows, entries
  * looked at}.  Near 0 for matrices with

@@ -281,7 +281,7 @@ extern "C" int lf_search_bucket_config(const int64_t* h_stats, const int64_t* h_
 // sees launches and L2 hits: a small product takes 5.4 us where kLaunchMs alone says 29, and many partitions
 // cost less than it thinks (132K rows of 300 entries, N = 128, 8 partitions x 2 windows: 1.43 then, 1.21 ms
 // now; 233K of 490, 16 x 2: 4.49 then, 3.76 now; one partition unchanged).  It errs towards
-// fewer partitions therefore.
+// fewer partitions therefore, and predict_launch_shape goes by lf_model_shape_ms (lf_spmm.hip).
 constexpr double kHbmBytesPerPs = 5.528;
 constexpr double kMallShare = 0.5534;
 constexpr double kMallBytes = 256.0 * 1048576.0;

@@ -1318,6 +1318,8 @@ __global__ void fill_bytes_kernel(uint32_t* __restrict__ p, long long n_words, u
         p[i] = value;
 }
 
+double slices_and_subs(int slices, int lg_subs, double us) { return us + 0.5 * std::log2((double)slices) + 0.35 * lg_subs; }
+
 }  // namespace
 
 // ====================================================================================
@@ -1673,7 +1675,7 @@ int lf_spmm_create(lf_spmm_plan** out_plan, const lf_bucket_desc* h_buckets, int
                                              [&](int n, int width, int lg_subs, double us) {
             const int lanes = std::min(64, std::max(8, width / vec));
             const double steps = (double)chunk_slots * lanes / (kWG * kUnroll);
-            return us + 0.5 * std::log2((double)n) + 0.35 * lg_subs + (chains ? 0.11 * steps : 0.0);
+            return slices_and_subs(n, lg_subs, us) + (chains ? 0.11 * steps : 0.0);
         });
         plan->slices = slices.n;
         plan->parts = slices.parts;
@@ -2079,6 +2081,47 @@ int lf_spmm_create(lf_spmm_plan** out_plan, const lf_bucket_desc* h_buckets, int
     return LF_OK;
 #undef LF_TRY
 #undef LF_TRY_HIP
+}
+
+// Launch shape.  A launch (one partition, one window) takes the price of its best feature slices (feature_slices), longer
+// where the memory-side cache holds so little of the part of B that HBM is what its misses wait for, by rows of B of which a
+// window reads 256 bytes or less, and before a later partition, whose additions to C keep its stores in the caches; 5.5 TB/s
+// for the stores of C and the additions; and 7 us for a launch more.
+// Before, lf_model_spmm_ms stood here: fitted to kernels without slices it kept to few partitions.  1120 matrices of 2K to
+// 2M rows, log-normal and power-law, N = 32 .. 512, f32 and bf16, up to 32 partitions and 4 windows each timed: its pick was
+// 5.2 % above the fastest on average and more than 5 % above for 22 % of them, this one's 1.1 % (0.9 % on 725 more matrices,
+// not fitted to, where it has the fastest but for 7 % that lose more than 5 %, 25 % at worst).  2.8 % of them take 3 % longer
+// than with the pick before, at worst 26 %; the best takes half the time (73K rows of 125, N = 352: 1.63 -> 0.85 ms).  The
+// constants below are fitted to the same matrices.
+int lf_model_shape_ms(const int64_t* h_stats, int32_t num_parts, int32_t n_windows, int64_t num_rows, int64_t num_cols,
+                      int32_t feat_size, int32_t b_dtype, double* h_ms) {
+    constexpr double kMallBytes = 140e6, kFabricOverHbm = 1.3, kBytesOfC = 5.5e6, kNextUs = 7.0, kFirstUs = 4.0;
+    constexpr double kNarrow = 0.02, kNotLast = 0.05;
+    LF_REQUIRE(h_stats && h_ms, LF_ERR_INVALID, "null argument");
+    LF_REQUIRE(num_parts >= 1 && n_windows >= 1 && num_rows >= 0 && num_cols >= 1, LF_ERR_INVALID, "bad shape");
+    LF_REQUIRE(feat_size >= 1 && feat_size % n_windows == 0, LF_ERR_INVALID, "feat_size %d is not a multiple of %d windows",
+               feat_size, n_windows);
+    LF_REQUIRE(b_dtype == LF_DTYPE_F32 || b_dtype == LF_DTYPE_BF16, LF_ERR_INVALID, "unknown B dtype %d", b_dtype);
+    double nnz = 0, added = 0;                             // of all partitions; rows that a later one adds to
+    for (int p = 0; p < num_parts; ++p) {
+        for (int k = 0; k < LF_MAX_CLASSES; ++k) {
+            const int64_t* st = h_stats + ((size_t)p * LF_MAX_CLASSES + k) * LF_STATS_FIELDS;
+            nnz += (double)st[1];
+            if (p > 0) added += (double)st[2];
+        }
+    }
+    const int feat = feat_size / n_windows;
+    const double g = (double)feat * (b_dtype == LF_DTYPE_BF16 ? 2.0 : 4.0), cols = std::ceil((double)num_cols / num_parts);
+    const Slices best = feature_slices((int64_t)cols, (int64_t)(nnz / num_parts), feat, b_dtype,
+                                       [](int n, int, int lg_subs, double us) { return slices_and_subs(n, lg_subs, us); });
+    const double lg = std::log2((double)n_windows);
+    const double narrow = 1.0 + (g < 512.0 ? kNarrow * lg * lg : 0.0);
+    const double cached = std::min(1.0, kMallBytes / (cols * g)) * (1.0 - std::min(1.0, (double)num_cols / std::max(nnz, 1.0)));
+    const double hbm = std::max(1.0, (1.0 - cached) * kFabricOverHbm);
+    const double window_us = (num_parts + kNotLast * (num_parts - 1)) * best.us * narrow * hbm + num_parts * kNextUs +
+                             ((double)num_rows * feat * 4.0 + added * feat * 8.0) / kBytesOfC;
+    *h_ms = 1e-3 * (window_us * n_windows + kFirstUs - kNextUs);
+    return LF_OK;
 }
 
 int lf_spmm_info(const lf_spmm_plan* plan, int64_t* h_info) {

@@ -511,6 +511,7 @@ __host__ __device__ __forceinline__ XcdPart xcd_part(const XcdParts& p, int x) {
 
 struct Slices {
     int n = 1, feat = 0;                                   // slices, and features of each but the last
+    double us = 0.0;                                       // their price
     XcdParts parts;
 };
 
@@ -561,7 +562,10 @@ inline Slices feature_slices(int64_t num_cols, int64_t entries, int feat, int dt
         const int wide = lf::ceil_div(pieces, n), width = whole ? wide * step : feat;
         if (lf::ceil_div(pieces, wide) != n) continue;
         int lpr, ch;
-        if (feature_shape(width, dtype, &lpr, &ch) != LF_OK) continue;
+        if (width % 32 != 0 || feature_shape(width, dtype, &lpr, &ch) != LF_OK) {     // no product, but a price
+            lpr = 64;
+            ch = (int)lf::ceil_div((int64_t)width * elem, 1024);
+        }
         // an XCD's part of a slice's tiles, of its bytes and of the lanes' (the last slice's, the longest, against the average)
         const double weight = slices_weight(pieces, wide);
         const double share = weight / (2.0 * wide * kXcds);
@@ -573,7 +577,7 @@ inline Slices feature_slices(int64_t num_cols, int64_t entries, int feat, int dt
         const int lg_subs = lf::ilog2(64 / lpr);
         const double price = adjust(n, width, lg_subs, lanes * hit / kHitRate * (1.0 + kPerSub * lg_subs) + bytes * miss + 8.0 * (double)entries * n / kMissRate);
         if (n == 1 || price < least) {
-            least = price;
+            least = slices.us = price;
             best = wide;
             slices.n = n;
         }

@@ -862,12 +862,16 @@ def row_overlap_device(g, max_samples: int = 8192) -> float:
 def model_spmm_ms(stats, windows: int, num_rows: int, num_cols: int, feat_size: int, b_dtype: str = "f32") -> float:
     """Predicted milliseconds of one product for the partitions described by ``stats``
     (``bucket_statistics``) and ``windows`` feature windows (lf_model_spmm_ms; host only)."""
+    return _modelled_ms("lf_model_spmm_ms", stats, windows, num_rows, num_cols, feat_size, b_dtype)
+
+
+def _modelled_ms(model: str, stats, windows: int, num_rows: int, num_cols: int, feat_size: int, b_dtype: str) -> float:
     lib = _lib.load()
     stats = np.ascontiguousarray(stats, dtype=np.int64)
     out = C.c_double(0.0)
     dt = {"f32": _lib.LF_DTYPE_F32, "bf16": _lib.LF_DTYPE_BF16}[b_dtype]
-    _lib.check(lib.lf_model_spmm_ms(_lib.np_ptr(stats, C.c_int64), int(stats.shape[0]), int(windows), int(num_rows),
-                                    int(num_cols), int(feat_size), dt, C.byref(out)))
+    _lib.check(getattr(lib, model)(_lib.np_ptr(stats, C.c_int64), int(stats.shape[0]), int(windows), int(num_rows),
+                                   int(num_cols), int(feat_size), dt, C.byref(out)))
     return float(out.value)
 
 
@@ -898,7 +902,7 @@ def predict_launch_shape(g, feat_size: int, b_dtype: str = "f32", candidates: Se
     Inputs: the bucket statistics of every candidate partition count (one pass over the row
     pointer each, on the GPU) and the share of columns consecutive rows have in common.  A
     structured matrix (stencil, band) reads B through the L2 whatever the shape: one
-    partition, one window.  Otherwise lf_model_spmm_ms prices every candidate and
+    partition, one window.  Otherwise lf_model_shape_ms prices every candidate and
     ``pick_launch_shape`` takes the cheapest; candidates above four partitions are priced only
     for matrices that use a row of B more than eight times on average.  Costs a few
     milliseconds of GPU time at most where ``choose_launch_shape`` spends hundreds composing and
@@ -924,7 +928,7 @@ def predict_launch_shape(g, feat_size: int, b_dtype: str = "f32", candidates: Se
                 except ValueError:
                     continue
             for w in windows:
-                predicted[(p, w)] = model_spmm_ms(stats, w, rows, cols, feat_size, b_dtype)
+                predicted[(p, w)] = _modelled_ms("lf_model_shape_ms", stats, w, rows, cols, feat_size, b_dtype)
         best = pick_launch_shape(predicted)
         # a statistics pass leaves its per-partition row bounds behind for the slab builder
         # ((P + 1) x rows words each); only those of the chosen partition count are of use

@@ -198,3 +198,28 @@ def test_model_argument_errors():
         model_spmm_ms(stats, 3, 1000, 1000, 128)       # 128 features do not split into 3 windows
     with pytest.raises(ValueError):
         model_spmm_ms(stats, 1, 1000, 0, 128)
+
+
+def split_stats(rows, degree, parts):
+    """... of the same matrix in column partitions, every row with entries in each."""
+    return np.concatenate([uniform_stats(rows, max(1, degree // parts)) for _ in range(parts)])
+
+
+@pytest.mark.parametrize("rows,degree,feat,b_dtype,want", [
+    (4096, 16, 32, "f32", [(1, 1)]),                             # all of B in an L2: one launch
+    (64_000, 100, 288, "f32", [(4, 1)]),                         # measured 0.44 ms, 1 partition 0.85, 8 0.50, 16 0.66
+    (132_000, 300, 96, "f32", [(4, 1), (8, 1)]),                 # measured 0.94 and 0.89 ms, 16 partitions 0.99
+    (2_450_000, 33, 64, "f32", [(1, 1)]), (2_450_000, 33, 128, "f32", [(1, 2)]),
+    (40, 5, 40, "f32", [(1, 1)]), (40, 5, 1, "bf16", [(1, 1)]),  # no products, but a shape
+])
+def test_launch_shapes_with_feature_slices(rows, degree, feat, b_dtype, want):
+    """What lf_model_shape_ms picks where the measured shapes are far apart."""
+    from liteform_ae_amd.format_algos import _modelled_ms, _window_candidates
+    table = {(p, w): _modelled_ms("lf_model_shape_ms", split_stats(rows, degree, p), w, rows, rows, feat, b_dtype)
+             for p in (1, 2, 4, 8, 16) if p <= 4 or degree > 8 * p for w in _window_candidates(feat, b_dtype)}
+    assert all(np.isfinite(t) and t > 0 for t in table.values())
+    assert pick_launch_shape(table) in want, table
+    with pytest.raises(ValueError):
+        _modelled_ms("lf_model_shape_ms", split_stats(rows, degree, 1), 3, rows, rows, 128, b_dtype)
+    with pytest.raises(ValueError):
+        _modelled_ms("lf_model_shape_ms", split_stats(rows, degree, 1), 1, rows, 0, feat, b_dtype)
