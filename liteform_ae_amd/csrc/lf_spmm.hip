@@ -1662,8 +1662,8 @@ int lf_spmm_create(lf_spmm_plan** out_plan, const lf_bucket_desc* h_buckets, int
     // A doubling of S costs 0.5 us in rows' starts and ends, one of the sub-waves to a wavefront 0.35, and sub-waves of fewer
     // lanes are more of them to share a long row's chunk, whose chain of gathers (0.11 us a step; it overlaps with other
     // work) sets the time of small power-law products.  3900 matrices of 2K to 2M rows, log-normal and power-law, N = 32 ..
-    // 512, f32 and bf16, every S timed at the shape that predict_launch_shape gives: 0.925 of the time with S = 1 on
-    // average, 1.6 % above the best S; 3 % of them more than 3 % slower than S = 1, 30 % at worst (products of 8 to 17
+    // 512, f32 and bf16, every S timed at the shape that was picked then: 0.927 of the time with S = 1 on average,
+    // 1.6 % above the best S; 3 % of them more than 3 % slower than S = 1, 30 % at worst (products of 8 to 17
     // us with a B of 4 to 5 MB).  S that are no power of two, us, S = 1 or 2 before -> now: 32K rows of 32 entries, N = 96
     // 40.6 -> 29.6, 160 81 -> 43, 192 78 -> 50, 224 118 -> 58; 64K rows of 32, N = 224 247 -> 168, 352 393 -> 331; 64K rows of
     // 100, N = 288 in 16 partitions 825 -> 662; 132K rows of 300, N = 96 in 16 partitions 1025 -> 993, in 8 1003 -> 891.
@@ -2085,17 +2085,16 @@ int lf_spmm_create(lf_spmm_plan** out_plan, const lf_bucket_desc* h_buckets, int
 
 // Launch shape.  A launch (one partition, one window) takes the price of its best feature slices (feature_slices), longer
 // where the memory-side cache holds so little of the part of B that HBM is what its misses wait for, by rows of B of which a
-// window reads 256 bytes or less, and before a later partition, whose additions to C keep its stores in the caches; 5.5 TB/s
+// window reads 256 bytes or less, and before a later partition, whose additions to C keep its stores in the caches; 7 TB/s
 // for the stores of C and the additions; and 7 us for a launch more.
 // Before, lf_model_spmm_ms stood here: fitted to kernels without slices it kept to few partitions.  1120 matrices of 2K to
 // 2M rows, log-normal and power-law, N = 32 .. 512, f32 and bf16, up to 32 partitions and 4 windows each timed: its pick was
-// 5.2 % above the fastest on average and more than 5 % above for 22 % of them, this one's 1.1 % (0.9 % on 725 more matrices,
-// not fitted to, where it has the fastest but for 7 % that lose more than 5 %, 25 % at worst).  2.8 % of them take 3 % longer
-// than with the pick before, at worst 26 %; the best takes half the time (73K rows of 125, N = 352: 1.63 -> 0.85 ms).  The
-// constants below are fitted to the same matrices.
+// 5.2 % above the fastest on average and more than 5 % above for 22 % of them.  This one's is 0.8 % above on these and 725 more, to
+// all of which its constants are fitted, and 0.6 % on 302 that were timed afterwards, 15 % at worst.  2.5 % of the matrices take 3 %
+// longer than with the pick before, at worst 26 %; the best takes half the time (73K rows of 125, N = 352: 1.63 -> 0.85 ms).
 int lf_model_shape_ms(const int64_t* h_stats, int32_t num_parts, int32_t n_windows, int64_t num_rows, int64_t num_cols,
                       int32_t feat_size, int32_t b_dtype, double* h_ms) {
-    constexpr double kMallBytes = 140e6, kFabricOverHbm = 1.3, kBytesOfC = 5.5e6, kNextUs = 7.0, kFirstUs = 4.0;
+    constexpr double kMallBytes = 140e6, kFabricOverHbm = 1.3, kBytesOfC = 7.0e6, kNextUs = 7.0, kFirstUs = 4.0;
     constexpr double kNarrow = 0.02, kNotLast = 0.05;
     LF_REQUIRE(h_stats && h_ms, LF_ERR_INVALID, "null argument");
     LF_REQUIRE(num_parts >= 1 && n_windows >= 1 && num_rows >= 0 && num_cols >= 1, LF_ERR_INVALID, "bad shape");

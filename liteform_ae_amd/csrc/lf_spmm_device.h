@@ -545,12 +545,16 @@ inline XcdParts xcd_parts(int pieces, int wide) {
 
 // The S of the least price in us: gathers that hit an L2 at 27 TB/s of what their lanes could take (5 % less for every
 // doubling of the sub-waves to a wavefront, which wait for the longest of their rows), those that miss and the entries at
-// 7.15 (misses of 128 bytes 9 % slower), the share that hits from the slice's size against 4.3 MB and from how often an XCD
+// 7.15 (misses of 128 bytes 6 % slower), the share that hits from the slice's size against 4.3 MB and from how often an XCD
 // uses a row of B (the first use misses, unless it meets that of another XCD: 0.4 of one); `adjust` adds what else S and the
 // sub-waves, 2^lg_subs to a wavefront, change.
+// For the price that is compared with that of other partitions (us), a slice of about an L2 misses more: 20 % at 5 MB, and 10 %
+// less for a doubling of the sub-waves (233K rows of 490, N = 128, slices of 3.7 MB in 8 partitions 3.81 ms, of 1.9 in 16
+// 3.12).  Slices chosen by that price were 1 % slower on average.
 template <typename Adjust>
 inline Slices feature_slices(int64_t num_cols, int64_t entries, int feat, int dtype, Adjust adjust) {
-    constexpr double kL2 = 4.3e6, kHitRate = 27e6, kMissRate = 7.15e6, kMiss128 = 1.09, kFirstUse = 0.4, kPerSub = 0.05;
+    constexpr double kL2 = 4.3e6, kHitRate = 27e6, kMissRate = 7.15e6, kMiss128 = 1.06, kFirstUse = 0.4, kPerSub = 0.05;
+    constexpr double kSoftL2 = 5.0e6, kSoftPerSub = 0.1;
     const int elem = dtype == LF_DTYPE_BF16 ? 2 : 4, step = slice_step(dtype);
     const double gathered = (double)entries * feat * elem;
     const bool whole = feat % step == 0;
@@ -572,12 +576,18 @@ inline Slices feature_slices(int64_t num_cols, int64_t entries, int feat, int dt
         const double bytes = gathered * weight / (2.0 * pieces);
         const double lanes = 16.0 * (double)entries * lpr * ch * weight / (wide + pieces - (n - 1) * wide);
         const double uses = (double)entries / (double)num_cols * share;
-        const double hit = std::min(1.0, kL2 / ((double)num_cols * width * elem)) * std::max(0.0, 1.0 - kFirstUse / uses);
-        const double miss = (1.0 - hit) / kMissRate * (width == step ? kMiss128 : 1.0);
+        const double again = std::max(0.0, 1.0 - kFirstUse / uses), slice_bytes = (double)num_cols * width * elem;
         const int lg_subs = lf::ilog2(64 / lpr);
-        const double price = adjust(n, width, lg_subs, lanes * hit / kHitRate * (1.0 + kPerSub * lg_subs) + bytes * miss + 8.0 * (double)entries * n / kMissRate);
+        auto priced = [&](double hit, double per_sub) {
+            return adjust(n, width, lg_subs, lanes * hit / kHitRate * (1.0 + per_sub * lg_subs) +
+                                             bytes * (1.0 - hit) / kMissRate * (width == step ? kMiss128 : 1.0) +
+                                             8.0 * (double)entries * n / kMissRate);
+        };
+        const double price = priced(std::min(1.0, kL2 / slice_bytes) * again, kPerSub);
         if (n == 1 || price < least) {
-            least = slices.us = price;
+            const double held = kSoftL2 / slice_bytes;
+            least = price;
+            slices.us = priced(held / std::cbrt(1.0 + held * held * held) * again, kSoftPerSub);
             best = wide;
             slices.n = n;
         }

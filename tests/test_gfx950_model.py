@@ -207,7 +207,7 @@ def split_stats(rows, degree, parts):
 
 @pytest.mark.parametrize("rows,degree,feat,b_dtype,want", [
     (4096, 16, 32, "f32", [(1, 1)]),                             # all of B in an L2: one launch
-    (64_000, 100, 288, "f32", [(4, 1)]),                         # measured 0.44 ms, 1 partition 0.85, 8 0.50, 16 0.66
+    (64_000, 100, 288, "f32", [(4, 1), (8, 1)]),                 # measured 0.44 ms, 1 partition 0.85, 8 0.50, 16 0.66
     (132_000, 300, 96, "f32", [(4, 1), (8, 1)]),                 # measured 0.94 and 0.89 ms, 16 partitions 0.99
     (2_450_000, 33, 64, "f32", [(1, 1)]), (2_450_000, 33, 128, "f32", [(1, 2)]),
     (40, 5, 40, "f32", [(1, 1)]), (40, 5, 1, "bf16", [(1, 1)]),  # no products, but a shape
