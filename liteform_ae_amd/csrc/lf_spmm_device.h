@@ -550,7 +550,7 @@ inline XcdParts xcd_parts(int pieces, int wide) {
 // sub-waves, 2^lg_subs to a wavefront, change.
 // For the price that is compared with that of other partitions (us), a slice of about an L2 misses more: 20 % at 5 MB, and 10 %
 // less for a doubling of the sub-waves (233K rows of 490, N = 128, slices of 3.7 MB in 8 partitions 3.81 ms, of 1.9 in 16
-// 3.12).  Slices chosen by that price were 1 % slower on average.
+// 3.12).  Of slices chosen by that price, 5 % would be more than 3 % slower than S = 1, instead of 3 %.
 template <typename Adjust>
 inline Slices feature_slices(int64_t num_cols, int64_t entries, int feat, int dtype, Adjust adjust) {
     constexpr double kL2 = 4.3e6, kHitRate = 27e6, kMissRate = 7.15e6, kMiss128 = 1.06, kFirstUse = 0.4, kPerSub = 0.05;
