@@ -1513,7 +1513,6 @@ int lf_spmm_create(lf_spmm_plan** out_plan, const lf_bucket_desc* h_buckets, int
     std::vector<const int32_t*> meta((size_t)num_buckets, nullptr);
     struct ChunkCount { int chunks = 0, heavy = 0, partials = 0; };
     std::vector<ChunkCount> counts((size_t)num_buckets);
-    std::vector<int> is_multi((size_t)num_buckets, 0), has_dense((size_t)num_buckets, 0), has_wide((size_t)num_buckets, 0);
     // Chunk size of the rows that a whole workgroup reduces.  The smaller the matrix, the more a chunk's
     // chain of gathers is of the whole: short chunks; where there is work enough to hide it, longer ones
     // leave fewer partial rows.  By total slots because nothing else is known before the scan; the
@@ -1649,14 +1648,18 @@ int lf_spmm_create(lf_spmm_plan** out_plan, const lf_bucket_desc* h_buckets, int
                                                         "or a segment that is incomplete or leaves the bucket)"));
         if (f[3]) return bail(lf::fail(LF_ERR_UNSUPPORTED, "a row is split over more than %d ELL rows", (1 << (31 - kMetaLenBits)) - 1));
     }
+    auto scanned = [&](int k, int i) { return h_counters[((size_t)kScanCounters * k + i) * kCounterLine]; };
+    auto is_multi = [&](int k) { return (scanned(k, 5) & 1) != 0; };       // rows split over several ELL rows
+    auto has_dense = [&](int k) { return (scanned(k, 5) & 2) != 0; };
+    auto has_wide = [&](int k) { return (scanned(k, 5) & 4) != 0; };
     const int n_zero = *back.as<int>(o_zero);
-    std::vector<int> chosen;                               // candidates whose sample shows shared columns
+    // Candidates whose sample shows shared columns.  Neither the groups nor the cells know segments, they store every
+    // ELL row as a row of C: a bucket that holds a split row stays with the tiles.
+    std::vector<int> chosen;
     for (int k : cand) {
         const unsigned long long* c = back.as<unsigned long long>(o_sample) + 3 * k;
-        if (!is_multi[k] && c[1] > 0 && c[0] * 100 <= c[1] * kRowGroupMaxPercent) chosen.push_back(k);
+        if (!is_multi(k) && c[1] > 0 && c[0] * 100 <= c[1] * kRowGroupMaxPercent) chosen.push_back(k);
     }
-
-    auto scanned = [&](int k, int i) { return h_counters[((size_t)kScanCounters * k + i) * kCounterLine]; };
 
     // ---- Feature slices; matrices whose kernels share gathers between rows read B through the L2s as it is.
     // A doubling of S costs 0.5 us in rows' starts and ends, one of the sub-waves to a wavefront 0.35, and sub-waves of fewer
@@ -1726,10 +1729,6 @@ int lf_spmm_create(lf_spmm_plan** out_plan, const lf_bucket_desc* h_buckets, int
         counts[k].chunks = scanned(k, 0) + (plan->coop_slots <= 64 ? scanned(k, 3) : 0) + (plan->coop_slots <= 128 ? scanned(k, 4) : 0);
         counts[k].heavy = scanned(k, 1);
         counts[k].partials = scanned(k, 2);
-        const int found = scanned(k, 5);
-        is_multi[k] = found & 1;
-        has_dense[k] = (found >> 1) & 1;
-        has_wide[k] = (found >> 2) & 1;
     }
     // ---- chunk tables, heavy-row table (grouped by bucket, hence by partition) and partial rows
     std::vector<Chunk*> d_chunks((size_t)num_buckets, nullptr);
@@ -1761,7 +1760,7 @@ int lf_spmm_create(lf_spmm_plan** out_plan, const lf_bucket_desc* h_buckets, int
         LF_TRY_HIP(hipGetLastError());
     }
     for (int k = 0; k < num_buckets; ++k) {
-        if (!has_dense[k] || counts[k].chunks == 0) continue;
+        if (!has_dense(k) || counts[k].chunks == 0) continue;
         // The chunks of dense rows go behind the others, in column order (ties: by row, so
         // the order is the same in every plan): some thousands of records, sorted on the host.
         std::vector<Chunk> h_chunks((size_t)counts[k].chunks);
@@ -1916,7 +1915,7 @@ int lf_spmm_create(lf_spmm_plan** out_plan, const lf_bucket_desc* h_buckets, int
         }
         const bool c_fits_l2 = (long long)num_rows * plan->window * 4 <= kL2Bytes;
         L.stream_c = rows_wide * 2 >= rows_all || (b_dtype == LF_DTYPE_F32 && !c_fits_l2);
-        for (int k : mine) L.wide_rows = L.wide_rows || has_wide[k];
+        for (int k : mine) L.wide_rows = L.wide_rows || has_wide(k);
         L.heavy_begin = mine.empty() ? 0 : heavy_base[mine.front()];
         L.n_heavy = mine.empty() ? 0 : heavy_base[mine.back() + 1] - L.heavy_begin;
         for (int k : mine) {
@@ -1940,7 +1939,7 @@ int lf_spmm_create(lf_spmm_plan** out_plan, const lf_bucket_desc* h_buckets, int
             g.log_w = lf::ilog2(b.width);
             const int fit = tile_slots(lpr, plan->resident && b_dtype == LF_DTYPE_F32) >> g.log_w;   // ELL rows whose slots fit the LDS tile
             const bool staged = fit >= sw;
-            g.type = staged ? (is_multi[k] ? kEllSeg : kEll) : kSeg;
+            g.type = staged ? (is_multi(k) ? kEllSeg : kEll) : kSeg;
             g.rows_per_tile = staged ? std::min(kTileRows, fit) : kSegRows;
             if (staged) {
                 // a small bucket is cut into more, shorter tiles so that it still spreads over

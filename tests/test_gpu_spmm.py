@@ -466,6 +466,28 @@ def test_rows_sharing_columns_are_served_in_groups(fa, torch, feat, b_dtype, mon
     assert info["row_group_buckets"] == 0
 
 
+@pytest.mark.parametrize("feat,b_dtype,windows", [(32, "f32", 1), (64, "f32", 1), (128, "f32", 1), (256, "f32", 1), (512, "f32", 2),
+                                                  (128, "bf16", 1), (256, "bf16", 1)])
+def test_split_rows_that_share_columns(fa, torch, feat, b_dtype, windows):
+    """Bands with a few rows wider than the widest bucket: the pieces of such a row share their columns with the
+    neighbours like everything else there, but they are one row of C."""
+    rng = np.random.default_rng(40 + feat)
+    for n, lengths, few, width in ((8000, (20, 31), 40, 32), (5003, (50, 61), 80, 64), (8000, (21, 22), 40, 32)):
+        deg = rng.integers(*lengths, size=n)
+        deg[rng.choice(n - 100, size=60, replace=False) + 50] = few
+        row = np.repeat(np.arange(n), deg)
+        at = np.arange(len(row)) - (np.cumsum(deg) - deg)[row]
+        col = np.clip(np.arange(n) - deg // 2, 0, n - deg)[row] + at
+        g = MTX.from_coo(row, col, (n, n), data=rng.uniform(-1, 1, size=len(row)).astype(np.float32))
+        assert fa.search_bucket_config(g, 1, fa.CostModelSettings(feat, 1)) == [[width]]       # as the package's own search has it
+        _, info = check(fa, torch, g, [[width]], feat, b_dtype, seed=feat, windows=windows)
+        assert info["row_group_buckets"] == 0 and info["cell_buckets"] == 0
+        _, info = check(fa, torch, g, [[width // 2, width], [width]], feat, b_dtype, seed=feat, windows=windows)
+        assert info["row_group_buckets"] == 0
+        _, info = check(fa, torch, g, [[width, 2 * width]], feat, b_dtype, seed=feat, windows=windows)
+        assert info["row_group_buckets"] >= 1                                  # the bucket without split rows shares its gathers
+
+
 def sliced_matrix(rng, nr, nc):
     """Rows of every kind that a plan treats in its own way, in mixed order: empty, 1..64 entries, 65..256 in such
     numbers that wavefronts take them (more than 1024 above 64 entries, more than 2048 above 128), and a few
