@@ -250,10 +250,39 @@ def test_triplets_through_bins_of_rows(fa, name, twice):
     if twice == "none":
         np.testing.assert_array_equal(got.view(np.int32), want.data.astype(np.float32).view(np.int32))
     else:
-        # float32 sums of up to 310 values below 1 in some order: 310 roundings of partial sums below 310
-        np.testing.assert_allclose(got, want.data, rtol=0, atol=310 * 2.0 ** -24 * (310 if twice == "many" else 4))
+        # the shapes of the library's sort: float32 sums in some order, a rounding of at most the sum of the magnitudes
+        # for each addition; the others: sums in 64 bits, rounded once
+        of_size = sp.coo_matrix((np.abs(val).astype(np.float64), (row, col)), shape=shape).tocsr()
+        times = sp.coo_matrix((np.ones(len(val)), (row, col)), shape=shape).tocsr()
+        of_size.sort_indices()
+        times.sort_indices()
+        in_float = name in ("a row past the limit", "few entries", "wide keys", "giant rows")      # (the last: 32,768 and a tenth again)
+        bound = (times.data - 1) * 2.0 ** -24 * of_size.data if in_float else 2.0 ** -24 * np.abs(want.data) + 2.0 ** -52 * times.data * of_size.data
+        assert (np.abs(got - want.data) <= bound).all()
     again = fa._DeviceCSR(MTX.from_coo(row, col, shape, data=val))
     assert np.array_equal(again.values.cpu().numpy().view(np.int32), got.view(np.int32))        # run to run the same bits
+
+
+@pytest.mark.parametrize("times", [2, 3, 17, 18, 27, 64, 81, 300, 4000, 8000])
+def test_sums_of_triplets_of_one_place(fa, times):
+    """Sums of 2 to 8000 triplets are at most one rounding off, in whatever order they come: the entries of
+    several places, beside each other and with the last one of the matrix among them."""
+    from liteform_ae_amd.format_matrix_market import MTX
+    rng = np.random.default_rng(times)
+    rows, cols = 400, 300
+    places = np.unique(np.concatenate([rng.choice(rows * cols, size=max(1, 8000 // times), replace=False), [rows * cols - 1]]))
+    once = np.setdiff1d(rng.choice(rows * cols, size=900, replace=False), places)
+    key = np.concatenate([np.repeat(places, times), once])
+    val = rng.uniform(-1, 1, size=len(key)).astype(np.float32)
+    order = rng.permutation(len(key))
+    dev = fa._DeviceCSR(MTX.from_coo((key // cols)[order].astype(np.int32), (key % cols)[order].astype(np.int32), (rows, cols), data=val[order]))
+    assert dev.nnz == len(places) + len(once)
+    got = dev.values.cpu().numpy().astype(np.float64)
+    at = np.searchsorted(np.sort(np.concatenate([places, once])), places)
+    sums = val[:len(places) * times].astype(np.float64).reshape(len(places), times)
+    want, of_size = sums.sum(1), np.abs(sums).sum(1)
+    # rounded once to 24 bits; either sum of `times` values in 53 bits
+    assert (np.abs(got[at] - want) <= 2.0 ** -24 * np.abs(want) + 2.0 ** -52 * times * of_size).all()
 
 
 def test_canonical_csr_input_goes_in_as_it_is(fa):
