@@ -350,6 +350,7 @@ int lf_csr_spmm_trusted_nnz(const int32_t* d_indptr, const int32_t* d_indices, c
  * CSR request (format_matrix_market.py:74-76).  d_coo_val NULL = all ones (the reference's
  * matrices, format_matrix_market.py:54, 63-64).  Outputs: d_indptr [num_rows + 1], d_indices
  * and d_values with room for nnz entries; *h_nnz_out = entries left after merging duplicates.
+ * d_indices and d_values may be the triplets' own arrays (d_coo_col, d_coo_val).
  * Synchronises the stream. */
 size_t lf_coo_to_csr_workspace_bytes(int64_t nnz, int64_t num_rows, int64_t num_cols);
 int lf_coo_to_csr(const int32_t* d_coo_row, const int32_t* d_coo_col, const float* d_coo_val, int64_t nnz,

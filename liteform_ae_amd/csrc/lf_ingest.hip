@@ -632,6 +632,10 @@ hipError_t ingest_layout(long long nnz, int key_bits, IngestLayout* L) {
     return hipSuccess;
 }
 
+bool overlap(const void* a, size_t a_bytes, const void* b, size_t b_bytes) {
+    return a && b && (uintptr_t)a < (uintptr_t)b + b_bytes && (uintptr_t)b < (uintptr_t)a + a_bytes;
+}
+
 int key_bits_for(long long rows, long long cols) {
     const unsigned long long top = (unsigned long long)rows * (unsigned long long)cols;
     int bits = 1;
@@ -710,7 +714,12 @@ int lf_coo_to_csr(const int32_t* d_coo_row, const int32_t* d_coo_col, const floa
                workspace_bytes, L.total);
     char* ws = (char*)d_workspace;
     const BinShape b = bin_shape(nnz, num_rows, num_cols);
-    if (b.bins > 0 && workspace_bytes >= b.total) {
+    // The bins write the results before it is known whether the triplets have to be read again; the sort does not.
+    bool in_place = false;
+    for (const void* in : {(const void*)d_coo_row, (const void*)d_coo_col, (const void*)d_coo_val})
+        in_place = in_place || overlap(in, (size_t)nnz * 4, d_indices, (size_t)nnz * 4) || overlap(in, (size_t)nnz * 4, d_values, (size_t)nnz * 4) ||
+                   overlap(in, (size_t)nnz * 4, d_indptr, (size_t)(num_rows + 1) * 4);
+    if (b.bins > 0 && workspace_bytes >= b.total && !in_place) {
         int *counts = (int*)(ws + b.counts), *totals = (int*)(ws + b.totals), *bases = (int*)(ws + b.bases);
         int *list = (int*)(ws + b.list), *flags = (int*)(ws + b.flags);
         uint2* records = (uint2*)(ws + b.records);

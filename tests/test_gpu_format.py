@@ -263,6 +263,33 @@ def test_triplets_through_bins_of_rows(fa, name, twice):
     assert np.array_equal(again.values.cpu().numpy().view(np.int32), got.view(np.int32))        # run to run the same bits
 
 
+@pytest.mark.parametrize("name", ["n=4097", "giant rows", "a row past the limit", "crowded columns", "long bins", "few entries"])
+def test_triplets_in_place(fa, name):
+    """The results in the triplets' own arrays: the same as in others, also where the bins cannot take the matrix."""
+    import ctypes as C
+    import torch
+    from liteform_ae_amd import _lib
+    row, col, shape = coo_case(name)
+    rng = np.random.default_rng(3)
+    again = rng.integers(0, len(row), size=len(row) // 10)
+    row, col = np.concatenate([row, row[again]]).astype(np.int32), np.concatenate([col, col[again]]).astype(np.int32)
+    val = rng.integers(-1000, 1000, size=len(row)).astype(np.float32)           # (sums that are exact in any order)
+    lib, n = _lib.load(), len(row)
+    nbytes = lib.lf_coo_to_csr_workspace_bytes(n, *shape)
+    ws = torch.empty(nbytes, dtype=torch.uint8, device="cuda")
+    results = []
+    for in_place in (False, True):
+        r, c, v = (torch.from_numpy(x).cuda() for x in (row, col, val))
+        indptr = torch.empty(shape[0] + 1, dtype=torch.int32, device="cuda")
+        indices, values = (c, v) if in_place else (torch.empty_like(c), torch.empty_like(v))
+        left = C.c_int64(0)
+        _lib.check(lib.lf_coo_to_csr(_lib.ptr(r), _lib.ptr(c), _lib.ptr(v), n, *shape, _lib.ptr(ws), nbytes, _lib.ptr(indptr),
+                                     _lib.ptr(indices), _lib.ptr(values), C.byref(left), None))
+        results.append([x.cpu().numpy() for x in (indptr, indices[:left.value], values[:left.value])])
+    for x, y in zip(*results):
+        np.testing.assert_array_equal(x, y)
+
+
 @pytest.mark.parametrize("times", [2, 3, 17, 18, 27, 64, 81, 300, 4000, 8000])
 def test_sums_of_triplets_of_one_place(fa, times):
     """Sums of 2 to 8000 triplets are at most one rounding off, in whatever order they come: the entries of
