@@ -63,12 +63,17 @@ __global__ void row_pointer_kernel(const unsigned long long* __restrict__ keys, 
 // A bin is 2^lg_rows consecutive rows, an entry in it one word - row in the bin, column - and its value.  Entries are
 // distributed to their bins (unordered within one), a workgroup then sorts a bin in LDS and writes its part of the
 // arrays and of the row pointer.  Bound by launches and by the latency of each kernel's two or three dependent passes.
-// With the wait for the flags, us, the library's sort with the kernels around it -> this: 6K entries 82 -> 43, 64K 80 -> 46,
-// 300K 166 -> 56, 760K of a power-law graph (a row of 13,000) 228 -> 105, 1.6M 200 -> 83, 4M 299 -> 193, 8M 590 -> 253;
-// with a duplicate 77 -> 71, 81 -> 76, 165 -> 90, 226 -> 148, 199 -> 135, 300 -> 275, 590 -> 477.  Beyond that many entries
-// bins outgrow the LDS, and the sort's few passes over memory are what counts.
-// flags: [kHard] an entry outside the matrix, a bin that does not fit or a duplicate in a very long row: the other way has
-// to be taken; [kLargeBins] bins left to bin_sort_large_kernel; [kTwice] duplicates, sorted and to be added up.
+// With the wait for the flags, us, the library's sort with the kernels around it -> this: 6K entries 65 -> 42, 64K 79 -> 45,
+// 300K 165 -> 55, 860K of a power-law graph (a row of 41,000) 234 -> 134, 1.6M 201 -> 79, 4M 350 -> 180, 7.8M 571 -> 340;
+// with a duplicate 61 -> 70, 80 -> 74, 166 -> 87, 230 -> 220, 202 -> 132, 349 -> 264, 578 -> 541.  Rows in the order of their
+// lengths, so that the first bins are large: 1.6M 204 -> 104, 4M 349 -> 213, 7.8M 573 -> 443.  Where the sort has to be
+// taken after all, counting and the wait are lost: 600K 208 -> 239, 2.4M 293 -> 338, 5M 472 -> 566, 7.6M 565 -> 666.
+// Beyond 8.4M entries bins outgrow the LDS, and the sort's few passes over memory are what counts.
+// flags: [kNotHere] an entry outside the matrix or bins of too many, known before anything is distributed, and
+// [kCrowded] a long row with too many of its columns beside each other: the other way has to be taken; [kReads] windows
+// that large bins' parts will read; [kLargeParts] parts left to bin_sort_large_kernel; [kTwice] duplicates, sorted and
+// to be added up.
+constexpr int kNotHere = 0, kReads = 1, kCrowded = 2, kLargeParts = 3, kTwice = 4, kFlags = 5;
 constexpr int kBinThreads = 512;
 constexpr int kBinChunk = 4096;            // entries that a workgroup distributes at least
 constexpr int kBinMaxChunks = 1024;
@@ -79,12 +84,17 @@ constexpr int kBinLgRows = 9;              // rows of a bin: the same
 constexpr int kBinFew = 128, kBinUsual = 1024;     // entries in a bin on average: the first up to kBinUsual bins, then the
 constexpr int kBinTargetMost = 2048;               // second, and this at most
 constexpr int kBinSmall = 4096;            // entries sorted in 48 KB of LDS
-constexpr int kBinLarge = 8192;            // ... in 96 KB, and again for every part of a row of up to kGiantMost
+constexpr int kBinLarge = 8192;            // ... in 96 KB, a part of a larger bin at a time
+constexpr int kBinWindow = kBinLarge / 2;  // parts of a large bin: every kBinWindow entries
+// Each part reads all of its bin: windows of a bin at most, and windows read in all for every kBinWindow entries of the
+// matrix, beyond one bin of the most.  Us, the library's sort -> with such bins: 520K entries, 120K of them in
+// one bin 190 -> 203; 7.8M, 1.2 windows read for each 570 -> 442; 7.6M in 60 bins of 120K, 29 for each 562 -> 1393.
+constexpr int kBinMostWindows = 32, kBinReadsMost = 6;
 constexpr int kBinLargeBytes = 3 * 4 * kBinLarge;
-constexpr int kBinLargeGrid = 64;
+constexpr int kBinLargeGrid = 256;
 
 struct BinShape {
-    int lg_rows, lg_cols, bins, chunks, per_chunk;     // bins == 0: too large, or more than 32 bits to an entry
+    int lg_rows, lg_cols, bins, chunks, per_chunk, most_reads;     // bins == 0: too large, or more than 32 bits to an entry
     size_t counts, totals, bases, list, flags, records, twice, before, partial, total;
 };
 
@@ -99,12 +109,13 @@ BinShape bin_shape(long long nnz, long long rows, long long cols) {
     b.bins = (int)((rows + (1ll << b.lg_rows) - 1) >> b.lg_rows);
     b.per_chunk = (int)align_up((size_t)std::max<long long>(kBinChunk, (nnz + kBinMaxChunks - 1) / kBinMaxChunks), kBinThreads);
     b.chunks = (int)((nnz + b.per_chunk - 1) / b.per_chunk);
+    b.most_reads = kBinMostWindows * kBinMostWindows + kBinReadsMost * (int)(nnz / kBinWindow);
     size_t off = 0;
     b.records = off; off += align_up((size_t)nnz * 8, 256);
     b.counts = off; off += align_up((size_t)b.bins * b.chunks * 4, 256);
     b.totals = off; off += align_up((size_t)b.bins * 4, 256);
     b.bases = off; off += align_up((size_t)b.bins * 4, 256);
-    b.list = off; off += align_up((size_t)b.bins * 4, 256);
+    b.list = off; off += align_up((size_t)(nnz / kBinWindow + b.bins) * 4, 256);
     b.flags = off; off += 256;
     b.twice = off; off += align_up((size_t)nnz * 4, 256);
     b.before = off; off += align_up((size_t)(nnz + 1) * 4, 256);
@@ -159,14 +170,14 @@ bin_count_kernel(const int32_t* __restrict__ row, const int32_t* __restrict__ co
         bad |= i < hi && !ok;
         count_up(s_count, r >> lg_rows, ok);
     }
-    if (__ballot(bad) != 0 && (threadIdx.x & 63) == 0) flags[0] = 1;
+    if (__ballot(bad) != 0 && (threadIdx.x & 63) == 0) flags[kNotHere] = 1;
     __syncthreads();
     for (int i = threadIdx.x; i < bins; i += kBinThreads) counts[(size_t)i * gridDim.x + blockIdx.x] = s_count[i];
 }
 
 // A wavefront to a bin: its counts become the chunks' offsets in it, totals[bin] their sum.
 __global__ void __launch_bounds__(256)
-bin_offsets_kernel(int* __restrict__ counts, int bins, int chunks, int* __restrict__ totals) {
+bin_offsets_kernel(int* __restrict__ counts, int bins, int chunks, int* __restrict__ totals, int most_reads, int* __restrict__ flags) {
     const int bin = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
     if (bin >= bins) return;
     int* mine = counts + (size_t)bin * chunks;
@@ -182,6 +193,10 @@ bin_offsets_kernel(int* __restrict__ counts, int bins, int chunks, int* __restri
         before += __shfl(incl, 63);
     }
     if (lane == 0) totals[bin] = before;
+    if (lane == 0 && before > kBinSmall) {
+        const int windows = (before + kBinWindow - 1) / kBinWindow, reads = windows * windows;
+        if (windows > kBinMostWindows || atomicAdd(&flags[kReads], reads) + reads > most_reads) flags[kNotHere] = 1;
+    }
 }
 
 // Distributes a chunk's entries.  Every workgroup scans the bins' totals for itself; the first leaves the bases.
@@ -189,11 +204,12 @@ __global__ void __launch_bounds__(kBinThreads)
 bin_distribute_kernel(const int32_t* __restrict__ row, const int32_t* __restrict__ col, const float* __restrict__ val, long long nnz,
                       long long rows, long long cols, int lg_rows, int lg_cols, int bins, int per_chunk,
                       const int* __restrict__ counts, const int* __restrict__ totals, int* __restrict__ bases,
-                      uint2* __restrict__ records) {
+                      uint2* __restrict__ records, const int* __restrict__ flags) {
     __shared__ int s_at[kBinMost];
     __shared__ int s_wave[kBinThreads / 64];
     constexpr int kPer = kBinMost / kBinThreads;           // consecutive bins of a thread
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, b0 = threadIdx.x * kPer;
+    const int not_here = flags[kNotHere];
     int sum = 0;
     for (int i = b0; i < min(b0 + kPer, bins); ++i) sum += totals[i];
     int incl = sum;
@@ -201,6 +217,7 @@ bin_distribute_kernel(const int32_t* __restrict__ row, const int32_t* __restrict
         const int y = __shfl_up(incl, d);
         if (lane >= d) incl += y;
     }
+    if (not_here) return;
     if (lane == 63) s_wave[wave] = incl;
     __syncthreads();
     int base = incl - sum;
@@ -217,7 +234,7 @@ bin_distribute_kernel(const int32_t* __restrict__ row, const int32_t* __restrict
         const long long i = i0 + threadIdx.x;
         const int r = i < hi ? row[i] : -1, c = i < hi ? col[i] : -1;
         const float v = i < hi && val ? val[i] : 1.0f;
-        const bool ok = in_matrix(r, c, rows, cols);       // (others are flagged: what is written here is not used)
+        const bool ok = in_matrix(r, c, rows, cols);       // (others are flagged, and none of this runs)
         const int at = count_up(s_at, r >> lg_rows, ok);
         if (ok) records[at] = make_uint2(((unsigned)(r & row_mask) << lg_cols) | (unsigned)c, __float_as_uint(v));
     }
@@ -251,19 +268,19 @@ struct BinSort {
 // One bin.  The rows are counted, which gives the row pointer.  A row of len entries then has len buckets, the i-th for
 // the i-th part of the columns: counting puts its entries together bucket by bucket (s_key, s_val), and an entry's
 // place follows from the few of its bucket, equal keys by value.  Where the columns of rows crowd into few buckets
-// (more than kBucketReads reads an entry) the part is sorted bitonically.  Rows of more than kGiantRow entries are
-// sorted after the others, a range of columns at a time (LARGE only; s_giant: row and offset).
+// (more than kBucketReads reads an entry) the part is sorted bitonically.
 // (Comparing an entry with its whole row: 57K rows of 28 entries 72 us for this kernel, 760K entries of a power-law
 // graph 79; so 25 and 22.)
+// LARGE: a part of a bin, the `window`-th kBinWindow of its sorted entries.  The rows that start in it and have no more than
+// that are at most 2 * kBinWindow - 1 entries.  A longer row is cut into as many ranges of columns as windows start inside
+// it, a window to a range.
 constexpr int kBinRows = 1 << kBinLgRows;
 constexpr int kBucketReads = 64;
-constexpr int kGiantRow = 1024, kGiantMost = 32768, kGiants = 256;
-constexpr int kHard = 0, kLargeBins = 1, kTwice = 2;       // flags
 template <int THREADS, int CAPACITY, bool LARGE>
-__device__ __forceinline__ void sort_bin(const BinSort& a, int bin, unsigned* s_key, unsigned* s_val, int* s_bucket, int* s_giant, int* s_wave) {
-    __shared__ int s_first[kBinRows + 1];      // of a row among the entries sorted together; a giant's: -1
+__device__ __forceinline__ void sort_bin(const BinSort& a, int bin, int window, unsigned* s_key, unsigned* s_val, int* s_bucket, int* s_wave) {
+    __shared__ int s_first[kBinRows];          // of a row in the bin; not sorted here: -1
     __shared__ int s_count[kBinRows];
-    __shared__ int s_giants, s_sorted;
+    __shared__ int s_from, s_long, s_long_at, s_before, s_sorted;
     __shared__ float s_squares;
     constexpr int kOwn = LARGE ? 16 : CAPACITY / THREADS;  // records in registers: usually all, loaded once
     const int base = a.bases[bin], n = a.totals[bin];
@@ -290,9 +307,9 @@ __device__ __forceinline__ void sort_bin(const BinSort& a, int bin, unsigned* s_
         }
     };
     auto fraction = [&](unsigned key) { return (key & col_mask) * a.inverse; };      // (below 2^32: column < columns)
-    bool twice = false, hard = false;
+    bool twice = false, crowded = false;
     // The records that `selected` takes: by bucket(key), which ascends with the key, and then in full; out(key, place)
-    // is where the place-th goes.  Their number; more than CAPACITY are too many.
+    // is where the place-th goes.  More than CAPACITY are too many.
     auto sort_part = [&](auto selected, auto bucket, auto out) {
         constexpr int kPer = CAPACITY / THREADS;
         for (int i = threadIdx.x; i < CAPACITY; i += THREADS) s_bucket[i] = 0;
@@ -321,8 +338,8 @@ __device__ __forceinline__ void sort_bin(const BinSort& a, int bin, unsigned* s_
         __syncthreads();
         const int sorted = s_sorted;
         if (sorted > CAPACITY) {
-            hard = true;
-            return sorted;
+            crowded = true;
+            return;
         }
         each([&](const uint2& x, bool in) {
             if (!in || !selected(x.x)) return;
@@ -375,71 +392,60 @@ __device__ __forceinline__ void sort_bin(const BinSort& a, int bin, unsigned* s_
                 twice |= i > 0 && s_key[i - 1] == key;
             }
         }
-        return sorted;
     };
 
     for (int r = threadIdx.x; r < n_rows; r += THREADS) s_count[r] = 0;
-    if (threadIdx.x == 0) s_giants = 0;
+    if (LARGE && threadIdx.x == 0) {
+        s_from = n;
+        s_long = -1;
+        s_before = 0;
+    }
     __syncthreads();
     each([&](const uint2& x, bool in) { count_up(s_count, (int)(x.x >> a.lg_cols), in); });
     __syncthreads();
-    // a thread's consecutive rows: offsets among all entries (the row pointer) and among those sorted together
+    // a thread's consecutive rows
     const int per = (n_rows + THREADS - 1) / THREADS, lo = min((int)threadIdx.x * per, n_rows), hi = min(lo + per, n_rows);
-    int all = 0, kept = 0;
+    int sum = 0;
+    for (int r = lo; r < hi; ++r) sum += s_count[r];
+    int at = scan_workgroup<THREADS>(sum, s_wave) - sum;
     for (int r = lo; r < hi; ++r) {
         const int len = s_count[r];
-        all += len;
-        if (!LARGE || len <= kGiantRow) kept += len;
-    }
-    int at_all = scan_workgroup<THREADS>(all, s_wave) - all, at = (LARGE ? scan_workgroup<THREADS>(kept, s_wave) : at_all + kept) - kept;
-    for (int r = lo; r < hi; ++r) {
-        const int len = s_count[r];
-        a.indptr[r0 + r] = base + at_all;
-        s_first[r] = at;
-        if (LARGE && len > kGiantRow) {
-            hard |= len > kGiantMost;
-            const int g = atomicAdd(&s_giants, 1);
-            if (g < kGiants) {
-                s_giant[2 * g] = r;
-                s_giant[2 * g + 1] = at_all;
-            }
-            s_first[r] = -1;
-        } else {
-            at += len;
+        const bool starts = !LARGE || min(at, n - 1) / kBinWindow == window;       // (empty rows behind the last entry: with it)
+        if (starts) a.indptr[r0 + r] = base + at;
+        const bool mine = starts && (!LARGE || len <= kBinWindow);
+        s_first[r] = mine ? at : -1;
+        if (LARGE && mine && len > 0) atomicMin(&s_from, at);
+        if (LARGE && len > kBinWindow && at < window * kBinWindow && at + len > window * kBinWindow) {       // one at most
+            s_long = r;
+            s_long_at = at;
         }
-        at_all += len;
+        at += len;
     }
     if (r0 + n_rows == a.rows && threadIdx.x == THREADS - 1) a.indptr[a.rows] = base + n;
-    if (LARGE && threadIdx.x == THREADS - 1) s_sorted = at;                // (behind the last row)
-    hard = __syncthreads_or(hard) != 0 || (LARGE && (s_giants > kGiants || s_sorted > CAPACITY));
-    if (!hard) {
-        sort_part([&](unsigned key) { return !LARGE || s_first[key >> a.lg_cols] >= 0; },
-                  [&](unsigned key) {
-                      const int r = (int)(key >> a.lg_cols);
-                      return s_first[r] + (int)__umulhi(fraction(key), (unsigned)s_count[r]);
-                  },
-                  [&](unsigned key, int place) {
-                      int to = base + place;
-                      if (LARGE)                           // giants before the row
-                          for (int g = 0; g < s_giants; ++g)
-                              if (s_giant[2 * g] < (int)(key >> a.lg_cols)) to += s_count[s_giant[2 * g]];
-                      return to;
-                  });
-        for (int g = 0; LARGE && g < s_giants && !hard; ++g) {
-            const unsigned row = (unsigned)s_giant[2 * g];
-            const unsigned ranges = ((unsigned)s_count[row] + (unsigned)s_count[row] / 4) / CAPACITY + 1;
-            int done = base + s_giant[2 * g + 1];
-            for (unsigned k = 0; k < ranges && !hard; ++k) {
-                __syncthreads();                           // the part before has been read out
-                auto scaled = [&](unsigned key) { return (unsigned long long)fraction(key) * ranges; };
-                done += sort_part([&](unsigned key) { return key >> a.lg_cols == row && scaled(key) >> 32 == k; },
-                                  [&](unsigned key) { return (int)__umulhi((unsigned)scaled(key), CAPACITY); },
-                                  [&](unsigned, int place) { return done + place; });
-            }
-        }
+    __syncthreads();
+    const int first = LARGE ? s_from : 0;                  // in the bin, of what is sorted together
+    sort_part([&](unsigned key) { return !LARGE || s_first[key >> a.lg_cols] >= 0; },
+              [&](unsigned key) {
+                  const int r = (int)(key >> a.lg_cols);
+                  return s_first[r] - first + (int)__umulhi(fraction(key), (unsigned)s_count[r]);
+              },
+              [&](unsigned, int place) { return base + first + place; });
+    if (LARGE && s_long >= 0) {
+        const unsigned row = (unsigned)s_long;
+        const int row_at = s_long_at;
+        __syncthreads();                                   // the rows have been read out
+        const unsigned before = (unsigned)(row_at / kBinWindow) + 1, k = (unsigned)window - before;
+        const unsigned ranges = (unsigned)((row_at + s_count[row] - 1) / kBinWindow) + 1 - before;
+        auto scaled = [&](unsigned key) { return (unsigned long long)fraction(key) * ranges; };
+        int lower = 0;
+        each([&](const uint2& x, bool in) { lower += in && x.x >> a.lg_cols == row && scaled(x.x) >> 32 < k; });
+        if (lower > 0) atomicAdd(&s_before, lower);
+        sort_part([&](unsigned key) { return key >> a.lg_cols == row && scaled(key) >> 32 == k; },
+                  [&](unsigned key) { return (int)__umulhi((unsigned)scaled(key), CAPACITY); },
+                  [&](unsigned, int place) { return base + row_at + s_before + place; });
     }
     if (__ballot(twice) != 0 && (threadIdx.x & 63) == 0) a.flags[kTwice] = 1;
-    if (__ballot(hard) != 0 && (threadIdx.x & 63) == 0) a.flags[kHard] = 1;
+    if (__ballot(crowded) != 0 && (threadIdx.x & 63) == 0) a.flags[kCrowded] = 1;
 }
 
 __global__ void __launch_bounds__(kBinThreads)
@@ -447,22 +453,30 @@ bin_sort_kernel(BinSort a) {
     __shared__ unsigned s_key[kBinSmall], s_val[kBinSmall];
     __shared__ int s_bucket[kBinSmall];
     __shared__ int s_wave[kBinThreads / 64];
-    if (a.totals[blockIdx.x] > kBinSmall) {
-        if (threadIdx.x == 0) a.list[atomicAdd(&a.flags[kLargeBins], 1)] = blockIdx.x;
+    const int n = a.totals[blockIdx.x];
+    if (a.flags[kNotHere]) return;
+    if (n > kBinSmall) {
+        const int windows = (n + kBinWindow - 1) / kBinWindow;
+        if (threadIdx.x < 64) {
+            int at = 0;
+            if (threadIdx.x == 0) at = atomicAdd(&a.flags[kLargeParts], windows);
+            at = __builtin_amdgcn_readfirstlane(at);
+            for (int i = threadIdx.x; i < windows; i += 64) a.list[at + i] = (int)blockIdx.x | i * kBinMost;
+        }
         return;
     }
-    sort_bin<kBinThreads, kBinSmall, false>(a, blockIdx.x, s_key, s_val, s_bucket, nullptr, s_wave);
+    sort_bin<kBinThreads, kBinSmall, false>(a, blockIdx.x, 0, s_key, s_val, s_bucket, s_wave);
 }
 
 __global__ void __launch_bounds__(1024)
 bin_sort_large_kernel(BinSort a) {
     extern __shared__ unsigned s_large[];                  // [3][kBinLarge]: keys, values, buckets
-    __shared__ int s_giant[2 * kGiants];
     __shared__ int s_wave[16];
-    const int n = a.flags[kLargeBins];
+    const int n = a.flags[kLargeParts];
     for (int i = blockIdx.x; i < n; i += gridDim.x) {
-        __syncthreads();                                   // the bin before has been read out
-        sort_bin<1024, kBinLarge, true>(a, a.list[i], s_large, s_large + kBinLarge, (int*)(s_large + 2 * kBinLarge), s_giant, s_wave);
+        const int item = a.list[i];
+        __syncthreads();                                   // the part before has been read out
+        sort_bin<1024, kBinLarge, true>(a, item % kBinMost, item / kBinMost, s_large, s_large + kBinLarge, (int*)(s_large + 2 * kBinLarge), s_wave);
     }
 }
 
@@ -726,21 +740,25 @@ int lf_coo_to_csr(const int32_t* d_coo_row, const int32_t* d_coo_col, const floa
         const unsigned inverse = (unsigned)std::min<unsigned long long>((1ull << 32) / (unsigned long long)num_cols, 0xFFFFFFFFull);
         const BinSort sort{records, bases, totals, num_rows, b.lg_rows, b.lg_cols, inverse, d_indptr, d_indices, d_values, list, flags};
         LF_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(bin_sort_large_kernel), hipFuncAttributeMaxDynamicSharedMemorySize, kBinLargeBytes));
-        clear_words_kernel<<<1, 64, 0, s>>>(flags, 3);
+        clear_words_kernel<<<1, 64, 0, s>>>(flags, kFlags);
         bin_count_kernel<<<b.chunks, kBinThreads, 0, s>>>(d_coo_row, d_coo_col, nnz, num_rows, num_cols, b.lg_rows, b.bins, b.per_chunk, counts, flags);
-        bin_offsets_kernel<<<(b.bins + 3) / 4, 256, 0, s>>>(counts, b.bins, b.chunks, totals);
+        bin_offsets_kernel<<<(b.bins + 3) / 4, 256, 0, s>>>(counts, b.bins, b.chunks, totals, b.most_reads, flags);
         bin_distribute_kernel<<<b.chunks, kBinThreads, 0, s>>>(d_coo_row, d_coo_col, d_coo_val, nnz, num_rows, num_cols, b.lg_rows, b.lg_cols, b.bins,
-                                                               b.per_chunk, counts, totals, bases, records);
+                                                               b.per_chunk, counts, totals, bases, records, flags);
         bin_sort_kernel<<<b.bins, kBinThreads, 0, s>>>(sort);
-        bin_sort_large_kernel<<<std::min(b.bins, kBinLargeGrid), 1024, kBinLargeBytes, s>>>(sort);
+        if (nnz > kBinSmall) {
+            const unsigned grid = (unsigned)std::min<long long>(nnz / kBinWindow + b.bins, kBinLargeGrid);
+            bin_sort_large_kernel<<<grid, 1024, kBinLargeBytes, s>>>(sort);
+        }
         LF_HIP(hipGetLastError());
-        int h_flags[3] = {0, 0, 0};
+        int h_flags[kFlags] = {};
         LF_HIP(lf::read_back(h_flags, flags, sizeof(h_flags), s));
-        if (h_flags[kHard] == 0 && h_flags[kTwice] == 0) {
+        const bool sorted = h_flags[kNotHere] == 0 && h_flags[kCrowded] == 0;
+        if (sorted && h_flags[kTwice] == 0) {
             *h_nnz_out = nnz;
             return LF_OK;
         }
-        if (h_flags[kHard] == 0) {
+        if (sorted) {
             int32_t *twice = (int32_t*)(ws + b.twice), *before = (int32_t*)(ws + b.before), *partial = (int32_t*)(ws + b.partial);
             int32_t* out_indices = (int32_t*)records;
             float* out_values = (float*)(out_indices + nnz);

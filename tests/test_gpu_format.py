@@ -210,7 +210,25 @@ def coo_case(name):
     shapes = {"giant rows": (600, 40_000, [1024, 1025, 4096, 4097, 9000, 32_768]), "a row past the limit": (40, 90_000, [32_769, 5000]),
               "crowded columns": (64, 1 << 21, [3000, 900, 2000, 1500]), "one column": (5000, 1, []), "one row": (1, 3000, [2500]),
               "few entries": (2_100_000, 50, []), "wide keys": (300_000, 1 << 23, []), "long bins": (512 * 40, 30_000, [4000] * 60)}
-    nr, nc, lens = shapes[name]
+    if name in shapes:
+        nr, nc, lens = shapes[name]
+    else:                                                  # 256 rows to a bin: what stands in the bins named
+        nr, nc = 200_000, 150_000
+        long_rows = [0, 2, 1100, 0, 3000, 1, 1025, 2048, 0, 5]
+        bins = {"adjacent long rows": {100: [*long_rows * 6, 4097, 0, 4500, 9000], 101: [1100] * 60, 781: long_rows},
+                # sums of whole windows with empty rows behind them, the last bin (64 rows) among them, and one more or less
+                "whole windows": {3: [4096], 4: [4097], 5: [4096, 4096], 6: [0, 4097, 4095], 7: [4095, 4098], 8: [8191, 1], 9: [8192], 10: [1, 8191, 0, 1],
+                                  11: [12_288, 0, 0, 1], 12: [1, 12_288], 13: [100] * 81 + [92], 14: [100] * 82, 15: [32] * 256, 781: [0, 5000, 3192]},
+                "rows by length": {i: rng.integers(max(1, 400 // (i + 1)), 500 // (i + 1) + 1, size=256) for i in range(60)},
+                "a bin of the most": {50: [70_000, 3, 0, 30_000, *[250] * 124, 69]}, "a bin past the limit": {50: [70_000, 3, 0, 30_000, *[250] * 124, 70]},
+                "a crowded long row": {50: [9000, 20]}}[name]
+        deg = np.zeros(nr, np.int64) if name == "whole windows" else (rng.random(nr) < 0.2).astype(np.int64)
+        for b, lens in bins.items():
+            deg[256 * b:256 * b + 256] = 0
+            deg[256 * b:256 * b + len(lens)] = lens
+        row = np.repeat(np.arange(nr), deg)
+        col = np.concatenate([rng.choice(10_000 if name == "a crowded long row" and d > 20 else nc, size=d, replace=False) for d in deg if d])
+        return row, col, (nr, nc)
     deg = np.minimum(rng.integers(0, 9, size=nr), nc) if nr < 1_000_000 else (rng.random(nr) < 0.01).astype(np.int64)
     deg[rng.choice(nr, size=len(lens), replace=False)] = lens
     row = np.repeat(np.arange(nr), deg)
@@ -221,10 +239,11 @@ def coo_case(name):
 
 @pytest.mark.parametrize("twice", ["none", "some", "many"])
 @pytest.mark.parametrize("name", ["n=1", "n=63", "n=4095", "n=4096", "n=4097", "n=130000", "giant rows", "a row past the limit", "crowded columns",
-                                  "one column", "one row", "few entries", "wide keys", "long bins"])
+                                  "one column", "one row", "few entries", "wide keys", "long bins", "adjacent long rows", "whole windows", "rows by length",
+                                  "a bin of the most", "a bin past the limit", "a crowded long row"])
 def test_triplets_through_bins_of_rows(fa, name, twice):
-    """Every way an entry can take: bins sorted by buckets or bitonically, large bins, rows that are sorted a range of
-    columns at a time, rows and bins past the limits, shapes that are left to the library's sort; without
+    """Every way an entry can take: bins sorted by buckets or bitonically, large bins in windows, rows that are sorted a
+    range of columns at a time, bins past the limits, shapes that are left to the library's sort; without
     duplicates (the values' bits are kept, not only numbers), with some and with 300 of one entry."""
     import scipy.sparse as sp
     from liteform_ae_amd.format_matrix_market import MTX
@@ -256,14 +275,14 @@ def test_triplets_through_bins_of_rows(fa, name, twice):
         times = sp.coo_matrix((np.ones(len(val)), (row, col)), shape=shape).tocsr()
         of_size.sort_indices()
         times.sort_indices()
-        in_float = name in ("a row past the limit", "few entries", "wide keys", "giant rows")      # (the last: 32,768 and a tenth again)
+        in_float = name in ("few entries", "wide keys", "a bin of the most", "a bin past the limit", "a crowded long row")      # (most: and duplicates)
         bound = (times.data - 1) * 2.0 ** -24 * of_size.data if in_float else 2.0 ** -24 * np.abs(want.data) + 2.0 ** -52 * times.data * of_size.data
         assert (np.abs(got - want.data) <= bound).all()
     again = fa._DeviceCSR(MTX.from_coo(row, col, shape, data=val))
     assert np.array_equal(again.values.cpu().numpy().view(np.int32), got.view(np.int32))        # run to run the same bits
 
 
-@pytest.mark.parametrize("name", ["n=4097", "giant rows", "a row past the limit", "crowded columns", "long bins", "few entries"])
+@pytest.mark.parametrize("name", ["n=4097", "giant rows", "a row past the limit", "crowded columns", "long bins", "few entries", "whole windows"])
 def test_triplets_in_place(fa, name):
     """The results in the triplets' own arrays: the same as in others, also where the bins cannot take the matrix."""
     import ctypes as C

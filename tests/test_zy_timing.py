@@ -1,7 +1,8 @@
 """Timing comparisons on the GPU, kept apart from the parity tests and collected after them
 (the file name sorts behind every other test file except the no-allocation entry point's):
-the launch shape the model picks against its measured competitors, and a bucket-width fold
-the MI355X cost model asks for against the unfolded widths.
+the launch shape the model picks against its measured competitors, a bucket-width fold
+the MI355X cost model asks for against the unfolded widths, and triplets whose long rows are
+neighbours against as many of even rows.
 
 Every comparison interleaves the candidates (A, B, C, A, B, C, ...) and compares medians, so
 that a slow or noisy box scales all of them alike; the bounds are far above the 8 % spread seen
@@ -88,3 +89,39 @@ def test_a_folded_choice_against_the_initial_widths():
     assert ms["folded"] <= 1.25 * ms["initial"], ms
     # same product either way (a row's terms are added in the same order, in pieces of 16 or 64)
     assert float((outs["folded"] - outs["initial"]).abs().max()) <= 1e-4
+
+
+def test_triplets_of_neighbouring_long_rows():
+    """20 neighbouring rows of 20,000 among rows of 2: sorting takes some times as long as the same number of triplets in
+    even rows (240 and 65 us) at most, not with every long row reading all of them again (10 ms)."""
+    import ctypes as C
+    import time
+    import torch
+    from liteform_ae_amd import _lib
+    lib, rng = _lib.load(), np.random.default_rng(20)
+    nr = nc = 100_000
+    long_rows = np.full(nr, 2)
+    long_rows[5000:5020] = 20_000
+    inputs = {}
+    for name, deg in (("long", long_rows), ("even", np.full(nr, 6))):
+        row = np.repeat(np.arange(nr), deg)
+        col = (rng.integers(nc, size=nr)[row] + 61_803 * (np.arange(len(row)) - np.repeat(np.cumsum(deg) - deg, deg))) % nc     # (gcd 1)
+        order = rng.permutation(len(row))
+        n, (row, col) = len(row), (torch.from_numpy(x[order].astype(np.int32)).cuda() for x in (row, col))
+        nbytes = lib.lf_coo_to_csr_workspace_bytes(n, nr, nc)
+        inputs[name] = (n, row, col, torch.empty(nbytes, dtype=torch.uint8, device="cuda"), torch.empty(nr + 1, dtype=torch.int32, device="cuda"),
+                        torch.empty(n, dtype=torch.int32, device="cuda"), torch.empty(n, dtype=torch.float32, device="cuda"))
+    ms = {name: [] for name in inputs}
+    for i in range(2 + 2 * ROUNDS):
+        for name, (n, row, col, ws, indptr, indices, values) in inputs.items():
+            left = C.c_int64(0)
+            torch.cuda.synchronize()
+            t = time.perf_counter()
+            _lib.check(lib.lf_coo_to_csr(_lib.ptr(row), _lib.ptr(col), None, n, nr, nc, _lib.ptr(ws), ws.numel(), _lib.ptr(indptr),
+                                         _lib.ptr(indices), _lib.ptr(values), C.byref(left), None))
+            if i >= 2:
+                ms[name].append(1e3 * (time.perf_counter() - t))
+            assert left.value == n
+    ms = {name: float(np.median(v)) for name, v in ms.items()}
+    print(f"\ntriplets: {ms}")
+    assert ms["long"] <= 12 * ms["even"], ms
