@@ -326,6 +326,11 @@ int lf_spmm_time_ms(lf_spmm_plan* plan, const void* d_B, float* d_C, int32_t war
 int lf_csr_check(const int32_t* d_indptr, const int32_t* d_indices, const float* d_values,
                  int64_t num_rows, int64_t num_cols, int64_t nnz, void* d_scratch, int32_t* h_flags,
                  lf_stream_t stream);
+/* The same, and *h_span (optional) receives how many columns four neighbouring rows span, on average over a sample:
+ * small for stencils and bands, next to num_cols for a random graph; 0 where the columns are not sorted or there are none. */
+int lf_csr_check_span(const int32_t* d_indptr, const int32_t* d_indices, const float* d_values,
+                      int64_t num_rows, int64_t num_cols, int64_t nnz, void* d_scratch, int32_t* h_flags,
+                      int64_t* h_span, lf_stream_t stream);
 
 /* Row-parallel CSR SpMM, the counterpart of bench_naive's kernel
  * (format_algos.py:1689-1755): C = A_csr . B with float32 values (NULL = ones).
@@ -334,7 +339,8 @@ int lf_csr_check(const int32_t* d_indptr, const int32_t* d_indices, const float*
  * they fail.  lf_csr_spmm_trusted is the same product without the check, for arrays that
  * lf_csr_check has accepted or that lf_coo_to_csr produced: it only enqueues the kernel.
  * lf_csr_spmm_trusted_nnz is told the number of entries, which helps it choose how the features
- * are split over the XCDs (0: unknown). */
+ * are split over the XCDs (0: unknown), and lf_csr_spmm_trusted_span the columns that neighbouring rows span as well
+ * (lf_csr_check_span; 0: unknown), which change the split where they are few. */
 int lf_csr_spmm(const int32_t* d_indptr, const int32_t* d_indices, const float* d_values,
                 int64_t num_rows, int64_t num_cols, int64_t nnz, int32_t feat_size, int32_t b_dtype,
                 const void* d_B, float* d_C, void* d_scratch, lf_stream_t stream);
@@ -344,6 +350,9 @@ int lf_csr_spmm_trusted(const int32_t* d_indptr, const int32_t* d_indices, const
 int lf_csr_spmm_trusted_nnz(const int32_t* d_indptr, const int32_t* d_indices, const float* d_values,
                             int64_t num_rows, int64_t num_cols, int64_t nnz, int32_t feat_size,
                             int32_t b_dtype, const void* d_B, float* d_C, lf_stream_t stream);
+int lf_csr_spmm_trusted_span(const int32_t* d_indptr, const int32_t* d_indices, const float* d_values,
+                             int64_t num_rows, int64_t num_cols, int64_t nnz, int64_t span, int32_t feat_size,
+                             int32_t b_dtype, const void* d_B, float* d_C, lf_stream_t stream);
 
 /* COO -> canonical CSR on the GPU: entries sorted by (row, column), duplicates added up,
  * row pointer built - what the reference's container does with scipy's coo.tocsr() on every

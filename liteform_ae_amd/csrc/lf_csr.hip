@@ -152,8 +152,8 @@ CsrFn csr_kernel(int lpr, int ch, int dtype, bool wide) {
 // timed: the pick takes 0.89 of the time of S = 1 on average, 2.6 % more than the best; 3 % of them are more than 3 % slower
 // than with S = 1, 21 % at worst (25K rows of 4, N = 160: 12.9 us, 15.6 with 5).  128K rows of 100, N = 96: 635 us with 1,
 // 564 with 3.
-Slices csr_slices(int64_t rows, int64_t groups, int64_t num_cols, int64_t nnz, int feat, int dtype) {
-    return feature_slices(num_cols, nnz, feat, dtype, [&](int s, int width, int lg_subs, double us) {
+Slices csr_slices(int64_t rows, int rows_per_group, int64_t groups, int64_t num_cols, int64_t nnz, int64_t span, int feat, int dtype) {
+    return feature_slices(num_cols, nnz, feat, dtype, Neighbours{(double)span, rows}, [&](int) { return (double)rows_per_group; }, [&](int s, int width, int lg_subs, double us) {
         return us * (1.0 + 0.16 * std::max(0.0, std::log2(2048.0 / ((double)groups * s))))
                   * (width * (dtype == LF_DTYPE_BF16 ? 2 : 4) > 512 ? 1.04 : 1.0) * (1.0 + 0.02 * std::log2((double)s))
                + 0.3 * lg_subs + 7e-6 * (double)rows * s;
@@ -164,9 +164,9 @@ Slices csr_slices(int64_t rows, int64_t groups, int64_t num_cols, int64_t nnz, i
 
 extern "C" {
 
-int lf_csr_spmm_trusted_nnz(const int32_t* d_indptr, const int32_t* d_indices, const float* d_values,
-                            int64_t num_rows, int64_t num_cols, int64_t nnz, int32_t feat_size, int32_t b_dtype,
-                            const void* d_B, float* d_C, lf_stream_t stream) {
+int lf_csr_spmm_trusted_span(const int32_t* d_indptr, const int32_t* d_indices, const float* d_values,
+                             int64_t num_rows, int64_t num_cols, int64_t nnz, int64_t span, int32_t feat_size,
+                             int32_t b_dtype, const void* d_B, float* d_C, lf_stream_t stream) {
     LF_REQUIRE(num_rows >= 0 && num_rows < (1ll << 31) && num_cols >= 1, LF_ERR_INVALID, "bad shape");
     if (num_rows == 0) return LF_OK;
     LF_REQUIRE(d_indptr && d_B && d_C, LF_ERR_INVALID, "null argument");
@@ -177,7 +177,7 @@ int lf_csr_spmm_trusted_nnz(const int32_t* d_indptr, const int32_t* d_indices, c
     CsrArgs a{};
     a.rows_per_group = num_rows >= kCsrManyRows ? kCsrRowsMany : kCsrRowsFew;
     a.n_groups = lf::ceil_div(num_rows, (int64_t)a.rows_per_group);
-    const Slices slices = csr_slices(num_rows, a.n_groups, num_cols, nnz, feat_size, b_dtype);
+    const Slices slices = csr_slices(num_rows, a.rows_per_group, a.n_groups, num_cols, nnz, span, feat_size, b_dtype);
     a.feat = slices.feat;
     a.parts = slices.parts;
     if (int rc = feature_shape(a.feat, b_dtype, &lpr, &ch)) return rc;
@@ -195,6 +195,12 @@ int lf_csr_spmm_trusted_nnz(const int32_t* d_indptr, const int32_t* d_indices, c
     csr_kernel(lpr, ch, b_dtype, a.b_bytes > kPastB)<<<grid, kCsrThreads, (kCsrThreads / 64) * a.feat * sizeof(float), (hipStream_t)stream>>>(a);
     LF_HIP(hipGetLastError());
     return LF_OK;
+}
+
+int lf_csr_spmm_trusted_nnz(const int32_t* d_indptr, const int32_t* d_indices, const float* d_values,
+                            int64_t num_rows, int64_t num_cols, int64_t nnz, int32_t feat_size, int32_t b_dtype,
+                            const void* d_B, float* d_C, lf_stream_t stream) {
+    return lf_csr_spmm_trusted_span(d_indptr, d_indices, d_values, num_rows, num_cols, nnz, 0, feat_size, b_dtype, d_B, d_C, stream);
 }
 
 int lf_csr_spmm_trusted(const int32_t* d_indptr, const int32_t* d_indices, const float* d_values,
@@ -215,10 +221,11 @@ int lf_csr_spmm(const int32_t* d_indptr, const int32_t* d_indices, const float* 
         if (int rc = feature_shape(feat_size, b_dtype, &lpr, &ch)) return rc;
     }
     // no gather before the index arrays have passed
-    if (int rc = lf::csr_check(d_indptr, d_indices, nullptr, num_rows, num_cols, nnz, d_scratch, nullptr, "lf_csr_spmm",
+    int64_t span = 0;
+    if (int rc = lf::csr_check(d_indptr, d_indices, nullptr, num_rows, num_cols, nnz, d_scratch, nullptr, &span, "lf_csr_spmm",
                                (hipStream_t)stream))
         return rc;
-    return lf_csr_spmm_trusted_nnz(d_indptr, d_indices, d_values, num_rows, num_cols, nnz, feat_size, b_dtype, d_B, d_C, stream);
+    return lf_csr_spmm_trusted_span(d_indptr, d_indices, d_values, num_rows, num_cols, nnz, span, feat_size, b_dtype, d_B, d_C, stream);
 }
 
 }  // extern "C"

@@ -683,6 +683,9 @@ constexpr long long kRowGroupMinRows = 4096;   // smaller buckets are not worth 
 constexpr int kRowGroupSample = 4096;          // the decision looks at about this many groups of a bucket first
 constexpr int kRowGroupMaxPercent = 70;        // merged entries / plain gathers at most, in percent
 constexpr int kRowGroupSampleEntries = 24;     // merged entries of a group that the sampling pass looks at
+constexpr long long kSampleMinRows = 1024;     // the sample tells how near each other neighbouring rows' columns are besides
+constexpr int kSampleMinWidth = 4;             // (four columns are read at a time)
+constexpr int kLdsOfCu = 160 << 10, kLdsStep = 1280;
 
 struct MergedBucket {
     long long n_groups;        // row groups
@@ -1051,7 +1054,8 @@ struct PlanBucket {
     int log_w;
     int part;
     int n_blocks;              // workgroups of plan_scan_kernel
-    int sample_stride;         // row-group sampling: every sample_stride-th group is looked at (0: no candidate)
+    int sample_stride;         // every sample_stride-th group of rows is looked at (0: none)
+    int all_cols;              // columns of a partition
 };
 
 // One pass over all buckets of a plan:
@@ -1176,10 +1180,11 @@ plan_scan_kernel(const PlanBucket* __restrict__ buckets, const int32_t* __restri
     }
 }
 
-// Every sample_stride-th group of four rows of the candidate buckets (blockIdx.y: all buckets of the
+// Every sample_stride-th group of four rows of the sampled buckets (blockIdx.y: all buckets of the
 // plan): counters[3 k ..] = merged entries among the first kRowGroupSampleEntries of a group, the
-// slots they consumed, the largest count.  Enqueued behind plan_scan_kernel, before its verdict has
-// been read: where a check failed nothing is followed through the slabs.
+// slots they consumed, the columns that the groups span (all, where it holds a part of a row, which says
+// nothing).  Enqueued behind plan_scan_kernel, before its verdict has been read: where a check failed nothing is followed
+// through the slabs.
 __global__ void __launch_bounds__(256)
 rowgroup_sample_kernel(const PlanBucket* __restrict__ buckets, const int* __restrict__ flags,
                        unsigned long long* __restrict__ counters) {
@@ -1188,10 +1193,33 @@ rowgroup_sample_kernel(const PlanBucket* __restrict__ buckets, const int* __rest
     if (bk.sample_stride == 0) return;
     const long long g = ((long long)blockIdx.x * blockDim.x + threadIdx.x) * bk.sample_stride;
     int m = 0, plain = 0;
-    if (g * kGroupRows < bk.n_rows)
+    long long span = 0;
+    if (g * kGroupRows < bk.n_rows) {
         m = merge_group<false>(bk.cols, nullptr, bk.meta, g, bk.n_rows, bk.log_w,
                                [](int, int, const float*, uint32_t) {}, kRowGroupSampleEntries, &plain);
-    add_rowgroup_counters(m, plain, counters + 3 * blockIdx.y);
+        int first = 0x7FFFFFFF, last = 0;
+        bool whole = true;
+#pragma unroll
+        for (int r = 0; r < kGroupRows; ++r) {
+            const long long e = min(g * kGroupRows + r, bk.n_rows - 1), at = e << bk.log_w;
+            const int meta = bk.meta[e];
+            whole = whole && meta >> kMetaLenBits == 1;
+            first = min(first, bk.cols[at]);
+            last = max(last, bk.cols[at + (meta & (int)kMetaLenMask) - 1]);
+        }
+        span = whole ? last - first : bk.all_cols;
+    }
+    for (int d = 32; d > 0; d >>= 1) {
+        m += __shfl_xor(m, d);
+        plain += __shfl_xor(plain, d);
+        span += __shfl_xor(span, d);
+    }
+    unsigned long long* c = counters + 3 * blockIdx.y;
+    if ((threadIdx.x & 63) == 0 && plain > 0) {
+        atomicAdd(&c[0], (unsigned long long)m);
+        atomicAdd(&c[1], (unsigned long long)plain);
+        atomicAdd(&c[2], (unsigned long long)span);
+    }
 }
 
 // Fills the chunk table of a bucket (rows of more than coop_slots slots, cut into chunks) and its
@@ -1334,7 +1362,7 @@ struct lf_spmm_plan {
     int device = 0, num_cus = 0, grid = 0;
     struct Launch {
         int group_begin = 0, n_groups = 0, grid = 0;
-        int dyn_lds = 0;             // bytes of dynamic LDS (balanced segment tiles)
+        int dyn_lds = 0;             // bytes of dynamic LDS (balanced segment tiles, or to have fewer tiles on a CU)
         int merged_begin = 0, n_merged = 0, merged_grid = 0;   // row-group buckets of this partition
         int cell_begin = 0, n_cell_buckets = 0, cell_grid = 0; // buckets rewritten as cells
         long long tiles = 0;
@@ -1583,6 +1611,7 @@ int lf_spmm_create(lf_spmm_plan** out_plan, const lf_bucket_desc* h_buckets, int
     const PlanBucket* d_table = (const PlanBucket*)(d_scratch + o_table);
     const int32_t* d_first = (const int32_t*)(d_scratch + o_table + nb_s * sizeof(PlanBucket));
     int scan_blocks = 0;
+    std::vector<long long> samples((size_t)num_buckets, 0);        // groups looked at
     long long most_samples = 0;
     for (int k = 0; k < num_buckets; ++k) {
         const lf_bucket_desc& b = h_buckets[k];
@@ -1615,11 +1644,14 @@ int lf_spmm_create(lf_spmm_plan** out_plan, const lf_bucket_desc* h_buckets, int
         h_first[k] = scan_blocks;
         scan_blocks += t.n_blocks;
         t.sample_stride = 0;
-        if (ch == 1 && !(env_groups && env_groups[0] == '0') && b.num_ell_rows >= kRowGroupMinRows && b.width >= kUnroll && b.width <= 64) {
+        t.all_cols = (int)cols_p;
+        if (b.num_ell_rows >= kSampleMinRows && b.width >= kSampleMinWidth) {
             const long long n_groups = lf::ceil_div(b.num_ell_rows, kGroupRows);
             t.sample_stride = (int)std::max<long long>(1, n_groups / kRowGroupSample);
-            most_samples = std::max<long long>(most_samples, lf::ceil_div(n_groups, t.sample_stride));
-            cand.push_back(k);
+            samples[k] = lf::ceil_div(n_groups, t.sample_stride);
+            most_samples = std::max(most_samples, samples[k]);
+            if (ch == 1 && !(env_groups && env_groups[0] == '0') && b.num_ell_rows >= kRowGroupMinRows && b.width >= kUnroll && b.width <= 64)
+                cand.push_back(k);
         }
     }
     if (num_buckets > 0) LF_TRY_HIP(hipMemcpyAsync(d_scratch + o_table, h_table, table_bytes, hipMemcpyHostToDevice, s));
@@ -1633,7 +1665,7 @@ int lf_spmm_create(lf_spmm_plan** out_plan, const lf_bucket_desc* h_buckets, int
         collect_uncovered_kernel<<<rgrid, 256, 0, s>>>(d_cov, num_rows, d_zero_count, nullptr);
         LF_TRY_HIP(hipGetLastError());
     }
-    if (!cand.empty()) {
+    if (most_samples > 0) {
         rowgroup_sample_kernel<<<dim3((unsigned)lf::ceil_div(most_samples, 256), (unsigned)num_buckets), 256, 0, s>>>(d_table, d_flags, d_sample);
         LF_TRY_HIP(hipGetLastError());
     }
@@ -1661,6 +1693,19 @@ int lf_spmm_create(lf_spmm_plan** out_plan, const lf_bucket_desc* h_buckets, int
         if (!is_multi(k) && c[1] > 0 && c[0] * 100 <= c[1] * kRowGroupMaxPercent) chosen.push_back(k);
     }
 
+    // Columns that neighbouring rows span, on average; 0: not known.
+    double span = 0.0;
+    {
+        double slots = 0.0;
+        for (int k = 0; k < num_buckets; ++k) {
+            if (samples[k] == 0) continue;
+            const double mine = (double)h_buckets[k].num_ell_rows * h_buckets[k].width;
+            span += mine * (double)back.as<unsigned long long>(o_sample)[3 * k + 2] / (double)samples[k];
+            slots += mine;
+        }
+        if (slots > 0.0) span /= slots;
+    }
+
     // ---- Feature slices; matrices whose kernels share gathers between rows read B through the L2s as it is.
     // A doubling of S costs 0.5 us in rows' starts and ends, one of the sub-waves to a wavefront 0.35, and sub-waves of fewer
     // lanes are more of them to share a long row's chunk, whose chain of gathers (0.11 us a step; it overlaps with other
@@ -1674,7 +1719,9 @@ int lf_spmm_create(lf_spmm_plan** out_plan, const lf_bucket_desc* h_buckets, int
         const int vec = b_dtype == LF_DTYPE_BF16 ? 8 : 4;
         bool chains = false;                               // rows of several chunks
         for (int k = 0; k < num_buckets; ++k) chains = chains || scanned(k, 1) > 0;
-        const Slices slices = feature_slices(lf::ceil_div(num_cols, (int64_t)num_parts), total_slots / num_parts, feat_size, b_dtype,
+        const double row_slots = (double)total_slots / ((double)num_parts * (double)std::max<int64_t>(num_rows, 1));
+        auto tile_rows = [&](int lanes) { return tile_slots(lanes, false) / std::max(row_slots, 1.0); };
+        const Slices slices = feature_slices(cols_p, total_slots / num_parts, feat_size, b_dtype, Neighbours{span, num_rows}, tile_rows,
                                              [&](int n, int width, int lg_subs, double us) {
             const int lanes = std::min(64, std::max(8, width / vec));
             const double steps = (double)chunk_slots * lanes / (kWG * kUnroll);
@@ -2049,6 +2096,17 @@ int lf_spmm_create(lf_spmm_plan** out_plan, const lf_bucket_desc* h_buckets, int
 
     KernelSet ks;
     LF_TRY(select_kernels(lpr, ch, b_dtype, &ks));
+    hipFuncAttributes attributes;
+    LF_TRY_HIP(hipFuncGetAttributes(&attributes, reinterpret_cast<const void*>(plan->resident ? ks.tiles_resident : ks.tiles)));
+    // Tiles whose rows have near columns, and all features of them, run four to a CU, or so many more are in flight that
+    // they push each other's rows of B out of the caches: 7-point stencils, us, without a limit (5 or 6 to a CU) / 4 / 3: 226K points,
+    // N = 64 32.5 / 29.8 / 32.7; 200K, N = 128 54.0 / 50.7 / 53.6; 729K, N = 64 112 / 107.4 / 105.8.  Little more than four to a CU
+    // would run in two rounds so (70K, N = 96: 17.8, 19.7).
+    if (is_near(span, cols_p) && plan->slices == 1 && chosen.empty()) {
+        const int most = kLdsOfCu / (kNearGroupsPerCu + 1) + kLdsStep;     // one more would not fit
+        for (auto& L : plan->launches)
+            if (2 * L.grid > 11 * plan->num_cus) L.dyn_lds = std::max(L.dyn_lds, most - (int)attributes.sharedSizeBytes);
+    }
     int dyn_lds = 0;
     plan->grid = 0;
     for (const auto& L : plan->launches) {
@@ -2059,11 +2117,7 @@ int lf_spmm_create(lf_spmm_plan** out_plan, const lf_bucket_desc* h_buckets, int
     plan->info[0] = total_tiles;
     plan->info[1] = plan->grid;
     plan->info[2] = num_parts;
-    {
-        hipFuncAttributes fa;
-        LF_TRY_HIP(hipFuncGetAttributes(&fa, reinterpret_cast<const void*>(plan->resident ? ks.tiles_resident : ks.tiles)));
-        plan->info[3] = (int64_t)fa.sharedSizeBytes + dyn_lds;
-    }
+    plan->info[3] = (int64_t)attributes.sharedSizeBytes + dyn_lds;
     plan->info[4] = n_heavy_total;
     plan->info[5] = n_partials;
     plan->info[6] = n_zero;
@@ -2111,6 +2165,7 @@ int lf_model_shape_ms(const int64_t* h_stats, int32_t num_parts, int32_t n_windo
     const int feat = feat_size / n_windows;
     const double g = (double)feat * (b_dtype == LF_DTYPE_BF16 ? 2.0 : 4.0), cols = std::ceil((double)num_cols / num_parts);
     const Slices best = feature_slices((int64_t)cols, (int64_t)(nnz / num_parts), feat, b_dtype,
+                                       Neighbours{}, [](int) { return 0.0; },
                                        [](int n, int, int lg_subs, double us) { return slices_and_subs(n, lg_subs, us); });
     const double lg = std::log2((double)n_windows);
     const double narrow = 1.0 + (g < 512.0 ? kNarrow * lg * lg : 0.0);

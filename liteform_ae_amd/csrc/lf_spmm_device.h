@@ -551,8 +551,23 @@ inline XcdParts xcd_parts(int pieces, int wide) {
 // For the price that is compared with that of other partitions (us), a slice of about an L2 misses more: 20 % at 5 MB, and 10 %
 // less for a doubling of the sub-waves (233K rows of 490, N = 128, slices of 3.7 MB in 8 partitions 3.81 ms, of 1.9 in 16
 // 3.12).  Of slices chosen by that price, 5 % would be more than 3 % slower than S = 1, instead of 3 %.
-template <typename Adjust>
-inline Slices feature_slices(int64_t num_cols, int64_t entries, int feat, int dtype, Adjust adjust) {
+//
+// In a matrix whose neighbouring rows have near columns (stencils, bands; `span`: the columns of four such rows, on
+// average) an XCD does not use all of B at a time but what its rows in flight span, four workgroups of
+// group_rows(lanes of a row) each to a CU, and hardly a row of B that another XCD uses.  Stencils of 4K to 800K points, us,
+// slices as if for a random matrix -> now, without any: plans, 27-point, 62K points, N = 416 124 -> 107, 107; 7-point, 21K, N = 256
+// 14.9 -> 13.3, 13.3; 7-point, 160K, N = 352 138 -> 98, 138; CSR, 27-point, 62K, N = 416 167 -> 121, 121; 7-point, 21K, N = 256
+// 18.1 -> 10.7, 10.7.  301 plans and 320 CSR products, every S timed: 4.5 and 7.1 % above the best S before, now 1.7 and
+// 1.6.
+constexpr int kNearGroupsPerCu = 4, kCusOfXcd = 32;
+struct Neighbours {
+    double span = 0.0;                                     // 0: not known
+    int64_t num_rows = 0;
+};
+inline bool is_near(double span, int64_t num_cols) { return span > 0.0 && 2.0 * span < (double)num_cols; }
+
+template <typename GroupRows, typename Adjust>
+inline Slices feature_slices(int64_t num_cols, int64_t entries, int feat, int dtype, Neighbours neighbours, GroupRows group_rows, Adjust adjust) {
     constexpr double kL2 = 4.3e6, kHitRate = 27e6, kMissRate = 7.15e6, kMiss128 = 1.06, kFirstUse = 0.4, kPerSub = 0.05;
     constexpr double kSoftL2 = 5.0e6, kSoftPerSub = 0.1;
     const int elem = dtype == LF_DTYPE_BF16 ? 2 : 4, step = slice_step(dtype);
@@ -575,8 +590,14 @@ inline Slices feature_slices(int64_t num_cols, int64_t entries, int feat, int dt
         const double share = weight / (2.0 * wide * kXcds);
         const double bytes = gathered * weight / (2.0 * pieces);
         const double lanes = 16.0 * (double)entries * lpr * ch * weight / (wide + pieces - (n - 1) * wide);
-        const double uses = (double)entries / (double)num_cols * share;
-        const double again = std::max(0.0, 1.0 - kFirstUse / uses), slice_bytes = (double)num_cols * width * elem;
+        double uses = (double)entries / (double)num_cols * share, in_use = (double)num_cols;
+        if (is_near(neighbours.span, num_cols)) {
+            const double rows = (double)neighbours.num_rows;
+            const double in_flight = std::min(rows * share, kNearGroupsPerCu * kCusOfXcd * group_rows(lpr));
+            in_use = std::min(in_use, neighbours.span + in_flight * (double)num_cols / rows);
+            uses = (double)entries / (double)num_cols;
+        }
+        const double again = std::max(0.0, 1.0 - kFirstUse / uses), slice_bytes = in_use * width * elem;
         const int lg_subs = lf::ilog2(64 / lpr);
         auto priced = [&](double hit, double per_sub) {
             return adjust(n, width, lg_subs, lanes * hit / kHitRate * (1.0 + per_sub * lg_subs) +

@@ -214,17 +214,34 @@ class _DeviceCSR:
         self._g = g
         self._seg_deg = {}
         self._stats_ws = {}          # num_parts -> statistics workspace holding the row bounds
+        self._span = None
         src = getattr(g, "_csr_source", None)
         if src is not None and self._from_csr(src, bool(getattr(g, "_unit_values", False))):
             self.path = "csr"
         else:
-            triplets = getattr(g, "_triplets", None)
-            if triplets is None:
-                coo = g.coo_mtx
-                triplets = (coo.row, coo.col, coo.data)
-            self._from_coo(*triplets[:3])
+            self._from_coo(*self._triplets())
             self.path = "coo"
         torch.cuda.current_stream().synchronize()
+
+    def _triplets(self):
+        triplets = getattr(self._g, "_triplets", None)
+        if triplets is None:
+            coo = self._g.coo_mtx
+            triplets = (coo.row, coo.col, coo.data)
+        return triplets[:3]
+
+    @property
+    def span(self) -> int:
+        """Columns that four neighbouring rows span, on average over a sample (0: not known): measured by the check of
+        CSR arrays; of triplets, in whatever order, twice the distance from the diagonal that one in ten exceeds."""
+        if self._span is None:
+            row, col, _ = self._triplets()
+            self._span = 0
+            if len(row):
+                at = np.linspace(0, len(row) - 1, 512).astype(np.int64)
+                away = np.abs(np.asarray(col)[at] - np.asarray(row)[at] * (self.num_cols / self.num_rows))
+                self._span = int(2 * np.partition(away, 460)[460])
+        return self._span
 
     def _from_csr(self, csr, unit_values: bool) -> bool:
         """Uploads the CSR arrays; False (nothing kept) when they are not canonical.  Raises
@@ -236,11 +253,12 @@ class _DeviceCSR:
         indices = _upload(csr.indices, np.int32)
         values = None if unit_values else _upload(csr.data, np.float32)
         scratch = torch.empty(4, dtype=torch.int32, device="cuda")
-        flags = C.c_int32(0)
-        _lib.check(lib.lf_csr_check(_lib.ptr(indptr), _lib.ptr(indices), _lib.ptr(values), self.num_rows, self.num_cols,
-                                    nnz, _lib.ptr(scratch), C.byref(flags), _stream()))
+        flags, span = C.c_int32(0), C.c_int64(0)
+        _lib.check(lib.lf_csr_check_span(_lib.ptr(indptr), _lib.ptr(indices), _lib.ptr(values), self.num_rows, self.num_cols,
+                                         nnz, _lib.ptr(scratch), C.byref(flags), C.byref(span), _stream()))
         if not flags.value & _lib.LF_CSR_CANONICAL:
             return False
+        self._span = int(span.value)
         self.indptr, self.indices, self.nnz = indptr, indices, nnz
         self.all_ones = unit_values or bool(flags.value & _lib.LF_CSR_UNIT_VALUES)
         self._values = values
@@ -643,9 +661,9 @@ def spmm_csr(g, B, b_dtype: str = "f32", use_values: bool = True):
     out = torch.empty((dev.num_rows, feat), dtype=torch.float32, device="cuda")
     vals = dev.values if use_values else None
     # the device arrays were made by lf_coo_to_csr or have passed lf_csr_check: no second check
-    rc = lib.lf_csr_spmm_trusted_nnz(dev.indptr.data_ptr(), dev.indices.data_ptr(), None if vals is None else vals.data_ptr(),
-                                     dev.num_rows, dev.num_cols, dev.nnz, feat, _B_DTYPES[b_dtype], B.data_ptr(),
-                                     out.data_ptr(), _stream())
+    rc = lib.lf_csr_spmm_trusted_span(dev.indptr.data_ptr(), dev.indices.data_ptr(), None if vals is None else vals.data_ptr(),
+                                      dev.num_rows, dev.num_cols, dev.nnz, dev.span, feat, _B_DTYPES[b_dtype], B.data_ptr(),
+                                      out.data_ptr(), _stream())
     if rc:
         _lib.check(rc)
     return out

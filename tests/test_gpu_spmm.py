@@ -550,3 +550,67 @@ def test_operands_of_more_than_4_gb(fa, torch, cols, feat, windows, parts, b_dty
     shape = (len(deg), len(used))
     ref = O.spmm_csr_f64(indptr, at, vals, shape, Bh)
     assert (np.abs(C.cpu().numpy() - ref) <= TOL * O.spmm_abs_bound(indptr, at, vals, shape, Bh) + 1e-30).all()
+
+
+@pytest.mark.parametrize("dims,points,feat,b_dtype,most,shuffled", [((46, 16, 84), 27, 416, "f32", 2, 7), ((23, 46, 20), 7, 256, "f32", 2, 8),
+                                                                    ((40, 40, 40), 7, 32, "f32", 1, 1), ((33, 55, 88), 7, 352, "f32", 8, 1),
+                                                                    ((60, 70, 60), 7, 128, "bf16", 2, 1), ((16, 16, 16), 7, 512, "f32", 2, 1)])
+def test_slices_of_matrices_with_near_columns(fa, torch, dims, points, feat, b_dtype, most, shuffled):
+    """Stencils: no more slices than what the rows in flight span asks for, and the same product with split rows and in
+    partitions; the same matrix with its columns shuffled has those of a random one."""
+    rng = np.random.default_rng(feat)
+    nx, ny, nz = dims
+    n = nx * ny * nz
+    at = np.arange(n)
+    x, y, z = at % nx, at // nx % ny, at // (nx * ny)
+    row, col = [], []
+    for dz in (-1, 0, 1):
+        for dy in (-1, 0, 1):
+            for dx in (-1, 0, 1):
+                if points == 7 and abs(dx) + abs(dy) + abs(dz) > 1:
+                    continue
+                ok = (x + dx >= 0) & (x + dx < nx) & (y + dy >= 0) & (y + dy < ny) & (z + dz >= 0) & (z + dz < nz)
+                row.append(at[ok])
+                col.append((at + dx + nx * (dy + ny * dz))[ok])
+    row, col = np.concatenate(row), np.concatenate(col)
+    vals = rng.uniform(-1, 1, size=len(row)).astype(np.float32)
+    g = MTX.from_coo(row.astype(np.int32), col.astype(np.int32), (n, n), data=vals)
+    wide = [[8]] if points == 7 else [[32]]
+    _, info = check(fa, torch, g, wide, feat, b_dtype, seed=feat)
+    near = info["grid"] / info["tiles"]
+    assert near < most + 1, info
+    check(fa, torch, g, [[2, 4], [8]], feat, b_dtype, seed=feat)
+    fmt = fa.build_hyb_format_device(MTX.from_coo(row.astype(np.int32), rng.permutation(n)[col].astype(np.int32), (n, n), data=vals), wide)
+    plan = fa.HybSpMM(fmt, feat, b_dtype)
+    far = plan.info["grid"] / plan.info["tiles"]
+    plan.close()
+    assert far >= shuffled, (far, near)
+
+
+def test_span_of_neighbouring_rows(fa, torch):
+    """lf_csr_check_span: bands, random graphs, rows without entries, one row; nothing said of unsorted columns."""
+    import ctypes as C
+    from liteform_ae_amd import _lib
+    lib, rng = _lib.load(), np.random.default_rng(4)
+    scratch = torch.zeros(4, dtype=torch.int32, device="cuda")
+
+    def span(deg, col, cols):
+        indptr = torch.from_numpy(np.concatenate([[0], np.cumsum(deg)]).astype(np.int32)).cuda()
+        indices = torch.from_numpy(np.asarray(col, dtype=np.int32)).cuda()
+        flags, out = C.c_int32(-1), C.c_int64(-1)
+        _lib.check(lib.lf_csr_check_span(_lib.ptr(indptr), _lib.ptr(indices) if len(col) else None, None, len(deg), cols, len(col),
+                                         _lib.ptr(scratch), C.byref(flags), C.byref(out), None))
+        return out.value
+
+    for n, half in ((500, 3), (1024, 9), (5000, 100), (300_000, 40_000)):
+        at = np.arange(n)
+        lo, hi = np.maximum(at - half, 0), np.minimum(at + half, n - 1)
+        # four rows at a time: 2 * half + 3 columns, fewer at the ends; in units of 1 / 4096 of the columns
+        got = span(np.full(n, 2), np.stack([lo, hi], 1).reshape(-1), n)
+        assert abs(got - (2 * half + 3)) <= n / 4096 + 4 * half * half / n + 8, (n, half, got)
+    n, deg = 20_000, np.arange(20_000) % 5
+    col = np.concatenate([np.sort(rng.choice(n, size=d, replace=False)) for d in deg if d])
+    assert 0.5 * n < span(deg, col, n) < n
+    assert span(np.array([3]), [5, 17, 99], 100) == int(94 * 4096 // 100 * 100 / 4096)
+    assert span(np.zeros(50, np.int64), [], 100) == 0
+    assert span(np.array([3]), [17, 5, 99], 100) == 0
