@@ -78,9 +78,12 @@ csr_spmm_kernel(CsrArgs a) {
     __syncthreads();
     const int total = __builtin_amdgcn_readlane(end, 63) - __builtin_amdgcn_readfirstlane(start);
     const unsigned long long longs = __ballot(end - start > max(kCsrLongRow, total / kWaves));      // the same in every wavefront
-    // as many sub-waves as give each one batch of gathers of an average row (half or twice as many: 1 - 7 % slower)
+    // As many sub-waves as give each at most one batch and a half of gathers of an average row: above one batch already, a
+    // row of nine entries left half of the gathers of two sub-waves empty (1.8M rows of 9.6 and 8.8, N = 96: 1250 and 1194 us so,
+    // 1190 and 1162 now, 1150 and 1128 with a sub-wave streaming over the ends of rows; 1.1M of 8.6, N = 192 1348, 1316, 1311;
+    // 300K of 12, N = 32 69.5, 71, 75).  Two batches: the same, but 72 for the last.
     int lg = 0;
-    while (lg < kLgSubs && ((long long)(n * kUnroll) << lg) < total) ++lg;
+    while (lg < kLgSubs && ((long long)(n * kUnroll * 3 / 2) << lg) < total) ++lg;
     const Teams<LPR, CH, BT, WIDE> teams(b, __builtin_amdgcn_readfirstlane(lg));
     const int lg_rows = kLgSubs - teams.lg, team = sub >> teams.lg;
     const int sets = (n + (1 << lg_rows) - 1) >> lg_rows;
