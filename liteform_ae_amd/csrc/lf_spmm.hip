@@ -11,8 +11,8 @@
 //     per lane, coalesced along the feature dimension (N = 128 fp32 -> 32 lanes, two rows
 //     per 64-lane wavefront);
 //   * narrow buckets stage their (row of B, value) tile in LDS with coalesced 16-byte loads
-//     and read it back as broadcasts; rows too wide to stage are streamed by a wavefront each, their slots spread
-//     over its sub-waves and broadcast by DPP;
+//     and read it back as broadcasts; rows too wide to stage are streamed by one or several sub-waves each, their slots
+//     broadcast by DPP;
 //   * a source row split over several ELL rows is summed by one owner; rows longer than
 //     coop_slots (64, 128 or 256) are reduced by a whole workgroup in chunks of 512 to 8192 slots: a row
 //     that fits one chunk is written directly, a longer one leaves one partial row per chunk, which the
@@ -306,17 +306,18 @@ __device__ __forceinline__ void run_ell_tile(const RowsOfB<LPR, CH, BT, WIDE>& b
 }
 
 // Bucket whose source rows may span several ELL rows, or whose rows are too wide to stage: the first ELL row of a
-// segment owns it, a wavefront sums all of its slots, every sub-wave its share; continuation rows and segments
+// segment owns it, a team of sub-waves sums all of its slots, each its share; continuation rows and segments
 // above coop_slots (handled as chunks) are skipped.
 template <int LPR, int CH, typename BT, bool WIDE>
 __device__ __forceinline__ void run_seg_tile(const RowsOfB<LPR, CH, BT, WIDE>& b, const Group& g, long long tile, const LaunchArgs& a) {
     constexpr int VEC = Dense<BT>::kVec;
     const int lane = threadIdx.x & 63;
     const Lane<LPR, CH, VEC> ln(lane % LPR, a.feat, a.ldb, a.ldc);
-    const Teams<LPR, CH, BT, WIDE> team(b, Teams<LPR, CH, BT, WIDE>::kLgSubs);
+    const Teams<LPR, CH, BT, WIDE> team(b, min(g.balanced, Teams<LPR, CH, BT, WIDE>::kLgSubs));
+    const int lanes = LPR << team.lg;
     const long long e0 = tile * g.rows_per_tile;
     const int n = (int)min((long long)g.rows_per_tile, g.n_items - e0);
-    for (int r = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6); r < n; r += kWG / 64) {
+    for (int r = (int)threadIdx.x / lanes; r < n; r += kWG / lanes) {
         const long long e = e0 + r;
         const int m = g.meta[e];
         if (m < 0) continue;                                   // continuation row
@@ -328,7 +329,7 @@ __device__ __forceinline__ void run_seg_tile(const RowsOfB<LPR, CH, BT, WIDE>& b
         acc.clear();
         team.sum(g.cols, g.vals, e << g.log_w, total, total, acc);
         team.combine(acc);
-        if (lane < LPR) store_row<LPR, CH, VEC>(a.C, g.rows[e], ln, acc, a.accumulate);
+        if (team.sub == 0) store_row<LPR, CH, VEC>(a.C, g.rows[e], ln, acc, a.accumulate);
     }
 }
 
@@ -357,11 +358,14 @@ __device__ __forceinline__ void load_pair_agent(const float* src, float& x, floa
     y = __uint_as_float((unsigned int)(v >> 32));
 }
 
-// Rows of a streamed tile: two to a wavefront.  A sub-wave per row, the form before, was a chain of up to 32 batches
-// for a row of 256 slots; a wavefront at N = 32 takes 4.  Log-normal rows, us, before -> now: 16000 x 128, N = 32
-// 25.5 -> 18.5, N = 64 35.3 -> 27.9; 32000 x 32, N = 32 16.7 -> 12.1.  (32 rows to a tile, as with sub-waves: 38.8, 38.6,
-// 27.6; 4 to a tile: within 3 % either way.)
-constexpr int kSegRows = 8;
+// Streamed rows: as many sub-waves to a row as have 64 of its slots each, 8 rows to a tile, 4 where rows of B take 32 lanes and
+// more.  A sub-wave to a row, with tiles of 16 and 32 rows, is a chain of up to 32 batches; all of a wavefront to a row leaves
+// batches of its sub-waves half empty, and an eighth row waits for two before it where a wavefront is one sub-wave.  Log-normal rows,
+// us, a sub-wave / a wavefront / this: 16000 x 128, N = 32 25.7 / 19.1 / 18.4, N = 64 35.6 / 28.2 / 28.1; 132K x 300 in eight
+// partitions, N = 32 363 / 371 / 359, N = 64 605 / 617 / 610; 207K x 175, N = 32 323 / 339 / 329; 4.5K x 91, N = 416 34.4 /
+// 37.2 / 29.6; 6.5K x 311, N = 416 149 / 153 / 138.  300 matrices of 3K to 250K rows of 50 to 400: 0.93 to 1.0 of
+// the time with a wavefront to a row; 16 rows to a tile are 1 % better above 32K such rows and up to 25 % worse below 16K.
+constexpr int kSegRows = 8, kLgTeamSlots = 6;
 constexpr int kSlice = 8;
 constexpr int kSlicedSlots = 128;
 
@@ -1987,7 +1991,8 @@ int lf_spmm_create(lf_spmm_plan** out_plan, const lf_bucket_desc* h_buckets, int
             const int fit = tile_slots(lpr, plan->resident && b_dtype == LF_DTYPE_F32) >> g.log_w;   // ELL rows whose slots fit the LDS tile
             const bool staged = fit >= sw;
             g.type = staged ? (is_multi(k) ? kEllSeg : kEll) : kSeg;
-            g.rows_per_tile = staged ? std::min(kTileRows, fit) : kSegRows;
+            g.rows_per_tile = staged ? std::min(kTileRows, fit) : lpr <= 16 ? kSegRows : kSegRows / 2;
+            if (!staged) g.balanced = std::max(0, g.log_w - kLgTeamSlots);
             if (staged) {
                 // a small bucket is cut into more, shorter tiles so that it still spreads over
                 // the CUs: at least one pass of every sub-wave (8 rows at a time in the

@@ -89,7 +89,8 @@ struct Group {
     int type;
     int log_w;
     int rows_per_tile;
-    int balanced;                 // kEllSeg: per-ELL-row sums through LDS (needs rows_per_tile * N floats)
+    int balanced;                 // kEllSeg: per-ELL-row sums through LDS (needs rows_per_tile * N floats); kSeg: log2 of the
+                                  // sub-waves to a row, or more than a wavefront has
     long long n_items;            // ELL rows / rows to clear / chunks
     long long n_tiles;
     const int32_t* rows;          // kEll, kSeg: source rows; kZero: rows to clear
