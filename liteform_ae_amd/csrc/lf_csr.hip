@@ -25,6 +25,7 @@ struct CsrArgs {
     const float* values;                   // null: ones
     long long n_rows, n_groups;
     int rows_per_group;
+    int share;                             // entries of a sub-wave, see csr_share
     int feat, ld;                          // features of a slice (the last may have fewer); elements between rows of B and of C
     XcdParts parts;
     const void* B;
@@ -78,12 +79,9 @@ csr_spmm_kernel(CsrArgs a) {
     __syncthreads();
     const int total = __builtin_amdgcn_readlane(end, 63) - __builtin_amdgcn_readfirstlane(start);
     const unsigned long long longs = __ballot(end - start > max(kCsrLongRow, total / kWaves));      // the same in every wavefront
-    // As many sub-waves as give each at most one batch and a half of gathers of an average row: above one batch already, a
-    // row of nine entries left half of the gathers of two sub-waves empty (1.8M rows of 9.6 and 8.8, N = 96: 1250 and 1194 us so,
-    // 1190 and 1162 now, 1150 and 1128 with a sub-wave streaming over the ends of rows; 1.1M of 8.6, N = 192 1348, 1316, 1311;
-    // 300K of 12, N = 32 69.5, 71, 75).  Two batches: the same, but 72 for the last.
+    // as many sub-waves as give each at most `share` entries of an average row
     int lg = 0;
-    while (lg < kLgSubs && ((long long)(n * kUnroll * 3 / 2) << lg) < total) ++lg;
+    while (lg < kLgSubs && ((long long)(n * a.share) << lg) < total) ++lg;
     const Teams<LPR, CH, BT, WIDE> teams(b, __builtin_amdgcn_readfirstlane(lg));
     const int lg_rows = kLgSubs - teams.lg, team = sub >> teams.lg;
     const int sets = (n + (1 << lg_rows) - 1) >> lg_rows;
@@ -132,6 +130,15 @@ csr_spmm_kernel(CsrArgs a) {
         __syncthreads();                                     // before the next row's parts
     }
 }
+
+// A sub-wave's entries of an average row at most.  One batch of gathers (half or twice as many: 1 - 7 % slower; 17K power-law
+// rows of 3, N = 64 8.4 us, a batch and a half 9.7).  But where B is past the memory-side cache too, what counts is how
+// many gathers are in flight, and two sub-waves on a row of nine leave half of theirs empty: a batch and a half.  1.8M rows of
+// 9.6 and 8.8, N = 96: 1190 and 1162 us, 1250 and 1194 with one batch (1150 and 1128 with a sub-wave streaming over the ends of
+// rows); 1.1M of 8.6, N = 192 1316, 1348, 1311.  (B of 53 to 210 MB: 500K rows of 9, N = 32 101 and 96; 147K of 11, N = 384 367
+// and 354.)
+constexpr unsigned long long kMallBytes = 256ull << 20;
+int csr_share(unsigned long long b_bytes) { return b_bytes > kMallBytes ? kUnroll * 3 / 2 : kUnroll; }
 
 using CsrFn = void (*)(CsrArgs);
 
@@ -192,6 +199,7 @@ int lf_csr_spmm_trusted_span(const int32_t* d_indptr, const int32_t* d_indices, 
     a.B = d_B;
     a.C = d_C;
     a.b_bytes = (unsigned long long)num_cols * feat_size * (b_dtype == LF_DTYPE_BF16 ? 2 : 4);
+    a.share = csr_share(a.b_bytes);
     long long longest = 0;
     for (int x = 0; x < kXcds; ++x) longest = std::max(longest, part_tiles(a.parts, x, a.n_groups));
     const unsigned grid = (unsigned)(longest * kXcds);
