@@ -690,6 +690,7 @@ constexpr int kRowGroupSampleEntries = 24;     // merged entries of a group that
 constexpr long long kSampleMinRows = 1024;     // the sample tells how near each other neighbouring rows' columns are besides
 constexpr int kSampleMinWidth = 4;             // (four columns are read at a time)
 constexpr int kLdsOfCu = 160 << 10, kLdsStep = 1280;
+constexpr double kFarSliceBytes = 64e6;
 
 struct MergedBucket {
     long long n_groups;        // row groups
@@ -2103,11 +2104,14 @@ int lf_spmm_create(lf_spmm_plan** out_plan, const lf_bucket_desc* h_buckets, int
     LF_TRY(select_kernels(lpr, ch, b_dtype, &ks));
     hipFuncAttributes attributes;
     LF_TRY_HIP(hipFuncGetAttributes(&attributes, reinterpret_cast<const void*>(plan->resident ? ks.tiles_resident : ks.tiles)));
-    // Tiles whose rows have near columns, and all features of them, run four to a CU, or so many more are in flight that
-    // they push each other's rows of B out of the caches: 7-point stencils, us, without a limit (5 or 6 to a CU) / 4 / 3: 226K points,
-    // N = 64 32.5 / 29.8 / 32.7; 200K, N = 128 54.0 / 50.7 / 53.6; 729K, N = 64 112 / 107.4 / 105.8.  Little more than four to a CU
-    // would run in two rounds so (70K, N = 96: 17.8, 19.7).
-    if (is_near(span, cols_p) && plan->slices == 1 && chosen.empty()) {
+    // Four tiles to a CU, where five and more would push each other's rows of B out of the caches for nothing:
+    // rows of near columns, and all features of them (7-point stencils, us, without a limit, 5 or 6 to a CU / 4 / 3: 226K points,
+    // N = 64 32.5 / 29.8 / 32.7; 200K, N = 128 54.0 / 50.7 / 53.6; 729K, N = 64 112 / 107.4 / 105.8), and parts of B of which the
+    // L2s hold little (522K rows of 15, bf16 N = 256 648 / 637 / 615; 170K power-law rows, N = 64 38.0 / 35.7 / 36.9; 630
+    // matrices with slices of more than 64 MB: 0.994 and 0.993 of the time on average, 1.02 and 1.05 at most; below 16 MB 1.03 to
+    // 1.1 and 1.1 to 1.3).  Little more than four to a CU would run in two rounds so (70K points, N = 96: 17.8, 19.7).
+    const double slice_bytes = (double)cols_p * feat_size * (b_dtype == LF_DTYPE_BF16 ? 2 : 4);
+    if (chosen.empty() && ((is_near(span, cols_p) && plan->slices == 1) || slice_bytes > kFarSliceBytes)) {
         const int most = kLdsOfCu / (kNearGroupsPerCu + 1) + kLdsStep;     // one more would not fit
         for (auto& L : plan->launches)
             if (2 * L.grid > 11 * plan->num_cus) L.dyn_lds = std::max(L.dyn_lds, most - (int)attributes.sharedSizeBytes);
