@@ -65,14 +65,14 @@ __global__ void row_pointer_kernel(const unsigned long long* __restrict__ keys, 
 // arrays and of the row pointer.  Bound by launches and by the latency of each kernel's two or three dependent passes.
 // With the wait for the flags, us, the library's sort with the kernels around it -> this: 6K entries 65 -> 42, 64K 79 -> 45,
 // 300K 165 -> 55, 860K of a power-law graph (a row of 41,000) 234 -> 134, 1.6M 201 -> 79, 4M 350 -> 180, 7.8M 571 -> 340;
-// with a duplicate 61 -> 70, 80 -> 74, 166 -> 87, 230 -> 220, 202 -> 132, 349 -> 264, 578 -> 541.  Rows in the order of their
+// with a duplicate 61 -> 68, 80 -> 72, 165 -> 86, 228 -> 214, 202 -> 130, 349 -> 266, 578 -> 535.  Rows in the order of their
 // lengths, so that the first bins are large: 1.6M 204 -> 104, 4M 349 -> 213, 7.8M 573 -> 443.  Where the sort has to be
 // taken after all, counting and the wait are lost: 600K 208 -> 239, 2.4M 293 -> 338, 5M 472 -> 566, 7.6M 565 -> 666.
 // Beyond 8.4M entries bins outgrow the LDS, and the sort's few passes over memory are what counts.
 // flags: [kNotHere] an entry outside the matrix or bins of too many, known before anything is distributed, and
 // [kCrowded] a long row with too many of its columns beside each other: the other way has to be taken; [kReads] windows
-// that large bins' parts will read; [kLargeParts] parts left to bin_sort_large_kernel; [kTwice] duplicates, sorted and
-// to be added up.
+// that large bins' parts will read; [kLargeParts] parts left to bin_sort_large_kernel; [kTwice] entries that are to be
+// added to another one of their place.
 constexpr int kNotHere = 0, kReads = 1, kCrowded = 2, kLargeParts = 3, kTwice = 4, kFlags = 5;
 constexpr int kBinThreads = 512;
 constexpr int kBinChunk = 4096;            // entries that a workgroup distributes at least
@@ -307,7 +307,8 @@ __device__ __forceinline__ void sort_bin(const BinSort& a, int bin, int window, 
         }
     };
     auto fraction = [&](unsigned key) { return (key & col_mask) * a.inverse; };      // (below 2^32: column < columns)
-    bool twice = false, crowded = false;
+    int repeats = 0;                                       // entries behind another one of their place
+    bool crowded = false;
     // The records that `selected` takes: by bucket(key), which ascends with the key, and then in full; out(key, place)
     // is where the place-th goes.  More than CAPACITY are too many.
     auto sort_part = [&](auto selected, auto bucket, auto out) {
@@ -352,15 +353,14 @@ __device__ __forceinline__ void sort_bin(const BinSort& a, int bin, int window, 
             for (int i = threadIdx.x; i < sorted; i += THREADS) {
                 const unsigned key = s_key[i], val = s_val[i];
                 const int q = bucket(key), first = q > 0 ? s_bucket[q - 1] : 0, end = s_bucket[q];
-                int place = first;
+                int place = first, ahead = 0;
                 for (int j = first; j < end; ++j) {
                     const unsigned other = s_key[j];
                     place += other < key;
-                    if (other == key && j != i) {          // by value, then as they lie here
-                        twice = true;
-                        place += s_val[j] < val || (s_val[j] == val && j < i);
-                    }
+                    if (other == key && j != i) ahead += s_val[j] < val || (s_val[j] == val && j < i);    // by value, then as they lie here
                 }
+                place += ahead;
+                repeats += ahead > 0;
                 const int to = out(key, place);
                 a.indices[to] = (int32_t)(key & col_mask);
                 a.values[to] = __uint_as_float(val);
@@ -389,7 +389,7 @@ __device__ __forceinline__ void sort_bin(const BinSort& a, int bin, int window, 
                 const int to = out(key, i);
                 a.indices[to] = (int32_t)(key & col_mask);
                 a.values[to] = __uint_as_float(s_val[i]);
-                twice |= i > 0 && s_key[i - 1] == key;
+                repeats += i > 0 && s_key[i - 1] == key;
             }
         }
     };
@@ -444,7 +444,10 @@ __device__ __forceinline__ void sort_bin(const BinSort& a, int bin, int window, 
                   [&](unsigned key) { return (int)__umulhi((unsigned)scaled(key), CAPACITY); },
                   [&](unsigned, int place) { return base + row_at + s_before + place; });
     }
-    if (__ballot(twice) != 0 && (threadIdx.x & 63) == 0) a.flags[kTwice] = 1;
+    if (__ballot(repeats > 0) != 0) {
+        for (int d = 32; d > 0; d >>= 1) repeats += __shfl_xor(repeats, d);
+        if ((threadIdx.x & 63) == 0) atomicAdd(&a.flags[kTwice], repeats);
+    }
     if (__ballot(crowded) != 0 && (threadIdx.x & 63) == 0) a.flags[kCrowded] = 1;
 }
 
@@ -801,9 +804,8 @@ int lf_coo_to_csr(const int32_t* d_coo_row, const int32_t* d_coo_col, const floa
             close_up_kernel<<<(unsigned)(std::max<long long>(num_rows + 1, nnz) + 255) / 256, 256, 0, s>>>(
                 d_indptr, before, num_rows, nnz, out_indices, out_values, d_indices, d_values);
             LF_HIP(hipGetLastError());
-            int h_count = 0;
-            LF_HIP(lf::read_back(&h_count, before + nnz, 4, s));
-            *h_nnz_out = nnz - h_count;
+            LF_HIP(hipStreamSynchronize(s));
+            *h_nnz_out = nnz - h_flags[kTwice];
             return LF_OK;
         }
     }

@@ -51,7 +51,7 @@ def measure(out_path, workloads, feats, parts_list):
                     ms = float(np.median(plan.time_ms(B, C, warmup=2, repeat=7)))
                     plan.close()
                     rec = {"name": name, "feat": feat, "dt": wl.b_dtype, "P": p, "W": w, "ms": ms,
-                           "pred": fa.model_spmm_ms(stats, w, rows, cols, feat, wl.b_dtype),
+                           "pred": fa._modelled_ms("lf_model_shape_ms", stats, w, rows, cols, feat, wl.b_dtype),
                            "rows": rows, "cols": cols, "nnz": wl.nnz, "stats": stats.tolist()}
                     out.write(json.dumps(rec) + "\n")
                     out.flush()
