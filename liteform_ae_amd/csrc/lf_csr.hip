@@ -163,7 +163,7 @@ CsrFn csr_kernel(int lpr, int ch, int dtype, bool wide) {
 // than with S = 1, 21 % at worst (25K rows of 4, N = 160: 12.9 us, 15.6 with 5).  128K rows of 100, N = 96: 635 us with 1,
 // 564 with 3.
 Slices csr_slices(int64_t rows, int rows_per_group, int64_t groups, int64_t num_cols, int64_t nnz, int64_t span, int feat, int dtype) {
-    return feature_slices(num_cols, nnz, feat, dtype, Neighbours{(double)span, rows}, [&](int) { return (double)rows_per_group; }, [&](int s, int width, int lg_subs, double us) {
+    return feature_slices(num_cols, nnz, feat, dtype, Neighbours{(double)span, rows, 0.05}, [&](int) { return (double)rows_per_group; }, [&](int s, int width, int lg_subs, double us) {
         return us * (1.0 + 0.16 * std::max(0.0, std::log2(2048.0 / ((double)groups * s))))
                   * (width * (dtype == LF_DTYPE_BF16 ? 2 : 4) > 512 ? 1.04 : 1.0) * (1.0 + 0.02 * std::log2((double)s))
                + 0.3 * lg_subs + 7e-6 * (double)rows * s;

@@ -584,7 +584,7 @@ csr_check_kernel(const int32_t* __restrict__ indptr, const int32_t* __restrict__
         if (r == 0) bad |= lo != 0;
         if (r == rows - 1) bad |= hi != nnz;
         if (hi > lo && lo > 0 && lo < nnz && indices[lo] <= indices[lo - 1]) ++boundary;
-        if (r % sample_stride == 0) {
+        if ((unsigned)r % (unsigned)sample_stride == 0) {
             int first = 0x7FFFFFFF, last = -1;
             for (long long q = r; q < min(r + 4, rows); ++q) {
                 const long long from = indptr[q], to = indptr[q + 1];

@@ -687,8 +687,6 @@ constexpr long long kRowGroupMinRows = 4096;   // smaller buckets are not worth 
 constexpr int kRowGroupSample = 4096;          // the decision looks at about this many groups of a bucket first
 constexpr int kRowGroupMaxPercent = 70;        // merged entries / plain gathers at most, in percent
 constexpr int kRowGroupSampleEntries = 24;     // merged entries of a group that the sampling pass looks at
-constexpr long long kSampleMinRows = 1024;     // the sample tells how near each other neighbouring rows' columns are besides
-constexpr int kSampleMinWidth = 4;             // (four columns are read at a time)
 constexpr int kLdsOfCu = 160 << 10, kLdsStep = 1280;
 constexpr double kFarSliceBytes = 64e6;
 
@@ -1058,8 +1056,9 @@ struct PlanBucket {
     long long n_rows;
     int log_w;
     int part;
-    int n_blocks;              // workgroups of plan_scan_kernel
-    int sample_stride;         // every sample_stride-th group of rows is looked at (0: none)
+    int n_blocks;              // workgroups of plan_scan_kernel, and one more unless there are none
+    int sample_stride;         // row-group sampling: every sample_stride-th group is looked at (0: no candidate)
+    int span_stride;           // every span_stride-th row is looked at for the span of neighbours' columns
     int all_cols;              // columns of a partition
 };
 
@@ -1071,7 +1070,9 @@ struct PlanBucket {
 //   * counts what lf_spmm_create sizes its tables by: counters[(kScanCounters k + i) * kCounterLine] of bucket
 //     k = chunks of the rows of more than kCoopSlots slots, rows with several chunks, their partial
 //     rows, rows of 65 .. 128 and of 129 .. kCoopSlots slots (a chunk each if they take the cooperative
-//     path), ChunkedRow::found of all rows;
+//     path), ChunkedRow::found of all rows; and by a workgroup of its own, not to lengthen the others, the columns that
+//     groups of kGroupRows neighbours span (every span_stride-th row and those behind it, in kSpanUnits of all columns; all,
+//     where one is a part of a row, which says nothing);
 //   * marks the rows that partition 0 writes.
 // Bound by the stream of the column slabs.  Workgroup -> bucket by the first workgroups of the
 // buckets, so that all of them share one launch however many there are: three launches per bucket
@@ -1080,7 +1081,8 @@ struct PlanBucket {
 constexpr int kScanSlotsPerBlock = 16384;
 constexpr int kScanMaxBlocks = 1024;       // per bucket: more only queue up at its counters
 constexpr int kScanUnroll = 4;             // 16-byte loads of columns in flight per thread
-constexpr int kScanCounters = 6;
+constexpr int kScanCounters = 7, kScanFound = 5, kScanSpan = 6;
+constexpr int kSpanUnits = 4096, kSpanSamples = 1024;      // (twice the samples at most: sums below 2^24)
 constexpr int kCounterLine = 32;           // words between the counters of a bucket: each has a 128-byte line of its
                                            // own, as atomics on one line are taken one after the other (17 ns each)
 __global__ void __launch_bounds__(256)
@@ -1098,6 +1100,26 @@ plan_scan_kernel(const PlanBucket* __restrict__ buckets, const int32_t* __restri
     const int32_t *rows = bk.rows, *meta = bk.meta;
     const int log_w = bk.log_w;
     const long long n_rows = bk.n_rows;
+    if (t0 >= stride) {                                       // the bucket's last workgroup
+        int span = 0;
+        for (long long e = (t0 - stride) * bk.span_stride; e < n_rows; e += 256ll * bk.span_stride) {
+            int first = 0x7FFFFFFF, last = 0;
+            bool whole = true;
+#pragma unroll
+            for (int r = 0; r < kGroupRows; ++r) {
+                const long long q = min(e + r, n_rows - 1), at = q << log_w;
+                const int m = meta[q], n = min(max(m & (int)kMetaLenMask, 1), 1 << log_w);       // (not checked yet)
+                whole = whole && m >> kMetaLenBits == 1;
+                first = min(first, bk.cols[at]);
+                last = max(last, bk.cols[at + n - 1]);
+            }
+            const long long columns = whole ? max((long long)last - first, 0ll) : bk.all_cols;
+            span += (int)min((long long)kSpanUnits, columns * kSpanUnits / bk.all_cols);
+        }
+        for (int d = 32; d > 0; d >>= 1) span += __shfl_xor(span, d);
+        if (lane == 0 && span > 0) atomicAdd(counters + ((size_t)kScanCounters * k + kScanSpan) * kCounterLine, span);
+        return;
+    }
     bool bad_col = false, bad_row = false, bad_meta = false;
     const long long n_slots = n_rows << log_w;
     const unsigned limit = (unsigned)num_cols;               // < 2^31
@@ -1115,7 +1137,7 @@ plan_scan_kernel(const PlanBucket* __restrict__ buckets, const int32_t* __restri
         for (int u = 0; u < kScanUnroll; ++u)
             bad_col |= (unsigned)c[u].x >= limit || (unsigned)c[u].y >= limit || (unsigned)c[u].z >= limit || (unsigned)c[u].w >= limit;
     }
-    constexpr int kSums = kScanCounters - 1;
+    constexpr int kSums = kScanFound;
     int sum[kSums] = {}, found = 0;
     for (long long e = t0; e < n_rows; e += stride) {
         const int row = rows[e];
@@ -1163,7 +1185,7 @@ plan_scan_kernel(const PlanBucket* __restrict__ buckets, const int32_t* __restri
     if (__ballot(bad_row) != 0 && lane == 0) flags[1] = 1;
     if (__ballot(bad_meta) != 0 && lane == 0) flags[2] = 1;
     // one atomic per workgroup and counter
-    __shared__ int s_sum[4][kScanCounters];
+    __shared__ int s_sum[4][kSums + 1];
     for (int d = 32; d > 0; d >>= 1) {
         found |= __shfl_xor(found, d);
         for (int i = 0; i < kSums; ++i) sum[i] += __shfl_xor(sum[i], d);
@@ -1185,11 +1207,10 @@ plan_scan_kernel(const PlanBucket* __restrict__ buckets, const int32_t* __restri
     }
 }
 
-// Every sample_stride-th group of four rows of the sampled buckets (blockIdx.y: all buckets of the
+// Every sample_stride-th group of four rows of the candidate buckets (blockIdx.y: all buckets of the
 // plan): counters[3 k ..] = merged entries among the first kRowGroupSampleEntries of a group, the
-// slots they consumed, the columns that the groups span (all, where it holds a part of a row, which says
-// nothing).  Enqueued behind plan_scan_kernel, before its verdict has been read: where a check failed nothing is followed
-// through the slabs.
+// slots they consumed, the largest count.  Enqueued behind plan_scan_kernel, before its verdict has
+// been read: where a check failed nothing is followed through the slabs.
 __global__ void __launch_bounds__(256)
 rowgroup_sample_kernel(const PlanBucket* __restrict__ buckets, const int* __restrict__ flags,
                        unsigned long long* __restrict__ counters) {
@@ -1198,33 +1219,10 @@ rowgroup_sample_kernel(const PlanBucket* __restrict__ buckets, const int* __rest
     if (bk.sample_stride == 0) return;
     const long long g = ((long long)blockIdx.x * blockDim.x + threadIdx.x) * bk.sample_stride;
     int m = 0, plain = 0;
-    long long span = 0;
-    if (g * kGroupRows < bk.n_rows) {
+    if (g * kGroupRows < bk.n_rows)
         m = merge_group<false>(bk.cols, nullptr, bk.meta, g, bk.n_rows, bk.log_w,
                                [](int, int, const float*, uint32_t) {}, kRowGroupSampleEntries, &plain);
-        int first = 0x7FFFFFFF, last = 0;
-        bool whole = true;
-#pragma unroll
-        for (int r = 0; r < kGroupRows; ++r) {
-            const long long e = min(g * kGroupRows + r, bk.n_rows - 1), at = e << bk.log_w;
-            const int meta = bk.meta[e];
-            whole = whole && meta >> kMetaLenBits == 1;
-            first = min(first, bk.cols[at]);
-            last = max(last, bk.cols[at + (meta & (int)kMetaLenMask) - 1]);
-        }
-        span = whole ? last - first : bk.all_cols;
-    }
-    for (int d = 32; d > 0; d >>= 1) {
-        m += __shfl_xor(m, d);
-        plain += __shfl_xor(plain, d);
-        span += __shfl_xor(span, d);
-    }
-    unsigned long long* c = counters + 3 * blockIdx.y;
-    if ((threadIdx.x & 63) == 0 && plain > 0) {
-        atomicAdd(&c[0], (unsigned long long)m);
-        atomicAdd(&c[1], (unsigned long long)plain);
-        atomicAdd(&c[2], (unsigned long long)span);
-    }
+    add_rowgroup_counters(m, plain, counters + 3 * blockIdx.y);
 }
 
 // Fills the chunk table of a bucket (rows of more than coop_slots slots, cut into chunks) and its
@@ -1616,7 +1614,6 @@ int lf_spmm_create(lf_spmm_plan** out_plan, const lf_bucket_desc* h_buckets, int
     const PlanBucket* d_table = (const PlanBucket*)(d_scratch + o_table);
     const int32_t* d_first = (const int32_t*)(d_scratch + o_table + nb_s * sizeof(PlanBucket));
     int scan_blocks = 0;
-    std::vector<long long> samples((size_t)num_buckets, 0);        // groups looked at
     long long most_samples = 0;
     for (int k = 0; k < num_buckets; ++k) {
         const lf_bucket_desc& b = h_buckets[k];
@@ -1647,16 +1644,15 @@ int lf_spmm_create(lf_spmm_plan** out_plan, const lf_bucket_desc* h_buckets, int
                                                     lf::ceil_div((long long)b.num_ell_rows << log_w, kScanSlotsPerBlock));
         t.n_blocks = (int)std::min<long long>(units, kScanMaxBlocks);
         h_first[k] = scan_blocks;
-        scan_blocks += t.n_blocks;
-        t.sample_stride = 0;
+        scan_blocks += t.n_blocks + (t.n_blocks > 0 ? 1 : 0);
+        t.span_stride = (int)std::max<long long>(kGroupRows, b.num_ell_rows / kSpanSamples);
         t.all_cols = (int)cols_p;
-        if (b.num_ell_rows >= kSampleMinRows && b.width >= kSampleMinWidth) {
+        t.sample_stride = 0;
+        if (ch == 1 && !(env_groups && env_groups[0] == '0') && b.num_ell_rows >= kRowGroupMinRows && b.width >= kUnroll && b.width <= 64) {
             const long long n_groups = lf::ceil_div(b.num_ell_rows, kGroupRows);
             t.sample_stride = (int)std::max<long long>(1, n_groups / kRowGroupSample);
-            samples[k] = lf::ceil_div(n_groups, t.sample_stride);
-            most_samples = std::max(most_samples, samples[k]);
-            if (ch == 1 && !(env_groups && env_groups[0] == '0') && b.num_ell_rows >= kRowGroupMinRows && b.width >= kUnroll && b.width <= 64)
-                cand.push_back(k);
+            most_samples = std::max<long long>(most_samples, lf::ceil_div(n_groups, t.sample_stride));
+            cand.push_back(k);
         }
     }
     if (num_buckets > 0) LF_TRY_HIP(hipMemcpyAsync(d_scratch + o_table, h_table, table_bytes, hipMemcpyHostToDevice, s));
@@ -1670,7 +1666,7 @@ int lf_spmm_create(lf_spmm_plan** out_plan, const lf_bucket_desc* h_buckets, int
         collect_uncovered_kernel<<<rgrid, 256, 0, s>>>(d_cov, num_rows, d_zero_count, nullptr);
         LF_TRY_HIP(hipGetLastError());
     }
-    if (most_samples > 0) {
+    if (!cand.empty()) {
         rowgroup_sample_kernel<<<dim3((unsigned)lf::ceil_div(most_samples, 256), (unsigned)num_buckets), 256, 0, s>>>(d_table, d_flags, d_sample);
         LF_TRY_HIP(hipGetLastError());
     }
@@ -1686,9 +1682,9 @@ int lf_spmm_create(lf_spmm_plan** out_plan, const lf_bucket_desc* h_buckets, int
         if (f[3]) return bail(lf::fail(LF_ERR_UNSUPPORTED, "a row is split over more than %d ELL rows", (1 << (31 - kMetaLenBits)) - 1));
     }
     auto scanned = [&](int k, int i) { return h_counters[((size_t)kScanCounters * k + i) * kCounterLine]; };
-    auto is_multi = [&](int k) { return (scanned(k, 5) & 1) != 0; };       // rows split over several ELL rows
-    auto has_dense = [&](int k) { return (scanned(k, 5) & 2) != 0; };
-    auto has_wide = [&](int k) { return (scanned(k, 5) & 4) != 0; };
+    auto is_multi = [&](int k) { return (scanned(k, kScanFound) & 1) != 0; };       // rows split over several ELL rows
+    auto has_dense = [&](int k) { return (scanned(k, kScanFound) & 2) != 0; };
+    auto has_wide = [&](int k) { return (scanned(k, kScanFound) & 4) != 0; };
     const int n_zero = *back.as<int>(o_zero);
     // Candidates whose sample shows shared columns.  Neither the groups nor the cells know segments, they store every
     // ELL row as a row of C: a bucket that holds a split row stays with the tiles.
@@ -1703,9 +1699,10 @@ int lf_spmm_create(lf_spmm_plan** out_plan, const lf_bucket_desc* h_buckets, int
     {
         double slots = 0.0;
         for (int k = 0; k < num_buckets; ++k) {
-            if (samples[k] == 0) continue;
+            if (h_buckets[k].num_ell_rows == 0) continue;
             const double mine = (double)h_buckets[k].num_ell_rows * h_buckets[k].width;
-            span += mine * (double)back.as<unsigned long long>(o_sample)[3 * k + 2] / (double)samples[k];
+            const double samples = (double)lf::ceil_div(h_buckets[k].num_ell_rows, (int64_t)h_table[k].span_stride);
+            span += mine * scanned(k, kScanSpan) / samples / kSpanUnits * (double)cols_p;
             slots += mine;
         }
         if (slots > 0.0) span /= slots;

@@ -558,12 +558,15 @@ inline XcdParts xcd_parts(int pieces, int wide) {
 // group_rows(lanes of a row) each to a CU, and hardly a row of B that another XCD uses.  Stencils of 4K to 800K points, us,
 // slices as if for a random matrix -> now, without any: plans, 27-point, 62K points, N = 416 124 -> 107, 107; 7-point, 21K, N = 256
 // 14.9 -> 13.3, 13.3; 7-point, 160K, N = 352 138 -> 98, 138; CSR, 27-point, 62K, N = 416 167 -> 121, 121; 7-point, 21K, N = 256
-// 18.1 -> 10.7, 10.7.  301 plans and 320 CSR products, every S timed: 4.5 and 7.1 % above the best S before, now 1.7 and
-// 1.6.
+// 18.1 -> 10.7, 10.7.  301 plans and 320 CSR products, every S timed: 4.5 and 7.1 % above the best S before,
+// now 1.2 and 1.0; of 250 more plans 4 % are more than 3 % slower than with the slices of a random matrix, 17 % at worst.
 constexpr int kNearGroupsPerCu = 4, kCusOfXcd = 32;
+// Near columns hit an L1 as well as an L2, and by 15 TB/s; what does not fit is lost faster, by the 1.4th power.
+constexpr double kNearHitRate = 15e6, kNearPower = 1.4;
 struct Neighbours {
     double span = 0.0;                                     // 0: not known
     int64_t num_rows = 0;
+    double per_sub = 0.0;                                  // what hits take longer for a doubling of the sub-waves to a wavefront
 };
 inline bool is_near(double span, int64_t num_cols) { return span > 0.0 && 2.0 * span < (double)num_cols; }
 
@@ -591,8 +594,9 @@ inline Slices feature_slices(int64_t num_cols, int64_t entries, int feat, int dt
         const double share = weight / (2.0 * wide * kXcds);
         const double bytes = gathered * weight / (2.0 * pieces);
         const double lanes = 16.0 * (double)entries * lpr * ch * weight / (wide + pieces - (n - 1) * wide);
+        const bool near = is_near(neighbours.span, num_cols);
         double uses = (double)entries / (double)num_cols * share, in_use = (double)num_cols;
-        if (is_near(neighbours.span, num_cols)) {
+        if (near) {
             const double rows = (double)neighbours.num_rows;
             const double in_flight = std::min(rows * share, kNearGroupsPerCu * kCusOfXcd * group_rows(lpr));
             in_use = std::min(in_use, neighbours.span + in_flight * (double)num_cols / rows);
@@ -601,11 +605,12 @@ inline Slices feature_slices(int64_t num_cols, int64_t entries, int feat, int dt
         const double again = std::max(0.0, 1.0 - kFirstUse / uses), slice_bytes = in_use * width * elem;
         const int lg_subs = lf::ilog2(64 / lpr);
         auto priced = [&](double hit, double per_sub) {
-            return adjust(n, width, lg_subs, lanes * hit / kHitRate * (1.0 + per_sub * lg_subs) +
+            return adjust(n, width, lg_subs, lanes * hit / (near ? kNearHitRate : kHitRate) * (1.0 + per_sub * lg_subs) +
                                              bytes * (1.0 - hit) / kMissRate * (width == step ? kMiss128 : 1.0) +
                                              8.0 * (double)entries * n / kMissRate);
         };
-        const double price = priced(std::min(1.0, kL2 / slice_bytes) * again, kPerSub);
+        const double held_share = std::min(1.0, kL2 / slice_bytes);
+        const double price = near ? priced(std::pow(held_share, kNearPower) * again, neighbours.per_sub) : priced(held_share * again, kPerSub);
         if (n == 1 || price < least) {
             const double held = kSoftL2 / slice_bytes;
             least = price;
