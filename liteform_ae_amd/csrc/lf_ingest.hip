@@ -2,9 +2,10 @@
 // the row pointer.  This is what the reference's matrix container does on the host every
 // time a CSR view is asked for (playground_pipline/format_matrix_market.py:74-76:
 // scipy's coo.tocsr(), which sorts columns and sums duplicates); it is the step that feeds
-// lf_bucket_stats / lf_hyb_build.  Up to some ten million entries without duplicates go through bins of rows
-// that are sorted in LDS, a kernel each for counting, offsets, distribution and sorting; anything else through plain
-// library primitives (rocPRIM radix sort and reduce-by-key on a 64-bit key row * cols + col), with kernels
+// lf_bucket_stats / lf_hyb_build.  Up to 8.4 million entries go through bins of rows that are sorted in LDS, a kernel each
+// for counting, offsets, distribution and sorting, and three more that add up duplicates; more of them, bins that do not
+// fit and entries outside the matrix through plain library
+// primitives (rocPRIM radix sort and reduce-by-key on a 64-bit key row * cols + col), with kernels
 // that pack / unpack keys and locate the row boundaries.
 //
 // Also here: the structural check of CSR arrays that come from a caller (lf_csr_check), which
