@@ -614,3 +614,27 @@ def test_span_of_neighbouring_rows(fa, torch):
     assert span(np.array([3]), [5, 17, 99], 100) == int(94 * 4096 // 100 * 100 / 4096)
     assert span(np.zeros(50, np.int64), [], 100) == 0
     assert span(np.array([3]), [17, 5, 99], 100) == 0
+
+
+def test_csr_product_of_near_columns_from_either_input(fa, torch):
+    """A stencil as CSR arrays and as triplets in no order: both know that its columns are near, a matrix with the columns
+    shuffled does not, and the products are those of the oracle."""
+    rng = np.random.default_rng(9)
+    g = grid_stencil(rng, (40, 24, 30))
+    indptr, indices, data = g.adj_tensors("csr")
+    n, feat = 40 * 24 * 30, 288
+    order = rng.permutation(len(indices))
+    row = np.repeat(np.arange(n, dtype=np.int32), np.diff(indptr))
+    shuffled = rng.permutation(n)[indices].astype(np.int32)
+    B = rng.uniform(-1, 1, size=(n, feat)).astype(np.float32)
+    Bd = torch.from_numpy(B).cuda()
+    for cols, near in ((np.asarray(indices), True), (shuffled, False)):
+        made = [MTX.from_coo(row[order], cols[order], (n, n), data=data[order])]
+        if near:
+            made.append(MTX.from_csr(indptr, indices, (n, n), data=data))
+        for m in made:
+            ip, ix, v = m.adj_tensors("csr")
+            C = fa.spmm_csr(m, Bd).cpu().numpy()
+            assert (np.abs(C - O.spmm_csr_f64(ip, ix, v, (n, n), B)) <= TOL * O.spmm_abs_bound(ip, ix, v, (n, n), B)).all()
+            span = fa._device_csr(m).span
+            assert (40 * 24 < span < n / 8) if near else span > n / 2, (span, m)
