@@ -488,6 +488,31 @@ def test_split_rows_that_share_columns(fa, torch, feat, b_dtype, windows):
         assert info["row_group_buckets"] >= 1                                  # the bucket without split rows shares its gathers
 
 
+@pytest.mark.parametrize("deg", [128, 256])
+@pytest.mark.parametrize("feat,b_dtype", [(32, "f32"), (64, "f32"), (128, "f32"), (256, "f32"), (64, "bf16"), (128, "bf16")])
+def test_long_rows_are_no_long_chains_of_additions(fa, torch, feat, b_dtype, deg):
+    """1, then values of a quarter of its last place: added one by one they are all lost.  A row has at most 64 entries to
+    a sub-wave, or all of them where a wavefront is one sub-wave: 7 additions in a batch of eight, one for every batch
+    and one for every doubling of the sub-waves, each of them off by 2^-24 of the sum at most."""
+    n, tiny = 2500, 2.0**-25
+    lanes = feat // (8 if b_dtype == "bf16" else 4)
+    rng = np.random.default_rng(deg)
+    col = np.sort((rng.integers(n, size=(n, 1)) + np.arange(deg)) % n, axis=1).ravel()
+    data = np.where(np.arange(n * deg) % deg == 0, 1.0, tiny).astype(np.float32)
+    g = MTX.from_coo(np.repeat(np.arange(n), deg), col, (n, n), data=data)
+    B = torch.ones((n, feat), dtype=torch.bfloat16 if b_dtype == "bf16" else torch.float32, device="cuda")
+    additions = 7 + max(64, deg * lanes // 64) // 8 + (64 // lanes).bit_length() - 1
+    results = {}
+    if b_dtype == "f32":
+        results["csr"] = fa.spmm_csr(g, B)
+    if lanes <= 16:                                        # with more, such rows are staged in LDS and not streamed
+        plan = fa.HybSpMM(fa.build_hyb_format_device(g, [[deg]]), feat, b_dtype)
+        results["plan"] = plan.run(B)
+        plan.close()
+    for name, C in results.items():
+        assert float((C.double() - (1.0 + (deg - 1) * tiny)).abs().max()) <= additions * 2.0**-24, name
+
+
 def sliced_matrix(rng, nr, nc):
     """Rows of every kind that a plan treats in its own way, in mixed order: empty, 1..64 entries, 65..256 in such
     numbers that wavefronts take them (more than 1024 above 64 entries, more than 2048 above 128), and a few
