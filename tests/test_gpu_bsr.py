@@ -144,6 +144,20 @@ def test_every_short_block_row(fa, torch, feat, bs):
     check(fa, torch, sp.bsr_matrix((data, indices, indptr), shape=(10 * bs, 12 * bs)), feat)
 
 
+@pytest.mark.parametrize("bs", [16, 32, 64])
+@pytest.mark.parametrize("feat,times", [(8, 1), (24, 1), (32, 1), (40, 1), (56, 1), (64, 1), (72, 1), (16, 60), (48, 60), (64, 60), (64, 300), (64, 70),
+                                        (128, 26), (136, 26)])
+def test_features_per_lane_and_paired_wavefronts(fa, torch, feat, times, bs):
+    """Two, four and eight features per lane, full and not, and for blocks of 64 both wavefronts of a
+    block row of 0 to 9 blocks, up to 512 of them (256 with four features per lane above 64)."""
+    rng = np.random.default_rng(bs + feat + times)
+    counts = np.concatenate([rng.permutation(10) for _ in range(times)])
+    indptr = np.concatenate([[0], np.cumsum(counts)]).astype(np.int32)
+    indices = np.concatenate([np.sort(rng.choice(12, size=n, replace=False)) for n in counts]).astype(np.int32)
+    data = rng.uniform(-1, 1, size=(len(indices), bs, bs)).astype(np.float16).astype(np.float32)
+    check(fa, torch, sp.bsr_matrix((data, indices, indptr), shape=(len(counts) * bs, 12 * bs)), feat)
+
+
 @pytest.mark.parametrize("mb,feat", [(4095, 40), (4096, 128), (4097, 40), (4099, 136)])
 def test_wavefronts_alone_and_in_fours(fa, torch, mb, feat):
     """Up to 4096 block rows of one feature tile go out as single wavefronts, more in workgroups of four."""
@@ -167,7 +181,7 @@ def test_long_block_rows_of_a_large_product(fa, torch, bs, mb, feat):
 
 
 @pytest.mark.parametrize("bs", [16, 32, 64])
-@pytest.mark.parametrize("feat", [40, 128])
+@pytest.mark.parametrize("feat", [24, 40, 128])
 def test_infinite_rows_of_x(fa, torch, feat, bs):
     """A row of X of +Inf or -Inf, met by block rows of 1 to 6 blocks as their first, a middle or their
     last block: Inf where the entries of A it meets are positive or negative, nothing elsewhere."""
