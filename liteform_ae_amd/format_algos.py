@@ -215,6 +215,9 @@ class _DeviceCSR:
         self._seg_deg = {}
         self._stats_ws = {}          # num_parts -> statistics workspace holding the row bounds
         self._span = None
+        self._long_rows = None       # list of long rows and its counts, see csr_work
+        self._csr_work = {}
+        self._csr_lock = threading.Lock()
         src = getattr(g, "_csr_source", None)
         if src is not None and self._from_csr(src, bool(getattr(g, "_unit_values", False))):
             self.path = "csr"
@@ -294,6 +297,29 @@ class _DeviceCSR:
         self._values = values[:self.nnz]
         # duplicates of unit entries add up to 2, 3, ...: only a duplicate-free unit matrix is "all ones"
         self.all_ones = ones and self.nnz == self.coo_nnz
+
+    def csr_work(self, feat: int, dtype: int):
+        """What the C call of a CSR product takes: ((rows, columns, entries, span), address of the list of long rows, address of
+        its counts, bytes of work space).  The list
+        (lf_csr_long_rows) is made for the matrix' first product and kept with it; a product that is recorded into a graph
+        before there is one does without."""
+        work = self._csr_work.get((feat, dtype))
+        if work is None:
+            lib = _lib.load()
+            with self._csr_lock:
+                if self._long_rows is None and not _torch().cuda.is_current_stream_capturing():
+                    rows = _gpu_torch.empty(lib.lf_csr_long_rows_bytes(self.nnz), dtype=_gpu_torch.uint8, device="cuda")
+                    counts = np.zeros(3, dtype=np.int64)
+                    _lib.check(lib.lf_csr_long_rows(self.indptr.data_ptr(), self.num_rows, self.nnz, rows.data_ptr(), rows.numel(),
+                                                    _lib.np_ptr(counts, C.c_int64), _stream()))
+                    self._long_rows = (rows, counts) if counts[0] else (None, None)
+            rows, counts = self._long_rows or (None, None)
+            at = None if rows is None else _lib.np_ptr(counts, C.c_int64)
+            sizes = (self.num_rows, self.num_cols, self.nnz, self.span)
+            work = (sizes, _lib.ptr(rows), at, lib.lf_csr_spmm_work_bytes(*sizes, at, feat, dtype))
+            if self._long_rows is not None:
+                self._csr_work[(feat, dtype)] = work
+        return work
 
     def seg_deg(self, num_parts: int):
         """Per-(partition,row) COO degrees on the device, or None when CSR lengths are the same."""
@@ -657,13 +683,18 @@ def spmm_csr(g, B, b_dtype: str = "f32", use_values: bool = True):
     torch = _torch()
     lib = _lib.load()
     dev = _device_csr(g)
-    feat = int(B.shape[1])
-    out = torch.empty((dev.num_rows, feat), dtype=torch.float32, device="cuda")
+    feat, dtype = int(B.shape[1]), _B_DTYPES[b_dtype]
+    out = dev.indptr.new_empty((dev.num_rows, feat), dtype=torch.float32)
     vals = dev.values if use_values else None
+    sizes, rows, counts, nbytes = dev._csr_work.get((feat, dtype)) or dev.csr_work(feat, dtype)
     # the device arrays were made by lf_coo_to_csr or have passed lf_csr_check: no second check
-    rc = lib.lf_csr_spmm_trusted_span(dev.indptr.data_ptr(), dev.indices.data_ptr(), None if vals is None else vals.data_ptr(),
-                                      dev.num_rows, dev.num_cols, dev.nnz, dev.span, feat, _B_DTYPES[b_dtype], B.data_ptr(),
-                                      out.data_ptr(), _stream())
+    if nbytes:
+        work = torch.empty(nbytes, dtype=torch.uint8, device="cuda")
+        rc = lib.lf_csr_spmm_trusted_work(dev.indptr.data_ptr(), dev.indices.data_ptr(), None if vals is None else vals.data_ptr(), *sizes,
+                                          rows, counts, work.data_ptr(), nbytes, feat, dtype, B.data_ptr(), out.data_ptr(), _stream())
+    else:
+        rc = lib.lf_csr_spmm_trusted_span(dev.indptr.data_ptr(), dev.indices.data_ptr(), None if vals is None else vals.data_ptr(), *sizes,
+                                          feat, dtype, B.data_ptr(), out.data_ptr(), _stream())
     if rc:
         _lib.check(rc)
     return out
