@@ -220,10 +220,10 @@ constexpr int kStatLine = 16;              // 64-bit words
 __host__ __device__ constexpr size_t stat_at(int p, int k, int f) { return (((size_t)p * LF_MAX_CLASSES + k) * 3 + f) * kStatLine; }
 
 // stats(p, k) += {cost rows, nnz, 1} for every segment of partition p = blockIdx.y.
-// A thread keeps the counters of its rows in registers; a workgroup adds its sums with one atomic
-// per counter.  (LDS atomics per row, from 2048 workgroups, took 48 us for 2.45M rows, this takes
-// 21.)
-constexpr int kCountGrid = 512;
+// A workgroup counts a contiguous range of rows in LDS - a 64-bit word {segments, entries} for every class and lane, so that the
+// lanes of a wavefront never meet - and adds its sums with one atomic per counter.  (One word per class took 48 us for 2.45M
+// rows, counters in registers, 33 selects a row, 22, this takes 12.)
+constexpr int kCountGrid = 256, kCountThreads = 1024;      // (atomics of 512 workgroups on a counter's line: 9 us)
 constexpr int kRowUnroll = 4;              // rows whose bounds a thread requests together
 
 // Degrees of the segments of rows r0, r0 + stride, ... (0 past `end`).
@@ -240,44 +240,60 @@ __device__ __forceinline__ void seg_degrees(const SegView& v, const int32_t* __r
     }
 }
 
-__global__ void __launch_bounds__(kBlock)
-class_count_kernel(SegView v, const int32_t* __restrict__ seg_deg, int kmax, unsigned long long* __restrict__ stats) {
-    constexpr int kStride = kBlock + 4;
-    __shared__ uint32_t s_sum[LF_MAX_CLASSES * 3 * kStride];
+// What the workgroups of class_count_kernel counted, for class_list_kernel: segments of class k of partition p in workgroup g;
+// kmax + 1: of the last class, those of more than kMarkBigSegment entries.
+constexpr int kCountClasses = 16;
+__host__ __device__ constexpr size_t count_at(int p, int k, int g) { return ((size_t)p * kCountClasses + k) * kCountGrid + g; }
+constexpr int kMarkBigSegment = 8192;      // longer segments are shared by all workgroups of their item, see below
+
+__global__ void __launch_bounds__(kCountThreads)
+class_count_kernel(SegView v, const int32_t* __restrict__ seg_deg, int kmax, unsigned long long* __restrict__ stats, int32_t* __restrict__ counts) {
+    static_assert(LF_MAX_CLASSES < kCountClasses && kCountThreads == 64 * kCountClasses);
+    constexpr int kCntShift = 40;          // entries of a lane's rows stay below 2^31, their number below 2^23
+    __shared__ unsigned long long s_sum[LF_MAX_CLASSES * 64];
+    __shared__ uint32_t s_more, s_big;     // cost rows beyond one a segment; segments of more than kMarkBigSegment entries
     const int p = blockIdx.y;
-    uint32_t cost[LF_MAX_CLASSES] = {}, nnz[LF_MAX_CLASSES] = {}, cnt[LF_MAX_CLASSES] = {};
-    const int64_t stride = (int64_t)gridDim.x * kBlock;
-    for (int64_t r0 = (int64_t)blockIdx.x * kBlock + threadIdx.x; r0 < v.rows; r0 += kRowUnroll * stride) {
+    for (int i = threadIdx.x; i < LF_MAX_CLASSES * 64; i += kCountThreads) s_sum[i] = 0;
+    if (threadIdx.x == 0) s_more = s_big = 0;
+    __syncthreads();
+    const int64_t per = (v.rows + gridDim.x - 1) / gridDim.x;
+    const int64_t lo = (int64_t)blockIdx.x * per, hi = lo + per < v.rows ? lo + per : v.rows;
+    unsigned long long* mine = s_sum + (threadIdx.x & 63);
+    for (int64_t r0 = lo + threadIdx.x; r0 < hi; r0 += kRowUnroll * kCountThreads) {
         int deg[kRowUnroll];
-        seg_degrees(v, seg_deg, p, r0, stride, v.rows, deg);
+        seg_degrees(v, seg_deg, p, r0, kCountThreads, hi, deg);
 #pragma unroll
         for (int u = 0; u < kRowUnroll; ++u) {
-            int k = -1, cost_rows = 0;
-            if (deg[u] > 0) width_class(deg[u], kmax, k, cost_rows);
-#pragma unroll
-            for (int i = 0; i < LF_MAX_CLASSES; ++i) {
-                cost[i] += k == i ? (uint32_t)cost_rows : 0u;
-                nnz[i] += k == i ? (uint32_t)deg[u] : 0u;
-                cnt[i] += k == i ? 1u : 0u;
-            }
+            if (deg[u] <= 0) continue;
+            int k, cost_rows;
+            width_class(deg[u], kmax, k, cost_rows);
+            atomicAdd(&mine[k * 64], (1ull << kCntShift) | (unsigned long long)deg[u]);
+            if (cost_rows > 1) atomicAdd(&s_more, (uint32_t)(cost_rows - 1));
+            if (deg[u] > kMarkBigSegment && k == kmax) atomicAdd(&s_big, 1u);
         }
     }
-#pragma unroll
-    for (int i = 0; i < LF_MAX_CLASSES; ++i) {
-        s_sum[(3 * i) * kStride + threadIdx.x] = cost[i];
-        s_sum[(3 * i + 1) * kStride + threadIdx.x] = nnz[i];
-        s_sum[(3 * i + 2) * kStride + threadIdx.x] = cnt[i];
-    }
     __syncthreads();
-    // four threads to a counter
-    const int c = threadIdx.x >> 2, part = threadIdx.x & 3;
-    if (c < 3 * LF_MAX_CLASSES) {
-        uint32_t sum = 0;
-        for (int i = part; i < kBlock; i += 4) sum += s_sum[c * kStride + i];
-        sum += __shfl_xor(sum, 1);
-        sum += __shfl_xor(sum, 2);
-        if (part == 0 && sum) atomicAdd(&stats[stat_at(p, c / 3, c % 3)], (unsigned long long)sum);
+    const int k = threadIdx.x >> 6;                                          // a wavefront to a class
+    unsigned long long nnz = 0;
+    uint32_t cnt = 0;
+    if (k < LF_MAX_CLASSES) {
+        const unsigned long long x = s_sum[threadIdx.x];
+        nnz = x & ((1ull << kCntShift) - 1);
+        cnt = (uint32_t)(x >> kCntShift);
     }
+    for (int d = 1; d < 64; d <<= 1) {
+        nnz += __shfl_xor(nnz, d);
+        cnt += __shfl_xor(cnt, d);
+    }
+    if ((threadIdx.x & 63) != 0) return;
+    const uint32_t big = s_big;
+    if (k < LF_MAX_CLASSES && cnt) {
+        atomicAdd(&stats[stat_at(p, k, 0)], (unsigned long long)cnt + (k == kmax ? s_more : 0u));
+        atomicAdd(&stats[stat_at(p, k, 1)], nnz);
+        atomicAdd(&stats[stat_at(p, k, 2)], (unsigned long long)cnt);
+        if (k == kmax && big) atomicAdd(&stats[stat_at(p, k, 2) + 2], (unsigned long long)big);      // (a spare word of the counter's line)
+    }
+    if (counts) counts[count_at(p, k, blockIdx.x)] = (int)(k == kmax + 1 ? big : k == kmax ? cnt - big : k < kmax ? cnt : 0u);
 }
 
 // ---- statistics of several partition counts at once
@@ -494,9 +510,7 @@ constexpr int kMarkMaxSlices = 8;          // every slice of a partition streams
 constexpr int64_t kMarkMinRows = 131072;
 constexpr int64_t kMarkMaxSegments = 1ll << 26;     // 8 bytes each in the workspace
 constexpr int kMarkUnrollB = 8;
-constexpr int kMarkBigSegment = 8192;      // longer segments are shared by all workgroups of their item
 constexpr int kMarkEntries = 16384;        // entries that are worth one more workgroup
-constexpr int kListGrid = 512;
 
 struct MarkShape {
     int slices;              // slices of a partition; 0: the bitmap path does not apply
@@ -519,49 +533,47 @@ MarkShape mark_shape(int64_t rows, int64_t cols, int parts) {
 }
 
 // lists[p * rows + first segment of class k ..) = (start, fill) of the segments of class k of partition
-// p; the classes follow one another, a class's segments are in no particular order except that those
-// of more than kMarkBigSegment entries are the last of the last class.
-__global__ void __launch_bounds__(kBlock)
-class_list_kernel(SegView v, const int32_t* __restrict__ seg_deg, int kmax,
-                  unsigned long long* __restrict__ stats,
-                  int2* __restrict__ lists) {
-    __shared__ uint32_t s_cnt[LF_MAX_CLASSES + 1], s_at[LF_MAX_CLASSES + 1];
+// p; the classes follow one another, a class's segments in the order of the workgroups' row ranges, those
+// of more than kMarkBigSegment entries behind the last class.  The ranges are class_count_kernel's, whose counts say where a
+// workgroup's segments go (a sweep of its own to count them again and an atomic per class and workgroup: 27 us for 2.45M rows, this 12).
+__global__ void __launch_bounds__(kCountThreads)
+class_list_kernel(SegView v, const int32_t* __restrict__ seg_deg, int kmax, const int32_t* __restrict__ counts, int2* __restrict__ lists) {
+    __shared__ uint32_t s_at[kCountClasses], s_all[kCountClasses];
     const int p = blockIdx.y;
-    if (threadIdx.x <= LF_MAX_CLASSES) s_cnt[threadIdx.x] = 0;
-    __syncthreads();
-    const int64_t per = (v.rows + gridDim.x - 1) / gridDim.x;
-    const int64_t lo = (int64_t)blockIdx.x * per, hi = lo + per < v.rows ? lo + per : v.rows;
-    for (int64_t r0 = lo + threadIdx.x; r0 < hi; r0 += kRowUnroll * kBlock) {
-        int deg[kRowUnroll];
-        seg_degrees(v, seg_deg, p, r0, kBlock, hi, deg);
-#pragma unroll
-        for (int u = 0; u < kRowUnroll; ++u) {
-            int k, cost_rows;
-            if (deg[u] <= 0) continue;
-            width_class(deg[u], kmax, k, cost_rows);
-            atomicAdd(&s_cnt[deg[u] > kMarkBigSegment && k == kmax ? kmax + 1 : k], 1u);
+    {
+        const int k = threadIdx.x >> 6, part = threadIdx.x & 63;
+        uint32_t before = 0, all = 0;
+        for (int g = part; g < (int)gridDim.x; g += 64) {
+            const uint32_t n = (uint32_t)counts[count_at(p, k, g)];
+            all += n;
+            before += g < (int)blockIdx.x ? n : 0u;
+        }
+        for (int d = 1; d < 64; d <<= 1) {
+            before += __shfl_xor(before, d);
+            all += __shfl_xor(all, d);
+        }
+        if (part == 0) {
+            s_at[k] = before;
+            s_all[k] = all;
         }
     }
     __syncthreads();
-    if (threadIdx.x <= (unsigned)kmax + 1) {
-        // (the cursors are spare words of the counters' lines; kmax + 1 are the last class's longest
-        // segments, listed from its end)
-        const int k = min((int)threadIdx.x, kmax), big = (int)threadIdx.x > kmax;
-        uint32_t first = 0;
-        for (int i = 0; i < k + big; ++i) first += (uint32_t)stats[stat_at(p, i, 2)];
-        const uint32_t n = s_cnt[threadIdx.x];
-        const uint32_t taken = n ? (uint32_t)atomicAdd(&stats[stat_at(p, k, 2) + 1 + big], (unsigned long long)n) : 0u;
-        s_at[threadIdx.x] = big ? first - taken - n : first + taken;
+    if (threadIdx.x < kCountClasses) {
+        uint32_t first = s_at[threadIdx.x];
+        for (int i = 0; i < (int)threadIdx.x; ++i) first += s_all[i];
+        s_at[threadIdx.x] = first;
     }
     __syncthreads();
+    const int64_t per = (v.rows + gridDim.x - 1) / gridDim.x;
+    const int64_t lo = (int64_t)blockIdx.x * per, hi = lo + per < v.rows ? lo + per : v.rows;
     int2* out = lists + (size_t)p * (size_t)v.rows;
-    for (int64_t r0 = lo + threadIdx.x; r0 < hi; r0 += kRowUnroll * kBlock) {
+    for (int64_t r0 = lo + threadIdx.x; r0 < hi; r0 += kRowUnroll * kCountThreads) {
         int deg[kRowUnroll], start[kRowUnroll], fill[kRowUnroll];
-        seg_degrees(v, seg_deg, p, r0, kBlock, hi, deg);
+        seg_degrees(v, seg_deg, p, r0, kCountThreads, hi, deg);
 #pragma unroll
         for (int u = 0; u < kRowUnroll; ++u) {
             start[u] = fill[u] = 0;
-            if (r0 + u * kBlock < hi) seg_range(v, r0 + u * kBlock, p, start[u], fill[u]);
+            if (r0 + u * kCountThreads < hi) seg_range(v, r0 + u * kCountThreads, p, start[u], fill[u]);
         }
 #pragma unroll
         for (int u = 0; u < kRowUnroll; ++u) {
@@ -869,32 +881,35 @@ __global__ void __launch_bounds__(1024)
 hyb_scan_kernel(int32_t* __restrict__ blockcnt, int nblk, long long* __restrict__ totals,
                 const int32_t* __restrict__ widths, int* __restrict__ done, BucketOffsets* __restrict__ offs) {
     __shared__ long long s_wave[16];
-    __shared__ long long s_carry;
     __shared__ int s_last;
     int32_t* a = blockcnt + (int64_t)blockIdx.x * nblk;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    if (threadIdx.x == 0) s_carry = 0;
+    // a thread's consecutive blocks, then one scan over the threads (a scan over 1024 blocks at a time, with its barriers,
+    // was 18 us for 9571 blocks, this is 7)
+    const int per = (nblk + 1023) / 1024, from = min((int)threadIdx.x * per, nblk), to = min(from + per, nblk);
+    long long mine = 0;
+#pragma unroll 8
+    for (int i = from; i < to; ++i) mine += a[i];
+    long long incl = mine;
+    for (int d = 1; d < 64; d <<= 1) {
+        const long long y = __shfl_up(incl, d);
+        if (lane >= d) incl += y;
+    }
+    if (lane == 63) s_wave[wave] = incl;
     __syncthreads();
-    for (int base = 0; base < nblk; base += 1024) {
-        const int i = base + threadIdx.x;
-        const long long x = i < nblk ? a[i] : 0;
-        long long incl = x;
-        for (int d = 1; d < 64; d <<= 1) {
-            const long long y = __shfl_up(incl, d);
-            if (lane >= d) incl += y;
-        }
-        if (lane == 63) s_wave[wave] = incl;
-        __syncthreads();
-        long long wave_off = 0;
-        for (int wv = 0; wv < wave; ++wv) wave_off += s_wave[wv];
-        const long long carry = s_carry;
-        if (i < nblk) a[i] = (int32_t)(carry + wave_off + incl - x);
-        __syncthreads();
-        if (threadIdx.x == 1023) s_carry = carry + wave_off + incl;
-        __syncthreads();
+    long long before = incl - mine, all = 0;
+    for (int w = 0; w < 16; ++w) {
+        before += w < wave ? s_wave[w] : 0;
+        all += s_wave[w];
+    }
+#pragma unroll 8
+    for (int i = from; i < to; ++i) {
+        const int x = a[i];
+        a[i] = (int32_t)before;
+        before += x;
     }
     if (threadIdx.x == 0) {
-        __hip_atomic_store(&totals[blockIdx.x], s_carry, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __hip_atomic_store(&totals[blockIdx.x], all, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         // (release: the total above is visible before the count; acquire: so are the others')
         s_last = __hip_atomic_fetch_add(done, 1, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT) == (int)gridDim.x - 1;
     }
@@ -1141,7 +1156,7 @@ hyb_fill_kernel(SegView v, const int32_t* __restrict__ seg_deg, const int32_t* _
 
 // ---------------------------------------------------------------------------- host helpers
 struct StatsLayout {
-    size_t bnd, planes, lists, bitmaps, table, stats, hist, total;
+    size_t bnd, planes, lists, counts, bitmaps, table, stats, hist, total;
 };
 
 StatsLayout stats_layout(int64_t rows, int64_t cols, int parts) {
@@ -1153,6 +1168,8 @@ StatsLayout stats_layout(int64_t rows, int64_t cols, int parts) {
     L.planes = L.lists = L.bitmaps = L.table = off;      // byte planes, or segment lists and bitmaps
     if (m.slices > 0) {
         off += align_up((size_t)parts * (size_t)rows * 8, 256);
+        L.counts = off;
+        off += align_up(count_at(parts, 0, 0) * 4, 256);
         L.bitmaps = off;
         off += align_up((size_t)m.groups * (size_t)m.words * 4, 256);
         L.table = off;
@@ -1300,14 +1317,15 @@ int lf_bucket_stats(const int32_t* d_indptr, const int32_t* d_indices, const int
         }
         SegView v{d_indptr, bnd, num_rows, num_parts};
         const int num_classes = lf::ilog2(width_limit) + 1;
-        class_count_kernel<<<dim3(std::min((nblk + kRowUnroll - 1) / kRowUnroll, kCountGrid), num_parts), kBlock, 0, s>>>(v, d_seg_deg, num_classes - 1, stats);
+        const dim3 count_grid((unsigned)std::min<int64_t>(lf::ceil_div(num_rows, kCountThreads), kCountGrid), (unsigned)num_parts);
+        int32_t* counts = h_colhist && !use_planes ? (int32_t*)(ws + L.counts) : nullptr;
+        class_count_kernel<<<count_grid, kCountThreads, 0, s>>>(v, d_seg_deg, num_classes - 1, stats, counts);
         LF_HIP(hipGetLastError());
-        if (h_colhist && !use_planes) {
+        if (counts) {
             int2* lists = (int2*)(ws + L.lists);
             uint32_t* bitmaps = (uint32_t*)(ws + L.bitmaps);
             int32_t* table = (int32_t*)(ws + L.table);
-            class_list_kernel<<<dim3(std::min(nblk, kListGrid), num_parts), kBlock, 0, s>>>(
-                v, d_seg_deg, num_classes - 1, stats, lists);
+            class_list_kernel<<<count_grid, kCountThreads, 0, s>>>(v, d_seg_deg, num_classes - 1, counts, lists);
             LF_HIP(hipGetLastError());
             LF_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(mark_columns_kernel),
                                        hipFuncAttributeMaxDynamicSharedMemorySize, kMarkMaxWords * 4));
@@ -1327,12 +1345,11 @@ int lf_bucket_stats(const int32_t* d_indptr, const int32_t* d_indices, const int
             LF_HIP(hipGetLastError());
         }
     }
-    const size_t lines_bytes = stat_at(num_parts, 0, 0) * 8;
+    const size_t lines_bytes = L.hist - L.stats;
     lf::PinnedLoan back(lines_bytes + (h_colhist ? hist_bytes : 0));
     LF_REQUIRE(back.ok(), LF_ERR_HIP, "out of host memory");
     const unsigned long long* h_lines = back.as<unsigned long long>();
-    LF_HIP(hipMemcpyAsync(back.as<char>(), stats, lines_bytes, hipMemcpyDeviceToHost, s));
-    if (h_colhist) LF_HIP(hipMemcpyAsync(back.as<char>(lines_bytes), hist, hist_bytes, hipMemcpyDeviceToHost, s));
+    LF_HIP(hipMemcpyAsync(back.as<char>(), stats, lines_bytes + (h_colhist ? hist_bytes : 0), hipMemcpyDeviceToHost, s));      // (hist is behind stats)
     LF_HIP(hipStreamSynchronize(s));
     for (int p = 0; p < num_parts; ++p)
         for (int k = 0; k < LF_MAX_CLASSES; ++k)

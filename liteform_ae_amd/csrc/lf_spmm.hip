@@ -720,7 +720,7 @@ __device__ __forceinline__ int merge_group(const int32_t* __restrict__ cols, con
 #pragma unroll
     for (int r = 0; r < kGroupRows; ++r) {
         const long long e = g * kGroupRows + r;
-        len[r] = e < n_rows ? (meta[e] & (int)kMetaLenMask) : 0;
+        len[r] = e < n_rows ? min(meta[e] & (int)kMetaLenMask, 1 << log_w) : 0;      // (meta words may not be checked yet)
         base[r] = e << log_w;
         pos[r] = 0;
         cbuf[r] = make_int4(0, 0, 0, 0);
@@ -1056,10 +1056,12 @@ struct PlanBucket {
     long long n_rows;
     int log_w;
     int part;
-    int n_blocks;              // workgroups of plan_scan_kernel, and one more unless there are none
+    int n_blocks;              // workgroups of plan_scan_kernel, behind n_first others
+    int n_first;               // one for the span, and those of the row-group sampling; none without n_blocks
     int sample_stride;         // row-group sampling: every sample_stride-th group is looked at (0: no candidate)
     int span_stride;           // every span_stride-th row is looked at for the span of neighbours' columns
     int all_cols;              // columns of a partition
+    int first_line, n_lines;   // of its counters
 };
 
 // One pass over all buckets of a plan:
@@ -1067,28 +1069,39 @@ struct PlanBucket {
 //     inside B, 1..W valid slots per ELL row, and segments (a head that announces n ELL rows followed
 //     by continuation rows 1..n-1 with the same row id) that are complete and stay inside the
 //     bucket.  flags[0] bad column, [1] bad row, [2] bad meta;
-//   * counts what lf_spmm_create sizes its tables by: counters[(kScanCounters k + i) * kCounterLine] of bucket
+//   * counts what lf_spmm_create sizes its tables by: counter i, in each of the bucket's lines, of bucket
 //     k = chunks of the rows of more than kCoopSlots slots, rows with several chunks, their partial
 //     rows, rows of 65 .. 128 and of 129 .. kCoopSlots slots (a chunk each if they take the cooperative
 //     path), ChunkedRow::found of all rows; and by a workgroup of its own, not to lengthen the others, the columns that
 //     groups of kGroupRows neighbours span (every span_stride-th row and those behind it, in kSpanUnits of all columns; all,
 //     where one is a part of a row, which says nothing);
-//   * marks the rows that partition 0 writes.
+//   * marks the rows that partition 0 writes;
+//   * samples the row-group candidates: of every sample_stride-th group of four rows, samples[3 k ..] = merged entries among the
+//     first kRowGroupSampleEntries, the slots they consumed, the largest count.  By workgroups of their own, which start first:
+//     chains of loads that a launch behind this one waited 20 to 26 us for.  (Nothing here is followed out of the slabs, whatever
+//     the meta words say; where a check fails the samples are not read.)
 // Bound by the stream of the column slabs.  Workgroup -> bucket by the first workgroups of the
 // buckets, so that all of them share one launch however many there are: three launches per bucket
 // (checks, counts, marks) were 60 us of GPU time for the 11 buckets of a 170K-row graph, whose slabs
-// take 3 us to read, and each read the row ids or the meta words again.
-constexpr int kScanSlotsPerBlock = 16384;
-constexpr int kScanMaxBlocks = 1024;       // per bucket: more only queue up at its counters
+// take 3 us to read, and each read the row ids or the meta words again.  Together the workgroups fill the GPU once: 1024 to a
+// bucket left a second, nearly empty round of them.  2.45M-row graph, widths 1 .. 32, behind the builder: 147 + 26 us with the samples, now 131
+// (its slabs at 3.5 TB/s; 107 us where nothing was written just before).
+constexpr int kScanSlotsPerBlock = 16384;  // at least
+constexpr int kScanBlocksPerCu = 7;
+constexpr int kScanRows = 4;               // ELL rows of a thread requested together
 constexpr int kScanUnroll = 4;             // 16-byte loads of columns in flight per thread
 constexpr int kScanCounters = 7, kScanFound = 5, kScanSpan = 6;
 constexpr int kSpanUnits = 4096, kSpanSamples = 1024;      // (twice the samples at most: sums below 2^24)
-constexpr int kCounterLine = 32;           // words between the counters of a bucket: each has a 128-byte line of its
+// Atomics on one line are taken one after the other, 17 to 40 ns each, and the workgroups of a bucket end together: up to 16
+// lines share them.
+constexpr int kScanLinesMost = 16, kScanBlocksPerLine = 64;
+constexpr int kCounterLine = 32;           // words between the cursors of a bucket: each has a 128-byte line of its
                                            // own, as atomics on one line are taken one after the other (17 ns each)
 __global__ void __launch_bounds__(256)
 plan_scan_kernel(const PlanBucket* __restrict__ buckets, const int32_t* __restrict__ first_block, int n_buckets,
                  long long num_rows, long long num_cols, int chunk_slots, long long dense_min_slots,
-                 int* __restrict__ counters, int* __restrict__ flags, uint8_t* __restrict__ covered) {
+                 int* __restrict__ counters, int* __restrict__ flags, uint8_t* __restrict__ covered,
+                 unsigned long long* __restrict__ samples) {
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     int k = -1;                                       // last bucket whose first workgroup is not behind this one
     for (int i = 0; i < n_buckets; i += 64)
@@ -1096,13 +1109,22 @@ plan_scan_kernel(const PlanBucket* __restrict__ buckets, const int32_t* __restri
     k = __builtin_amdgcn_readfirstlane(k);
     const PlanBucket bk = buckets[k];
     const long long stride = (long long)bk.n_blocks * 256;
-    const long long t0 = ((long long)blockIdx.x - first_block[k]) * 256 + threadIdx.x;
+    const int place = (int)blockIdx.x - first_block[k];
+    const long long t0 = ((long long)place - bk.n_first) * 256 + threadIdx.x;
     const int32_t *rows = bk.rows, *meta = bk.meta;
     const int log_w = bk.log_w;
     const long long n_rows = bk.n_rows;
-    if (t0 >= stride) {                                       // the bucket's last workgroup
+    if (place > 0 && place < bk.n_first) {                    // samples
+        const long long g = ((long long)(place - 1) * 256 + threadIdx.x) * bk.sample_stride;
+        int m = 0, plain = 0;
+        if (g * kGroupRows < n_rows)
+            m = merge_group<false>(bk.cols, nullptr, meta, g, n_rows, log_w, [](int, int, const float*, uint32_t) {}, kRowGroupSampleEntries, &plain);
+        add_rowgroup_counters(m, plain, samples + 3 * k);
+        return;
+    }
+    if (place == 0) {                                         // span
         int span = 0;
-        for (long long e = (t0 - stride) * bk.span_stride; e < n_rows; e += 256ll * bk.span_stride) {
+        for (long long e = (long long)threadIdx.x * bk.span_stride; e < n_rows; e += 256ll * bk.span_stride) {
             int first = 0x7FFFFFFF, last = 0;
             bool whole = true;
 #pragma unroll
@@ -1117,13 +1139,14 @@ plan_scan_kernel(const PlanBucket* __restrict__ buckets, const int32_t* __restri
             span += (int)min((long long)kSpanUnits, columns * kSpanUnits / bk.all_cols);
         }
         for (int d = 32; d > 0; d >>= 1) span += __shfl_xor(span, d);
-        if (lane == 0 && span > 0) atomicAdd(counters + ((size_t)kScanCounters * k + kScanSpan) * kCounterLine, span);
+        if (lane == 0 && span > 0) atomicAdd(counters + (size_t)bk.first_line * kCounterLine + kScanSpan, span);
         return;
     }
     bool bad_col = false, bad_row = false, bad_meta = false;
     const long long n_slots = n_rows << log_w;
     const unsigned limit = (unsigned)num_cols;               // < 2^31
-    for (long long i = t0 * 4; i < n_slots; i += stride * 4 * kScanUnroll) {
+    const long long round = stride * 4 * kScanUnroll;       // from the end: what the builder wrote last may still be in the memory-side cache (143 -> 131 us)
+    for (long long i = t0 * 4 + (n_slots - 1) / round * round; i >= 0; i -= round) {
         int4 c[kScanUnroll];
 #pragma unroll
         for (int u = 0; u < kScanUnroll; ++u) {
@@ -1139,12 +1162,24 @@ plan_scan_kernel(const PlanBucket* __restrict__ buckets, const int32_t* __restri
     }
     constexpr int kSums = kScanFound;
     int sum[kSums] = {}, found = 0;
-    for (long long e = t0; e < n_rows; e += stride) {
-        const int row = rows[e];
+    for (long long e0 = t0; e0 < n_rows; e0 += stride * kScanRows) {
+        int row_of[kScanRows], meta_of[kScanRows], next_of[kScanRows];
+#pragma unroll
+        for (int u = 0; u < kScanRows; ++u) {                 // requested together
+            const long long e = min(e0 + u * stride, n_rows - 1);
+            row_of[u] = rows[e];
+            meta_of[u] = meta[e];
+            next_of[u] = meta[min(e + 1, n_rows - 1)];
+        }
+#pragma unroll
+    for (int u = 0; u < kScanRows; ++u) {
+        const long long e = e0 + u * stride;
+        if (e >= n_rows) break;
+        const int row = row_of[u];
         const bool row_ok = (unsigned)row < (unsigned long long)num_rows;
         bad_row |= !row_ok;
         if (bk.part == 0 && row_ok) covered[row] = 1;
-        const int m = meta[e];
+        const int m = meta_of[u];
         const int len = m & (int)kMetaLenMask;
         bad_meta |= len < 1 || len > (1 << log_w);
         const long long field = (long long)(((uint32_t)m & 0x7FFFFFFFu) >> kMetaLenBits);
@@ -1166,7 +1201,7 @@ plan_scan_kernel(const PlanBucket* __restrict__ buckets, const int32_t* __restri
         }
         if (e == 0) bad_meta |= m < 0;
         if (e + 1 < n_rows) {
-            const int nm = meta[e + 1];
+            const int nm = next_of[u];
             const long long nf = (long long)(((uint32_t)nm & 0x7FFFFFFFu) >> kMetaLenBits);
             bad_meta |= want == 0 ? nm < 0 : (nm >= 0 || nf != want);
         } else {
@@ -1180,6 +1215,7 @@ plan_scan_kernel(const PlanBucket* __restrict__ buckets, const int32_t* __restri
         const long long slots = m >= 0 ? field << log_w : 0;     // of the row that starts here
         sum[3] += slots > 64 && slots <= 128;
         sum[4] += slots > 128 && slots <= kCoopSlots;
+    }
     }
     if (__ballot(bad_col) != 0 && lane == 0) flags[0] = 1;
     if (__ballot(bad_row) != 0 && lane == 0) flags[1] = 1;
@@ -1196,7 +1232,7 @@ plan_scan_kernel(const PlanBucket* __restrict__ buckets, const int32_t* __restri
     }
     __syncthreads();
     const int i = threadIdx.x;
-    int* mine = counters + ((size_t)kScanCounters * k + min(i, kSums)) * kCounterLine;
+    int* mine = counters + (size_t)(bk.first_line + place % bk.n_lines) * kCounterLine + min(i, kSums);
     if (i < kSums) {
         const int all = s_sum[0][i] + s_sum[1][i] + s_sum[2][i] + s_sum[3][i];
         if (all) atomicAdd(mine, all);
@@ -1207,102 +1243,95 @@ plan_scan_kernel(const PlanBucket* __restrict__ buckets, const int32_t* __restri
     }
 }
 
-// Every sample_stride-th group of four rows of the candidate buckets (blockIdx.y: all buckets of the
-// plan): counters[3 k ..] = merged entries among the first kRowGroupSampleEntries of a group, the
-// slots they consumed, the largest count.  Enqueued behind plan_scan_kernel, before its verdict has
-// been read: where a check failed nothing is followed through the slabs.
-__global__ void __launch_bounds__(256)
-rowgroup_sample_kernel(const PlanBucket* __restrict__ buckets, const int* __restrict__ flags,
-                       unsigned long long* __restrict__ counters) {
-    if (flags[0] | flags[1] | flags[2] | flags[3]) return;
-    const PlanBucket& bk = buckets[blockIdx.y];
-    if (bk.sample_stride == 0) return;
-    const long long g = ((long long)blockIdx.x * blockDim.x + threadIdx.x) * bk.sample_stride;
-    int m = 0, plain = 0;
-    if (g * kGroupRows < bk.n_rows)
-        m = merge_group<false>(bk.cols, nullptr, bk.meta, g, bk.n_rows, bk.log_w,
-                               [](int, int, const float*, uint32_t) {}, kRowGroupSampleEntries, &plain);
-    add_rowgroup_counters(m, plain, counters + 3 * blockIdx.y);
-}
-
-// Fills the chunk table of a bucket (rows of more than coop_slots slots, cut into chunks) and its
-// part of the heavy-row table.  counters (kCounterLine words apart): chunks, rows with several chunks
+// Fills the chunk tables of up to kChunkBuckets buckets (rows of more than coop_slots slots, cut into chunks) and their
+// parts of the heavy-row table.  cursors (kCounterLine words apart): chunks, rows with several chunks
 // and their partial rows handed out so far.  Table order depends on scheduling, results do not: every row's partials are
 // private and are summed in chunk order.
-// A workgroup owns a contiguous range of ELL rows and takes its ranges of the tables with one atomic
-// per counter: a sweep over its rows counts, a second one fills.  With one atomic per wavefront and
-// counter, counting and filling the widest bucket of a folded 2.45M-row graph (850K ELL rows)
-// took 1.35 ms, all of it updates of one cache line; now the filling pass takes 0.04.
-constexpr int kPlanChunksGrid = 512;
-__global__ void __launch_bounds__(256)
-plan_chunks_kernel(const int32_t* __restrict__ rows, const int32_t* __restrict__ meta,
-                   const int32_t* __restrict__ cols, long long n_rows, int log_w, int* __restrict__ counters,
-                   Chunk* __restrict__ chunks, HeavyRow* __restrict__ heavy,
-                   int partial_base, int heavy_base, int n_heavy, int slices, int coop_slots, int chunk_slots, long long dense_min_slots) {
-    __shared__ int s_sum[4][3];
+// A workgroup takes kChunkRows ELL rows, all their loads in flight together, and its ranges of the tables with one atomic
+// per counter.  With one atomic per wavefront and counter, counting and filling the widest bucket of a folded 2.45M-row graph (850K
+// ELL rows) took 1.35 ms, all of it updates of one cache line; a sweep that counts and one that fills, 448 rows to a wavefront one after the
+// other, 43 us; now 26.  (One workgroup to 1024 rows 40: the atomics.)  One launch for the buckets of a plan: each waited for the one before.
+constexpr int kChunkBuckets = 12, kChunkThreads = 1024, kChunkRowsOfThread = 4, kChunkRows = kChunkThreads * kChunkRowsOfThread;
+struct ChunkBucket {
+    const int32_t *rows, *meta, *cols;
+    long long n_rows;
+    Chunk* chunks;
+    int* cursors;
+    int log_w, partial_base, heavy_base, first_block;
+};
+struct ChunkBuckets {
+    ChunkBucket of[kChunkBuckets];
+    int n;
+};
+__global__ void __launch_bounds__(kChunkThreads)
+plan_chunks_kernel(ChunkBuckets buckets, HeavyRow* __restrict__ heavy, int n_heavy, int slices, int coop_slots, int chunk_slots,
+                   long long dense_min_slots) {
+    __shared__ int s_wave[3][kChunkThreads / 64];
     __shared__ int s_base[3];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const long long per_wave = ((n_rows + (long long)gridDim.x * 4 - 1) / ((long long)gridDim.x * 4) + 63) / 64 * 64;
-    const long long lo = ((long long)blockIdx.x * 4 + wave) * per_wave;
-    const long long hi = min(lo + per_wave, n_rows);
-    int sum[3] = {0, 0, 0};
-    for (long long e = lo + lane; e < hi; e += 64) {
-        const ChunkedRow x = chunked_row(meta, e, n_rows, log_w, coop_slots, chunk_slots, dense_min_slots);
-        sum[0] += x.n_chunks;
-        sum[1] += x.n_chunks > 1;
-        sum[2] += x.n_chunks > 1 ? x.n_chunks : 0;
+    int k = 0;
+    while (k + 1 < buckets.n && buckets.of[k + 1].first_block <= (int)blockIdx.x) ++k;
+    const ChunkBucket& b = buckets.of[k];
+    const int log_w = b.log_w;
+    const long long e0 = ((long long)blockIdx.x - b.first_block) * kChunkRows + threadIdx.x;
+    ChunkedRow x[kChunkRowsOfThread];
+    int mine[3] = {0, 0, 0};                 // chunks, rows with several, their partial rows
+#pragma unroll
+    for (int u = 0; u < kChunkRowsOfThread; ++u) {
+        const long long e = e0 + u * kChunkThreads;
+        x[u] = ChunkedRow{0, 0, chunk_slots, 0};
+        if (e < b.n_rows) x[u] = chunked_row(b.meta, e, b.n_rows, log_w, coop_slots, chunk_slots, dense_min_slots);
+        mine[0] += x[u].n_chunks;
+        mine[1] += x[u].n_chunks > 1;
+        mine[2] += x[u].n_chunks > 1 ? x[u].n_chunks : 0;
     }
-    for (int d = 32; d > 0; d >>= 1) {
-        for (int i = 0; i < 3; ++i) sum[i] += __shfl_xor(sum[i], d);
+    if (__syncthreads_or(mine[0]) == 0) return;
+    int at[3];
+#pragma unroll
+    for (int i = 0; i < 3; ++i) {
+        int incl = mine[i];
+        for (int d = 1; d < 64; d <<= 1) {
+            const int y = __shfl_up(incl, d);
+            if (lane >= d) incl += y;
+        }
+        if (lane == 63) s_wave[i][wave] = incl;
+        at[i] = incl - mine[i];
     }
-    if (lane == 0)
-        for (int i = 0; i < 3; ++i) s_sum[wave][i] = sum[i];
     __syncthreads();
     if (threadIdx.x < 3) {
-        const int all = s_sum[0][threadIdx.x] + s_sum[1][threadIdx.x] + s_sum[2][threadIdx.x] + s_sum[3][threadIdx.x];
-        s_base[threadIdx.x] = all ? atomicAdd(&counters[threadIdx.x * kCounterLine], all) : 0;
+        int all = 0;
+        for (int w = 0; w < kChunkThreads / 64; ++w) all += s_wave[threadIdx.x][w];
+        s_base[threadIdx.x] = all ? atomicAdd(&b.cursors[threadIdx.x * kCounterLine], all) : 0;
     }
     __syncthreads();
-    int at[3];
+#pragma unroll
     for (int i = 0; i < 3; ++i) {
-        at[i] = s_base[i];
-        for (int w = 0; w < wave; ++w) at[i] += s_sum[w][i];
+        at[i] += s_base[i];
+        for (int w = 0; w < wave; ++w) at[i] += s_wave[i][w];
     }
-    for (long long e0 = lo; e0 < hi && sum[0] > 0; e0 += 64) {
-        const long long e = e0 + lane;
-        ChunkedRow x{0, 0, chunk_slots, 0};
-        if (e < hi) x = chunked_row(meta, e, n_rows, log_w, coop_slots, chunk_slots, dense_min_slots);
-        const bool several = x.n_chunks > 1;
-        const unsigned long long votes = __ballot(several);
-        if (__ballot(x.n_chunks > 0) == 0) continue;
-        const int part = several ? x.n_chunks : 0;
-        int incl_c = x.n_chunks, incl_p = part;
-        for (int d = 1; d < 64; d <<= 1) {
-            const int yc = __shfl_up(incl_c, d), yp = __shfl_up(incl_p, d);
-            if (lane >= d) { incl_c += yc; incl_p += yp; }
-        }
-        const int c0 = at[0] + incl_c - x.n_chunks;
-        const int h = at[1] + __popcll(votes & ((1ull << lane) - 1ull));
-        const int p0 = at[2] + incl_p - part;
-        at[0] += __shfl(incl_c, 63);
-        at[1] += __popcll(votes);
-        at[2] += __shfl(incl_p, 63);
-        if (x.n_chunks == 0) continue;
-        const int row = rows[e];
-        for (int i = 0; i < x.n_chunks; ++i) {
-            const long long first = (long long)i * x.chunk_slots;
+#pragma unroll
+    for (int u = 0; u < kChunkRowsOfThread; ++u) {
+        if (x[u].n_chunks == 0) continue;
+        const long long e = e0 + u * kChunkThreads;
+        const bool several = x[u].n_chunks > 1;
+        const int row = b.rows[e], partial = b.partial_base + at[2], h = b.heavy_base + at[1];
+        for (int i = 0; i < x[u].n_chunks; ++i) {
+            const long long first = (long long)i * x[u].chunk_slots;
             Chunk ck;
             ck.slot_begin = (e << log_w) + first;
-            ck.n_slots = (int)min((long long)x.chunk_slots, x.total - first) | (x.found & 2 ? kChunkDenseBit : 0);
-            ck.partial = several ? partial_base + p0 + i : -1;
+            ck.n_slots = (int)min((long long)x[u].chunk_slots, x[u].total - first) | (x[u].found & 2 ? kChunkDenseBit : 0);
+            ck.partial = several ? partial + i : -1;
             ck.row = row;
-            ck.first_col = cols[ck.slot_begin];
-            ck.heavy = heavy_base + h;
+            ck.first_col = b.cols[ck.slot_begin];
+            ck.heavy = h;
             ck.pad_ = 0;
-            chunks[c0 + i] = ck;
+            b.chunks[at[0] + i] = ck;
         }
         for (int i = 0; i < slices && several; ++i)          // every feature slice counts its chunks
-            heavy[(size_t)i * n_heavy + heavy_base + h] = HeavyRow{row, partial_base + p0, x.n_chunks, 0};
+            heavy[(size_t)i * n_heavy + h] = HeavyRow{row, partial, x[u].n_chunks, 0};
+        at[0] += x[u].n_chunks;
+        at[1] += several;
+        at[2] += several ? x[u].n_chunks : 0;
     }
 }
 
@@ -1580,7 +1609,17 @@ int lf_spmm_create(lf_spmm_plan** out_plan, const lf_bucket_desc* h_buckets, int
     // Scratch: the words that are read back (chunk counters and fill cursors of every bucket, sampling
     // counters, flags), then the coverage bytes - cleared by one launch - then the bucket table.
     const size_t nb_s = (size_t)num_buckets;
-    const size_t o_counters = 0, o_cursors = o_counters + nb_s * kScanCounters * kCounterLine * 4, o_flags = o_cursors + nb_s * 3 * kCounterLine * 4;
+    long long scan_units = 0;                              // of kScanSlotsPerBlock slots, or 1024 rows
+    auto units_of = [](const lf_bucket_desc& b) {
+        return std::max<long long>(lf::ceil_div(b.num_ell_rows, (int64_t)1024), lf::ceil_div(b.num_ell_rows * b.width, (int64_t)kScanSlotsPerBlock));
+    };
+    for (int k = 0; k < num_buckets; ++k) scan_units += units_of(h_buckets[k]);
+    const long long units_per_block = std::max<long long>(1, lf::ceil_div(scan_units, (int64_t)kScanBlocksPerCu * plan->num_cus));
+    auto scan_blocks_of = [&](int k) { return (int)lf::ceil_div(units_of(h_buckets[k]), units_per_block); };
+    auto scan_lines_of = [&](int k) { return std::min(kScanLinesMost, std::max(1, scan_blocks_of(k) / kScanBlocksPerLine)); };
+    int scan_lines = 0;
+    for (int k = 0; k < num_buckets; ++k) scan_lines += scan_lines_of(k);
+    const size_t o_counters = 0, o_cursors = o_counters + (size_t)scan_lines * kCounterLine * 4, o_flags = o_cursors + nb_s * 3 * kCounterLine * 4;
     const size_t o_zero = o_flags + 16, o_sample = o_zero + 16, back_bytes = o_sample + nb_s * 24;
     const size_t o_covered = (back_bytes + 255) / 256 * 256;
     const size_t o_table = (o_covered + (size_t)num_rows + 255) / 256 * 256;
@@ -1614,7 +1653,7 @@ int lf_spmm_create(lf_spmm_plan** out_plan, const lf_bucket_desc* h_buckets, int
     const PlanBucket* d_table = (const PlanBucket*)(d_scratch + o_table);
     const int32_t* d_first = (const int32_t*)(d_scratch + o_table + nb_s * sizeof(PlanBucket));
     int scan_blocks = 0;
-    long long most_samples = 0;
+    scan_lines = 0;
     for (int k = 0; k < num_buckets; ++k) {
         const lf_bucket_desc& b = h_buckets[k];
         const int log_w = lf::ilog2(b.width);
@@ -1640,34 +1679,32 @@ int lf_spmm_create(lf_spmm_plan** out_plan, const lf_bucket_desc* h_buckets, int
         t.n_rows = b.num_ell_rows;
         t.log_w = log_w;
         t.part = b.part;
-        const long long units = std::max<long long>(lf::ceil_div(b.num_ell_rows, 1024),
-                                                    lf::ceil_div((long long)b.num_ell_rows << log_w, kScanSlotsPerBlock));
-        t.n_blocks = (int)std::min<long long>(units, kScanMaxBlocks);
-        h_first[k] = scan_blocks;
-        scan_blocks += t.n_blocks + (t.n_blocks > 0 ? 1 : 0);
+        t.n_blocks = scan_blocks_of(k);
+        t.first_line = scan_lines;
+        t.n_lines = scan_lines_of(k);
+        scan_lines += t.n_lines;
+        t.n_first = t.n_blocks > 0 ? 1 : 0;
         t.span_stride = (int)std::max<long long>(kGroupRows, b.num_ell_rows / kSpanSamples);
         t.all_cols = (int)cols_p;
         t.sample_stride = 0;
         if (ch == 1 && !(env_groups && env_groups[0] == '0') && b.num_ell_rows >= kRowGroupMinRows && b.width >= kUnroll && b.width <= 64) {
             const long long n_groups = lf::ceil_div(b.num_ell_rows, kGroupRows);
             t.sample_stride = (int)std::max<long long>(1, n_groups / kRowGroupSample);
-            most_samples = std::max<long long>(most_samples, lf::ceil_div(n_groups, t.sample_stride));
+            t.n_first += (int)lf::ceil_div(lf::ceil_div(n_groups, (long long)t.sample_stride), 256ll);
             cand.push_back(k);
         }
+        h_first[k] = scan_blocks;
+        scan_blocks += t.n_first + t.n_blocks;
     }
     if (num_buckets > 0) LF_TRY_HIP(hipMemcpyAsync(d_scratch + o_table, h_table, table_bytes, hipMemcpyHostToDevice, s));
     if (scan_blocks > 0) {
         plan_scan_kernel<<<scan_blocks, 256, 0, s>>>(d_table, d_first, num_buckets, num_rows, num_cols, chunk_slots,
-                                                     dense_min_slots, d_counters, d_flags, d_cov);
+                                                     dense_min_slots, d_counters, d_flags, d_cov, d_sample);
         LF_TRY_HIP(hipGetLastError());
     }
     const int rgrid = (int)std::min<int64_t>((num_rows + 255) / 256, 1024);
     if (num_rows > 0) {
         collect_uncovered_kernel<<<rgrid, 256, 0, s>>>(d_cov, num_rows, d_zero_count, nullptr);
-        LF_TRY_HIP(hipGetLastError());
-    }
-    if (!cand.empty()) {
-        rowgroup_sample_kernel<<<dim3((unsigned)lf::ceil_div(most_samples, 256), (unsigned)num_buckets), 256, 0, s>>>(d_table, d_flags, d_sample);
         LF_TRY_HIP(hipGetLastError());
     }
     LF_TRY_HIP(read_back());
@@ -1681,7 +1718,15 @@ int lf_spmm_create(lf_spmm_plan** out_plan, const lf_bucket_desc* h_buckets, int
                                                         "or a segment that is incomplete or leaves the bucket)"));
         if (f[3]) return bail(lf::fail(LF_ERR_UNSUPPORTED, "a row is split over more than %d ELL rows", (1 << (31 - kMetaLenBits)) - 1));
     }
-    auto scanned = [&](int k, int i) { return h_counters[((size_t)kScanCounters * k + i) * kCounterLine]; };
+    std::vector<int> scan_sums(nb_s * kScanCounters, 0);
+    for (int k = 0; k < num_buckets; ++k)
+        for (int l = 0; l < h_table[k].n_lines; ++l)
+            for (int i = 0; i < kScanCounters; ++i) {
+                const int x = h_counters[(size_t)(h_table[k].first_line + l) * kCounterLine + i];
+                int& sum = scan_sums[(size_t)kScanCounters * k + i];
+                sum = i == kScanFound ? sum | x : sum + x;
+            }
+    auto scanned = [&](int k, int i) { return scan_sums[(size_t)kScanCounters * k + i]; };
     auto is_multi = [&](int k) { return (scanned(k, kScanFound) & 1) != 0; };       // rows split over several ELL rows
     auto has_dense = [&](int k) { return (scanned(k, kScanFound) & 2) != 0; };
     auto has_wide = [&](int k) { return (scanned(k, kScanFound) & 4) != 0; };
@@ -1798,15 +1843,22 @@ int lf_spmm_create(lf_spmm_plan** out_plan, const lf_bucket_desc* h_buckets, int
     }
     Chunk* d_chunks_all = nullptr;
     LF_TRY(dev_alloc(plan, &d_chunks_all, (size_t)chunk_base[num_buckets]));
+    ChunkBuckets chunk_buckets{};
+    int chunk_blocks = 0;
     for (int k = 0; k < num_buckets; ++k) {
-        if (counts[k].chunks == 0) continue;
-        const lf_bucket_desc& b = h_buckets[k];
-        d_chunks[k] = d_chunks_all + chunk_base[k];
-        const int grid = (int)std::min<long long>((b.num_ell_rows + 255) / 256, kPlanChunksGrid);
-        plan_chunks_kernel<<<grid, 256, 0, s>>>(b.d_rows, meta[k], b.d_cols, b.num_ell_rows, lf::ilog2(b.width), d_cursors + (size_t)3 * k * kCounterLine,
-                                                d_chunks[k], plan->d_heavy, partial_base[k], heavy_base[k], n_heavy_total, plan->slices, plan->coop_slots,
-                                                chunk_slots, dense_min_slots);
-        LF_TRY_HIP(hipGetLastError());
+        const bool last = k + 1 == num_buckets;
+        if (counts[k].chunks > 0) {
+            const lf_bucket_desc& b = h_buckets[k];
+            d_chunks[k] = d_chunks_all + chunk_base[k];
+            chunk_buckets.of[chunk_buckets.n++] = ChunkBucket{b.d_rows, meta[k], b.d_cols, b.num_ell_rows, d_chunks[k], d_cursors + (size_t)3 * k * kCounterLine,
+                                                              lf::ilog2(b.width), partial_base[k], heavy_base[k], chunk_blocks};
+            chunk_blocks += (int)lf::ceil_div(b.num_ell_rows, (int64_t)kChunkRows);
+        }
+        if (chunk_buckets.n == kChunkBuckets || (last && chunk_buckets.n > 0)) {
+            plan_chunks_kernel<<<chunk_blocks, kChunkThreads, 0, s>>>(chunk_buckets, plan->d_heavy, n_heavy_total, plan->slices, plan->coop_slots, chunk_slots, dense_min_slots);
+            LF_TRY_HIP(hipGetLastError());
+            chunk_buckets.n = chunk_blocks = 0;
+        }
     }
     for (int k = 0; k < num_buckets; ++k) {
         if (!has_dense(k) || counts[k].chunks == 0) continue;

@@ -417,3 +417,28 @@ def test_parts_of_b_that_the_l2_holds(fa, torch, feat, b_dtype, parts, n_rows):
     Bh = B.float().cpu().numpy()
     assert (np.abs(got - O.spmm_csr_f64(indptr, indices, data, (n_rows, nc), Bh))
             <= 1e-5 * O.spmm_abs_bound(indptr, indices, data, (n_rows, nc), Bh)).all()
+
+
+@pytest.mark.parametrize("parts,b_dtype", [(16, "f32"), (3, "bf16")])
+def test_chunk_tables_of_many_buckets(fa, torch, parts, b_dtype):
+    """Plans whose chunked rows lie in more buckets than one launch of the table's kernel takes, and in
+    buckets of more ELL rows than one of its workgroups: widths of 8 split every row into many."""
+    rng = np.random.default_rng(parts)
+    nr, nc = 3000, 60_000
+    lens = rng.integers(0, 40, size=nr)
+    lens[::97] = rng.integers(2200 * parts, 2400 * parts, size=len(lens[::97]))
+    indptr = np.concatenate([[0], np.cumsum(lens)]).astype(np.int32)
+    indices = np.concatenate([np.sort(rng.choice(nc, size=n, replace=False)) for n in lens]).astype(np.int32)
+    vals = rng.uniform(-1, 1, size=len(indices)).astype(np.float32)
+    g = MTX.from_csr(indptr, indices, (nr, nc), data=vals)
+    B = torch.from_numpy(rng.uniform(-1, 1, size=(nc, 64)).astype(np.float32)).cuda()
+    B = B.to(torch.bfloat16) if b_dtype == "bf16" else B
+    Bh = B.float().cpu().numpy()
+    ref = O.spmm_csr_f64(indptr, indices, vals, (nr, nc), Bh)
+    bound = 1e-5 * O.spmm_abs_bound(indptr, indices, vals, (nr, nc), Bh)
+    for widths in ([[1, 8, 1024]] * parts, [[8]] * parts, [[4, 512, 1024], [8]] + [[2, 1024]] * (parts - 2)):
+        plan = fa.HybSpMM(fa.build_hyb_format_device(g, widths), 64, b_dtype)
+        out = plan.run(B)
+        assert plan.info["heavy_rows"] > 0 or widths[-1] == [2, 1024], widths      # (there chunks of 8192 slots)
+        assert (np.abs(out.cpu().numpy() - ref) <= bound).all()
+        plan.close()
