@@ -1,6 +1,7 @@
 // Error state and status strings of the C ABI, and the pool of page-locked read-back buffers.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cstdlib>
 #include <mutex>
 #include <vector>
@@ -69,6 +70,34 @@ PinnedLoan::~PinnedLoan() {
         }
     }
     (void)hipHostFree(p_);
+}
+
+namespace {
+__global__ void __launch_bounds__(256)
+move_words_kernel(const uint32_t* up_from, uint32_t* up_to, long long up, uint32_t* clear, long long n_clear, const uint32_t* down_from,
+                  uint32_t* down_to, long long down) {
+    const long long t = (long long)blockIdx.x * 256 + threadIdx.x, stride = (long long)gridDim.x * 256;
+    for (long long i = t; i < up; i += stride) up_to[i] = up_from[i];
+    for (long long i = t; i < n_clear; i += stride) clear[i] = 0;
+    for (long long i = t; i < down; i += stride) down_to[i] = down_from[i];
+}
+}  // namespace
+
+hipError_t move_words(Words up, bool up_pinned, void* clear, size_t clear_bytes, Words down, bool down_pinned, hipStream_t s) {
+    hipError_t e = hipSuccess;
+    if (up.bytes && !up_pinned) {
+        e = hipMemcpyAsync(up.to, up.from, up.bytes, hipMemcpyHostToDevice, s);
+        up.bytes = 0;
+    }
+    const size_t down_bytes = down_pinned ? down.bytes : 0, most = std::max(std::max(up.bytes, down_bytes), clear_bytes) / 4;
+    if (e == hipSuccess && most > 0) {
+        move_words_kernel<<<(unsigned)std::min<size_t>((most + 255) / 256, 4096), 256, 0, s>>>(
+            (const uint32_t*)up.from, (uint32_t*)up.to, (long long)(up.bytes / 4), (uint32_t*)clear, (long long)(clear_bytes / 4),
+            (const uint32_t*)down.from, (uint32_t*)down.to, (long long)(down_bytes / 4));
+        e = hipGetLastError();
+    }
+    if (e == hipSuccess && down.bytes && !down_pinned) e = hipMemcpyAsync(down.to, down.from, down.bytes, hipMemcpyDeviceToHost, s);
+    return e;
 }
 
 }  // namespace lf

@@ -158,13 +158,13 @@ row_features_kernel(const int32_t* __restrict__ indptr, int64_t rows, unsigned l
 constexpr int kOverlapEntries = 64;
 constexpr int kOverlapThreads = 1024;      // few, large workgroups: each ends with two atomics on one line
 constexpr int kOverlapGrid = 128;
-__global__ void __launch_bounds__(kOverlapThreads)
-row_overlap_kernel(const int32_t* __restrict__ indptr, const int32_t* __restrict__ indices, int64_t rows,
-                   int64_t stride, unsigned long long* __restrict__ out) {
+__device__ __forceinline__ void
+row_overlap(const int32_t* __restrict__ indptr, const int32_t* __restrict__ indices, int64_t rows,
+            int64_t stride, unsigned long long* __restrict__ out, int group, int groups) {
     const int lane = threadIdx.x & 63;
     uint32_t both = 0, seen = 0;
-    const int64_t waves = (int64_t)gridDim.x * (kOverlapThreads / 64);
-    for (int64_t i = (int64_t)blockIdx.x * (kOverlapThreads / 64) + (threadIdx.x >> 6);; i += waves) {
+    const int64_t waves = (int64_t)groups * (kOverlapThreads / 64);
+    for (int64_t i = (int64_t)group * (kOverlapThreads / 64) + (threadIdx.x >> 6);; i += waves) {
         const int64_t r = 1 + i * stride;
         if (r >= rows) break;
         const int a = indptr[r - 1], b = indptr[r];
@@ -195,10 +195,20 @@ row_overlap_kernel(const int32_t* __restrict__ indptr, const int32_t* __restrict
     }
 }
 
+__global__ void __launch_bounds__(kOverlapThreads)
+row_overlap_kernel(const int32_t* __restrict__ indptr, const int32_t* __restrict__ indices, int64_t rows,
+                   int64_t stride, unsigned long long* __restrict__ out) {
+    row_overlap(indptr, indices, rows, stride, out, blockIdx.x, gridDim.x);
+}
+
+inline int overlap_groups(int64_t rows, int64_t stride) {
+    const int64_t samples = (rows - 1 + stride - 1) / stride, per = kOverlapThreads / 64;
+    return (int)std::min<int64_t>((samples + per - 1) / per, kOverlapGrid);
+}
+
 inline hipError_t launch_row_overlap(const int32_t* indptr, const int32_t* indices, int64_t rows, int64_t stride,
                                      unsigned long long* out, hipStream_t s) {
-    const int64_t samples = (rows - 1 + stride - 1) / stride, per = kOverlapThreads / 64;
-    row_overlap_kernel<<<(int)std::min<int64_t>((samples + per - 1) / per, kOverlapGrid), kOverlapThreads, 0, s>>>(indptr, indices, rows, stride, out);
+    row_overlap_kernel<<<overlap_groups(rows, stride), kOverlapThreads, 0, s>>>(indptr, indices, rows, stride, out);
     return hipGetLastError();
 }
 
@@ -307,7 +317,7 @@ class_count_kernel(SegView v, const int32_t* __restrict__ seg_deg, int kmax, uns
 // 235 us, now 86 with the Python around it).
 constexpr int kShapeCands = 16;
 constexpr int kShapeParts = 128;           // partitions of all candidates together
-constexpr int kShapeGrid = 512;
+constexpr int kShapeGrid = 1024;
 struct ShapeCands {
     int n, total;
     int parts[kShapeCands];
@@ -320,11 +330,12 @@ constexpr int shape_words(int total) { return total * (LF_MAX_CLASSES + 1); }
 __global__ void __launch_bounds__(kBlock)
 shape_stats_kernel(const int32_t* __restrict__ indptr, const int32_t* __restrict__ indices, int64_t rows, int64_t cols,
                    ShapeCands cands, int kmax, unsigned long long* __restrict__ partial,
-                   unsigned long long* __restrict__ overlap) {
+                   unsigned long long* __restrict__ out, int n_out) {
     __shared__ unsigned long long s_cnt[shape_words(kShapeParts)];
     const int n_words = shape_words(cands.total);
     for (int i = threadIdx.x; i < n_words; i += kBlock) s_cnt[i] = 0;
-    if (blockIdx.x == 0 && threadIdx.x < 2) overlap[threadIdx.x] = 0;      // for row_overlap_kernel behind this one
+    if (blockIdx.x == 0)                                       // for the launch behind this one
+        for (int i = threadIdx.x; i < n_out; i += kBlock) out[i] = 0;
     __syncthreads();
     for (int64_t r = (int64_t)blockIdx.x * kBlock + threadIdx.x; r < rows; r += (int64_t)gridDim.x * kBlock) {
         const int lo = indptr[r], hi = indptr[r + 1];
@@ -350,11 +361,19 @@ shape_stats_kernel(const int32_t* __restrict__ indptr, const int32_t* __restrict
     for (int i = threadIdx.x; i < n_words; i += kBlock) partial[(size_t)blockIdx.x * n_words + i] = s_cnt[i];
 }
 
-// out[q][k] = {cost rows, nnz, segments, 0}: 64 words to a workgroup, 16 threads add up each.
+// out[q][k] = {cost rows, nnz, segments, 0}: 64 words to a workgroup, 16 threads add up each.  The workgroups behind those sample
+// the row overlap, whose two sums follow the statistics.
+static_assert(kOverlapThreads == 1024);
 __global__ void __launch_bounds__(1024)
 shape_reduce_kernel(const unsigned long long* __restrict__ partial, int n_groups, int total, int kmax,
-                    unsigned long long* __restrict__ out) {
+                    unsigned long long* __restrict__ out, const int32_t* __restrict__ indptr, const int32_t* __restrict__ indices,
+                    int64_t rows, int64_t stride) {
     __shared__ unsigned long long s_sum[16][64];
+    const int reducers = (shape_words(total) + 63) / 64;
+    if ((int)blockIdx.x >= reducers) {
+        row_overlap(indptr, indices, rows, stride, out + (size_t)total * LF_MAX_CLASSES * LF_STATS_FIELDS, blockIdx.x - reducers, gridDim.x - reducers);
+        return;
+    }
     const int n_words = shape_words(total);
     const int w = blockIdx.x * 64 + (threadIdx.x & 63), slice = threadIdx.x >> 6;
     unsigned long long sum = 0;
@@ -876,10 +895,11 @@ __host__ __device__ inline void flat_layout_step(int64_t ell_rows, int64_t width
 
 // Exclusive scan over blocks, one workgroup per bucket; totals[k] = ELL rows of bucket k.  The
 // workgroup that ends last derives the flat layout from the totals, so that the fill needs
-// nothing more from the host.
+// nothing more from the host, and leaves flags and totals in the host's (pinned) memory, if that is given.
 __global__ void __launch_bounds__(1024)
 hyb_scan_kernel(int32_t* __restrict__ blockcnt, int nblk, long long* __restrict__ totals,
-                const int32_t* __restrict__ widths, int* __restrict__ done, BucketOffsets* __restrict__ offs) {
+                const int32_t* __restrict__ widths, int* __restrict__ done, BucketOffsets* __restrict__ offs,
+                const int* __restrict__ flags, int* h_flags, long long* h_totals) {
     __shared__ long long s_wave[16];
     __shared__ int s_last;
     int32_t* a = blockcnt + (int64_t)blockIdx.x * nblk;
@@ -916,6 +936,7 @@ hyb_scan_kernel(int32_t* __restrict__ blockcnt, int nblk, long long* __restrict_
     __syncthreads();
     if (!s_last) return;
     const int nb = gridDim.x;
+    if (h_flags && threadIdx.x == 0) *h_flags = *flags;           // (hyb_count_kernel's)
     int64_t row = 0, slot = 0;                        // carried by thread 0
     for (int base = 0; base < nb; base += 1024) {     // staged through LDS: the layout is a serial sum
         __shared__ long long s_rows[1024];
@@ -932,6 +953,7 @@ hyb_scan_kernel(int32_t* __restrict__ blockcnt, int nblk, long long* __restrict_
                 flat_layout_step(s_rows[k], s_width[k], &row, &slot);
             }
         }
+        if (h_totals && i < nb) h_totals[i] = s_rows[threadIdx.x];
         __syncthreads();
     }
 }
@@ -1428,12 +1450,11 @@ int lf_shape_stats(const int32_t* d_indptr, const int32_t* d_indices, int64_t nu
     unsigned long long* partial = (unsigned long long*)((char*)d_workspace + align_up((n_stats + 2) * 8, 256));
     const int grid = (int)std::min<int64_t>((num_rows + kBlock - 1) / kBlock, kShapeGrid);
     const int kmax = lf::ilog2(width_limit);
-    LF_HIP(fill_u32(out, (int64_t)n_stats * 2, 0u, s));
-    shape_stats_kernel<<<grid, kBlock, 0, s>>>(d_indptr, d_indices, num_rows, num_cols, cands, kmax, partial, out + n_stats);
+    shape_stats_kernel<<<grid, kBlock, 0, s>>>(d_indptr, d_indices, num_rows, num_cols, cands, kmax, partial, out, (int)n_stats + 2);
     LF_HIP(hipGetLastError());
-    shape_reduce_kernel<<<(shape_words(cands.total) + 63) / 64, 1024, 0, s>>>(partial, grid, cands.total, kmax, out);
+    shape_reduce_kernel<<<(shape_words(cands.total) + 63) / 64 + (num_rows > 1 ? overlap_groups(num_rows, sample_stride) : 0), 1024, 0, s>>>(
+        partial, grid, cands.total, kmax, out, d_indptr, d_indices, num_rows, sample_stride);
     LF_HIP(hipGetLastError());
-    if (num_rows > 1) LF_HIP(launch_row_overlap(d_indptr, d_indices, num_rows, sample_stride, out + n_stats, s));
     lf::PinnedLoan back((n_stats + 2) * 8);
     LF_REQUIRE(back.ok(), LF_ERR_HIP, "out of host memory");
     LF_HIP(hipMemcpyAsync(back.as<char>(), out, (n_stats + 2) * 8, hipMemcpyDeviceToHost, s));
@@ -1545,8 +1566,8 @@ int lf_hyb_plan(const int32_t* d_indptr, const int32_t* d_indices, const int32_t
     if (nb > 0) std::memcpy(up.as<char>(L.widths - L.wtab), h_widths_flat, (size_t)nb * 4);
     // The loans go back when this returns: every way out from here on waits for the stream first.
     struct Wait { hipStream_t s; ~Wait() { (void)hipStreamSynchronize(s); } } wait{s};
-    LF_HIP(hipMemcpyAsync(wtab, h_wtab, up_bytes, hipMemcpyHostToDevice, s));
-    LF_HIP(fill_u32(flags, (int64_t)(back_bytes / 4), 0u, s));
+    LF_HIP(lf::move_words({h_wtab, wtab, up_bytes}, up.pinned(), flags, back_bytes, {}, true, s));
+    const bool direct = back.pinned() && num_rows > 0 && nb > 0;
     if (num_rows > 0) {
         if (num_parts > 1 && d_seg_bounds) {       // bounds already known (the statistics pass made them)
             LF_HIP(hipMemcpyAsync(bnd, d_seg_bounds, (size_t)(num_parts + 1) * num_rows * 4,
@@ -1560,11 +1581,12 @@ int lf_hyb_plan(const int32_t* d_indptr, const int32_t* d_indices, const int32_t
         LF_HIP(hipGetLastError());
         if (nb > 0) {
             hyb_scan_kernel<<<nb, 1024, 0, s>>>(blockcnt, L.nblk, totals, (const int32_t*)(ws + L.widths), flags + 1,
-                                                (BucketOffsets*)(ws + L.scatter));
+                                                (BucketOffsets*)(ws + L.scatter), flags, direct ? back.as<int>() : nullptr,
+                                                direct ? back.as<long long>(L.totals - L.flags) : nullptr);
             LF_HIP(hipGetLastError());
         }
     }
-    LF_HIP(hipMemcpyAsync(back.as<char>(), flags, back_bytes, hipMemcpyDeviceToHost, s));
+    if (!direct) LF_HIP(hipMemcpyAsync(back.as<char>(), flags, back_bytes, hipMemcpyDeviceToHost, s));
     LF_HIP(hipStreamSynchronize(s));
     const int32_t h_flags = *back.as<int32_t>();
     if (h_flags & 1)

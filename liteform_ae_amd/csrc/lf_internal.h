@@ -39,11 +39,21 @@ public:
     PinnedLoan& operator=(const PinnedLoan&) = delete;
     template <typename T> T* as(size_t byte_offset = 0) const { return reinterpret_cast<T*>((char*)p_ + byte_offset); }
     bool ok() const { return p_ != nullptr; }
+    bool pinned() const { return pinned_; }            // a kernel may read and write it
 
 private:
     void* p_ = nullptr;
     bool pinned_ = false;
 };
+
+// Words from `up` to the GPU, `n_clear` cleared there, words from there to `down`, in one launch where the loans are pinned: a copy, a
+// fill and a copy are three, 5 us each of a call that waits for them.  (A few KB of either: the kernel's loads and stores cross PCIe.)
+struct Words {
+    const void* from = nullptr;
+    void* to = nullptr;
+    size_t bytes = 0;              // a multiple of 4
+};
+hipError_t move_words(Words up, bool up_pinned, void* clear, size_t clear_bytes, Words down, bool down_pinned, hipStream_t s);
 
 // A few words from the GPU, and the wait for them.
 inline hipError_t read_back(void* h_dst, const void* d_src, size_t bytes, hipStream_t s) {

@@ -1641,11 +1641,6 @@ int lf_spmm_create(lf_spmm_plan** out_plan, const lf_bucket_desc* h_buckets, int
         if (e == hipSuccess) e = hipStreamSynchronize(s);
         return e;
     };
-    {
-        const long long words = (long long)(o_table / 4);
-        fill_bytes_kernel<<<(int)std::min<long long>((words + 255) / 256, 4096), 256, 0, s>>>((uint32_t*)d_scratch, words, 0u);
-        LF_TRY_HIP(hipGetLastError());
-    }
     const char* env_groups = getenv("LF_ROW_GROUPS");
     std::vector<int> cand;                                 // buckets that may be rewritten as row groups or cells
     PlanBucket* h_table = table.as<PlanBucket>();
@@ -1653,21 +1648,15 @@ int lf_spmm_create(lf_spmm_plan** out_plan, const lf_bucket_desc* h_buckets, int
     const PlanBucket* d_table = (const PlanBucket*)(d_scratch + o_table);
     const int32_t* d_first = (const int32_t*)(d_scratch + o_table + nb_s * sizeof(PlanBucket));
     int scan_blocks = 0;
+    std::vector<std::pair<int, int32_t*>> derived;         // buckets that come without meta words
     scan_lines = 0;
     for (int k = 0; k < num_buckets; ++k) {
         const lf_bucket_desc& b = h_buckets[k];
         const int log_w = lf::ilog2(b.width);
         if (b.num_ell_rows > 0 && !b.d_meta) {
-            int32_t *m = nullptr, *blk_first = nullptr, *blk_last = nullptr;
-            const int n_blocks = (int)((b.num_ell_rows + 255) / 256);
+            int32_t* m = nullptr;
             LF_TRY(dev_alloc(plan, &m, (size_t)b.num_ell_rows));
-            LF_TRY(dev_alloc(plan, &blk_first, (size_t)n_blocks, true));
-            LF_TRY(dev_alloc(plan, &blk_last, (size_t)n_blocks, true));
-            derive_heads_kernel<<<n_blocks, 256, 0, s>>>(b.d_rows, b.num_ell_rows, blk_first, blk_last);
-            LF_TRY_HIP(hipGetLastError());
-            derive_meta_kernel<<<n_blocks, 256, 0, s>>>(b.d_rows, b.d_vals, b.num_ell_rows, log_w, blk_first,
-                                                        blk_last, n_blocks, m, d_flags);
-            LF_TRY_HIP(hipGetLastError());
+            derived.push_back({k, m});
             meta[k] = m;
         } else if (b.num_ell_rows > 0) {
             meta[k] = b.d_meta;
@@ -1696,7 +1685,19 @@ int lf_spmm_create(lf_spmm_plan** out_plan, const lf_bucket_desc* h_buckets, int
         h_first[k] = scan_blocks;
         scan_blocks += t.n_first + t.n_blocks;
     }
-    if (num_buckets > 0) LF_TRY_HIP(hipMemcpyAsync(d_scratch + o_table, h_table, table_bytes, hipMemcpyHostToDevice, s));
+    LF_TRY_HIP(lf::move_words({h_table, d_scratch + o_table, table_bytes}, table.pinned(), d_scratch, o_table, {}, true, s));
+    for (const auto& [k, m] : derived) {
+        const lf_bucket_desc& b = h_buckets[k];
+        int32_t *blk_first = nullptr, *blk_last = nullptr;
+        const int n_blocks = (int)((b.num_ell_rows + 255) / 256);
+        LF_TRY(dev_alloc(plan, &blk_first, (size_t)n_blocks, true));
+        LF_TRY(dev_alloc(plan, &blk_last, (size_t)n_blocks, true));
+        derive_heads_kernel<<<n_blocks, 256, 0, s>>>(b.d_rows, b.num_ell_rows, blk_first, blk_last);
+        LF_TRY_HIP(hipGetLastError());
+        derive_meta_kernel<<<n_blocks, 256, 0, s>>>(b.d_rows, b.d_vals, b.num_ell_rows, lf::ilog2(b.width), blk_first,
+                                                    blk_last, n_blocks, m, d_flags);
+        LF_TRY_HIP(hipGetLastError());
+    }
     if (scan_blocks > 0) {
         plan_scan_kernel<<<scan_blocks, 256, 0, s>>>(d_table, d_first, num_buckets, num_rows, num_cols, chunk_slots,
                                                      dense_min_slots, d_counters, d_flags, d_cov, d_sample);
@@ -2134,6 +2135,7 @@ int lf_spmm_create(lf_spmm_plan** out_plan, const lf_bucket_desc* h_buckets, int
     const size_t tables_bytes = o_cells + cells.size() * sizeof(LfCellBucket);
     lf::PinnedLoan h_tables(tables_bytes);
     if (!h_tables.ok()) return bail(lf::fail(LF_ERR_HIP, "out of host memory"));
+    lf::Words up;                              // sent with the read-back below
     if (tables_bytes > 0) {
         char* d_tables = nullptr;
         LF_TRY(dev_alloc(plan, &d_tables, tables_bytes));
@@ -2143,7 +2145,7 @@ int lf_spmm_create(lf_spmm_plan** out_plan, const lf_bucket_desc* h_buckets, int
         put(0, groups.data(), groups.size() * sizeof(Group));
         put(o_merged, merged.data(), merged.size() * sizeof(MergedBucket));
         put(o_cells, cells.data(), cells.size() * sizeof(LfCellBucket));
-        LF_TRY_HIP(hipMemcpyAsync(d_tables, h_tables.as<char>(), tables_bytes, hipMemcpyHostToDevice, s));
+        up = lf::Words{h_tables.as<char>(), d_tables, tables_bytes};
         plan->d_groups = (Group*)d_tables;
         plan->d_merged = (MergedBucket*)(d_tables + o_merged);
         plan->d_cells = (LfCellBucket*)(d_tables + o_cells);
@@ -2181,7 +2183,8 @@ int lf_spmm_create(lf_spmm_plan** out_plan, const lf_bucket_desc* h_buckets, int
     plan->info[6] = n_zero;
     plan->info[7] = (int64_t)(merged.size() + cells.size());
     plan->info[8] = (int64_t)cells.size();
-    LF_TRY_HIP(read_back());                 // the tables are complete: the plan may run on any stream
+    LF_TRY_HIP(lf::move_words(up, h_tables.pinned(), nullptr, 0, {d_scratch + o_cursors, back.as<char>(o_cursors), o_flags - o_cursors}, back.pinned(), s));
+    LF_TRY_HIP(hipStreamSynchronize(s));     // the tables are complete: the plan may run on any stream
     for (int k = 0; k < num_buckets; ++k) {  // the filling pass must have taken the counted ranges
         const int* c = back.as<int>(o_cursors) + (size_t)3 * k * kCounterLine;
         if (counts[k].chunks > 0 && (c[0] != counts[k].chunks || c[kCounterLine] != counts[k].heavy || c[2 * kCounterLine] != counts[k].partials))
