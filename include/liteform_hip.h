@@ -331,6 +331,10 @@ int lf_csr_check(const int32_t* d_indptr, const int32_t* d_indices, const float*
 int lf_csr_check_span(const int32_t* d_indptr, const int32_t* d_indices, const float* d_values,
                       int64_t num_rows, int64_t num_cols, int64_t nnz, void* d_scratch, int32_t* h_flags,
                       int64_t* h_span, lf_stream_t stream);
+/* The same, and *h_longest receives the entries of the longest row (d_scratch: 32 bytes). */
+int lf_csr_check_rows(const int32_t* d_indptr, const int32_t* d_indices, const float* d_values,
+                      int64_t num_rows, int64_t num_cols, int64_t nnz, void* d_scratch, int32_t* h_flags,
+                      int64_t* h_span, int64_t* h_longest, lf_stream_t stream);
 
 /* Row-parallel CSR SpMM, the counterpart of bench_naive's kernel
  * (format_algos.py:1689-1755): C = A_csr . B with float32 values (NULL = ones).
@@ -357,12 +361,14 @@ int lf_csr_spmm_trusted_span(const int32_t* d_indptr, const int32_t* d_indices, 
  * space: lf_csr_spmm_work_bytes bytes of device memory, 16-byte aligned, that no other product uses meanwhile (none: d_work
  * NULL, and the product is that of lf_csr_spmm_trusted_span).  The chunks are those of lf_csr_long_rows, which fills d_list
  * (lf_csr_long_rows_bytes bytes) once for a matrix, and h_counts[0..2] = chunks, rows, entries of the longest row; it
- * synchronises.  Without them (NULL) long rows stay whole.  The product only enqueues kernels. */
+ * synchronises.  Without them (NULL) long rows stay whole; lf_csr_spmm_work_bytes is then told the entries of the longest
+ * row (lf_csr_check_rows; 0: unknown) and answers -1 where the product would be faster with the list.  The product only
+ * enqueues kernels. */
 size_t lf_csr_long_rows_bytes(int64_t nnz);
 int lf_csr_long_rows(const int32_t* d_indptr, int64_t num_rows, int64_t nnz, void* d_list, size_t list_bytes,
                      int64_t* h_counts, lf_stream_t stream);
-size_t lf_csr_spmm_work_bytes(int64_t num_rows, int64_t num_cols, int64_t nnz, int64_t span, const int64_t* h_counts,
-                              int32_t feat_size, int32_t b_dtype);
+int64_t lf_csr_spmm_work_bytes(int64_t num_rows, int64_t num_cols, int64_t nnz, int64_t span, const int64_t* h_counts,
+                               int64_t longest, int32_t feat_size, int32_t b_dtype);
 int lf_csr_spmm_trusted_work(const int32_t* d_indptr, const int32_t* d_indices, const float* d_values,
                              int64_t num_rows, int64_t num_cols, int64_t nnz, int64_t span, const void* d_list,
                              const int64_t* h_counts, void* d_work, size_t work_bytes, int32_t feat_size,

@@ -79,13 +79,14 @@ SIGNATURES = {
     "lf_spmm_time_ms": (C.c_int, [vp, vp, vp, C.c_int32, C.c_int32, vp, C.c_size_t, f32p, vp]),
     "lf_csr_check": (C.c_int, [vp, vp, vp, C.c_int64, C.c_int64, C.c_int64, vp, i32p, vp]),
     "lf_csr_check_span": (C.c_int, [vp, vp, vp, C.c_int64, C.c_int64, C.c_int64, vp, i32p, i64p, vp]),
+    "lf_csr_check_rows": (C.c_int, [vp, vp, vp, C.c_int64, C.c_int64, C.c_int64, vp, i32p, i64p, i64p, vp]),
     "lf_csr_spmm": (C.c_int, [vp, vp, vp, C.c_int64, C.c_int64, C.c_int64, C.c_int32, C.c_int32, vp, vp, vp, vp]),
     "lf_csr_spmm_trusted": (C.c_int, [vp, vp, vp, C.c_int64, C.c_int64, C.c_int32, C.c_int32, vp, vp, vp]),
     "lf_csr_spmm_trusted_nnz": (C.c_int, [vp, vp, vp, C.c_int64, C.c_int64, C.c_int64, C.c_int32, C.c_int32, vp, vp, vp]),
     "lf_csr_spmm_trusted_span": (C.c_int, [vp, vp, vp, C.c_int64, C.c_int64, C.c_int64, C.c_int64, C.c_int32, C.c_int32, vp, vp, vp]),
     "lf_csr_long_rows_bytes": (C.c_size_t, [C.c_int64]),
     "lf_csr_long_rows": (C.c_int, [vp, C.c_int64, C.c_int64, vp, C.c_size_t, i64p, vp]),
-    "lf_csr_spmm_work_bytes": (C.c_size_t, [C.c_int64, C.c_int64, C.c_int64, C.c_int64, i64p, C.c_int32, C.c_int32]),
+    "lf_csr_spmm_work_bytes": (C.c_int64, [C.c_int64, C.c_int64, C.c_int64, C.c_int64, i64p, C.c_int64, C.c_int32, C.c_int32]),
     "lf_csr_spmm_trusted_work": (C.c_int, [vp, vp, vp, C.c_int64, C.c_int64, C.c_int64, C.c_int64, vp, i64p, vp, C.c_size_t, C.c_int32, C.c_int32, vp,
                                            vp, vp]),
     "lf_coo_to_csr_workspace_bytes": (C.c_size_t, [C.c_int64, C.c_int64, C.c_int64]),

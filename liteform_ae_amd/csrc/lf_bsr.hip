@@ -285,7 +285,7 @@ int lf_bsr_spmm(const int32_t* d_indptr, const int32_t* d_indices, const void* d
     LF_REQUIRE(num_block_rows >= 0 && num_block_rows < (1ll << 26) && num_block_cols >= 1 &&
                    num_block_cols < (1ll << 26), LF_ERR_INVALID, "bad block shape");
     // no gather before the block index arrays have passed
-    if (int rc = lf::csr_check(d_indptr, d_indices, nullptr, num_block_rows, num_block_cols, nnz_blocks, d_scratch, nullptr, nullptr,
+    if (int rc = lf::csr_check(d_indptr, d_indices, nullptr, num_block_rows, num_block_cols, nnz_blocks, d_scratch, nullptr, nullptr, nullptr,
                                "lf_bsr_spmm", (hipStream_t)stream))
         return rc;
     return lf_bsr_spmm_trusted_nnz(d_indptr, d_indices, d_data, num_block_rows, num_block_cols, nnz_blocks, block_size,

@@ -383,11 +383,15 @@ int lf_csr_long_rows(const int32_t* d_indptr, int64_t num_rows, int64_t nnz, voi
 
 size_t lf_csr_long_rows_bytes(int64_t nnz) { return ListLayout(nullptr, nnz).bytes; }
 
-size_t lf_csr_spmm_work_bytes(int64_t num_rows, int64_t num_cols, int64_t nnz, int64_t span, const int64_t* h_counts, int32_t feat_size,
-                              int32_t b_dtype) {
+int64_t lf_csr_spmm_work_bytes(int64_t num_rows, int64_t num_cols, int64_t nnz, int64_t span, const int64_t* h_counts, int64_t longest,
+                               int32_t feat_size, int32_t b_dtype) {
     int lpr, ch;
     if (num_rows <= 0 || num_cols < 1 || feature_shape(feat_size, b_dtype, &lpr, &ch) != LF_OK) return 0;
-    return work_bytes_of(csr_shape(num_rows, num_cols, nnz, span, feat_size, b_dtype, h_counts, true), num_rows, feat_size);
+    const int64_t guess[3] = {1, 1, longest};
+    const bool unknown = !h_counts && longest > kCsrChunkedRow;
+    const CsrShape shape = csr_shape(num_rows, num_cols, nnz, span, feat_size, b_dtype, unknown ? guess : h_counts, true);
+    if (unknown && shape.n_chunks > 0) return -1;
+    return (int64_t)work_bytes_of(shape, num_rows, feat_size);
 }
 
 int lf_csr_spmm_trusted_work(const int32_t* d_indptr, const int32_t* d_indices, const float* d_values,
@@ -486,7 +490,7 @@ int lf_csr_spmm(const int32_t* d_indptr, const int32_t* d_indices, const float* 
     }
     // no gather before the index arrays have passed
     int64_t span = 0;
-    if (int rc = lf::csr_check(d_indptr, d_indices, nullptr, num_rows, num_cols, nnz, d_scratch, nullptr, &span, "lf_csr_spmm",
+    if (int rc = lf::csr_check(d_indptr, d_indices, nullptr, num_rows, num_cols, nnz, d_scratch, nullptr, &span, nullptr, "lf_csr_spmm",
                                (hipStream_t)stream))
         return rc;
     return lf_csr_spmm_trusted_span(d_indptr, d_indices, d_values, num_rows, num_cols, nnz, span, feat_size, b_dtype, d_B, d_C, stream);

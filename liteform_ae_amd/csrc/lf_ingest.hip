@@ -562,7 +562,7 @@ __global__ void clear_words_kernel(int* __restrict__ p, int n) {
 // duplicates) exactly when the two counts are equal.  out[3] is raised when a value differs
 // from 1 (values == nullptr: not looked at).  That is bit 0 of out[0] and out[3]; above it are sums over every
 // `sample_stride`-th row with entries in it or the three rows behind it: of the columns between the least first and the
-// largest last one, in kSpanUnits of all, and of ones.
+// largest last one, in kSpanUnits of all, and of ones.  *longest (optional): the entries of the longest row.
 // Bound by the two streams (8 bytes an entry).  81M entries with values: 2.25 ms with one atomic
 // per wavefront and counter (65K updates of one cache line), 0.29 ms with one per workgroup of a
 // grid that is resident at once, and 16-byte loads.
@@ -574,14 +574,16 @@ struct __attribute__((packed, aligned(4))) Packed4f { float x, y, z, w; };
 __global__ void __launch_bounds__(256)
 csr_check_kernel(const int32_t* __restrict__ indptr, const int32_t* __restrict__ indices,
                  const float* __restrict__ values, long long rows, long long cols, long long nnz, int sample_stride,
-                 unsigned int* __restrict__ out) {
+                 unsigned int* __restrict__ out, int* __restrict__ longest) {
     const long long stride = (long long)gridDim.x * blockDim.x;
     const long long t0 = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+    int most = 0;
     bool bad = false, not_one = false;
     unsigned int descents = 0, boundary = 0, span = 0, samples = 0;
     for (long long r = t0; r < rows; r += stride) {
         const long long lo = indptr[r], hi = indptr[r + 1];
         bad |= lo < 0 || hi < lo || hi > nnz;
+        most = max(most, (int)(hi - lo));
         if (r == 0) bad |= lo != 0;
         if (r == rows - 1) bad |= hi != nnz;
         if (hi > lo && lo > 0 && lo < nnz && indices[lo] <= indices[lo - 1]) ++boundary;
@@ -626,10 +628,12 @@ csr_check_kernel(const int32_t* __restrict__ indptr, const int32_t* __restrict__
         boundary += __shfl_xor(boundary, d);
         span += __shfl_xor(span, d);
         samples += __shfl_xor(samples, d);
+        most = max(most, __shfl_xor(most, d));
     }
     __shared__ unsigned int s_sum[4][4];
+    __shared__ int s_most[4];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    if (lane == 0) { s_sum[0][wave] = descents; s_sum[1][wave] = boundary; s_sum[2][wave] = span; s_sum[3][wave] = samples; }
+    if (lane == 0) { s_sum[0][wave] = descents; s_sum[1][wave] = boundary; s_sum[2][wave] = span; s_sum[3][wave] = samples; s_most[wave] = most; }
     const bool any_bad = __syncthreads_or(bad) != 0;
     const bool any_not_one = __syncthreads_or(not_one) != 0;
     if (threadIdx.x == 0) {
@@ -643,6 +647,10 @@ csr_check_kernel(const int32_t* __restrict__ indptr, const int32_t* __restrict__
         if (samples) atomicAdd(&out[3], samples << 1);
         if (descents) atomicAdd(&out[1], descents);
         if (boundary) atomicAdd(&out[2], boundary);
+        if (longest) {
+            most = max(max(s_most[0], s_most[1]), max(s_most[2], s_most[3]));
+            if (most > __hip_atomic_load(longest, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicMax(longest, most);
+        }
     }
 }
 
@@ -688,12 +696,13 @@ int key_bits_for(long long rows, long long cols) {
 namespace lf {
 
 int csr_check(const int32_t* d_indptr, const int32_t* d_indices, const float* d_values, int64_t num_rows,
-              int64_t num_cols, int64_t nnz, void* d_scratch, int32_t* h_flags, int64_t* h_span, const char* what, hipStream_t s) {
+              int64_t num_cols, int64_t nnz, void* d_scratch, int32_t* h_flags, int64_t* h_span, int64_t* h_longest, const char* what, hipStream_t s) {
     LF_REQUIRE(num_rows >= 0 && num_rows < (1ll << 31) && num_cols >= 1 && num_cols < (1ll << 31), LF_ERR_INVALID,
                "bad shape %lld x %lld", (long long)num_rows, (long long)num_cols);
     LF_REQUIRE(nnz >= 0 && nnz < (1ll << 31), LF_ERR_UNSUPPORTED, "nnz must be below 2^31");
     if (h_flags) *h_flags = LF_CSR_CANONICAL | (d_values ? LF_CSR_UNIT_VALUES : 0);
     if (h_span) *h_span = 0;
+    if (h_longest) *h_longest = 0;
     if (num_rows == 0) {
         LF_REQUIRE(nnz == 0, LF_ERR_INVALID, "%s: a matrix without rows holds %lld entries", what, (long long)nnz);
         return LF_OK;
@@ -701,18 +710,20 @@ int csr_check(const int32_t* d_indptr, const int32_t* d_indices, const float* d_
     LF_REQUIRE(d_indptr && (nnz == 0 || d_indices), LF_ERR_INVALID, "%s: null index array", what);
     LF_REQUIRE(d_scratch && (uintptr_t)d_scratch % 4 == 0, LF_ERR_INVALID, "%s: the check needs 16 bytes of device scratch", what);
     unsigned int* out = (unsigned int*)d_scratch;
-    LF_HIP(hipMemsetAsync(out, 0, 16, s));
+    const size_t bytes = h_longest ? 20 : 16;
+    LF_HIP(hipMemsetAsync(out, 0, bytes, s));
     const long long units = std::max<long long>(num_rows, (nnz + 3) / 4);
     const int grid = (int)std::min<long long>((units + 255) / 256, kCheckGrid);
     csr_check_kernel<<<grid, 256, 0, s>>>(d_indptr, d_indices, d_values, num_rows, num_cols, nnz,
-                                     (int)std::max<long long>(1, num_rows / kSpanSamples), out);
+                                     (int)std::max<long long>(1, num_rows / kSpanSamples), out, h_longest ? (int*)out + 4 : nullptr);
     LF_HIP(hipGetLastError());
-    unsigned int h[4] = {0, 0, 0, 0};
-    LF_HIP(lf::read_back(h, out, 16, s));
+    unsigned int h[5] = {0, 0, 0, 0, 0};
+    LF_HIP(lf::read_back(h, out, bytes, s));
     LF_REQUIRE((h[0] & 1) == 0, LF_ERR_INVALID,
                "%s: the row pointer is not a non-decreasing sequence from 0 to nnz = %lld, or an index lies outside [0, %lld)",
                what, (long long)nnz, (long long)num_cols);
     if (h_flags) *h_flags = (h[1] == h[2] ? LF_CSR_CANONICAL : 0) | (d_values && (h[3] & 1) == 0 ? LF_CSR_UNIT_VALUES : 0);
+    if (h_longest) *h_longest = h[4];
     if (h_span && h[1] == h[2] && h[3] >> 1 > 0)
         *h_span = (int64_t)((double)(h[0] >> 1) / (h[3] >> 1) * (double)num_cols / kSpanUnits);
     return LF_OK;
@@ -724,13 +735,19 @@ extern "C" {
 
 int lf_csr_check(const int32_t* d_indptr, const int32_t* d_indices, const float* d_values, int64_t num_rows,
                  int64_t num_cols, int64_t nnz, void* d_scratch, int32_t* h_flags, lf_stream_t stream) {
-    return lf::csr_check(d_indptr, d_indices, d_values, num_rows, num_cols, nnz, d_scratch, h_flags, nullptr, "CSR arrays",
+    return lf::csr_check(d_indptr, d_indices, d_values, num_rows, num_cols, nnz, d_scratch, h_flags, nullptr, nullptr, "CSR arrays",
                          (hipStream_t)stream);
 }
 
 int lf_csr_check_span(const int32_t* d_indptr, const int32_t* d_indices, const float* d_values, int64_t num_rows,
                       int64_t num_cols, int64_t nnz, void* d_scratch, int32_t* h_flags, int64_t* h_span, lf_stream_t stream) {
-    return lf::csr_check(d_indptr, d_indices, d_values, num_rows, num_cols, nnz, d_scratch, h_flags, h_span, "CSR arrays",
+    return lf::csr_check(d_indptr, d_indices, d_values, num_rows, num_cols, nnz, d_scratch, h_flags, h_span, nullptr, "CSR arrays",
+                         (hipStream_t)stream);
+}
+
+int lf_csr_check_rows(const int32_t* d_indptr, const int32_t* d_indices, const float* d_values, int64_t num_rows,
+                      int64_t num_cols, int64_t nnz, void* d_scratch, int32_t* h_flags, int64_t* h_span, int64_t* h_longest, lf_stream_t stream) {
+    return lf::csr_check(d_indptr, d_indices, d_values, num_rows, num_cols, nnz, d_scratch, h_flags, h_span, h_longest, "CSR arrays",
                          (hipStream_t)stream);
 }
 

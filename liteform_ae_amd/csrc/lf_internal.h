@@ -68,9 +68,10 @@ inline hipError_t read_back(void* h_dst, const void* d_src, size_t bytes, hipStr
 
 // Structural check of caller-supplied CSR (or BSR block) index arrays on the GPU, behind
 // lf_csr_check and in front of lf_csr_spmm / lf_bsr_spmm; `what` names the arrays in the
-// error message.  h_span (optional): see lf_csr_check_span.  Synchronises `s`.
+// error message.  h_span, h_longest (optional): see lf_csr_check_span, lf_csr_check_rows.  Synchronises `s`.
 int csr_check(const int32_t* d_indptr, const int32_t* d_indices, const float* d_values, int64_t num_rows,
-              int64_t num_cols, int64_t nnz, void* d_scratch, int32_t* h_flags, int64_t* h_span, const char* what, hipStream_t s);
+              int64_t num_cols, int64_t nnz, void* d_scratch, int32_t* h_flags, int64_t* h_span, int64_t* h_longest, const char* what,
+              hipStream_t s);
 }  // namespace lf
 #endif
 

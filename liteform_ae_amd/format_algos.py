@@ -215,6 +215,7 @@ class _DeviceCSR:
         self._seg_deg = {}
         self._stats_ws = {}          # num_parts -> statistics workspace holding the row bounds
         self._span = None
+        self._longest = None         # entries of the longest row, where the arrays were checked
         self._long_rows = None       # list of long rows and its counts, see csr_work
         self._csr_work = {}
         self._csr_lock = threading.Lock()
@@ -255,13 +256,13 @@ class _DeviceCSR:
         indptr = _upload(csr.indptr, np.int32)
         indices = _upload(csr.indices, np.int32)
         values = None if unit_values else _upload(csr.data, np.float32)
-        scratch = torch.empty(4, dtype=torch.int32, device="cuda")
-        flags, span = C.c_int32(0), C.c_int64(0)
-        _lib.check(lib.lf_csr_check_span(_lib.ptr(indptr), _lib.ptr(indices), _lib.ptr(values), self.num_rows, self.num_cols,
-                                         nnz, _lib.ptr(scratch), C.byref(flags), C.byref(span), _stream()))
+        scratch = torch.empty(8, dtype=torch.int32, device="cuda")
+        flags, span, longest = C.c_int32(0), C.c_int64(0), C.c_int64(0)
+        _lib.check(lib.lf_csr_check_rows(_lib.ptr(indptr), _lib.ptr(indices), _lib.ptr(values), self.num_rows, self.num_cols,
+                                         nnz, _lib.ptr(scratch), C.byref(flags), C.byref(span), C.byref(longest), _stream()))
         if not flags.value & _lib.LF_CSR_CANONICAL:
             return False
-        self._span = int(span.value)
+        self._span, self._longest = int(span.value), int(longest.value)
         self.indptr, self.indices, self.nnz = indptr, indices, nnz
         self.all_ones = unit_values or bool(flags.value & _lib.LF_CSR_UNIT_VALUES)
         self._values = values
@@ -301,25 +302,39 @@ class _DeviceCSR:
     def csr_work(self, feat: int, dtype: int):
         """What the C call of a CSR product takes: ((rows, columns, entries, span), address of the list of long rows, address of
         its counts, bytes of work space).  The list
-        (lf_csr_long_rows) is made for the matrix' first product and kept with it; a product that is recorded into a graph
-        before there is one does without."""
+        (lf_csr_long_rows) is made for the first product that wants it and kept with the matrix; a product that is recorded into
+        a graph before there is one does without."""
         work = self._csr_work.get((feat, dtype))
         if work is None:
             lib = _lib.load()
-            with self._csr_lock:
-                if self._long_rows is None and not _torch().cuda.is_current_stream_capturing():
-                    rows = _gpu_torch.empty(lib.lf_csr_long_rows_bytes(self.nnz), dtype=_gpu_torch.uint8, device="cuda")
-                    counts = np.zeros(3, dtype=np.int64)
-                    _lib.check(lib.lf_csr_long_rows(self.indptr.data_ptr(), self.num_rows, self.nnz, rows.data_ptr(), rows.numel(),
-                                                    _lib.np_ptr(counts, C.c_int64), _stream()))
-                    self._long_rows = (rows, counts) if counts[0] else (None, None)
-            rows, counts = self._long_rows or (None, None)
-            at = None if rows is None else _lib.np_ptr(counts, C.c_int64)
             sizes = (self.num_rows, self.num_cols, self.nnz, self.span)
-            work = (sizes, _lib.ptr(rows), at, lib.lf_csr_spmm_work_bytes(*sizes, at, feat, dtype))
-            if self._long_rows is not None:
+            rows = counts = None
+            nbytes = -1
+            if self._long_rows is None and self._longest is not None:
+                nbytes = lib.lf_csr_spmm_work_bytes(*sizes, None, self._longest, feat, dtype)
+            keep = nbytes >= 0
+            if not keep:
+                rows, counts = self._long_row_list()
+                keep = self._long_rows is not None
+                nbytes = lib.lf_csr_spmm_work_bytes(*sizes, counts, 0, feat, dtype)
+            work = (sizes, rows, counts, nbytes)
+            if keep:
                 self._csr_work[(feat, dtype)] = work
         return work
+
+    def _long_row_list(self):
+        """Addresses of the list of long rows and of its counts; None where there are no such rows, or no list yet and the
+        stream is being recorded."""
+        with self._csr_lock:
+            if self._long_rows is None and not _torch().cuda.is_current_stream_capturing():
+                lib = _lib.load()
+                rows = _gpu_torch.empty(lib.lf_csr_long_rows_bytes(self.nnz), dtype=_gpu_torch.uint8, device="cuda")
+                counts = np.zeros(3, dtype=np.int64)
+                _lib.check(lib.lf_csr_long_rows(self.indptr.data_ptr(), self.num_rows, self.nnz, rows.data_ptr(), rows.numel(),
+                                                _lib.np_ptr(counts, C.c_int64), _stream()))
+                self._long_rows = (rows, counts) if counts[0] else (None, None)
+            rows, counts = self._long_rows or (None, None)
+        return (None, None) if rows is None else (rows.data_ptr(), _lib.np_ptr(counts, C.c_int64))
 
     def seg_deg(self, num_parts: int):
         """Per-(partition,row) COO degrees on the device, or None when CSR lengths are the same."""
