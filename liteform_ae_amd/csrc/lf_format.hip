@@ -515,7 +515,10 @@ colmask_hist_kernel(const uint8_t* __restrict__ planes, int num_classes, int64_t
 // columns into a bitmap in LDS and writes the bitmap out once; colbits_hist_kernel ORs the bitmaps
 // of the workgroups that shared an item and counts the class masks.  The indices are streamed once
 // per slice, everything else stays in the CU.  2.45M columns (two slices), 81M entries: the
-// column pass takes 0.25 ms where the planes took 1.38 (marking 0.20, listing 0.03, histogram 0.02).
+// column pass takes 0.16 ms where the planes took 1.38 (marking 0.13, listing 0.01, histogram 0.02).
+// Marking is bound by the lines of the class's scattered segments (4.6M past the L2s, 0.6 GB) and by what a CU has under way.  It took
+// 202 us with loads behind a condition, one of a wavefront under way at a time, the slices' workgroups wherever they fell (8.8M
+// lines past the L2s) and shares by the lanes of a step: the last workgroups ended 50 us after most.
 //
 // Segments are first listed by class (class_list_kernel), because a class is a scattered subset of
 // the rows: finding it again in every workgroup would cost 11 sweeps over the row pointer.
@@ -529,6 +532,7 @@ constexpr int kMarkMaxSlices = 8;          // every slice of a partition streams
 constexpr int64_t kMarkMinRows = 131072;
 constexpr int64_t kMarkMaxSegments = 1ll << 26;     // 8 bytes each in the workspace
 constexpr int kMarkUnrollB = 8;
+constexpr int kMarkFours = 4;              // loads of four entries in flight, of a segment that a wavefront walks alone
 constexpr int kMarkEntries = 16384;        // entries that are worth one more workgroup
 
 struct MarkShape {
@@ -604,19 +608,31 @@ class_list_kernel(SegView v, const int32_t* __restrict__ seg_deg, int kmax, cons
     }
 }
 
-// Marks up to 64 * kMarkUnrollB entries of a segment from its entry j on.
+// Four entries of a segment with one load, which need only be aligned as they are; the last lanes of a segment move back to end where
+// it ends and mark entries twice.
+struct __attribute__((packed, aligned(4))) Four { uint32_t c[4]; };
+constexpr int kMarkPiece = 256 * kMarkFours;
+
+// Marks up to kMarkPiece entries of a segment from its entry j on.
+template <int N, typename Mark>
+__device__ __forceinline__ void mark_fours(const int32_t* __restrict__ first, int j, int fill, Mark mark) {
+    const int lane = threadIdx.x & 63;
+    Four f[N];
+#pragma unroll
+    for (int u = 0; u < N; ++u) f[u] = *(const Four*)(first + min(j + u * 256 + lane * 4, fill - 4));
+#pragma unroll
+    for (int u = 0; u < N; ++u)
+        for (int i = 0; i < 4; ++i) mark(f[u].c[i], j + u * 256 + lane * 4 < fill);
+}
 template <typename Mark>
 __device__ __forceinline__ void mark_piece(const int32_t* __restrict__ indices, int start, int j, int fill, Mark mark) {
     const int lane = threadIdx.x & 63;
-    uint32_t c[kMarkUnrollB];
-#pragma unroll
-    for (int u = 0; u < kMarkUnrollB; ++u) {
-        const int i = j + u * 64 + lane;
-        c[u] = i < fill ? (uint32_t)indices[start + i] : 0xFFFFFFFFu;
-    }
-#pragma unroll
-    for (int u = 0; u < kMarkUnrollB; ++u)
-        if (c[u] != 0xFFFFFFFFu) mark(c[u]);
+    if (fill - j > 256)
+        mark_fours<kMarkFours>(indices + start, j, fill, mark);
+    else if (fill >= 4)
+        mark_fours<1>(indices + start, j, fill, mark);
+    else if (lane < fill)
+        mark((uint32_t)indices[start + lane], true);
 }
 
 // The segments of the last class, of any length, one at a time per wavefront.
@@ -625,62 +641,113 @@ __device__ __forceinline__ void mark_long(const int32_t* __restrict__ indices, c
                                           int first_wave, int waves, Mark mark) {
     int2 seg = first_wave < n_seg ? list[first_wave] : make_int2(0, 0);
     for (int i = first_wave; i < n_seg; i += waves) {
-        const int2 cur = seg;
+        const int start = __builtin_amdgcn_readfirstlane(seg.x), fill = __builtin_amdgcn_readfirstlane(seg.y);
         if (i + waves < n_seg) seg = list[i + waves];                // a round ahead
-        for (int j = 0; j < cur.y; j += 64 * kMarkUnrollB) mark_piece(indices, cur.x, j, cur.y, mark);
+        for (int j = 0; j < fill; j += kMarkPiece) mark_piece(indices, start, j, fill, mark);
     }
 }
 
-// Marks the segments of class k (at most 2^k entries) that fall to one wavefront; K = min(k, 6).
-// The wavefront takes a group of segments at a time, one lane holding each, and walks it in steps of
-// 64 entries - 64 / 2^K segments side by side, or a 64-entry piece of a longer one - eight steps'
-// loads in flight.
+// Lanes that hold no segment of `least` entries or more point to one that another lane holds, with no entries: then every lane can
+// load.  (Loads behind a condition are branches, and the compiler waited for each before it used the next one's registers: one load
+// of a wavefront under way at a time instead of eight.)  False where no lane holds one.
+__device__ __forceinline__ bool spare_lanes(int2& seg, int least) {
+    const unsigned long long held = __ballot(seg.y >= least);
+    if (held == 0) return false;
+    const int start = __builtin_amdgcn_readlane(seg.x, __builtin_ctzll(held));
+    if (seg.y < least) seg = make_int2(start, 0);
+    return true;
+}
+
+// Marks the segments of class k < 3 (at most 2^k entries) that fall to one wavefront.
+// The wavefront takes 64 segments at a time, one lane holding each, and walks them in steps of 64 >> K segments side by side, eight
+// steps' loads in flight.
 template <int K, typename Mark>
-__device__ __forceinline__ void mark_class(const int32_t* __restrict__ indices, const int2* __restrict__ list, int n_seg,
-                                           int k, int first_wave, int waves, Mark mark) {
-    constexpr int kSide = 64 >> K;                     // segments side by side
+__device__ __forceinline__ void mark_short(const int32_t* __restrict__ indices, const int2* __restrict__ list, int n_seg,
+                                           int first_wave, int waves, Mark mark) {
+    constexpr int kSide = 64 >> K, kSteps = 1 << K, kFlight = kSteps < kMarkUnrollB ? kSteps : kMarkUnrollB;
     const int lane = threadIdx.x & 63;
     const int q = lane & ((1 << K) - 1), sub = lane >> K;
-    const int log_pieces = k - K;
-    const int group = K < 6 ? 64 : (64 >> (log_pieces < 4 ? log_pieces : 4));     // segments of a group
+    int64_t i0 = (int64_t)first_wave * 64;
+    const int64_t stride = (int64_t)waves * 64;
+    int2 seg = make_int2(0, 0);
+    if (i0 + lane < n_seg) seg = list[i0 + lane];
+    for (; i0 < n_seg; i0 += stride) {
+        int2 cur = seg;
+        seg = make_int2(0, 0);
+        if (i0 + stride + lane < n_seg) seg = list[i0 + stride + lane];      // a round ahead
+        if (!spare_lanes(cur, 1)) continue;
+#pragma unroll
+        for (int t0 = 0; t0 < kSteps; t0 += kFlight) {
+            uint32_t c[kFlight];
+            bool on[kFlight];
+#pragma unroll
+            for (int u = 0; u < kFlight; ++u) {
+                const int start = __shfl(cur.x, (t0 + u) * kSide + sub), fill = __shfl(cur.y, (t0 + u) * kSide + sub);
+                on[u] = q < fill;
+                c[u] = (uint32_t)indices[start + max(min(q, fill - 1), 0)];
+            }
+#pragma unroll
+            for (int u = 0; u < kFlight; ++u)
+                mark(c[u], on[u]);
+        }
+    }
+}
+
+// Marks the segments of class k >= 3 (at most 2^k entries) that fall to one wavefront; L = min(k - 2, 6).
+// A lane takes four entries with one load of 16 bytes, which need only be aligned as the entries are; the last lane of a segment
+// moves back to end where it ends and marks up to three entries twice.  So 64 >> L segments are walked side by side, or 256 entries of a
+// longer one.
+template <int L, typename Mark>
+__device__ __forceinline__ void mark_class(const int32_t* __restrict__ indices, const int2* __restrict__ list, int n_seg,
+                                           int k, int first_wave, int waves, Mark mark) {
+    constexpr int kSide = 64 >> L;                     // segments side by side
+    constexpr int kFlight = L < 3 ? 1 << L : 8;        // (never more than a group's steps; 8 against 4: 130 -> 124 us)
+    const int lane = threadIdx.x & 63;
+    const int q = lane & ((1 << L) - 1), sub = lane >> L;
+    const int log_pieces = k - 2 - L;                  // L < 6: 0
+    const int group = max(64 >> max(k - 6, 0), 4);     // segments of a group: about as many entries in every class
     const int steps = (group / kSide) << log_pieces;
     int64_t i0 = (int64_t)first_wave * group;
     const int64_t stride = (int64_t)waves * group;
     int2 seg = make_int2(0, 0);
     if (lane < group && i0 + lane < n_seg) seg = list[i0 + lane];
     for (; i0 < n_seg; i0 += stride) {
-        const int2 cur = seg;
+        int2 cur = seg;
         seg = make_int2(0, 0);
         if (lane < group && i0 + stride + lane < n_seg) seg = list[i0 + stride + lane];      // a round ahead
-        for (int t0 = 0; t0 < steps; t0 += kMarkUnrollB) {
-            uint32_t c[kMarkUnrollB];
-            bool on[kMarkUnrollB];
+        // (a segment's class is that of its degree, which may count twice what the structure holds once)
+        if (__ballot(cur.y > 0 && cur.y < 4) != 0)
+            for (int i = 0; i < cur.y && cur.y < 4; ++i) mark((uint32_t)indices[cur.x + i]);
+        if (!spare_lanes(cur, 4)) continue;
+        for (int t0 = 0; t0 < steps; t0 += kFlight) {
+            Four f[kFlight];
+            bool on[kFlight];
 #pragma unroll
-            for (int u = 0; u < kMarkUnrollB; ++u) {
+            for (int u = 0; u < kFlight; ++u) {
                 const int t = t0 + u;
-                int start, fill, at = q;
-                if constexpr (K == 6) {
+                int start, fill, at = q * 4;
+                if constexpr (L == 6) {
                     const int src = (t >> log_pieces) & 63;
                     start = __builtin_amdgcn_readlane(cur.x, src);
                     fill = __builtin_amdgcn_readlane(cur.y, src);
-                    at = ((t & ((1 << log_pieces) - 1)) << 6) + lane;
+                    at += (t & ((1 << log_pieces) - 1)) << 8;
                 } else {
                     start = __shfl(cur.x, (t * kSide + sub) & 63);
                     fill = __shfl(cur.y, (t * kSide + sub) & 63);
                 }
-                on[u] = t < steps && at < fill;
-                c[u] = on[u] ? (uint32_t)indices[start + at] : 0u;
+                on[u] = at < fill;
+                f[u] = *(const Four*)(indices + start + max(min(at, fill - 4), 0));
             }
 #pragma unroll
-            for (int u = 0; u < kMarkUnrollB; ++u)
-                if (on[u]) mark(c[u]);
+            for (int u = 0; u < kFlight; ++u)
+                for (int j = 0; j < 4; ++j) mark(f[u].c[j], on[u]);
         }
     }
 }
 
-// One workgroup per share of an item (partition p, slice s, class k), i = (p * slices + s) * classes
-// + k: workgroups are dealt out in proportion to the entries of the item's class, at least one to an
-// item that has any.  table[i] = first workgroup of item i, table[n_items] = workgroups in use.
+// One workgroup per slice and share of an item (partition p, class k), i = p * classes + k: places for a workgroup of every slice are
+// dealt out in proportion to the entries of the item, at least one to an item that has any.  table[i] = first place of item i,
+// table[n_items] = places in use; slice s of place j writes bitmap s * (groups / slices) + j.
 __global__ void __launch_bounds__(kMarkThreads)
 mark_columns_kernel(const int32_t* __restrict__ indices, const int2* __restrict__ lists, int64_t rows, int parts,
                     int num_classes, MarkShape shape, int64_t psize, int64_t cols,
@@ -692,16 +759,29 @@ mark_columns_kernel(const int32_t* __restrict__ indices, const int2* __restrict_
     __shared__ int s_cnt[kMarkThreads / 64];
     __shared__ int s_item;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int n_items = parts * shape.slices * num_classes;
+    const int n_items = parts * num_classes;
+
+    // ---- workgroup -> (slice s, place j): the workgroups of a place are eight apart, on one XCD, and read the same lines
+    const int S = shape.slices, places = gridDim.x / S, whole = gridDim.x / (8 * S) * 8;      // whole: places in full rounds of eight
+    int s, j;
+    if ((int)blockIdx.x < whole * S) {
+        s = (int)blockIdx.x / 8 % S;
+        j = (int)blockIdx.x / (8 * S) * 8 + (int)blockIdx.x % 8;
+    } else {
+        const int rest = (int)blockIdx.x - whole * S, left = max(places - whole, 1);
+        s = rest / left;
+        j = whole + rest % left;
+        if (s >= S || j >= places) return;
+    }
 
     // ---- which item, and which share of it
-    unsigned long long w = 0;                          // entries and unused lanes (a step costs what it costs)
+    unsigned long long w = 0;
     if (tid < n_items) {
-        const int kk = tid % num_classes, pp = tid / num_classes / shape.slices;
+        const int kk = tid % num_classes, pp = tid / num_classes;
         const unsigned long long entries = stats[stat_at(pp, kk, 1)], segs = stats[stat_at(pp, kk, 2)];
-        w = kk <= 6 ? segs << kk : entries + 32 * segs;
-        if (kk == num_classes - 1) w += entries;
-        if (kk < 3) w *= 4 - kk;                       // (short segments: every lane or pair of lanes on a line of its own)
+        w = entries + 6 * segs;                        // as their times were; fewer loads are under way
+        if (kk < 3) w += w / 2;                        // where a group's steps are few
+        if (kk == num_classes - 1) w += w / 8;         // or a wavefront has one segment
     }
     unsigned long long sum = w;
     for (int d = 32; d > 0; d >>= 1) sum += __shfl_xor(sum, d);
@@ -713,7 +793,7 @@ mark_columns_kernel(const int32_t* __restrict__ indices, const int2* __restrict_
     int nz = 0;
     for (int i = 0; i < kMarkThreads / 64; ++i) { total += s_sum[i]; nz += s_cnt[i]; }
     const unsigned long long worth = total / kMarkEntries;      // a small matrix is not spread over more bitmaps than it pays for
-    const unsigned long long more = worth < gridDim.x - nz ? worth : gridDim.x - nz;
+    const unsigned long long more = worth < (unsigned long long)(places - nz) ? worth : places - nz;
     const int m = w > 0 ? 1 + (int)(more * w / total) : 0;
     int incl = m;
     for (int d = 1; d < 64; d <<= 1) {
@@ -729,17 +809,17 @@ mark_columns_kernel(const int32_t* __restrict__ indices, const int2* __restrict_
     if (tid < n_items) {
         s_first[tid] = before;
         if (tid == n_items - 1) s_first[n_items] = before + m;
-        if ((int)blockIdx.x >= before && (int)blockIdx.x < before + m) s_item = tid;
+        if (j >= before && j < before + m) s_item = tid;
     }
     for (int i = tid; i < shape.words; i += kMarkThreads) s_bits[i] = 0;
     __syncthreads();
     if (blockIdx.x == 0)
         for (int i = tid; i <= n_items; i += kMarkThreads) table[i] = s_first[i];
     const int item = s_item;
-    if (item < 0) return;                              // more workgroups than shares
+    if (item < 0) return;                              // more places than shares
 
-    const int k = item % num_classes, s = item / num_classes % shape.slices, p = item / num_classes / shape.slices;
-    const int share = (int)blockIdx.x - s_first[item], shares = s_first[item + 1] - s_first[item];
+    const int k = item % num_classes, p = item / num_classes;
+    const int share = j - s_first[item], shares = s_first[item + 1] - s_first[item];
     const int64_t c0 = (int64_t)p * psize + (int64_t)s * shape.slice_cols;
     int64_t c1 = c0 + shape.slice_cols;
     if (c1 > (int64_t)(p + 1) * psize) c1 = (int64_t)(p + 1) * psize;
@@ -751,20 +831,22 @@ mark_columns_kernel(const int32_t* __restrict__ indices, const int2* __restrict_
     const int n_big = k == num_classes - 1 ? (int)stats[stat_at(p, k, 2) + 2] : 0;
     const int n_seg = (int)stats[stat_at(p, k, 2)] - n_big;
     const int2* list = lists + (size_t)p * (size_t)rows + first;
-    auto mark = [&](uint32_t c) {
+    auto mark = [&](uint32_t c, bool on = true) {
         const uint32_t x = c - base_col;               // (wraps to a large value below the slice)
-        if (x < span) atomicOr(&s_bits[x >> 5], 1u << (x & 31u));
+        if (x < (on ? span : 0u)) atomicOr(&s_bits[x >> 5], 1u << (x & 31u));
     };
 
     const int waves = shares * (kMarkThreads / 64);
     const int first_wave = share * (kMarkThreads / 64) + wave;
     switch (k < num_classes - 1 ? k : LF_MAX_CLASSES) {
-        case 0: mark_class<0>(indices, list, n_seg, k, first_wave, waves, mark); break;
-        case 1: mark_class<1>(indices, list, n_seg, k, first_wave, waves, mark); break;
-        case 2: mark_class<2>(indices, list, n_seg, k, first_wave, waves, mark); break;
-        case 3: mark_class<3>(indices, list, n_seg, k, first_wave, waves, mark); break;
-        case 4: mark_class<4>(indices, list, n_seg, k, first_wave, waves, mark); break;
-        case 5: mark_class<5>(indices, list, n_seg, k, first_wave, waves, mark); break;
+        case 0: mark_short<0>(indices, list, n_seg, first_wave, waves, mark); break;
+        case 1: mark_short<1>(indices, list, n_seg, first_wave, waves, mark); break;
+        case 2: mark_short<2>(indices, list, n_seg, first_wave, waves, mark); break;
+        case 3: mark_class<1>(indices, list, n_seg, k, first_wave, waves, mark); break;
+        case 4: mark_class<2>(indices, list, n_seg, k, first_wave, waves, mark); break;
+        case 5: mark_class<3>(indices, list, n_seg, k, first_wave, waves, mark); break;
+        case 6: mark_class<4>(indices, list, n_seg, k, first_wave, waves, mark); break;
+        case 7: mark_class<5>(indices, list, n_seg, k, first_wave, waves, mark); break;
         default:
             if (k < num_classes - 1) mark_class<6>(indices, list, n_seg, k, first_wave, waves, mark);
             break;
@@ -772,12 +854,12 @@ mark_columns_kernel(const int32_t* __restrict__ indices, const int2* __restrict_
     if (k == num_classes - 1) mark_long(indices, list, n_seg, first_wave, waves, mark);
     for (int i = 0; i < n_big; ++i) {
         const int2 seg = list[n_seg + i];
-        const int64_t stride = (int64_t)waves * 64 * kMarkUnrollB;
-        for (int64_t j = (int64_t)first_wave * 64 * kMarkUnrollB; j < seg.y; j += stride)
-            mark_piece(indices, seg.x, (int)j, seg.y, mark);
+        const int64_t stride = (int64_t)waves * kMarkPiece;
+        for (int64_t at = (int64_t)first_wave * kMarkPiece; at < seg.y; at += stride)
+            mark_piece(indices, seg.x, (int)at, seg.y, mark);
     }
     __syncthreads();
-    uint32_t* out = bitmaps + (size_t)blockIdx.x * shape.words;
+    uint32_t* out = bitmaps + ((size_t)s * places + j) * shape.words;
     for (int i = tid; i < shape.words; i += kMarkThreads) out[i] = s_bits[i];
 }
 
@@ -801,8 +883,9 @@ colbits_hist_kernel(const uint32_t* __restrict__ bitmaps, const int32_t* __restr
     const int k = threadIdx.x >> 6, word = threadIdx.x & 63;
     int g0 = 0, g1 = 0;
     if (k < num_classes) {
-        g0 = table[(int)blockIdx.y * num_classes + k];
-        g1 = table[(int)blockIdx.y * num_classes + k + 1];
+        const int first = s * (shape.groups / shape.slices);
+        g0 = first + table[p * num_classes + k];
+        g1 = first + table[p * num_classes + k + 1];
     }
     for (int w0 = blockIdx.x * 64; w0 < shape.words && c0 + (int64_t)w0 * 32 < c1; w0 += gridDim.x * 64) {      // uniform
         uint32_t bits = 0;

@@ -89,6 +89,31 @@ def test_column_sets_of_large_matrices(fa, nr, nc, parts, limit):
             assert stats[p, c].tolist() == [rows, f[on].sum(), on.sum(), 0]
 
 
+@pytest.mark.parametrize("nc,parts", [(30_000, 1), (1_300_000, 1), (2_600_000, 1), (2_600_000, 3)])       # slices: 1, 2, 3, 1
+@pytest.mark.parametrize("copies", [1, 3])       # of every entry: the class follows the degree, the columns are there once
+def test_column_sets_by_length(fa, nc, parts, copies):
+    nr = 131072
+    rng = np.random.default_rng(nc + copies)
+    edges = np.array([1, 2, 3, 4, 5, 7, 8, 9, 12, 13, 16, 17, 31, 32, 33, 63, 64, 65, 128, 129, 255, 256, 257, 260, 512, 513, 1025, 1300])
+    deg = rng.choice([1, 2, 3, 4, 6], size=nr)
+    deg[-2 * len(edges):] = np.concatenate([edges, edges[::-1]])  # among them the last segments of the index array, of one entry
+    row = np.repeat(np.arange(nr), deg)
+    col = (rng.integers(0, nc, size=nr)[row] + np.arange(len(row))) % nc if parts == 1 else rng.integers(0, nc, size=len(row))
+    key = np.unique(row * nc + col)
+    row, col = key // nc, key % nc
+    g = MTX.from_coo(np.tile(row, copies), np.tile(col, copies), (nr, nc))
+    stats, hist = fa.bucket_statistics(g, parts)
+    psize = -(-nc // parts)
+    seg = (col // psize) * nr + row
+    fill = np.bincount(seg, minlength=parts * nr) * copies
+    k = np.minimum(np.ceil(np.log2(np.maximum(fill, 1))).astype(np.int64), 10)
+    touched = np.unique(k[seg] * nc + col)
+    masks = np.zeros(nc, np.int64)
+    np.add.at(masks, touched % nc, 1 << (touched // nc))
+    for p in range(parts):
+        np.testing.assert_array_equal(hist[p], np.bincount(masks[p * psize:(p + 1) * psize], minlength=2048))
+
+
 @pytest.mark.parametrize("seed", range(8))
 def test_search_matches_oracle(fa, seed):
     rng = np.random.default_rng(60 + seed)
