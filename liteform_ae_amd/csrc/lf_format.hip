@@ -236,17 +236,26 @@ __host__ __device__ constexpr size_t stat_at(int p, int k, int f) { return (((si
 constexpr int kCountGrid = 256, kCountThreads = 1024;      // (atomics of 512 workgroups on a counter's line: 9 us)
 constexpr int kRowUnroll = 4;              // rows whose bounds a thread requests together
 
-// Degrees of the segments of rows r0, r0 + stride, ... (0 past `end`).
+// Segments of rows r0 < end, r0 + stride, ... and their degrees (0 past `end`).  Every lane loads: behind a condition the loads of a
+// row would wait for those of the row before.
 __device__ __forceinline__ void seg_degrees(const SegView& v, const int32_t* __restrict__ seg_deg, int p, int64_t r0,
-                                            int64_t stride, int64_t end, int (&deg)[kRowUnroll]) {
+                                            int64_t stride, int64_t end, int (&start)[kRowUnroll], int (&fill)[kRowUnroll], int (&deg)[kRowUnroll]) {
+    const int32_t *first = v.parts == 1 ? v.indptr : v.bnd + (int64_t)p * v.rows, *last = v.parts == 1 ? v.indptr + 1 : first + v.rows;
 #pragma unroll
     for (int u = 0; u < kRowUnroll; ++u) {
-        const int64_t r = r0 + u * stride;
-        deg[u] = 0;
-        if (r >= end) continue;
-        int start;
-        seg_range(v, r, p, start, deg[u]);
-        if (seg_deg) deg[u] = seg_deg[(int64_t)p * v.rows + r];
+        const int64_t r = min(r0 + u * stride, end - 1);
+        start[u] = first[r];
+        fill[u] = last[r];
+    }
+    if (seg_deg) {
+#pragma unroll
+        for (int u = 0; u < kRowUnroll; ++u) deg[u] = seg_deg[(int64_t)p * v.rows + min(r0 + u * stride, end - 1)];
+    }
+#pragma unroll
+    for (int u = 0; u < kRowUnroll; ++u) {
+        fill[u] -= start[u];
+        if (!seg_deg) deg[u] = fill[u];
+        if (r0 + u * stride >= end) deg[u] = 0;
     }
 }
 
@@ -270,8 +279,8 @@ class_count_kernel(SegView v, const int32_t* __restrict__ seg_deg, int kmax, uns
     const int64_t lo = (int64_t)blockIdx.x * per, hi = lo + per < v.rows ? lo + per : v.rows;
     unsigned long long* mine = s_sum + (threadIdx.x & 63);
     for (int64_t r0 = lo + threadIdx.x; r0 < hi; r0 += kRowUnroll * kCountThreads) {
-        int deg[kRowUnroll];
-        seg_degrees(v, seg_deg, p, r0, kCountThreads, hi, deg);
+        int start[kRowUnroll], fill[kRowUnroll], deg[kRowUnroll];
+        seg_degrees(v, seg_deg, p, r0, kCountThreads, hi, start, fill, deg);
 #pragma unroll
         for (int u = 0; u < kRowUnroll; ++u) {
             if (deg[u] <= 0) continue;
@@ -318,6 +327,9 @@ class_count_kernel(SegView v, const int32_t* __restrict__ seg_deg, int kmax, uns
 constexpr int kShapeCands = 16;
 constexpr int kShapeParts = 128;           // partitions of all candidates together
 constexpr int kShapeGrid = 1024;
+// A lane searches the boundaries of a row one after the other, each search a chain of loads; those of a longer row are searched by the
+// lanes of the wavefront side by side (170K rows, the longest of 13,000 entries, 7 partitions: 21.5 -> 17 us; from 8 entries on 21.6, from 16 18.6).
+constexpr int kShapeLongRow = 64;
 struct ShapeCands {
     int n, total;
     int parts[kShapeCands];
@@ -332,28 +344,49 @@ shape_stats_kernel(const int32_t* __restrict__ indptr, const int32_t* __restrict
                    ShapeCands cands, int kmax, unsigned long long* __restrict__ partial,
                    unsigned long long* __restrict__ out, int n_out) {
     __shared__ unsigned long long s_cnt[shape_words(kShapeParts)];
+    __shared__ int64_t s_end[kShapeParts];                     // first column behind a partition; behind a candidate's last: none
+    __shared__ uint8_t s_first[kShapeParts];                   // a candidate's first partition
     const int n_words = shape_words(cands.total);
     for (int i = threadIdx.x; i < n_words; i += kBlock) s_cnt[i] = 0;
+    for (int c = 0, q = 0; c < cands.n; q += cands.parts[c++]) {
+        const int parts = cands.parts[c];
+        const int64_t psize = (cols + parts - 1) / parts;
+        for (int p = threadIdx.x; p < parts; p += kBlock) {
+            s_end[q + p] = p + 1 < parts ? (p + 1) * psize : INT64_MAX;
+            s_first[q + p] = p == 0;
+        }
+    }
     if (blockIdx.x == 0)                                       // for the launch behind this one
         for (int i = threadIdx.x; i < n_out; i += kBlock) out[i] = 0;
     __syncthreads();
-    for (int64_t r = (int64_t)blockIdx.x * kBlock + threadIdx.x; r < rows; r += (int64_t)gridDim.x * kBlock) {
-        const int lo = indptr[r], hi = indptr[r + 1];
-        if (lo >= hi) continue;
-        int q = 0;
-        for (int c = 0; c < cands.n; ++c) {
-            const int parts = cands.parts[c];
-            const int64_t psize = (cols + parts - 1) / parts;
-            int cur = lo;
-            for (int p = 0; p < parts; ++p, ++q) {
-                const int end = p + 1 < parts ? lower_bound_i32(indices, cur, hi, (int64_t)(p + 1) * psize) : hi;
-                const int fill = end - cur;
-                cur = end;
-                if (fill <= 0) continue;
-                int k, cost_rows;
-                width_class(fill, kmax, k, cost_rows);
-                atomicAdd(&s_cnt[q * LF_MAX_CLASSES + k], (1ull << 32) | (unsigned long long)fill);
-                if (cost_rows > 1) atomicAdd(&s_cnt[cands.total * LF_MAX_CLASSES + q], (unsigned long long)(cost_rows - 1));
+    const int lane = threadIdx.x & 63;
+    auto count = [&](int q, int fill) {
+        if (fill <= 0) return;
+        int k, cost_rows;
+        width_class(fill, kmax, k, cost_rows);
+        atomicAdd(&s_cnt[q * LF_MAX_CLASSES + k], (1ull << 32) | (unsigned long long)fill);
+        if (cost_rows > 1) atomicAdd(&s_cnt[cands.total * LF_MAX_CLASSES + q], (unsigned long long)(cost_rows - 1));
+    };
+    for (int64_t r0 = (int64_t)blockIdx.x * kBlock + threadIdx.x - lane; r0 < rows; r0 += (int64_t)gridDim.x * kBlock) {
+        const int64_t r = min(r0 + lane, rows - 1);
+        const int lo = indptr[r], hi = r0 + lane < rows ? indptr[r + 1] : lo;
+        const bool alone = hi - lo <= kShapeLongRow;
+        for (int q = 0, cur = lo; q < cands.total && alone; ++q) {
+            const int from = s_first[q] ? lo : cur;
+            cur = s_end[q] < INT64_MAX ? lower_bound_i32(indices, from, hi, s_end[q]) : hi;
+            count(q, cur - from);
+        }
+        for (unsigned long long pending = __ballot(!alone); pending != 0; pending &= pending - 1) {
+            const int src = __builtin_ctzll(pending), first = __shfl(lo, src), last = __shfl(hi, src);
+            int before = first;                                // end of the partition before this round's
+            for (int q0 = 0; q0 < cands.total; q0 += 64) {
+                const int q = min(q0 + lane, cands.total - 1);
+                const int end = s_end[q] < INT64_MAX ? lower_bound_i32(indices, first, last, s_end[q]) : last;
+                int from = __shfl_up(end, 1);
+                if (lane == 0) from = before;
+                if (s_first[q]) from = first;
+                if (q0 + lane < cands.total) count(q, end - from);
+                before = __shfl(end, 63);
             }
         }
     }
@@ -592,12 +625,7 @@ class_list_kernel(SegView v, const int32_t* __restrict__ seg_deg, int kmax, cons
     int2* out = lists + (size_t)p * (size_t)v.rows;
     for (int64_t r0 = lo + threadIdx.x; r0 < hi; r0 += kRowUnroll * kCountThreads) {
         int deg[kRowUnroll], start[kRowUnroll], fill[kRowUnroll];
-        seg_degrees(v, seg_deg, p, r0, kCountThreads, hi, deg);
-#pragma unroll
-        for (int u = 0; u < kRowUnroll; ++u) {
-            start[u] = fill[u] = 0;
-            if (r0 + u * kCountThreads < hi) seg_range(v, r0 + u * kCountThreads, p, start[u], fill[u]);
-        }
+        seg_degrees(v, seg_deg, p, r0, kCountThreads, hi, start, fill, deg);
 #pragma unroll
         for (int u = 0; u < kRowUnroll; ++u) {
             int k, cost_rows;
@@ -1052,7 +1080,8 @@ hyb_scan_kernel(int32_t* __restrict__ blockcnt, int nblk, long long* __restrict_
 //     padding included, with 16-byte accesses wherever a group lies inside one row.
 // Reading in row order matters: a source row is ~130 bytes at an arbitrary offset, and when
 // the slabs were filled bucket by bucket every row cost two full cache lines (1.27 GB fetched
-// for 0.65 GB of entries on an 81.6M-nonzero matrix).
+// for 0.65 GB of entries on an 81.6M-nonzero matrix).  Bound by memory: that matrix, 0.65 GB read and 0.75 GB written, takes 295 us, 4.8
+// TB/s (322 with the loads of a group behind conditions, which made a step of four groups wait four times).
 constexpr int kFillUnroll = 4;
 constexpr int kPartGroup = 4;        // column partitions whose segments are walked together
 // four consecutive 32-bit values at a 4-byte aligned address (one 16-byte load)
@@ -1080,6 +1109,7 @@ hyb_fill_kernel(SegView v, const int32_t* __restrict__ seg_deg, const int32_t* _
     __shared__ uint32_t s_wave[kBlock / 64];
     const int64_t r = (int64_t)blockIdx.x * kBlock + threadIdx.x;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int nnz = v.indptr[v.rows];
 
     for (int p0 = 0; p0 < v.parts; p0 += kPartGroup) {
         const int pg = min(kPartGroup, v.parts - p0);
@@ -1193,68 +1223,79 @@ hyb_fill_kernel(SegView v, const int32_t* __restrict__ seg_deg, const int32_t* _
         const int n_seg = kBlock * pg;
         const int steps = 8 + (pg > 1) + (pg > 2);       // ceil(log2(n_seg))
         const uint32_t total = s_off[n_seg];
-        for (uint32_t j0 = 0; j0 < total; j0 += kBlock * kFillUnroll * 4) {
-            long long at[kFillUnroll];
-            int len[kFillUnroll];                     // slots of the group inside its segment (0: none)
-            int4 c[kFillUnroll];
-            float4 x[kFillUnroll], m[kFillUnroll];
+        // Every lane loads four entries, whatever the group holds of them: behind a condition each load would be waited for before the
+        // next.  The last groups of the index array move back to end where it ends and shift.
+        auto walk = [&](auto tiny) {                  // tiny: the array has fewer than four entries
+            for (uint32_t j0 = 0; j0 < total; j0 += kBlock * kFillUnroll * 4) {
+                long long at[kFillUnroll];
+                int len[kFillUnroll];                 // slots of the group inside its segment (0: none)
+                int live[kFillUnroll], shift[kFillUnroll];
+                int4 c[kFillUnroll];
+                float4 x[kFillUnroll];
 #pragma unroll
-            for (int u = 0; u < kFillUnroll; ++u) {
-                const uint32_t j = j0 + (u * kBlock + threadIdx.x) * 4;
-                at[u] = 0;
-                len[u] = 0;
-                c[u] = make_int4(0, 0, 0, 0);
-                x[u] = make_float4(0.f, 0.f, 0.f, 0.f);
-                m[u] = make_float4(0.f, 0.f, 0.f, 0.f);
-                if (j < total) {
+                for (int u = 0; u < kFillUnroll; ++u) {
+                    const uint32_t mine = j0 + (u * kBlock + threadIdx.x) * 4, j = min(mine, total - 4);
                     int lo = 0, hi = n_seg - 1;        // last segment whose offset is <= j
                     for (int step = 0; step < steps; ++step) {
                         const int mid = (lo + hi + 1) >> 1;
                         if (s_off[mid] <= j) lo = mid; else hi = mid - 1;
                     }
                     const int q = (int)(j - s_off[lo]);
-                    const int live = s_fill[lo] - q;  // entries of the source row from q on
+                    live[u] = s_fill[lo] - q;          // entries of the source row from q on
                     at[u] = s_dst[lo] + q;
-                    len[u] = min(4, (int)s_len[lo] - q);
-                    const int src = s_start[lo] + q;
-                    if (live >= 4) {
-                        const Packed4i ci = *reinterpret_cast<const Packed4i*>(indices + src);
+                    len[u] = mine < total ? min(4, (int)s_len[lo] - q) : 0;
+                    const int src = s_start[lo] + q, from = tiny ? 0 : min(src, nnz - 4);
+                    shift[u] = live[u] > 0 ? src - from : 0;
+                    x[u] = make_float4(1.f, 1.f, 1.f, 1.f);
+                    if constexpr (tiny) {
+                        const int last = max(nnz - 1, 0);
+                        if (nnz > 0) {
+                            c[u] = make_int4(indices[0], indices[min(1, last)], indices[min(2, last)], 0);
+                            if (values) x[u] = make_float4(values[0], values[min(1, last)], values[min(2, last)], 0.f);
+                        }
+                    } else {
+                        const Packed4i ci = *reinterpret_cast<const Packed4i*>(indices + from);
                         c[u] = make_int4(ci.x, ci.y, ci.z, ci.w);
                         if (values) {
-                            const Packed4f xv = *reinterpret_cast<const Packed4f*>(values + src);
+                            const Packed4f xv = *reinterpret_cast<const Packed4f*>(values + from);
                             x[u] = make_float4(xv.x, xv.y, xv.z, xv.w);
-                        } else {
-                            x[u] = make_float4(1.f, 1.f, 1.f, 1.f);
                         }
-                        m[u] = make_float4(1.f, 1.f, 1.f, 1.f);
+                    }
+                }
+#pragma unroll
+                for (int u = 0; u < kFillUnroll; ++u) {
+                    if (__ballot(shift[u] != 0) != 0)
+                        for (int i = 0; i < 3; ++i)
+                            if (shift[u] > i) {
+                                c[u].x = c[u].y, c[u].y = c[u].z, c[u].z = c[u].w;
+                                x[u].x = x[u].y, x[u].y = x[u].z, x[u].z = x[u].w;
+                            }
+                    const bool v0 = live[u] > 0, v1 = live[u] > 1, v2 = live[u] > 2, v3 = live[u] > 3;
+                    const int4 cc4 = make_int4(v0 ? c[u].x : 0, v1 ? c[u].y : 0, v2 ? c[u].z : 0, v3 ? c[u].w : 0);
+                    const float4 xx4 = make_float4(v0 ? x[u].x : 0.f, v1 ? x[u].y : 0.f, v2 ? x[u].z : 0.f, v3 ? x[u].w : 0.f);
+                    const float4 mm4 = make_float4(v0, v1, v2, v3);
+                    if (len[u] == 4 && (at[u] & 3) == 0) {
+                        *reinterpret_cast<int4*>(out_cols + at[u]) = cc4;
+                        *reinterpret_cast<float4*>(out_vals + at[u]) = xx4;
+                        if (out_mask) *reinterpret_cast<float4*>(out_mask + at[u]) = mm4;
                     } else {
-                        if (live > 0) { c[u].x = indices[src];     x[u].x = values ? values[src] : 1.f;     m[u].x = 1.f; }
-                        if (live > 1) { c[u].y = indices[src + 1]; x[u].y = values ? values[src + 1] : 1.f; m[u].y = 1.f; }
-                        if (live > 2) { c[u].z = indices[src + 2]; x[u].z = values ? values[src + 2] : 1.f; m[u].z = 1.f; }
-                    }
-                }
-            }
+                        const int cc[4] = {cc4.x, cc4.y, cc4.z, cc4.w};
+                        const float xx[4] = {xx4.x, xx4.y, xx4.z, xx4.w};
+                        const float mm[4] = {mm4.x, mm4.y, mm4.z, mm4.w};
 #pragma unroll
-            for (int u = 0; u < kFillUnroll; ++u) {
-                if (len[u] == 4 && (at[u] & 3) == 0) {
-                    *reinterpret_cast<int4*>(out_cols + at[u]) = c[u];
-                    *reinterpret_cast<float4*>(out_vals + at[u]) = x[u];
-                    if (out_mask) *reinterpret_cast<float4*>(out_mask + at[u]) = m[u];
-                } else {
-                    const int cc[4] = {c[u].x, c[u].y, c[u].z, c[u].w};
-                    const float xx[4] = {x[u].x, x[u].y, x[u].z, x[u].w};
-                    const float mm[4] = {m[u].x, m[u].y, m[u].z, m[u].w};
-#pragma unroll
-                    for (int i = 0; i < 4; ++i) {
-                        if (i < len[u]) {
-                            out_cols[at[u] + i] = cc[i];
-                            out_vals[at[u] + i] = xx[i];
-                            if (out_mask) out_mask[at[u] + i] = mm[i];
+                        for (int i = 0; i < 4; ++i) {
+                            if (i < len[u]) {
+                                out_cols[at[u] + i] = cc[i];
+                                out_vals[at[u] + i] = xx[i];
+                                if (out_mask) out_mask[at[u] + i] = mm[i];
+                            }
                         }
                     }
                 }
             }
-        }
+        };
+        if (nnz >= 4) walk(std::false_type{});
+        else walk(std::true_type{});
         __syncthreads();          // the tables are rewritten for the next group of partitions
     }
 }

@@ -172,6 +172,22 @@ def test_builder_edge_cases(fa):
     assert rows[0][1].shape == (0,) and cols[0][1].shape == (0, 2) and mask[0][2].shape == (0, 4)
 
 
+@pytest.mark.parametrize("lists", [[[2]], [[], [0, 3], []], [[5], [1, 2]], [[0], [1], [2]], [[1], [0, 2, 3]], [[0, 1, 2, 3, 4], [6]], [[3], list(range(9)), [0, 1]]])
+@pytest.mark.parametrize("widths", [[1], [2, 8], [4], [16]])
+def test_builder_of_few_entries(fa, lists, widths):
+    # groups of four slots end where the index array ends, or hold all of it
+    row, col = np.array([(i, j) for i, cols in enumerate(lists) for j in cols]).T
+    g = MTX.from_coo(row, col, (len(lists), 10), data=np.arange(1, len(row) + 1, dtype=np.float32))
+    assert_hyb_equal(fa.build_hyb_format(g, [widths]), O.build_hyb_format_sequential(g, [widths]))
+    fmt = fa.build_hyb_format_device(g, [widths])
+    seen = []
+    for k in range(fmt.num_buckets):
+        rows, cols, vals = (x.cpu().numpy() for x in fmt.slab(k)[:3])
+        at = np.flatnonzero(vals)
+        seen += zip(vals[at].tolist(), rows[at // widths[k]].tolist(), cols[at].tolist())
+    assert sorted(seen) == [(i + 1.0, r, c) for i, (r, c) in enumerate(zip(row.tolist(), col.tolist()))]
+
+
 def test_duplicate_coo_entries(fa):
     """COO duplicates raise the degree but not the fill (format_algos.py:250-254)."""
     from liteform_ae_amd.format_matrix_market import MTX
