@@ -708,8 +708,7 @@ struct MergedBucket {
 template <bool kEmit, typename Emit>
 __device__ __forceinline__ int merge_group(const int32_t* __restrict__ cols, const float* __restrict__ vals,
                                            const int32_t* __restrict__ meta, long long g, long long n_rows,
-                                           int log_w, Emit emit, int max_entries = 0x7FFFFFFF,
-                                           int* consumed = nullptr) {
+                                           int log_w, Emit emit) {
     // Four columns (and values) of every row are held in registers and refilled with one
     // 16-byte load: a row starts at a multiple of its width (>= 8 slots), so the loads are
     // aligned, and the chain of dependent loads is a quarter as long.
@@ -720,7 +719,7 @@ __device__ __forceinline__ int merge_group(const int32_t* __restrict__ cols, con
 #pragma unroll
     for (int r = 0; r < kGroupRows; ++r) {
         const long long e = g * kGroupRows + r;
-        len[r] = e < n_rows ? min(meta[e] & (int)kMetaLenMask, 1 << log_w) : 0;      // (meta words may not be checked yet)
+        len[r] = e < n_rows ? (meta[e] & (int)kMetaLenMask) : 0;
         base[r] = e << log_w;
         pos[r] = 0;
         cbuf[r] = make_int4(0, 0, 0, 0);
@@ -758,9 +757,8 @@ __device__ __forceinline__ int merge_group(const int32_t* __restrict__ cols, con
             }
         }
         if (kEmit) emit(m, cmin, v, mask);
-        if (++m >= max_entries) break;
+        ++m;
     }
-    if (consumed) *consumed = pos[0] + pos[1] + pos[2] + pos[3];
     return m;
 }
 
@@ -776,8 +774,7 @@ struct RowGroupCand {
 };
 
 // One atomic per wavefront and counter: [0] sum of m, [1] sum of plain, [2] largest m.
-__device__ __forceinline__ void add_rowgroup_counters(int m, int plain, unsigned long long* __restrict__ c) {
-    int sm = m, sp = plain, mx = m;
+__device__ __forceinline__ void add_rowgroup_counters(int sm, int sp, int mx, unsigned long long* __restrict__ c) {
     for (int d = 32; d > 0; d >>= 1) {
         sm += __shfl_xor(sm, d);
         sp += __shfl_xor(sp, d);
@@ -805,7 +802,7 @@ rowgroup_count_kernel(const RowGroupCand* __restrict__ cands, unsigned long long
         }
         cd.m_out[g] = m;
     }
-    add_rowgroup_counters(m, plain, counters + 3 * blockIdx.y);
+    add_rowgroup_counters(m, plain, m, counters + 3 * blockIdx.y);
 }
 
 __global__ void __launch_bounds__(256)
@@ -1023,10 +1020,13 @@ struct ChunkedRow {
     int found;           // 1 part of a split row, 2 dense row, 4 more than kWideFinalPartials chunks
 };
 
-__device__ __forceinline__ ChunkedRow chunked_row(const int32_t* __restrict__ meta, long long e, long long n_rows,
-                                                  int log_w, int coop_slots, int chunk_slots, long long dense_min_slots) {
+// Row e of a bucket, whose meta word is m; tail: the meta word at tail_of(m, e, n_rows).
+__device__ __forceinline__ long long tail_of(int m, long long e, long long n_rows) {
+    return m < 0 ? e : min(max(e + (int)((uint32_t)m >> kMetaLenBits) - 1, e), n_rows - 1);
+}
+__device__ __forceinline__ ChunkedRow chunked_row(int m, int tail, long long e, long long n_rows, int log_w, int coop_slots, int chunk_slots,
+                                                  long long dense_min_slots) {
     ChunkedRow x{0, 0, chunk_slots, 0};
-    const int m = meta[e];
     if (m < 0) {
         x.found = 1;
         return x;
@@ -1037,7 +1037,7 @@ __device__ __forceinline__ ChunkedRow chunked_row(const int32_t* __restrict__ me
     // read: a head that announces more ELL rows than the bucket holds (which the checks flag and
     // the plan is then refused) must not be followed past the array.
     if (((long long)seg << log_w) > coop_slots && e + seg <= n_rows) {
-        x.total = ((long long)(seg - 1) << log_w) + (meta[e + seg - 1] & (int)kMetaLenMask);
+        x.total = ((long long)(seg - 1) << log_w) + (tail & (int)kMetaLenMask);
         if (x.total >= dense_min_slots) {
             x.chunk_slots = kDenseChunkSlots;
             x.found |= 2;
@@ -1077,20 +1077,23 @@ struct PlanBucket {
 //     where one is a part of a row, which says nothing);
 //   * marks the rows that partition 0 writes;
 //   * samples the row-group candidates: of every sample_stride-th group of four rows, samples[3 k ..] = merged entries among the
-//     first kRowGroupSampleEntries, the slots they consumed, the largest count.  By workgroups of their own, which start first:
-//     chains of loads that a launch behind this one waited 20 to 26 us for.  (Nothing here is followed out of the slabs, whatever
-//     the meta words say; where a check fails the samples are not read.)
+//     first kRowGroupSampleEntries, the slots they consumed, the largest count.  By workgroups of their own, which start first
+//     and stage the first slots of their rows in LDS (merged out of memory, a group to a lane, each step waited for a load: 19 us of
+//     the 21 that the scan of a 170K-row graph took, now 10 of 13; 115 behind the stream of a large one, now 20).  (Nothing here is
+//     followed out of the slabs, whatever the meta words say; where a check fails the samples are not read.)
 // Bound by the stream of the column slabs.  Workgroup -> bucket by the first workgroups of the
 // buckets, so that all of them share one launch however many there are: three launches per bucket
 // (checks, counts, marks) were 60 us of GPU time for the 11 buckets of a 170K-row graph, whose slabs
 // take 3 us to read, and each read the row ids or the meta words again.  Together the workgroups fill the GPU once: 1024 to a
-// bucket left a second, nearly empty round of them.  2.45M-row graph, widths 1 .. 32, behind the builder: 147 + 26 us with the samples, now 131
-// (its slabs at 3.5 TB/s; 107 us where nothing was written just before).
-constexpr int kScanSlotsPerBlock = 16384;  // at least
+// bucket left a second, nearly empty round of them.  No load is behind a condition, where it would wait for the one before.
+// 2.45M-row graph, widths 1 .. 32, behind the builder: 147 + 26 us with the samples, now 123, of which 60 take its slabs at 5.7 TB/s
+// and as many the rows.
+constexpr int kScanSlotsPerBlock = 16384, kScanRowsPerBlock = 1024;  // at least
 constexpr int kScanBlocksPerCu = 7;
 constexpr int kScanRows = 4;               // ELL rows of a thread requested together
 constexpr int kScanUnroll = 4;             // 16-byte loads of columns in flight per thread
 constexpr int kScanCounters = 7, kScanFound = 5, kScanSpan = 6;
+constexpr int kSampleGroups = 64, kSampleRound = 32;       // of a workgroup, and staged together
 constexpr int kSpanUnits = 4096, kSpanSamples = 1024;      // (twice the samples at most: sums below 2^24)
 // Atomics on one line are taken one after the other, 17 to 40 ns each, and the workgroups of a bucket end together: up to 16
 // lines share them.
@@ -1111,15 +1114,60 @@ plan_scan_kernel(const PlanBucket* __restrict__ buckets, const int32_t* __restri
     const long long stride = (long long)bk.n_blocks * 256;
     const int place = (int)blockIdx.x - first_block[k];
     const long long t0 = ((long long)place - bk.n_first) * 256 + threadIdx.x;
-    const int32_t *rows = bk.rows, *meta = bk.meta;
+    // (pointers out of a table are generic to the compiler: flat loads, which wait for the LDS counter too)
+    typedef const int32_t __attribute__((address_space(1)))* GlobalInts;
+    typedef int Four __attribute__((ext_vector_type(4), aligned(4)));
+    typedef const Four __attribute__((address_space(1)))* GlobalFours;
+    const GlobalInts rows = (GlobalInts)(uintptr_t)bk.rows, meta = (GlobalInts)(uintptr_t)bk.meta, cols = (GlobalInts)(uintptr_t)bk.cols;
     const int log_w = bk.log_w;
     const long long n_rows = bk.n_rows;
     if (place > 0 && place < bk.n_first) {                    // samples
-        const long long g = ((long long)(place - 1) * 256 + threadIdx.x) * bk.sample_stride;
-        int m = 0, plain = 0;
-        if (g * kGroupRows < n_rows)
-            m = merge_group<false>(bk.cols, nullptr, meta, g, n_rows, log_w, [](int, int, const float*, uint32_t) {}, kRowGroupSampleEntries, &plain);
-        add_rowgroup_counters(m, plain, samples + 3 * k);
+        constexpr int kSlots = kRowGroupSampleEntries, kFours = kSlots / 4, kLine = kGroupRows * kSlots + 1;      // slots of a row that are looked at
+        __shared__ int s_cols[kSampleRound][kLine];
+        __shared__ int s_len[kSampleRound][kGroupRows];
+        const int width = 1 << log_w;
+        int merged = 0, plain = 0, most = 0;
+        for (int g0 = 0; g0 < kSampleGroups; g0 += kSampleRound) {
+            auto row_at = [&](int g, int r) { return ((long long)(place - 1) * kSampleGroups + g0 + g) * bk.sample_stride * kGroupRows + r; };
+            Four c[kSampleRound * kGroupRows * kFours / 256];
+#pragma unroll
+            for (int t = 0; t < kSampleRound * kGroupRows * kFours / 256; ++t) {
+                const int i = t * 256 + threadIdx.x, q = i % kFours, r = i / kFours % kGroupRows, g = i / (kFours * kGroupRows);
+                c[t] = *(GlobalFours)(cols + (min(row_at(g, r), n_rows - 1) << log_w) + min(q * 4, width - 4));
+            }
+            if (threadIdx.x < kSampleRound * kGroupRows) {
+                const int r = threadIdx.x % kGroupRows, g = threadIdx.x / kGroupRows;
+                const int m = meta[min(row_at(g, r), n_rows - 1)];
+                s_len[g][r] = row_at(g, r) < n_rows ? min(m & (int)kMetaLenMask, width) : 0;      // (not checked yet)
+            }
+#pragma unroll
+            for (int t = 0; t < kSampleRound * kGroupRows * kFours / 256; ++t) {
+                const int i = t * 256 + threadIdx.x, q = i % kFours, r = i / kFours % kGroupRows, g = i / (kFours * kGroupRows);
+                int* to = &s_cols[g][r * kSlots + q * 4];
+                to[0] = c[t].x, to[1] = c[t].y, to[2] = c[t].z, to[3] = c[t].w;
+            }
+            __syncthreads();
+            if (threadIdx.x < kSampleRound) {
+                const int g = threadIdx.x;
+                int pos[kGroupRows] = {}, head[kGroupRows], m = 0;
+                for (; m < kRowGroupSampleEntries; ++m) {
+                    int least = 0x7FFFFFFF;
+#pragma unroll
+                    for (int r = 0; r < kGroupRows; ++r) {
+                        head[r] = pos[r] < s_len[g][r] ? s_cols[g][r * kSlots + pos[r]] : 0x7FFFFFFF;
+                        least = min(least, head[r]);
+                    }
+                    if (least == 0x7FFFFFFF) break;
+#pragma unroll
+                    for (int r = 0; r < kGroupRows; ++r) pos[r] += head[r] == least;
+                }
+                plain += pos[0] + pos[1] + pos[2] + pos[3];
+                merged += m;
+                most = max(most, m);
+            }
+            __syncthreads();
+        }
+        if (threadIdx.x < 64) add_rowgroup_counters(merged, plain, most, samples + 3 * k);
         return;
     }
     if (place == 0) {                                         // span
@@ -1132,8 +1180,8 @@ plan_scan_kernel(const PlanBucket* __restrict__ buckets, const int32_t* __restri
                 const long long q = min(e + r, n_rows - 1), at = q << log_w;
                 const int m = meta[q], n = min(max(m & (int)kMetaLenMask, 1), 1 << log_w);       // (not checked yet)
                 whole = whole && m >> kMetaLenBits == 1;
-                first = min(first, bk.cols[at]);
-                last = max(last, bk.cols[at + n - 1]);
+                first = min(first, cols[at]);
+                last = max(last, cols[at + n - 1]);
             }
             const long long columns = whole ? max((long long)last - first, 0ll) : bk.all_cols;
             span += (int)min((long long)kSpanUnits, columns * kSpanUnits / bk.all_cols);
@@ -1146,19 +1194,18 @@ plan_scan_kernel(const PlanBucket* __restrict__ buckets, const int32_t* __restri
     const long long n_slots = n_rows << log_w;
     const unsigned limit = (unsigned)num_cols;               // < 2^31
     const long long round = stride * 4 * kScanUnroll;       // from the end: what the builder wrote last may still be in the memory-side cache (143 -> 131 us)
-    for (long long i = t0 * 4 + (n_slots - 1) / round * round; i >= 0; i -= round) {
-        int4 c[kScanUnroll];
+    if (n_slots < 4) {
+        if (t0 < n_slots) bad_col = (unsigned)cols[t0] >= limit;
+    } else {
+        for (long long i = t0 * 4 + (n_slots - 1) / round * round; i >= 0; i -= round) {
+            Four c[kScanUnroll];
 #pragma unroll
-        for (int u = 0; u < kScanUnroll; ++u) {
-            const long long j = i + u * stride * 4;
-            c[u] = make_int4(0, 0, 0, 0);
-            if (j + 4 <= n_slots) c[u] = *reinterpret_cast<const int4*>(bk.cols + j);
-            else if (j < n_slots)
-                for (long long q = j; q < n_slots; ++q) bad_col |= (unsigned)bk.cols[q] >= limit;
+            for (int u = 0; u < kScanUnroll; ++u)                // (no load behind a condition: they would wait for one another)
+                c[u] = *(GlobalFours)(cols + min(i + u * stride * 4, n_slots - 4));
+#pragma unroll
+            for (int u = 0; u < kScanUnroll; ++u)
+                bad_col |= (unsigned)c[u].x >= limit || (unsigned)c[u].y >= limit || (unsigned)c[u].z >= limit || (unsigned)c[u].w >= limit;
         }
-#pragma unroll
-        for (int u = 0; u < kScanUnroll; ++u)
-            bad_col |= (unsigned)c[u].x >= limit || (unsigned)c[u].y >= limit || (unsigned)c[u].z >= limit || (unsigned)c[u].w >= limit;
     }
     constexpr int kSums = kScanFound;
     int sum[kSums] = {}, found = 0;
@@ -1170,6 +1217,14 @@ plan_scan_kernel(const PlanBucket* __restrict__ buckets, const int32_t* __restri
             row_of[u] = rows[e];
             meta_of[u] = meta[e];
             next_of[u] = meta[min(e + 1, n_rows - 1)];
+        }
+        int there_meta[kScanRows], there_row[kScanRows];      // of a segment's head its last ELL row, of the others the head
+#pragma unroll
+        for (int u = 0; u < kScanRows; ++u) {
+            const long long e = min(e0 + u * stride, n_rows - 1), back = (long long)(((uint32_t)meta_of[u] & 0x7FFFFFFFu) >> kMetaLenBits);
+            const long long there = meta_of[u] < 0 ? max(e - back, 0ll) : tail_of(meta_of[u], e, n_rows);
+            there_meta[u] = meta[there];
+            there_row[u] = rows[there];
         }
 #pragma unroll
     for (int u = 0; u < kScanRows; ++u) {
@@ -1193,9 +1248,9 @@ plan_scan_kernel(const PlanBucket* __restrict__ buckets, const int32_t* __restri
             if (field < 1 || h < 0) {
                 bad_meta = true;
             } else {
-                const int hm = meta[h];
+                const int hm = there_meta[u];
                 const long long n = (long long)((uint32_t)hm >> kMetaLenBits);
-                bad_meta |= hm < 0 || field >= n || rows[h] != row;
+                bad_meta |= hm < 0 || field >= n || there_row[u] != row;
                 want = field + 1 < n ? field + 1 : 0;
             }
         }
@@ -1207,7 +1262,7 @@ plan_scan_kernel(const PlanBucket* __restrict__ buckets, const int32_t* __restri
         } else {
             bad_meta |= want != 0;
         }
-        const ChunkedRow x = chunked_row(meta, e, n_rows, log_w, kCoopSlots, chunk_slots, dense_min_slots);
+        const ChunkedRow x = chunked_row(m, there_meta[u], e, n_rows, log_w, kCoopSlots, chunk_slots, dense_min_slots);
         found |= x.found;
         sum[0] += x.n_chunks;
         sum[1] += x.n_chunks > 1;
@@ -1275,12 +1330,17 @@ plan_chunks_kernel(ChunkBuckets buckets, HeavyRow* __restrict__ heavy, int n_hea
     const int log_w = b.log_w;
     const long long e0 = ((long long)blockIdx.x - b.first_block) * kChunkRows + threadIdx.x;
     ChunkedRow x[kChunkRowsOfThread];
+    int m[kChunkRowsOfThread], tail[kChunkRowsOfThread];
+#pragma unroll
+    for (int u = 0; u < kChunkRowsOfThread; ++u) m[u] = b.meta[min(e0 + u * kChunkThreads, b.n_rows - 1)];
+#pragma unroll
+    for (int u = 0; u < kChunkRowsOfThread; ++u) tail[u] = b.meta[tail_of(m[u], min(e0 + u * kChunkThreads, b.n_rows - 1), b.n_rows)];
     int mine[3] = {0, 0, 0};                 // chunks, rows with several, their partial rows
 #pragma unroll
     for (int u = 0; u < kChunkRowsOfThread; ++u) {
         const long long e = e0 + u * kChunkThreads;
         x[u] = ChunkedRow{0, 0, chunk_slots, 0};
-        if (e < b.n_rows) x[u] = chunked_row(b.meta, e, b.n_rows, log_w, coop_slots, chunk_slots, dense_min_slots);
+        if (e < b.n_rows) x[u] = chunked_row(m[u], tail[u], e, b.n_rows, log_w, coop_slots, chunk_slots, dense_min_slots);
         mine[0] += x[u].n_chunks;
         mine[1] += x[u].n_chunks > 1;
         mine[2] += x[u].n_chunks > 1 ? x[u].n_chunks : 0;
@@ -1609,9 +1669,9 @@ int lf_spmm_create(lf_spmm_plan** out_plan, const lf_bucket_desc* h_buckets, int
     // Scratch: the words that are read back (chunk counters and fill cursors of every bucket, sampling
     // counters, flags), then the coverage bytes - cleared by one launch - then the bucket table.
     const size_t nb_s = (size_t)num_buckets;
-    long long scan_units = 0;                              // of kScanSlotsPerBlock slots, or 1024 rows
+    long long scan_units = 0;                              // of kScanSlotsPerBlock slots or kScanRowsPerBlock rows
     auto units_of = [](const lf_bucket_desc& b) {
-        return std::max<long long>(lf::ceil_div(b.num_ell_rows, (int64_t)1024), lf::ceil_div(b.num_ell_rows * b.width, (int64_t)kScanSlotsPerBlock));
+        return std::max<long long>(lf::ceil_div(b.num_ell_rows, (int64_t)kScanRowsPerBlock), lf::ceil_div(b.num_ell_rows * b.width, (int64_t)kScanSlotsPerBlock));
     };
     for (int k = 0; k < num_buckets; ++k) scan_units += units_of(h_buckets[k]);
     const long long units_per_block = std::max<long long>(1, lf::ceil_div(scan_units, (int64_t)kScanBlocksPerCu * plan->num_cus));
@@ -1679,7 +1739,7 @@ int lf_spmm_create(lf_spmm_plan** out_plan, const lf_bucket_desc* h_buckets, int
         if (ch == 1 && !(env_groups && env_groups[0] == '0') && b.num_ell_rows >= kRowGroupMinRows && b.width >= kUnroll && b.width <= 64) {
             const long long n_groups = lf::ceil_div(b.num_ell_rows, kGroupRows);
             t.sample_stride = (int)std::max<long long>(1, n_groups / kRowGroupSample);
-            t.n_first += (int)lf::ceil_div(lf::ceil_div(n_groups, (long long)t.sample_stride), 256ll);
+            t.n_first += (int)lf::ceil_div(lf::ceil_div(n_groups, (long long)t.sample_stride), (long long)kSampleGroups);
             cand.push_back(k);
         }
         h_first[k] = scan_blocks;
