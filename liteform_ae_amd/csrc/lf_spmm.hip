@@ -826,7 +826,11 @@ __global__ void __launch_bounds__(kWG)
 spmm_rowgroup_kernel(const MergedBucket* __restrict__ buckets, int n_buckets, LaunchArgs a) {
     constexpr int VEC = Dense<BT>::kVec;
     constexpr int SW = kWG / LPR;
-    constexpr int U = VEC == 4 ? 8 : 4;          // gathers in flight per sub-wave
+    // Gathers of a sub-wave, and staged entries of a thread, requested together.  27-point stencils, N = 128 .. 256 bf16, 4 and 8 gathers: 30.6,
+    // 28.8 us (38 x 71 x 22), 31.3, 29.1 (34 x 40 x 45); N = 448, where a sub-wave is a wavefront and skips rows: 111, 120.  Entries by 1, 2, 4:
+    // N = 448 111, 107, 100; N = 128 30.6, 29.7, 30.2; f32 N = 224 32.4, 31.7, 32.1.
+    constexpr bool kWideRow = VEC == 8 && LPR == 64;
+    constexpr int U = kWideRow ? 4 : 8, kStage = kWideRow ? 4 : 2;
     __shared__ float4 s_val[kMergedCap];
     __shared__ int s_col[kMergedCap];
     __shared__ int s_goff[kMergedTileGroups + 1];
@@ -842,7 +846,13 @@ spmm_rowgroup_kernel(const MergedBucket* __restrict__ buckets, int n_buckets, La
         const long long g0 = (lo + v) * b.groups_per_tile;
         const int n = (int)min((long long)b.groups_per_tile, b.n_groups - g0);
         const int tid = threadIdx.x;
-        for (int i = tid; i <= n; i += kWG) s_goff[i] = b.goff[g0 + i];
+        // (pointers out of a table are generic to the compiler: flat loads, which wait for the LDS counter too)
+        typedef const int32_t __attribute__((address_space(1)))* GlobalInts;
+        typedef float Four __attribute__((ext_vector_type(4)));
+        const GlobalInts goff = (GlobalInts)(uintptr_t)b.goff, ecol = (GlobalInts)(uintptr_t)b.ecol, rows = (GlobalInts)(uintptr_t)b.rows;
+        const auto eval = (const Four __attribute__((address_space(1)))*)(uintptr_t)b.eval;
+        const auto emask = (const uint8_t __attribute__((address_space(1)))*)(uintptr_t)b.emask;
+        for (int i = tid; i <= n; i += kWG) s_goff[i] = goff[g0 + i];
         __syncthreads();
         const int sw = tid / LPR, sl = tid % LPR;
         const Lane<LPR, 1, VEC> ln(sl, a.feat, a.ldb, a.ldc);
@@ -853,10 +863,24 @@ spmm_rowgroup_kernel(const MergedBucket* __restrict__ buckets, int n_buckets, La
             int gb = ga + 1;
             while (gb < n && s_goff[gb + 1] - base <= kMergedCap) ++gb;      // uniform
             const int n_entries = s_goff[gb] - base;
-            for (int i = tid; i < n_entries; i += kWG) {
-                s_col[i] = b.ecol[base + i];
-                s_val[i] = b.eval[base + i];
-                s_msk[i] = b.emask[base + i];
+            for (int i0 = tid; i0 < n_entries; i0 += kStage * kWG) {
+                Four v[kStage];
+                int c[kStage];
+                uint8_t k[kStage];
+#pragma unroll
+                for (int u = 0; u < kStage; ++u) {
+                    const int i = base + min(i0 + u * kWG, n_entries - 1);
+                    v[u] = eval[i];
+                    c[u] = ecol[i];
+                    k[u] = emask[i];
+                }
+#pragma unroll
+                for (int u = 0; u < kStage; ++u) {
+                    const int i = min(i0 + u * kWG, n_entries - 1);
+                    s_col[i] = c[u];
+                    s_val[i] = make_float4(v[u].x, v[u].y, v[u].z, v[u].w);
+                    s_msk[i] = k[u];
+                }
             }
             __syncthreads();
             for (int gi = ga + sw; gi < gb; gi += SW) {
@@ -905,7 +929,7 @@ spmm_rowgroup_kernel(const MergedBucket* __restrict__ buckets, int n_buckets, La
 #pragma unroll
                 for (int r = 0; r < kGroupRows; ++r) {
                     const long long e = (g0 + gi) * kGroupRows + r;
-                    if (e < b.n_rows) store_row<LPR, 1, VEC>(a.C, b.rows[e], ln, acc[r], a.accumulate);
+                    if (e < b.n_rows) store_row<LPR, 1, VEC>(a.C, rows[e], ln, acc[r], a.accumulate);
                 }
             }
             ga = gb;
