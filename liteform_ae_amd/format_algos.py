@@ -86,6 +86,7 @@ _STAGE_LARGE = 64 << 20
 _STAGE_SHAPES = {False: (2 << 20, 6), True: (16 << 20, 3)}
 _stages = {}
 _stage_lock = threading.Lock()
+_long_rows_lock = threading.Lock()
 _TORCH_TYPES = ("bool", "uint8", "int8", "int16", "int32", "int64", "float16", "float32", "float64")
 
 
@@ -218,7 +219,6 @@ class _DeviceCSR:
         self._longest = None         # entries of the longest row, where the arrays were checked
         self._long_rows = None       # list of long rows and its counts, see csr_work
         self._csr_work = {}
-        self._csr_lock = threading.Lock()
         src = getattr(g, "_csr_source", None)
         if src is not None and self._from_csr(src, bool(getattr(g, "_unit_values", False))):
             self.path = "csr"
@@ -300,10 +300,10 @@ class _DeviceCSR:
         self.all_ones = ones and self.nnz == self.coo_nnz
 
     def csr_work(self, feat: int, dtype: int):
-        """What the C call of a CSR product takes: ((rows, columns, entries, span), address of the list of long rows, address of
-        its counts, bytes of work space).  The list
-        (lf_csr_long_rows) is made for the first product that wants it and kept with the matrix; a product that is recorded into
-        a graph before there is one does without."""
+        """What the C call of a CSR product takes: ((rows, columns, entries, span), list of long rows, its counts, bytes of work
+        space).  The list (lf_csr_long_rows) is made for the first product that wants it and kept with the matrix; a product
+        that is recorded into a graph before there is one does without.  (Tensor and array, no addresses: the matrix may be
+        copied with what it holds.)"""
         work = self._csr_work.get((feat, dtype))
         if work is None:
             lib = _lib.load()
@@ -316,16 +316,16 @@ class _DeviceCSR:
             if not keep:
                 rows, counts = self._long_row_list()
                 keep = self._long_rows is not None
-                nbytes = lib.lf_csr_spmm_work_bytes(*sizes, counts, 0, feat, dtype)
+                nbytes = lib.lf_csr_spmm_work_bytes(*sizes, _lib.ptr(counts), 0, feat, dtype)
             work = (sizes, rows, counts, nbytes)
             if keep:
                 self._csr_work[(feat, dtype)] = work
         return work
 
     def _long_row_list(self):
-        """Addresses of the list of long rows and of its counts; None where there are no such rows, or no list yet and the
-        stream is being recorded."""
-        with self._csr_lock:
+        """The list of long rows and its counts; None where there are no such rows, or no list yet and the stream is being
+        recorded."""
+        with _long_rows_lock:
             if self._long_rows is None and not _torch().cuda.is_current_stream_capturing():
                 lib = _lib.load()
                 rows = _gpu_torch.empty(lib.lf_csr_long_rows_bytes(self.nnz), dtype=_gpu_torch.uint8, device="cuda")
@@ -333,8 +333,7 @@ class _DeviceCSR:
                 _lib.check(lib.lf_csr_long_rows(self.indptr.data_ptr(), self.num_rows, self.nnz, rows.data_ptr(), rows.numel(),
                                                 _lib.np_ptr(counts, C.c_int64), _stream()))
                 self._long_rows = (rows, counts) if counts[0] else (None, None)
-            rows, counts = self._long_rows or (None, None)
-        return (None, None) if rows is None else (rows.data_ptr(), _lib.np_ptr(counts, C.c_int64))
+            return self._long_rows or (None, None)
 
     def seg_deg(self, num_parts: int):
         """Per-(partition,row) COO degrees on the device, or None when CSR lengths are the same."""
@@ -706,7 +705,8 @@ def spmm_csr(g, B, b_dtype: str = "f32", use_values: bool = True):
     if nbytes:
         work = torch.empty(nbytes, dtype=torch.uint8, device="cuda")
         rc = lib.lf_csr_spmm_trusted_work(dev.indptr.data_ptr(), dev.indices.data_ptr(), None if vals is None else vals.data_ptr(), *sizes,
-                                          rows, counts, work.data_ptr(), nbytes, feat, dtype, B.data_ptr(), out.data_ptr(), _stream())
+                                          _lib.ptr(rows), _lib.ptr(counts), work.data_ptr(), nbytes, feat, dtype, B.data_ptr(),
+                                          out.data_ptr(), _stream())
     else:
         rc = lib.lf_csr_spmm_trusted_span(dev.indptr.data_ptr(), dev.indices.data_ptr(), None if vals is None else vals.data_ptr(), *sizes,
                                           feat, dtype, B.data_ptr(), out.data_ptr(), _stream())

@@ -1,6 +1,8 @@
 """CSR products in panels of columns and with long rows in chunks, against scipy in float64.
 
 Tolerance: |C - ref| <= 1e-5 * sum|a||b|, the bound of every product of this package."""
+import copy
+
 import numpy as np
 import pytest
 
@@ -92,6 +94,8 @@ def test_long_rows_in_chunks(fa, torch, feat, b_dtype):
     ref = O.spmm_csr_f64(indptr, indices, values, (len(lens), cols), Bh)
     bound = 1e-5 * O.spmm_abs_bound(indptr, indices, values, (len(lens), cols), Bh)
     assert (np.abs(got.cpu().numpy() - ref) <= bound).all()
+    twin = copy.deepcopy(g)                                    # with its own list of long rows
+    assert torch.equal(got, fa.spmm_csr(twin, B, b_dtype))
     fresh = MTX.from_csr(indptr, indices, (len(lens), cols), data=values)
     fa._device_csr(fresh)                                      # on the GPU, but without a product yet
     for m in (g, fresh):
