@@ -18,6 +18,7 @@ LF_ERR_HIP = -3
 LF_ERR_CONFIG = -4
 LF_ERR_UNSUPPORTED = -5
 LF_ERR_WORKSPACE = -6
+LF_WANTS_WORK = 1
 
 LF_MAX_CLASSES = 11
 LF_STATS_FIELDS = 4
@@ -89,6 +90,7 @@ SIGNATURES = {
     "lf_csr_spmm_work_bytes": (C.c_int64, [C.c_int64, C.c_int64, C.c_int64, C.c_int64, i64p, C.c_int64, C.c_int32, C.c_int32]),
     "lf_csr_spmm_trusted_work": (C.c_int, [vp, vp, vp, C.c_int64, C.c_int64, C.c_int64, C.c_int64, vp, i64p, vp, C.c_size_t, C.c_int32, C.c_int32, vp,
                                            vp, vp]),
+    "lf_csr_spmm_trusted_rows": (C.c_int, [vp, vp, vp, C.c_int64, C.c_int64, C.c_int64, C.c_int64, C.c_int64, C.c_int32, C.c_int32, vp, vp, vp]),
     "lf_coo_to_csr_workspace_bytes": (C.c_size_t, [C.c_int64, C.c_int64, C.c_int64]),
     "lf_coo_to_csr": (C.c_int, [vp, vp, vp, C.c_int64, C.c_int64, C.c_int64, vp, C.c_size_t, vp, vp, vp, i64p, vp]),
     "lf_bsr_spmm": (C.c_int, [vp, vp, vp, C.c_int64, C.c_int64, C.c_int64, C.c_int32, C.c_int32, vp, vp, vp, vp]),

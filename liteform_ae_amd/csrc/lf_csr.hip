@@ -394,11 +394,14 @@ int64_t lf_csr_spmm_work_bytes(int64_t num_rows, int64_t num_cols, int64_t nnz, 
     return (int64_t)work_bytes_of(shape, num_rows, feat_size);
 }
 
-int lf_csr_spmm_trusted_work(const int32_t* d_indptr, const int32_t* d_indices, const float* d_values,
-                             int64_t num_rows, int64_t num_cols, int64_t nnz, int64_t span, const void* d_list, const int64_t* h_counts,
-                             void* d_work, size_t work_bytes, int32_t feat_size,
-                             int32_t b_dtype, const void* d_B, float* d_C, lf_stream_t stream) {
-    hipStream_t s = (hipStream_t)stream;
+}  // extern "C"
+
+namespace {
+
+// (longest: see lf_csr_spmm_trusted_rows; negative: the product takes what it is given)
+int csr_product(const int32_t* d_indptr, const int32_t* d_indices, const float* d_values, int64_t num_rows, int64_t num_cols, int64_t nnz,
+                int64_t span, int64_t longest, const void* d_list, const int64_t* h_counts, void* d_work, size_t work_bytes, int32_t feat_size,
+                int32_t b_dtype, const void* d_B, float* d_C, hipStream_t s) {
     LF_REQUIRE(num_rows >= 0 && num_rows < (1ll << 31) && num_cols >= 1, LF_ERR_INVALID, "bad shape");
     if (num_rows == 0) return LF_OK;
     LF_REQUIRE(d_indptr && d_B && d_C, LF_ERR_INVALID, "null argument");
@@ -407,7 +410,11 @@ int lf_csr_spmm_trusted_work(const int32_t* d_indptr, const int32_t* d_indices, 
                "B, C and the work space must be 16-byte aligned");
     int lpr, ch;
     if (int rc = feature_shape(feat_size, b_dtype, &lpr, &ch)) return rc;
-    const CsrShape shape = csr_shape(num_rows, num_cols, nnz, span, feat_size, b_dtype, d_work && d_list ? h_counts : nullptr, d_work != nullptr);
+    const bool ask = longest >= 0;
+    const int64_t guess[3] = {longest > kCsrChunkedRow ? 1 : 0, 1, longest};
+    const CsrShape shape = csr_shape(num_rows, num_cols, nnz, span, feat_size, b_dtype, ask ? guess : d_work && d_list ? h_counts : nullptr,
+                                     ask || d_work != nullptr);
+    if (ask && work_bytes_of(shape, num_rows, feat_size) > 0) return LF_WANTS_WORK;
     const int64_t n_chunks = shape.n_chunks;
     LF_REQUIRE(!d_work || work_bytes >= work_bytes_of(shape, num_rows, feat_size), LF_ERR_INVALID, "the product needs %zu bytes of work space",
                work_bytes_of(shape, num_rows, feat_size));
@@ -458,11 +465,31 @@ int lf_csr_spmm_trusted_work(const int32_t* d_indptr, const int32_t* d_indices, 
     return LF_OK;
 }
 
+}  // namespace
+
+extern "C" {
+
+int lf_csr_spmm_trusted_work(const int32_t* d_indptr, const int32_t* d_indices, const float* d_values,
+                             int64_t num_rows, int64_t num_cols, int64_t nnz, int64_t span, const void* d_list, const int64_t* h_counts,
+                             void* d_work, size_t work_bytes, int32_t feat_size,
+                             int32_t b_dtype, const void* d_B, float* d_C, lf_stream_t stream) {
+    return csr_product(d_indptr, d_indices, d_values, num_rows, num_cols, nnz, span, -1, d_list, h_counts, d_work, work_bytes, feat_size, b_dtype,
+                       d_B, d_C, (hipStream_t)stream);
+}
+
+int lf_csr_spmm_trusted_rows(const int32_t* d_indptr, const int32_t* d_indices, const float* d_values,
+                             int64_t num_rows, int64_t num_cols, int64_t nnz, int64_t span, int64_t longest, int32_t feat_size,
+                             int32_t b_dtype, const void* d_B, float* d_C, lf_stream_t stream) {
+    LF_REQUIRE(longest >= 0, LF_ERR_INVALID, "bad length of the longest row");
+    return csr_product(d_indptr, d_indices, d_values, num_rows, num_cols, nnz, span, longest, nullptr, nullptr, nullptr, 0, feat_size, b_dtype, d_B, d_C,
+                       (hipStream_t)stream);
+}
+
 int lf_csr_spmm_trusted_span(const int32_t* d_indptr, const int32_t* d_indices, const float* d_values,
                              int64_t num_rows, int64_t num_cols, int64_t nnz, int64_t span, int32_t feat_size,
                              int32_t b_dtype, const void* d_B, float* d_C, lf_stream_t stream) {
-    return lf_csr_spmm_trusted_work(d_indptr, d_indices, d_values, num_rows, num_cols, nnz, span, nullptr, nullptr, nullptr, 0, feat_size, b_dtype, d_B,
-                                    d_C, stream);
+    return csr_product(d_indptr, d_indices, d_values, num_rows, num_cols, nnz, span, -1, nullptr, nullptr, nullptr, 0, feat_size, b_dtype, d_B, d_C,
+                       (hipStream_t)stream);
 }
 
 int lf_csr_spmm_trusted_nnz(const int32_t* d_indptr, const int32_t* d_indices, const float* d_values,

@@ -700,8 +700,17 @@ def spmm_csr(g, B, b_dtype: str = "f32", use_values: bool = True):
     feat, dtype = int(B.shape[1]), _B_DTYPES[b_dtype]
     out = dev.indptr.new_empty((dev.num_rows, feat), dtype=torch.float32)
     vals = dev.values if use_values else None
-    sizes, rows, counts, nbytes = dev._csr_work.get((feat, dtype)) or dev.csr_work(feat, dtype)
+    work = dev._csr_work.get((feat, dtype))
     # the device arrays were made by lf_coo_to_csr or have passed lf_csr_check: no second check
+    if work is None and dev._longest is not None and dev._long_rows is None:
+        sizes = (dev.num_rows, dev.num_cols, dev.nnz, dev.span)
+        rc = lib.lf_csr_spmm_trusted_rows(dev.indptr.data_ptr(), dev.indices.data_ptr(), None if vals is None else vals.data_ptr(), *sizes,
+                                          dev._longest, feat, dtype, B.data_ptr(), out.data_ptr(), _stream())
+        if rc != _lib.LF_WANTS_WORK:
+            _lib.check(rc)
+            dev._csr_work[(feat, dtype)] = (sizes, None, None, 0)
+            return out
+    sizes, rows, counts, nbytes = work or dev.csr_work(feat, dtype)
     if nbytes:
         work = torch.empty(nbytes, dtype=torch.uint8, device="cuda")
         rc = lib.lf_csr_spmm_trusted_work(dev.indptr.data_ptr(), dev.indices.data_ptr(), None if vals is None else vals.data_ptr(), *sizes,
