@@ -357,7 +357,8 @@ int lf_csr_spmm_trusted_nnz(const int32_t* d_indptr, const int32_t* d_indices, c
 int lf_csr_spmm_trusted_span(const int32_t* d_indptr, const int32_t* d_indices, const float* d_values,
                              int64_t num_rows, int64_t num_cols, int64_t nnz, int64_t span, int32_t feat_size,
                              int32_t b_dtype, const void* d_B, float* d_C, lf_stream_t stream);
-/* lf_csr_spmm_trusted_work may also cut a dense matrix into panels of columns, and long rows into chunks.  Both need work
+/* lf_csr_spmm_trusted_work may also cut a dense matrix into panels of columns, and long rows into chunks.  The panels are found by
+ * bisection: the columns of a row must ascend (LF_CSR_CANONICAL, or the result of lf_coo_to_csr).  Both need work
  * space: lf_csr_spmm_work_bytes bytes of device memory, 16-byte aligned, that no other product uses meanwhile (none: d_work
  * NULL, and the product is that of lf_csr_spmm_trusted_span).  The chunks are those of lf_csr_long_rows, which fills d_list
  * (lf_csr_long_rows_bytes bytes) once for a matrix, and h_counts[0..2] = chunks, rows, entries of the longest row; it
