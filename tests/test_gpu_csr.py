@@ -110,3 +110,29 @@ def test_long_rows_in_chunks(fa, torch, feat, b_dtype):
             if m is g:
                 assert torch.equal(out, got)
             assert (np.abs(out.cpu().numpy() - ref) <= bound).all()
+
+
+@pytest.mark.parametrize("rows,average", [(1, 95), (1, 96), (3, 207), (5, 208), (700, 300), (12_288, 96), (12_288, 208), (12_289, 96), (12_289, 208),
+                                          (24_575, 208), (24_576, 208)])
+def test_rows_of_a_workgroup(fa, torch, rows, average):
+    """Where 2, 4, 8 or 16 rows go to a workgroup; rows of the average, empty ones and some of twice as much."""
+    rng = np.random.default_rng(rows + average)
+    cols = 3_001
+    lens = np.full(rows, average)
+    if rows > 3:
+        lens[1:rows - rows % 4:4], lens[2:rows - rows % 4:4] = 0, 2 * average
+    assert lens.sum() == average * rows
+    indptr = np.concatenate([[0], np.cumsum(lens)]).astype(np.int32)
+    first = rng.integers(0, cols, size=rows)
+    at = np.arange(indptr[-1]) - np.repeat(indptr[:-1], lens)
+    step = np.maximum(1, (cols - 1) // np.maximum(lens, 1))
+    indices = (np.repeat(first % step, lens) + at * np.repeat(step, lens)).astype(np.int32)
+    assert indices.max() < cols
+    values = rng.uniform(-1, 1, size=len(indices)).astype(np.float32)
+    g = MTX.from_csr(indptr, indices, (rows, cols), data=values)
+    B = operand(torch, rng, cols, 64, "f32")
+    got = fa.spmm_csr(g, B).cpu().numpy()
+    Bh = B.cpu().numpy()
+    ref = O.spmm_csr_f64(indptr, indices, values, (rows, cols), Bh)
+    bound = 1e-5 * O.spmm_abs_bound(indptr, indices, values, (rows, cols), Bh)
+    assert (np.abs(got - ref) <= bound).all()
