@@ -374,7 +374,7 @@ int lf_csr_spmm_trusted_work(const int32_t* d_indptr, const int32_t* d_indices, 
                              int64_t num_rows, int64_t num_cols, int64_t nnz, int64_t span, const void* d_list,
                              const int64_t* h_counts, void* d_work, size_t work_bytes, int32_t feat_size,
                              int32_t b_dtype, const void* d_B, float* d_C, lf_stream_t stream);
-/* For the first product of a matrix whose longest row is known: that of lf_csr_spmm_trusted_span, unless it would be faster
+/* For a matrix whose longest row is known (lf_csr_check_rows): the product of lf_csr_spmm_trusted_span, unless it would be faster
  * with work space - then LF_WANTS_WORK is returned and nothing is enqueued. */
 #define LF_WANTS_WORK 1
 int lf_csr_spmm_trusted_rows(const int32_t* d_indptr, const int32_t* d_indices, const float* d_values,

@@ -702,14 +702,14 @@ def spmm_csr(g, B, b_dtype: str = "f32", use_values: bool = True):
     vals = dev.values if use_values else None
     work = dev._csr_work.get((feat, dtype))
     # the device arrays were made by lf_coo_to_csr or have passed lf_csr_check: no second check
-    if work is None and dev._longest is not None and dev._long_rows is None:
-        sizes = (dev.num_rows, dev.num_cols, dev.nnz, dev.span)
-        rc = lib.lf_csr_spmm_trusted_rows(dev.indptr.data_ptr(), dev.indices.data_ptr(), None if vals is None else vals.data_ptr(), *sizes,
-                                          dev._longest, feat, dtype, B.data_ptr(), out.data_ptr(), _stream())
+    if work is None and dev._longest is not None:
+        rc = lib.lf_csr_spmm_trusted_rows(dev.indptr.data_ptr(), dev.indices.data_ptr(), None if vals is None else vals.data_ptr(),
+                                          dev.num_rows, dev.num_cols, dev.nnz, dev._span, dev._longest, feat, dtype, B.data_ptr(),
+                                          out.data_ptr(), _stream())
+        if rc == 0:
+            return out
         if rc != _lib.LF_WANTS_WORK:
             _lib.check(rc)
-            dev._csr_work[(feat, dtype)] = (sizes, None, None, 0)
-            return out
     sizes, rows, counts, nbytes = work or dev.csr_work(feat, dtype)
     if nbytes:
         work = torch.empty(nbytes, dtype=torch.uint8, device="cuda")
