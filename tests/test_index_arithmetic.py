@@ -1,0 +1,44 @@
+"""The index arithmetic of the kernels (csrc/lf_index.h), compiled for the host, at the largest arrays that are accepted:
+no GPU, and no array of that size, is needed to see a 32-bit sum pass 2^31."""
+import ctypes
+import os
+import shutil
+import subprocess
+
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+MOST = 2**31 - 1                       # entries of a matrix
+
+SOURCE = """
+#include "lf_index.h"
+extern "C" int group_source(int start, int fill, int q) { return lf::group_source(start, fill, q); }
+"""
+
+
+@pytest.fixture(scope="module")
+def host(tmp_path_factory):
+    cxx = shutil.which("g++") or shutil.which("c++")
+    if cxx is None:
+        pytest.skip("no host compiler")
+    where = tmp_path_factory.mktemp("index")
+    (where / "index.cpp").write_text(SOURCE)
+    lib = str(where / "index.so")
+    # (sums that wrap, as the GPU's do)
+    subprocess.run([cxx, "-std=c++17", "-O1", "-fwrapv", "-shared", "-fPIC", "-I", os.path.join(ROOT, "liteform_ae_amd", "csrc"),
+                    str(where / "index.cpp"), "-o", lib], check=True)
+    return ctypes.CDLL(lib)
+
+
+@pytest.mark.parametrize("start,fill,width", [(MOST - 16, 16, 32), (2**31 - 20, 17, 32), (MOST - 1, 1, 1024), (MOST - 3, 3, 4), (MOST - 1025, 1025, 1024),
+                                              (0, 5, 8), (7, 0, 8), (MOST, 0, 4)])
+def test_padding_of_the_last_rows_reads_inside_the_arrays(host, start, fill, width):
+    """Groups of four slots of a segment's ELL rows: the ones that hold entries start at theirs, the others somewhere
+    in the segment."""
+    slots = -(-fill // width) * width
+    for q in range(0, max(slots, 4), 4):
+        source = host.group_source(start, fill, q)
+        if q < fill:
+            assert source == start + q
+        else:
+            assert start <= source <= max(start + fill - 1, start)
