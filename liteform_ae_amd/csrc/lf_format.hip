@@ -648,10 +648,10 @@ __device__ __forceinline__ void mark_fours(const int32_t* __restrict__ first, in
     const int lane = threadIdx.x & 63;
     Four f[N];
 #pragma unroll
-    for (int u = 0; u < N; ++u) f[u] = *(const Four*)(first + lf::fours_source(j, u * 256 + lane * 4, fill));
+    for (int u = 0; u < N; ++u) f[u] = *(const Four*)(first + min(j + u * 256 + lane * 4, fill - 4));
 #pragma unroll
     for (int u = 0; u < N; ++u)
-        for (int i = 0; i < 4; ++i) mark(f[u].c[i], lf::fours_inside(j, u * 256 + lane * 4, fill));
+        for (int i = 0; i < 4; ++i) mark(f[u].c[i], j + u * 256 + lane * 4 < fill);
 }
 template <typename Mark>
 __device__ __forceinline__ void mark_piece(const int32_t* __restrict__ indices, int start, int j, int fill, Mark mark) {

@@ -13,14 +13,5 @@ constexpr int group_source(int start, int fill, int q) {
     return start + (q < last ? q : last);
 }
 
-// A segment of `fill` >= 4 entries is walked from its entry j, a lane's four entries `ahead` (below 2^16) from there: whether they
-// start inside the segment, and where they are loaded, which is back from its end where they pass it.  (j + ahead may pass
-// 2^31 at the end of a segment of nearly that many entries.)
-constexpr bool fours_inside(int j, int ahead, int fill) { return (unsigned)j + (unsigned)ahead < (unsigned)fill; }
-constexpr int fours_source(int j, int ahead, int fill) {
-    const unsigned at = (unsigned)j + (unsigned)ahead, most = (unsigned)(fill - 4);
-    return (int)(at < most ? at : most);
-}
-
 }  // namespace lf
 #endif

@@ -13,8 +13,6 @@ MOST = 2**31 - 1                       # entries of a matrix
 SOURCE = """
 #include "lf_index.h"
 extern "C" int group_source(int start, int fill, int q) { return lf::group_source(start, fill, q); }
-extern "C" int fours_inside(int j, int ahead, int fill) { return lf::fours_inside(j, ahead, fill); }
-extern "C" int fours_source(int j, int ahead, int fill) { return lf::fours_source(j, ahead, fill); }
 """
 
 
@@ -44,13 +42,3 @@ def test_padding_of_the_last_rows_reads_inside_the_arrays(host, start, fill, wid
             assert source == start + q
         else:
             assert start <= source <= max(start + fill - 1, start)
-
-
-@pytest.mark.parametrize("fill", [4, 5, 255, 256, 257, 1023, 1024, 1025, 8193, 2**31 - 1024, 2**31 - 1023, MOST - 1, MOST])
-def test_the_end_of_a_long_segment_is_walked_inside_it(host, fill):
-    """The last pieces of 1024 entries of a segment, four to a lane: every entry is loaded, nothing past the end is."""
-    for j in {max((fill - 1) // 1024 * 1024 - k * 1024, 0) for k in range(2)}:
-        for ahead in range(0, 1024, 4):
-            inside = j + ahead < fill
-            assert host.fours_inside(j, ahead, fill) == inside
-            assert host.fours_source(j, ahead, fill) == min(j + ahead, fill - 4)
