@@ -6,6 +6,7 @@
 // or a row each, as the lengths of the workgroup's rows ask for.
 #include <hip/hip_runtime.h>
 
+#include "lf_index.h"
 #include "lf_internal.h"
 #include "lf_spmm_device.h"
 
@@ -226,7 +227,7 @@ csr_long_rows_kernel(const int32_t* __restrict__ indptr, long long n_rows, int2*
     if (r >= n_rows) return;
     const int start = indptr[r], len = indptr[r + 1] - start;
     if (len <= kCsrChunkedRow) return;
-    const int n = (len + kCsrChunk - 1) / kCsrChunk;
+    const int n = lf::chunks_of(len, kCsrChunk);
     const int at = atomicAdd(&counters[0], n), row = atomicAdd(&counters[1], 1);
     atomicMax(&counters[2], len);
     rows[row] = make_int4((int)r, at, n, 0);

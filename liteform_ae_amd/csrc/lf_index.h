@@ -13,5 +13,8 @@ constexpr int group_source(int start, int fill, int q) {
     return start + (q < last ? q : last);
 }
 
+// Chunks of at most `chunk` entries that a row of `len` > 0 entries is cut into.
+constexpr int chunks_of(int len, int chunk) { return (len - 1) / chunk + 1; }
+
 }  // namespace lf
 #endif

@@ -13,6 +13,7 @@ MOST = 2**31 - 1                       # entries of a matrix
 SOURCE = """
 #include "lf_index.h"
 extern "C" int group_source(int start, int fill, int q) { return lf::group_source(start, fill, q); }
+extern "C" int chunks_of(int len, int chunk) { return lf::chunks_of(len, chunk); }
 """
 
 
@@ -42,3 +43,8 @@ def test_padding_of_the_last_rows_reads_inside_the_arrays(host, start, fill, wid
             assert source == start + q
         else:
             assert start <= source <= max(start + fill - 1, start)
+
+
+@pytest.mark.parametrize("length", [1, 511, 512, 513, 1024, 2**31 - 513, 2**31 - 511, MOST])
+def test_chunks_of_the_longest_rows(host, length):
+    assert host.chunks_of(length, 512) == -(-length // 512)
