@@ -76,8 +76,12 @@ struct CsrMore {
 //
 // MORE: panels and chunks.  An instantiation of its own: their arguments and tests cost every workgroup of the other launches (13.6K
 // rows of 4, N = 480: 21.1 us, 24.7 with them).
+//
+// Three wavefronts to a SIMD at least for up to 1024 float features: left to itself the compiler took 174 registers, which are two, and
+// products of more than 512 features 4 - 11 % more time (150K power-law rows, N = 544 / 1024 300 / 443 us, 335 / 472 so; 300K, N = 800 767, 833).
+constexpr int csr_waves(int ch, bool floats, bool wide, bool more) { return ch == 4 && floats && !wide && !more ? 3 : 1; }
 template <int LPR, int CH, typename BT, bool WIDE, bool MORE>
-__global__ void __launch_bounds__(kCsrThreads)
+__global__ void __launch_bounds__(kCsrThreads, csr_waves(CH, sizeof(BT) == 4, WIDE, MORE))
 csr_spmm_kernel(CsrArgs a, CsrMore more) {
     constexpr int VEC = Dense<BT>::kVec;
     constexpr int kWaves = kCsrThreads / 64;
