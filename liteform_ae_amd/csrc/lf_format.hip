@@ -1245,8 +1245,8 @@ hyb_fill_kernel(SegView v, const int32_t* __restrict__ seg_deg, const int32_t* _
                     live[u] = s_fill[lo] - q;          // entries of the source row from q on
                     at[u] = s_dst[lo] + q;
                     len[u] = mine < total ? min(4, (int)s_len[lo] - q) : 0;
-                    const int src = lf::group_source(s_start[lo], s_fill[lo], q), from = tiny ? 0 : min(src, nnz - 4);
-                    shift[u] = live[u] > 0 ? src - from : 0;
+                    const int from = tiny ? 0 : lf::group_source(s_start[lo], q, nnz);
+                    shift[u] = live[u] > 0 ? s_start[lo] + q - from : 0;
                     x[u] = make_float4(1.f, 1.f, 1.f, 1.f);
                     if constexpr (tiny) {
                         const int last = max(nnz - 1, 0);

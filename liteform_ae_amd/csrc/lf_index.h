@@ -5,12 +5,12 @@
 
 namespace lf {
 
-// Source of the group of four slots that starts at slot q of a segment (first entry `start`, `fill` entries): the group's first
-// entry, or the segment's last one where the group is padding, which is loaded and dropped.  (start + q itself passes 2^31 in
-// the padding of the last rows of a matrix of nearly 2^31 entries.)
-constexpr int group_source(int start, int fill, int q) {
-    const int last = fill > 0 ? fill - 1 : 0;
-    return start + (q < last ? q : last);
+// Where the group of four slots that starts at slot q of a segment (first entry `start`) is loaded from arrays of n >= 4 entries: its
+// first entry, or back from the arrays' end where it passes that.  (q runs on into the segment's padding, whose groups are loaded and
+// dropped: up to 1023 past its last entry, and so past 2^31 in the last rows of a matrix of nearly that many entries.)
+constexpr int group_source(int start, int q, int n) {
+    const unsigned at = (unsigned)start + (unsigned)q, most = (unsigned)(n - 4);
+    return (int)(at < most ? at : most);
 }
 
 // Chunks of at most `chunk` entries that a row of `len` > 0 entries is cut into.

@@ -12,7 +12,7 @@ MOST = 2**31 - 1                       # entries of a matrix
 
 SOURCE = """
 #include "lf_index.h"
-extern "C" int group_source(int start, int fill, int q) { return lf::group_source(start, fill, q); }
+extern "C" int group_source(int start, int q, int n) { return lf::group_source(start, q, n); }
 extern "C" int chunks_of(int len, int chunk) { return lf::chunks_of(len, chunk); }
 """
 
@@ -31,18 +31,13 @@ def host(tmp_path_factory):
     return ctypes.CDLL(lib)
 
 
-@pytest.mark.parametrize("start,fill,width", [(MOST - 16, 16, 32), (2**31 - 20, 17, 32), (MOST - 1, 1, 1024), (MOST - 3, 3, 4), (MOST - 1025, 1025, 1024),
-                                              (0, 5, 8), (7, 0, 8), (MOST, 0, 4)])
-def test_padding_of_the_last_rows_reads_inside_the_arrays(host, start, fill, width):
-    """Groups of four slots of a segment's ELL rows: the ones that hold entries start at theirs, the others somewhere
-    in the segment."""
+@pytest.mark.parametrize("start,fill,width,entries", [(MOST - 16, 16, 32, MOST), (2**31 - 20, 17, 32, MOST), (MOST - 1, 1, 1024, MOST), (MOST - 3, 3, 4, MOST),
+                                                      (MOST - 1025, 1025, 1024, MOST), (0, MOST, 1024, MOST), (0, 5, 8, 9), (0, 4, 8, 4), (7, 2, 8, 9)])
+def test_groups_of_the_last_rows_are_loaded_inside_the_arrays(host, start, fill, width, entries):
+    """Groups of four slots of a segment's ELL rows, its padding among them."""
     slots = -(-fill // width) * width
-    for q in range(0, max(slots, 4), 4):
-        source = host.group_source(start, fill, q)
-        if q < fill:
-            assert source == start + q
-        else:
-            assert start <= source <= max(start + fill - 1, start)
+    for q in sorted({*range(0, min(slots, 2048), 4), *range(max(slots - 2048, 0), slots, 4)}):
+        assert host.group_source(start, q, entries) == min(start + q, entries - 4)
 
 
 @pytest.mark.parametrize("length", [1, 511, 512, 513, 1024, 2**31 - 513, 2**31 - 511, MOST])
