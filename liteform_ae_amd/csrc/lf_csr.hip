@@ -312,6 +312,12 @@ Slices csr_slices(int64_t rows, int rows_per_group, int64_t groups, int64_t num_
 // 154K of 144, N = 160 1930 -> 1290; 65.7K of 131, N = 384 1525 -> 898; 183K of 118, N = 384 4165 -> 3330.  Where they would lose: 333K
 // of 13, N = 480 1210, in two 1350; 253K of 14, N = 160 326, 351.  (A hyb plan, whose partitions hold their rows by length, takes 850,
 // 960, 930 and 820 for the first four.)  Rows share a sub-wave up to two batches here: 3 to 8 % better.
+// Not below kPanelMinUs of price, where the launches cost what they save: 57K of 28, N = 64 41.4, in two 62.9; 57K of 60, N = 64 75.1, 90.9; 120K of
+// 28, N = 64 111, 118; 24K of 60, N = 128 53.8, 63.2; beyond it 65K of 153, N = 64 320 -> 212, 200K of 60, N = 64 404 -> 377.
+// Nor where few rows meet a B that the eight L2s nearly hold together (32 MB): one launch is faster than its price there, and the tails of
+// several count.  5790 rows of 170, N = 704, B of 26 MB 153, in three 187; 6785 of 263, N = 960, 31 MB 324, 383; 9138 of 197, N = 672, 19 MB 218, 237;
+// 11,060 of 164, N = 480, 39 MB 194, 207.  On the other side of both lines: 8834 of 127, N = 992, 49 MB 258 -> 209; 52.7K of 239, N = 128, 33 MB
+// 572 -> 423; 125K of 290, N = 64, 24 MB 955 -> 712.  92 products whose price says panels: 12 of them were slower, up to 22 %; of the 69 that remain none.
 //
 // Long rows.  A row is summed by the four wavefronts of a workgroup at most, in steps of a batch to every sub-wave, up to 0.6 us each.
 // Where the longest one would take as long as a quarter of the product, rows of more than kCsrChunkedRow entries are cut into
@@ -326,6 +332,7 @@ struct CsrShape {
 CsrShape csr_shape(int64_t num_rows, int64_t num_cols, int64_t nnz, int64_t span, int feat, int dtype, const int64_t* counts, bool may_panel) {
     constexpr double kPanelMinUs = 150.0, kPanelUs = 7.0, kBoundsUs = 8.0, kRowUs = 1e-4, kBytesOfC = 7e6, kWorth = 0.9;
     constexpr int kUsesOfB = 16;
+    constexpr int64_t kPanelBytesOfB = 40'000'000;
     CsrShape shape;
     shape.width = (int)num_cols;
     const int price_rows = num_rows >= kCsrManyRows ? kCsrRowsMany : kCsrRowsFew;
@@ -335,7 +342,8 @@ CsrShape csr_shape(int64_t num_rows, int64_t num_cols, int64_t nnz, int64_t span
     };
     shape.slices = priced(1);
     double least = shape.slices.us;
-    if (may_panel && least > kPanelMinUs && nnz > kUsesOfB * num_cols && !is_near((double)span, num_cols)) {
+    const bool large = num_rows >= kCsrManyRows || num_cols * feat * (dtype == LF_DTYPE_BF16 ? 2 : 4) >= kPanelBytesOfB;
+    if (may_panel && large && least > kPanelMinUs && nnz > kUsesOfB * num_cols && !is_near((double)span, num_cols)) {
         const double one = least;
         for (int panels : {2, 3, 4, 6, 8}) {
             const Slices x = priced(panels);
