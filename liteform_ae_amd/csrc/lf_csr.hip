@@ -32,7 +32,7 @@ int rows_of_group(int64_t num_rows, int64_t entries) {
     return few && entries >= kCsrLongAverage * num_rows ? 4 : kCsrRowsFew;
 }
 constexpr int kCsrChunkedRow = 512, kCsrChunk = 512;      // rows of more entries are cut into chunks, see csr_shape
-constexpr double kStepUs = 0.6, kFinalUs = 8.0, kTail = 0.25;
+constexpr double kSmallBatchUs = 0.35, kBatchUs = 0.6, kFinalUs = 10.0, kTail = 0.15;
 constexpr int kCsrLongRow = 256;           // a row of more entries, and more than a wavefront's share, takes the whole workgroup
 
 struct CsrArgs {
@@ -319,11 +319,14 @@ Slices csr_slices(int64_t rows, int rows_per_group, int64_t groups, int64_t num_
 // 11,060 of 164, N = 480, 39 MB 194, 207.  On the other side of both lines: 8834 of 127, N = 992, 49 MB 258 -> 209; 52.7K of 239, N = 128, 33 MB
 // 572 -> 423; 125K of 290, N = 64, 24 MB 955 -> 712.  92 products whose price says panels: 12 of them were slower, up to 22 %; of the 69 that remain none.
 //
-// Long rows.  A row is summed by the four wavefronts of a workgroup at most, in steps of a batch to every sub-wave, up to 0.6 us each.
-// Where the longest one would take as long as a quarter of the product, rows of more than kCsrChunkedRow entries are cut into
-// chunks, a workgroup to each, and a second kernel (3 us) adds up their sums.  Power-law graphs, us, without -> with: 116K rows,
-// longest 6613, N = 352 212 -> 127; 53K, 4273, N = 480 97.6 -> 78.2; 15.6K, 9208, N = 96 18.4 -> 14.2; 28K, 6361, N = 96 22.6 -> 19.5.
-// Always, it would lose where rows are short or B is in the L2s: 57K rows of 28, longest 1000, N = 64 40.9, 46; 6.5K, N = 64 7.2, 11.4.
+// Long rows.  A row is summed by the four wavefronts of a workgroup at most, a batch (8 entries where a wavefront has eight sub-waves, 16
+// otherwise) to every sub-wave at a time, each 0.35 or 0.6 us behind the one before.  Where the longest row takes 10 us more than 0.15 of the
+// product's price, rows of more than kCsrChunkedRow entries are cut into chunks, a workgroup to each, and a second kernel adds up their sums; the 10 us
+// are that launch, the allocation of the work space and a larger kernel, 5 to 8 us together, and what a tail of that length hides behind
+// anyway.  Power-law graphs, us, without -> with: 116K rows, longest 6613, N = 352 212 -> 127; 150K, 13,000, N = 320 299 -> 149; 60K, 4000, N = 96
+// 40.1 -> 26.6; 9K, 10,951, N = 672 90.3 -> 30.8.  On the other side of the line: 16K, 2636, N = 64 11.3, with chunks 15.9; 21K, 5468,
+// N = 256 24.5, 32.7; 57K rows of 28, longest 1000, N = 64 40.9, 46; 2000 rows of 90, longest 1528, N = 800 44.3, 54.1.  530 products of 2000 to 150,000
+// rows, N = 32 .. 1024, both ways: the 84 that take chunks take 0.64 of the time, 0.98 at most.
 struct CsrShape {
     int rows_per_group = 0, panels = 1, width = 0;
     int64_t n_groups = 0, n_chunks = 0;
@@ -360,8 +363,9 @@ CsrShape csr_shape(int64_t num_rows, int64_t num_cols, int64_t nnz, int64_t span
     shape.n_groups = lf::ceil_div(num_rows, (int64_t)shape.rows_per_group);
     int lpr, ch;
     if (counts && counts[0] > 0 && feature_shape(shape.slices.feat, dtype, &lpr, &ch) == LF_OK) {
-        const double steps = (double)counts[2] * lpr / (kCsrThreads * kUnroll);
-        if (kStepUs * steps > kFinalUs + kTail * least) shape.n_chunks = counts[0];
+        const int batch = lpr < 16 ? lpr : 16;
+        const double batches = (double)counts[2] * lpr / (kCsrThreads * batch);
+        if ((lpr < 16 ? kSmallBatchUs : kBatchUs) * batches > kFinalUs + kTail * least) shape.n_chunks = counts[0];
     }
     return shape;
 }

@@ -24,3 +24,19 @@ def test_no_panels_where_one_launch_is_faster(rows, cols, degree, feat):
 def test_panels_where_they_are_faster(rows, cols, degree, feat):
     panels, rest = divmod(work_bytes(rows, cols, degree, feat), 4 * rows)
     assert 1 <= panels <= 7 and rest == 0
+
+
+# rows, columns, entries a row, N, longest row
+@pytest.mark.parametrize("rows,cols,degree,feat,longest", [(15_976, 30_245, 3, 64, 2636), (20_968, 25_716, 3, 256, 5468), (23_998, 33_355, 3, 256, 6192),
+                                                           (4000, 4141, 3, 96, 1500), (2000, 1377, 21, 672, 591), (2000, 2000, 90, 800, 1528),
+                                                           (2391, 4700, 47, 192, 1900), (57_000, 57_000, 28, 64, 1000), (6500, 6500, 5, 64, 1200)])
+def test_long_rows_stay_whole_where_that_is_faster(rows, cols, degree, feat, longest):
+    assert work_bytes(rows, cols, degree, feat, longest) == 0
+    assert work_bytes(rows, cols, degree, feat, counts=(7, 3, longest)) == 0
+
+
+@pytest.mark.parametrize("rows,cols,degree,feat,longest", [(116_000, 116_000, 4, 352, 6613), (150_000, 176_328, 4, 320, 13_000), (60_000, 74_951, 3, 96, 4000),
+                                                           (9000, 10_951, 3, 672, 10_951), (9000, 10_178, 3, 128, 10_178)])
+def test_long_rows_in_chunks_where_that_is_faster(rows, cols, degree, feat, longest):
+    assert work_bytes(rows, cols, degree, feat, longest) == -1
+    assert work_bytes(rows, cols, degree, feat, counts=(31, 5, longest)) == 31 * 4 * feat
