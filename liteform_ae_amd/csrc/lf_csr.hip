@@ -8,29 +8,14 @@
 
 #include "lf_index.h"
 #include "lf_internal.h"
+#include "lf_rules.h"
 #include "lf_spmm_device.h"
 
 namespace {
 
-// A workgroup of four wavefronts takes kCsrRowsFew or kCsrRowsMany consecutive rows; a wavefront takes the next rows
+// A workgroup of four wavefronts takes 2, 8 or 16 consecutive rows (csr_rows_of_group); a wavefront takes the next rows
 // off a counter whenever it is through with its own, so that nothing waits for the longest row but itself.
 constexpr int kCsrThreads = 256;
-constexpr int kCsrRowsFew = 8, kCsrRowsMany = 16;
-constexpr long long kCsrManyRows = 24576;
-// Few long rows: 4 or 2 to a workgroup, as the last workgroups of 8 are left alone for a part of the product that counts.  8 -> 4 -> 2
-// rows, us: 2000 rows of 400, N = 32 12.6 -> 10.6 -> 8.8; 3500 of 400, N = 512 136 -> 128 -> 116; 6000 of 250, N = 96 39.5 -> 37.1 -> 37.0;
-// 16,000 of 250, N = 256 187 -> 179 -> 180; 3500 of 120, N = 32 7.3 -> 6.9 -> 6.8.  31 drawn products by this rule: 0.95 of the time, 0.77 to
-// 1.01, but for two of uneven rows, many of which the whole of a smaller workgroup takes: 3000 rows of 192, N = 128 17.3, 18.3, 18.7, 3900 of 150, N
-// = 32 10.3, 10.6.  Beyond it, 8, 4, 2 rows: 2000 rows of 120, N = 128 10.6, 10.4, 11.4; 16,000 of 30, N = 256 43.2, 46.7, 57.8; of 120,
-// N = 96 51.7, 53.0, 54.6; 24,000 of 60 in three panels, N = 512 224, 250, 362.
-constexpr long long kCsrFewRows = 12288;
-constexpr int kCsrLongAverage = 96, kCsrVeryLongAverage = 208;
-int rows_of_group(int64_t num_rows, int64_t entries) {
-    if (num_rows >= kCsrManyRows) return kCsrRowsMany;
-    const bool few = num_rows <= kCsrFewRows;
-    if (entries >= kCsrVeryLongAverage * num_rows) return few ? 2 : 4;
-    return few && entries >= kCsrLongAverage * num_rows ? 4 : kCsrRowsFew;
-}
 constexpr int kCsrChunkedRow = 512, kCsrChunk = 512;      // rows of more entries are cut into chunks, see csr_shape
 constexpr double kSmallBatchUs = 0.35, kBatchUs = 0.6, kFinalUs = 10.0, kTail = 0.15;
 constexpr int kCsrLongRow = 256;           // a row of more entries, and more than a wavefront's share, takes the whole workgroup
@@ -338,14 +323,14 @@ CsrShape csr_shape(int64_t num_rows, int64_t num_cols, int64_t nnz, int64_t span
     constexpr int64_t kPanelBytesOfB = 40'000'000;
     CsrShape shape;
     shape.width = (int)num_cols;
-    const int price_rows = num_rows >= kCsrManyRows ? kCsrRowsMany : kCsrRowsFew;
+    const int price_rows = num_rows >= lf::kCsrManyRows ? lf::kCsrRowsMany : lf::kCsrRowsFew;
     auto priced = [&](int panels) {
         return csr_slices(num_rows, price_rows, lf::ceil_div(num_rows, (int64_t)price_rows), lf::ceil_div(num_cols, (int64_t)panels), nnz / panels, span, feat,
                           dtype);
     };
     shape.slices = priced(1);
     double least = shape.slices.us;
-    const bool large = num_rows >= kCsrManyRows || num_cols * feat * (dtype == LF_DTYPE_BF16 ? 2 : 4) >= kPanelBytesOfB;
+    const bool large = num_rows >= lf::kCsrManyRows || num_cols * feat * (dtype == LF_DTYPE_BF16 ? 2 : 4) >= kPanelBytesOfB;
     if (may_panel && large && least > kPanelMinUs && nnz > kUsesOfB * num_cols && !is_near((double)span, num_cols)) {
         const double one = least;
         for (int panels : {2, 3, 4, 6, 8}) {
@@ -359,7 +344,7 @@ CsrShape csr_shape(int64_t num_rows, int64_t num_cols, int64_t nnz, int64_t span
             }
         }
     }
-    shape.rows_per_group = rows_of_group(num_rows, nnz / shape.panels);
+    shape.rows_per_group = lf::csr_rows_of_group(num_rows, nnz, counts ? counts[2] : 0, shape.panels);
     shape.n_groups = lf::ceil_div(num_rows, (int64_t)shape.rows_per_group);
     int lpr, ch;
     if (counts && counts[0] > 0 && feature_shape(shape.slices.feat, dtype, &lpr, &ch) == LF_OK) {

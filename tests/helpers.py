@@ -1,5 +1,11 @@
 """Shared helpers for the test-suite (not collected by pytest)."""
+import ctypes
+import os
+import shutil
+import subprocess
+
 import numpy as np
+import pytest
 
 from liteform_ae_amd.format_matrix_market import MTX
 from oracle import liteform_oracle as O
@@ -59,3 +65,14 @@ def assert_hyb_equal(got, want):
             for b, (x, y) in enumerate(zip(ab, bb)):
                 assert x.shape == y.shape, (name, p, b, x.shape, y.shape)
                 np.testing.assert_array_equal(x, y, err_msg=f"{name}[{p}][{b}]")
+
+
+def host_library(where, source):
+    """`source`, which may include the headers of csrc, compiled for the host and loaded (sums that wrap, as the GPU's do)."""
+    cxx = shutil.which("g++") or shutil.which("c++")
+    if cxx is None:
+        pytest.skip("no host compiler")
+    (where / "host.cpp").write_text(source)
+    csrc = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "liteform_ae_amd", "csrc")
+    subprocess.run([cxx, "-std=c++17", "-O1", "-fwrapv", "-shared", "-fPIC", "-I", csrc, str(where / "host.cpp"), "-o", str(where / "host.so")], check=True)
+    return ctypes.CDLL(str(where / "host.so"))

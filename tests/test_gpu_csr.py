@@ -136,3 +136,23 @@ def test_rows_of_a_workgroup(fa, torch, rows, average):
     ref = O.spmm_csr_f64(indptr, indices, values, (rows, cols), Bh)
     bound = 1e-5 * O.spmm_abs_bound(indptr, indices, values, (rows, cols), Bh)
     assert (np.abs(got - ref) <= bound).all()
+
+
+@pytest.mark.parametrize("rows,average", [(4, 96), (7, 100), (1001, 97), (5120, 96), (5119, 250), (5121, 250)])
+def test_few_uneven_rows(fa, torch, rows, average):
+    """Two rows to a workgroup, and the least number of rows that takes eight again: rows of the average, empty ones, some of twice
+    as much and a long one."""
+    rng = np.random.default_rng(rows + average)
+    cols = 3_001
+    lens = np.full(rows, average)
+    lens[1::4], lens[3::4] = 0, 2 * average                    # the average still, or a little below it
+    lens[0] = 1600
+    indptr, indices, values = matrix(rng, lens, cols)
+    assert indptr[-1] >= 96 * rows and lens.max() * rows >= 3 * indptr[-1]
+    g = MTX.from_csr(indptr, indices, (rows, cols), data=values)
+    B = operand(torch, rng, cols, 96, "f32")
+    got = fa.spmm_csr(g, B).cpu().numpy()
+    Bh = B.cpu().numpy()
+    ref = O.spmm_csr_f64(indptr, indices, values, (rows, cols), Bh)
+    bound = 1e-5 * O.spmm_abs_bound(indptr, indices, values, (rows, cols), Bh)
+    assert (np.abs(got - ref) <= bound).all()

@@ -1,13 +1,9 @@
 """The index arithmetic of the kernels (csrc/lf_index.h), compiled for the host, at the largest arrays that are accepted:
 no GPU, and no array of that size, is needed to see a 32-bit sum pass 2^31."""
-import ctypes
-import os
-import shutil
-import subprocess
-
 import pytest
 
-ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+from helpers import host_library
+
 MOST = 2**31 - 1                       # entries of a matrix
 
 SOURCE = """
@@ -19,16 +15,7 @@ extern "C" int chunks_of(int len, int chunk) { return lf::chunks_of(len, chunk);
 
 @pytest.fixture(scope="module")
 def host(tmp_path_factory):
-    cxx = shutil.which("g++") or shutil.which("c++")
-    if cxx is None:
-        pytest.skip("no host compiler")
-    where = tmp_path_factory.mktemp("index")
-    (where / "index.cpp").write_text(SOURCE)
-    lib = str(where / "index.so")
-    # (sums that wrap, as the GPU's do)
-    subprocess.run([cxx, "-std=c++17", "-O1", "-fwrapv", "-shared", "-fPIC", "-I", os.path.join(ROOT, "liteform_ae_amd", "csrc"),
-                    str(where / "index.cpp"), "-o", lib], check=True)
-    return ctypes.CDLL(lib)
+    return host_library(tmp_path_factory.mktemp("index"), SOURCE)
 
 
 @pytest.mark.parametrize("start,fill,width,entries", [(MOST - 16, 16, 32, MOST), (2**31 - 20, 17, 32, MOST), (MOST - 1, 1, 1024, MOST), (MOST - 3, 3, 4, MOST),
