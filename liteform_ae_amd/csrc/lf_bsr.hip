@@ -34,6 +34,7 @@
 #include <algorithm>
 
 #include "lf_internal.h"
+#include "lf_rules.h"
 
 namespace {
 
@@ -58,21 +59,6 @@ constexpr int64_t kStreamYBytes = 64ll << 20;
 
 typedef _Float16 half8_t __attribute__((ext_vector_type(8)));
 typedef float float4_t __attribute__((ext_vector_type(4)));
-
-// Features per lane.  Rows of X of up to 64 features fill half of 128, or a quarter: lanes past the last feature
-// would load and multiply for nothing, in registers that other wavefronts could use (blocks of 32: 198 with 8 features,
-// 102 with 4, 65 with 2).  8 features a lane -> 4 or 2, us: blocks of 32, 20,000 block rows of 4, F = 16 / 32 / 48 / 64 52.1 /
-// 60.1 / 74.4 / 82.0 -> 37.9 / 52.7 / 64.3 / 79.9; of 10, F = 16 126.7 -> 90.0; blocks of 16, 22,282 block rows of 8, F = 16 34.4 ->
-// 25.3.  40 products of 2000 to 800,000 rows, F = 16 .. 128: 0.90 of the time on average, with the pairs below.  From 49 features on
-// there is little to gain, and where blocks of 64 or many blocks of 16 keep the memory busy 4 features a lane lose: 2400 block rows
-// of 10 of 64, F = 64 64.2 and 68.3 (800 of them 22.4 and 20.4), 33,636 of 10 of 16, F = 56 107.5 and 108.6.  Above 64 features two
-// tiles of 4 a lane lose up to 20 % or gain 4, by the sizes.
-constexpr long long kNarrowRows16 = 16384, kNarrowRows64 = 2048;
-int lane_features(int feat, int block, long long block_rows) {
-    if (feat <= 32) return 2;
-    const bool narrow = feat <= 48 || block == 32 || block_rows <= (block == 16 ? kNarrowRows16 : kNarrowRows64);
-    return feat <= 64 && narrow ? 4 : 8;
-}
 
 // A block row of 64 is two steps a block, one after the other, and few block rows leave CUs idle: two wavefronts share each
 // then, and the second one's sums go through LDS.  us, alone -> by two: 100 block rows of 10, F = 32 6.9 -> 6.4, F = 64 9.6 ->
@@ -252,7 +238,7 @@ int lf_bsr_spmm_trusted_nnz(const int32_t* d_indptr, const int32_t* d_indices, c
     const bool few_blocks = nnz_blocks < kPairedBlocks * num_block_rows;      // (also where their number is not known)
     const long long tiles_of_128 = lf::ceil_div(feat_size, kFeatTile);
     const bool paired = block_size == 64 && num_block_rows * tiles_of_128 <= kPairedRows && !few_blocks;
-    const int vf = paired && feat_size > 64 && num_block_rows * tiles_of_128 <= kPairedNarrowRows ? 4 : lane_features(feat_size, block_size, num_block_rows);
+    const int vf = paired && feat_size > 64 && num_block_rows * tiles_of_128 <= kPairedNarrowRows ? 4 : lf::bsr_lane_features(feat_size, block_size, num_block_rows, nnz_blocks);
     const int n_tiles = (int)lf::ceil_div(feat_size, 16 * vf);
     const long long units = (long long)num_block_rows * n_tiles;
     const bool stream_y = (int64_t)num_block_rows * block_size * feat_size * 2 >= kStreamYBytes;

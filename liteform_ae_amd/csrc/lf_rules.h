@@ -22,5 +22,24 @@ constexpr int csr_rows_of_group(long long rows, long long entries, long long lon
     return rows <= kCsrFewRows && uneven && entries / panels >= kCsrLongAverage * rows ? 2 : kCsrRowsFew;
 }
 
+// ---- features to a lane of the BSR product
+// Rows of X of up to 64 features fill half of the 128 that a wavefront takes with 8 to a lane, or a quarter: lanes past the last feature
+// would load and multiply for nothing, in registers that other wavefronts could use (blocks of 32: 198 with 8 features,
+// 102 with 4, 65 with 2).  8 features a lane -> 4 or 2, us: blocks of 32, 20,000 block rows of 4, F = 16 / 32 / 48 52.1 / 60.1 / 74.4 ->
+// 37.9 / 52.7 / 64.3; of 10, F = 16 126.7 -> 90.0; blocks of 16, 22,282 block rows of 8, F = 16 34.4 -> 25.3; blocks of 64, 1500 of 10,
+// F = 40 39.8 -> 29.8.  From 49 features on (57 with blocks of 32) half of the lanes or fewer are idle, and where many blocks keep the
+// memory busy 4 features a lane lose to the wider loads of 8.  Inside the lines: blocks of 64, 1397 block rows of 7, F = 56 30.3 -> 24.8, of 32,
+// 7757 of 8, F = 64 54.6 -> 53.5, of 16, 10,176 of 6, F = 64 24.5 -> 24.2; beyond: of 64, 1948 of 8, F = 56 37.8, 40.1; of 32, 18,331 of 5, F = 64
+// 85.7, 87.9; of 16, 10,169 of 10, F = 64 34.2, 35.0.  177 products of 32,000 to 800,000 rows, F = 16 .. 64: the 155 with 4 or 2 take 0.90 of
+// the time, and no more than with 8 where the kernel is longer than a call (7.5 us).  Above 64 features two tiles of 4 a lane lose up to 20 % or
+// gain 4, by the sizes.
+constexpr int bsr_lane_features(int feat, int block, long long block_rows, long long blocks) {       // blocks == 0: not known
+    if (feat <= 32) return 2;
+    if (feat > 64) return 8;
+    if (feat <= 48 || (block == 32 && feat <= 56)) return 4;
+    const long long most_rows = block == 16 ? 16384 : block == 32 ? (1ll << 62) : 2048, most_blocks = block == 64 ? 12288 : 65536;
+    return blocks > 0 && blocks <= most_blocks && block_rows <= most_rows ? 4 : 8;
+}
+
 }  // namespace lf
 #endif

@@ -9,6 +9,7 @@ from helpers import host_library
 SOURCE = """
 #include "lf_rules.h"
 extern "C" int csr_rows(long long rows, long long entries, long long longest, int panels) { return lf::csr_rows_of_group(rows, entries, longest, panels); }
+extern "C" int bsr_features(int feat, int block, long long rows, long long blocks) { return lf::bsr_lane_features(feat, block, rows, blocks); }
 """
 
 
@@ -32,3 +33,13 @@ def test_rows_of_a_csr_workgroup(rules, rows, average, longest, group):
 def test_rows_of_a_csr_workgroup_in_panels(rules):
     size = ctypes.c_longlong
     assert [rules.csr_rows(size(5000), size(5000 * 200), size(2000), panels) for panels in (1, 2, 3)] == [2, 2, 8]
+
+
+@pytest.mark.parametrize("feat,block,rows,blocks,features", [
+    (8, 16, 50_000, 500_000, 2), (32, 64, 12_500, 120_000, 2), (40, 16, 50_000, 500_000, 4), (48, 64, 12_500, 120_000, 4), (72, 16, 100, 300, 8), (128, 64, 100, 1000, 8),
+    (56, 64, 1397, 9_761, 4), (56, 64, 2048, 12_288, 4), (56, 64, 2048, 12_289, 8), (64, 64, 2049, 4_100, 8), (56, 64, 1936, 17_390, 8),
+    (56, 32, 21_398, 192_515, 4), (64, 32, 6553, 65_536, 4), (64, 32, 6553, 65_537, 8), (64, 32, 18_331, 91_639, 8),
+    (64, 16, 10_176, 61_041, 4), (56, 16, 16_384, 65_536, 4), (56, 16, 16_385, 40_000, 8), (56, 16, 16_384, 65_537, 8), (64, 16, 14_770, 132_930, 8),
+    (56, 16, 1000, 0, 8), (56, 32, 1000, 0, 4), (64, 64, 100, 0, 8)])                       # 0: their number is not known
+def test_features_of_a_bsr_lane(rules, feat, block, rows, blocks, features):
+    assert rules.bsr_features(feat, block, ctypes.c_longlong(rows), ctypes.c_longlong(blocks)) == features
