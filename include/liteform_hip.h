@@ -363,7 +363,7 @@ int lf_csr_spmm_trusted_span(const int32_t* d_indptr, const int32_t* d_indices, 
  * NULL, and the product is that of lf_csr_spmm_trusted_span).  The chunks are those of lf_csr_long_rows, which fills d_list
  * (lf_csr_long_rows_bytes bytes) once for a matrix, and h_counts[0..2] = chunks, rows, entries of the longest row; it
  * synchronises.  Without them (NULL) long rows stay whole; lf_csr_spmm_work_bytes is then told the entries of the longest
- * row (lf_csr_check_rows; 0: unknown) and answers -1 where the product would be faster with the list.  The product only
+ * row, or more (lf_csr_check_rows, lf_coo_to_csr_rows; 0: unknown), and answers -1 where the product would be faster with the list.  The product only
  * enqueues kernels. */
 size_t lf_csr_long_rows_bytes(int64_t nnz);
 int lf_csr_long_rows(const int32_t* d_indptr, int64_t num_rows, int64_t nnz, void* d_list, size_t list_bytes,
@@ -374,7 +374,7 @@ int lf_csr_spmm_trusted_work(const int32_t* d_indptr, const int32_t* d_indices, 
                              int64_t num_rows, int64_t num_cols, int64_t nnz, int64_t span, const void* d_list,
                              const int64_t* h_counts, void* d_work, size_t work_bytes, int32_t feat_size,
                              int32_t b_dtype, const void* d_B, float* d_C, lf_stream_t stream);
-/* For a matrix whose longest row is known (lf_csr_check_rows): the product of lf_csr_spmm_trusted_span, unless it would be faster
+/* For a matrix whose longest row is known (lf_csr_check_rows, lf_coo_to_csr_rows): the product of lf_csr_spmm_trusted_span, unless it would be faster
  * with work space - then LF_WANTS_WORK is returned and nothing is enqueued. */
 #define LF_WANTS_WORK 1
 int lf_csr_spmm_trusted_rows(const int32_t* d_indptr, const int32_t* d_indices, const float* d_values,
@@ -393,6 +393,12 @@ int lf_coo_to_csr(const int32_t* d_coo_row, const int32_t* d_coo_col, const floa
                   int64_t num_rows, int64_t num_cols, void* d_workspace, size_t workspace_bytes,
                   int32_t* d_indptr, int32_t* d_indices, float* d_values, int64_t* h_nnz_out,
                   lf_stream_t stream);
+/* The same, and *h_longest receives the entries of the longest row; where duplicates were added up it may be more, up to the
+ * most triplets of a row. */
+int lf_coo_to_csr_rows(const int32_t* d_coo_row, const int32_t* d_coo_col, const float* d_coo_val, int64_t nnz,
+                       int64_t num_rows, int64_t num_cols, void* d_workspace, size_t workspace_bytes,
+                       int32_t* d_indptr, int32_t* d_indices, float* d_values, int64_t* h_nnz_out, int64_t* h_longest,
+                       lf_stream_t stream);
 
 /* Block-sparse SpMM on the matrix cores, the counterpart of bench_bsrmm's kernel
  * (format_algos.py:1182-1643): Y = A_bsr . X with square fp16 blocks of block_size = 16, 32 or

@@ -30,7 +30,8 @@ inline size_t align_up(size_t x, size_t a) { return (x + a - 1) / a * a; }
 
 __global__ void pack_keys_kernel(const int32_t* __restrict__ row, const int32_t* __restrict__ col,
                                  const float* __restrict__ val, long long nnz, long long cols,
-                                 unsigned long long* __restrict__ keys, float* __restrict__ vals) {
+                                 unsigned long long* __restrict__ keys, float* __restrict__ vals, int* __restrict__ longest) {
+    if (blockIdx.x == 0 && threadIdx.x == 0) *longest = 0;     // for row_pointer_kernel
     for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < nnz;
          i += (long long)gridDim.x * blockDim.x) {
         keys[i] = (unsigned long long)row[i] * (unsigned long long)cols + (unsigned long long)col[i];
@@ -46,18 +47,26 @@ __global__ void unpack_cols_kernel(const unsigned long long* __restrict__ keys, 
         indices[i] = (int32_t)(keys[i] % (unsigned long long)cols);
 }
 
-// indptr[r] = number of unique keys below r * cols (keys are sorted)
-__global__ void row_pointer_kernel(const unsigned long long* __restrict__ keys, const int* __restrict__ n_unique,
-                                   long long rows, long long cols, int32_t* __restrict__ indptr) {
-    const long long r = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (r > rows) return;
-    const unsigned long long bound = (unsigned long long)r * (unsigned long long)cols;
+// indptr[r] = number of unique keys below r * cols (keys are sorted).  A workgroup's last row is the next one's first, so that it
+// knows the lengths of all but that one.
+constexpr int kPointerThreads = 256, kPointerRows = kPointerThreads - 1;
+__global__ void __launch_bounds__(kPointerThreads)
+row_pointer_kernel(const unsigned long long* __restrict__ keys, const int* __restrict__ n_unique,
+                   long long rows, long long cols, int32_t* __restrict__ indptr, int* __restrict__ longest) {
+    __shared__ int s_first[kPointerThreads];
+    const long long r = (long long)blockIdx.x * kPointerRows + threadIdx.x;
     long long lo = 0, hi = *n_unique;
+    const unsigned long long bound = (unsigned long long)min(r, rows) * (unsigned long long)cols;
     while (lo < hi) {
         const long long mid = (lo + hi) >> 1;
         if (keys[mid] < bound) lo = mid + 1; else hi = mid;
     }
-    indptr[r] = (int32_t)lo;
+    if (r <= rows) indptr[r] = (int32_t)lo;
+    s_first[threadIdx.x] = (int)lo;
+    __syncthreads();
+    int most = threadIdx.x < kPointerRows ? s_first[threadIdx.x + 1] - (int)lo : 0;
+    for (int d = 32; d > 0; d >>= 1) most = max(most, __shfl_xor(most, d));
+    if ((threadIdx.x & 63) == 0 && most > __hip_atomic_load(longest, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicMax(longest, most);
 }
 
 // ---- bins of rows sorted in LDS
@@ -73,8 +82,9 @@ __global__ void row_pointer_kernel(const unsigned long long* __restrict__ keys, 
 // flags: [kNotHere] an entry outside the matrix or bins of too many, known before anything is distributed, and
 // [kCrowded] a long row with too many of its columns beside each other: the other way has to be taken; [kReads] windows
 // that large bins' parts will read; [kLargeParts] parts left to bin_sort_large_kernel; [kTwice] entries that are to be
-// added to another one of their place.
-constexpr int kNotHere = 0, kReads = 1, kCrowded = 2, kLargeParts = 3, kTwice = 4, kFlags = 5;
+// added to another one of their place.  From [kLongest] on: entries of the longest row of every bin, of which bin_report_kernel takes the
+// largest (an atomic of every bin on one word was 7 - 13 us).
+constexpr int kNotHere = 0, kReads = 1, kCrowded = 2, kLargeParts = 3, kTwice = 4, kFlags = 5, kLongest = kFlags;
 constexpr int kBinThreads = 512;
 constexpr int kBinChunk = 4096;            // entries that a workgroup distributes at least
 constexpr int kBinMaxChunks = 1024;
@@ -117,7 +127,7 @@ BinShape bin_shape(long long nnz, long long rows, long long cols) {
     b.totals = off; off += align_up((size_t)b.bins * 4, 256);
     b.bases = off; off += align_up((size_t)b.bins * 4, 256);
     b.list = off; off += align_up((size_t)(nnz / kBinWindow + b.bins) * 4, 256);
-    b.flags = off; off += 256;
+    b.flags = off; off += align_up((size_t)(kLongest + b.bins) * 4, 256);
     b.twice = off; off += align_up((size_t)nnz * 4, 256);
     b.before = off; off += align_up((size_t)(nnz + 1) * 4, 256);
     b.partial = off; off += align_up((size_t)(nnz / 1024 + 2) * 4, 256);
@@ -281,7 +291,7 @@ template <int THREADS, int CAPACITY, bool LARGE>
 __device__ __forceinline__ void sort_bin(const BinSort& a, int bin, int window, unsigned* s_key, unsigned* s_val, int* s_bucket, int* s_wave) {
     __shared__ int s_first[kBinRows];          // of a row in the bin; not sorted here: -1
     __shared__ int s_count[kBinRows];
-    __shared__ int s_from, s_long, s_long_at, s_before, s_sorted;
+    __shared__ int s_from, s_long, s_long_at, s_before, s_sorted, s_most;
     __shared__ float s_squares;
     constexpr int kOwn = LARGE ? 16 : CAPACITY / THREADS;  // records in registers: usually all, loaded once
     const int base = a.bases[bin], n = a.totals[bin];
@@ -396,6 +406,7 @@ __device__ __forceinline__ void sort_bin(const BinSort& a, int bin, int window, 
     };
 
     for (int r = threadIdx.x; r < n_rows; r += THREADS) s_count[r] = 0;
+    if (threadIdx.x == 0) s_most = 0;
     if (LARGE && threadIdx.x == 0) {
         s_from = n;
         s_long = -1;
@@ -406,8 +417,11 @@ __device__ __forceinline__ void sort_bin(const BinSort& a, int bin, int window, 
     __syncthreads();
     // a thread's consecutive rows
     const int per = (n_rows + THREADS - 1) / THREADS, lo = min((int)threadIdx.x * per, n_rows), hi = min(lo + per, n_rows);
-    int sum = 0;
-    for (int r = lo; r < hi; ++r) sum += s_count[r];
+    int sum = 0, most = 0;
+    for (int r = lo; r < hi; ++r) {
+        sum += s_count[r];
+        most = max(most, s_count[r]);
+    }
     int at = scan_workgroup<THREADS>(sum, s_wave) - sum;
     for (int r = lo; r < hi; ++r) {
         const int len = s_count[r];
@@ -423,7 +437,12 @@ __device__ __forceinline__ void sort_bin(const BinSort& a, int bin, int window, 
         at += len;
     }
     if (r0 + n_rows == a.rows && threadIdx.x == THREADS - 1) a.indptr[a.rows] = base + n;
+    if (__ballot(most > 0) != 0) {                         // (an atomic of every lane on one word is 64 rounds)
+        for (int d = 32; d > 0; d >>= 1) most = max(most, __shfl_xor(most, d));
+        if ((threadIdx.x & 63) == 0) atomicMax(&s_most, most);
+    }
     __syncthreads();
+    if (threadIdx.x == 0) a.flags[kLongest + bin] = s_most;        // (every window of a large bin the same)
     const int first = LARGE ? s_from : 0;                  // in the bin, of what is sorted together
     sort_part([&](unsigned key) { return !LARGE || s_first[key >> a.lg_cols] >= 0; },
               [&](unsigned key) {
@@ -482,6 +501,19 @@ bin_sort_large_kernel(BinSort a) {
         __syncthreads();                                   // the part before has been read out
         sort_bin<1024, kBinLarge, true>(a, item % kBinMost, item / kBinMost, s_large, s_large + kBinLarge, (int*)(s_large + 2 * kBinLarge), s_wave);
     }
+}
+
+// The flags, and in [kLongest] the entries of the longest row of all bins: to `out`, which may be the host's.
+__global__ void __launch_bounds__(256)
+bin_report_kernel(const int* __restrict__ flags, int bins, int* out) {
+    __shared__ int s_most[4];
+    int most = 0;
+    for (int i = threadIdx.x; i < bins; i += 256) most = max(most, flags[kLongest + i]);
+    for (int d = 32; d > 0; d >>= 1) most = max(most, __shfl_xor(most, d));
+    if ((threadIdx.x & 63) == 0) s_most[threadIdx.x >> 6] = most;
+    __syncthreads();
+    if (threadIdx.x < kFlags) out[threadIdx.x] = flags[threadIdx.x];
+    if (threadIdx.x == kFlags) out[kLongest] = max(max(s_most[0], s_most[1]), max(s_most[2], s_most[3]));
 }
 
 // ---- duplicates in the sorted arrays: marked, counted up to every entry, and added up into its first.  They lie in the
@@ -762,12 +794,22 @@ int lf_coo_to_csr(const int32_t* d_coo_row, const int32_t* d_coo_col, const floa
                   int64_t num_rows, int64_t num_cols, void* d_workspace, size_t workspace_bytes,
                   int32_t* d_indptr, int32_t* d_indices, float* d_values, int64_t* h_nnz_out,
                   lf_stream_t stream) {
+    int64_t longest = 0;
+    return lf_coo_to_csr_rows(d_coo_row, d_coo_col, d_coo_val, nnz, num_rows, num_cols, d_workspace, workspace_bytes, d_indptr, d_indices, d_values,
+                              h_nnz_out, &longest, stream);
+}
+
+int lf_coo_to_csr_rows(const int32_t* d_coo_row, const int32_t* d_coo_col, const float* d_coo_val, int64_t nnz,
+                       int64_t num_rows, int64_t num_cols, void* d_workspace, size_t workspace_bytes,
+                       int32_t* d_indptr, int32_t* d_indices, float* d_values, int64_t* h_nnz_out, int64_t* h_longest,
+                       lf_stream_t stream) {
     hipStream_t s = (hipStream_t)stream;
     LF_REQUIRE(num_rows >= 0 && num_rows < (1ll << 31) && num_cols >= 1 && num_cols < (1ll << 31), LF_ERR_INVALID,
                "bad shape %lld x %lld", (long long)num_rows, (long long)num_cols);
     LF_REQUIRE(nnz >= 0 && nnz < (1ll << 31), LF_ERR_UNSUPPORTED, "nnz must be below 2^31");
-    LF_REQUIRE(d_indptr && h_nnz_out, LF_ERR_INVALID, "null output");
+    LF_REQUIRE(d_indptr && h_nnz_out && h_longest, LF_ERR_INVALID, "null output");
     if (nnz == 0) {
+        *h_longest = 0;
         LF_HIP(hipMemsetAsync(d_indptr, 0, (size_t)(num_rows + 1) * 4, s));
         LF_HIP(hipStreamSynchronize(s));
         *h_nnz_out = 0;
@@ -804,9 +846,20 @@ int lf_coo_to_csr(const int32_t* d_coo_row, const int32_t* d_coo_col, const floa
             bin_sort_large_kernel<<<grid, 1024, kBinLargeBytes, s>>>(sort);
         }
         LF_HIP(hipGetLastError());
-        int h_flags[kFlags] = {};
-        LF_HIP(lf::read_back(h_flags, flags, sizeof(h_flags), s));
+        // The loan goes back when this returns: every way out from here on has waited for the stream.
+        lf::PinnedLoan back((kLongest + 1) * 4);
+        LF_REQUIRE(back.ok(), LF_ERR_HIP, "out of host memory");
+        int* report = back.pinned() ? back.as<int>() : (int*)(ws + b.totals);
+        bin_report_kernel<<<1, 256, 0, s>>>(flags, b.bins, report);
+        hipError_t reported = hipGetLastError();
+        if (reported == hipSuccess && !back.pinned())
+            reported = hipMemcpyAsync(back.as<char>(), report, (kLongest + 1) * 4, hipMemcpyDeviceToHost, s);
+        const hipError_t waited = hipStreamSynchronize(s);
+        LF_HIP(reported);
+        LF_HIP(waited);
+        const int* h_flags = back.as<int>();
         const bool sorted = h_flags[kNotHere] == 0 && h_flags[kCrowded] == 0;
+        if (sorted) *h_longest = h_flags[kLongest];
         if (sorted && h_flags[kTwice] == 0) {
             *h_nnz_out = nnz;
             return LF_OK;
@@ -835,7 +888,7 @@ int lf_coo_to_csr(const int32_t* d_coo_row, const int32_t* d_coo_col, const floa
     size_t temp_bytes = L.temp_bytes;
 
     const int grid = (int)std::min<long long>((nnz + 255) / 256, 65535);
-    pack_keys_kernel<<<grid, 256, 0, s>>>(d_coo_row, d_coo_col, d_coo_val, nnz, num_cols, keys_a, d_values);
+    pack_keys_kernel<<<grid, 256, 0, s>>>(d_coo_row, d_coo_col, d_coo_val, nnz, num_cols, keys_a, d_values, count + 1);
     LF_HIP(hipGetLastError());
     // sorted keys -> keys_b, values in the same order -> vals_a
     LF_HIP(rocprim::radix_sort_pairs(temp, temp_bytes, keys_a, keys_b, d_values, vals_a, (size_t)nnz, 0u,
@@ -846,11 +899,13 @@ int lf_coo_to_csr(const int32_t* d_coo_row, const int32_t* d_coo_col, const floa
                                   rocprim::plus<float>(), rocprim::equal_to<unsigned long long>(), s));
     unpack_cols_kernel<<<grid, 256, 0, s>>>(keys_a, count, num_cols, d_indices);
     LF_HIP(hipGetLastError());
-    row_pointer_kernel<<<(int)((num_rows + 1 + 255) / 256), 256, 0, s>>>(keys_a, count, num_rows, num_cols, d_indptr);
+    row_pointer_kernel<<<(unsigned)std::max<int64_t>(1, (num_rows + kPointerRows - 1) / kPointerRows), kPointerThreads, 0, s>>>(
+        keys_a, count, num_rows, num_cols, d_indptr, count + 1);
     LF_HIP(hipGetLastError());
-    int h_count = 0;
-    LF_HIP(lf::read_back(&h_count, count, 4, s));
-    *h_nnz_out = h_count;
+    int h_count[2] = {0, 0};                                   // entries, those of the longest row
+    LF_HIP(lf::read_back(h_count, count, sizeof(h_count), s));
+    *h_nnz_out = h_count[0];
+    *h_longest = h_count[1];
     return LF_OK;
 }
 

@@ -216,7 +216,7 @@ class _DeviceCSR:
         self._seg_deg = {}
         self._stats_ws = {}          # num_parts -> statistics workspace holding the row bounds
         self._span = None
-        self._longest = None         # entries of the longest row, where the arrays were checked
+        self._longest = 0            # entries of the longest row, or more (lf_coo_to_csr_rows)
         self._long_rows = None       # list of long rows and its counts, see csr_work
         self._csr_work = {}
         src = getattr(g, "_csr_source", None)
@@ -289,11 +289,11 @@ class _DeviceCSR:
         values = torch.empty(n, dtype=torch.float32, device="cuda")
         nbytes = lib.lf_coo_to_csr_workspace_bytes(self.coo_nnz, self.num_rows, self.num_cols)
         ws = torch.empty(max(nbytes, 256), dtype=torch.uint8, device="cuda")
-        out = C.c_int64(0)
-        _lib.check(lib.lf_coo_to_csr(_lib.ptr(row), _lib.ptr(col), _lib.ptr(val), self.coo_nnz, self.num_rows,
-                                     self.num_cols, _lib.ptr(ws), nbytes, _lib.ptr(self.indptr),
-                                     _lib.ptr(indices), _lib.ptr(values), C.byref(out), _stream()))
-        self.nnz = int(out.value)
+        out, longest = C.c_int64(0), C.c_int64(0)
+        _lib.check(lib.lf_coo_to_csr_rows(_lib.ptr(row), _lib.ptr(col), _lib.ptr(val), self.coo_nnz, self.num_rows,
+                                          self.num_cols, _lib.ptr(ws), nbytes, _lib.ptr(self.indptr),
+                                          _lib.ptr(indices), _lib.ptr(values), C.byref(out), C.byref(longest), _stream()))
+        self.nnz, self._longest = int(out.value), int(longest.value)
         self.indices = indices[:self.nnz]
         self._values = values[:self.nnz]
         # duplicates of unit entries add up to 2, 3, ...: only a duplicate-free unit matrix is "all ones"
@@ -310,7 +310,7 @@ class _DeviceCSR:
             sizes = (self.num_rows, self.num_cols, self.nnz, self.span)
             rows = counts = None
             nbytes = -1
-            if self._long_rows is None and self._longest is not None:
+            if self._long_rows is None:
                 nbytes = lib.lf_csr_spmm_work_bytes(*sizes, None, self._longest, feat, dtype)
             keep = nbytes >= 0
             if not keep:
@@ -702,10 +702,10 @@ def spmm_csr(g, B, b_dtype: str = "f32", use_values: bool = True):
     vals = dev.values if use_values else None
     work = dev._csr_work.get((feat, dtype))
     # the device arrays were made by lf_coo_to_csr or have passed lf_csr_check: no second check
-    if work is None and dev._longest is not None:
+    if work is None:
         rc = lib.lf_csr_spmm_trusted_rows(dev.indptr.data_ptr(), dev.indices.data_ptr(), None if vals is None else vals.data_ptr(),
-                                          dev.num_rows, dev.num_cols, dev.nnz, dev._span, dev._longest, feat, dtype, B.data_ptr(),
-                                          out.data_ptr(), _stream())
+                                          dev.num_rows, dev.num_cols, dev.nnz, dev.span if dev._span is None else dev._span, dev._longest,
+                                          feat, dtype, B.data_ptr(), out.data_ptr(), _stream())
         if rc == 0:
             return out
         if rc != _lib.LF_WANTS_WORK:

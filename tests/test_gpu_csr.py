@@ -156,3 +156,70 @@ def test_few_uneven_rows(fa, torch, rows, average):
     ref = O.spmm_csr_f64(indptr, indices, values, (rows, cols), Bh)
     bound = 1e-5 * O.spmm_abs_bound(indptr, indices, values, (rows, cols), Bh)
     assert (np.abs(got - ref) <= bound).all()
+
+
+def triplets(rng, lens, cols, twice=0):
+    """Triplets of rows of `lens` distinct columns in random order, `twice` of them given again."""
+    indptr, indices, values = matrix(rng, lens, cols)
+    row = np.repeat(np.arange(len(lens)), lens)
+    order = rng.permutation(len(row))
+    order = np.concatenate([order, order[:twice]])
+    return row[order].astype(np.int32), indices[order], values[order]
+
+
+@pytest.mark.parametrize("rows,cols,average,longest,twice", [
+    (1, 60, 40, 40, 0), (3001, 4001, 20, 700, 0), (3001, 4001, 20, 700, 9), (70_001, 3000, 12, 40, 0),
+    (4, 9000, 1200, 5000, 0),                                  # a bin of more than 4096 entries
+    (2_000_003, 2_000_003, 1, 1000, 0), (255, 8_400_000, 30, 90, 0), (256, 8_400_000, 30, 90, 3), (511, 8_400_000, 30, 90, 0)])      # not in bins
+def test_triplets_know_their_longest_row(fa, torch, rows, cols, average, longest, twice):
+    """The first product of a matrix made from triplets is the one call that it is for CSR arrays: no list of long rows unless they are cut."""
+    rng = np.random.default_rng(rows + twice)
+    lens = rng.integers(0, average + 1, size=rows)
+    lens[rows // 2] = longest
+    if rows == 511:
+        lens[254], lens[rows // 2] = longest, 1                # the last row of a workgroup's
+    row, col, data = triplets(rng, lens, cols, twice)
+    g = MTX.from_coo(row, col, (rows, cols), data=data)
+    dev = fa._device_csr(g)
+    assert dev.path == "coo" and (dev._longest == longest if not twice else longest <= dev._longest <= longest + twice)
+    B = torch.rand((cols, 32), device="cuda", generator=torch.Generator(device="cuda").manual_seed(1)) - 0.5
+    got = fa.spmm_csr(g, B)
+    assert dev._long_rows is None and not dev._csr_work
+    at, inverse = np.unique(col, return_inverse=True)          # the rows of B that are met
+    ref = torch.zeros((rows, 32), dtype=torch.float64, device="cuda")
+    bound = torch.zeros_like(ref)
+    rows_at, met = torch.from_numpy(row).cuda().long(), B[torch.from_numpy(at).cuda().long()].double()[torch.from_numpy(inverse).cuda()]
+    products = torch.from_numpy(data).cuda().double()[:, None] * met
+    ref.index_add_(0, rows_at, products)
+    bound.index_add_(0, rows_at, products.abs())
+    assert bool(((got - ref).abs() <= 1e-5 * bound).all())
+
+
+def test_no_triplets(fa, torch):
+    none = np.zeros(0, dtype=np.int32)
+    g = MTX.from_coo(none, none, (5, 7), data=np.zeros(0, dtype=np.float32))
+    assert fa._device_csr(g)._longest == 0
+    assert not fa.spmm_csr(g, torch.rand((7, 32), device="cuda")).any()
+
+
+@pytest.mark.parametrize("twice", [0, 300])
+def test_panels_and_chunks_of_a_matrix_from_triplets(fa, torch, twice):
+    rng = np.random.default_rng(twice)
+    rows, cols, feat = 24_577, 30_011, 512
+    lens = rng.integers(0, 180, size=rows)
+    lens[7] = cols
+    row, col, data = triplets(rng, lens, cols, twice)
+    g = MTX.from_coo(row, col, (rows, cols), data=data)
+    B = operand(torch, rng, cols, feat, "f32")
+    got = fa.spmm_csr(g, B)
+    chunks = 4 * feat * sum(-(-n // 512) for n in lens.tolist() if n > 512)
+    both = work_bytes(fa, g, feat, "f32")
+    assert both > chunks and (both - chunks) % (4 * rows) == 0
+    some = np.unique(np.concatenate([np.arange(0, rows, 37), [7, rows - 1]]))
+    mine = np.isin(row, some)
+    A = np.searchsorted(some, row[mine])
+    Bh = B.cpu().numpy()
+    import scipy.sparse as sp
+    S = sp.coo_matrix((data[mine].astype(np.float64), (A, col[mine])), shape=(len(some), cols)).tocsr()
+    bound = 1e-5 * (abs(S) @ np.abs(Bh.astype(np.float64)))
+    assert (np.abs(got.cpu().numpy()[some] - S @ Bh.astype(np.float64)) <= bound).all()
