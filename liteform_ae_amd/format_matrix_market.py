@@ -15,6 +15,7 @@ Differences, all additive:
 """
 from __future__ import annotations
 
+import os
 from os.path import basename, splitext
 
 import numpy as np
@@ -38,10 +39,27 @@ def _are_plain_triplets(row, col, data, shape):
     return all(_inside(i, n) for i, n in zip((row, col), shape))
 
 
+_BY_THREADS = 1 << 16        # entries
+_forked = {}                 # process id -> whether it is a fork that runs its parent's program
+
+
+def _is_forked() -> bool:
+    """Whether this process is a fork that has not started a program of its own.  The threads that its parent had are gone in
+    it, and torch, which does not know, would wait for them for ever.  (The kernel's flag PF_FORKNOEXEC; unknown counts as one.)"""
+    pid = os.getpid()
+    if pid not in _forked:
+        try:
+            with open("/proc/self/stat") as stat:
+                _forked[pid] = bool(int(stat.read().rpartition(")")[2].split()[6]) & 0x40)
+        except (OSError, ValueError, IndexError):
+            _forked[pid] = True
+    return _forked[pid]
+
+
 def _inside(index, n) -> bool:
-    """Whether every entry of an int32 array is in [0, n); by the host's threads where it is long (3M entries
-    160 us with one, 25 so)."""
-    if len(index) >= 1 << 16 and index.flags.c_contiguous and index.flags.writeable:
+    """Whether every entry of an int32 array is in [0, n); by torch's threads where the array is long and the process has
+    them."""
+    if len(index) >= _BY_THREADS and index.flags.c_contiguous and index.flags.writeable and not _is_forked():
         import torch
         lo, hi = torch.aminmax(torch.from_numpy(index))
         return 0 <= int(lo) and int(hi) < n
