@@ -16,6 +16,7 @@ Differences, all additive:
 from __future__ import annotations
 
 import os
+import sys
 from os.path import basename, splitext
 
 import numpy as np
@@ -58,9 +59,9 @@ def _is_forked() -> bool:
 
 def _inside(index, n) -> bool:
     """Whether every entry of an int32 array is in [0, n); by torch's threads where the array is long and the process has
-    them."""
-    if len(index) >= _BY_THREADS and index.flags.c_contiguous and index.flags.writeable and not _is_forked():
-        import torch
+    them (a process that works with host arrays only does not load torch for this)."""
+    if len(index) >= _BY_THREADS and index.flags.c_contiguous and index.flags.writeable and "torch" in sys.modules and not _is_forked():
+        torch = sys.modules["torch"]
         lo, hi = torch.aminmax(torch.from_numpy(index))
         return 0 <= int(lo) and int(hi) < n
     return int(index.view(np.uint32).max()) < n
