@@ -14,6 +14,32 @@ ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 LONG = fmm._BY_THREADS
 
 
+@pytest.mark.parametrize("length", [1, 1000, LONG - 1, LONG, LONG + 1])
+@pytest.mark.parametrize("kind", ["plain", "read-only", "strided"])
+def test_every_index_is_looked_at(length, kind):
+    """The first and last index allowed, the ones beside them and the least one, at the first, a middle and the last entry."""
+    n = 70_000
+    good = np.random.default_rng(length).integers(0, n, size=length).astype(np.int32)
+    data = np.ones(length, dtype=np.float32)
+    for place in {0, length // 2, length - 1}:
+        for value in (0, n - 1, n, -1, -2**31):
+            index = good.copy()
+            index[place] = value
+            if kind == "read-only":
+                index.flags.writeable = False
+            elif kind == "strided":
+                index = np.repeat(index, 2)[::2]
+            inside = 0 <= value < n
+            assert fmm._inside(index, n) == inside
+            for row, col in ((index, good), (good, index)):
+                assert fmm._are_plain_triplets(row, col, data, (n, n)) == inside
+                if inside:
+                    assert MTX.from_coo(row, col, (n, n), data=data).num_edges() == length
+                else:
+                    with pytest.raises(ValueError):
+                        MTX.from_coo(row, col, (n, n), data=data)
+
+
 def _in_child(answers, index):
     answers.put(MTX.from_coo(index, index, (LONG, LONG)).num_edges())
 
