@@ -283,6 +283,37 @@ def test_bad_slabs_are_refused_at_plan_creation(env):
     assert create(rows_nd, cols_nd, mask_nd, m)[0] == L.LF_ERR_INVALID
 
 
+@pytest.mark.parametrize("width,rows", [(1, 1), (1, 2), (1, 3), (1, 4), (1, 5), (1, 4093), (1, 4094), (1, 4095), (1, 70_001), (2, 1), (2, 3), (8, 1), (8, 40_000),
+                                        (64, 2_051), (64, 40_000), (1024, 131)])
+def test_a_bad_column_is_found_in_every_slot(env, width, rows):
+    """The first slot, the last ones and slots of every round of the check, in buckets of one slot, of less than a load, of no whole
+    load at the end, of several rounds and of those that are sampled for row groups; padding counts.  Status only."""
+    lib, L, torch = env
+    num_cols, slots = 1000, width * rows
+    cols = torch.randint(0, num_cols, (slots,), dtype=torch.int32, device="cuda")
+    row_ids = torch.arange(rows, dtype=torch.int32, device="cuda")
+    vals = torch.ones(slots, device="cuda")
+    meta = torch.full((rows,), 1 | 1 << 11, dtype=torch.int32, device="cuda")      # one valid slot, the others padding
+    desc = (L.BucketDesc * 1)(L.BucketDesc(width, 0, rows, row_ids.data_ptr(), cols.data_ptr(), vals.data_ptr(), meta.data_ptr()))
+
+    def create():
+        plan = C.c_void_p()
+        rc = lib.lf_spmm_create(C.byref(plan), desc, 1, 1, rows, num_cols, 64, 0, None)
+        if rc == 0:
+            assert lib.lf_spmm_destroy(plan) == 0
+        return rc
+
+    assert create() == 0
+    places = {0, 1, slots // 2, *range(max(slots - 5, 0), slots), *range(0, slots, max(slots // 37, 1))}
+    for at in sorted(p for p in places if p < slots):
+        good = int(cols[at])
+        cols[at] = (num_cols, -1, 2**31 - 1)[at % 3]
+        rc = create()
+        cols[at] = good
+        assert rc == L.LF_ERR_INVALID and "column index" in L.last_error(), at
+    assert create() == 0
+
+
 def test_a_head_announcing_a_huge_segment_is_refused(env):
     """A head word that announces 100,000 ELL rows in a 64-wide bucket of a few rows: the
     announced segment is long enough for the cooperative (chunked) path, whose counting pass
