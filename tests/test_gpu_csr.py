@@ -223,3 +223,27 @@ def test_panels_and_chunks_of_a_matrix_from_triplets(fa, torch, twice):
     S = sp.coo_matrix((data[mine].astype(np.float64), (A, col[mine])), shape=(len(some), cols)).tocsr()
     bound = 1e-5 * (abs(S) @ np.abs(Bh.astype(np.float64)))
     assert (np.abs(got.cpu().numpy()[some] - S @ Bh.astype(np.float64)) <= bound).all()
+
+
+@pytest.mark.parametrize("b_dtype,cols", [("f32", 1_060_003), ("bf16", 2_110_003)])
+def test_long_rows_in_chunks_of_a_b_past_4_gb(fa, torch, b_dtype, cols):
+    rng = np.random.default_rng(cols)
+    feat = 1024
+    lens = rng.integers(0, 6, size=300)
+    lens[[0, 7, 150, 299]] = [513, 60_000, 1025, 20_000]
+    indptr, indices, values = matrix(rng, lens, cols)
+    indices[indptr[8] - 1] = cols - 1                          # the last row of B
+    g = MTX.from_csr(indptr, indices, (len(lens), cols), data=values)
+    gen = torch.Generator(device="cuda").manual_seed(cols)
+    B = torch.rand((cols, feat), device="cuda", generator=gen, dtype=torch.float32 if b_dtype == "f32" else torch.bfloat16).sub_(0.5)
+    assert B.numel() * B.element_size() > 2**32
+    got = fa.spmm_csr(g, B, b_dtype).double()
+    assert work_bytes(fa, g, feat, b_dtype) == 4 * feat * sum(-(-n // 512) for n in lens.tolist() if n > 512)
+    for r, n in enumerate(lens):
+        if n == 0:
+            assert not got[r].any()
+            continue
+        at = torch.from_numpy(indices[indptr[r]:indptr[r + 1]]).cuda().long()
+        x = torch.from_numpy(values[indptr[r]:indptr[r + 1]]).cuda().double()
+        rows_of_b = B[at].double()
+        assert bool(((got[r] - x @ rows_of_b).abs() <= 1e-5 * (x.abs() @ rows_of_b.abs())).all()), r
