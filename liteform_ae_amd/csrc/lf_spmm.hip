@@ -1251,50 +1251,50 @@ plan_scan_kernel(const PlanBucket* __restrict__ buckets, const int32_t* __restri
             there_row[u] = rows[there];
         }
 #pragma unroll
-    for (int u = 0; u < kScanRows; ++u) {
-        const long long e = e0 + u * stride;
-        if (e >= n_rows) break;
-        const int row = row_of[u];
-        const bool row_ok = (unsigned)row < (unsigned long long)num_rows;
-        bad_row |= !row_ok;
-        if (bk.part == 0 && row_ok) covered[row] = 1;
-        const int m = meta_of[u];
-        const int len = m & (int)kMetaLenMask;
-        bad_meta |= len < 1 || len > (1 << log_w);
-        const long long field = (long long)(((uint32_t)m & 0x7FFFFFFFu) >> kMetaLenBits);
-        // what the next ELL row must be: a continuation row with index `want`, or a head (0)
-        long long want = 0;
-        if (m >= 0) {
-            bad_meta |= field < 1 || e + field > n_rows;
-            want = field > 1 ? 1 : 0;
-        } else {
-            const long long h = e - field;
-            if (field < 1 || h < 0) {
-                bad_meta = true;
+        for (int u = 0; u < kScanRows; ++u) {
+            const long long e = e0 + u * stride;
+            if (e >= n_rows) break;
+            const int row = row_of[u];
+            const bool row_ok = (unsigned)row < (unsigned long long)num_rows;
+            bad_row |= !row_ok;
+            if (bk.part == 0 && row_ok) covered[row] = 1;
+            const int m = meta_of[u];
+            const int len = m & (int)kMetaLenMask;
+            bad_meta |= len < 1 || len > (1 << log_w);
+            const long long field = (long long)(((uint32_t)m & 0x7FFFFFFFu) >> kMetaLenBits);
+            // what the next ELL row must be: a continuation row with index `want`, or a head (0)
+            long long want = 0;
+            if (m >= 0) {
+                bad_meta |= field < 1 || e + field > n_rows;
+                want = field > 1 ? 1 : 0;
             } else {
-                const int hm = there_meta[u];
-                const long long n = (long long)((uint32_t)hm >> kMetaLenBits);
-                bad_meta |= hm < 0 || field >= n || there_row[u] != row;
-                want = field + 1 < n ? field + 1 : 0;
+                const long long h = e - field;
+                if (field < 1 || h < 0) {
+                    bad_meta = true;
+                } else {
+                    const int hm = there_meta[u];
+                    const long long n = (long long)((uint32_t)hm >> kMetaLenBits);
+                    bad_meta |= hm < 0 || field >= n || there_row[u] != row;
+                    want = field + 1 < n ? field + 1 : 0;
+                }
             }
+            if (e == 0) bad_meta |= m < 0;
+            if (e + 1 < n_rows) {
+                const int nm = next_of[u];
+                const long long nf = (long long)(((uint32_t)nm & 0x7FFFFFFFu) >> kMetaLenBits);
+                bad_meta |= want == 0 ? nm < 0 : (nm >= 0 || nf != want);
+            } else {
+                bad_meta |= want != 0;
+            }
+            const ChunkedRow x = chunked_row(m, there_meta[u], e, n_rows, log_w, kCoopSlots, chunk_slots, dense_min_slots);
+            found |= x.found;
+            sum[0] += x.n_chunks;
+            sum[1] += x.n_chunks > 1;
+            sum[2] += x.n_chunks > 1 ? x.n_chunks : 0;
+            const long long slots = m >= 0 ? field << log_w : 0;     // of the row that starts here
+            sum[3] += slots > 64 && slots <= 128;
+            sum[4] += slots > 128 && slots <= kCoopSlots;
         }
-        if (e == 0) bad_meta |= m < 0;
-        if (e + 1 < n_rows) {
-            const int nm = next_of[u];
-            const long long nf = (long long)(((uint32_t)nm & 0x7FFFFFFFu) >> kMetaLenBits);
-            bad_meta |= want == 0 ? nm < 0 : (nm >= 0 || nf != want);
-        } else {
-            bad_meta |= want != 0;
-        }
-        const ChunkedRow x = chunked_row(m, there_meta[u], e, n_rows, log_w, kCoopSlots, chunk_slots, dense_min_slots);
-        found |= x.found;
-        sum[0] += x.n_chunks;
-        sum[1] += x.n_chunks > 1;
-        sum[2] += x.n_chunks > 1 ? x.n_chunks : 0;
-        const long long slots = m >= 0 ? field << log_w : 0;     // of the row that starts here
-        sum[3] += slots > 64 && slots <= 128;
-        sum[4] += slots > 128 && slots <= kCoopSlots;
-    }
     }
     if (__ballot(bad_col) != 0 && lane == 0) flags[0] = 1;
     if (__ballot(bad_row) != 0 && lane == 0) flags[1] = 1;
