@@ -17,7 +17,7 @@ namespace {
 // off a counter whenever it is through with its own, so that nothing waits for the longest row but itself.
 constexpr int kCsrThreads = 256;
 constexpr int kCsrChunkedRow = 512, kCsrChunk = 512;      // rows of more entries are cut into chunks, see csr_shape
-constexpr double kSmallBatchUs = 0.35, kBatchUs = 0.6, kFinalUs = 10.0, kTail = 0.15;
+constexpr double kSmallBatchUs = 0.35, kBatchUs = 0.6, kFinalUs = 10.0, kTail = 0.02, kPanelTail = 0.15, kFewOfACu = 4.0;
 constexpr int kCsrLongRow = 256;           // a row of more entries, and more than a wavefront's share, takes the whole workgroup
 
 struct CsrArgs {
@@ -305,19 +305,22 @@ Slices csr_slices(int64_t rows, int rows_per_group, int64_t groups, int64_t num_
 // 572 -> 423; 125K of 290, N = 64, 24 MB 955 -> 712.  92 products whose price says panels: 12 of them were slower, up to 22 %; of the 69 that remain none.
 //
 // Long rows.  A row is summed by the four wavefronts of a workgroup at most, a batch (8 entries where a wavefront has eight sub-waves, 16
-// otherwise) to every sub-wave at a time, each 0.35 or 0.6 us behind the one before.  Where the longest row takes 10 us more than 0.15 of the
-// product's price, rows of more than kCsrChunkedRow entries are cut into chunks, a workgroup to each, and a second kernel adds up their sums; the 10 us
+// otherwise) to every sub-wave at a time, each 0.35 or 0.6 us behind the one before.  Where the longest row takes 10 us more than 0.02 of the
+// product's price (0.15 in panels: 9000 rows of 184, longest 5018, N = 800 355 us, with chunks 399), rows of more than kCsrChunkedRow entries are cut into chunks, a workgroup to each, and a second kernel adds up their sums; the 10 us
 // are that launch, the allocation of the work space and a larger kernel, 5 to 8 us together, and what a tail of that length hides behind
-// anyway.  Power-law graphs, us, without -> with: 116K rows, longest 6613, N = 352 212 -> 127; 150K, 13,000, N = 320 299 -> 149; 60K, 4000, N = 96
-// 40.1 -> 26.6; 9K, 10,951, N = 672 90.3 -> 30.8.  On the other side of the line: 16K, 2636, N = 64 11.3, with chunks 15.9; 21K, 5468,
-// N = 256 24.5, 32.7; 57K rows of 28, longest 1000, N = 64 40.9, 46; 2000 rows of 90, longest 1528, N = 800 44.3, 54.1.  530 products of 2000 to 150,000
-// rows, N = 32 .. 1024, both ways: the 84 that take chunks take 0.64 of the time, 0.98 at most.
+// anyway.  Up to kFewOfACu workgroups to a CU all start at once, and what counts is how many the fullest CU has: where chunks raise
+// that the price goes up with it.  us, without -> with: 116K power-law rows, longest 6613, N = 352 212 -> 127; 150K, 13,000, N = 320 299 -> 149; 9K,
+// 10,951, N = 672 90.3 -> 30.8; 2932 rows of 311, 5251, N = 128 38 -> 27.  On the other side of the lines: 16K power-law rows, 2636, N = 64 11.3, with
+// chunks 15.9; 21K, 5468, N = 256 24.5, 32.7; 57K rows of 28, 1000, N = 64 40.9, 46; 2000 rows of 90, 1528, N = 800, two workgroups to a CU
+// and with chunks three, 44.3, 54.1.  860 products of 2000 to 200,000 rows, N = 32 .. 1024, both ways: the 196 that take chunks take 0.74 of the time, four of
+// them 1.01 to 1.05.
 struct CsrShape {
     int rows_per_group = 0, panels = 1, width = 0;
     int64_t n_groups = 0, n_chunks = 0;
     Slices slices;
 };
-CsrShape csr_shape(int64_t num_rows, int64_t num_cols, int64_t nnz, int64_t span, int feat, int dtype, const int64_t* counts, bool may_panel) {
+// longest: entries of the longest row (0: not known); counts: chunks, rows they are cut from, entries of the longest (null: no chunks)
+CsrShape csr_shape(int64_t num_rows, int64_t num_cols, int64_t nnz, int64_t span, int feat, int dtype, int64_t longest, const int64_t* counts, bool may_panel) {
     constexpr double kPanelMinUs = 150.0, kPanelUs = 7.0, kBoundsUs = 8.0, kRowUs = 1e-4, kBytesOfC = 7e6, kWorth = 0.9;
     constexpr int kUsesOfB = 16;
     constexpr int64_t kPanelBytesOfB = 40'000'000;
@@ -344,13 +347,15 @@ CsrShape csr_shape(int64_t num_rows, int64_t num_cols, int64_t nnz, int64_t span
             }
         }
     }
-    shape.rows_per_group = lf::csr_rows_of_group(num_rows, nnz, counts ? counts[2] : 0, shape.panels);
+    shape.rows_per_group = lf::csr_rows_of_group(num_rows, nnz, longest, shape.panels);
     shape.n_groups = lf::ceil_div(num_rows, (int64_t)shape.rows_per_group);
     int lpr, ch;
     if (counts && counts[0] > 0 && feature_shape(shape.slices.feat, dtype, &lpr, &ch) == LF_OK) {
         const int batch = lpr < 16 ? lpr : 16;
         const double batches = (double)counts[2] * lpr / (kCsrThreads * batch);
-        if ((lpr < 16 ? kSmallBatchUs : kBatchUs) * batches > kFinalUs + kTail * least) shape.n_chunks = counts[0];
+        const double per_cu = (double)shape.slices.n / (kXcds * kCusOfXcd), of_a_cu = (double)shape.n_groups * per_cu;
+        const double fuller = of_a_cu <= kFewOfACu ? std::ceil((double)(shape.n_groups + counts[0]) * per_cu) / std::ceil(of_a_cu) - 1.0 : 0.0;
+        if ((lpr < 16 ? kSmallBatchUs : kBatchUs) * batches > kFinalUs + ((shape.panels > 1 ? kPanelTail : kTail) + fuller) * least) shape.n_chunks = counts[0];
     }
     return shape;
 }
@@ -405,9 +410,9 @@ int64_t lf_csr_spmm_work_bytes(int64_t num_rows, int64_t num_cols, int64_t nnz, 
                                int32_t feat_size, int32_t b_dtype) {
     int lpr, ch;
     if (num_rows <= 0 || num_cols < 1 || feature_shape(feat_size, b_dtype, &lpr, &ch) != LF_OK) return 0;
-    const int64_t guess[3] = {1, 1, longest};
+    const int64_t guess[3] = {longest / kCsrChunk, 1, longest};                // (chunks at least)
     const bool unknown = !h_counts && longest > kCsrChunkedRow;
-    const CsrShape shape = csr_shape(num_rows, num_cols, nnz, span, feat_size, b_dtype, unknown ? guess : h_counts, true);
+    const CsrShape shape = csr_shape(num_rows, num_cols, nnz, span, feat_size, b_dtype, h_counts ? h_counts[2] : longest, unknown ? guess : h_counts, true);
     if (unknown && shape.n_chunks > 0) return -1;
     return (int64_t)work_bytes_of(shape, num_rows, feat_size);
 }
@@ -429,9 +434,9 @@ int csr_product(const int32_t* d_indptr, const int32_t* d_indices, const float* 
     int lpr, ch;
     if (int rc = feature_shape(feat_size, b_dtype, &lpr, &ch)) return rc;
     const bool ask = longest >= 0;
-    const int64_t guess[3] = {longest > kCsrChunkedRow ? 1 : 0, 1, longest};
-    const CsrShape shape = csr_shape(num_rows, num_cols, nnz, span, feat_size, b_dtype, ask ? guess : d_work && d_list ? h_counts : nullptr,
-                                     ask || d_work != nullptr);
+    const int64_t guess[3] = {longest > kCsrChunkedRow ? longest / kCsrChunk : 0, 1, longest};       // (chunks at least)
+    const CsrShape shape = csr_shape(num_rows, num_cols, nnz, span, feat_size, b_dtype, ask ? longest : h_counts ? h_counts[2] : 0,
+                                     ask ? guess : d_work && d_list ? h_counts : nullptr, ask || d_work != nullptr);
     if (ask && work_bytes_of(shape, num_rows, feat_size) > 0) return LF_WANTS_WORK;
     const int64_t n_chunks = shape.n_chunks;
     LF_REQUIRE(!d_work || work_bytes >= work_bytes_of(shape, num_rows, feat_size), LF_ERR_INVALID, "the product needs %zu bytes of work space",

@@ -711,14 +711,10 @@ def spmm_csr(g, B, b_dtype: str = "f32", use_values: bool = True):
         if rc != _lib.LF_WANTS_WORK:
             _lib.check(rc)
     sizes, rows, counts, nbytes = work or dev.csr_work(feat, dtype)
-    if nbytes:
-        work = torch.empty(nbytes, dtype=torch.uint8, device="cuda")
-        rc = lib.lf_csr_spmm_trusted_work(dev.indptr.data_ptr(), dev.indices.data_ptr(), None if vals is None else vals.data_ptr(), *sizes,
-                                          _lib.ptr(rows), _lib.ptr(counts), work.data_ptr(), nbytes, feat, dtype, B.data_ptr(),
-                                          out.data_ptr(), _stream())
-    else:
-        rc = lib.lf_csr_spmm_trusted_span(dev.indptr.data_ptr(), dev.indices.data_ptr(), None if vals is None else vals.data_ptr(), *sizes,
-                                          feat, dtype, B.data_ptr(), out.data_ptr(), _stream())
+    work = torch.empty(nbytes, dtype=torch.uint8, device="cuda") if nbytes else None
+    rc = lib.lf_csr_spmm_trusted_work(dev.indptr.data_ptr(), dev.indices.data_ptr(), None if vals is None else vals.data_ptr(), *sizes,
+                                      _lib.ptr(rows), _lib.ptr(counts), _lib.ptr(work), nbytes, feat, dtype, B.data_ptr(),
+                                      out.data_ptr(), _stream())
     if rc:
         _lib.check(rc)
     return out

@@ -28,7 +28,7 @@ def test_panels_where_they_are_faster(rows, cols, degree, feat):
 
 # rows, columns, entries a row, N, longest row
 @pytest.mark.parametrize("rows,cols,degree,feat,longest", [(15_976, 30_245, 3, 64, 2636), (20_968, 25_716, 3, 256, 5468), (23_998, 33_355, 3, 256, 6192),
-                                                           (4000, 4141, 3, 96, 1500), (2000, 1377, 21, 672, 591), (2000, 2000, 90, 800, 1528),
+                                                           (4000, 4141, 3, 96, 1500), (2000, 1377, 21, 672, 591),
                                                            (2391, 4700, 47, 192, 1900), (57_000, 57_000, 28, 64, 1000), (6500, 6500, 5, 64, 1200)])
 def test_long_rows_stay_whole_where_that_is_faster(rows, cols, degree, feat, longest):
     assert work_bytes(rows, cols, degree, feat, longest) == 0
@@ -36,7 +36,14 @@ def test_long_rows_stay_whole_where_that_is_faster(rows, cols, degree, feat, lon
 
 
 @pytest.mark.parametrize("rows,cols,degree,feat,longest", [(116_000, 116_000, 4, 352, 6613), (150_000, 176_328, 4, 320, 13_000), (60_000, 74_951, 3, 96, 4000),
-                                                           (9000, 10_951, 3, 672, 10_951), (9000, 10_178, 3, 128, 10_178)])
+                                                           (9000, 10_951, 3, 672, 10_951), (9000, 10_178, 3, 128, 10_178), (2932, 5251, 311, 128, 5251)])
 def test_long_rows_in_chunks_where_that_is_faster(rows, cols, degree, feat, longest):
     assert work_bytes(rows, cols, degree, feat, longest) == -1
     assert work_bytes(rows, cols, degree, feat, counts=(31, 5, longest)) == 31 * 4 * feat
+
+
+def test_chunks_that_fill_the_cus_unevenly():
+    """250 workgroups of rows and two slices of B are two to a CU; 41 chunks make them three."""
+    assert work_bytes(2000, 2000, 90, 800, 1528) == -1         # how many chunks there are is not known yet
+    assert work_bytes(2000, 2000, 90, 800, counts=(5, 2, 1528)) == 5 * 4 * 800
+    assert work_bytes(2000, 2000, 90, 800, counts=(41, 19, 1528)) == 0
