@@ -299,10 +299,11 @@ Slices csr_slices(int64_t rows, int rows_per_group, int64_t groups, int64_t num_
 // 960, 930 and 820 for the first four.)  Rows share a sub-wave up to two batches here: 3 to 8 % better.
 // Not below kPanelMinUs of price, where the launches cost what they save: 57K of 28, N = 64 41.4, in two 62.9; 57K of 60, N = 64 75.1, 90.9; 120K of
 // 28, N = 64 111, 118; 24K of 60, N = 128 53.8, 63.2; beyond it 65K of 153, N = 64 320 -> 212, 200K of 60, N = 64 404 -> 377.
-// Nor where few rows meet a B that the eight L2s nearly hold together (32 MB): one launch is faster than its price there, and the tails of
-// several count.  5790 rows of 170, N = 704, B of 26 MB 153, in three 187; 6785 of 263, N = 960, 31 MB 324, 383; 9138 of 197, N = 672, 19 MB 218, 237;
-// 11,060 of 164, N = 480, 39 MB 194, 207.  On the other side of both lines: 8834 of 127, N = 992, 49 MB 258 -> 209; 52.7K of 239, N = 128, 33 MB
-// 572 -> 423; 125K of 290, N = 64, 24 MB 955 -> 712.  92 products whose price says panels: 12 of them were slower, up to 22 %; of the 69 that remain none.
+// Where few rows meet a B that the eight L2s nearly hold together (32 MB) they have to be 21 % cheaper: one launch is faster than its price there,
+// and the tails of several count.  Price and us of one launch, in panels: 5790 rows of 170, N = 704, B of 26 MB 0.88, 153, 187; 6785 of 263, N =
+// 960, 31 MB 0.81, 324, 383; 11,060 of 164, N = 480, 39 MB 0.84, 194, 207; but 18,984 of 256, N = 320, 37 MB 0.72, 443, 310; 11,316 of 133, N = 608, 36
+// MB 0.77, 255, 203.  On the other side of both lines: 8834 of 127, N = 992, 49 MB 0.81, 258, 209; 52.7K of 239, N = 128, 33 MB 0.74, 572, 423; 125K of
+// 290, N = 64, 24 MB 0.67, 955, 712.  92 products that are 10 % cheaper: 12 of them were slower, up to 22 %; of the 78 that remain none.
 //
 // Long rows.  A row is summed by the four wavefronts of a workgroup at most, a batch (8 entries where a wavefront has eight sub-waves, 16
 // otherwise) to every sub-wave at a time, each 0.35 or 0.6 us behind the one before.  Where the longest row takes 10 us more than 0.02 of the
@@ -321,7 +322,7 @@ struct CsrShape {
 };
 // longest: entries of the longest row (0: not known); counts: chunks, rows they are cut from, entries of the longest (null: no chunks)
 CsrShape csr_shape(int64_t num_rows, int64_t num_cols, int64_t nnz, int64_t span, int feat, int dtype, int64_t longest, const int64_t* counts, bool may_panel) {
-    constexpr double kPanelMinUs = 150.0, kPanelUs = 7.0, kBoundsUs = 8.0, kRowUs = 1e-4, kBytesOfC = 7e6, kWorth = 0.9;
+    constexpr double kPanelMinUs = 150.0, kPanelUs = 7.0, kBoundsUs = 8.0, kRowUs = 1e-4, kBytesOfC = 7e6, kWorth = 0.9, kWorthOfFew = 0.79;
     constexpr int kUsesOfB = 16;
     constexpr int64_t kPanelBytesOfB = 40'000'000;
     CsrShape shape;
@@ -334,12 +335,12 @@ CsrShape csr_shape(int64_t num_rows, int64_t num_cols, int64_t nnz, int64_t span
     shape.slices = priced(1);
     double least = shape.slices.us;
     const bool large = num_rows >= lf::kCsrManyRows || num_cols * feat * (dtype == LF_DTYPE_BF16 ? 2 : 4) >= kPanelBytesOfB;
-    if (may_panel && large && least > kPanelMinUs && nnz > kUsesOfB * num_cols && !is_near((double)span, num_cols)) {
+    if (may_panel && least > kPanelMinUs && nnz > kUsesOfB * num_cols && !is_near((double)span, num_cols)) {
         const double one = least;
         for (int panels : {2, 3, 4, 6, 8}) {
             const Slices x = priced(panels);
             const double us = panels * x.us + kBoundsUs + (panels - 1) * ((double)num_rows * feat * 8.0 / kBytesOfC + kPanelUs + kRowUs * (double)num_rows * x.n);
-            if (us < least && us < kWorth * one) {
+            if (us < least && us < (large ? kWorth : kWorthOfFew) * one) {
                 least = us;
                 shape.slices = x;
                 shape.panels = panels;

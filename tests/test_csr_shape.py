@@ -20,7 +20,7 @@ def test_no_panels_where_one_launch_is_faster(rows, cols, degree, feat):
 
 
 @pytest.mark.parametrize("rows,cols,degree,feat", [(82_900, 82_900, 91, 480), (154_000, 154_000, 144, 160), (65_457, 124_653, 153, 64), (52_653, 64_065, 239, 128),
-                                                   (15_953, 21_959, 68, 608), (8_834, 12_228, 127, 992)])
+                                                   (15_953, 21_959, 68, 608), (8_834, 12_228, 127, 992), (18_984, 29_149, 256, 320), (11_316, 14_603, 133, 608)])
 def test_panels_where_they_are_faster(rows, cols, degree, feat):
     panels, rest = divmod(work_bytes(rows, cols, degree, feat), 4 * rows)
     assert 1 <= panels <= 7 and rest == 0
