@@ -13,7 +13,7 @@
 
 namespace {
 
-// A workgroup of four wavefronts takes 2, 8 or 16 consecutive rows (csr_rows_of_group); a wavefront takes the next rows
+// A workgroup of four wavefronts takes 2, 4, 8 or 16 consecutive rows (csr_rows_of_group); a wavefront takes the next rows
 // off a counter whenever it is through with its own, so that nothing waits for the longest row but itself.
 constexpr int kCsrThreads = 256;
 constexpr int kCsrChunkedRow = 512, kCsrChunk = 512;      // rows of more entries are cut into chunks, see csr_shape

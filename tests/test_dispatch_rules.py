@@ -20,10 +20,11 @@ def rules(tmp_path_factory):
 
 @pytest.mark.parametrize("rows,average,longest,group", [
     (2461, 367, 2301, 2), (4972, 271, 4533, 2), (2975, 162, 751, 2), (5120, 96, 288, 2),
-    (10_026, 276, 502, 8), (2840, 214, 287, 8), (5120, 96, 287, 8),            # rows of about one length
-    (5817, 266, 4201, 8), (9140, 107, 1051, 8), (5121, 96, 288, 8),            # more rows
+    (6149, 286, 4223, 2), (12_288, 208, 624, 2), (12_289, 208, 624, 4), (24_575, 400, 5000, 4),
+    (10_026, 276, 502, 8), (2840, 214, 287, 8), (5120, 96, 287, 8), (12_289, 208, 623, 8),      # rows of about one length
+    (9140, 107, 1051, 8), (5121, 207, 5000, 8),                                # more rows
     (2000, 60, 800, 8), (5120, 95, 288, 8), (3000, 200, 0, 8),                 # short rows; the longest one is not known
-    (24_575, 400, 5000, 8), (24_576, 400, 5000, 16), (2_000_000, 2, 100, 16)])
+    (24_576, 400, 5000, 16), (2_000_000, 2, 100, 16)])
 def test_rows_of_a_csr_workgroup(rules, rows, average, longest, group):
     size = ctypes.c_longlong
     assert rules.csr_rows(size(rows), size(rows * average), size(longest), 1) == group

@@ -138,9 +138,9 @@ def test_rows_of_a_workgroup(fa, torch, rows, average):
     assert (np.abs(got - ref) <= bound).all()
 
 
-@pytest.mark.parametrize("rows,average", [(4, 96), (7, 100), (1001, 97), (5120, 96), (5119, 250), (5121, 250)])
+@pytest.mark.parametrize("rows,average", [(4, 96), (7, 100), (1001, 97), (5120, 96), (5119, 250), (5121, 150), (12_288, 250), (12_289, 250), (24_573, 210)])
 def test_few_uneven_rows(fa, torch, rows, average):
-    """Two rows to a workgroup, and the least number of rows that takes eight again: rows of the average, empty ones, some of twice
+    """Two rows to a workgroup and four, and the least numbers of rows that take four and eight: rows of the average, empty ones, some of twice
     as much and a long one."""
     rng = np.random.default_rng(rows + average)
     cols = 3_001
