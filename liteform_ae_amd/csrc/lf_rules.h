@@ -10,17 +10,19 @@ constexpr long long kCsrManyRows = 24576;
 // Few long rows, some much longer than others: 2 to a workgroup, or 4 where they are more, as the last workgroups of 8 are left alone with
 // their longest rows for a part of the product that counts.  8 -> 2 rows, us: 2461 rows of 367, longest 2301, N = 64 34.7 -> 21.3; 4972 of 271, 4533,
 // N = 64 29.6 -> 22.7; 3025 of 227, 888, N = 192 32.5 -> 26.3; 2975 of 162, 751, N = 128 16.8 -> 15.9 (4 rows: 18.0); 12,890 of 212, 2179, N = 128, 4
-// rows 71.5 -> 66.5.  Beyond the lines: rows of one length, 10,026 of 276, longest 502, N = 64 34.4, with 2 35.3, 2840 of 214, 287, N = 160
-// 21.4, 22.3; more rows of less than kCsrVeryLong, 9140 of 107, 1051, N = 160 39.5, 40.3; 24,000 of 250, N = 96 with 2 6 % more, with 4 1; shorter ones,
-// 2000 of 60, N = 96 as long.  295 products of 2000 to 17,000 rows, N = 32 .. 512: the 162 by this rule take 0.90 of the time, 4 of them 1.01
-// to 1.07 (6714 of 352, N = 96 1.04 with one set of columns, 0.81 with another).
-constexpr long long kCsrFewRows = 5120, kCsrFewVeryLongRows = 12288;
-constexpr int kCsrLong = 96, kCsrVeryLong = 208, kCsrUneven = 3;
+// rows 71.5 -> 66.5; of one length, 4137 of 377, 703, N = 32 16.0 -> 13.5.  Beyond the lines: rows of one length, 10,026 of 276, longest 502, N = 64
+// 34.4, with 2 35.3, 2840 of 214, 287, N = 160 21.4, 22.3, 4705 of 235, 530, N = 96 24.4, 25.6; more rows of less than kCsrVeryLong, 9140 of
+// 107, 1051, N = 160 39.5, 40.3; 24,000 of 250, N = 96 with 2 6 % more, with 4 1; shorter ones, 2000 of 60, N = 96 as long.  295 products of
+// 2000 to 17,000 rows, N = 32 .. 512: the 179 by this rule take 0.90 of the time, 5 of them 1.01 to 1.07 (6714 of 352, N = 96 1.04 with one set
+// of columns, 0.81 with another).
+constexpr long long kCsrFewRows = 5120, kCsrFewEvenRows = 6144, kCsrFewVeryLongRows = 12288;
+constexpr int kCsrLong = 96, kCsrVeryLong = 208, kCsrEvenLong = 300;
 // entries: of the rows; longest: of all their entries (0: unknown); panels: that the entries are spread over, one of which the launch is for
 constexpr int csr_rows_of_group(long long rows, long long entries, long long longest, int panels) {
     if (rows >= kCsrManyRows) return kCsrRowsMany;
-    if (longest * rows < kCsrUneven * entries) return kCsrRowsFew;
     const long long of_panel = entries / panels;
+    if (rows <= kCsrFewEvenRows && of_panel >= kCsrEvenLong * rows) return 2;
+    if (2 * longest * rows < 5 * entries) return kCsrRowsFew;                  // (no row of two and a half times the average)
     if (of_panel >= kCsrVeryLong * rows) return rows <= kCsrFewVeryLongRows ? 2 : 4;
     return rows <= kCsrFewRows && of_panel >= kCsrLong * rows ? 2 : kCsrRowsFew;
 }

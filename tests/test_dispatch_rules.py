@@ -19,9 +19,10 @@ def rules(tmp_path_factory):
 
 
 @pytest.mark.parametrize("rows,average,longest,group", [
-    (2461, 367, 2301, 2), (4972, 271, 4533, 2), (2975, 162, 751, 2), (5120, 96, 288, 2),
-    (6149, 286, 4223, 2), (12_288, 208, 624, 2), (12_289, 208, 624, 4), (24_575, 400, 5000, 4),
-    (10_026, 276, 502, 8), (2840, 214, 287, 8), (5120, 96, 287, 8), (12_289, 208, 623, 8),      # rows of about one length
+    (2461, 367, 2301, 2), (4972, 271, 4533, 2), (2975, 162, 751, 2), (5120, 96, 240, 2),
+    (6149, 286, 4223, 2), (12_288, 208, 520, 2), (12_289, 208, 520, 4), (24_575, 400, 5000, 4),
+    (4137, 377, 703, 2), (6144, 300, 300, 2), (6144, 299, 400, 8), (6145, 300, 400, 8),         # rows of about one length
+    (10_026, 276, 502, 8), (2840, 214, 287, 8), (5120, 96, 239, 8), (12_289, 208, 519, 8),
     (9140, 107, 1051, 8), (5121, 207, 5000, 8),                                # more rows
     (2000, 60, 800, 8), (5120, 95, 288, 8), (3000, 200, 0, 8),                 # short rows; the longest one is not known
     (24_576, 400, 5000, 16), (2_000_000, 2, 100, 16)])
